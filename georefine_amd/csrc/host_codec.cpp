@@ -10,15 +10,14 @@
 // with the same argument meaning, ownership and status codes.  The
 // implementation is organised differently from the reference: one table
 // object (`SymbolTables`) validates the frequency rows once and answers
-// slot -> symbol queries through a 4096-entry coarse index followed by a short
-// forward scan of the inclusive prefix sums, and one templated walker serves
+// slot -> symbol queries with one bucket entry (a search in the prefix sums where
+// a bucket holds several symbols), and one templated walker serves
 // plain decoding and checkpoint recording for both wire formats.  No function
 // keeps state between calls, so all of them may run concurrently.
 #include <algorithm>
 #include <cstdint>
 #include <cstdlib>
 #include <cstring>
-#include <functional>
 #include <limits>
 #include <new>
 #include <vector>
@@ -28,8 +27,6 @@ namespace {
 constexpr uint32_t kScaleBits = 16;
 constexpr uint32_t kTotal = 1u << kScaleBits;
 constexpr uint32_t kLow = 1u << 23;
-constexpr uint32_t kCoarseShift = 4;  // 4096 coarse buckets per context
-constexpr uint32_t kCoarse = kTotal >> kCoarseShift;
 
 inline uint32_t main_symbol(uint16_t w) { return (w >> 5) & 0x3FFu; }
 inline uint32_t residual_symbol(uint16_t w) { return ((uint32_t)(w >> 15) << 5) | (w & 31u); }
@@ -37,16 +34,26 @@ inline uint32_t residual_symbol(uint16_t w) { return ((uint32_t)(w >> 15) << 5) 
 enum class Walk { ok, bad_context, dead_context, bad_symbol, overflow, overrun, bad_tail, bad_head };
 
 // Validated frequency rows plus the lookup structures derived from them.
+//
+// A context's 65536 slots are cut into kBuckets buckets, and a bucket's entry holds the symbol that
+// owns most of its slots, with the symbol's start and frequency: one load answers a query, unless a
+// symbol boundary inside the bucket put the slot elsewhere (a search in the prefix sums then).
+// 512 buckets: the four contexts that are live in a row of a frame (its row class by every column
+// class) take 16 KiB and stay in the first-level cache with the stream, where 1024 buckets do not;
+// about one query in twenty searches (a predicted branch otherwise).
 class SymbolTables {
  public:
   enum class Check { ok, overflow, bad_sum };
+  struct Entry {
+    uint16_t symbol, start;
+    uint32_t freq;  // 0 in contexts that are not live: no slot is ever inside
+  };
   // A row is usable ("live") when it sums to the total.  Rows that overflow the
   // total are always an error; rows with any other sum are an error unless
   // `partial_rows_are_dead` (then they only fail when a symbol selects them).
   Check build(const uint32_t *freq, uint32_t nctx, uint32_t vocab, bool partial_rows_are_dead = false) {
     nctx_ = nctx;
     vocab_ = vocab;
-    freq_ = freq;
     prefix_.assign((size_t)nctx * (vocab + 1), 0);
     live_.assign(nctx, 0);
     for (uint32_t c = 0; c < nctx; ++c) {
@@ -61,41 +68,45 @@ class SymbolTables {
       if (run != 0 && run != kTotal && !partial_rows_are_dead) return Check::bad_sum;
       live_[c] = run == kTotal;
     }
-    {
-      coarse_.assign((size_t)nctx * kCoarse, 0);
-      for (uint32_t c = 0; c < nctx; ++c) {
-        if (!live_[c]) continue;
-        const uint32_t *p = prefix_.data() + (size_t)c * (vocab + 1);
-        uint16_t *q = coarse_.data() + (size_t)c * kCoarse;
-        uint32_t s = 0;
-        for (uint32_t b = 0; b < kCoarse; ++b) {
-          const uint32_t first = b << kCoarseShift;
-          while (p[s + 1] <= first) ++s;
-          q[b] = (uint16_t)s;
+    entries_.assign((size_t)nctx * kBuckets, Entry{0, 0, 0});
+    for (uint32_t c = 0; c < nctx; ++c) {
+      if (!live_[c]) continue;
+      const uint32_t *p = prefix_.data() + (size_t)c * (vocab + 1);
+      Entry *q = entries_.data() + (size_t)c * kBuckets;
+      uint32_t s = 0;
+      for (uint32_t b = 0; b < kBuckets; ++b) {
+        const uint32_t lo = b << kBucketShift, hi = lo + (1u << kBucketShift);
+        while (p[s + 1] <= lo) ++s;
+        uint32_t best = s, most = 0;
+        for (uint32_t k = s; p[k] < hi; ++k) {
+          const uint32_t held = std::min(p[k + 1], hi) - std::max(p[k], lo);
+          if (held > most) best = k, most = held;
+          if (p[k + 1] >= hi) break;
         }
+        q[b] = Entry{(uint16_t)best, (uint16_t)p[best], p[best + 1] - p[best]};
       }
     }
     return Check::ok;
   }
   bool live(uint32_t c) const { return live_[c] != 0; }
   uint32_t nctx() const { return nctx_; }
-  uint32_t vocab() const { return vocab_; }
-  // symbol whose half-open slot range contains `slot`; context must be live
-  inline uint32_t find(uint32_t c, uint32_t slot, uint32_t &start, uint32_t &f) const {
+  const Entry *entries() const { return entries_.data(); }
+  // symbol whose half-open slot range contains `slot`, by a scan from symbol `s`; context must be live
+  Entry find(uint32_t c, uint32_t slot, uint32_t s) const {
     const uint32_t *p = prefix_.data() + (size_t)c * (vocab_ + 1);
-    uint32_t s = coarse_[(size_t)c * kCoarse + (slot >> kCoarseShift)];
+    while (p[s] > slot) --s;
     while (p[s + 1] <= slot) ++s;
-    start = p[s];
-    f = p[s + 1] - p[s];
-    return s;
+    return Entry{(uint16_t)s, (uint16_t)p[s], p[s + 1] - p[s]};
   }
-  inline uint32_t start_of(uint32_t c, uint32_t s) const { return prefix_[(size_t)c * (vocab_ + 1) + s]; }
+  const Entry &bucket(uint32_t c, uint32_t slot) const {
+    return entries_[((size_t)c << kBucketBits) + (slot >> kBucketShift)];
+  }
+  static constexpr uint32_t kBucketBits = 9, kBuckets = 1u << kBucketBits, kBucketShift = kScaleBits - kBucketBits;
 
  private:
   uint32_t nctx_ = 0, vocab_ = 0;
-  const uint32_t *freq_ = nullptr;
   std::vector<uint32_t> prefix_;
-  std::vector<uint16_t> coarse_;
+  std::vector<Entry> entries_;
   std::vector<uint8_t> live_;
 };
 
@@ -105,69 +116,176 @@ inline bool read_head(const uint8_t *s, size_t bytes, uint32_t &state) {
   return state >= kLow;
 }
 
-// One forward pass over a stream.  `context(i)` yields the model row of symbol i,
-// `mark(i, state, ip)` is called before symbol i is decoded.
-template <class ContextFn, class MarkFn>
-Walk walk_stream(const uint8_t *stream, size_t bytes, uint64_t n, const SymbolTables &t, ContextFn context,
-                 MarkFn mark, uint16_t *out) {
+struct Position {
   uint32_t state;
-  if (!read_head(stream, bytes, state)) return Walk::bad_head;
-  size_t ip = 4;
-  for (uint64_t i = 0; i < n; ++i) {
-    mark(i, state, ip);
+  size_t ip;
+};
+
+// `count` symbols from `at`, every one checked: contexts, stream bounds, state overflow.
+template <class ContextFn>
+Walk walk_checked(const SymbolTables &t, const uint8_t *stream, size_t bytes, ContextFn context, uint32_t count,
+                  Position &at, uint16_t *out) {
+  for (uint32_t i = 0; i < count; ++i) {
     const uint32_t c = context(i);
     if (c >= t.nctx()) return Walk::bad_context;
     if (!t.live(c)) return Walk::dead_context;
-    const uint32_t slot = state & (kTotal - 1);
-    uint32_t start, f;
-    const uint32_t s = t.find(c, slot, start, f);
-    out[i] = (uint16_t)s;
-    const uint64_t next = (uint64_t)f * (state >> kScaleBits) + (slot - start);
+    const uint32_t slot = at.state & (kTotal - 1);
+    const SymbolTables::Entry e = t.find(c, slot, t.bucket(c, slot).symbol);
+    out[i] = e.symbol;
+    const uint64_t next = (uint64_t)e.freq * (at.state >> kScaleBits) + (slot - e.start);
     if (next > std::numeric_limits<uint32_t>::max()) return Walk::overflow;
-    state = (uint32_t)next;
-    while (state < kLow) {
-      if (ip >= bytes) return Walk::overrun;
-      state = (state << 8) | stream[ip++];
+    at.state = (uint32_t)next;
+    while (at.state < kLow) {
+      if (at.ip >= bytes) return Walk::overrun;
+      at.state = (at.state << 8) | stream[at.ip++];
     }
   }
-  return (ip == bytes && state == kLow) ? Walk::ok : Walk::bad_tail;
+  return Walk::ok;
+}
+
+// value < limit ? then : otherwise, as a conditional move (left alone the compiler branches, which
+// mispredicts on half of the symbols).
+template <uint32_t limit>
+inline uint32_t select_below(bool below, uint32_t value, uint32_t then, uint32_t otherwise) {
+#if defined(__x86_64__)
+  (void)below;
+  asm("cmpl %[limit], %[value]\n\tcmovb %[then], %[result]"
+      : [result] "+r"(otherwise)
+      : [value] "r"(value), [limit] "i"(limit), [then] "r"(then)
+      : "cc");
+  return otherwise;
+#else
+  (void)value;
+  return below ? then : otherwise;
+#endif
+}
+
+// The same where nothing has to be checked but the contexts' liveness: contexts in range, a state
+// in [2^23, 2^31) and at least two bytes a symbol and two more in the stream.  The state is the
+// serial chain: bucket, entry load, multiply, refill.  The refill takes no branch (its outcome is
+// as random as the stream) and no count either: the states after zero, one and two bytes are all
+// made and two compares pick one, which is four cycles of the chain where a count and two shifts
+// are eight.  Returns false on a context that is not live.
+template <class ContextFn>
+bool walk_fast(const SymbolTables &t, const uint8_t *stream, ContextFn context, uint32_t count, Position &at, uint16_t *out) {
+  const uint8_t *entries = reinterpret_cast<const uint8_t *>(t.entries());
+  constexpr uint32_t kPitchBits = SymbolTables::kBucketBits + 3;  // of a context's entries, in bytes
+  uint32_t x = at.state;
+  const uint8_t *ip = stream + at.ip;
+  for (uint32_t i = 0; i < count; ++i) {
+    const uint32_t c = context(i), slot = x & (kTotal - 1);
+    uint16_t two;
+    std::memcpy(&two, ip, 2);
+    two = __builtin_bswap16(two);
+    // (three loads of the entry's fields side by side, not one that the chain then shifts apart)
+    const uint8_t *of_context = entries + ((size_t)c << kPitchBits);
+    asm("" : "+r"(of_context));  // (made ahead of the chain: the bucket's offset goes into the loads' address)
+    const auto *at_bucket = reinterpret_cast<const SymbolTables::Entry *>(
+        of_context + ((x >> (SymbolTables::kBucketShift - 3)) & ((1u << kPitchBits) - 8)));
+    uint32_t freq = at_bucket->freq, rel = slot - at_bucket->start, symbol = at_bucket->symbol;
+    if (__builtin_expect(rel >= freq, 0)) {
+      if (!t.live(c)) return false;
+      const SymbolTables::Entry e = t.find(c, slot, symbol);
+      freq = e.freq, rel = slot - e.start, symbol = e.symbol;
+    }
+    out[i] = (uint16_t)symbol;
+    x = freq * (x >> kScaleBits) + rel;
+    const uint32_t one_more = (x << 8) | (two >> 8), two_more = (x << 16) | two;
+    const bool low = x < kLow, lower = x < (kLow >> 8);
+    ip += (size_t)low + (size_t)lower;
+    x = select_below<(kLow >> 8)>(lower, x, two_more, select_below<kLow>(low, x, one_more, x));
+  }
+  at.state = x;
+  at.ip = (size_t)(ip - stream);
+  return true;
+}
+
+// One forward pass over a stream, in runs: `context.run(i, most)` gives the length of the next run
+// (from symbol i, at most `most`) and `context.of(k)` the model row of its k-th symbol;
+// `mark(i, state, ip)` is called before symbol i where `mark.next()` says so.
+template <class Contexts, class Mark>
+Walk walk_stream(const uint8_t *stream, size_t bytes, uint64_t n, const SymbolTables &t, Contexts contexts, Mark &mark,
+                 uint16_t *out) {
+  Position at{0, 4};
+  if (!read_head(stream, bytes, at.state)) return Walk::bad_head;
+  const bool in_range = contexts.in_range(t.nctx());
+  for (uint64_t i = 0; i < n;) {
+    if (i == mark.next()) mark(i, at.state, at.ip);
+    // (towards the stream's end shorter runs, so that only its last symbols are walked with every check)
+    const size_t room = bytes - at.ip > 130 ? (bytes - at.ip - 2) / 2 : 64;
+    const uint32_t count = contexts.run(i, (uint32_t)std::min<uint64_t>({n - i, mark.next() - i, room, 1u << 16}));
+    auto context = contexts.of();
+    if (in_range && at.state < 0x80000000u && at.ip + 2 * (size_t)count + 2 <= bytes) {
+      if (!walk_fast(t, stream, context, count, at, out + i)) return Walk::dead_context;
+    } else {
+      const Walk w = walk_checked(t, stream, bytes, context, count, at, out + i);
+      if (w != Walk::ok) return w;
+    }
+    i += count;
+  }
+  return (at.ip == bytes && at.state == kLow) ? Walk::ok : Walk::bad_tail;
 }
 
 struct NoMark {
-  void operator()(uint64_t, uint32_t, size_t) const {}
+  uint64_t next() const { return std::numeric_limits<uint64_t>::max(); }
+  void operator()(uint64_t, uint32_t, size_t) {}
 };
 
 struct StrideMark {
   uint32_t stride;
   uint32_t *states, *offsets;
-  uint64_t next = 0;
+  uint64_t at = 0;
   size_t k = 0;
-  void operator()(uint64_t i, uint32_t state, size_t ip) {
-    if (i == next) {
-      states[k] = state;
-      offsets[k] = (uint32_t)ip;
-      ++k;
-      next += stride;
-    }
+  uint64_t next() const { return at; }
+  void operator()(uint64_t, uint32_t state, size_t ip) {
+    states[k] = state;
+    offsets[k] = (uint32_t)ip;
+    ++k;
+    at += stride;
   }
 };
 
-// Row-major (row class, column class) context without a division per symbol.
+// Row-major (row class, column class) contexts; a run stays inside a row.
 struct GridContext {
   const uint8_t *rc, *cc;
-  uint32_t cols, nc, row = 0, col = 0;
-  uint32_t operator()(uint64_t) {
-    const uint32_t c = (uint32_t)rc[row] * nc + cc[col];
-    if (++col == cols) {
-      col = 0;
-      ++row;
-    }
-    return c;
+  uint32_t rows, cols, nc;
+  uint32_t row = 0, col = 0;  // where the next run begins
+  uint32_t base = 0;          // of the current run: its row's first context ...
+  const uint8_t *classes = nullptr;  // ... and its columns' classes
+  bool in_range(uint32_t nctx) const {
+    uint32_t top_row = 0, top_col = 0;
+    for (uint32_t r = 0; r < rows; ++r) top_row = std::max<uint32_t>(top_row, rc[r]);
+    for (uint32_t c = 0; c < cols; ++c) top_col = std::max<uint32_t>(top_col, cc[c]);
+    return top_row * nc + top_col < nctx;
+  }
+  uint32_t run(uint64_t, uint32_t most) {
+    base = (uint32_t)rc[row] * nc;
+    classes = cc + col;
+    const uint32_t count = std::min(most, cols - col);
+    col += count;
+    if (col == cols) col = 0, ++row;
+    return count;
+  }
+  auto of() const {
+    return [base = base, classes = classes](uint32_t k) { return base + classes[k]; };
   }
 };
 struct ArrayContext {
   const uint16_t *ctx;
-  uint32_t operator()(uint64_t i) const { return ctx[i]; }
+  uint64_t n;
+  const uint16_t *at = nullptr;
+  bool in_range(uint32_t nctx) const {
+    uint32_t top = 0;
+    for (uint64_t i = 0; i < n; ++i) top = std::max<uint32_t>(top, ctx[i]);
+    return top < nctx;
+  }
+  uint32_t run(uint64_t i, uint32_t most) {
+    at = ctx + i;
+    return most;
+  }
+  auto of() const {
+    return [at = at](uint32_t k) { return (uint32_t)at[k]; };
+  }
 };
 
 // ---- frequency normalisation: largest remainders, deterministic ties ----
@@ -263,8 +381,7 @@ void bcx_count_and_normalize(const uint16_t *w, uint64_t n, uint32_t cols, const
   if (kind) {
     for (uint64_t i = 0; i < n; ++i) ++hist[(size_t)main_symbol(w[i]) * 64 + residual_symbol(w[i])];
   } else {
-    GridContext g{rc, cc, cols, nc};
-    for (uint64_t i = 0; i < n; ++i) ++hist[(size_t)g(i) * 1024 + main_symbol(w[i])];
+    for (uint64_t i = 0; i < n; ++i) ++hist[((size_t)rc[i / cols] * nc + cc[i % cols]) * 1024 + main_symbol(w[i])];
   }
   for (uint32_t c = 0; c < sh.nctx; ++c)
     normalize_row(hist.data() + (size_t)c * sh.vocab, sh.vocab, freq + (size_t)c * sh.vocab);
@@ -280,8 +397,9 @@ int bcx_decode_any(const uint8_t *stream, size_t bytes, uint64_t n, uint32_t row
   SymbolTables t;
   // the reference bounds each frequency by the room left in its row
   if (t.build(freq, sh.nctx, sh.vocab) != SymbolTables::Check::ok) return 2;
-  Walk w = kind ? walk_stream(stream, bytes, n, t, ArrayContext{resctx}, NoMark{}, out)
-                : walk_stream(stream, bytes, n, t, GridContext{rc, cc, cols, nc}, NoMark{}, out);
+  NoMark none;
+  Walk w = kind ? walk_stream(stream, bytes, n, t, ArrayContext{resctx, n}, none, out)
+                : walk_stream(stream, bytes, n, t, GridContext{rc, cc, rows, cols, nc}, none, out);
   return w == Walk::ok ? 0 : 2;
 }
 
@@ -432,9 +550,8 @@ int bcx_checkpoint(const uint8_t *stream, size_t stream_bytes, uint64_t n, uint3
         std::vector<uint32_t> st(count), of(count);
         std::vector<uint16_t> sym((size_t)n);
         StrideMark mark{stride, st.data(), of.data()};
-        Walk w = kind ? walk_stream(stream, stream_bytes, n, t, ArrayContext{resctx}, std::ref(mark), sym.data())
-                      : walk_stream(stream, stream_bytes, n, t, GridContext{rc, cc, cols, nc}, std::ref(mark),
-                                    sym.data());
+        Walk w = kind ? walk_stream(stream, stream_bytes, n, t, ArrayContext{resctx, n}, mark, sym.data())
+                      : walk_stream(stream, stream_bytes, n, t, GridContext{rc, cc, rows, cols, nc}, mark, sym.data());
         switch (w) {
           case Walk::ok:
             break;
@@ -519,7 +636,8 @@ int p_decode(const uint8_t *st, size_t bytes, uint64_t n, const uint16_t *cx, ui
         SymbolTables t;
         // a row whose sum is wrong only fails (4) when a symbol selects it
         if (t.build(f, nc, vocab, true) != SymbolTables::Check::ok) return 3;
-        switch (walk_stream(st, bytes, n, t, ArrayContext{cx}, NoMark{}, out)) {
+        NoMark none;
+        switch (walk_stream(st, bytes, n, t, ArrayContext{cx, n}, none, out)) {
           case Walk::ok:
             return 0;
           case Walk::bad_context:
@@ -552,7 +670,7 @@ static int ppcx_checkpoint_impl(const uint8_t *stream, size_t bytes, uint64_t n,
         const size_t count = (size_t)((n + stride - 1) / stride);
         std::vector<uint32_t> st(count), of(count);
         StrideMark mark{stride, st.data(), of.data()};
-        switch (walk_stream(stream, bytes, n, t, ArrayContext{ctx}, std::ref(mark), symbols)) {
+        switch (walk_stream(stream, bytes, n, t, ArrayContext{ctx, n}, mark, symbols)) {
           case Walk::ok:
             break;
           case Walk::bad_context:

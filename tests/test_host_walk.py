@@ -1,0 +1,34 @@
+"""The host coder's walks against the oracle where their cuts fall: runs at row ends and marks, the
+last symbols of a stream, contexts that are one symbol, symbols behind a bucket's boundary."""
+import numpy as np
+import pytest
+
+from georefine_amd import bitexact_context_codec as codec
+from georefine_amd.bitexact_context_gpu import checkpoints
+
+
+def _words(kind, rows, cols):
+    rng = np.random.default_rng(rows * 1009 + cols)
+    if kind == "weights":  # a few dozen symbols per context, as coded weights have
+        w = (rng.standard_normal((rows, cols)) * 0.02 * rng.lognormal(0, 0.5, (rows, 1))).astype(np.float32)
+        return (w.view(np.uint32) >> 16).astype(np.uint16)
+    if kind == "flat":  # every symbol in every context: several a bucket
+        return rng.integers(0, 65536, (rows, cols), dtype=np.uint16)
+    return np.where(rng.random((rows, cols)) < 0.01, 0x4000, 0x3F80).astype(np.uint16)
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 1), (3, 63), (64, 65), (5, 4099), (300, 300)])
+@pytest.mark.parametrize("kind", ["weights", "flat", "two"])
+def test_walks_match_the_oracle(oracle, kind, rows, cols):
+    words = _words(kind, rows, cols)
+    rc, cc = codec._labels(words, 4, 4)
+    for stream_kind in (0, 1):
+        main = ((words >> 5) & 0x3FF).ravel() if stream_kind else None
+        freq, stream = codec._encode_kind(codec._lib(), words, rc, cc, 4, 4, stream_kind)
+        table = np.frombuffer(freq, dtype="<u4").reshape((1024, 64) if stream_kind else (16, 1024))
+        want_freq, want_stream = oracle.bcx_encode_kind(words, rc, cc, 4, 4, stream_kind)
+        assert np.array_equal(table.ravel(), np.asarray(want_freq).ravel()) and stream == bytes(want_stream)
+        for stride in (1, 64, rows * cols):
+            got = checkpoints(stream, table, rc, cc, (rows, cols), 4, 4, stride, main)
+            want = oracle.bcx_checkpoint(stream, table, rc, cc, rows, cols, 4, 4, stride, main)
+            assert all(np.array_equal(a, b) for a, b in zip(got, want))
