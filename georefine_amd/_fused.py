@@ -7,10 +7,14 @@ become a coarse u8 lookup plus a sparse table of the symbols that occur.
 """
 from __future__ import annotations
 
+import ctypes
+import heapq
 import math
 import os
 
 import numpy as np
+
+from . import _native
 
 MAX_LDS = 160 * 1024
 LUT_BUDGET = int(os.environ.get("GEOREFINE_FUSED_LUT_BYTES", 32 * 1024))
@@ -60,35 +64,17 @@ def sparse_tables(freq, nr, nc, shift, image=None):
         raise FusedUnsupported("no live context")
     if tabn > 255:
         raise FusedUnsupported("more than 255 distinct symbols in one context")
-    lognb = 16 - shift
-    nb = 1 << lognb
-    lut = np.zeros((nr, nc, nb), dtype=np.uint8)
-    tab = np.zeros((nr, nc, tabn + 1), dtype=np.uint64)
-    lo_slot = (np.arange(nb, dtype=np.int64) << shift)
-    hi_slot = lo_slot + (1 << shift)
-    for rho in range(nr):
-        for c in range(nc):
-            f = freq[rho * nc + c].astype(np.int64)
-            syms = np.flatnonzero(f)
-            if syms.size == 0:
-                continue
-            fs = f[syms]
-            starts = np.concatenate(([0], np.cumsum(fs)[:-1]))
-            ends = starts + fs
-            lo = starts | ((fs & 0xFFFF) << 16)
-            hi = syms << 5 if image is None else image(syms)
-            tab[rho, c, :syms.size] = (lo.astype(np.uint64) | (hi.astype(np.uint64) << np.uint64(32)))
-            first = np.searchsorted(starts, lo_slot, side="right") - 1
-            last = np.searchsorted(starts, hi_slot - 1, side="right") - 1
-            best, best_overlap = first.copy(), np.zeros(nb, dtype=np.int64)
-            for k in range(int((last - first).max()) + 1):
-                cand = np.minimum(first + k, last)
-                overlap = np.minimum(ends[cand], hi_slot) - np.maximum(starts[cand], lo_slot)
-                better = overlap > best_overlap
-                best = np.where(better, cand, best)
-                best_overlap = np.where(better, overlap, best_overlap)
-            lut[rho, c] = best.astype(np.uint8)
-    return lut.reshape(nr, nc * nb), tab.reshape(nr, nc * (tabn + 1)), tabn
+    nb = 1 << (16 - shift)
+    freq = np.ascontiguousarray(freq, dtype=np.uint32)
+    symbols = np.arange(freq.shape[1])
+    images = np.ascontiguousarray(symbols << 5 if image is None else image(symbols), dtype=np.uint32)
+    lut = np.empty((nr, nc * nb), dtype=np.uint8)
+    tab = np.empty((nr, nc * (tabn + 1)), dtype=np.uint64)
+    if _native.codec().grf_sparse_tables(_native.ptr(freq, ctypes.c_uint32), nr * nc, freq.shape[1], shift,
+                                         _native.ptr(images, ctypes.c_uint32), tabn, _native.ptr(lut, ctypes.c_uint8),
+                                         _native.ptr(tab, ctypes.c_uint64)):
+        raise FusedUnsupported("frequencies of a context do not add up to 65536")
+    return lut, tab, tabn
 
 
 X_PAD = 8
@@ -166,11 +152,18 @@ def _tiles(class_rows, r):
     return sum(-(-int(cnt) // r) for cnt in class_rows if cnt)
 
 
-def _spread_rows(class_rows, r, capacity, floor=1):
+def _tile_counts(class_rows, most):
+    """[.., tiles of r rows, ..] for r = 0 (unused) .. most: the planners look these up thousands
+    of times a matrix."""
+    r = np.arange(1, most + 1, dtype=np.int64)
+    return [0] + (-(-np.asarray(class_rows, dtype=np.int64)[:, None] // r)).sum(axis=0).tolist()
+
+
+def _spread_rows(tile_counts, r, capacity, floor=1):
     """Fewer rows per tile while the tiles still fit the workgroup slots of the rounds
     already paid for: idle lanes do not slow a workgroup down, idle CUs do (measured +4 % on
     17408 x 5120 going from 464 tiles of 38 rows to 512 of 34)."""
-    while r > floor and _tiles(class_rows, r - 1) <= capacity:
+    while r > floor and tile_counts[r - 1] <= capacity:
         r -= 1
     return r
 
@@ -198,6 +191,7 @@ def choose_tiling(spr, class_rows, piece_cap_fn, lds_fn, cus=256, seg_len=64, ta
     thread_choices = range(1024, 0, -64)
     lane_choices = None
     forced_rows = None
+    tile_counts = _tile_counts(class_rows, 1024)
     if forced:
         t_, p_, *rest = (int(v) for v in forced.split(","))
         thread_choices, lane_choices = [t_], [min(p_, spr)]
@@ -214,7 +208,7 @@ def choose_tiling(spr, class_rows, piece_cap_fn, lds_fn, cus=256, seg_len=64, ta
                 continue  # a narrower slab of the same count wastes fewer lanes; it was scored already
             lanes = p * r
             lane_eff = spr / (n_slabs * p) * (lanes / threads)
-            tiles = _tiles(class_rows, r)
+            tiles = tile_counts[r]
             fill = total_rows / (tiles * r)
             cap = piece_cap_fn(p)
             lds = lds_fn(p, r, cap)
@@ -240,8 +234,8 @@ def choose_tiling(spr, class_rows, piece_cap_fn, lds_fn, cus=256, seg_len=64, ta
     best = max((c for c in candidates if c[0] >= 0.985 * top), key=lambda c: (-c[4], c[0], c[1]))
     _, threads, p, r, n_slabs, tiles, cap, lds, capacity = best
     if not forced_rows:
-        r = _spread_rows(class_rows, r, capacity)
-        tiles, lds = _tiles(class_rows, r), lds_fn(p, r, cap)
+        r = _spread_rows(tile_counts, r, capacity)
+        tiles, lds = tile_counts[r], lds_fn(p, r, cap)
     return threads, p, r, n_slabs, tiles, cap, lds
 
 
@@ -278,6 +272,7 @@ def choose_wave_tiling(spr, class_rows, piece_cap_fn, lds_fn, cus=256, seg_len=6
         n_slabs = -(-spr // p_)
         return t_, p_, r_, n_slabs, _tiles(class_rows, r_), cap, lds_fn(t_, p_, r_, n_slabs, cap)
     best = None
+    tile_counts = _tile_counts(class_rows, 128)
     table_steps = 3 + table_bytes / 12288
     for p in (4, 8, 16, 32, 64):
         if p > 4 and p // 2 >= spr:
@@ -294,7 +289,7 @@ def choose_wave_tiling(spr, class_rows, piece_cap_fn, lds_fn, cus=256, seg_len=6
                     break
                 # six waves per SIMD by registers; a little LDS stays with the system
                 per_cu = max(1, min(24 // nwaves, (MAX_LDS - 1024) // lds))
-                tiles = _tiles(class_rows, r)
+                tiles = tile_counts[r]
                 rounds = -(-tiles // (cus * per_cu))
                 units = -(-r // rpw) * n_slabs
                 busiest = 0.5 * -(-units // nwaves) + 0.5 * units / nwaves
@@ -327,6 +322,7 @@ def choose_gemm_tiling(spr, class_rows, piece_cap_fn, lds_fn, cus=256, seg_len=6
     capacity, LDS bytes, k)."""
     best = None
     total_rows = sum(int(c) for c in class_rows)
+    tile_counts = _tile_counts(class_rows, 1024)
     forced = os.environ.get("GEOREFINE_FUSED_GEMM_TILING")  # "lanes_per_row,rows[,k_parts]": experiments only
     if forced:
         values = [int(v) for v in forced.split(",")]
@@ -349,9 +345,9 @@ def choose_gemm_tiling(spr, class_rows, piece_cap_fn, lds_fn, cus=256, seg_len=6
         per_simd = -(-(threads // 64) // 4)
         per_cu = max(1, min(GEMM_WAVES_PER_SIMD // per_simd, MAX_LDS // lds))
         slots = cus * per_cu
-        rounds = -(-(_tiles(class_rows, r) * k) // slots)
-        r_used = r if forced else _spread_rows(class_rows, r, rounds * slots // k, floor=16 * (row_blocks - 1) + 1)
-        tiles_used = _tiles(class_rows, r_used) * k
+        rounds = -(-(tile_counts[r] * k) // slots)
+        r_used = r if forced else _spread_rows(tile_counts, r, rounds * slots // k, floor=16 * (row_blocks - 1) + 1)
+        tiles_used = tile_counts[r_used] * k
         slabs_each = -(-n_slabs // k)
         # work = lane-steps; capacity = every wave slot of every round for the whole walk
         work = total_rows * spr
@@ -374,11 +370,7 @@ def order_residuals(raw, rows, cols, seg_len, block, position, held):
     segment s of position q at (((q // block * G + t) * spr + s) * block + q % block) * 12 with
     G = seg_len // 16.  A permutation of groups (no field is touched); positions that no row
     has hold zeros."""
-    spr, groups = cols // seg_len, seg_len // 16
-    ordered = np.zeros((held, groups, spr, 12), dtype=np.uint8)
-    ordered[position] = np.asarray(raw).reshape(rows, spr, groups, 12).transpose(0, 2, 1, 3)
-    ordered = ordered.reshape(held // block, block, groups, spr, 12).transpose(0, 2, 3, 1, 4)
-    return np.ascontiguousarray(ordered).reshape(-1)
+    return order_records(raw, rows, cols, seg_len, block, position, held, 16, 12)
 
 
 def order_index(values, rows, spr, block, position, held):
@@ -405,11 +397,14 @@ def order_records(raw, rows, cols, seg_len, block, position, held, record_symbol
     (((q // block * U + t) * spr + s) * block + q % block) * record_bytes, U = seg_len //
     record_symbols; positions that no row has hold zeros."""
     spr, per_seg = cols // seg_len, seg_len // record_symbols
-    ordered = np.zeros((held, per_seg, spr, record_bytes), dtype=np.uint8)
-    ordered[position] = np.asarray(raw)[:rows * spr * per_seg * record_bytes].reshape(
-        rows, spr, per_seg, record_bytes).transpose(0, 2, 1, 3)
-    ordered = ordered.reshape(held // block, block, per_seg, spr, record_bytes).transpose(0, 2, 3, 1, 4)
-    return np.ascontiguousarray(ordered).reshape(-1)
+    raw = np.ascontiguousarray(raw, dtype=np.uint8)[:rows * spr * per_seg * record_bytes]
+    position = np.ascontiguousarray(position, dtype=np.uint32)
+    ordered = np.zeros(held * spr * per_seg * record_bytes, dtype=np.uint8)
+    if raw.size != rows * spr * per_seg * record_bytes or _native.codec().grf_order_records(
+            _native.ptr(raw, ctypes.c_uint8), rows, spr, per_seg, record_bytes, block, _native.ptr(position, ctypes.c_uint32),
+            held, _native.ptr(ordered, ctypes.c_uint8)):
+        raise ValueError("records do not fit the order")
+    return ordered
 
 
 def build_tiles(row_class, nr, r):
@@ -447,11 +442,16 @@ def build_balanced_tiles(row_class, nr, unit_rows, slots, max_rows):
     units = {rho: -(-int(counts[rho]) // unit_rows) for rho in live}
     tiles = {rho: 1 for rho in live}
     height = lambda rho: -(-units[rho] // tiles[rho])
-    for _ in range(slots - len(live)):  # the next tile to the class whose tiles are tallest
-        rho = max(live, key=lambda c: (height(c), units[c] / tiles[c]))  # (among equals: the fullest tiles)
+    # the next tile to the class whose tiles are tallest (among equals: the fullest tiles, then the first class)
+    order_of = lambda rho: (-height(rho), -units[rho] / tiles[rho], rho)
+    queue = [order_of(rho) for rho in live]
+    heapq.heapify(queue)
+    for _ in range(slots - len(live)):
+        rho = queue[0][2]
         if height(rho) <= 1:
             break
         tiles[rho] += 1
+        heapq.heapreplace(queue, order_of(rho))
     tallest = max(height(rho) for rho in live) * unit_rows
     if tallest > max_rows:
         return None
@@ -540,7 +540,7 @@ class FramePlan:
         self.seg_offset = np.concatenate((seg_offsets, [main_bytes])).astype(np.uint32)
         self.row_class = np.asarray(row_class)
         self.class_rows = np.bincount(self.row_class, minlength=nr)
-        self._caps = {}
+        self._caps, self._tilings = {}, {}
 
     def residual_order(self, block=None):
         """(block rows B, row positions u32[rows], rows of the array) of the resident residual
@@ -592,20 +592,30 @@ class FramePlan:
         (m = 0: the store sink).  ``waves``: the wave-unit scheme of the GEMV, one tiling for
         every row count (launches carry at most two rows each)."""
         if waves and m:
-            self._wave_limits()
-            threads, p, r, n_slabs, n_tiles, cap, lds = choose_wave_tiling(
-                self.spr, self.class_rows, self._cap,
-                lambda t_, p_, r_, s_, cap_: lds_bytes_waves(self.nc, self.lognb, self.tabn, WAVE_ROWS_PER_PASS, t_, p_,
-                                                             r_, s_, cap_),
-                seg_len=self.seg_len, table_bytes=self.table_bytes())
-        else:
-            threads, p, r, n_slabs, n_tiles, cap, lds = choose_tiling(
-                self.spr, self.class_rows, self._cap,
-                lambda p_, r_, cap_: lds_bytes(self.nc, self.lognb, self.tabn, m, p_, self.seg_len, r_, cap_),
-                seg_len=self.seg_len, table_bytes=self.table_bytes())
+            key = "waves", os.environ.get("GEOREFINE_FUSED_WAVE_TILING")
+            if key not in self._tilings:  # (one for every row count; the residual order asks for it too)
+                self._tilings[key] = self._wave_tiling()
+            return self._tilings[key]
+        threads, p, r, n_slabs, n_tiles, cap, lds = choose_tiling(
+            self.spr, self.class_rows, self._cap,
+            lambda p_, r_, cap_: lds_bytes(self.nc, self.lognb, self.tabn, m, p_, self.seg_len, r_, cap_),
+            seg_len=self.seg_len, table_bytes=self.table_bytes())
         tile_rows, tile_class = build_tiles(self.row_class, self.nr, r)
         assert len(tile_class) == n_tiles
-        if waves and m and not os.environ.get("GEOREFINE_FUSED_WAVE_TILING"):
+        return dict(tile_rows=tile_rows, tile_class=tile_class,
+                    scalars=dict(threads=threads, lanes_per_row=p, rows_per_tile=r, n_slabs=n_slabs,
+                                 n_tiles=n_tiles, piece_cap=cap, scheme=SCHEME_SLABS), lds=lds)
+
+    def _wave_tiling(self):
+        self._wave_limits()
+        threads, p, r, n_slabs, n_tiles, cap, lds = choose_wave_tiling(
+            self.spr, self.class_rows, self._cap,
+            lambda t_, p_, r_, s_, cap_: lds_bytes_waves(self.nc, self.lognb, self.tabn, WAVE_ROWS_PER_PASS, t_, p_,
+                                                         r_, s_, cap_),
+            seg_len=self.seg_len, table_bytes=self.table_bytes())
+        tile_rows, tile_class = build_tiles(self.row_class, self.nr, r)
+        assert len(tile_class) == n_tiles
+        if not os.environ.get("GEOREFINE_FUSED_WAVE_TILING"):
             # classes of very different sizes: the same workgroup slots, cut so that no tile is
             # taller than it has to be (the kernel walks a tile's real height)
             nwaves, rpw = threads // 64, 64 // p
@@ -618,8 +628,7 @@ class FramePlan:
                 lds = lds_bytes_waves(self.nc, self.lognb, self.tabn, WAVE_ROWS_PER_PASS, threads, p, r, n_slabs, cap)
         return dict(tile_rows=tile_rows, tile_class=tile_class,
                     scalars=dict(threads=threads, lanes_per_row=p, rows_per_tile=r, n_slabs=n_slabs,
-                                 n_tiles=n_tiles, piece_cap=cap,
-                                 scheme=SCHEME_WAVES if waves and m else SCHEME_SLABS), lds=lds)
+                                 n_tiles=n_tiles, piece_cap=cap, scheme=SCHEME_WAVES), lds=lds)
 
     def gather_scalars(self):
         """Scalars of a tiling that gives every requested row a tile of its own, all of its

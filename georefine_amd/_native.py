@@ -110,6 +110,13 @@ def codec():
                                          _u32, U32P, U32P, U16P]
             L.grf_bctx_join.argtypes = [U16P, U16P, _u64, U16P]
             L.grf_bctx_join.restype = _int
+            L.grf_bctx_words.argtypes = [U8P, _sz, _u32, _u32, U8P, U8P, _u32, _u32, U32P, _u32, U32P, U32P, U8P, _sz, U32P,
+                                         U16P, ctypes.POINTER(_u64)]
+            L.grf_bctx_words.restype = _int
+            L.grf_sparse_tables.argtypes = [U32P, _u32, _u32, _u32, U32P, _u32, U8P, ctypes.POINTER(_u64)]
+            L.grf_sparse_tables.restype = _int
+            L.grf_order_records.argtypes = [U8P, _u32, _u32, _u32, _u32, _u32, U32P, _u32, U8P]
+            L.grf_order_records.restype = _int
             L.p_encode.argtypes = [U16P, U16P, _u64, _u32, _u32, ctypes.POINTER(U32P), ctypes.POINTER(U8P),
                                    ctypes.POINTER(_sz)]
             L.p_decode.argtypes = [U8P, _sz, _u64, U16P, _u32, _u32, U32P, U16P]

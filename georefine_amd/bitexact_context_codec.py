@@ -18,7 +18,9 @@ import ctypes
 import hashlib
 import os
 import struct
+import time
 import zlib
+from concurrent.futures import ThreadPoolExecutor
 
 import numpy as np
 
@@ -227,11 +229,34 @@ def parse(frame):
 
     Returns a dict: ``mode nr nc shape digest`` and, for coded modes, ``rows columns
     main_freq [residual_freq] main_stream residual_stream``; for mode 1 ``raw``."""
+    frame = _frame_bytes(frame)
+    if not _frame_digests(frame)[0]:
+        raise CodecError("frame checksum mismatch")
+    info = _split(frame)
+    for name in ("main_stream", "residual_stream"):
+        if name in info:
+            info[name] = bytes(info[name])
+    return info
+
+
+def _frame_bytes(frame):
     if not isinstance(frame, (bytes, bytearray, memoryview)) or len(frame) < HEADER.size:
         raise CodecError("short frame")
-    frame = bytes(frame)
-    if len(frame) < HEADER.size + 32 or hashlib.sha256(frame[:-32]).digest() != frame[-32:]:
-        raise CodecError("frame checksum mismatch")
+    return bytes(frame)
+
+
+def _frame_digests(frame):
+    """(whether the frame's own checksum holds, SHA-256 of the whole frame in hex): one pass."""
+    if len(frame) < HEADER.size + 32:
+        return False, None
+    sha = hashlib.sha256(memoryview(frame)[:-32])
+    own = sha.digest() == frame[-32:]
+    sha.update(frame[-32:])
+    return own, sha.hexdigest()
+
+
+def _split(frame):
+    """``parse`` without the checksum; the streams are views of the frame."""
     magic, ver, mode, nr, nc, r, c, ml, tl, sl, dl, dig = HEADER.unpack_from(frame)
     if magic != MAGIC or ver != VERSION or nr not in ROWS or nc not in COLS:
         raise CodecError("unsupported frame header")
@@ -243,7 +268,7 @@ def parse(frame):
     if mode == 1:
         if ml or tl or sl or dl or len(frame) != end + 2 * n + 32:
             raise CodecError("invalid raw frame length")
-        raw = frame[end:-32]
+        raw = memoryview(frame)[end:-32]
         if hashlib.sha256(raw).digest() != dig:
             raise CodecError("raw checksum mismatch")
         info["raw"] = np.frombuffer(raw, dtype="<u2").copy().reshape(r, c)
@@ -263,27 +288,117 @@ def parse(frame):
     info["main_freq"] = np.frombuffer(tables[:main_bytes], dtype="<u4").copy().reshape(nr * nc, MAIN_VOCAB)
     if mode == 128:
         info["residual_freq"] = np.frombuffer(tables[main_bytes:], dtype="<u4").copy().reshape(RES_CONTEXTS, RES_VOCAB)
-    info["main_stream"] = frame[at:at + sl]
-    info["residual_stream"] = frame[at + sl:at + sl + dl]
+    info["main_stream"] = memoryview(frame)[at:at + sl]
+    info["residual_stream"] = memoryview(frame)[at + sl:at + sl + dl]
     return info
+
+
+class _Now:
+    """A result that was computed at once (what a pool's future is for small inputs)."""
+
+    def __init__(self, value):
+        self.value = value
+
+    def result(self):
+        return self.value
+
+
+class Beside:
+    """One thread for work beside the caller's (hashing, a second stream), for as long as the
+    ``with`` block; inputs under ``BESIDE_FROM`` bytes are not worth one and run at once."""
+
+    BESIDE_FROM = 1 << 18
+
+    def __init__(self, nbytes, workers=1):
+        self.pool = ThreadPoolExecutor(max_workers=workers) if nbytes >= self.BESIDE_FROM else None
+
+    def __enter__(self):
+        return self
+
+    def __exit__(self, *exc):
+        if self.pool is not None:
+            self.pool.shutdown()
+
+    def run(self, fn, *args):
+        return self.pool.submit(fn, *args) if self.pool is not None else _Now(fn(*args))
+
+
+def _sha_following(words, progress):
+    """SHA-256 of ``words`` while they are written: ``progress[0]`` of them are final.  None if
+    the walk gave up (a count beyond the end)."""
+    sha, view, done, step = hashlib.sha256(), memoryview(words).cast("B"), 0, 1 << 17
+    while done < words.size:
+        ready = int(progress[0])
+        if ready > words.size:
+            return None
+        if ready - done < min(step, words.size - done):
+            time.sleep(1e-4)
+            continue
+        sha.update(view[2 * done:2 * ready])
+        done = ready
+    return sha.digest()
+
+
+def read_words(frame, stride=0, failed="rANS decode failed ({})"):
+    """A whole frame decoded and checked against its own checksum: the dict of ``parse`` with
+    ``words`` (one-dimensional), ``words_digest`` and ``frame_sha256``; with ``stride`` also
+    the main stream's index, ``main_states`` and ``main_offsets``.  The walk runs on the caller's
+    thread (and one in the library); the frame and the finished words are hashed beside it."""
+    frame = _frame_bytes(frame)
+    with Beside(len(frame)) as beside:
+        digests = beside.run(_frame_digests, frame)
+        try:
+            info = _split(frame)
+            if info["mode"] == 1:
+                info["words"], info["words_digest"] = info["raw"].reshape(-1), info["digest"]
+            else:
+                _walk(info, stride, failed, beside)
+        except CodecError:
+            if not digests.result()[0]:
+                raise CodecError("frame checksum mismatch") from None
+            raise
+        own, info["frame_sha256"] = digests.result()
+        if not own:
+            raise CodecError("frame checksum mismatch")
+        if not isinstance(info["words_digest"], bytes):
+            info["words_digest"] = info["words_digest"].result()
+    return info
+
+
+def _walk(info, stride, failed, beside):
+    r, c = info["shape"]
+    words = info["words"] = np.empty(r * c, dtype="<u2")
+    progress = np.zeros(1, dtype=np.uint64)
+    states = offsets = None
+    if stride:
+        states, offsets = (np.empty(-(-words.size // stride), dtype=np.uint32) for _ in range(2))
+        info["main_states"], info["main_offsets"] = states, offsets
+    # (a thread hashes behind the walk; without one the hash follows it)
+    digest = beside.run(_sha_following, words, progress) if beside.pool is not None else None
+    streams = [np.frombuffer(s, dtype=np.uint8) if len(s) else np.zeros(1, np.uint8)
+               for s in (info["main_stream"], info["residual_stream"])]
+    p = lambda a, t: _native.ptr(a, t) if a is not None else ctypes.POINTER(t)()
+    status = -1
+    try:
+        status = _lib().grf_bctx_words(
+            p(streams[0], ctypes.c_uint8), len(info["main_stream"]), r, c, p(info["rows"], ctypes.c_uint8),
+            p(info["columns"], ctypes.c_uint8), info["nr"], info["nc"], p(info["main_freq"], ctypes.c_uint32), stride,
+            p(states, ctypes.c_uint32), p(offsets, ctypes.c_uint32), p(streams[1], ctypes.c_uint8),
+            len(info["residual_stream"]), p(info.get("residual_freq"), ctypes.c_uint32), p(words, ctypes.c_uint16),
+            p(progress, ctypes.c_uint64))
+    finally:
+        if status:  # whatever went wrong: nothing follows the walk any more
+            progress[0] = np.uint64(0xFFFFFFFFFFFFFFFF)
+    if status:
+        raise CodecError("invalid raw residual stream" if status == 33 else failed.format(status % 16))
+    info["words_digest"] = digest if digest is not None else hashlib.sha256(words).digest()
 
 
 def decode(frame):
     """Decode a complete frame on the host and verify the source checksum."""
-    info = parse(frame)
-    if info["mode"] == 1:
-        return info["raw"]
-    r, c = info["shape"]
-    nr, nc = info["nr"], info["nc"]
-    lib = _lib()
-    main = _decode_kind(lib, info["main_stream"], info["main_freq"].tobytes(), info["rows"], info["columns"],
-                        r, c, nr, nc, 0)
-    if info["mode"] == 128:
-        residual = _decode_kind(lib, info["residual_stream"], info["residual_freq"].tobytes(), info["rows"],
-                                info["columns"], r, c, nr, nc, 1, main)
-    else:
-        residual = _unpack6(lib, info["residual_stream"], r * c)
-    out = np.ascontiguousarray(recombine(main, residual).reshape(r, c))
-    if hashlib.sha256(out.tobytes()).digest() != info["digest"]:
+    if os.environ.get("GEOREFINE_CONTEXT_COMPACT_RANS") not in (None, "0", "1"):
+        raise CodecError("GEOREFINE_CONTEXT_COMPACT_RANS must be 0 or 1")
+    info = read_words(frame)
+    if info["words_digest"] != info["digest"]:
         raise CodecError("decoded checksum mismatch")
-    return out
+    return info["words"].reshape(info["shape"])

@@ -68,44 +68,40 @@ def index_frame(frame: bytes, stride: int = 1024, *, fused_segment=None, raw6_re
         raise base.CodecError("invalid checkpoint stride")
     if len(frame) < base.HEADER.size + 32:
         raise base.CodecError("invalid frame checksum/length")
-    info = base.parse(frame)
+    mode = base.HEADER.unpack_from(frame)[2]
+    repack = raw6_residual and mode == 128
+    fine = fused_segment if fused_segment and (mode == 0 or repack) else None
+    one_walk = fine is not None and stride % fine == 0  # every stride // fine-th entry of the fine index is the coarse one
+    info = base.read_words(frame, fine if one_walk else stride, "checkpoint validation failed ({})")
     r, c = info["shape"]
-    out = {"shape": (r, c), "mode": info["mode"], "nr": info["nr"], "nc": info["nc"], "stride": stride,
-           "source_sha256": info["digest"].hex(), "frame_sha256": hashlib.sha256(frame).hexdigest(),
-           "frame_bytes": len(frame)}
-    if info["mode"] == 1:
+    out = {"shape": (r, c), "mode": mode, "nr": info["nr"], "nc": info["nc"], "stride": stride,
+           "source_sha256": info["digest"].hex(), "frame_sha256": info["frame_sha256"], "frame_bytes": len(frame)}
+    if mode == 1:
         out["raw"] = info["raw"].reshape(-1).astype(np.uint16)
         out["resident_mode"] = 1
         return out
-    rows, columns, sf = info["rows"], info["columns"], info["main_freq"]
-    sy, rs = info["main_stream"], info["residual_stream"]
-    repack = raw6_residual and info["mode"] == 128
-    out["resident_mode"] = 0 if repack else info["mode"]
-    fine = fused_segment if (fused_segment and out["resident_mode"] == 0) else None
-    if fine and stride % fine == 0:
-        fs, fo, main = checkpoints(sy, sf, rows, columns, (r, c), info["nr"], info["nc"], fine)
-        states, offsets = fs[::stride // fine].copy(), fo[::stride // fine].copy()
-    else:
-        states, offsets, main = checkpoints(sy, sf, rows, columns, (r, c), info["nr"], info["nc"], stride)
-        if fine:
-            fs, fo, _ = checkpoints(sy, sf, rows, columns, (r, c), info["nr"], info["nc"], fine)
-    if fine:
-        out.update(fused_states=fs, fused_offsets=fo, fused_segment=fine)
-    out.update(rows=rows, columns=columns, main_freq=sf, main_stream=np.frombuffer(sy, dtype=np.uint8).copy(),
-               main_states=states, main_offsets=offsets, residual_stream=np.frombuffer(rs, dtype=np.uint8).copy())
-    if info["mode"] == 128:
-        rf = info["residual_freq"]
-        states, offsets, residual = checkpoints(rs, rf, rows, columns, (r, c), info["nr"], info["nc"],
-                                                r * c if repack else stride, main)
-        if not repack:
-            out.update(residual_freq=rf, residual_states=states, residual_offsets=offsets)
-    else:
-        residual = base._unpack6(base._lib(), rs, r * c)
-    words = base.recombine(main, residual)
-    if hashlib.sha256(words.tobytes()).digest() != info["digest"]:
+    if info["words_digest"] != info["digest"]:
         raise base.CodecError("indexed source checksum mismatch")
+    rows, columns, sf = info["rows"], info["columns"], info["main_freq"]
+    out["resident_mode"] = 0 if repack else mode
+    states, offsets = info["main_states"], info["main_offsets"]
+    if one_walk:
+        out.update(fused_states=states, fused_offsets=offsets, fused_segment=fine)
+        states, offsets = states[::stride // fine].copy(), offsets[::stride // fine].copy()
+    elif fine:
+        fs, fo, _ = checkpoints(info["main_stream"], sf, rows, columns, (r, c), info["nr"], info["nc"], fine)
+        out.update(fused_states=fs, fused_offsets=fo, fused_segment=fine)
+    residual = info["residual_stream"]
     if repack:
-        out["residual_stream"] = np.frombuffer(base._pack6(base._lib(), words), dtype=np.uint8).copy()
+        residual = base._pack6(base._lib(), info["words"])
+    elif mode == 128:
+        main = (info["words"] >> 5) & np.uint16(0x3FF)
+        rf = info["residual_freq"]
+        out.update(zip(("residual_freq", "residual_states", "residual_offsets"),
+                       (rf, *checkpoints(residual, rf, rows, columns, (r, c), info["nr"], info["nc"], stride, main)[:2])))
+    # (views of the frame: nothing here writes to the streams)
+    out.update(rows=rows, columns=columns, main_freq=sf, main_stream=np.frombuffer(info["main_stream"], dtype=np.uint8),
+               main_states=states, main_offsets=offsets, residual_stream=np.frombuffer(residual, dtype=np.uint8))
     return out
 
 
@@ -276,7 +272,8 @@ class HipContextTensor:
         self._raw6_segment, self._raw6_block = prepared["raw6_segment"], prepared["raw6_block"]
         for name, array in indexed.items():
             if isinstance(array, np.ndarray):
-                self.buffers[name] = torch.from_numpy(np.ascontiguousarray(array)).to(self.device)
+                array = np.ascontiguousarray(array) if array.flags.writeable else array.copy()  # (torch wants it writable)
+                self.buffers[name] = torch.from_numpy(array).to(self.device)
         for name in ("main", "residual"):
             if name + "_freq" in indexed:
                 cum = _tables.cumulative(indexed[name + "_freq"])

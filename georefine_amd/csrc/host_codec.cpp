@@ -20,6 +20,9 @@
 #include <cstring>
 #include <limits>
 #include <new>
+#include <system_error>
+#include <thread>
+#include <type_traits>
 #include <vector>
 
 namespace {
@@ -31,7 +34,7 @@ constexpr uint32_t kLow = 1u << 23;
 inline uint32_t main_symbol(uint16_t w) { return (w >> 5) & 0x3FFu; }
 inline uint32_t residual_symbol(uint16_t w) { return ((uint32_t)(w >> 15) << 5) | (w & 31u); }
 
-enum class Walk { ok, bad_context, dead_context, bad_symbol, overflow, overrun, bad_tail, bad_head };
+enum class Walk { ok, abandoned, bad_context, dead_context, bad_symbol, overflow, overrun, bad_tail, bad_head };
 
 // Validated frequency rows plus the lookup structures derived from them.
 //
@@ -203,9 +206,13 @@ bool walk_fast(const SymbolTables &t, const uint8_t *stream, ContextFn context, 
 // One forward pass over a stream, in runs: `context.run(i, most)` gives the length of the next run
 // (from symbol i, at most `most`) and `context.of(k)` the model row of its k-th symbol;
 // `mark(i, state, ip)` is called before symbol i where `mark.next()` says so.
-template <class Contexts, class Mark>
+struct NoProgress {
+  void reached(uint64_t) {}
+  bool wait_for(uint64_t) { return true; }
+};
+template <class Contexts, class Mark, class Progress = NoProgress>
 Walk walk_stream(const uint8_t *stream, size_t bytes, uint64_t n, const SymbolTables &t, Contexts contexts, Mark &mark,
-                 uint16_t *out) {
+                 uint16_t *out, Progress progress = Progress{}) {
   Position at{0, 4};
   if (!read_head(stream, bytes, at.state)) return Walk::bad_head;
   const bool in_range = contexts.in_range(t.nctx());
@@ -214,6 +221,7 @@ Walk walk_stream(const uint8_t *stream, size_t bytes, uint64_t n, const SymbolTa
     // (towards the stream's end shorter runs, so that only its last symbols are walked with every check)
     const size_t room = bytes - at.ip > 130 ? (bytes - at.ip - 2) / 2 : 64;
     const uint32_t count = contexts.run(i, (uint32_t)std::min<uint64_t>({n - i, mark.next() - i, room, 1u << 16}));
+    if (!progress.wait_for(i + count)) return Walk::abandoned;
     auto context = contexts.of();
     if (in_range && at.state < 0x80000000u && at.ip + 2 * (size_t)count + 2 <= bytes) {
       if (!walk_fast(t, stream, context, count, at, out + i)) return Walk::dead_context;
@@ -222,6 +230,7 @@ Walk walk_stream(const uint8_t *stream, size_t bytes, uint64_t n, const SymbolTa
       if (w != Walk::ok) return w;
     }
     i += count;
+    progress.reached(i);
   }
   return (at.ip == bytes && at.state == kLow) ? Walk::ok : Walk::bad_tail;
 }
@@ -365,6 +374,50 @@ bool encode_stream(uint64_t n, const uint32_t *freq, uint32_t nctx, uint32_t voc
   out[3] = (uint8_t)(state >> 24);
   std::reverse_copy(tail.begin(), tail.end(), out.begin() + 4);
   return true;
+}
+
+// How far a walk has got, published now and then for a thread that follows it.
+struct Counter {
+  uint64_t *at = nullptr;  // symbols done; kGaveUp once the walk has failed
+  uint64_t seen = 0;
+  static constexpr uint64_t kGaveUp = std::numeric_limits<uint64_t>::max();
+  void publish(uint64_t i) const { __atomic_store_n(at, i, __ATOMIC_RELEASE); }
+  // false: the walk that is followed failed
+  bool await(uint64_t i) {
+    for (uint32_t spins = 0; seen < i; ++spins) {
+      seen = __atomic_load_n(at, __ATOMIC_ACQUIRE);
+      if (seen >= i) break;
+      if (spins > 64) std::this_thread::yield();
+    }
+    return seen != kGaveUp;
+  }
+};
+
+// Contexts of a residual walk that follows the walk of the main symbols: `ctx` is written while it is read,
+// so its range is the main alphabet's, which the tables of that walk guarantee.
+struct FollowingContext : ArrayContext {
+  uint32_t step = 0;  // symbols it is allowed to ask for at once
+  uint32_t run(uint64_t i, uint32_t most) { return ArrayContext::run(i, std::min(most, step)); }
+  bool in_range(uint32_t nctx) const { return nctx >= 1024; }
+};
+
+// words[i] = main symbol on entry; the BF16 word of it and the i-th packed 6-bit field on return
+void join6(uint16_t *words, const uint8_t *packed, uint64_t lo, uint64_t hi) {  // lo: a multiple of four
+  auto word = [](uint32_t m, uint32_t r) { return (uint16_t)((m << 5) | (r & 31u) | ((r & 32u) << 10)); };
+  const uint8_t *q = packed + lo / 4 * 3;
+  uint64_t i = lo;
+  for (; i + 4 <= hi; i += 4, q += 3) {
+    const uint32_t v = (uint32_t)q[0] << 16 | (uint32_t)q[1] << 8 | q[2];
+    words[i] = word(words[i], v >> 18);
+    words[i + 1] = word(words[i + 1], (v >> 12) & 63);
+    words[i + 2] = word(words[i + 2], (v >> 6) & 63);
+    words[i + 3] = word(words[i + 3], v & 63);
+  }
+  for (uint32_t k = 0; i < hi; ++i, ++k) {  // the last one to three of a matrix
+    uint32_t r = 0;
+    for (uint32_t b = 0; b < 6; ++b) r = r << 1 | ((q[(6 * k + b) / 8] >> (7 - (6 * k + b) % 8)) & 1u);
+    words[i] = word(words[i], r);
+  }
 }
 
 struct BcxShape {
@@ -568,6 +621,165 @@ int bcx_checkpoint(const uint8_t *stream, size_t stream_bytes, uint64_t n, uint3
         return 0;
       },
       5, 6);
+}
+
+int grf_bctx_words(const uint8_t *stream, size_t stream_bytes, uint32_t rows, uint32_t cols, const uint8_t *rc,
+                   const uint8_t *cc, uint32_t nr, uint32_t nc, const uint32_t *freq, uint32_t stride, uint32_t *states,
+                   uint32_t *offsets, const uint8_t *residual, size_t residual_bytes, const uint32_t *residual_freq,
+                   uint16_t *words, uint64_t *progress) {
+  // Two chains: the main symbols, and what makes words of them -- the packed fields, or the
+  // conditional stream, whose contexts they are.  The second follows the first a few thousand
+  // symbols behind on a thread of its own (small matrices: afterwards), and `progress` tells a
+  // third, the caller's, how many words are done (to hash them meanwhile).
+  constexpr uint64_t kThreadFrom = 1u << 18, kStep = 1u << 13;
+  Counter main_done{}, words_done{progress};
+  uint64_t main_at = 0, own_at = 0;
+  if (!progress) words_done.at = &own_at;
+  main_done.at = &main_at;
+  const int status = guarded(
+      [&]() -> int {
+        if (!stream || !rc || !cc || !freq || !rows || !cols || !nr || !nc || nr > 64 || nc > 16 || !residual || !words ||
+            stream_bytes < 4 || stream_bytes > std::numeric_limits<uint32_t>::max() || (stride && (!states || !offsets)))
+          return 1;
+        if (std::any_of(rc, rc + rows, [&](uint8_t v) { return v >= nr; })) return 1;
+        if (std::any_of(cc, cc + cols, [&](uint8_t v) { return v >= nc; })) return 1;
+        const uint64_t n = (uint64_t)rows * cols;
+        if (!residual_freq) {
+          if (residual_bytes != (n * 6 + 7) / 8) return 33;
+          const unsigned tail_bits = (unsigned)(n * 6 % 8);
+          if (tail_bits && (residual[residual_bytes - 1] & ((1u << (8 - tail_bits)) - 1))) return 33;
+        }
+        SymbolTables main_tables, residual_tables;
+        if (main_tables.build(freq, nr * nc, 1024) != SymbolTables::Check::ok) return 2;
+        if (residual_freq && residual_tables.build(residual_freq, 1024, 64) != SymbolTables::Check::ok) return 18;
+        std::vector<uint16_t> fields(residual_freq ? (size_t)n : 0);
+
+        // the second chain; a failed walk before it ends it too
+        int second = 0;
+        auto follow = [&] {
+          Counter behind = main_done;
+          if (!residual_freq) {
+            for (uint64_t i = 0; i < n;) {
+              const uint64_t to = std::min(n, i + kStep);
+              if (!behind.await(to)) return words_done.publish(Counter::kGaveUp);
+              join6(words, residual, i, to);
+              words_done.publish(i = to);
+            }
+            return;
+          }
+          struct Behind {
+            Counter *main, *done;
+            uint16_t *words;
+            const uint16_t *fields;
+            uint64_t joined = 0, next = 0;
+            bool wait_for(uint64_t i) { return main->await(i); }
+            void reached(uint64_t i) {
+              for (; joined < i; ++joined) {
+                const uint32_t r = fields[joined];
+                words[joined] = (uint16_t)((words[joined] << 5) | (r & 31u) | ((r & 32u) << 10));
+              }
+              if (i >= next) done->publish(i), next = i + kStep;
+            }
+          };
+          NoMark unmarked;
+          FollowingContext contexts;
+          contexts.ctx = words;
+          contexts.n = n;
+          contexts.step = kStep;
+          Behind progress_behind{&behind, &words_done, words, fields.data()};
+          const Walk w = walk_stream(residual, residual_bytes, n, residual_tables, contexts, unmarked, fields.data(),
+                                     progress_behind);
+          second = w == Walk::ok || w == Walk::abandoned ? 0 : w == Walk::dead_context ? 18 : 19;
+          words_done.publish(w == Walk::ok ? n : Counter::kGaveUp);
+        };
+
+        struct Ahead {
+          Counter *done;
+          uint64_t next = 0;
+          bool wait_for(uint64_t) { return true; }
+          void reached(uint64_t i) {
+            if (i >= next) done->publish(i), next = i + kStep;
+          }
+        } ahead{&main_done};
+        std::thread other;
+        if (n >= kThreadFrom) try {
+            other = std::thread(follow);
+          } catch (const std::system_error &) {  // (no thread to be had: afterwards, then)
+          }
+        NoMark unmarked;
+        StrideMark marked{stride, states, offsets};
+        const GridContext grid{rc, cc, rows, cols, nc};
+        const Walk w = stride ? walk_stream(stream, stream_bytes, n, main_tables, grid, marked, words, ahead)
+                              : walk_stream(stream, stream_bytes, n, main_tables, grid, unmarked, words, ahead);
+        // (a stream that ends in the wrong place is found out after its last symbol)
+        main_done.publish(w == Walk::ok ? n : Counter::kGaveUp);
+        if (other.joinable()) other.join();
+        else follow();
+        if (w != Walk::ok) return w == Walk::dead_context || w == Walk::bad_context ? 2 : 3;
+        return second;
+      },
+      5, 6);
+  if (status) words_done.publish(Counter::kGaveUp);
+  return status;
+}
+
+int grf_sparse_tables(const uint32_t *freq, uint32_t nctx, uint32_t vocab, uint32_t shift, const uint32_t *image,
+                      uint32_t tabn, uint8_t *lut, uint64_t *tab) {
+  if (!freq || !image || !lut || !tab || !nctx || !vocab || shift > 16 || !tabn || tabn > 255) return 1;
+  const uint32_t nb = kTotal >> shift;
+  std::memset(lut, 0, (size_t)nctx * nb);
+  std::memset(tab, 0, (size_t)nctx * (tabn + 1) * 8);
+  std::vector<uint32_t> ends(tabn);
+  for (uint32_t c = 0; c < nctx; ++c) {
+    const uint32_t *f = freq + (size_t)c * vocab;
+    uint8_t *q = lut + (size_t)c * nb;
+    uint64_t *e = tab + (size_t)c * (tabn + 1);
+    uint32_t k = 0, start = 0;
+    for (uint32_t s = 0; s < vocab; ++s) {
+      if (!f[s]) continue;
+      if (k == tabn || f[s] > kTotal - start) return 2;
+      e[k] = (uint64_t)image[s] << 32 | (f[s] & 0xFFFFu) << 16 | start;
+      ends[k++] = start += f[s];
+    }
+    if (!k) continue;
+    if (start != kTotal) return 2;
+    uint32_t i = 0;
+    for (uint32_t b = 0; b < nb; ++b) {
+      const uint32_t lo = b << shift, hi = lo + (1u << shift);
+      while (ends[i] <= lo) ++i;
+      uint32_t best = i, most = std::min(ends[i], hi) - lo;
+      for (uint32_t j = i; ends[j] < hi; ++j) {  // the symbols that begin inside the bucket
+        const uint32_t held = std::min(ends[j + 1], hi) - ends[j];
+        if (held > most) best = j + 1, most = held;
+      }
+      q[b] = (uint8_t)best;
+    }
+  }
+  return 0;
+}
+
+int grf_order_records(const uint8_t *src, uint32_t rows, uint32_t spr, uint32_t per_segment, uint32_t record_bytes,
+                      uint32_t block, const uint32_t *position, uint32_t held, uint8_t *dst) {
+  if (!src || !dst || !position || !block || record_bytes % 4 || !record_bytes || record_bytes > 32) return 1;
+  for (uint32_t row = 0; row < rows; ++row)
+    if (position[row] >= held) return 1;
+  auto move = [&](auto size) {
+    constexpr size_t n = decltype(size)::value;
+    for (uint32_t row = 0; row < rows; ++row) {
+      const uint32_t q = position[row], within = q % block;
+      const uint8_t *from = src + (size_t)row * spr * per_segment * n;
+      for (uint32_t s = 0; s < spr; ++s)
+        for (uint32_t t = 0; t < per_segment; ++t, from += n)
+          std::memcpy(dst + ((((size_t)(q / block) * per_segment + t) * spr + s) * block + within) * n, from, n);
+    }
+  };
+  switch (record_bytes) {
+    case 12: move(std::integral_constant<size_t, 12>{}); break;
+    case 16: move(std::integral_constant<size_t, 16>{}); break;
+    case 20: move(std::integral_constant<size_t, 20>{}); break;
+    default: return 1;
+  }
+  return 0;
 }
 
 // 10-bit main symbols + 6-bit residuals -> BF16 words (no reference counterpart:

@@ -61,6 +61,27 @@ int bcx_checkpoint(const uint8_t *stream, size_t stream_bytes, uint64_t n, uint3
 /* Symbol pair -> BF16 word, the inverse of the split at GCR/bitexact_context_ans.cpp:9-12
  * (the reference does this step in numpy, GCR/bitexact_context_codec.py:426). 2 = symbol out of range. */
 int grf_bctx_join(const uint16_t *main_sym, const uint16_t *res_sym, uint64_t n, uint16_t *out);
+/* A whole frame's words at once (no single reference counterpart: bcx_checkpoint / bcx_decode of both streams
+ * and the recombination): the main stream walked, its index recorded before every stride-th symbol (stride 0:
+ * none), and the words made of its symbols and the packed 6-bit fields (residual_freq null) or the conditional
+ * stream.  `progress` (may be null) counts finished words while the call runs, for a thread that consumes them;
+ * it ends as all ones when the call fails.  1 arguments, 2 main tables/contexts, 3 main stream, 18/19 the
+ * same of the conditional stream, 33 packed fields, 5/6 internal; states/offsets/words hold no result then. */
+int grf_bctx_words(const uint8_t *stream, size_t stream_bytes, uint32_t rows, uint32_t cols, const uint8_t *rc,
+                   const uint8_t *cc, uint32_t nr, uint32_t nc, const uint32_t *freq, uint32_t stride, uint32_t *states,
+                   uint32_t *offsets, const uint8_t *residual, size_t residual_bytes, const uint32_t *residual_freq,
+                   uint16_t *words, uint64_t *progress);
+/* The fused kernels' lookup tables of a frame (no reference counterpart): per context `tabn + 1` entries
+ * start | (freq & 0xFFFF) << 16 | image[symbol] << 32 of the symbols that occur (unused ones 0) and, per bucket of
+ * 2^shift slots, the index of the entry that owns most of the bucket (the first of them on a tie).  2: a
+ * context holds more than tabn symbols, or its frequencies are neither none nor 65536 in all. */
+int grf_sparse_tables(const uint32_t *freq, uint32_t nctx, uint32_t vocab, uint32_t shift, const uint32_t *image,
+                      uint32_t tabn, uint8_t *lut, uint64_t *tab);
+/* Fixed-size records of a matrix (per_segment of record_bytes each in every one of a row's spr segments) from the
+ * frame's order to the resident one: record t of segment s of the row at position q goes to
+ * (((q / block * per_segment + t) * spr + s) * block + q % block).  dst holds `held` rows. */
+int grf_order_records(const uint8_t *src, uint32_t rows, uint32_t spr, uint32_t per_segment, uint32_t record_bytes,
+                      uint32_t block, const uint32_t *position, uint32_t held, uint8_t *dst);
 /* GCR/bitexact_predictive_ans.cpp:10-12  generic context coder of the predictive frames */
 int p_encode(const uint16_t *v, const uint16_t *cx, uint64_t n, uint32_t nc, uint32_t vocab, uint32_t **freq,
              uint8_t **stream, size_t *stream_n);
