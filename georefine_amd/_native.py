@@ -113,6 +113,10 @@ def codec():
             L.grf_bctx_words.argtypes = [U8P, _sz, _u32, _u32, U8P, U8P, _u32, _u32, U32P, _u32, U32P, U32P, U8P, _sz, U32P,
                                          U16P, ctypes.POINTER(_u64)]
             L.grf_bctx_words.restype = _int
+            L.grf_bctx_encode.argtypes = [U16P, _u32, _u32, U8P, U8P, _u32, _u32, _u32, U32P, U8P, _sz, ctypes.POINTER(_sz)]
+            L.grf_bctx_encode.restype = _int
+            L.grf_bctx_sums.argtypes = [U16P, _u32, _u32, ctypes.POINTER(_u64), ctypes.POINTER(_u64)]
+            L.grf_bctx_sums.restype = _int
             L.grf_sparse_tables.argtypes = [U32P, _u32, _u32, _u32, U32P, _u32, U8P, ctypes.POINTER(_u64)]
             L.grf_sparse_tables.restype = _int
             L.grf_order_records.argtypes = [U8P, _u32, _u32, _u32, _u32, _u32, U32P, _u32, U8P]
