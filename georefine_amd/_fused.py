@@ -140,11 +140,12 @@ def piece_capacity(offsets, rows, spr, p):
 def quad_piece_capacity(offsets, rows, spr):
     """LDS bytes of a GEMM wave's row piece: four consecutive segments of a row from any first
     segment (fewer at the row's end), from the 16-byte aligned start, plus the refill's window."""
-    off = offsets[:-1].reshape(rows, spr).astype(np.int64)
-    end_of_row = np.concatenate((off[1:, 0], [int(offsets[-1])]))
-    ends = np.concatenate((off, end_of_row[:, None]), axis=1)  # ends[:, s] = start of segment s, [:, spr] = row end
-    last = np.minimum(np.arange(spr) + 4, spr)
-    longest = int((ends[:, last] - (off & ~15)).max())
+    off = offsets[:-1].reshape(rows, spr)
+    end_of_row = np.concatenate((off[1:, :1], offsets[-1:, None]))
+    aligned = off & off.dtype.type(0xFFFFFFF0)
+    whole = max(0, spr - 4)  # first segments that have four and a further one behind them
+    longest = int((off[:, 4:] - aligned[:, :whole]).max()) if whole else 0
+    longest = max(longest, int((end_of_row - aligned[:, whole:]).max()))
     return (longest + WINDOW + 15) // 16 * 16
 
 

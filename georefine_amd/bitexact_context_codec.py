@@ -88,24 +88,24 @@ def _u8(a):
     return np.ascontiguousarray(a, dtype=np.uint8)
 
 
-def _encode_stream(lib, a, rc, cc, nr, nc, kind):
-    """(frequency rows as bytes, the stream as a view of the buffer it was written to)."""
-    vocab, nctx = _shape_of(kind, nr, nc)
-    freq = np.zeros(nctx * vocab, dtype="<u4")
+def _encode_stream(lib, a, rc, cc, nr, nc, kind, freq):
+    """The stream of one kind with the given frequency rows (bytes), as a view of the buffer it
+    was written to."""
     rc, cc = _u8(rc), _u8(cc)
+    rows = np.frombuffer(freq, dtype="<u4")
     buffer, begin = np.empty(2 * a.size + 8, dtype=np.uint8), ctypes.c_size_t()
     status = lib.grf_bctx_encode(_native.ptr(a, ctypes.c_uint16), a.shape[0], a.shape[1],
                                  _native.ptr(rc, ctypes.c_uint8), _native.ptr(cc, ctypes.c_uint8), nr, nc, kind,
-                                 _native.ptr(freq, ctypes.c_uint32), _native.ptr(buffer, ctypes.c_uint8), buffer.size,
+                                 _native.ptr(rows, ctypes.c_uint32), _native.ptr(buffer, ctypes.c_uint8), buffer.size,
                                  ctypes.byref(begin))
     if status:
         raise CodecError(f"rANS encode failed ({status})")
-    return freq.tobytes(), memoryview(buffer)[begin.value:]
+    return memoryview(buffer)[begin.value:]
 
 
 def _encode_kind(lib, a, rc, cc, nr, nc, kind):
-    freq, stream = _encode_stream(lib, a, rc, cc, nr, nc, kind)
-    return freq, bytes(stream)
+    freq = _frequencies_kind(lib, a, rc, cc, nr, nc, kind)
+    return freq, bytes(_encode_stream(lib, a, rc, cc, nr, nc, kind, freq))
 
 
 def _frequencies_kind(lib, a, rc, cc, nr, nc, kind):
@@ -221,28 +221,30 @@ def encode(words, *, row_classes=16, col_classes=4, residual="auto"):
     raw = memoryview(a).cast("B")
     none = np.zeros(max(r, c), dtype=np.uint8)  # (the conditional stream's contexts are not the classes)
 
-    def conditional():
-        return _encode_stream(lib, a, none[:r], none[:c], row_classes, col_classes, 1)
+    classes = row_classes, col_classes
 
-    with Beside(len(raw), workers=2) as beside:
-        res = beside.run(conditional) if residual == "auto" else None
+    with Beside(len(raw), workers=3) as beside:
+        if residual == "auto":
+            res_freq = beside.run(_frequencies_kind, lib, a, none[:r], none[:c], *classes, 1)
+            res_stream = beside.run(lambda: _encode_stream(lib, a, none[:r], none[:c], *classes, 1, res_freq.result()))
         sha = beside.run(lambda: hashlib.sha256(raw).digest())
-        packed = beside.run(_pack6, lib, a)  # (behind the hash, beside the streams)
-        rc, cc = _labels(a, row_classes, col_classes)
+        rc, cc = _labels(a, *classes)
+        main_freq = _frequencies_kind(lib, a, rc, cc, *classes, 0)
+        table = beside.run(zlib.compress, main_freq, 6)
+        if residual == "auto":
+            both = beside.run(lambda: zlib.compress(main_freq + res_freq.result(), 6))
+        packed = beside.run(_pack6, lib, a)
         meta = zlib.compress(rc.tobytes() + cc.tobytes(), 6)
-        main_freq, main_stream = _encode_stream(lib, a, rc, cc, row_classes, col_classes, 0)
-        table = zlib.compress(main_freq, 6)
-        dig = sha.result()
+        main_stream = _encode_stream(lib, a, rc, cc, *classes, 0, main_freq)
+        dig, table, packed = sha.result(), table.result(), packed.result()
         fixed = HEADER.size + len(meta) + len(main_stream) + 32
-        packed = packed.result()
         size = fixed + len(table) + len(packed)
-        if res is not None:
-            res_freq, res_stream = res.result()
-            both = zlib.compress(main_freq + res_freq, 6)
+        if residual == "auto":
+            both, res_stream = both.result(), res_stream.result()
             conditional_size = fixed + len(both) + len(res_stream)
-    if min(size, conditional_size if res is not None else size) >= HEADER.size + len(raw) + 32:
+    if min(size, conditional_size if residual == "auto" else size) >= HEADER.size + len(raw) + 32:
         return _sealed(_sections(1, row_classes, col_classes, r, c, b"", b"", b"", b"", raw, dig))
-    if res is not None and conditional_size < size:
+    if residual == "auto" and conditional_size < size:
         return _sealed(_sections(128, row_classes, col_classes, r, c, meta, both, main_stream, res_stream, b"", dig))
     return _sealed(_sections(0, row_classes, col_classes, r, c, meta, table, main_stream, packed, b"", dig))
 

@@ -503,11 +503,10 @@ void bcx_count_and_normalize(const uint16_t *w, uint32_t rows, uint32_t cols, co
   }
 }
 
-// count, normalise and encode one symbol stream into [begin, end); its first byte, or null
+// one symbol stream with the frequencies bcx_count_and_normalize gives, into [begin, end); its first byte, or null
 uint8_t *bcx_encode_stream(const uint16_t *w, uint32_t rows, uint32_t cols, const uint8_t *rc, const uint8_t *cc, uint32_t nr,
-                           uint32_t nc, uint32_t kind, uint32_t *freq, uint8_t *begin, uint8_t *end) {
+                           uint32_t nc, uint32_t kind, const uint32_t *freq, uint8_t *begin, uint8_t *end) {
   const BcxShape sh = bcx_shape(kind, nr, nc);
-  bcx_count_and_normalize(w, rows, cols, rc, cc, nc, kind, sh, freq);
   const std::vector<EncodeCell> cells = encode_cells(freq, sh.nctx, sh.vocab);
   const EncodeCell *e = cells.data();
   const uint64_t n = (uint64_t)rows * cols;
@@ -569,6 +568,7 @@ int bcx_encode(const uint16_t *w, uint64_t n, uint32_t rows, uint32_t cols, cons
         if (!w || !rc || !cc || !freq || !stream || !stream_n || n != (uint64_t)rows * cols) return 1;
         const std::unique_ptr<uint8_t[]> bytes(new uint8_t[2 * n + 8]);
         uint8_t *end = bytes.get() + 2 * n + 8;
+        bcx_count_and_normalize(w, rows, cols, rc, cc, nc, kind, bcx_shape(kind, nr, nc), freq);
         const uint8_t *at = bcx_encode_stream(w, rows, cols, rc, cc, nr, nc, kind, freq, bytes.get(), end);
         if (!at) return 3;
         auto *p = (uint8_t *)std::malloc((size_t)(end - at));
@@ -582,7 +582,7 @@ int bcx_encode(const uint16_t *w, uint64_t n, uint32_t rows, uint32_t cols, cons
 }
 
 int grf_bctx_encode(const uint16_t *w, uint32_t rows, uint32_t cols, const uint8_t *rc, const uint8_t *cc, uint32_t nr,
-                    uint32_t nc, uint32_t kind, uint32_t *freq, uint8_t *buffer, size_t buffer_bytes, size_t *begin) {
+                    uint32_t nc, uint32_t kind, const uint32_t *freq, uint8_t *buffer, size_t buffer_bytes, size_t *begin) {
   return guarded(
       [&]() -> int {
         if (!w || !rc || !cc || !freq || !buffer || !begin || !rows || !cols) return 1;

@@ -82,9 +82,11 @@ int grf_sparse_tables(const uint32_t *freq, uint32_t nctx, uint32_t vocab, uint3
  * (((q / block * per_segment + t) * spr + s) * block + q % block).  dst holds `held` rows. */
 int grf_order_records(const uint8_t *src, uint32_t rows, uint32_t spr, uint32_t per_segment, uint32_t record_bytes,
                       uint32_t block, const uint32_t *position, uint32_t held, uint8_t *dst);
-/* bcx_encode into the caller's buffer of at least 2 n + 8 bytes: the stream is buffer[*begin .. buffer_bytes). */
+/* The stream bcx_encode writes, given the frequencies of bcx_frequencies, in the caller's buffer of at least
+ * 2 n + 8 bytes: the stream is buffer[*begin .. buffer_bytes). */
 int grf_bctx_encode(const uint16_t *w, uint32_t rows, uint32_t cols, const uint8_t *rc, const uint8_t *cc, uint32_t nr,
-                    uint32_t nc, uint32_t kind, uint32_t *freq, uint8_t *buffer, size_t buffer_bytes, size_t *begin);
+                    uint32_t nc, uint32_t kind, const uint32_t *freq, uint8_t *buffer, size_t buffer_bytes,
+                    size_t *begin);
 /* sums of the words' magnitude bits (w & 0x7FFF) over every row and column: what the class labels rank
  * (GCR/bitexact_context_codec.py:183-203) */
 int grf_bctx_sums(const uint16_t *w, uint32_t rows, uint32_t cols, uint64_t *row_sum, uint64_t *col_sum);
