@@ -282,7 +282,11 @@ def choose_wave_tiling(spr, class_rows, piece_cap_fn, lds_fn, cus=256, seg_len=6
         n_slabs = -(-spr // p)
         cap = piece_cap_fn(p)
         unit_steps = seg_len + WAVE_UNIT_OVERHEAD + WAVE_PIECE_OVERHEAD * rpw
-        for threads in (1024, 768, 512):
+        # (768 threads, two workgroups a compute unit, where the LDS allows: a matrix with a few long
+        # rows needs larger pieces, and one wave less per workgroup then keeps two of them resident --
+        # 17408 x 5120 with pieces of 912 bytes: 68.7 us with 11 waves against 95.0 with 12 and
+        # tiles cut down to 8 rows)
+        for threads in (1024, 768, 704, 640, 576, 512):
             nwaves = threads // 64
             for r in range(rpw, 129, rpw):
                 lds = lds_fn(threads, p, r, n_slabs, cap)
