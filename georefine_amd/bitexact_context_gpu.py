@@ -320,7 +320,7 @@ class HipContextTensor:
             self.fused_reason = ""
             try:
                 self._tiling(1)
-                self._tiling(0)
+                self._store_tiling()
             except _fused.FusedUnsupported as exc:
                 self.fused, self.fused_reason = None, str(exc)
                 return
@@ -399,6 +399,11 @@ class HipContextTensor:
             self.resident_bytes += rows.numel() * 4 + classes.numel()
         return self._tilings[bucket]
 
+    def _store_tiling(self):
+        """The tiling decode() uses: the GEMV's wave units (their blocks of rows are the blocks of
+        the resident residual order); the slab tiling of the store sink only with the slab GEMV."""
+        return self._tiling(1 if GEMV_WAVES else 0)
+
     # ------------------------------------------------------------------ decode
     def _decode_blocks(self, blocks=None, *, check=True):
         import torch
@@ -446,7 +451,7 @@ class HipContextTensor:
         out = torch.empty(self.n, device=self.device, dtype=torch.uint16)
         if check:  # between checks the word keeps what earlier launches reported
             self.error.zero_()
-        self._launch(self._lib.grf_bctx_fused_decode, ctypes.byref(self.fused), ctypes.byref(self._tiling(0)[0]),
+        self._launch(self._lib.grf_bctx_fused_decode, ctypes.byref(self.fused), ctypes.byref(self._store_tiling()[0]),
                      out.data_ptr(), self.error.data_ptr())
         self._check(check)
         return out.view(torch.bfloat16).reshape(self.shape)

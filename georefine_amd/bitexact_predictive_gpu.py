@@ -283,7 +283,7 @@ class HipPredictiveTensor:
         f.raw_interleaved = self._raw5_block if self._raw5_segment else 0
         f.row_pos = b["row_pos"].data_ptr() if self._raw5_segment else None
         self.fused = f
-        store = self._tiling_for(0)
+        store = self._tiling_for("waves")
         self.fused_plan = dict(sc, **store[3])
 
     def index_slot(self, row, segment):
@@ -443,7 +443,7 @@ class HipPredictiveTensor:
                 bins, status = self._contexts(reference_bf16_device)
                 if not status:
                     status = self._lib.grf_ppcx_fused_decode(ctypes.byref(self.fused),
-                                                             ctypes.byref(self._tiling_for(0)[0]), bins.data_ptr(),
+                                                             ctypes.byref(self._tiling_for("waves")[0]), bins.data_ptr(),
                                                              out.data_ptr(), self.error.data_ptr(),
                                                              torch.cuda.current_stream(self.device).cuda_stream)
             self._status(status, check)

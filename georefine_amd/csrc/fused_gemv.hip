@@ -20,7 +20,7 @@ int check_fused_frame(const grf_bctx_fused &f, const grf_fused_tiling &g, const 
     if (g.scheme != GRF_TILE_WAVES) return bad("the GEMM takes a wave tiling (piece_cap for pieces of four segments)");
     if (!g.lanes_per_row || !g.rows_per_tile) return bad("empty tile");
   } else if (g.scheme == GRF_TILE_WAVES) {
-    if (use != kGemvTiling) return bad("this entry point takes slab tilings only");
+    if (use != kGemvTiling && use != kStoreTiling) return bad("this entry point takes slab tilings only");
     const uint32_t lanes = g.lanes_per_row;
     if (lanes < 4 || lanes > 64 || (lanes & (lanes - 1))) return bad("a wave unit has 4, 8, 16, 32 or 64 lanes per row");
     if (!g.rows_per_tile) return bad("empty tile");
@@ -124,7 +124,7 @@ int validate_fused_host(const grf_bctx_fused &f, const grf_fused_tiling &g, Tili
   }
   uint32_t lds = 0;
   if (use == kGemmTiling) lds = GemmLdsLayout(f, g).total;
-  else if (g.scheme == GRF_TILE_WAVES) lds = WaveLdsLayout(f, g, kWaveRowsPerPass).total;
+  else if (g.scheme == GRF_TILE_WAVES) lds = WaveLdsLayout(f, g, use == kStoreTiling ? 0 : kWaveRowsPerPass).total;
   else lds = FusedLdsLayout(f, g, use == kGemvTiling ? 1 : 0).total;
   if (lds > 160 * 1024) return bad("the launch needs " + std::to_string(lds) + " bytes of LDS");
   return GRF_OK;
@@ -146,7 +146,10 @@ int grf_bctx_fused_validate_host(const grf_bctx_fused *frame, const grf_fused_ti
   if (!frame || !tiling) return grf::set_error(GRF_BAD_ARGUMENT, "grf_bctx_fused_validate_host: null argument");
   if (use < 0 || use > 3) return grf::set_error(GRF_BAD_ARGUMENT, "grf_bctx_fused_validate_host: use is 0, 1, 2 or 3");
   try {
-    const grf::TilingUse kind = use == 1 ? grf::kGemvTiling : use == 2 ? grf::kGemmTiling : grf::kSlabTiling;
+    const grf::TilingUse kind = use == 0   ? grf::kStoreTiling
+                                : use == 1 ? grf::kGemvTiling
+                                : use == 2 ? grf::kGemmTiling
+                                           : grf::kSlabTiling;
     return grf::validate_fused_host(*frame, *tiling, kind, use != 3, seg_offset, tile_rows, tile_class, row_class,
                                     row_pos);
   } catch (...) {
@@ -168,7 +171,10 @@ int grf_bctx_fused_decode(const grf_bctx_fused *frame, const grf_fused_tiling *t
                           int32_t *error, void *hip_stream) {
   if (!frame || !tiling || !out || !error)
     return grf::set_error(GRF_BAD_ARGUMENT, "grf_bctx_fused_decode: null argument");
-  if (int rc = grf::check_fused_frame(*frame, *tiling, "grf_bctx_fused_decode")) return rc;
+  if (int rc = grf::check_fused_frame(*frame, *tiling, "grf_bctx_fused_decode", grf::kStoreTiling)) return rc;
+  if (((uintptr_t)out & 15)) return grf::set_error(GRF_BAD_ARGUMENT, "grf_bctx_fused_decode: out must be 16-byte aligned");
+  if (tiling->scheme == GRF_TILE_WAVES)
+    return grf::launch_wave_store<grf::SegmentWalk>(*frame, *tiling, out, error, (hipStream_t)hip_stream);
   if (grf::reads_ahead(*frame))
     return grf::launch_walk<grf::SegmentWalkAhead, 1, grf::kStore>(*frame, *tiling, nullptr, 0, nullptr, 0, nullptr,
                                                                    out, error, (hipStream_t)hip_stream);

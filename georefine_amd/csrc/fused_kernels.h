@@ -40,7 +40,7 @@
 namespace grf {
 int set_error(int code, const std::string &what);                                          // decode_general.hip
 // fused_gemv.hip; wave_units: the entry point takes GRF_TILE_WAVES tilings
-enum TilingUse { kSlabTiling, kGemvTiling, kGemmTiling };  // what an entry point does with the tiling it is given
+enum TilingUse { kSlabTiling, kGemvTiling, kGemmTiling, kStoreTiling };  // what an entry point does with the tiling it is given
 // pointers: also refuse null device pointers (a host-side validation has none to give)
 int check_fused_frame(const grf_bctx_fused &f, const grf_fused_tiling &g, const char *who, TilingUse use = kSlabTiling,
                       bool pointers = true);
@@ -304,10 +304,116 @@ __device__ __forceinline__ float group_sum_to_first_lane(float v, uint32_t logp)
   return v;
 }
 
-template <class Walk, int M, int SCAN>
+// A lane that decodes 32 columns holds 64 bytes of the output, four 16-byte units, and its
+// neighbours hold the runs next to it: stored as they are, every instruction of a wave touches 64
+// lines with 16 bytes each, the second-level cache takes four times the write requests, and lines
+// leave it half written.  So the four lanes of a quad exchange units first (two butterfly stages
+// of lane permutes, one or two instructions a column): afterwards lane j holds unit j of all four
+// runs, and one store of a quad writes 64 bytes in a row.
+// u[unit][dword]: on return u[k] of lane j is what lane k of the quad held in u[j].
+__device__ __forceinline__ void transpose_quad(uint32_t (&u)[4][4], uint32_t lane) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  auto moved = [](uint32_t v, auto ctrl) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, decltype(ctrl)::value, 0xF, 0xF, false);
+  };
+  const bool odd = lane & 1, high = lane & 2;
+#pragma unroll
+  for (int i = 0; i < 4; i += 2)
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+      const uint32_t a = u[i][d], b = u[i + 1][d];
+      const uint32_t from_b = moved(b, std::integral_constant<int, 0xB1>{}), from_a = moved(a, std::integral_constant<int, 0xB1>{});
+      u[i][d] = odd ? from_b : a;
+      u[i + 1][d] = odd ? b : from_a;
+    }
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+      const uint32_t a = u[i][d], b = u[i + 2][d];
+      const uint32_t from_b = moved(b, std::integral_constant<int, 0x4E>{}), from_a = moved(a, std::integral_constant<int, 0x4E>{});
+      u[i][d] = high ? from_b : a;
+      u[i + 2][d] = high ? b : from_a;
+    }
+#else
+  (void)u, (void)lane;
+#endif
+}
+
+// Keeps four finished pairs of words in four registers: left alone, the compiler puts the merge of
+// symbols and residuals off to where the words are used, and what they are merged from takes
+// three times the registers meanwhile (and was spilled in the loop).
+__device__ __forceinline__ void pin_words(uint32_t (&v)[4]) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]));
+#else
+  (void)v;
+#endif
+}
+
+// The walk of a unit whose words go to the dense matrix; every lane of the wave takes part (the
+// exchange above reads all of a quad's lanes), those without a segment (`walks` false) store nothing.
+// first: the segment's first word in the output.  S is a multiple of 16.
+template <class Walk, int SCAN>
+__device__ __forceinline__ void store_segment(Walk &w, const grf::FusedParams &q, uint32_t S, bool walks, uint32_t first,
+                                              uint16_t *out, uint32_t lane) {
+  constexpr uint32_t kNowhere = 0xFFFFFFFFu;
+  if (S % 32) {  // segments of 16 words: a lane's 32 bytes, next to its neighbours'
+    for (uint32_t t = 0; walks && t < S; t += 16) {
+      uint32_t pair[8];
+      w.begin16(t, S);
+      w.template half<0, SCAN>(q, reinterpret_cast<uint32_t(&)[4]>(pair[0]));
+      w.template half<1, SCAN>(q, reinterpret_cast<uint32_t(&)[4]>(pair[4]));
+      uint4 *dst = reinterpret_cast<uint4 *>(out + ((size_t)first + t));
+      dst[0] = make_uint4(pair[0], pair[1], pair[2], pair[3]);
+      dst[1] = make_uint4(pair[4], pair[5], pair[6], pair[7]);
+    }
+    return;
+  }
+  uint32_t unit = walks ? first / 8 : kNowhere;  // in 16-byte units: fits 32 bits (rows are multiples of 16 words)
+  if (walks) w.begin16(0, S);
+  for (uint32_t t = 0; t < S; t += 32) {
+    uint32_t u[4][4];
+    if (walks) {
+      w.template half<0, SCAN>(q, u[0]);
+      pin_words(u[0]);
+      w.template half<1, SCAN>(q, u[1]);
+      pin_words(u[1]);
+      w.begin16(t + 16, S);
+      w.template half<0, SCAN>(q, u[2]);
+      pin_words(u[2]);
+      w.template half<1, SCAN>(q, u[3]);
+      pin_words(u[3]);
+      // (the next group's loads leave before the stores: memory operations complete in order, so a
+      // wait for a load that followed them would wait for them too)
+      if (t + 32 < S) w.begin16(t + 32, S);
+    }
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+v"(unit));  // (the quad's places are told again at every flush: no registers over the walk)
+#endif
+    transpose_quad(u, lane);
+    auto flush = [&](auto k, const uint32_t (&v)[4]) {
+#if defined(__HIP_DEVICE_COMPILE__)
+      const uint32_t at = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)unit, 0x55 * decltype(k)::value, 0xF, 0xF, false);
+#else
+      const uint32_t at = unit;
+#endif
+      if (at != kNowhere)
+        reinterpret_cast<uint4 *>(out)[(size_t)at + t / 8 + (lane & 3)] = make_uint4(v[0], v[1], v[2], v[3]);
+    };
+    flush(std::integral_constant<int, 0>{}, u[0]);
+    flush(std::integral_constant<int, 1>{}, u[1]);
+    flush(std::integral_constant<int, 2>{}, u[2]);
+    flush(std::integral_constant<int, 3>{}, u[3]);
+  }
+}
+
+// SINK kDot: products with M activation rows; kStore: the words to `out` (M = 0).
+template <class Walk, int M, int SCAN, int SINK = kDot>
 __device__ __forceinline__ void fused_wave_body(uint8_t *lds, const grf_bctx_fused &f, const grf_fused_tiling &g,
                                                 const uint16_t *x, uint32_t ldx, uint16_t *y, uint32_t ldy,
-                                                const uint16_t *bias, int32_t *error, uint32_t tile) {
+                                                const uint16_t *bias, int32_t *error, uint32_t tile,
+                                                uint16_t *out = nullptr) {
   const WaveLdsLayout L(f, g, M);
   const uint32_t tid = threadIdx.x, nthreads = blockDim.x;
   const uint32_t lane = tid % 64, nwaves = nthreads / 64;
@@ -349,7 +455,7 @@ __device__ __forceinline__ void fused_wave_body(uint8_t *lds, const grf_bctx_fus
     if (has) r_real = i0 + 64 - (uint32_t)__builtin_clzll(has);
   }
   const uint32_t groups = (r_real + rpw - 1) / rpw, units = groups * g.n_slabs;
-  const bool by_slab = K * 2u * M > kUnitsBySlabBytes;
+  const bool by_slab = SINK == kDot && K * 2u * M > kUnitsBySlabBytes;
   const uint32_t n_minor = max(1u, by_slab ? groups : g.n_slabs);
   const uint32_t step_major = nwaves / n_minor, step_minor = nwaves % n_minor;
   uint32_t bad = 0;
@@ -442,20 +548,26 @@ __device__ __forceinline__ void fused_wave_body(uint8_t *lds, const grf_bctx_fus
       default: __builtin_amdgcn_s_setprio(3); break;
     }
 #endif
-    float acc[M];
+    if constexpr (SINK == kStore) {
+      store_segment<Walk, SCAN>(w, q, S, walks, walks ? mul24(row, K) + col0 : 0, out, lane);
+      if (walks && !w.ended_on_checkpoint(f)) bad |= GRF_ERR_CHECKPOINT;
+      continue;
+    }
+    float acc[M > 0 ? M : 1];
 #pragma unroll
     for (int m = 0; m < M; ++m) acc[m] = 0.f;
-    if (walks) {
+    if (SINK == kDot && walks) {
       // The activations are read eight columns (16 bytes per row) at a time, each load issued
       // while the eight symbols before it are decoded: two register sets, one for the first and
       // one for the second half of a group of 16, so nothing is copied between them.
-      uint4 xa[M], xb[M];
-      auto load_x = [&](uint4 (&xs)[M], uint32_t t) {  // (uniform base, 32-bit lane offset in bytes)
+      constexpr int MX = M > 0 ? M : 1;
+      uint4 xa[MX], xb[MX];
+      auto load_x = [&](uint4 (&xs)[MX], uint32_t t) {  // (uniform base, 32-bit lane offset in bytes)
 #pragma unroll
         for (int m = 0; m < M; ++m)
           xs[m] = *reinterpret_cast<const uint4 *>(reinterpret_cast<const uint8_t *>(x) + ((uint32_t)m * ldx + col0 + t) * 2u);
       };
-      auto contract = [&](const uint32_t (&pair)[4], const uint4 (&xs)[M]) {
+      auto contract = [&](const uint32_t (&pair)[4], const uint4 (&xs)[MX]) {
 #pragma unroll
         for (int m = 0; m < M; ++m) {
           acc[m] = dot2_bf16(pair[0], xs[m].x, acc[m]);
@@ -503,6 +615,10 @@ __device__ __forceinline__ void fused_wave_body(uint8_t *lds, const grf_bctx_fus
       }
     }
   }
+  if constexpr (SINK == kStore) {
+    if (bad) atomicOr(error, (int)bad);
+    return;
+  }
   __syncthreads();
   // A row's unit sums -> its output.  The order is the same for every tiling: the tree that a
   // unit began over its P segments is carried on over aligned blocks of 64 segments (64 / P
@@ -543,6 +659,37 @@ __global__ __launch_bounds__(grf::kFusedMaxThreads) __attribute__((amdgpu_waves_
     const uint16_t *bias, int32_t *error) {
   extern __shared__ __align__(16) uint8_t lds[];
   fused_wave_body<Walk, M, SCAN>(lds, f, g, x, ldx, y, ldy, bias, error, blockIdx.x);
+}
+
+// The store sink over wave units (decode()).  Bound by the walk (VALU issue, as the GEMV) and the
+// traffic behind it together: 17408 x 5120 takes 98.6 us where the walk alone takes 70 and its 307 MB
+// at the rate of a large copy 59; slab tilings with 64-byte runs stored by the lanes that decoded
+// them took 148.  Output held back to whole 128-byte lines (88 registers, 16 waves a compute unit)
+// measured the same (93-98 us), streaming stores 2 % more.
+template <class Walk, int SCAN>
+__global__ __launch_bounds__(grf::kFusedMaxThreads) __attribute__((amdgpu_waves_per_eu(6))) void fused_wave_store_kernel(
+    grf_bctx_fused f, grf_fused_tiling g, uint16_t *out, int32_t *error) {
+  extern __shared__ __align__(16) uint8_t lds[];
+  fused_wave_body<Walk, 0, SCAN, kStore>(lds, f, g, nullptr, 0, nullptr, 0, nullptr, error, blockIdx.x, out);
+}
+
+template <class Walk>
+int launch_wave_store(const grf_bctx_fused &f, const grf_fused_tiling &g, uint16_t *out, int32_t *error, hipStream_t s) {
+  const WaveLdsLayout L(f, g, 0);
+  if (L.total > 160 * 1024) return grf::set_error(GRF_UNSUPPORTED, "fused decode: LDS demand exceeds 160 KiB");
+  auto launch = [&](auto scan) -> int {
+    constexpr auto kernel = &fused_wave_store_kernel<Walk, decltype(scan)::value>;
+    if (L.total > 64 * 1024)
+      if (int rc = allow_full_lds<kernel>()) return rc;
+    hipLaunchKernelGGL(kernel, dim3(g.n_tiles), dim3(g.threads), L.total, s, f, g, out, error);
+    return GRF_OK;
+  };
+  if (int rc = f.whole_range ? launch(std::integral_constant<int, grf::kScanAny>{})
+                             : launch(std::integral_constant<int, grf::kScanNoWholeRange>{}))
+    return rc;
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return grf::set_error(GRF_LAUNCH_FAILED, std::string("fused decode: ") + hipGetErrorString(e));
+  return GRF_OK;
 }
 
 template <class Walk, int M, int SCAN>

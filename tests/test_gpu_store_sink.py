@@ -1,0 +1,34 @@
+"""decode() through wave units at the edges of the quad exchange: rows whose segments do not fill a
+quad, segments of 16 and 32 words, tiles with empty slots, one row, one segment."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("rows", [3, 67, 130])
+@pytest.mark.parametrize("cols,segment", [(64, 64), (64 * 5, 64), (64 * 33, 64), (32 * 7, 32), (16 * 9, 16), (96, 48), (128 * 3, 128)])
+def test_wave_units_store_every_word(rows, cols, segment):
+    import torch
+    from georefine_amd import bitexact_context_codec as codec
+    from georefine_amd import bitexact_predictive_codec as predictive
+    from georefine_amd.bitexact_context_gpu import HipContextTensor
+    from georefine_amd.bitexact_predictive_gpu import HipPredictiveTensor
+    rng = np.random.default_rng(rows * 131 + cols)
+    # (few distinct exponents, so that even the smallest frame is coded and not raw words)
+    words = (rng.choice([0x3C00, 0x3C20, 0x3D00], (rows, cols)) | rng.integers(0, 32, (rows, cols))
+             | rng.integers(0, 2, (rows, cols)) << 15).astype(np.uint16)
+    frame = codec.encode(words)
+    if rows * cols < 1000 and frame[5] == 1:
+        pytest.skip("too small to be coded")
+    t = HipContextTensor(frame, fused_segment=segment)
+    assert t.fused is not None and t.fused_plan["seg_len"] == segment and t._store_tiling()[3]["scheme"] == 1
+    guard = torch.full((rows * cols + 64,), 0x5A5A, device="cuda", dtype=torch.int16)  # what the launch must not touch
+    t._launch(t._lib.grf_bctx_fused_decode, t.fused, t._store_tiling()[0], guard.data_ptr(), t.error.data_ptr())
+    got = guard.cpu().numpy().view(np.uint16)
+    assert np.array_equal(got[:rows * cols].reshape(words.shape), words) and (got[rows * cols:] == 0x5A5A).all()
+    assert np.array_equal(t.decode().view(torch.int16).cpu().numpy().view(np.uint16), words)
+    if segment % 32 == 0:
+        p = HipPredictiveTensor(predictive.encode(words, words ^ np.uint16(1)), words ^ np.uint16(1), fused_segment=segment)
+        if p.fused is not None:
+            assert np.array_equal(p.decode(None).view(torch.int16).cpu().numpy().view(np.uint16), words)
