@@ -525,6 +525,12 @@ def build_gemm_tiles(row_class, nr, r, first_tile=0, lead=0, cus=256):
     return np.ascontiguousarray(table).reshape(-1), tile_class, r, n_tall
 
 
+# Segments a wave of the row gather walks.  Fewer than a wave has lanes: more waves issue the table
+# copy and hide each other's steps (8192 x 5120: 64 rows 13.3 -> 12.7 us, 2048 rows 34.4 -> 33.8, 777
+# rows 17.2 -> 17.9); at 12 the waves' issue slots are the limit (777 rows: 30 us).
+GATHER_LANES = 32
+
+
 class FramePlan:
     """Frame-level derived arrays (shared by every tiling) and a tiling factory."""
 
@@ -635,17 +641,15 @@ class FramePlan:
                     scalars=dict(threads=threads, lanes_per_row=p, rows_per_tile=r, n_slabs=n_slabs,
                                  n_tiles=n_tiles, piece_cap=cap, scheme=SCHEME_WAVES), lds=lds)
 
-    def gather_scalars(self):
-        """Scalars of a tiling that gives every requested row a tile of its own, all of its
-        segments walked at once where a workgroup has the lanes (rows need no grouping by class
-        then); the caller supplies the rows and their classes per call."""
-        p = min(self.spr, 1024)
-        cap = self._cap(p)
-        lds = lds_bytes(self.nc, self.lognb, self.tabn, 0, p, self.seg_len, 1, cap)
-        if lds > MAX_LDS:
+    def gather_shape(self):
+        """(segments a wave walks, piece capacity) of the row gather: every requested row has a
+        workgroup of its own, which walks all of the row's segments at once where it has the lanes."""
+        waves = min(16, -(-self.spr // GATHER_LANES))
+        lanes = min(64, -(-(-(-self.spr // waves)) // 4) * 4)  # dealt evenly, whole quads
+        cap = self._cap(min(self.spr, lanes))
+        if (self.table_bytes() + 15) // 16 * 16 + waves * cap > MAX_LDS:
             raise FusedUnsupported("gather tile does not fit in LDS")
-        return dict(threads=-(-p // 64) * 64, lanes_per_row=p, rows_per_tile=1, n_slabs=-(-self.spr // p),
-                    piece_cap=cap), lds
+        return lanes, cap
 
     def _wave_limits(self):
         """Kernels over wave tilings address rows and segments with 24-bit multiplies."""

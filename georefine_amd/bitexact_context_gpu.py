@@ -122,6 +122,11 @@ GEMV_UP_TO = 2             # activation rows linear() gives to the vector-ALU ke
 GEMM_TWO_ROWS_FROM = 8192  # row length from which two activation rows go to the matrix-core kernel
 DENSE_ABOVE = 128          # activation rows above which linear() decodes to a dense transient
 
+# Words of pinned host memory that launches report to and their callers read after a wait; a call
+# takes one and gives it back zeroed (a list: taking and giving are atomic), at most this many stay.
+_host_words = []
+HOST_WORDS_KEPT = 16
+
 
 def route_rows(m, cols, invariant=False):
     """The kernel family that takes ``m`` activation rows of a matrix with ``cols`` columns:
@@ -143,6 +148,23 @@ def route_rows(m, cols, invariant=False):
     if m == 0 or m > GEMV_UP_TO or (m == 2 and cols >= GEMM_TWO_ROWS_FROM):
         return "gemm"
     return "gemv"
+
+
+def device_index(device):
+    """The ordinal of a torch device ("cuda" alone: the current one)."""
+    import torch
+    return device.index if device.index is not None else torch.cuda.current_device()
+
+
+def launch_on(index, fn, *args):
+    """``fn(*args, stream)`` with GPU ``index`` current, on its current stream.  (The handle as
+    torch's own generated code takes it, and the device switched only when it is another one: the
+    stream object and the context manager cost more than the launch.)"""
+    import torch
+    if torch._C._cuda_getDevice() == index:
+        return fn(*args, torch._C._cuda_getCurrentRawStream(index))
+    with torch.cuda.device(index):
+        return fn(*args, torch._C._cuda_getCurrentRawStream(index))
 
 
 class PackedActivations:
@@ -265,6 +287,8 @@ class HipContextTensor:
         self.frame_sha256 = indexed["frame_sha256"]
         self.frame_bytes = indexed["frame_bytes"]
         self.device = torch.device(device)
+        self._index = device_index(self.device)
+        self._error_open = True  # the error word may hold what an unchecked launch reported
         self.buffers = {}
         self.fused = None
         self.fused_reason = prepared["reason"]
@@ -303,7 +327,7 @@ class HipContextTensor:
             f.main.n_bytes = self._main_bytes
             self._frame = f
         self._tilings = {}
-        self._gather = None  # scalars of the row-gather tiling once planned; False: not possible
+        self._gather = None  # (lanes, piece capacity) of the row gather once planned; False: not possible
         if plan is not None:
             d = _hip_abi.GrfBctxFused()
             b = self.buffers
@@ -417,10 +441,9 @@ class HipContextTensor:
         result = torch.empty(count * self.stride, device=self.device, dtype=torch.uint16)
         if check:  # between checks the word keeps what earlier launches reported
             self.error.zero_()
-        with torch.cuda.device(self.device):
-            stream = torch.cuda.current_stream(self.device).cuda_stream
-            status = self._lib.grf_bctx_decode(ctypes.byref(self._frame), ids, count, result.data_ptr(),
-                                               self.error.data_ptr(), stream)
+        self._error_open = True
+        status = launch_on(self._index, self._lib.grf_bctx_decode, ctypes.byref(self._frame), ids, count, result.data_ptr(),
+                           self.error.data_ptr())
         if status:
             raise base.CodecError(f"device decode launch failed ({status}): "
                                   + self._lib.grf_last_error().decode(errors="replace"))
@@ -429,9 +452,7 @@ class HipContextTensor:
         return result.view(torch.bfloat16)
 
     def _launch(self, fn, *args):
-        import torch
-        with torch.cuda.device(self.device):
-            status = fn(*args, torch.cuda.current_stream(self.device).cuda_stream)
+        status = launch_on(self._index, fn, *args)
         if status:
             raise base.CodecError(f"device launch failed ({status}): "
                                   + self._lib.grf_last_error().decode(errors="replace"))
@@ -451,6 +472,7 @@ class HipContextTensor:
         out = torch.empty(self.n, device=self.device, dtype=torch.uint16)
         if check:  # between checks the word keeps what earlier launches reported
             self.error.zero_()
+        self._error_open = True
         self._launch(self._lib.grf_bctx_fused_decode, ctypes.byref(self.fused), ctypes.byref(self._store_tiling()[0]),
                      out.data_ptr(), self.error.data_ptr())
         self._check(check)
@@ -492,6 +514,7 @@ class HipContextTensor:
         y = torch.empty((packed.rows, self.shape[0]), device=self.device, dtype=torch.bfloat16)
         if check:  # between checks the word keeps what earlier launches reported
             self.error.zero_()
+        self._error_open = True
         tiling = self._gemm_tiling()[0]
         space = packed.ensure(self._lib.grf_gemm_workspace_bytes_split(self.shape[1], self.shape[0], tiling.k_parts,
                                                                        packed.rows))
@@ -508,6 +531,7 @@ class HipContextTensor:
         if x2.shape[0]:
             if check:  # between checks the word keeps what earlier launches reported
                 self.error.zero_()
+            self._error_open = True
             extra = ()
             if workspace:  # transient: the activations in the matrix cores' operand order (+ the parts' sums)
                 size = self._lib.grf_gemm_workspace_bytes_split(self.shape[1], self.shape[0], tiling.k_parts,
@@ -577,37 +601,55 @@ class HipContextTensor:
         ids = ids.to(device=self.device, dtype=torch.int64)
         if ids.numel() == 0:
             return torch.empty((*ids.shape, self.shape[1]), device=self.device, dtype=torch.bfloat16)
+        if self.fused is not None and self._gather is None:
+            try:
+                self._gather = self._plan.gather_shape()
+            except _fused.FusedUnsupported:
+                self._gather = False
+        if self.fused is not None and self._gather:
+            return self._gather_fused(ids, check, validate)
         if validate:
             if torch.any((ids < 0) | (ids >= self.shape[0])).item():
                 raise IndexError("embedding row outside tensor")
         else:
             ids = ids.clamp(0, self.shape[0] - 1)
-        if self.fused is not None and self._gather is not False:
-            if self._gather is None:
-                try:
-                    self._gather = self._plan.gather_scalars()[0]
-                except _fused.FusedUnsupported:
-                    self._gather = False
-            if self._gather:
-                flat = ids.reshape(-1)
-                rows = flat.to(torch.int32)
-                classes = self.buffers["rows"][flat]
-                g = _hip_abi.GrfFusedTiling()
-                g.tile_rows, g.tile_class, g.n_tiles = rows.data_ptr(), classes.data_ptr(), flat.numel()
-                for key, value in self._gather.items():
-                    setattr(g, key, value)
-                out = torch.empty((flat.numel(), self.shape[1]), device=self.device, dtype=torch.uint16)
-                if check:  # between checks the word keeps what earlier launches reported
-                    self.error.zero_()
-                self._launch(self._lib.grf_bctx_fused_gather, ctypes.byref(self.fused), ctypes.byref(g), out.data_ptr(),
-                             self.error.data_ptr())
-                self._check(check)
-                return out.view(torch.bfloat16).reshape(*ids.shape, self.shape[1])
         if self.mode == 1 or self.shape[1] % self.stride:
             return self.decode(check=check)[ids]
         per_row = self.shape[1] // self.stride
         blocks = (ids.reshape(-1, 1) * per_row + torch.arange(per_row, device=self.device)).reshape(-1)
         return self._decode_blocks(blocks, check=check).reshape(*ids.shape, self.shape[1])
+
+    def _gather_fused(self, ids, check, validate):
+        """One launch, which also looks up classes and tests the ids, and one wait for it: what it
+        finds wrong it writes to a word of pinned host memory, which nothing has to copy back."""
+        import torch
+        ids = ids.contiguous()
+        out = torch.empty((*ids.shape, self.shape[1]), device=self.device, dtype=torch.bfloat16)
+        word = None
+        if check or validate:
+            word = _host_words.pop() if _host_words else torch.zeros(1, dtype=torch.int32, pin_memory=True)
+        if check and self._error_open:  # between checks the word keeps what earlier launches reported
+            self.error.zero_()
+            self._error_open = False
+        elif not check:
+            self._error_open = True
+        self._launch(self._lib.grf_bctx_gather_rows, ctypes.byref(self.fused), *self._gather, self.buffers["rows"].data_ptr(),
+                     ids.data_ptr(), ids.numel(), out.data_ptr(), word.data_ptr() if check else self.error.data_ptr(),
+                     word.data_ptr() if validate else None)
+        if word is not None:
+            torch.cuda.current_stream(self.device).synchronize()
+            found = int(word[0])
+            if found:
+                word[0] = 0
+            if len(_host_words) < HOST_WORDS_KEPT:
+                _host_words.append(word)
+            if found & _hip_abi.ERR_INDEX:
+                raise IndexError("embedding row outside tensor")
+            if found:
+                self.error.fill_(found)
+                self._error_open = True
+                raise base.CodecError("HIP decoder checkpoint mismatch")
+        return out
 
 
 class HipLinearGroup:

@@ -191,4 +191,21 @@ int grf_bctx_fused_gather(const grf_bctx_fused *frame, const grf_fused_tiling *t
                                                              error, (hipStream_t)hip_stream);
 }
 
+int grf_bctx_gather_rows(const grf_bctx_fused *frame, uint32_t lanes, uint32_t piece_cap, const uint8_t *row_class,
+                         const int64_t *ids, uint32_t count, uint16_t *out, int32_t *error, int32_t *index_error, void *hip_stream) {
+  if (!frame || !row_class || !ids || !out || !error)
+    return grf::set_error(GRF_BAD_ARGUMENT, "grf_bctx_gather_rows: null argument");
+  grf_fused_tiling one{};  // (the frame's own checks, with a tiling that cannot fail them)
+  one.tile_rows = reinterpret_cast<const uint32_t *>(ids);
+  one.tile_class = row_class;
+  one.threads = 64;
+  one.lanes_per_row = 64;
+  one.rows_per_tile = one.n_tiles = 1;
+  one.n_slabs = (frame->segs_per_row + 63) / 64;
+  one.piece_cap = piece_cap;
+  if (int rc = grf::check_fused_frame(*frame, one, "grf_bctx_gather_rows")) return rc;
+  return grf::launch_gather<grf::SegmentWalk>("grf_bctx_gather_rows", *frame, lanes, piece_cap, row_class, ids, count, out,
+                                              error, index_error, (hipStream_t)hip_stream);
+}
+
 }  // extern "C"

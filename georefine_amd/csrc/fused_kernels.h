@@ -692,6 +692,107 @@ int launch_wave_store(const grf_bctx_fused &f, const grf_fused_tiling &g, uint16
   return GRF_OK;
 }
 
+// ---------------------------------------------------------------- row gather
+//
+// Rows by index (the embedding lookup): one workgroup per requested row, all of whose segments it
+// walks at once, `lanes` a wave; the row's class, its place in the resident order and whether it exists
+// are looked up here, so that the caller prepares nothing per call.  Latency: three dependent reads
+// (id; class and position; checkpoints), the table copy beside the last of them, one segment of
+// dependent steps; `flag` (may be null: ids are clamped then) gets GRF_ERR_INDEX for an id outside the
+// matrix.  error and flag may be host memory, hence the system-wide atomics.
+// 777 rows of 8192 x 5120: 17.9 us (the slab kernel behind four lookups and tests in torch: 23.6 + 12); the
+// pieces' LDS counts, four workgroups a compute unit take 777 rows at once and three do not (27.5).
+struct GatherLdsLayout {
+  uint32_t block_pitch, stream, total;
+  __host__ __device__ GatherLdsLayout(const grf_bctx_fused &f, uint32_t waves, uint32_t piece_cap) {
+    block_pitch = grf::fused_table_bytes(f) + (1u << f.lognb);
+    stream = grf::align_up(f.nc * block_pitch, 16);
+    total = grf::align_up(stream + waves * piece_cap, 16);
+  }
+};
+
+template <class Walk, int SCAN>
+__global__ __launch_bounds__(grf::kFusedMaxThreads) void fused_gather_kernel(grf_bctx_fused f, uint32_t lanes,
+                                                                              uint32_t piece_cap, const uint8_t *row_class, const int64_t *ids,
+                                                                              uint16_t *out, int32_t *error, int32_t *flag) {
+  extern __shared__ __align__(16) uint8_t lds[];
+  const uint32_t tid = threadIdx.x, nthreads = blockDim.x, nwaves = nthreads / 64, lane = tid % 64;
+#if defined(__HIP_DEVICE_COMPILE__)
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid / 64);
+#else
+  const uint32_t wave = tid / 64;
+#endif
+  const int64_t id = ids[blockIdx.x];
+  uint32_t row = (uint32_t)id;
+  if (id < 0 || id >= (int64_t)f.rows) {  // uniform
+    if (flag) {
+      if (tid == 0) atomicOr_system(flag, GRF_ERR_INDEX);
+      return;
+    }
+    row = id < 0 ? 0 : f.rows - 1;
+  }
+  const GatherLdsLayout L(f, nwaves, piece_cap);
+  uint32_t cls = row_class[row], rpos = row_position(f, row);
+#if defined(__HIP_DEVICE_COMPILE__)  // (told to the compiler as the scalars they are)
+  cls = __builtin_amdgcn_readfirstlane(cls);
+  rpos = __builtin_amdgcn_readfirstlane(rpos);
+#endif
+  const grf::FusedParams q{f.shift, L.block_pitch, grf::fused_table_bytes(f), f.whole_range};
+  if (grf::fused_tables_by_dma(f)) grf::fused_load_tables_dma(lds, 0, L.block_pitch, f, cls, wave, nwaves, lane);
+  const uint32_t S = f.seg_len, units = (f.segs_per_row + lanes - 1) / lanes, region = L.stream + wave * piece_cap;
+  uint16_t *dst = out + (size_t)blockIdx.x * f.cols;
+  uint32_t bad = 0;
+  for (uint32_t u = wave; u - wave < units; u += nwaves) {  // uniform, and as many trips for every wave (the barrier)
+    const bool any = u < units;
+    const uint32_t first_seg = any ? u * lanes : 0, nseg = any ? min(lanes, f.segs_per_row - first_seg) : 0;
+    const bool walks = lane < nseg;
+    const uint32_t seg = first_seg + (walks ? lane : 0), col0 = seg * S;
+    const uint32_t slot = grf::fused_seg_slot(f, row, rpos, first_seg);
+    const uint32_t g0 = grf::fused_index_entry(f.seg_offset, slot);
+    const uint32_t g1 = grf::fused_index_entry(f.seg_offset, slot + nseg * grf::fused_seg_step(f));
+    const uint32_t a0 = grf::fused_stage_piece_dma(lds, region, piece_cap, f, g0, g1, lane, 6, 1);
+    Walk w;
+    w.prefetch(f, grf::fused_seg_slot(f, row, rpos, seg), row * f.cols + col0, col0, seg, rpos);
+    w.start(region, a0);
+    if (u == wave) {  // the tables are in place
+      if (!grf::fused_tables_by_dma(f)) grf::fused_load_tables(lds, 0, L.block_pitch, f, cls, tid, nthreads);
+#if defined(__HIP_DEVICE_COMPILE__)
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#endif
+      __syncthreads();
+    }
+    __builtin_amdgcn_wave_barrier();
+    store_segment<Walk, SCAN>(w, q, S, walks, col0, dst, lane);
+    if (walks && !w.ended_on_checkpoint(f)) bad |= GRF_ERR_CHECKPOINT;
+  }
+  if (bad) atomicOr_system(error, (int)bad);
+}
+
+template <class Walk>
+int launch_gather(const char *who, const grf_bctx_fused &f, uint32_t lanes, uint32_t piece_cap, const uint8_t *row_class, const int64_t *ids,
+                  uint32_t count, uint16_t *out, int32_t *error, int32_t *flag, hipStream_t s) {
+  if (piece_cap % 16 || piece_cap < 16) return grf::set_error(GRF_BAD_ARGUMENT, std::string(who) + ": piece capacity");
+  if (!lanes || lanes > 64 || lanes % 4) return grf::set_error(GRF_BAD_ARGUMENT, std::string(who) + ": 4, 8, .. 64 lanes per wave");
+  if (((uintptr_t)out & 15)) return grf::set_error(GRF_BAD_ARGUMENT, std::string(who) + ": out must be 16-byte aligned");
+  if (!count) return GRF_OK;
+  const uint32_t waves = std::min(16u, (f.segs_per_row + lanes - 1) / lanes);
+  const GatherLdsLayout L(f, waves, piece_cap);
+  if (L.total > 160 * 1024) return grf::set_error(GRF_UNSUPPORTED, std::string(who) + ": LDS demand exceeds 160 KiB");
+  auto launch = [&](auto scan) -> int {
+    constexpr auto kernel = &fused_gather_kernel<Walk, decltype(scan)::value>;
+    if (L.total > 64 * 1024)
+      if (int rc = allow_full_lds<kernel>()) return rc;
+    hipLaunchKernelGGL(kernel, dim3(count), dim3(waves * 64), L.total, s, f, lanes, piece_cap, row_class, ids, out, error, flag);
+    return GRF_OK;
+  };
+  if (int rc = f.whole_range ? launch(std::integral_constant<int, grf::kScanAny>{})
+                             : launch(std::integral_constant<int, grf::kScanNoWholeRange>{}))
+    return rc;
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return grf::set_error(GRF_LAUNCH_FAILED, std::string(who) + ": " + hipGetErrorString(e));
+  return GRF_OK;
+}
+
 template <class Walk, int M, int SCAN>
 int launch_wave_scan(const grf_bctx_fused &f, const grf_fused_tiling &g, const uint16_t *x, uint32_t ldx, uint16_t *y,
                      uint32_t ldy, const uint16_t *bias, int32_t *error, hipStream_t s) {

@@ -111,6 +111,7 @@ int ppcx_checkpoint_binary(const uint8_t *stream, size_t bytes, uint64_t n, cons
 #define GRF_ERR_OVERRUN 2     /* decoder wanted bytes past the end of a stream */
 #define GRF_ERR_UNDERFLOW 4   /* state still below 2^23 after two refill bytes */
 #define GRF_ERR_CHECKPOINT 8  /* segment did not end on the next checkpoint */
+#define GRF_ERR_INDEX 16      /* a row id outside the matrix (grf_bctx_gather_rows) */
 
 /* return codes of the launch functions */
 #define GRF_OK 0
@@ -339,6 +340,14 @@ int grf_bctx_fused_decode(const grf_bctx_fused *frame, const grf_fused_tiling *t
  * grouping at all.  Rows outside the matrix are the caller's to reject. */
 int grf_bctx_fused_gather(const grf_bctx_fused *frame, const grf_fused_tiling *tiling, uint16_t *out,
                           int32_t *error, void *hip_stream);
+
+/* The same lookup from row ids as the caller has them: out[j][cols] = row ids[j], `count` ids in any order, any
+ * number of times; row_class: u8 [rows]; a wave walks `lanes` (4, 8, .. 64) segments of a row, and piece_cap is the
+ * capacity of a piece of that many.  An id
+ * outside the matrix sets GRF_ERR_INDEX in *index_error and leaves its output as it was; with index_error null
+ * ids are clamped into the matrix.  error and index_error may be device memory or pinned host memory. */
+int grf_bctx_gather_rows(const grf_bctx_fused *frame, uint32_t lanes, uint32_t piece_cap, const uint8_t *row_class,
+                         const int64_t *ids, uint32_t count, uint16_t *out, int32_t *error, int32_t *index_error, void *hip_stream);
 
 /* Fused decode-GEMM on the matrix cores for any number of activation rows; same operand
  * meaning as grf_bctx_gemv.  Batch-invariant in the sense of GS/bi_csrc/bi_gemm.cuh:1-17:

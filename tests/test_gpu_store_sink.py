@@ -32,3 +32,31 @@ def test_wave_units_store_every_word(rows, cols, segment):
         p = HipPredictiveTensor(predictive.encode(words, words ^ np.uint16(1)), words ^ np.uint16(1), fused_segment=segment)
         if p.fused is not None:
             assert np.array_equal(p.decode(None).view(torch.int16).cpu().numpy().view(np.uint16), words)
+
+
+@pytest.mark.parametrize("cols,segment", [(64 * 65, 64), (16 * 9, 16), (32 * 64, 32), (64 * 2, 64)])
+def test_row_gather_clamps_rejects_and_reports(cols, segment):
+    """Ids outside the matrix: an IndexError, or clamped where the caller vouches for them; a
+    miss is reported to the call that checks and only there; waves without segments."""
+    import torch
+    from georefine_amd import bitexact_context_codec as codec
+    from georefine_amd.bitexact_context_gpu import HipContextTensor
+    rng = np.random.default_rng(cols)
+    words = (rng.choice([0x3C00, 0x3C20, 0x3D00], (70, cols)) | rng.integers(0, 32, (70, cols))).astype(np.uint16)
+    t = HipContextTensor(codec.encode(words), fused_segment=segment)
+    assert t.fused is not None
+    ids = torch.tensor([[-5, 0, 69], [70, 3, 1 << 40]])
+    got = t.gather_rows(ids, check=False, validate=False).view(torch.int16).cpu().numpy().view(np.uint16)
+    assert np.array_equal(got, words[ids.clamp(0, 69).numpy()])
+    for bad in (70, -1, 1 << 32):
+        with pytest.raises(IndexError):
+            t.gather_rows(torch.tensor([1, bad]))
+    assert np.array_equal(t.gather_rows(torch.tensor([1]).cuda()).view(torch.int16).cpu().numpy().view(np.uint16), words[[1]])
+    t.buffers["fused_seg_state"].view(torch.int32)[t.index_slot(7, 1)] += 1  # forced from the host; kernels finish normally
+    t.gather_rows(torch.tensor([7]), check=False)
+    assert t.error.item() != 0
+    t.gather_rows(torch.tensor([8]))
+    assert t.error.item() == 0
+    with pytest.raises(codec.CodecError):
+        t.gather_rows(torch.tensor([7]))
+    assert t.error.item() != 0
