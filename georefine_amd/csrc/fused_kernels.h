@@ -1130,7 +1130,7 @@ __device__ __forceinline__ void fused_gemm_body(uint8_t *lds, const grf_bctx_fus
     const bool active = row != grf::kNoRow && p4 < nseg;
     const uint32_t col0 = mul24(first_seg + p4, S);
     // the pieces first: their ranges arrived during the walk before
-    const uint32_t a0 = grf::fused_stage_piece_dma(lds, region, g.piece_cap, f, g0, g1, lane, 0, 16);
+    const uint32_t a0 = grf::fused_stage_rows_dma(lds, region, g.piece_cap, f, g0, g1, lane);
     Walk w;
     {
       const uint32_t seg = grf::fused_seg_slot<true>(f, active ? row : 0, active ? rpos : 0, active ? first_seg + p4 : 0);
@@ -1165,17 +1165,18 @@ __device__ __forceinline__ void fused_gemm_body(uint8_t *lds, const grf_bctx_fus
     uint32_t xl = ((feeds ? col0 / 8 : K / 8) * m_pad + ln % 16) * 16;
     uint4 xa[MT];
     gemm_load_x<MT>(xa, xp, xl);
+    // (zeros for the lanes that do not walk, once: a walking lane overwrites its own)
+    uint32_t words[4] = {0u, 0u, 0u, 0u};
     for (uint32_t t = 0; t < S; t += 16) {
-      uint32_t lo[4] = {0u, 0u, 0u, 0u}, hi[4] = {0u, 0u, 0u, 0u};
       if (active) {
         w.begin16(t, S);
-        w.template half<0, SCAN>(q, lo);
+        w.template half<0, SCAN>(q, words);
       }
-      gemm_contract<MT>(acc, xa, lo);
+      gemm_contract<MT>(acc, xa, words);
       xl += x_step;
       gemm_load_x<MT>(xa, xp, xl);
-      if (active) w.template half<1, SCAN>(q, hi);
-      gemm_contract<MT>(acc, xa, hi);
+      if (active) w.template half<1, SCAN>(q, words);
+      gemm_contract<MT>(acc, xa, words);
       xl += x_step;
       gemm_load_x<MT>(xa, xp, xl);
     }
