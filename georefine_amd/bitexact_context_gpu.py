@@ -167,6 +167,26 @@ def launch_on(index, fn, *args):
         return fn(*args, torch._C._cuda_getCurrentRawStream(index))
 
 
+def rows_for(x, cols, index, device):
+    """``x`` as rows of ``cols`` BF16 values the kernels can read where they are (16-byte aligned,
+    rows a multiple of 8 apart); the common case, a contiguous tensor on the device, as it is."""
+    if x.get_device() == index and x.is_contiguous() and not x.data_ptr() & 15:
+        return x, cols
+    x2 = x.reshape(-1, cols).to(device)
+    if x2.stride(-1) != 1 or x2.stride(0) % 8 or x2.data_ptr() & 15:
+        import torch
+        x2 = x2.clone(memory_format=torch.contiguous_format)
+    return x2, x2.stride(0)
+
+
+def bias_for(bias, index, device):
+    """A bias vector as the kernels take it (BF16, contiguous, on the device)."""
+    import torch
+    if bias is None or (bias.dtype is torch.bfloat16 and bias.get_device() == index and bias.is_contiguous()):
+        return bias
+    return bias.to(device=device, dtype=torch.bfloat16).contiguous()
+
+
 class PackedActivations:
     """Activation rows copied once into the operand order of the matrix-core kernels, for
     several coded matrices that take the same input (q/k/v, gate/up): ``gemm`` and
@@ -327,6 +347,7 @@ class HipContextTensor:
             f.main.n_bytes = self._main_bytes
             self._frame = f
         self._tilings = {}
+        self._workspace = {}  # bytes by (activation rows, parts along K)
         self._gather = None  # (lanes, piece capacity) of the row gather once planned; False: not possible
         if plan is not None:
             d = _hip_abi.GrfBctxFused()
@@ -404,6 +425,8 @@ class HipContextTensor:
         one wave-unit tiling for every row count; under GEOREFINE_FUSED_GEMV=slabs (experiments
         and tests of the slab kernels) tilings are made for m in {1, 2, 4, 8} and shared by
         the row counts in between."""
+        if m and GEMV_WAVES and "waves" in self._tilings:
+            return self._tilings["waves"]
         import torch
         if m == 0:
             bucket = 0
@@ -454,8 +477,10 @@ class HipContextTensor:
     def _launch(self, fn, *args):
         status = launch_on(self._index, fn, *args)
         if status:
-            raise base.CodecError(f"device launch failed ({status}): "
-                                  + self._lib.grf_last_error().decode(errors="replace"))
+            self._raise_launch(status)
+
+    def _raise_launch(self, status):
+        raise base.CodecError(f"device launch failed ({status}): " + self._lib.grf_last_error().decode(errors="replace"))
 
     def _check(self, check):
         if check and self.error.item() != 0:
@@ -479,8 +504,8 @@ class HipContextTensor:
         return out.view(torch.bfloat16).reshape(self.shape)
 
     def _gemm_tiling(self):
-        import torch
         if "gemm" not in self._tilings:
+            import torch
             host = self._plan.gemm_tiling()
             rows = torch.from_numpy(host["tile_rows"]).to(self.device)
             classes = torch.from_numpy(host["tile_class"]).to(self.device)
@@ -492,25 +517,12 @@ class HipContextTensor:
             self.resident_bytes += rows.numel() * 4 + classes.numel()
         return self._tilings["gemm"]
 
-    def _prepare_activations(self, x, bias, align):
-        import torch
-        if x.dtype != torch.bfloat16 or x.shape[-1] != self.shape[1]:
-            raise ValueError("activation must be bfloat16 with the weight's input width")
-        x2 = x.reshape(-1, self.shape[1]).to(self.device)
-        if x2.stride(-1) != 1 or x2.stride(0) % align or x2.data_ptr() % (2 * align):
-            x2 = x2.clone(memory_format=torch.contiguous_format)
-        if bias is not None:
-            bias = bias.to(device=self.device, dtype=torch.bfloat16).contiguous()
-        y = torch.empty((x2.shape[0], self.shape[0]), device=self.device, dtype=torch.bfloat16)
-        return x2, bias, y
-
     def _packed_call(self, packed, bias, check):
         """The GEMM on rows that were packed before (x == NULL in the C call)."""
         import torch
         if packed.cols != self.shape[1] or packed.buffer.device != self.device:
             raise ValueError("packed activations of another width or device")
-        if bias is not None:
-            bias = bias.to(device=self.device, dtype=torch.bfloat16).contiguous()
+        bias = bias_for(bias, self._index, self.device)
         y = torch.empty((packed.rows, self.shape[0]), device=self.device, dtype=torch.bfloat16)
         if check:  # between checks the word keeps what earlier launches reported
             self.error.zero_()
@@ -526,30 +538,41 @@ class HipContextTensor:
 
     def _fused_call(self, fn, tiling, x, bias, check, *, workspace=False):
         import torch
-        lead = x.shape[:-1]
-        x2, bias, y = self._prepare_activations(x, bias, 8)
-        if x2.shape[0]:
+        rows, cols = self.shape
+        if x.dtype is not torch.bfloat16 or x.shape[-1] != cols:
+            raise ValueError("activation must be bfloat16 with the weight's input width")
+        x2, ldx = rows_for(x, cols, self._index, self.device)
+        bias = bias_for(bias, self._index, self.device)
+        m = x2.numel() // cols
+        y = x2.new_empty((*x.shape[:-1], rows))
+        if m:
             if check:  # between checks the word keeps what earlier launches reported
                 self.error.zero_()
             self._error_open = True
             extra = ()
             if workspace:  # transient: the activations in the matrix cores' operand order (+ the parts' sums)
-                size = self._lib.grf_gemm_workspace_bytes_split(self.shape[1], self.shape[0], tiling.k_parts,
-                                                                x2.shape[0])
-                packed = torch.empty(size, device=self.device, dtype=torch.uint8)
+                key = m if m <= PackedActivations.MAX_ROWS else PackedActivations.MAX_ROWS
+                size = self._workspace.get((key, tiling.k_parts))
+                if size is None:
+                    size = self._lib.grf_gemm_workspace_bytes_split(cols, rows, tiling.k_parts, key)
+                    self._workspace[key, tiling.k_parts] = size
+                packed = x2.new_empty((size + 1) // 2)
                 extra = (packed.data_ptr(), size)
-            self._launch(fn, ctypes.byref(self.fused), ctypes.byref(tiling), x2.data_ptr(), x2.stride(0),
-                         x2.shape[0], y.data_ptr(), y.stride(0), bias.data_ptr() if bias is not None else None,
-                         *extra, self.error.data_ptr())
-            self._check(check)
-        return y.reshape(*lead, self.shape[0])
+            status = launch_on(self._index, fn, ctypes.byref(self.fused), ctypes.byref(tiling), x2.data_ptr(), ldx, m,
+                               y.data_ptr(), rows, bias.data_ptr() if bias is not None else None, *extra,
+                               self.error.data_ptr())
+            if status:
+                self._raise_launch(status)
+            if check:
+                self._check(check)
+        return y
 
     def gemv(self, x, bias=None, *, check=False):
         """Fused decode-GEMV (vector ALUs) for 1..8 activation rows; the result of a row does
         not depend on how many rows the call carries."""
         if self.fused is None:
             raise base.CodecError("frame is not eligible for the fused kernels: " + self.fused_reason)
-        m = math.prod(x.shape[:-1])
+        m = x.numel() // x.shape[-1] if x.shape[-1] else 0
         if not 1 <= m <= 8:
             raise ValueError("gemv takes 1..8 activation rows")
         return self._fused_call(self._lib.grf_bctx_gemv, self._tiling(m)[0], x, bias, check)
@@ -576,14 +599,15 @@ class HipContextTensor:
         ``linear(x[:6])[:1]`` bit for bit.  Frames the fused kernels cannot take are decoded on
         the device and multiplied densely.  ``check=True`` reads the error word back (a host
         sync)."""
-        import torch.nn.functional as F
         if isinstance(x, PackedActivations):  # packed for the matrix-core kernel, which is what it gets
             return self.gemm(x, bias, check=check)
         if batch_invariant is None:
             batch_invariant = self.m_invariant
-        m = math.prod(x.shape[:-1])
+        width = x.shape[-1]
+        m = x.numel() // width if width else math.prod(x.shape[:-1])
         route = "dense" if self.fused is None else route_rows(m, self.shape[1], batch_invariant)
         if route == "dense":
+            import torch.nn.functional as F
             return F.linear(x.to(self.device), self.decode(check=check), bias)
         if route == "gemm":
             return self.gemm(x, bias, check=check)
@@ -670,12 +694,12 @@ class HipLinearGroup:
                 raise base.CodecError("frame is not eligible for the fused kernels: " + t.fused_reason)
             if t.shape[1] != first.shape[1] or t.device != first.device:
                 raise ValueError("group members need one width and one device")
-        self.device, self._lib = first.device, first._lib
+        self.device, self._lib, self._index = first.device, first._lib, first._index
         # the members' policy unless given: a group of members that keep rows bit-equal across
         # row counts does so too
         self.m_invariant = any(t.m_invariant for t in self.tensors) if m_invariant is None else bool(m_invariant)
         self.error = torch.zeros((), device=self.device, dtype=torch.int32)
-        self._tilings, self._pointer_arrays = {}, {}
+        self._tilings, self._pointer_arrays, self._workspace = {}, {}, {}
         for key in (1, 2, "gemm"):
             self._tiling(key)  # raises FusedUnsupported when the members cannot share a tiling
 
@@ -701,15 +725,15 @@ class HipLinearGroup:
 
     def _arrays(self, key, outs, biases):
         n = len(self.tensors)
-        if key not in self._pointer_arrays:  # the frames and tilings do not change between calls
+        if key not in self._pointer_arrays:  # frames, tilings and row counts do not change between calls
             tilings = self._tiling(key)
             self._pointer_arrays[key] = (
                 (ctypes.POINTER(_hip_abi.GrfBctxFused) * n)(*[ctypes.pointer(t.fused) for t in self.tensors]),
-                (ctypes.POINTER(_hip_abi.GrfFusedTiling) * n)(*[ctypes.pointer(g[0]) for g in tilings]))
-        frames, tiles = self._pointer_arrays[key]
-        ys = (ctypes.c_void_p * n)(*[y.data_ptr() for y in outs])
-        ldy = (ctypes.c_uint32 * n)(*[y.stride(0) for y in outs])
-        bias = (ctypes.c_void_p * n)(*[b.data_ptr() if b is not None else None for b in biases])
+                (ctypes.POINTER(_hip_abi.GrfFusedTiling) * n)(*[ctypes.pointer(g[0]) for g in tilings]),
+                (ctypes.c_uint32 * n)(*[t.shape[0] for t in self.tensors]), ctypes.c_void_p * n)
+        frames, tiles, ldy, pointers = self._pointer_arrays[key]
+        ys = pointers(*[y.data_ptr() for y in outs])
+        bias = pointers(*[b.data_ptr() if b is not None else None for b in biases]) if biases else None
         return frames, tiles, ys, ldy, bias
 
     def linear(self, x, biases=None, *, check=False, batch_invariant=None):
@@ -719,54 +743,62 @@ class HipLinearGroup:
         rows the members' own decode + matmul."""
         import torch
         n = len(self.tensors)
-        biases = list(biases) if biases is not None else [None] * n
-        if len(biases) != n:
-            raise ValueError("one bias (or None) per member")
-        packed = x if isinstance(x, PackedActivations) else None
-        m = packed.rows if packed else math.prod(x.shape[:-1])
-        lead = packed.lead if packed else tuple(x.shape[:-1])
+        if biases is not None:
+            biases = list(biases)
+            if len(biases) != n:
+                raise ValueError("one bias (or None) per member")
+            if not any(b is not None for b in biases):
+                biases = None
         cols = self.tensors[0].shape[1]
+        packed = x if isinstance(x, PackedActivations) else None
+        if packed is not None:
+            m, lead = packed.rows, packed.lead
+        else:
+            lead, width = x.shape[:-1], x.shape[-1]
+            m = x.numel() // width if width else math.prod(lead)
         if batch_invariant is None:
             batch_invariant = self.m_invariant
         route = "gemm" if packed is not None else route_rows(m, cols, batch_invariant)
         if route == "dense":
-            return [t.linear(x, b, check=check, batch_invariant=False) for t, b in zip(self.tensors, biases)]
+            return [t.linear(x, b, check=check, batch_invariant=False)
+                    for t, b in zip(self.tensors, biases if biases is not None else [None] * n)]
         if packed is not None:
             if packed.cols != cols or packed.buffer.device != self.device:
                 raise ValueError("packed activations of another width or device")
-            x2 = None
+            x2, xp, ldx, make = None, None, 0, self.error.new_empty
         else:
-            if x.dtype != torch.bfloat16 or x.shape[-1] != cols:
+            if x.dtype is not torch.bfloat16 or width != cols:
                 raise ValueError("activation must be bfloat16 with the weights' input width")
-            x2 = x.reshape(-1, cols).to(self.device)
-            if x2.stride(-1) != 1 or x2.stride(0) % 8 or x2.data_ptr() % 16:
-                x2 = x2.clone(memory_format=torch.contiguous_format)
-        biases = [b.to(device=self.device, dtype=torch.bfloat16).contiguous() if b is not None else None for b in biases]
-        outs = [torch.empty((m, t.shape[0]), device=self.device, dtype=torch.bfloat16) for t in self.tensors]
+            x2, ldx = rows_for(x, cols, self._index, self.device)
+            xp, make = x2.data_ptr(), x2.new_empty
+        if biases is not None:
+            biases = [bias_for(b, self._index, self.device) for b in biases]
+        outs = [make((*lead, t.shape[0]), dtype=torch.bfloat16) for t in self.tensors]
         if m:
             if check:
                 self.error.zero_()
-            use_gemm = route == "gemm"
-            with torch.cuda.device(self.device):
-                stream = torch.cuda.current_stream(self.device).cuda_stream
-                if use_gemm:
-                    arrays = self._arrays("gemm", outs, biases)
-                    space = packed.buffer if packed else torch.empty(
-                        self._lib.grf_gemm_workspace_bytes(cols, m), device=self.device, dtype=torch.uint8)
-                    status = self._lib.grf_bctx_gemm_group(
-                        n, arrays[0], arrays[1], x2.data_ptr() if x2 is not None else None,
-                        x2.stride(0) if x2 is not None else 0, m, arrays[2], arrays[3], arrays[4], space.data_ptr(),
-                        space.numel(), self.error.data_ptr(), stream)
+            if route == "gemm":
+                frames, tiles, ys, ldy, bias = self._arrays("gemm", outs, biases)
+                if packed is not None:
+                    space, size = packed.buffer, packed.buffer.numel()
                 else:
-                    arrays = self._arrays(next(v for v in (1, 2, 4, 8) if v >= m), outs, biases)
-                    status = self._lib.grf_bctx_gemv_group(n, arrays[0], arrays[1], x2.data_ptr(), x2.stride(0), m,
-                                                           arrays[2], arrays[3], arrays[4], self.error.data_ptr(), stream)
+                    key = m if m <= PackedActivations.MAX_ROWS else PackedActivations.MAX_ROWS
+                    size = self._workspace.get(key)
+                    if size is None:
+                        size = self._workspace[key] = self._lib.grf_gemm_workspace_bytes(cols, key)
+                    space = x2.new_empty((size + 1) // 2)
+                status = launch_on(self._index, self._lib.grf_bctx_gemm_group, n, frames, tiles, xp, ldx, m, ys, ldy, bias,
+                                   space.data_ptr(), size, self.error.data_ptr())
+            else:
+                frames, tiles, ys, ldy, bias = self._arrays(next(v for v in (1, 2, 4, 8) if v >= m), outs, biases)
+                status = launch_on(self._index, self._lib.grf_bctx_gemv_group, n, frames, tiles, xp, ldx, m, ys, ldy, bias,
+                                   self.error.data_ptr())
             if status:
                 raise base.CodecError(f"device launch failed ({status}): "
                                       + self._lib.grf_last_error().decode(errors="replace"))
             if check and self.error.item() != 0:
                 raise base.CodecError("HIP decoder checkpoint mismatch")
-        return [y.reshape(*lead, t.shape[0]) for y, t in zip(outs, self.tensors)]
+        return outs
 
 
 # The loaders name the class they expect; keep that name importable.

@@ -184,7 +184,9 @@ class HipPredictiveTensor:
                 self.buffers[name + "_cum"] = torch.from_numpy(cum).to(self.device)
                 self.buffers[name + "_bucket"] = torch.from_numpy(_tables.coarse_buckets(cum)).to(self.device)
         self.error = torch.zeros((), device=self.device, dtype=torch.int32)
-        self._tilings = {}
+        from .bitexact_context_gpu import device_index
+        self._index = device_index(self.device)
+        self._tilings, self._workspace = {}, {}
         self._bind()
         # What the tile walker needs of the reference is the 4-bit bin of every word (the
         # decoded word itself comes from the frame's symbols alone), and the reference is given
@@ -245,7 +247,7 @@ class HipPredictiveTensor:
         other = copy.copy(self)
         other.buffers = {k: v.clone() for k, v in self.buffers.items()}
         other.error = torch.zeros_like(self.error)
-        other._tilings = {}
+        other._tilings, other._workspace = {}, {}
         other._bind()
         return other
 
@@ -299,8 +301,8 @@ class HipPredictiveTensor:
     def _tiling_for(self, key):
         """Device copy of a tiling: key 0 = store sink, "waves" = the GEMV (wave units, one tiling
         for every row count), 1/2/4/8 = GEMV row buckets of the slab kernels, "gemm"."""
-        import torch
         if key not in self._tilings:
+            import torch
             host = (self._plan.gemm_tiling() if key == "gemm" else
                     self._plan.tiling(_fused.WAVE_ROWS_PER_PASS, waves=True) if key == "waves" else self._plan.tiling(key))
             rows = torch.from_numpy(host["tile_rows"].view(np.int32)).to(self.device)
@@ -357,7 +359,7 @@ class HipPredictiveTensor:
             return self._product(reference_bf16_device, x, bias, check, True)
         if batch_invariant is None:  # the tensor's policy
             batch_invariant = self.m_invariant
-        m = math.prod(x.shape[:-1])
+        m = x.numel() // x.shape[-1] if x.shape[-1] else 0
         if self.fused is None or x.dtype != torch.bfloat16 or (m > self.DENSE_ABOVE and not batch_invariant):
             return torch.nn.functional.linear(x, self.decode(reference_bf16_device, check=check), bias)
         return self._product(reference_bf16_device, x, bias, check, batch_invariant or m > self.GEMV_UP_TO)
@@ -377,50 +379,51 @@ class HipPredictiveTensor:
         import torch
         if self.fused is None:
             raise codec.CodecError("frame is not eligible for the fused kernels: " + str(self.fused_reason))
-        from .bitexact_context_gpu import PackedActivations
+        from .bitexact_context_gpu import PackedActivations, bias_for, launch_on, rows_for
         packed = x if isinstance(x, PackedActivations) else None
+        rows, cols = self.shape
         if packed is not None:
-            if not use_gemm or packed.cols != self.shape[1] or packed.buffer.device != self.device:
+            if not use_gemm or packed.cols != cols or packed.buffer.device != self.device:
                 raise ValueError("packed activations go to the GEMM of a weight of their width on their device")
-            m, lead, x2 = packed.rows, packed.lead, None
+            m, lead, xp, ldx = packed.rows, packed.lead, None, 0
+            y = torch.empty((*lead, rows), device=self.device, dtype=torch.bfloat16)
         else:
-            if x.dtype != torch.bfloat16:
+            if x.dtype is not torch.bfloat16:
                 raise ValueError("activation must be bfloat16")
-            m, lead = math.prod(x.shape[:-1]), tuple(x.shape[:-1])
-            x2 = x.reshape(-1, x.shape[-1]).to(self.device)
-            if x2.shape[-1] != self.shape[1]:
+            if x.shape[-1] != cols:
                 raise ValueError("activation width does not match the weight")
-            align = 4 if use_gemm else 8  # elements: the GEMM reads 8 bytes at a time, the GEMV 16
-            if x2.stride(-1) != 1 or x2.stride(0) % align or x2.data_ptr() % (2 * align):
-                x2 = x2.clone(memory_format=torch.contiguous_format)
-        if bias is not None:
-            bias = bias.to(device=self.device, dtype=torch.bfloat16).contiguous()
-        y = torch.empty((m, self.shape[0]), device=self.device, dtype=torch.bfloat16)
+            x2, ldx = rows_for(x, cols, self._index, self.device)
+            m, xp = x2.numel() // cols, x2.data_ptr()
+            y = x2.new_empty((*x.shape[:-1], rows))
+        bias = bias_for(bias, self._index, self.device)
         if m:
             if check:  # between checks the word keeps what earlier launches reported
                 self.error.zero_()
-            with torch.cuda.device(self.device):
-                bins, status = self._contexts(reference_bf16_device)
-                if not status:
-                    extra = ()
-                    if use_gemm:
-                        fn, tiling = self._lib.grf_ppcx_gemm, self._tiling_for("gemm")[0]
-                        size = self._lib.grf_gemm_workspace_bytes_split(self.shape[1], self.shape[0], tiling.k_parts, m)
-                        if packed is not None:
-                            space = packed.ensure(size)
-                        else:  # transient: the activations in the matrix cores' operand order (+ the parts' sums)
-                            space = torch.empty(size, device=self.device, dtype=torch.uint8)
-                        extra = (space.data_ptr(), space.numel())
-                    else:
-                        fn = self._lib.grf_ppcx_gemv
-                        tiling = self._tiling_for("waves")[0]
-                    status = fn(ctypes.byref(self.fused), ctypes.byref(tiling), bins.data_ptr(),
-                                x2.data_ptr() if x2 is not None else None, x2.stride(0) if x2 is not None else 0,
-                                m, y.data_ptr(), y.stride(0),
-                                bias.data_ptr() if bias is not None else None, *extra, self.error.data_ptr(),
-                                torch.cuda.current_stream(self.device).cuda_stream)
+            if self.has_contexts:
+                bins, status = self.buffers["context_bins"], 0
+            else:
+                with torch.cuda.device(self.device):
+                    bins, status = self._contexts(reference_bf16_device)
+            if not status:
+                extra = ()
+                if use_gemm:
+                    fn, tiling = self._lib.grf_ppcx_gemm, self._tiling_for("gemm")[0]
+                    key = m if m <= PackedActivations.MAX_ROWS else PackedActivations.MAX_ROWS
+                    size = self._workspace.get((key, tiling.k_parts))
+                    if size is None:
+                        size = self._lib.grf_gemm_workspace_bytes_split(cols, rows, tiling.k_parts, key)
+                        self._workspace[key, tiling.k_parts] = size
+                    # transient: the activations in the matrix cores' operand order (+ the parts' sums)
+                    space = packed.ensure(size) if packed is not None else x2.new_empty((size + 1) // 2)
+                    extra = (space.data_ptr(), size)
+                else:
+                    fn = self._lib.grf_ppcx_gemv
+                    tiling = self._tiling_for("waves")[0]
+                status = launch_on(self._index, fn, ctypes.byref(self.fused), ctypes.byref(tiling), bins.data_ptr(), xp, ldx,
+                                   m, y.data_ptr(), rows, bias.data_ptr() if bias is not None else None, *extra,
+                                   self.error.data_ptr())
             self._status(status, check)
-        return y.reshape(*lead, self.shape[0])
+        return y
 
     def _status(self, status, check):
         if status:
@@ -508,15 +511,15 @@ class HipPredictiveGroup:
 
     def _arrays(self, key, outs, biases):
         n = len(self.tensors)
-        if key not in self._pointer_arrays:  # frames, tilings and planes do not change between calls
+        if key not in self._pointer_arrays:  # frames, tilings, planes and row counts do not change between calls
             self._pointer_arrays[key] = (
                 (ctypes.POINTER(_hip_abi.GrfPpcxFused) * n)(*[ctypes.pointer(t.fused) for t in self.tensors]),
                 (ctypes.POINTER(_hip_abi.GrfFusedTiling) * n)(*[ctypes.pointer(g[0]) for g in self._tiling(key)]),
-                (ctypes.c_void_p * n)(*[t.buffers["context_bins"].data_ptr() for t in self.tensors]))
-        frames, tiles, bins = self._pointer_arrays[key]
-        ys = (ctypes.c_void_p * n)(*[y.data_ptr() for y in outs])
-        ldy = (ctypes.c_uint32 * n)(*[y.stride(0) for y in outs])
-        bias = (ctypes.c_void_p * n)(*[b.data_ptr() if b is not None else None for b in biases])
+                (ctypes.c_void_p * n)(*[t.buffers["context_bins"].data_ptr() for t in self.tensors]),
+                (ctypes.c_uint32 * n)(*[t.shape[0] for t in self.tensors]), ctypes.c_void_p * n)
+        frames, tiles, bins, ldy, pointers = self._pointer_arrays[key]
+        ys = pointers(*[y.data_ptr() for y in outs])
+        bias = pointers(*[b.data_ptr() if b is not None else None for b in biases])
         return frames, tiles, bins, ys, ldy, bias
 
     def linear(self, x, biases=None, *, check=False, batch_invariant=None):
@@ -524,7 +527,7 @@ class HipPredictiveGroup:
         One activation row goes to the vector-ALU kernel, up to 128 to the matrix cores (every
         row count under ``batch_invariant``), more than that to the members' own ``linear``."""
         import torch
-        from .bitexact_context_gpu import PackedActivations
+        from .bitexact_context_gpu import PackedActivations, bias_for, launch_on, rows_for
         n = len(self.tensors)
         biases = list(biases) if biases is not None else [None] * n
         if len(biases) != n:
@@ -544,35 +547,31 @@ class HipPredictiveGroup:
                 raise ValueError("packed activations of another width or device")
             x2 = None
         else:
-            if x.dtype != torch.bfloat16 or x.shape[-1] != cols:
+            if x.dtype is not torch.bfloat16 or x.shape[-1] != cols:
                 raise ValueError("activation must be bfloat16 with the weights' input width")
-            x2 = x.reshape(-1, cols).to(self.device)
-            if x2.stride(-1) != 1 or x2.stride(0) % 8 or x2.data_ptr() % 16:
-                x2 = x2.clone(memory_format=torch.contiguous_format)
-        biases = [b.to(device=self.device, dtype=torch.bfloat16).contiguous() if b is not None else None for b in biases]
-        outs = [torch.empty((m, t.shape[0]), device=self.device, dtype=torch.bfloat16) for t in self.tensors]
+            x2, ldx = rows_for(x, cols, first._index, self.device)
+        biases = [bias_for(b, first._index, self.device) for b in biases]
+        outs = [torch.empty((*lead, t.shape[0]), device=self.device, dtype=torch.bfloat16) for t in self.tensors]
         if m:
             if check:
                 self.error.zero_()
-            with torch.cuda.device(self.device):
-                stream = torch.cuda.current_stream(self.device).cuda_stream
-                xp, ldx = (x2.data_ptr(), x2.stride(0)) if x2 is not None else (None, 0)
-                if use_gemm:
-                    a = self._arrays("gemm", outs, biases)
-                    space = packed.buffer if packed else torch.empty(
-                        self._lib.grf_gemm_workspace_bytes(cols, m), device=self.device, dtype=torch.uint8)
-                    status = self._lib.grf_ppcx_gemm_group(n, a[0], a[1], a[2], xp, ldx, m, a[3], a[4], a[5],
-                                                           space.data_ptr(), space.numel(), self.error.data_ptr(), stream)
-                else:
-                    a = self._arrays("waves", outs, biases)
-                    status = self._lib.grf_ppcx_gemv_group(n, a[0], a[1], a[2], xp, ldx, m, a[3], a[4], a[5],
-                                                           self.error.data_ptr(), stream)
+            xp, ldx = (x2.data_ptr(), ldx) if x2 is not None else (None, 0)
+            if use_gemm:
+                frames, tiles, bins, ys, ldy, bias = self._arrays("gemm", outs, biases)
+                space = packed.buffer if packed else torch.empty(
+                    self._lib.grf_gemm_workspace_bytes(cols, m), device=self.device, dtype=torch.uint8)
+                status = launch_on(first._index, self._lib.grf_ppcx_gemm_group, n, frames, tiles, bins, xp, ldx, m, ys, ldy,
+                                   bias, space.data_ptr(), space.numel(), self.error.data_ptr())
+            else:
+                frames, tiles, bins, ys, ldy, bias = self._arrays("waves", outs, biases)
+                status = launch_on(first._index, self._lib.grf_ppcx_gemv_group, n, frames, tiles, bins, xp, ldx, m, ys, ldy,
+                                   bias, self.error.data_ptr())
             if status:
                 raise codec.CodecError(f"device launch failed ({status}): "
                                        + self._lib.grf_last_error().decode(errors="replace"))
             if check and self.error.item() != 0:
                 raise codec.CodecError("HIP PPCX checkpoint/context mismatch")
-        return [y.reshape(*lead, t.shape[0]) for y, t in zip(outs, self.tensors)]
+        return outs
 
 
 CudaPredictiveTensor = HipPredictiveTensor
