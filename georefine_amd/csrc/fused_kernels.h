@@ -1033,6 +1033,33 @@ __device__ __forceinline__ void gemm_load_x(uint4 (&xa)[MT], const uint4 *xp, ui
   }
 }
 
+// The activations of a launch: the packed copy (pitch 0), or the caller's own rows, `pitch` bytes
+// apart and `bytes` from the first value to past the last.
+struct GemmX {
+  const void *data;
+  uint32_t pitch, bytes;
+};
+
+// The same operands from the caller's own rows.  Loads through a buffer descriptor: a row the
+// launch does not have, and a lane that feeds zeros, read past the descriptor's end, which
+// yields zeros without a memory access, so neither needs a branch or padding.
+template <int MT>
+__device__ __forceinline__ void gemm_load_rows(uint4 (&xa)[MT], const GemmX &x, uint32_t at) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  typedef uint32_t uint4v __attribute__((ext_vector_type(4)));
+  const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(x.data), 0, (int)x.bytes, 0x00020000);
+#pragma unroll
+  for (int j = 0; j < MT; ++j) {
+    const uint4v v = __builtin_bit_cast(uint4v, __builtin_amdgcn_raw_buffer_load_b128(rsrc, at + (uint32_t)j * 16u * x.pitch, 0, 0));
+    xa[j] = make_uint4(v.x, v.y, v.z, v.w);
+  }
+#else
+  (void)xa;
+  (void)x;
+  (void)at;
+#endif
+}
+
 template <int MT>
 __device__ __forceinline__ void gemm_contract(float4v (&acc)[MT], const uint4 (&xa)[MT], const uint32_t (&w)[4]) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -1048,16 +1075,17 @@ __device__ __forceinline__ void gemm_contract(float4v (&acc)[MT], const uint4 (&
 #endif
 }
 
-// MT: 16-row activation tiles of this launch (m_rows <= 16 * MT, xp packed with m_pad = 16 * MT)
+// MT: 16-row activation tiles of this launch (m_rows <= 16 * MT).  ROWS: x is the caller's rows (a
+// small product, own_rows); else the packed copy, with m_pad = 16 * MT.
 // With g.k_parts > 1 the launch's tiles are k_parts copies of the row tiles, part-major: copy
 // `part` walks the slabs [part * spp, (part + 1) * spp) with spp = ceil(n_slabs / k_parts) and
 // leaves its sums as fp32 in `partials` [k_parts][m_rows][rows]; gemm_sum_parts_kernel adds the
 // parts in order, then the bias, and rounds.  That lets a matrix with few rows be cut along K
 // until its tiles fill the machine with full blocks of sixteen rows, in a fixed order of
 // additions (the tiling is the matrix's, whatever the batch).
-template <class Walk, int MT, int SCAN>
+template <class Walk, int MT, int SCAN, bool ROWS>
 __device__ __forceinline__ void fused_gemm_body(uint8_t *lds, const grf_bctx_fused &f, const grf_fused_tiling &g,
-                                                const uint4 *xp, uint32_t m_rows, uint16_t *y, uint32_t ldy,
+                                                const GemmX &x, uint32_t m_rows, uint16_t *y, uint32_t ldy,
                                                 const uint16_t *bias, float *partials, int32_t *error,
                                                 uint32_t launch_tile) {
   const GemmLdsLayout L(f, g);
@@ -1156,15 +1184,21 @@ __device__ __forceinline__ void fused_gemm_body(uint8_t *lds, const grf_bctx_fus
     // they read the chunk of zeros that ends the packed copy and never move on.  The load
     // after a segment's last half group reads the chunk that follows it, at most that one.
     const bool feeds = p4 < nseg;
-    const uint32_t x_step = feeds ? m_pad * 16 : 0;  // bytes from one 8-column chunk to the next
+    // bytes from one 8-column chunk to the next
+    const uint32_t x_step = feeds ? (ROWS ? 16u : m_pad * 16) : 0;
+    auto load_x = [&](uint4 (&to)[MT], uint32_t at) {
+      if constexpr (ROWS) gemm_load_rows<MT>(to, x, at);
+      else gemm_load_x<MT>(to, static_cast<const uint4 *>(x.data), at);
+    };
     // (the lane's number is worked out again here rather than kept in a register over the walks)
     uint32_t ln = __lane_id();
 #if defined(__HIP_DEVICE_COMPILE__)
     asm volatile("" : "+v"(ln));
 #endif
-    uint32_t xl = ((feeds ? col0 / 8 : K / 8) * m_pad + ln % 16) * 16;
+    uint32_t xl = ROWS ? (feeds ? (ln % 16) * x.pitch + col0 * 2 : x.bytes)
+                       : ((feeds ? col0 / 8 : K / 8) * m_pad + ln % 16) * 16;
     uint4 xa[MT];
-    gemm_load_x<MT>(xa, xp, xl);
+    load_x(xa, xl);
     // (zeros for the lanes that do not walk, once: a walking lane overwrites its own)
     uint32_t words[4] = {0u, 0u, 0u, 0u};
     for (uint32_t t = 0; t < S; t += 16) {
@@ -1174,11 +1208,11 @@ __device__ __forceinline__ void fused_gemm_body(uint8_t *lds, const grf_bctx_fus
       }
       gemm_contract<MT>(acc, xa, words);
       xl += x_step;
-      gemm_load_x<MT>(xa, xp, xl);
+      load_x(xa, xl);
       if (active) w.template half<1, SCAN>(q, words);
       gemm_contract<MT>(acc, xa, words);
       xl += x_step;
-      gemm_load_x<MT>(xa, xp, xl);
+      load_x(xa, xl);
     }
     if (active && !w.ended_on_checkpoint(f)) bad |= GRF_ERR_CHECKPOINT;
   }
@@ -1229,40 +1263,40 @@ __device__ __forceinline__ void fused_gemm_body(uint8_t *lds, const grf_bctx_fus
 }
 
 // Up to four activation tiles: 80 vector registers, six waves per SIMD.
-template <class Walk, int MT, int SCAN>
+template <class Walk, int MT, int SCAN, bool ROWS>
 __global__ __launch_bounds__(grf::kFusedMaxThreads) __attribute__((amdgpu_waves_per_eu(6))) void fused_gemm_kernel(
-    grf_bctx_fused f, grf_fused_tiling g, const uint4 *xp, uint32_t m_rows, uint16_t *y, uint32_t ldy,
+    grf_bctx_fused f, grf_fused_tiling g, GemmX x, uint32_t m_rows, uint16_t *y, uint32_t ldy,
     const uint16_t *bias, float *partials, int32_t *error) {
   extern __shared__ __align__(16) uint8_t lds[];
-  fused_gemm_body<Walk, MT, SCAN>(lds, f, g, xp, m_rows, y, ldy, bias, partials, error, blockIdx.x);
+  fused_gemm_body<Walk, MT, SCAN, ROWS>(lds, f, g, x, m_rows, y, ldy, bias, partials, error, blockIdx.x);
 }
 
 // Eight activation tiles: the accumulators and operands alone take 64 registers, so fewer
 // waves are resident; still cheaper than decoding the matrix twice.
 template <class Walk, int MT, int SCAN>
 __global__ __launch_bounds__(grf::kFusedMaxThreads) void fused_gemm_wide_kernel(grf_bctx_fused f, grf_fused_tiling g,
-                                                                                 const uint4 *xp, uint32_t m_rows,
+                                                                                 GemmX x, uint32_t m_rows,
                                                                                  uint16_t *y, uint32_t ldy,
                                                                                  const uint16_t *bias, float *partials, int32_t *error) {
   extern __shared__ __align__(16) uint8_t lds[];
-  fused_gemm_body<Walk, MT, SCAN>(lds, f, g, xp, m_rows, y, ldy, bias, partials, error, blockIdx.x);
+  fused_gemm_body<Walk, MT, SCAN, false>(lds, f, g, x, m_rows, y, ldy, bias, partials, error, blockIdx.x);
 }
 
-template <class Walk, int MT, int SCAN>
+template <class Walk, int MT, int SCAN, bool ROWS>
 __global__ __launch_bounds__(grf::kFusedMaxThreads) __attribute__((amdgpu_waves_per_eu(6))) void fused_gemm_group_kernel(
-    FusedGroup a, const uint4 *xp, uint32_t m_rows, int32_t *error) {
+    FusedGroup a, GemmX x, uint32_t m_rows, int32_t *error) {
   extern __shared__ __align__(16) uint8_t lds[];
   const uint32_t i = group_member(a, blockIdx.x);
-  fused_gemm_body<Walk, MT, SCAN>(lds, a.f[i], a.g[i], xp, m_rows, a.y[i], a.ldy[i], a.bias[i], nullptr, error,
+  fused_gemm_body<Walk, MT, SCAN, ROWS>(lds, a.f[i], a.g[i], x, m_rows, a.y[i], a.ldy[i], a.bias[i], nullptr, error,
                                   blockIdx.x - a.first_tile[i]);
 }
 
 template <class Walk, int MT, int SCAN>
-__global__ __launch_bounds__(grf::kFusedMaxThreads) void fused_gemm_wide_group_kernel(FusedGroup a, const uint4 *xp,
+__global__ __launch_bounds__(grf::kFusedMaxThreads) void fused_gemm_wide_group_kernel(FusedGroup a, GemmX x,
                                                                                        uint32_t m_rows, int32_t *error) {
   extern __shared__ __align__(16) uint8_t lds[];
   const uint32_t i = group_member(a, blockIdx.x);
-  fused_gemm_body<Walk, MT, SCAN>(lds, a.f[i], a.g[i], xp, m_rows, a.y[i], a.ldy[i], a.bias[i], nullptr, error,
+  fused_gemm_body<Walk, MT, SCAN, false>(lds, a.f[i], a.g[i], x, m_rows, a.y[i], a.ldy[i], a.bias[i], nullptr, error,
                                   blockIdx.x - a.first_tile[i]);
 }
 
@@ -1280,28 +1314,58 @@ static __global__ __launch_bounds__(256) void gemm_sum_parts_kernel(const float 
   y[(size_t)m * ldy + n] = round_bf16(sum);
 }
 
+// A small product reads the activations from the caller's own rows, which saves the launch of
+// the packing kernel (2.3 us of the host's time, 1.5 to 2.5 us of the GPU's).  In return a load's
+// lanes touch a cache line each instead of sharing eight or so, measured at 16 ns per million
+// (weights x rows): 17408 and 17408 x 5120 at 16 rows 143 -> 184 us, 6144 + 1024 + 1024 x 5120 at
+// 32 rows 43 -> 61, but 1024 x 5120 at 8 rows 17.8 -> 16.0, 1500 x 2048 at 20 rows 17.2 -> 15.5.
+// They break even near 200 million; the line is drawn at 128.  (Above four tiles of rows such a
+// matrix has two million weights at most and the copy is a small part of the product.)
+inline constexpr uint32_t kOwnRowsMax = 64;
+inline constexpr uint64_t kOwnRowsWork = 128u << 20;
+
+inline bool own_rows(const uint16_t *x, uint32_t ldx, uint32_t m_rows, uint64_t weights) {
+  return x && m_rows <= kOwnRowsMax && weights * m_rows <= kOwnRowsWork &&
+         (uint64_t)ldx * 2 * 16 * gemm_tiles(m_rows) < (1u << 31);  // (offsets are 32 bits wide)
+}
+
+inline GemmX gemm_source(const uint16_t *x, uint32_t ldx, uint32_t m_rows, uint32_t cols, uint64_t weights, uint4 *xp,
+                         hipStream_t s) {
+  if (own_rows(x, ldx, m_rows, weights)) return GemmX{x, ldx * 2, ((m_rows - 1) * ldx + cols) * 2};
+  if (x) launch_pack(x, ldx, m_rows, cols, gemm_tiles(m_rows) * 16, xp, s);  // else the caller packed these rows already
+  return GemmX{xp, 0, 0};
+}
+
+// launch(scan, rows) for the scan the frames need and the activations' form
+template <int MT, class Launch>
+int launch_scan_and_rows(bool whole_range, bool rows, const Launch &launch) {
+  using Any = std::integral_constant<int, grf::kScanAny>;
+  using Usual = std::integral_constant<int, grf::kScanNoWholeRange>;
+  if constexpr (MT * 16 <= kOwnRowsMax)
+    if (rows) return whole_range ? launch(Any{}, std::true_type{}) : launch(Usual{}, std::true_type{});
+  return whole_range ? launch(Any{}, std::false_type{}) : launch(Usual{}, std::false_type{});
+}
+
 template <class Walk, int MT>
 int launch_gemm_rows(const grf_bctx_fused &f, const grf_fused_tiling &g, const uint16_t *x, uint32_t ldx, uint32_t m_rows,
                      uint16_t *y, uint32_t ldy, const uint16_t *bias, uint4 *xp, float *partials, int32_t *error,
                      hipStream_t s) {
   const GemmLdsLayout L(f, g);
   if (L.total > 160 * 1024) return grf::set_error(GRF_UNSUPPORTED, "fused GEMM: LDS demand exceeds 160 KiB");
-  if (x) launch_pack(x, ldx, m_rows, f.cols, MT * 16, xp, s);  // else the caller packed these rows already
-  auto launch = [&](auto scan) -> int {
+  const GemmX source = gemm_source(x, ldx, m_rows, f.cols, (uint64_t)f.rows * f.cols, xp, s);
+  auto launch = [&](auto scan, auto rows) -> int {
     constexpr int SCAN = decltype(scan)::value;
     constexpr auto kernel = [] {
-      if constexpr (MT <= 4) return &fused_gemm_kernel<Walk, MT, SCAN>;
+      if constexpr (MT <= 4) return &fused_gemm_kernel<Walk, MT, SCAN, decltype(rows)::value>;
       else return &fused_gemm_wide_kernel<Walk, MT, SCAN>;
     }();
     if (L.total > 64 * 1024)
       if (int rc = allow_full_lds<kernel>()) return rc;
-    hipLaunchKernelGGL(kernel, dim3(g.n_tiles), dim3(g.threads), L.total, s, f, g, xp, m_rows, y, ldy, bias, partials,
-                       error);
+    hipLaunchKernelGGL(kernel, dim3(g.n_tiles), dim3(g.threads), L.total, s, f, g, source, m_rows, y, ldy, bias,
+                       partials, error);
     return GRF_OK;
   };
-  if (int rc = f.whole_range ? launch(std::integral_constant<int, grf::kScanAny>{})
-                             : launch(std::integral_constant<int, grf::kScanNoWholeRange>{}))
-    return rc;
+  if (int rc = launch_scan_and_rows<MT>(f.whole_range, source.pitch != 0, launch)) return rc;
   if (g.k_parts > 1)
     hipLaunchKernelGGL(gemm_sum_parts_kernel, dim3((m_rows * f.rows + 255) / 256), dim3(256), 0, s, partials, g.k_parts,
                        m_rows, f.rows, bias, y, ldy);
@@ -1504,26 +1568,24 @@ int launch_gemv_group(const char *who, const GroupSpec &spec, const uint16_t *x,
 }
 
 template <class Walk, int MT>
-int launch_gemm_group_rows(const FusedGroup &a, uint32_t m_rows, const uint4 *xp, int32_t *error, hipStream_t s) {
+int launch_gemm_group_rows(const FusedGroup &a, uint32_t m_rows, const GemmX &source, int32_t *error, hipStream_t s) {
   uint32_t lds = 0;
   for (uint32_t i = 0; i < a.n; ++i) lds = std::max(lds, GemmLdsLayout(a.f[i], a.g[i]).total);
   if (lds > 160 * 1024) return grf::set_error(GRF_UNSUPPORTED, "fused GEMM: LDS demand exceeds 160 KiB");
   bool whole = false;  // one member with a whole-range context: the scan that knows them, for all
   for (uint32_t i = 0; i < a.n; ++i) whole = whole || a.f[i].whole_range;
-  auto launch = [&](auto scan) -> int {
+  auto launch = [&](auto scan, auto rows) -> int {
     constexpr int SCAN = decltype(scan)::value;
     constexpr auto kernel = [] {
-      if constexpr (MT <= 4) return &fused_gemm_group_kernel<Walk, MT, SCAN>;
+      if constexpr (MT <= 4) return &fused_gemm_group_kernel<Walk, MT, SCAN, decltype(rows)::value>;
       else return &fused_gemm_wide_group_kernel<Walk, MT, SCAN>;
     }();
     if (lds > 64 * 1024)
       if (int rc = allow_full_lds<kernel>()) return rc;
-    hipLaunchKernelGGL(kernel, dim3(a.first_tile[a.n]), dim3(a.g[0].threads), lds, s, a, xp, m_rows, error);
+    hipLaunchKernelGGL(kernel, dim3(a.first_tile[a.n]), dim3(a.g[0].threads), lds, s, a, source, m_rows, error);
     return GRF_OK;
   };
-  if (int rc = whole ? launch(std::integral_constant<int, grf::kScanAny>{})
-                     : launch(std::integral_constant<int, grf::kScanNoWholeRange>{}))
-    return rc;
+  if (int rc = launch_scan_and_rows<MT>(whole, source.pitch != 0, launch)) return rc;
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return grf::set_error(GRF_LAUNCH_FAILED, std::string("fused GEMM: ") + hipGetErrorString(e));
   return GRF_OK;
@@ -1546,16 +1608,18 @@ int launch_gemm_group(const char *who, const GroupSpec &spec, const uint16_t *x,
   if (!workspace || ((uintptr_t)workspace & 15) || workspace_bytes < gemm_workspace_bytes(cols, m_rows))
     return grf::set_error(GRF_BAD_ARGUMENT, std::string(who) + ": workspace missing, misaligned or too small");
   uint4 *xp = static_cast<uint4 *>(workspace);
+  uint64_t weights = 0;
+  for (uint32_t i = 0; i < a.n; ++i) weights += (uint64_t)a.f[i].rows * cols;
   for (uint32_t m0 = 0; m0 < m_rows; m0 += kMaxRowsPerLaunch) {
     const uint32_t m = m_rows - m0 < kMaxRowsPerLaunch ? m_rows - m0 : kMaxRowsPerLaunch;
     FusedGroup part = a;
     for (uint32_t i = 0; i < a.n; ++i) part.y[i] = a.y[i] + (size_t)m0 * a.ldy[i];
-    if (x) launch_pack(x + (size_t)m0 * ldx, ldx, m, cols, gemm_tiles(m) * 16, xp, s);
+    const GemmX source = gemm_source(x ? x + (size_t)m0 * ldx : nullptr, ldx, m, cols, weights, xp, s);
     int rc;
-    if (m <= 16) rc = launch_gemm_group_rows<Walk, 1>(part, m, xp, error, s);
-    else if (m <= 32) rc = launch_gemm_group_rows<Walk, 2>(part, m, xp, error, s);
-    else if (m <= 64) rc = launch_gemm_group_rows<Walk, 4>(part, m, xp, error, s);
-    else rc = launch_gemm_group_rows<Walk, 8>(part, m, xp, error, s);
+    if (m <= 16) rc = launch_gemm_group_rows<Walk, 1>(part, m, source, error, s);
+    else if (m <= 32) rc = launch_gemm_group_rows<Walk, 2>(part, m, source, error, s);
+    else if (m <= 64) rc = launch_gemm_group_rows<Walk, 4>(part, m, source, error, s);
+    else rc = launch_gemm_group_rows<Walk, 8>(part, m, source, error, s);
     if (rc) return rc;
   }
   return GRF_OK;
