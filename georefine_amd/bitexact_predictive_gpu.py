@@ -47,9 +47,13 @@ def _checkpoints(stream, ctx, freq, vocab, stride):
     return states, offsets, symbols
 
 
-# Sixteen bin contexts share the lookup bytes: 1 KiB each measured faster at one activation row
-# than 2 KiB (-10 %: more workgroups fit a CU; equal on the decode and GEMM sinks).
-_LUT_BUDGET = int(os.environ.get("GEOREFINE_FUSED_LUT_BYTES", 16 * 1024))
+# Sixteen bin contexts share the lookup bytes.  A wave scans on whenever one of its 64 lanes meets
+# a bucket's minority symbol: 35 % of the steps with 1 KiB per context, 21 % with 2 KiB, 12 % with
+# 4 KiB.  At 64 KiB one workgroup of sixteen waves has a compute unit to itself instead of two of
+# twelve, and still wins throughout (4096 x 4096, 16 / 32 / 64 KiB in all: decode 32.3 / 26.5 /
+# 27.4 us, one row 31.0 / 25.7 / 26.9, 16 rows 39.6 / 37.9 / 37.5, 96 rows 59.2 / 61.6 / 44.7;
+# 512 x 1024, one row 12.1 / 12.1 / 10.6, 64 rows 19.3 / 19.6 / 12.9).
+_LUT_BUDGET = int(os.environ.get("GEOREFINE_FUSED_LUT_BYTES", 64 * 1024))
 
 
 def _word_image(main):
