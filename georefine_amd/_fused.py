@@ -364,7 +364,15 @@ def choose_gemm_tiling(spr, class_rows, piece_cap_fn, lds_fn, cus=256, seg_len=6
         per_cu = max(1, min(GEMM_WAVES_PER_SIMD // per_simd, MAX_LDS // lds))
         slots = cus * per_cu
         rounds = -(-(tile_counts[r] * k) // slots)
-        r_used = r if forced else _spread_rows(tile_counts, r, rounds * slots // k, floor=16 * (row_blocks - 1) + 1)
+        # Spread over idle workgroup slots, except a single block of rows where one workgroup has a
+        # compute unit to itself, or where whole blocks take half of the slots at most: the block's
+        # wave issues the same for fewer rows, and every further workgroup copies the tables (256
+        # tiles of 13 or 15 rows against 192 and 256 of 16, 20 activation rows: 1024 x 5120 17.2
+        # -> 16.2 us, 901 x 8192 20.1 -> 19.2; 257 tiles of one row against 17: 257 x 560 10.7 ->
+        # 8.9).  Where they pay: 3000 x 3072, 512 tiles of 12 rows 21.2, 384 of 16 21.7.
+        whole = row_blocks == 1 and (per_cu == 1 or 2 * tile_counts[r] * k <= slots)
+        r_used = r if forced or whole else _spread_rows(tile_counts, r, rounds * slots // k,
+                                                        floor=16 * (row_blocks - 1) + 1)
         tiles_used = tile_counts[r_used] * k
         slabs_each = -(-n_slabs // k)
         # work = lane-steps; capacity = every wave slot of every round for the whole walk
