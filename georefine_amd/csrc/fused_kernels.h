@@ -1060,14 +1060,14 @@ __device__ __forceinline__ void gemm_load_rows(uint4 (&xa)[MT], const GemmX &x, 
 #endif
 }
 
-template <int MT>
-__device__ __forceinline__ void gemm_contract(float4v (&acc)[MT], const uint4 (&xa)[MT], const uint32_t (&w)[4]) {
+template <int FIRST, int MT, int XT>
+__device__ __forceinline__ void gemm_contract(float4v (&acc)[MT], const uint4 (&xa)[XT], const uint32_t (&w)[4]) {
 #if defined(__HIP_DEVICE_COMPILE__)
   const uint4 wv = make_uint4(w[0], w[1], w[2], w[3]);
   const bf16x8_t b = __builtin_bit_cast(bf16x8_t, wv);
 #pragma unroll
-  for (int j = 0; j < MT; ++j)
-    acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, xa[j]), b, acc[j], 0, 0, 0);
+  for (int j = 0; j < XT; ++j)
+    acc[FIRST + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, xa[j]), b, acc[FIRST + j], 0, 0, 0);
 #else
   (void)acc;
   (void)xa;
@@ -1083,7 +1083,9 @@ __device__ __forceinline__ void gemm_contract(float4v (&acc)[MT], const uint4 (&
 // parts in order, then the bias, and rounds.  That lets a matrix with few rows be cut along K
 // until its tiles fill the machine with full blocks of sixteen rows, in a fixed order of
 // additions (the tiling is the matrix's, whatever the batch).
-template <class Walk, int MT, int SCAN, bool ROWS>
+// XT: activation tiles whose operands a lane holds at a time: all of them, loaded a half group
+// ahead, or two, the other six loaded and contracted in turn (fused_gemm_shared_kernel).
+template <class Walk, int MT, int SCAN, bool ROWS, int XT = MT>
 __device__ __forceinline__ void fused_gemm_body(uint8_t *lds, const grf_bctx_fused &f, const grf_fused_tiling &g,
                                                 const GemmX &x, uint32_t m_rows, uint16_t *y, uint32_t ldy,
                                                 const uint16_t *bias, float *partials, int32_t *error,
@@ -1186,9 +1188,9 @@ __device__ __forceinline__ void fused_gemm_body(uint8_t *lds, const grf_bctx_fus
     const bool feeds = p4 < nseg;
     // bytes from one 8-column chunk to the next
     const uint32_t x_step = feeds ? (ROWS ? 16u : m_pad * 16) : 0;
-    auto load_x = [&](uint4 (&to)[MT], uint32_t at) {
-      if constexpr (ROWS) gemm_load_rows<MT>(to, x, at);
-      else gemm_load_x<MT>(to, static_cast<const uint4 *>(x.data), at);
+    auto load_x = [&](auto &to, uint32_t at) {
+      if constexpr (ROWS) gemm_load_rows(to, x, at);
+      else gemm_load_x(to, static_cast<const uint4 *>(x.data), at);
     };
     // (the lane's number is worked out again here rather than kept in a register over the walks)
     uint32_t ln = __lane_id();
@@ -1197,20 +1199,33 @@ __device__ __forceinline__ void fused_gemm_body(uint8_t *lds, const grf_bctx_fus
 #endif
     uint32_t xl = ROWS ? (feeds ? (ln % 16) * x.pitch + col0 * 2 : x.bytes)
                        : ((feeds ? col0 / 8 : K / 8) * m_pad + ln % 16) * 16;
-    uint4 xa[MT];
-    load_x(xa, xl);
     // (zeros for the lanes that do not walk, once: a walking lane overwrites its own)
     uint32_t words[4] = {0u, 0u, 0u, 0u};
+    uint4 xa[XT];
+    load_x(xa, xl);
+    auto contract = [&]() {
+      gemm_contract<0>(acc, xa, words);
+      auto next = [&](auto first) {  // (XT < MT only)
+        load_x(xa, xl + decltype(first)::value * 256u);
+        gemm_contract<decltype(first)::value>(acc, xa, words);
+      };
+      if constexpr (XT < MT) {
+        static_assert(MT == 4 * XT && !ROWS);
+        next(std::integral_constant<int, XT>{});
+        next(std::integral_constant<int, 2 * XT>{});
+        next(std::integral_constant<int, 3 * XT>{});
+      }
+    };
     for (uint32_t t = 0; t < S; t += 16) {
       if (active) {
         w.begin16(t, S);
         w.template half<0, SCAN>(q, words);
       }
-      gemm_contract<MT>(acc, xa, words);
+      contract();
       xl += x_step;
       load_x(xa, xl);
       if (active) w.template half<1, SCAN>(q, words);
-      gemm_contract<MT>(acc, xa, words);
+      contract();
       xl += x_step;
       load_x(xa, xl);
     }
@@ -1282,6 +1297,35 @@ __global__ __launch_bounds__(grf::kFusedMaxThreads) void fused_gemm_wide_kernel(
   fused_gemm_body<Walk, MT, SCAN, false>(lds, f, g, x, m_rows, y, ldy, bias, partials, error, blockIdx.x);
 }
 
+// Eight activation tiles where two workgroups can share a compute unit (shares_units): 80 registers,
+// six waves per SIMD, by holding the operands of two tiles at a time; ten waves more are resident in
+// return for waiting on the L2 three times a half group.  128 rows: q+k+v 6144 + 1024 + 1024 x 5120
+// 68.1 -> 59.5 us, gate+up 251 -> 234; 2048 x 5120 at 100 rows 34.1 -> 30.2.
+template <class Walk, int MT, int SCAN>
+__global__ __launch_bounds__(grf::kFusedMaxThreads) __attribute__((amdgpu_waves_per_eu(6))) void fused_gemm_shared_kernel(
+    grf_bctx_fused f, grf_fused_tiling g, GemmX x, uint32_t m_rows, uint16_t *y, uint32_t ldy, const uint16_t *bias,
+    float *partials, int32_t *error) {
+  extern __shared__ __align__(16) uint8_t lds[];
+  fused_gemm_body<Walk, MT, SCAN, false, 2>(lds, f, g, x, m_rows, y, ldy, bias, partials, error, blockIdx.x);
+}
+
+template <class Walk, int MT, int SCAN>
+__global__ __launch_bounds__(grf::kFusedMaxThreads) __attribute__((amdgpu_waves_per_eu(6))) void fused_gemm_shared_group_kernel(
+    FusedGroup a, GemmX x, uint32_t m_rows, int32_t *error) {
+  extern __shared__ __align__(16) uint8_t lds[];
+  const uint32_t i = group_member(a, blockIdx.x);
+  fused_gemm_body<Walk, MT, SCAN, false, 2>(lds, a.f[i], a.g[i], x, m_rows, a.y[i], a.ldy[i], a.bias[i], nullptr, error,
+                                            blockIdx.x - a.first_tile[i]);
+}
+
+// Whether a launch above four activation tiles takes the kernels that let two workgroups share a
+// compute unit: there have to be more workgroups than units, of ten waves at most (twelve gain
+// nothing: 5120 x 6144 at 100 rows 69.7 us, 70.9 shared), whose LDS fits twice.  Workgroups that
+// have a unit to themselves only lose by the waits: 4096 x 4096 29.5 -> 33.9, 3500 x 1024 16.7 -> 19.5.
+inline bool shares_units(uint32_t tiles, uint32_t threads, uint32_t lds) {
+  return tiles > 256 && threads <= 640 && lds <= 79 * 1024;
+}
+
 template <class Walk, int MT, int SCAN, bool ROWS>
 __global__ __launch_bounds__(grf::kFusedMaxThreads) __attribute__((amdgpu_waves_per_eu(6))) void fused_gemm_group_kernel(
     FusedGroup a, GemmX x, uint32_t m_rows, int32_t *error) {
@@ -1336,6 +1380,9 @@ inline GemmX gemm_source(const uint16_t *x, uint32_t ldx, uint32_t m_rows, uint3
   return GemmX{xp, 0, 0};
 }
 
+template <auto Kernel>
+struct KernelOf { static constexpr auto value = Kernel; };
+
 // launch(scan, rows) for the scan the frames need and the activations' form
 template <int MT, class Launch>
 int launch_scan_and_rows(bool whole_range, bool rows, const Launch &launch) {
@@ -1355,15 +1402,17 @@ int launch_gemm_rows(const grf_bctx_fused &f, const grf_fused_tiling &g, const u
   const GemmX source = gemm_source(x, ldx, m_rows, f.cols, (uint64_t)f.rows * f.cols, xp, s);
   auto launch = [&](auto scan, auto rows) -> int {
     constexpr int SCAN = decltype(scan)::value;
-    constexpr auto kernel = [] {
-      if constexpr (MT <= 4) return &fused_gemm_kernel<Walk, MT, SCAN, decltype(rows)::value>;
-      else return &fused_gemm_wide_kernel<Walk, MT, SCAN>;
-    }();
-    if (L.total > 64 * 1024)
-      if (int rc = allow_full_lds<kernel>()) return rc;
-    hipLaunchKernelGGL(kernel, dim3(g.n_tiles), dim3(g.threads), L.total, s, f, g, source, m_rows, y, ldy, bias,
-                       partials, error);
-    return GRF_OK;
+    auto with = [&](auto which) -> int {
+      constexpr auto kernel = decltype(which)::value;
+      if (L.total > 64 * 1024)
+        if (int rc = allow_full_lds<kernel>()) return rc;
+      hipLaunchKernelGGL(kernel, dim3(g.n_tiles), dim3(g.threads), L.total, s, f, g, source, m_rows, y, ldy, bias,
+                         partials, error);
+      return GRF_OK;
+    };
+    if constexpr (MT <= 4) return with(KernelOf<&fused_gemm_kernel<Walk, MT, SCAN, decltype(rows)::value>>{});
+    else if (shares_units(g.n_tiles, g.threads, L.total)) return with(KernelOf<&fused_gemm_shared_kernel<Walk, MT, SCAN>>{});
+    else return with(KernelOf<&fused_gemm_wide_kernel<Walk, MT, SCAN>>{});
   };
   if (int rc = launch_scan_and_rows<MT>(f.whole_range, source.pitch != 0, launch)) return rc;
   if (g.k_parts > 1)
@@ -1576,14 +1625,16 @@ int launch_gemm_group_rows(const FusedGroup &a, uint32_t m_rows, const GemmX &so
   for (uint32_t i = 0; i < a.n; ++i) whole = whole || a.f[i].whole_range;
   auto launch = [&](auto scan, auto rows) -> int {
     constexpr int SCAN = decltype(scan)::value;
-    constexpr auto kernel = [] {
-      if constexpr (MT <= 4) return &fused_gemm_group_kernel<Walk, MT, SCAN, decltype(rows)::value>;
-      else return &fused_gemm_wide_group_kernel<Walk, MT, SCAN>;
-    }();
-    if (lds > 64 * 1024)
-      if (int rc = allow_full_lds<kernel>()) return rc;
-    hipLaunchKernelGGL(kernel, dim3(a.first_tile[a.n]), dim3(a.g[0].threads), lds, s, a, source, m_rows, error);
-    return GRF_OK;
+    auto with = [&](auto which) -> int {
+      constexpr auto kernel = decltype(which)::value;
+      if (lds > 64 * 1024)
+        if (int rc = allow_full_lds<kernel>()) return rc;
+      hipLaunchKernelGGL(kernel, dim3(a.first_tile[a.n]), dim3(a.g[0].threads), lds, s, a, source, m_rows, error);
+      return GRF_OK;
+    };
+    if constexpr (MT <= 4) return with(KernelOf<&fused_gemm_group_kernel<Walk, MT, SCAN, decltype(rows)::value>>{});
+    else if (shares_units(a.first_tile[a.n], a.g[0].threads, lds)) return with(KernelOf<&fused_gemm_shared_group_kernel<Walk, MT, SCAN>>{});
+    else return with(KernelOf<&fused_gemm_wide_group_kernel<Walk, MT, SCAN>>{});
   };
   if (int rc = launch_scan_and_rows<MT>(whole, source.pitch != 0, launch)) return rc;
   hipError_t e = hipGetLastError();
