@@ -398,13 +398,13 @@ def _walk(info, stride, failed, beside):
     if stride:
         states, offsets = (np.empty(-(-words.size // stride), dtype=np.uint32) for _ in range(2))
         info["main_states"], info["main_offsets"] = states, offsets
-    # (a thread hashes behind the walk; without one the hash follows it)
-    digest = beside.run(_sha_following, words, progress) if beside.pool is not None else None
-    streams = [np.frombuffer(s, dtype=np.uint8) if len(s) else np.zeros(1, np.uint8)
-               for s in (info["main_stream"], info["residual_stream"])]
     p = lambda a, t: _native.ptr(a, t) if a is not None else ctypes.POINTER(t)()
-    status = -1
+    digest, status = None, -1
     try:
+        if beside.pool is not None:  # a thread hashes behind the walk; without one the hash follows it
+            digest = beside.run(_sha_following, words, progress)
+        streams = [np.frombuffer(s, dtype=np.uint8) if len(s) else np.zeros(1, np.uint8)
+                   for s in (info["main_stream"], info["residual_stream"])]
         status = _lib().grf_bctx_words(
             p(streams[0], ctypes.c_uint8), len(info["main_stream"]), r, c, p(info["rows"], ctypes.c_uint8),
             p(info["columns"], ctypes.c_uint8), info["nr"], info["nc"], p(info["main_freq"], ctypes.c_uint32), stride,
@@ -412,7 +412,7 @@ def _walk(info, stride, failed, beside):
             len(info["residual_stream"]), p(info.get("residual_freq"), ctypes.c_uint32), p(words, ctypes.c_uint16),
             p(progress, ctypes.c_uint64))
     finally:
-        if status:  # whatever went wrong: nothing follows the walk any more
+        if status:  # whatever went wrong, from the thread's start on: nothing follows the walk any more
             progress[0] = np.uint64(0xFFFFFFFFFFFFFFFF)
     if status:
         raise CodecError("invalid raw residual stream" if status == 33 else failed.format(status % 16))

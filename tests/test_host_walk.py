@@ -1,5 +1,9 @@
 """The host coder's walks against the oracle where their cuts fall: runs at row ends and marks, the
 last symbols of a stream, contexts that are one symbol, symbols behind a bucket's boundary."""
+import subprocess
+import sys
+from pathlib import Path
+
 import numpy as np
 import pytest
 
@@ -32,3 +36,35 @@ def test_walks_match_the_oracle(oracle, kind, rows, cols):
             got = checkpoints(stream, table, rc, cc, (rows, cols), 4, 4, stride, main)
             want = oracle.bcx_checkpoint(stream, table, rc, cc, rows, cols, 4, 4, stride, main)
             assert all(np.array_equal(a, b) for a, b in zip(got, want))
+
+
+_NO_MEMORY_IN_THE_WALK = """
+import sys
+import numpy as np
+from georefine_amd import bitexact_context_codec as codec
+rng = np.random.default_rng(0)
+frame = codec.encode((rng.integers(0, 4, (600, 640)) << 7 | rng.integers(0, 64, (600, 640))).astype(np.uint16))
+assert frame[5] != 1 and len(frame) >= codec.Beside.BESIDE_FROM  # hashed beside the walk
+
+class Numpy:  # numpy, but stream views made inside the walk find no memory
+    def __getattr__(self, name):
+        return getattr(np, name)
+    def frombuffer(self, *args, **kw):
+        if "_walk" in (sys._getframe(1).f_code.co_name, sys._getframe(2).f_code.co_name):
+            raise MemoryError
+        return np.frombuffer(*args, **kw)
+
+codec.np = Numpy()
+try:
+    codec.decode(frame)
+except MemoryError:
+    print("raised")
+"""
+
+
+def test_an_exception_beside_the_hashing_thread_reaches_the_caller():
+    """Whatever is raised once the thread that follows the walk may run ends that thread too (in a
+    process of its own: a thread left behind would keep this one from ending)."""
+    done = subprocess.run([sys.executable, "-c", _NO_MEMORY_IN_THE_WALK], cwd=Path(__file__).resolve().parent.parent,
+                          capture_output=True, text=True, timeout=60)
+    assert done.stdout == "raised\n", done.stderr[-2000:]
