@@ -364,11 +364,17 @@ def _sha_following(words, progress):
     return sha.digest()
 
 
-def read_words(frame, stride=0, failed="rANS decode failed ({})"):
+def _decode_failed(status):
+    """The message of a failed walk as ``bcx_decode`` reports it: 3 internal, 2 anything else."""
+    return f"rANS decode failed ({3 if status in (5, 6) else 2})"
+
+
+def read_words(frame, stride=0, failed=_decode_failed):
     """A whole frame decoded and checked against its own checksum: the dict of ``parse`` with
     ``words`` (one-dimensional), ``words_digest`` and ``frame_sha256``; with ``stride`` also
     the main stream's index, ``main_states`` and ``main_offsets``.  The walk runs on the caller's
-    thread (and one in the library); the frame and the finished words are hashed beside it."""
+    thread (and one in the library); the frame and the finished words are hashed beside it.
+    ``failed``: the message of a walk's status (``grf_bctx_words``, whichever stream's)."""
     frame = _frame_bytes(frame)
     with Beside(len(frame)) as beside:
         digests = beside.run(_frame_digests, frame)
@@ -415,7 +421,7 @@ def _walk(info, stride, failed, beside):
         if status:  # whatever went wrong, from the thread's start on: nothing follows the walk any more
             progress[0] = np.uint64(0xFFFFFFFFFFFFFFFF)
     if status:
-        raise CodecError("invalid raw residual stream" if status == 33 else failed.format(status % 16))
+        raise CodecError("invalid raw residual stream" if status == 33 else failed(status % 16))
     info["words_digest"] = digest if digest is not None else hashlib.sha256(words).digest()
 
 

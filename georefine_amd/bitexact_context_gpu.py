@@ -72,7 +72,7 @@ def index_frame(frame: bytes, stride: int = 1024, *, fused_segment=None, raw6_re
     repack = raw6_residual and mode == 128
     fine = fused_segment if fused_segment and (mode == 0 or repack) else None
     one_walk = fine is not None and stride % fine == 0  # every stride // fine-th entry of the fine index is the coarse one
-    info = base.read_words(frame, fine if one_walk else stride, "checkpoint validation failed ({})")
+    info = base.read_words(frame, fine if one_walk else stride, "checkpoint validation failed ({})".format)
     r, c = info["shape"]
     out = {"shape": (r, c), "mode": mode, "nr": info["nr"], "nc": info["nc"], "stride": stride,
            "source_sha256": info["digest"].hex(), "frame_sha256": info["frame_sha256"], "frame_bytes": len(frame)}

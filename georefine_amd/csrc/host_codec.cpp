@@ -816,7 +816,7 @@ int grf_bctx_words(const uint8_t *stream, size_t stream_bytes, uint32_t rows, ui
           Behind progress_behind{&behind, &words_done, words, fields.data()};
           const Walk w = walk_stream(residual, residual_bytes, n, residual_tables, contexts, unmarked, fields.data(),
                                      progress_behind);
-          second = w == Walk::ok || w == Walk::abandoned ? 0 : w == Walk::dead_context ? 18 : 19;
+          second = w == Walk::ok || w == Walk::abandoned ? 0 : residual_bytes < 4 ? 17 : w == Walk::dead_context ? 18 : 19;
           words_done.publish(w == Walk::ok ? n : Counter::kGaveUp);
         };
 

@@ -65,7 +65,7 @@ int grf_bctx_join(const uint16_t *main_sym, const uint16_t *res_sym, uint64_t n,
  * and the recombination): the main stream walked, its index recorded before every stride-th symbol (stride 0:
  * none), and the words made of its symbols and the packed 6-bit fields (residual_freq null) or the conditional
  * stream.  `progress` (may be null) counts finished words while the call runs, for a thread that consumes them;
- * it ends as all ones when the call fails.  1 arguments, 2 main tables/contexts, 3 main stream, 18/19 the
+ * it ends as all ones when the call fails.  1 arguments, 2 main tables/contexts, 3 main stream, 17/18/19 the
  * same of the conditional stream, 33 packed fields, 5/6 internal; states/offsets/words hold no result then. */
 int grf_bctx_words(const uint8_t *stream, size_t stream_bytes, uint32_t rows, uint32_t cols, const uint8_t *rc,
                    const uint8_t *cc, uint32_t nr, uint32_t nc, const uint32_t *freq, uint32_t stride, uint32_t *states,

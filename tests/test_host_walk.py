@@ -1,5 +1,6 @@
 """The host coder's walks against the oracle where their cuts fall: runs at row ends and marks, the
 last symbols of a stream, contexts that are one symbol, symbols behind a bucket's boundary."""
+import hashlib
 import subprocess
 import sys
 from pathlib import Path
@@ -8,7 +9,7 @@ import numpy as np
 import pytest
 
 from georefine_amd import bitexact_context_codec as codec
-from georefine_amd.bitexact_context_gpu import checkpoints
+from georefine_amd.bitexact_context_gpu import checkpoints, index_frame
 
 
 def _words(kind, rows, cols):
@@ -68,3 +69,73 @@ def test_an_exception_beside_the_hashing_thread_reaches_the_caller():
     done = subprocess.run([sys.executable, "-c", _NO_MEMORY_IN_THE_WALK], cwd=Path(__file__).resolve().parent.parent,
                           capture_output=True, text=True, timeout=60)
     assert done.stdout == "raised\n", done.stderr[-2000:]
+
+
+def _one_stream_after_the_other(frame, index):
+    """What a frame's walk reports, stream by stream through the entry points the reference binds."""
+    info = codec.parse(frame)
+    (r, c), nr, nc = info["shape"], info["nr"], info["nc"]
+    tables = info["main_freq"], info.get("residual_freq")
+    classes = info["rows"], info["columns"]
+    try:
+        main = (checkpoints(info["main_stream"], tables[0], *classes, (r, c), nr, nc, 1024)[2] if index else
+                codec._decode_kind(codec._lib(), info["main_stream"], tables[0].tobytes(), *classes, r, c, nr, nc, 0))
+        if tables[1] is None:
+            residual = codec._unpack6(codec._lib(), info["residual_stream"], r * c)
+        elif index:
+            residual = checkpoints(info["residual_stream"], tables[1], *classes, (r, c), nr, nc, 1024, main)[2]
+        else:
+            residual = codec._decode_kind(codec._lib(), info["residual_stream"], tables[1].tobytes(), *classes, r, c, nr,
+                                          nc, 1, main)
+    except codec.CodecError as exc:
+        return str(exc)
+    words = codec.recombine(main, residual)
+    if hashlib.sha256(words.tobytes()).digest() != info["digest"]:
+        return "indexed source checksum mismatch" if index else "decoded checksum mismatch"
+    return words.reshape(r, c)
+
+
+def _with_streams(frame, main=None, residual=None):
+    """The frame with another stream or two, sealed with a checksum that holds."""
+    header = list(codec.HEADER.unpack_from(frame))
+    at = codec.HEADER.size + header[7] + header[8]
+    streams = [frame[at:at + header[9]], frame[at + header[9]:at + header[9] + header[10]]]
+    for i, change in enumerate((main, residual)):
+        if change is not None:
+            streams[i] = change(streams[i])
+            header[9 + i] = len(streams[i])
+    return codec._sealed([codec.HEADER.pack(*header), frame[codec.HEADER.size:at], *streams])
+
+
+def _flipped(at):
+    return lambda s: s[:at] + bytes([s[at] ^ 0x55]) + s[at + 1:]
+
+
+_DAMAGE = {
+    "whole": None, "head": _flipped(3), "early": _flipped(9), "middle": lambda s: _flipped(len(s) // 2)(s),
+    "last": lambda s: _flipped(len(s) - 1)(s), "cut": lambda s: s[:-3], "half": lambda s: s[:len(s) // 2],
+    "longer": lambda s: s + b"\0\0", "no head": lambda s: s[:3], "empty": lambda s: b"",
+}
+
+
+@pytest.mark.parametrize("rows,cols", [(37, 210), (700, 511)])  # the second: two threads in the library, one beside it
+@pytest.mark.parametrize("mode", [0, 128])
+def test_damaged_streams_are_reported_as_by_one_walk_after_the_other(rows, cols, mode):
+    rng = np.random.default_rng(rows + mode)
+    fields = rng.integers(0, 64 if mode == 0 else 3, (rows, cols))
+    main = rng.geometric(0.1, (rows, cols)) % 60
+    words = (main << 5 | (fields & 31) | (fields & 32) << 10).astype(np.uint16)
+    frame = codec.encode(words, residual="raw6" if mode == 0 else "auto")
+    assert frame[5] == mode and (words.size >= 1 << 18) == (rows > 100)
+    for stream in ("main", "residual"):
+        for name, damage in _DAMAGE.items():
+            broken = _with_streams(frame, **{stream: damage})
+            for index in (False, True):
+                want = _one_stream_after_the_other(broken, index)
+                try:
+                    got = codec.decode(broken) if not index else index_frame(broken, 1024)
+                except codec.CodecError as exc:
+                    assert str(exc) == want, (stream, name, index)
+                else:
+                    assert isinstance(want, np.ndarray), (stream, name, index)
+                    assert index or np.array_equal(got, want)
