@@ -766,8 +766,10 @@ int grf_bctx_words(const uint8_t *stream, size_t stream_bytes, uint32_t rows, ui
   const int status = guarded(
       [&]() -> int {
         if (!stream || !rc || !cc || !freq || !rows || !cols || !nr || !nc || nr > 64 || nc > 16 || !residual || !words ||
-            stream_bytes < 4 || stream_bytes > std::numeric_limits<uint32_t>::max() || (stride && (!states || !offsets)))
+            stream_bytes < 4)
           return 1;
+        // (only the index has to hold its offsets in 32 bits)
+        if (stride && (!states || !offsets || stream_bytes > std::numeric_limits<uint32_t>::max())) return 1;
         if (std::any_of(rc, rc + rows, [&](uint8_t v) { return v >= nr; })) return 1;
         if (std::any_of(cc, cc + cols, [&](uint8_t v) { return v >= nc; })) return 1;
         const uint64_t n = (uint64_t)rows * cols;

@@ -1,5 +1,6 @@
 """The host coder's walks against the oracle where their cuts fall: runs at row ends and marks, the
 last symbols of a stream, contexts that are one symbol, symbols behind a bucket's boundary."""
+import ctypes
 import hashlib
 import subprocess
 import sys
@@ -8,6 +9,7 @@ from pathlib import Path
 import numpy as np
 import pytest
 
+from georefine_amd import _native
 from georefine_amd import bitexact_context_codec as codec
 from georefine_amd.bitexact_context_gpu import checkpoints, index_frame
 
@@ -139,3 +141,21 @@ def test_damaged_streams_are_reported_as_by_one_walk_after_the_other(rows, cols,
                 else:
                     assert isinstance(want, np.ndarray), (stream, name, index)
                     assert index or np.array_equal(got, want)
+
+
+def test_a_stream_of_any_length_is_decoded_and_one_past_32_bits_is_not_indexed():
+    """The index holds byte offsets of 32 bits; words alone need none.  (The length is claimed, not
+    allocated: the walk ends with its last symbol, finds the stream's end elsewhere and says so.)"""
+    n = 64
+    buffer = np.full(4 * n + 64, 0x80, dtype=np.uint8)
+    classes, freq = np.zeros(n, dtype=np.uint8), np.zeros(1024, dtype=np.uint32)
+    freq[:2] = 32768
+    packed, words = np.zeros(n * 6 // 8, dtype=np.uint8), np.zeros(n, dtype=np.uint16)
+    states, offsets = np.zeros(n, dtype=np.uint32), np.zeros(n, dtype=np.uint32)
+    p = lambda a, t: _native.ptr(a, t)
+    for stride, status in ((0, 3), (1, 1)):
+        assert codec._lib().grf_bctx_words(
+            p(buffer, ctypes.c_uint8), (1 << 32) + 5, 1, n, p(classes, ctypes.c_uint8), p(classes, ctypes.c_uint8), 1, 1,
+            p(freq, ctypes.c_uint32), stride, p(states, ctypes.c_uint32), p(offsets, ctypes.c_uint32),
+            p(packed, ctypes.c_uint8), packed.size, ctypes.POINTER(ctypes.c_uint32)(), p(words, ctypes.c_uint16),
+            ctypes.POINTER(ctypes.c_uint64)()) == status
