@@ -63,7 +63,19 @@ def index_frame(frame: bytes, stride: int = 1024, *, fused_segment=None, raw6_re
     ``raw6_residual``: a mode-128 frame's residual section is validated, decoded and
     re-packed into the 6-bit raw form (the form the encoder itself emits for mode 0,
     GCR/bitexact_context_ans.cpp:328-345); the result then carries ``resident_mode`` 0 and
-    no residual index.  The main stream's bytes are never altered."""
+    no residual index.  The main stream's bytes are never altered.
+
+    The arrays are the caller's own: writable, and none of them keeps the frame alive."""
+    out = _index_views(frame, stride, fused_segment, raw6_residual)
+    for name in ("main_stream", "residual_stream"):
+        if name in out:
+            out[name] = out[name].copy()
+    return out
+
+
+def _index_views(frame, stride, fused_segment, raw6_residual):
+    """``index_frame`` with the two streams as read-only views (of the frame; a re-packed residual
+    section: of its own bytes), for a caller that makes arrays of its own from them."""
     if not isinstance(stride, int) or not 1 <= stride <= 65536:
         raise base.CodecError("invalid checkpoint stride")
     if len(frame) < base.HEADER.size + 32:
@@ -99,7 +111,6 @@ def index_frame(frame: bytes, stride: int = 1024, *, fused_segment=None, raw6_re
         rf = info["residual_freq"]
         out.update(zip(("residual_freq", "residual_states", "residual_offsets"),
                        (rf, *checkpoints(residual, rf, rows, columns, (r, c), info["nr"], info["nc"], stride, main)[:2])))
-    # (views of the frame: nothing here writes to the streams)
     out.update(rows=rows, columns=columns, main_freq=sf, main_stream=np.frombuffer(info["main_stream"], dtype=np.uint8),
                main_states=states, main_offsets=offsets, residual_stream=np.frombuffer(residual, dtype=np.uint8))
     return out
@@ -243,7 +254,7 @@ class HipContextTensor:
                 segment = _fused.choose_segment(header[6], fused_segment, rows=header[5])
             except _fused.FusedUnsupported:
                 segment = None
-        indexed = index_frame(frame, stride, fused_segment=segment, raw6_residual=segment is not None)
+        indexed = _index_views(frame, stride, segment, segment is not None)
         plan, reason = None, "disabled" if not fused else "frame mode or geometry"
         if "fused_states" in indexed:
             try:
@@ -279,6 +290,9 @@ class HipContextTensor:
                 states = _fused.order_index(states, rows_, spr_, block, position, held)
                 offsets = _fused.order_index(offsets, rows_, spr_, block, position, held)
             indexed.update(fused_seg_state=states, fused_seg_offset=offsets, fused_lut=plan.lut, fused_tab=plan.tab)
+        for name in ("main_stream", "residual_stream"):  # what is still a view: callers may keep the result for long
+            if name in indexed and not indexed[name].flags.writeable:
+                indexed[name] = indexed[name].copy()
         return {"indexed": indexed, "plan": plan, "reason": reason, "stride": stride, "fused": fused,
                 "main_bytes": main_bytes, "raw6_segment": raw6_segment, "raw6_block": raw6_block}
 
@@ -316,8 +330,7 @@ class HipContextTensor:
         self._raw6_segment, self._raw6_block = prepared["raw6_segment"], prepared["raw6_block"]
         for name, array in indexed.items():
             if isinstance(array, np.ndarray):
-                array = np.ascontiguousarray(array) if array.flags.writeable else array.copy()  # (torch wants it writable)
-                self.buffers[name] = torch.from_numpy(array).to(self.device)
+                self.buffers[name] = torch.from_numpy(np.ascontiguousarray(array)).to(self.device)
         for name in ("main", "residual"):
             if name + "_freq" in indexed:
                 cum = _tables.cumulative(indexed[name + "_freq"])

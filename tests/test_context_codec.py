@@ -10,7 +10,7 @@ import pytest
 from conftest import SPECIAL_WORDS, weight_like
 from georefine_amd import _native
 from georefine_amd import bitexact_context_codec as codec
-from georefine_amd.bitexact_context_gpu import checkpoints, index_frame
+from georefine_amd.bitexact_context_gpu import HipContextTensor, checkpoints, index_frame
 
 
 def _ptr(a, t):
@@ -39,6 +39,28 @@ def test_index_frame_raw_and_checksum_rejection():
         index_frame(frame[:-1] + bytes([frame[-1] ^ 1]))
     with pytest.raises(codec.CodecError, match="stride"):
         index_frame(frame, 0)
+
+
+@pytest.mark.parametrize("words", [np.full((64, 128), 0x3F80, dtype=np.uint16), np.arange(64 * 128, dtype=np.uint16).reshape(64, 128) % 97])
+def test_indexed_arrays_are_the_callers_own(words):
+    """Writable, and not views that keep the whole frame (or anything else) alive."""
+    def root(a):
+        while isinstance(a, np.ndarray) and a.base is not None:
+            a = a.base
+        return a
+
+    for mode, residual in ((128, "auto"), (0, "raw6")):
+        frame = codec.encode(words, residual=residual)
+        assert frame[5] == mode
+        made = [index_frame(frame, 1024), index_frame(frame, 1024, fused_segment=64, raw6_residual=True),
+                HipContextTensor.host_prepare(frame)["indexed"], HipContextTensor.host_prepare(frame, fused=False)["indexed"]]
+        for indexed in made:
+            for name, a in indexed.items():
+                if isinstance(a, np.ndarray):
+                    assert a.flags.writeable and isinstance(root(a), np.ndarray), name
+        made[0]["main_stream"][:] = 0
+        made[0]["residual_stream"][:] = 0
+        assert codec.decode(frame).tobytes() == words.tobytes()
 
 
 def test_fused_index_is_the_fine_index_and_mode128_residual_is_repacked():
