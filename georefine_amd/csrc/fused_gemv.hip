@@ -172,7 +172,6 @@ int grf_bctx_fused_decode(const grf_bctx_fused *frame, const grf_fused_tiling *t
   if (!frame || !tiling || !out || !error)
     return grf::set_error(GRF_BAD_ARGUMENT, "grf_bctx_fused_decode: null argument");
   if (int rc = grf::check_fused_frame(*frame, *tiling, "grf_bctx_fused_decode", grf::kStoreTiling)) return rc;
-  if (((uintptr_t)out & 15)) return grf::set_error(GRF_BAD_ARGUMENT, "grf_bctx_fused_decode: out must be 16-byte aligned");
   if (tiling->scheme == GRF_TILE_WAVES)
     return grf::launch_wave_store<grf::SegmentWalk>(*frame, *tiling, out, error, (hipStream_t)hip_stream);
   if (grf::reads_ahead(*frame))

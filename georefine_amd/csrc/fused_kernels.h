@@ -80,6 +80,11 @@ __device__ __forceinline__ uint16_t round_bf16(float v) {
   return (uint16_t)((u + 0x7FFFu + ((u >> 16) & 1u)) >> 16);
 }
 
+// Eight decoded words to the dense output, which may begin at any word: a caller's buffer need not
+// be aligned to the 16 bytes of a store (the type says so; the unaligned form is the same single
+// instruction, so aligned outputs pay nothing).
+typedef uint32_t words8_t __attribute__((ext_vector_type(4), aligned(2)));
+
 // What a lane does with the words it decodes: multiply them into M activation rows, store
 // them where the row lies in the dense matrix, or store them in the slot the row has in the
 // tiling (row tile * R + r of a compact [n_tiles * R][cols] output: a gather of rows).
@@ -182,12 +187,12 @@ __device__ __forceinline__ void fused_walk_body(uint8_t *lds, const grf_bctx_fus
               // would wait for them too
               if (t + 16 * (k + 1) < S) w.begin16(t + 16 * (k + 1), S);
             }
-          uint4 *dst = reinterpret_cast<uint4 *>(out + at + t);
+          words8_t *dst = reinterpret_cast<words8_t *>(out + at + t);
 #pragma unroll
           for (int k = 0; k < kHold; ++k)
             if (k < groups) {
-              dst[2 * k] = make_uint4(hold[k][0], hold[k][1], hold[k][2], hold[k][3]);
-              dst[2 * k + 1] = make_uint4(hold[k][4], hold[k][5], hold[k][6], hold[k][7]);
+              dst[2 * k] = (words8_t){hold[k][0], hold[k][1], hold[k][2], hold[k][3]};
+              dst[2 * k + 1] = (words8_t){hold[k][4], hold[k][5], hold[k][6], hold[k][7]};
             }
         }
       }
@@ -364,9 +369,9 @@ __device__ __forceinline__ void store_segment(Walk &w, const grf::FusedParams &q
       w.begin16(t, S);
       w.template half<0, SCAN>(q, reinterpret_cast<uint32_t(&)[4]>(pair[0]));
       w.template half<1, SCAN>(q, reinterpret_cast<uint32_t(&)[4]>(pair[4]));
-      uint4 *dst = reinterpret_cast<uint4 *>(out + ((size_t)first + t));
-      dst[0] = make_uint4(pair[0], pair[1], pair[2], pair[3]);
-      dst[1] = make_uint4(pair[4], pair[5], pair[6], pair[7]);
+      words8_t *dst = reinterpret_cast<words8_t *>(out + ((size_t)first + t));
+      dst[0] = (words8_t){pair[0], pair[1], pair[2], pair[3]};
+      dst[1] = (words8_t){pair[4], pair[5], pair[6], pair[7]};
     }
     return;
   }
@@ -399,7 +404,7 @@ __device__ __forceinline__ void store_segment(Walk &w, const grf::FusedParams &q
       const uint32_t at = unit;
 #endif
       if (at != kNowhere)
-        reinterpret_cast<uint4 *>(out)[(size_t)at + t / 8 + (lane & 3)] = make_uint4(v[0], v[1], v[2], v[3]);
+        reinterpret_cast<words8_t *>(out)[(size_t)at + t / 8 + (lane & 3)] = (words8_t){v[0], v[1], v[2], v[3]};
     };
     flush(std::integral_constant<int, 0>{}, u[0]);
     flush(std::integral_constant<int, 1>{}, u[1]);

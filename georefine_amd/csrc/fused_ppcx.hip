@@ -283,7 +283,6 @@ int grf_ppcx_fused_decode(const grf_ppcx_fused *frame, const grf_fused_tiling *t
   if (!out || !error) return grf::set_error(GRF_BAD_ARGUMENT, "grf_ppcx_fused_decode: null argument");
   grf_bctx_fused f;
   if (int rc = walker_frame(frame, tiling, bins, "grf_ppcx_fused_decode", f, grf::kStoreTiling)) return rc;
-  if (((uintptr_t)out & 15)) return grf::set_error(GRF_BAD_ARGUMENT, "grf_ppcx_fused_decode: out must be 16-byte aligned");
   if (tiling->scheme == GRF_TILE_WAVES)
     return grf::launch_wave_store<PpcxWalk>(f, *tiling, out, error, (hipStream_t)hip_stream);
   return grf::launch_walk<PpcxWalk, 1, grf::kStore>(f, *tiling, nullptr, 0, nullptr, 0, nullptr, out, error,

@@ -327,7 +327,8 @@ int grf_bctx_fused_validate_host(const grf_bctx_fused *frame, const grf_fused_ti
                                  const uint32_t *seg_offset, const uint32_t *tile_rows, const uint8_t *tile_class,
                                  const uint8_t *row_class, const uint32_t *row_pos);
 
-/* Same walker with a store sink: out[rows*cols] BF16 words (decode() for fused frames). */
+/* Same walker with a store sink: out[rows*cols] BF16 words (decode() for fused frames), from any
+ * word's address on. */
 int grf_bctx_fused_decode(const grf_bctx_fused *frame, const grf_fused_tiling *tiling, uint16_t *out,
                           int32_t *error, void *hip_stream);
 

@@ -34,6 +34,40 @@ def test_wave_units_store_every_word(rows, cols, segment):
             assert np.array_equal(p.decode(None).view(torch.int16).cpu().numpy().view(np.uint16), words)
 
 
+@pytest.mark.parametrize("first", [0, 1, 2, 4, 7])
+@pytest.mark.parametrize("cols,segment", [(64 * 5, 64), (16 * 9, 16), (32 * 7, 32)])
+def test_output_begins_at_any_word(cols, segment, first):
+    """The C entry points store to a caller's buffer from any word on, by the wave units and by
+    slab tilings, and touch nothing on either side."""
+    import ctypes
+    import torch
+    from georefine_amd import bitexact_context_codec as codec
+    from georefine_amd import bitexact_predictive_codec as predictive
+    from georefine_amd.bitexact_context_gpu import HipContextTensor
+    from georefine_amd.bitexact_predictive_gpu import HipPredictiveTensor
+    rng = np.random.default_rng(cols)
+    words = (rng.choice([0x3C00, 0x3C20, 0x3D00], (67, cols)) | rng.integers(0, 32, (67, cols))).astype(np.uint16)
+    t = HipContextTensor(codec.encode(words), fused_segment=segment)
+    assert t.fused is not None
+    stream = torch.cuda.current_stream().cuda_stream
+    launches = [(t._lib.grf_bctx_fused_decode, t, (), t._tiling(1)), (t._lib.grf_bctx_fused_decode, t, (), t._tiling(0))]
+    if segment % 32 == 0:
+        p = HipPredictiveTensor(predictive.encode(words, words ^ np.uint16(1)), words ^ np.uint16(1), fused_segment=segment)
+        assert p.fused is not None
+        bins = (p.buffers["context_bins"].data_ptr(),)
+        launches += [(p._lib.grf_ppcx_fused_decode, p, bins, p._tiling_for("waves")),
+                     (p._lib.grf_ppcx_fused_decode, p, bins, p._tiling_for(0))]
+    for fn, tensor, extra, (tiling, _, _, scalars) in launches:
+        guard = torch.full((first + words.size + 64,), 0x5A5A, device="cuda", dtype=torch.int16)
+        tensor.error.zero_()
+        status = fn(ctypes.byref(tensor.fused), ctypes.byref(tiling), *extra, guard.data_ptr() + 2 * first,
+                    tensor.error.data_ptr(), stream)
+        assert status == 0 and tensor.error.item() == 0
+        got = guard.cpu().numpy().view(np.uint16)
+        assert np.array_equal(got[first:first + words.size].reshape(words.shape), words), scalars["scheme"]
+        assert (got[:first] == 0x5A5A).all() and (got[first + words.size:] == 0x5A5A).all()
+
+
 @pytest.mark.parametrize("cols,segment", [(64 * 65, 64), (16 * 9, 16), (32 * 64, 32), (64 * 2, 64)])
 def test_row_gather_clamps_rejects_and_reports(cols, segment):
     """Ids outside the matrix: an IndexError, or clamped where the caller vouches for them; a
