@@ -134,9 +134,19 @@ GEMM_TWO_ROWS_FROM = 8192  # row length from which two activation rows go to the
 DENSE_ABOVE = 128          # activation rows above which linear() decodes to a dense transient
 
 # Words of pinned host memory that launches report to and their callers read after a wait; a call
-# takes one and gives it back zeroed (a list: taking and giving are atomic), at most this many stay.
+# takes one and gives it back zeroed, at most this many stay.
 _host_words = []
 HOST_WORDS_KEPT = 16
+
+
+def _host_word():
+    """One of the kept words, or a new one.  (Asked for by taking it: between a look at the list and
+    the taking another thread may take the last.)"""
+    try:
+        return _host_words.pop()
+    except IndexError:
+        import torch
+        return torch.zeros(1, dtype=torch.int32, pin_memory=True)
 
 
 def route_rows(m, cols, invariant=False):
@@ -664,7 +674,7 @@ class HipContextTensor:
         out = torch.empty((*ids.shape, self.shape[1]), device=self.device, dtype=torch.bfloat16)
         word = None
         if check or validate:
-            word = _host_words.pop() if _host_words else torch.zeros(1, dtype=torch.int32, pin_memory=True)
+            word = _host_word()
         if check and self._error_open:  # between checks the word keeps what earlier launches reported
             self.error.zero_()
             self._error_open = False

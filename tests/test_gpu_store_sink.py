@@ -94,3 +94,25 @@ def test_row_gather_clamps_rejects_and_reports(cols, segment):
     with pytest.raises(codec.CodecError):
         t.gather_rows(torch.tensor([7]))
     assert t.error.item() != 0
+
+
+def test_row_gather_when_another_thread_took_the_last_word(monkeypatch):
+    """The words that gathers report to are shared by threads: a list that was not empty a moment ago
+    is no row outside the matrix."""
+    import torch
+    from georefine_amd import bitexact_context_codec as codec
+    from georefine_amd import bitexact_context_gpu as gpu
+    rng = np.random.default_rng(5)
+    words = (rng.choice([0x3C00, 0x3C20, 0x3D00], (70, 128)) | rng.integers(0, 32, (70, 128))).astype(np.uint16)
+    t = gpu.HipContextTensor(codec.encode(words))
+
+    class Taken(list):  # looks as it did before the other thread's turn
+        def __bool__(self):
+            return True
+
+    kept = Taken()
+    monkeypatch.setattr(gpu, "_host_words", kept)
+    for _ in range(2):
+        got = t.gather_rows(torch.tensor([3, 69]))
+        assert np.array_equal(got.view(torch.int16).cpu().numpy().view(np.uint16), words[[3, 69]])
+        assert len(kept) == 1 and kept[0].item() == 0  # given back, and taken the second time
