@@ -15,12 +15,14 @@ def test_wave_units_store_every_word(rows, cols, segment):
     from georefine_amd.bitexact_context_gpu import HipContextTensor
     from georefine_amd.bitexact_predictive_gpu import HipPredictiveTensor
     rng = np.random.default_rng(rows * 131 + cols)
-    # (few distinct exponents, so that even the smallest frame is coded and not raw words)
+    # (few distinct exponents, and one class where 64 contexts' tables would outgrow the words, so that
+    # even the smallest frame is coded and not raw words)
     words = (rng.choice([0x3C00, 0x3C20, 0x3D00], (rows, cols)) | rng.integers(0, 32, (rows, cols))
              | rng.integers(0, 2, (rows, cols)) << 15).astype(np.uint16)
     frame = codec.encode(words)
-    if rows * cols < 1000 and frame[5] == 1:
-        pytest.skip("too small to be coded")
+    if rows * cols < 1000:
+        frame = codec.encode(words, row_classes=1, col_classes=1)
+    assert frame[5] != 1
     t = HipContextTensor(frame, fused_segment=segment)
     assert t.fused is not None and t.fused_plan["seg_len"] == segment and t._store_tiling()[3]["scheme"] == 1
     guard = torch.full((rows * cols + 64,), 0x5A5A, device="cuda", dtype=torch.int16)  # what the launch must not touch
@@ -30,6 +32,7 @@ def test_wave_units_store_every_word(rows, cols, segment):
     assert np.array_equal(t.decode().view(torch.int16).cpu().numpy().view(np.uint16), words)
     if segment % 32 == 0:
         p = HipPredictiveTensor(predictive.encode(words, words ^ np.uint16(1)), words ^ np.uint16(1), fused_segment=segment)
+        assert (p.fused is None) == (p.mode == 2)  # (a handful of words is kept raw)
         if p.fused is not None:
             assert np.array_equal(p.decode(None).view(torch.int16).cpu().numpy().view(np.uint16), words)
 
