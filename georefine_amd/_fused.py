@@ -285,40 +285,72 @@ def choose_wave_tiling(spr, class_rows, piece_cap_fn, lds_fn, cus=256, seg_len=6
         cap = piece_cap_fn(p_)
         n_slabs = -(-spr // p_)
         return t_, p_, r_, n_slabs, _tiles(class_rows, r_), cap, lds_fn(t_, p_, r_, n_slabs, cap)
+    threads, p, (r,), tiles, cap, lds = search_wave_tilings(
+        [(spr, seg_len, class_rows)], piece_cap_fn, lambda t_, p_, heights, cap_: lds_fn(t_, p_, heights[0], -(-spr // p_), cap_),
+        cus, table_bytes)
+    return threads, p, r, -(-spr // p), tiles, cap, lds
+
+
+def search_wave_tilings(lengths, piece_cap_fn, lds_fn, cus, table_bytes):
+    """The fastest wave tiling by ``choose_wave_tiling``'s model, as (threads, lanes per row, rows per
+    tile of every length, tiles, piece capacity, LDS bytes), of a launch over matrices of one width
+    indexed at several ``lengths``: (segments per row, segment length, rows per class) each, the one
+    that sets the pace first.  The tiles of another length are as tall as they can be without
+    taking their waves longer (at one height for all, the units of the shorter segments are twice as
+    many a tile and go a second round: 2048 x 2560 at 32 with 1024 x 2560 at 16, one row: 17.7 us,
+    so 16.2)."""
     best = None
-    tile_counts = _tile_counts(class_rows, 128)
+    counts, others = [_tile_counts(class_rows, 128) for _, _, class_rows in lengths], range(1, len(lengths))
     table_steps = 3 + table_bytes / 12288
     for p in (4, 8, 16, 32, 64):
-        if p > 4 and p // 2 >= spr:
+        if p > 4 and all(p // 2 >= spr for spr, _, _ in lengths):
             continue  # half the lanes of every unit would idle
         rpw = 64 // p
-        n_slabs = -(-spr // p)
         cap = piece_cap_fn(p)
-        unit_steps = seg_len + WAVE_UNIT_OVERHEAD + WAVE_PIECE_OVERHEAD * rpw
+        slabs = [-(-spr // p) for spr, _, _ in lengths]
+        unit_steps = [seg_len + WAVE_UNIT_OVERHEAD + WAVE_PIECE_OVERHEAD * rpw for _, seg_len, _ in lengths]
         # (768 threads, two workgroups a compute unit, where the LDS allows: a matrix with a few long
         # rows needs larger pieces, and one wave less per workgroup then keeps two of them resident --
         # 17408 x 5120 with pieces of 912 bytes: 68.7 us with 11 waves against 95.0 with 12 and
         # tiles cut down to 8 rows)
         for threads in (1024, 768, 704, 640, 576, 512):
             nwaves = threads // 64
+            busiest = lambda units: 0.5 * -(-units // nwaves) + 0.5 * units / nwaves  # units of the wave that has most
+            heights = [rpw] * len(lengths)
             for r in range(rpw, 129, rpw):
-                lds = lds_fn(threads, p, r, n_slabs, cap)
+                heights[0] = r
+                units = r // rpw * slabs[0]
+                longest = busiest(units) * unit_steps[0]
+                tiles = counts[0][r]
+                steps = tiles * (units * unit_steps[0] + nwaves * table_steps)
+                for k in others:
+                    while heights[k] + rpw <= 128 and busiest((heights[k] // rpw + 1) * slabs[k]) * unit_steps[k] <= longest:
+                        heights[k] += rpw
+                    units = heights[k] // rpw * slabs[k]
+                    longest = max(longest, busiest(units) * unit_steps[k])
+                    tiles += counts[k][heights[k]]
+                    steps += counts[k][heights[k]] * (units * unit_steps[k] + nwaves * table_steps)
+                lds = lds_fn(threads, p, heights, cap)
                 if lds > MAX_LDS:
                     break
                 # six waves per SIMD by registers; a little LDS stays with the system
                 per_cu = max(1, min(24 // nwaves, (MAX_LDS - 1024) // lds))
-                tiles = tile_counts[r]
                 rounds = -(-tiles // (cus * per_cu))
-                units = -(-r // rpw) * n_slabs
-                busiest = 0.5 * -(-units // nwaves) + 0.5 * units / nwaves
-                chain = rounds * (busiest * unit_steps + table_steps) * WAVE_LATENCY_RATIO
-                issue = tiles / cus * (units * unit_steps + nwaves * table_steps) / 4
+                chain = rounds * (longest + table_steps) * WAVE_LATENCY_RATIO
+                issue = steps / cus / 4
                 time = (chain ** 3 + issue ** 3) ** (1 / 3)
                 if best is None or time < best[0] * 0.9999:
-                    best = (time, threads, p, r, n_slabs, tiles, cap, lds)
+                    best = (time, threads, p, tuple(heights), tiles, cap, lds, rounds * cus * per_cu)
     if best is None:
         raise FusedUnsupported("no wave-unit tiling fits in LDS")
-    return best[1:]
+    _, threads, p, heights, tiles, cap, lds, capacity = best
+    if others:  # (idle workgroup slots of the rounds already paid for: 2560 x 5120 at 64 with 2048 at 32 31.1 -> 29.6)
+        heights, rpw = list(heights), 64 // p
+        for k in others:
+            while heights[k] > rpw and tiles + counts[k][heights[k] - rpw] - counts[k][heights[k]] <= capacity:
+                tiles += counts[k][heights[k] - rpw] - counts[k][heights[k]]
+                heights[k] -= rpw
+    return threads, p, tuple(heights), tiles, cap, lds
 
 
 GEMM_WAVES_PER_SIMD = int(os.environ.get("GEOREFINE_GEMM_WAVES", "6"))
@@ -694,17 +726,25 @@ class FramePlan:
                                  n_tiles=n_tiles, piece_cap=cap, scheme=SCHEME_WAVES, k_parts=k), lds=lds)
 
 
-def plan_group(plans, m=None, gemm=False, waves=False):
+def plan_group(plans, m=None, gemm=False, waves=False, mixed=False):
     """Tilings of several frames of one width for one grouped launch: planned as if the
     members' row classes belonged to one matrix (so a small member's tiles fill the
     workgroup slots a large one leaves), with one thread count, lanes per row and rows per
-    tile for all; returns one tiling (as ``FramePlan.tiling``) per member."""
-    first = plans[0]
-    if any(pl.spr != first.spr or pl.seg_len != first.seg_len or pl.cols != first.cols for pl in plans):
+    tile for all; returns one tiling (as ``FramePlan.tiling``) per member.
+
+    ``mixed``: the members may be indexed at different segment lengths (what ``choose_segment``
+    gives siblings of different sizes); the length of the member with the most rows sets the
+    pace, the others walk theirs in more slabs or fewer.  One and eight rows, us: 2048 + 512 + 512 x
+    2048 at 32, 16, 16 15.0 17.0, all at 32 14.8 19.8, a launch each 30.5 39.6; 2560 + 2048 x 5120 at
+    64, 32 30.7 41.4, both at 64 33.1 43.0; 1536 + 512 x 4096 at 32, 16 16.3 24.2, both at 32 15.1
+    26.6 (the one case of seven where one row is slower for the mixture)."""
+    first = max(plans, key=lambda pl: pl.rows)
+    if any(pl.cols != first.cols or (pl.seg_len != first.seg_len and not mixed) for pl in plans):
         raise FusedUnsupported("group members need one width and one segment length")
     class_rows = np.concatenate([pl.class_rows for pl in plans])
     cap_fn = lambda lanes: max(pl._cap(lanes) for pl in plans)
     table = max(pl.table_bytes() for pl in plans)
+    slabs = lambda pl, lanes: -(-pl.spr // lanes)
     scheme = SCHEME_SLABS
     if gemm or waves:
         for pl in plans:
@@ -713,19 +753,27 @@ def plan_group(plans, m=None, gemm=False, waves=False):
         scheme = SCHEME_WAVES
         lds_fn = lambda p_, r_, cap_: max(lds_bytes_gemm(pl.nc, pl.lognb, pl.tabn, p_, r_, cap_) for pl in plans)
         quad_cap = max(pl.quad_cap() for pl in plans)
-        threads, p, r, n_slabs, _, cap, lds, _ = choose_gemm_tiling(first.spr, class_rows, lambda lanes: quad_cap, lds_fn,
-                                                                    seg_len=first.seg_len, table_bytes=table)
+        threads, p, r, _, _, cap, lds, _ = choose_gemm_tiling(first.spr, class_rows, lambda lanes: quad_cap, lds_fn,
+                                                              seg_len=first.seg_len, table_bytes=table)
     elif waves:
         scheme = SCHEME_WAVES
-        lds_fn = lambda t_, p_, r_, s_, cap_: max(lds_bytes_waves(pl.nc, pl.lognb, pl.tabn, WAVE_ROWS_PER_PASS, t_, p_, r_,
-                                                                  s_, cap_) for pl in plans)
-        threads, p, r, n_slabs, _, cap, lds = choose_wave_tiling(first.spr, class_rows, cap_fn, lds_fn,
-                                                                 seg_len=first.seg_len, table_bytes=table)
+        seg_lens = list(dict.fromkeys(pl.seg_len for pl in [first, *plans]))
+        lengths = [(first.cols // n, n, np.concatenate([pl.class_rows for pl in plans if pl.seg_len == n])) for n in seg_lens]
+        lds_fn = lambda t_, p_, heights, cap_: max(
+            lds_bytes_waves(pl.nc, pl.lognb, pl.tabn, WAVE_ROWS_PER_PASS, t_, p_, heights[seg_lens.index(pl.seg_len)],
+                            slabs(pl, p_), cap_) for pl in plans)
+        forced = os.environ.get("GEOREFINE_FUSED_WAVE_TILING")  # "threads,lanes_per_row,rows": experiments only
+        if forced:
+            threads, p, r = (int(v) for v in forced.split(","))
+            heights, cap = [r] * len(seg_lens), cap_fn(p)
+            lds = lds_fn(threads, p, heights, cap)
+        else:
+            threads, p, heights, _, cap, lds = search_wave_tilings(lengths, cap_fn, lds_fn, 256, table)
+        height_of = dict(zip(seg_lens, heights))
     else:
-        lds_fn = lambda p_, r_, cap_: max(lds_bytes(pl.nc, pl.lognb, pl.tabn, m, p_, first.seg_len, r_, cap_)
-                                          for pl in plans)
-        threads, p, r, n_slabs, _, cap, lds = choose_tiling(first.spr, class_rows, cap_fn, lds_fn,
-                                                            seg_len=first.seg_len, table_bytes=table)
+        lds_fn = lambda p_, r_, cap_: max(lds_bytes(pl.nc, pl.lognb, pl.tabn, m, p_, pl.seg_len, r_, cap_) for pl in plans)
+        threads, p, r, _, _, cap, lds = choose_tiling(first.spr, class_rows, cap_fn, lds_fn,
+                                                      seg_len=first.seg_len, table_bytes=table)
     tilings = []
     if gemm:  # whole blocks of sixteen rows per tile; one slot stride and LDS demand for all members
         cut, at, lead = [], 0, 0
@@ -734,19 +782,20 @@ def plan_group(plans, m=None, gemm=False, waves=False):
             at, lead = at + len(cut[-1][1]), lead + cut[-1][3]
         height = max(c[2] for c in cut)
         lds = lds_fn(p, height, cap)
-        for tile_rows, tile_class, r_, _ in cut:
+        for pl, (tile_rows, tile_class, r_, _) in zip(plans, cut):
             if r_ != height:  # (a member the cut did not pay for: its slots widened to the common stride)
                 wide = np.full((len(tile_class), height), 0xFFFFFFFF, dtype=np.uint32)
                 wide[:, :r_] = tile_rows.reshape(-1, r_)
                 tile_rows = wide.reshape(-1)
             tilings.append(dict(tile_rows=tile_rows, tile_class=tile_class,
-                                scalars=dict(threads=threads, lanes_per_row=p, rows_per_tile=height, n_slabs=n_slabs,
+                                scalars=dict(threads=threads, lanes_per_row=p, rows_per_tile=height, n_slabs=slabs(pl, p),
                                              n_tiles=len(tile_class), piece_cap=cap, scheme=scheme), lds=lds))
         return tilings
     for pl in plans:
-        tile_rows, tile_class = build_tiles(pl.row_class, pl.nr, r)
+        height = height_of[pl.seg_len] if waves else r
+        tile_rows, tile_class = build_tiles(pl.row_class, pl.nr, height)
         tilings.append(dict(tile_rows=tile_rows, tile_class=tile_class,
-                            scalars=dict(threads=threads, lanes_per_row=p, rows_per_tile=r, n_slabs=n_slabs,
+                            scalars=dict(threads=threads, lanes_per_row=p, rows_per_tile=height, n_slabs=slabs(pl, p),
                                          n_tiles=len(tile_class), piece_cap=cap, scheme=scheme), lds=lds))
     return tilings
 

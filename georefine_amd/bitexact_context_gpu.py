@@ -304,7 +304,7 @@ class HipContextTensor:
             if name in indexed and not indexed[name].flags.writeable:
                 indexed[name] = indexed[name].copy()
         return {"indexed": indexed, "plan": plan, "reason": reason, "stride": stride, "fused": fused,
-                "main_bytes": main_bytes, "raw6_segment": raw6_segment, "raw6_block": raw6_block}
+                "asked_segment": fused_segment, "main_bytes": main_bytes, "raw6_segment": raw6_segment, "raw6_block": raw6_block}
 
     def __init__(self, frame: bytes, *, stride: int = 1024, device="cuda:0", fused=True, fused_segment=None,
                  m_invariant=False, prepared=None, residual_block=None):
@@ -321,6 +321,7 @@ class HipContextTensor:
         elif prepared["stride"] != stride or prepared["fused"] != fused:
             raise ValueError("the frame was prepared with another stride or fused setting")
         indexed, plan = prepared["indexed"], prepared["plan"]
+        self.asked_segment = prepared["asked_segment"]  # None: the length was left to ``choose_segment``
         self.shape = indexed["shape"]
         self.n = math.prod(self.shape)
         self.stride = stride
@@ -703,8 +704,9 @@ class HipLinearGroup:
     """Coded matrices of one width that take the same activations (q/k/v, gate/up), multiplied
     in one launch: the members' tiles share the grid, so a small matrix fills the workgroup
     slots a large one leaves, and the launch overhead is paid once.  The members stay usable
-    on their own.  They must have been indexed with one segment length
-    (``HipContextTensor(..., fused_segment=...)``)."""
+    on their own.  Members whose index was left to the default go together whatever lengths their
+    sizes gave them; lengths that were asked for (``HipContextTensor(..., fused_segment=...)``)
+    must be one."""
 
     def __init__(self, tensors, *, m_invariant=None):
         import torch
@@ -717,6 +719,8 @@ class HipLinearGroup:
                 raise base.CodecError("frame is not eligible for the fused kernels: " + t.fused_reason)
             if t.shape[1] != first.shape[1] or t.device != first.device:
                 raise ValueError("group members need one width and one device")
+        if len({t.asked_segment for t in self.tensors} - {None}) > 1:
+            raise _fused.FusedUnsupported("group members were asked to have different segment lengths")
         self.device, self._lib, self._index = first.device, first._lib, first._index
         # the members' policy unless given: a group of members that keep rows bit-equal across
         # row counts does so too
@@ -732,8 +736,8 @@ class HipLinearGroup:
         import torch
         if key not in self._tilings:
             plans = [t._plan for t in self.tensors]
-            hosts = (_fused.plan_group(plans, gemm=True) if key == "gemm"
-                     else _fused.plan_group(plans, m=key, waves=GEMV_WAVES))
+            hosts = (_fused.plan_group(plans, gemm=True, mixed=True) if key == "gemm"
+                     else _fused.plan_group(plans, m=key, waves=GEMV_WAVES, mixed=True))
             made = []
             for host in hosts:
                 rows = torch.from_numpy(host["tile_rows"]).to(self.device)

@@ -227,6 +227,30 @@ def test_group_plans_share_one_tile_shape_and_keep_every_member_complete():
         _fused.plan_group([plans[0], other], m=1)
 
 
+@pytest.mark.parametrize("members", [((96, 32), (32, 16), (33, 16)), ((64, 64), (200, 16)), ((20, 128), (17, 32), (300, 64), (5, 16))],
+                         ids=lambda m: "+".join(f"{r}at{s}" for r, s in m))
+def test_group_plans_of_members_indexed_at_different_lengths(members):
+    """Siblings of different sizes get different segment lengths by default: one shape for all, every
+    member's own length in its slab count, what the kernels take on trust checked by the library."""
+    rng = np.random.default_rng(len(members))
+    plans = [_plan(weight_like(rng, rows, 640), segment=segment)[1] for rows, segment in members]
+    with pytest.raises(_fused.FusedUnsupported):
+        _fused.plan_group(plans, m=2, waves=True)
+    for use, kwargs in (("gemv", dict(m=1)), ("gemv", dict(m=8)), ("gemv", dict(m=2, waves=True)), ("gemm", dict(gemm=True))):
+        tilings = _fused.plan_group(plans, mixed=True, **kwargs)
+        shapes = {(t["scalars"]["threads"], t["scalars"]["lanes_per_row"], t["scalars"]["piece_cap"], t["lds"]) for t in tilings}
+        assert len(shapes) == 1 and len(tilings) == len(members)
+        heights = {(plan.seg_len, t["scalars"]["rows_per_tile"]) for plan, t in zip(plans, tilings)}
+        assert len(heights) == len({plan.seg_len for plan in plans})  # one height a length
+        for plan, t in zip(plans, tilings):
+            s = t["scalars"]
+            assert s["n_slabs"] == -(-plan.spr // s["lanes_per_row"]) and t["lds"] <= _fused.MAX_LDS
+            rows = t["tile_rows"].reshape(s["n_tiles"], s["rows_per_tile"])
+            assert sorted(rows[rows != 0xFFFFFFFF].tolist()) == list(range(plan.rows))
+            block, position, _ = plan.residual_order()
+            _fused.validate_host(plan, t, use, row_pos=position, block=block)
+
+
 @pytest.mark.parametrize("shape,nr", [((200, 1280), 16), ((96, 640), 4), ((33, 256), 1)],
                          ids=lambda v: f"{v[0]}x{v[1]}" if isinstance(v, tuple) else f"nr{v}")
 def test_resident_residual_order(shape, nr):

@@ -68,6 +68,38 @@ def test_group_products(shapes):
     assert group.linear(x[:0], biases)[0].shape == (0, shapes[0][0])
 
 
+@pytest.mark.parametrize("shapes,segments", [
+    ([(2048, 2048), (512, 2048), (512, 2048)], (32, 16, 16)), ([(2048, 2560), (1024, 2560)], (32, 16)),
+    ([(1536, 4096), (512, 4096)], (32, 16)), ([(2048, 5120), (2560, 5120)], (32, 64)),
+], ids=lambda v: "+".join("x".join(map(str, s)) if isinstance(s, tuple) else str(s) for s in v))
+def test_group_of_members_indexed_by_default(shapes, segments):
+    """Siblings whose sizes give them different segment lengths by default (grouped-query q/k/v): one
+    launch, for one and two rows with the bits of the members' own launches."""
+    import torch
+    from georefine_amd.bitexact_context_gpu import HipLinearGroup
+    words, tensors = _members(shapes, seed=31, segment=None)
+    assert tuple(t.fused_plan["seg_len"] for t in tensors) == segments
+    group = HipLinearGroup(tensors)
+    cols = shapes[0][1]
+    x = torch.from_numpy(bf16_words(np.random.default_rng(6).normal(0, 1, size=(128, cols)))).view(torch.bfloat16).cuda()
+    dense = [torch.from_numpy(w).view(torch.bfloat16).cuda().float() for w in words]
+    for rows in (1, 2):
+        for y, t in zip(group.linear(x[:rows], check=True, batch_invariant=False), tensors):
+            assert torch.equal(y.view(torch.uint16), t.gemv(x[:rows]).view(torch.uint16)), rows
+    full = group.linear(x, check=True, batch_invariant=True)
+    for y, w in zip(full, dense):
+        want = torch.nn.functional.linear(x.float(), w)
+        scale = torch.nn.functional.linear(x.float().abs(), w.abs())
+        assert bool((y.float() - want).abs().le(1e-2 * want.abs().clamp_min(1e-3 * scale) + 1e-30).all())
+    for rows in (1, 7, 17, 64, 100):
+        for y, f in zip(group.linear(x[:rows], batch_invariant=True), full):
+            assert torch.equal(y.view(torch.uint16), f[:rows].view(torch.uint16)), rows
+    tensors[1].buffers["fused_seg_state"].view(torch.int32)[tensors[1].index_slot(2, 1)] += 1  # forced from the host; kernels finish normally
+    for rows in (1, 5):
+        with pytest.raises(Exception):
+            group.linear(x[:rows], check=True)
+
+
 def test_group_reports_a_member_that_misses_its_checkpoints_and_rejects_mismatches():
     import torch
     from georefine_amd import bitexact_context_codec as codec
