@@ -7,6 +7,7 @@ become a coarse u8 lookup plus a sparse table of the symbols that occur.
 """
 from __future__ import annotations
 
+import copy
 import ctypes
 import heapq
 import math
@@ -353,6 +354,19 @@ def search_wave_tilings(lengths, piece_cap_fn, lds_fn, cus, table_bytes):
     return threads, p, tuple(heights), tiles, cap, lds
 
 
+def wave_time(tiling, seg_len, table_bytes, cus=256):
+    """What ``choose_wave_tiling``'s model says of one tiling (as ``FramePlan.tiling`` returns it), in
+    decode steps of a SIMD."""
+    g = tiling["scalars"]
+    nwaves, rpw = g["threads"] // 64, 64 // g["lanes_per_row"]
+    unit_steps, table_steps = seg_len + WAVE_UNIT_OVERHEAD + WAVE_PIECE_OVERHEAD * rpw, 3 + table_bytes / 12288
+    units = -(-g["rows_per_tile"] // rpw) * g["n_slabs"]
+    rounds = -(-g["n_tiles"] // (cus * max(1, min(24 // nwaves, (MAX_LDS - 1024) // tiling["lds"]))))
+    chain = rounds * ((0.5 * -(-units // nwaves) + 0.5 * units / nwaves) * unit_steps + table_steps) * WAVE_LATENCY_RATIO
+    issue = g["n_tiles"] / cus * (units * unit_steps + nwaves * table_steps) / 4
+    return (chain ** 3 + issue ** 3) ** (1 / 3)
+
+
 GEMM_WAVES_PER_SIMD = int(os.environ.get("GEOREFINE_GEMM_WAVES", "6"))
 # a single matrix's GEMM may be cut along K ("0": never; experiments and tests of the uncut kernel)
 GEMM_SPLIT = os.environ.get("GEOREFINE_FUSED_GEMM_SPLIT", "1") != "0"
@@ -605,6 +619,42 @@ class FramePlan:
         self.row_class = np.asarray(row_class)
         self.class_rows = np.bincount(self.row_class, minlength=nr)
         self._caps, self._tilings = {}, {}
+
+    def for_vector_alus(self, main_freq, budget, image=None):
+        """This plan, or one like it with lookups of at most ``budget`` bytes where the launches of
+        the wave units (one row, the store sink) are the faster for them: where this plan's waves
+        have more than a unit each and the smaller tables' tiling is modelled 14 % faster.  Fewer bytes
+        mean more scans (of the predictive codec's wave steps 21 % at 32 KiB, 12 % at 64), and leave
+        the LDS two workgroups a compute unit, which cut the rows finer.  One row and the store
+        sink, us, predictive frames at 64 / 32 KiB, by units a wave and the modelled advantage:
+          4096 x 4096   1.1 units, 1.35   31.8 34.3 / 27.5 29.0
+          8192 x 4096   2.1 units, 1.23   43.0 51.3 / 39.2 49.3
+          5120 x 8192   2.6 units, 1.17   48.4 57.2 / 48.6 56.9
+          4096 x 11008  3.2 units, 1.15   53.8 62.2 / 49.1 60.0
+          5120 x 17408  6.2 units, 1.10   92.2 112.5 / 92.9 117.7
+          5120 x 5120   1.9 units, 1.10   34.7 41.7 / 35.6 45.6
+          1024 x 1024   0.2 units, 1.16   11.7 11.3 / 13.8 13.2
+          3000 x 4096   0.8 units, 1.11   21.2 22.9 / 25.2 26.9"""
+        other = self.with_lookups(main_freq, budget, image)
+        if other.lognb >= self.lognb:
+            return self
+        try:
+            tall, fine = self.tiling(1, waves=True), other.tiling(1, waves=True)
+        except FusedUnsupported:
+            return self
+        g = tall["scalars"]
+        units = -(-g["rows_per_tile"] // (64 // g["lanes_per_row"])) * g["n_slabs"]
+        gain = wave_time(tall, self.seg_len, self.table_bytes()) / wave_time(fine, self.seg_len, other.table_bytes())
+        return other if units > g["threads"] // 64 and gain >= 1.14 else self
+
+    def with_lookups(self, main_freq, budget, image=None):
+        """This plan with lookups of at most ``budget`` bytes."""
+        other = copy.copy(self)
+        other.shift = choose_shift(self.nc, budget)
+        other.lognb = 16 - other.shift
+        other.lut = sparse_tables(main_freq, self.nr, self.nc, other.shift, image)[0]
+        other._tilings = {}
+        return other
 
     def residual_order(self, block=None):
         """(block rows B, row positions u32[rows], rows of the array) of the resident residual

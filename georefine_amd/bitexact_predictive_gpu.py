@@ -50,10 +50,12 @@ def _checkpoints(stream, ctx, freq, vocab, stride):
 # Sixteen bin contexts share the lookup bytes.  A wave scans on whenever one of its 64 lanes meets
 # a bucket's minority symbol: 35 % of the steps with 1 KiB per context, 21 % with 2 KiB, 12 % with
 # 4 KiB.  At 64 KiB one workgroup of sixteen waves has a compute unit to itself instead of two of
-# twelve, and still wins throughout (4096 x 4096, 16 / 32 / 64 KiB in all: decode 32.3 / 26.5 /
-# 27.4 us, one row 31.0 / 25.7 / 26.9, 16 rows 39.6 / 37.9 / 37.5, 96 rows 59.2 / 61.6 / 44.7;
-# 512 x 1024, one row 12.1 / 12.1 / 10.6, 64 rows 19.3 / 19.6 / 12.9).
-_LUT_BUDGET = int(os.environ.get("GEOREFINE_FUSED_LUT_BYTES", 64 * 1024))
+# twelve, and still wins for products on the matrix cores (16 / 32 / 64 KiB in all, us: 4096 x 4096
+# at 96 rows 61.2 / 53.9 / 51.8, 3000 x 4096 36.4 / 32.6 / 31.9, 5120 x 17408 164 / 140 / 137, 512 x 1024 at
+# 64 rows 15.8 / 15.2 / 15.1).  One row and decode() take 32 KiB where those are faster
+# (FramePlan.for_vector_alus); the tensor then keeps both lookups, half a MiB more.
+_LUT_BUDGET, _WALK_LUT_BUDGET = ((int(os.environ["GEOREFINE_FUSED_LUT_BYTES"]),) * 2
+                                 if "GEOREFINE_FUSED_LUT_BYTES" in os.environ else (64 * 1024, 32 * 1024))
 
 
 def _word_image(main):
@@ -76,8 +78,9 @@ def _fused_segment(shape, segment=None):
 
 def _read_frame(frame, reference, stride, *, fused=False, fused_segment=None):
     """Parse, validate and index a frame against its reference words.  With ``fused`` the
-    result also carries ``fused_plan`` (or ``fused_reason``) and keeps the residuals in the
-    packed 5-bit form whatever the frame's mode (``resident_mode`` 0)."""
+    result also carries ``fused_plan`` (or ``fused_reason``) with ``walk_plan``, the same with the lookups
+    of the vector-ALU launches, and keeps the residuals in the packed 5-bit form whatever the
+    frame's mode (``resident_mode`` 0)."""
     if not isinstance(frame, (bytes, bytearray, memoryview)):
         raise codec.CodecError("frame must be bytes")
     info = codec.parse(frame, reference)
@@ -117,6 +120,7 @@ def _read_frame(frame, reference, stride, *, fused=False, fused_segment=None):
         try:
             result["fused_plan"] = _fused.FramePlan((r, c), 16, 16, info["labels"], freq, fs, fo, len(info["stream"]),
                                                     seg_len, image=_word_image, lut_budget=_LUT_BUDGET)
+            result["walk_plan"] = result["fused_plan"].for_vector_alus(freq, _WALK_LUT_BUDGET, _word_image)
             result["resident_mode"] = 0
         except _fused.FusedUnsupported as exc:
             result["fused_reason"] = str(exc)
@@ -158,7 +162,8 @@ class HipPredictiveTensor:
         self.n = math.prod(self.shape)
         self.stride, self.mode = stride, ix["mode"]
         self.resident_mode = ix.get("resident_mode", self.mode)
-        self._plan = ix.pop("fused_plan", None)
+        self._plan = ix.pop("fused_plan", None)         # of the matrix-core launches ...
+        self._walk_plan = ix.pop("walk_plan", None)     # ... and of the others (the same one for most matrices)
         self.fused_reason = ix.pop("fused_reason", None)
         self.device = torch.device(device)
         for key in ("source_sha256", "target_sha256", "reference_sha256", "frame_sha256", "frame_bytes"):
@@ -172,7 +177,7 @@ class HipPredictiveTensor:
         # read one run of bytes per visit and a 128-byte line is not visited four times).
         self._raw5_segment = self._raw5_block = self._rows_held = 0
         if self._plan is not None and "raw5" in ix and self.resident_mode == 0:
-            block, position, held = self._plan.residual_order()
+            block, position, held = self._walk_plan.residual_order()
             rows_, cols_ = self.shape
             ix["raw5"] = _fused.order_records(ix["raw5"], rows_, cols_, self._plan.seg_len, block, position, held, 32, 20)
             ix["row_pos"] = position
@@ -236,7 +241,7 @@ class HipPredictiveTensor:
             f.rows, f.cols = self.shape
             f.mode, f.stride = self.resident_mode, self.stride
             self._frame = f
-        self.fused = None
+        self.fused = self.fused_gemm = None
         if self._plan is not None:
             try:
                 self._prepare_fused()
@@ -271,26 +276,32 @@ class HipPredictiveTensor:
             spr, position = self.shape[1] // self._raw5_segment, b["row_pos"].cpu().numpy()
             states = _fused.order_index(states, self.shape[0], spr, self._raw5_block, position, self._rows_held)
             offsets = _fused.order_index(offsets, self.shape[0], spr, self._raw5_block, position, self._rows_held)
-        for name, array in (("fused_seg_state", states), ("fused_seg_offset", offsets),
-                            ("fused_lut", plan.lut), ("fused_tab", plan.tab.view(np.int64))):
+        walk = self._walk_plan
+        arrays = {"fused_seg_state": states, "fused_seg_offset": offsets, "fused_lut": plan.lut, "fused_tab": plan.tab.view(np.int64)}
+        if walk is not plan:
+            arrays["fused_walk_lut"] = walk.lut
+        for name, array in arrays.items():
             if name not in b:  # (a clone already holds its copies)
                 b[name] = torch.from_numpy(np.ascontiguousarray(array)).to(self.device)
-        f = _hip_abi.GrfPpcxFused()
-        f.main_bytes, f.raw5 = b["main_stream"].data_ptr(), b["raw5"].data_ptr()
-        f.seg_state, f.seg_offset = b["fused_seg_state"].data_ptr(), b["fused_seg_offset"].data_ptr()
-        f.lut, f.tab = b["fused_lut"].data_ptr(), b["fused_tab"].data_ptr()
-        f.main_n_bytes = b["main_stream"].numel() - 16
-        f.rows, f.cols = self.shape
-        f.n_labels = 16
-        sc = plan.scalars()
-        f.seg_len, f.segs_per_row, f.shift, f.lognb, f.tabn = (sc["seg_len"], sc["segs_per_row"], sc["shift"],
-                                                                sc["lognb"], sc["tabn"])
-        f.whole_range = sc["whole_range"]
-        f.raw_interleaved = self._raw5_block if self._raw5_segment else 0
-        f.row_pos = b["row_pos"].data_ptr() if self._raw5_segment else None
-        self.fused = f
-        store = self._tiling_for("waves")
-        self.fused_plan = dict(sc, **store[3])
+
+        def frame(of, lut):
+            f = _hip_abi.GrfPpcxFused()
+            f.main_bytes, f.raw5 = b["main_stream"].data_ptr(), b["raw5"].data_ptr()
+            f.seg_state, f.seg_offset = b["fused_seg_state"].data_ptr(), b["fused_seg_offset"].data_ptr()
+            f.lut, f.tab = b[lut].data_ptr(), b["fused_tab"].data_ptr()
+            f.main_n_bytes = b["main_stream"].numel() - 16
+            f.rows, f.cols = self.shape
+            f.n_labels = 16
+            sc = of.scalars()
+            for key in ("seg_len", "segs_per_row", "shift", "lognb", "tabn", "whole_range"):
+                setattr(f, key, sc[key])
+            f.raw_interleaved = self._raw5_block if self._raw5_segment else 0
+            f.row_pos = b["row_pos"].data_ptr() if self._raw5_segment else None
+            return f
+
+        self.fused_gemm = frame(plan, "fused_lut")
+        self.fused = self.fused_gemm if walk is plan else frame(walk, "fused_walk_lut")
+        self.fused_plan = dict(walk.scalars(), **self._tiling_for("waves")[3])
 
     def index_slot(self, row, segment):
         """Where the checkpoint of ``segment`` (0..segments per row; the last is the end of the
@@ -303,12 +314,13 @@ class HipPredictiveTensor:
         return ((q // block) * (spr + 1) + segment) * block + q % block
 
     def _tiling_for(self, key):
-        """Device copy of a tiling: key 0 = store sink, "waves" = the GEMV (wave units, one tiling
-        for every row count), 1/2/4/8 = GEMV row buckets of the slab kernels, "gemm"."""
+        """Device copy of a tiling: "waves" = the GEMV and the store sink (wave units, one tiling for
+        every row count), "gemm"; of the slab kernels, which only callers of the C entry points
+        reach: 0 = store sink, 1/2/4/8 = GEMV row buckets."""
         if key not in self._tilings:
             import torch
-            host = (self._plan.gemm_tiling() if key == "gemm" else
-                    self._plan.tiling(_fused.WAVE_ROWS_PER_PASS, waves=True) if key == "waves" else self._plan.tiling(key))
+            host = (self._plan.gemm_tiling() if key == "gemm" else self._walk_plan.tiling(_fused.WAVE_ROWS_PER_PASS, waves=True)
+                    if key == "waves" else self._walk_plan.tiling(key))
             rows = torch.from_numpy(host["tile_rows"].view(np.int32)).to(self.device)
             classes = torch.from_numpy(host["tile_class"]).to(self.device)
             g = _hip_abi.GrfFusedTiling()
@@ -411,7 +423,7 @@ class HipPredictiveTensor:
             if not status:
                 extra = ()
                 if use_gemm:
-                    fn, tiling = self._lib.grf_ppcx_gemm, self._tiling_for("gemm")[0]
+                    fn, frame, tiling = self._lib.grf_ppcx_gemm, self.fused_gemm, self._tiling_for("gemm")[0]
                     key = m if m <= PackedActivations.MAX_ROWS else PackedActivations.MAX_ROWS
                     size = self._workspace.get((key, tiling.k_parts))
                     if size is None:
@@ -421,9 +433,8 @@ class HipPredictiveTensor:
                     space = packed.ensure(size) if packed is not None else x2.new_empty((size + 1) // 2)
                     extra = (space.data_ptr(), size)
                 else:
-                    fn = self._lib.grf_ppcx_gemv
-                    tiling = self._tiling_for("waves")[0]
-                status = launch_on(self._index, fn, ctypes.byref(self.fused), ctypes.byref(tiling), bins.data_ptr(), xp, ldx,
+                    fn, frame, tiling = self._lib.grf_ppcx_gemv, self.fused, self._tiling_for("waves")[0]
+                status = launch_on(self._index, fn, ctypes.byref(frame), ctypes.byref(tiling), bins.data_ptr(), xp, ldx,
                                    m, y.data_ptr(), rows, bias.data_ptr() if bias is not None else None, *extra,
                                    self.error.data_ptr())
             self._status(status, check)
@@ -498,9 +509,8 @@ class HipPredictiveGroup:
     def _tiling(self, key):
         import torch
         if key not in self._tilings:
-            plans = [t._plan for t in self.tensors]
-            hosts = (_fused.plan_group(plans, gemm=True) if key == "gemm"
-                     else _fused.plan_group(plans, m=_fused.WAVE_ROWS_PER_PASS, waves=True))
+            hosts = (_fused.plan_group([t._plan for t in self.tensors], gemm=True) if key == "gemm"
+                     else _fused.plan_group([t._walk_plan for t in self.tensors], m=_fused.WAVE_ROWS_PER_PASS, waves=True))
             made = []
             for host in hosts:
                 rows = torch.from_numpy(host["tile_rows"].view(np.int32)).to(self.device)
@@ -517,7 +527,8 @@ class HipPredictiveGroup:
         n = len(self.tensors)
         if key not in self._pointer_arrays:  # frames, tilings, planes and row counts do not change between calls
             self._pointer_arrays[key] = (
-                (ctypes.POINTER(_hip_abi.GrfPpcxFused) * n)(*[ctypes.pointer(t.fused) for t in self.tensors]),
+                (ctypes.POINTER(_hip_abi.GrfPpcxFused) * n)(*[ctypes.pointer(t.fused_gemm if key == "gemm" else t.fused)
+                                                             for t in self.tensors]),
                 (ctypes.POINTER(_hip_abi.GrfFusedTiling) * n)(*[ctypes.pointer(g[0]) for g in self._tiling(key)]),
                 (ctypes.c_void_p * n)(*[t.buffers["context_bins"].data_ptr() for t in self.tensors]),
                 (ctypes.c_uint32 * n)(*[t.shape[0] for t in self.tensors]), ctypes.c_void_p * n)

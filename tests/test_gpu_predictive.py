@@ -289,3 +289,35 @@ def test_every_predictive_sink_on_a_random_case(oracle, rows, cols, mode, kind, 
     assert close(y70)
     for m in (1, 8, 17, 40):
         assert torch.equal(t.gemm(ref_dev, x[:m]).view(torch.uint16), y70[:m].view(torch.uint16))
+
+
+@pytest.mark.parametrize("shape", [(200, 1280), (67, 320)])
+def test_one_row_and_decode_with_lookups_of_their_own(shape, monkeypatch):
+    """A tensor that keeps two lookups (large matrices: FramePlan.for_vector_alus): one row and
+    decode() through the smaller ones, the matrix cores through the larger, alone, as a clone and
+    in a group, bit for bit what one lookup for all gives."""
+    import torch
+    from georefine_amd import _fused
+    from georefine_amd import bitexact_predictive_codec as predictive
+    from georefine_amd.bitexact_predictive_gpu import HipPredictiveGroup, HipPredictiveTensor
+    rng = np.random.default_rng(shape[0])
+    target = weight_like(rng, *shape)
+    ref = bf16_words((target.astype(np.uint32) << 16).view(np.float32) + rng.normal(0, 0.003, shape).astype(np.float32))
+    frame = predictive.encode(target, ref)
+    one = HipPredictiveTensor(frame, ref)
+    assert one.fused is not None and one._walk_plan is one._plan and one.fused_gemm is one.fused
+    monkeypatch.setattr(_fused.FramePlan, "for_vector_alus", _fused.FramePlan.with_lookups)
+    two = HipPredictiveTensor(frame, ref)
+    assert two.fused.lognb == 11 and two.fused_gemm.lognb == 12 and two.fused.lut != two.fused_gemm.lut
+    assert two.resident_bytes >= one.resident_bytes + two.buffers["fused_walk_lut"].numel()
+    copy = two.clone()
+    assert copy.fused.lut not in (two.fused.lut, 0) and copy.fused_gemm.lut not in (two.fused_gemm.lut, copy.fused.lut)
+    x = torch.from_numpy(bf16_words(rng.normal(0, 1, size=(100, shape[1])))).view(torch.bfloat16).cuda()
+    for t in (two, copy):
+        assert np.array_equal(t.decode(None).view(torch.int16).cpu().numpy().view(np.uint16), target)
+        for rows in (1, 2, 40, 100):
+            assert torch.equal(t.linear(None, x[:rows], check=True), one.linear(None, x[:rows])), rows
+    mixed, plain = HipPredictiveGroup([two, one, copy]), HipPredictiveGroup([one, one, one])
+    for rows in (1, 40):
+        for a, b in zip(mixed.linear(x[:rows], check=True), plain.linear(x[:rows], check=True)):
+            assert torch.equal(a, b), rows

@@ -29,3 +29,38 @@ def test_row_blocks_stay_whole_where_workgroups_do_not_share_a_unit(class_rows, 
         spr, np.array(class_rows), lambda lanes: 208, lds, seg_len=32, table_bytes=table, split=True)
     assert threads == _fused.gemm_shape(p, r)[2] and tiles == sum(-(-c // r) for c in class_rows) * k
     assert (r % 16 == 0) == whole
+
+
+def _predictive_plan(rows, cols, symbols=130):
+    """A plan as a predictive frame has it (16 labels, 16 bins), without the frame."""
+    from georefine_amd import bitexact_predictive_gpu as gpu
+    rng = np.random.default_rng(rows)
+    seg = gpu._fused_segment((rows, cols))
+    freq = np.zeros((256, 2048), dtype=np.uint32)
+    for c in range(256):
+        f = np.exp(-0.5 * ((np.arange(symbols) - rng.uniform(20, symbols - 20)) / 8) ** 2) + 1e-5
+        f = np.maximum(1, (f / f.sum() * 65536).astype(np.int64))
+        f[np.argmax(f)] += 65536 - f.sum()
+        freq[c, 300:300 + symbols] = f
+    labels = np.sort(rng.integers(0, 16, rows)).astype(np.uint8)
+    n = rows * cols // seg
+    offsets = 4 + np.arange(n, dtype=np.int64) * seg * 3 // 8 + rng.integers(0, 4, n)
+    return freq, _fused.FramePlan((rows, cols), 16, 16, labels, freq, np.full(n, 1 << 23, dtype=np.uint32), offsets,
+                                  int(offsets[-1]) + 40, seg, image=gpu._word_image, lut_budget=gpu._LUT_BUDGET)
+
+
+@pytest.mark.parametrize("rows,cols,both", [(4096, 4096, True), (8192, 4096, True), (2048, 4096, False), (1024, 1024, False),
+                                            (9000, 1024, False)])
+def test_vector_alu_launches_take_the_smaller_lookups_where_those_are_faster(rows, cols, both):
+    from georefine_amd import bitexact_predictive_gpu as gpu
+    freq, plan = _predictive_plan(rows, cols)
+    walk = plan.for_vector_alus(freq, gpu._WALK_LUT_BUDGET, gpu._word_image)
+    assert (walk is not plan) == both and plan.lognb == 12
+    if both:
+        assert walk.lognb == 11 and walk.lut.shape == (16, 16 << 11) and plan.lut.shape == (16, 16 << 12)
+        assert np.array_equal(walk.lut, _fused.sparse_tables(freq, 16, 16, 5, gpu._word_image)[0])
+        tall, fine = (p.tiling(1, waves=True) for p in (plan, walk))
+        assert tall["scalars"]["n_tiles"] <= 256 < fine["scalars"]["n_tiles"] and 2 * fine["lds"] <= _fused.MAX_LDS
+        assert fine["lds"] == _fused.lds_bytes_waves(16, 11, walk.tabn, 2, *(fine["scalars"][k] for k in (
+            "threads", "lanes_per_row", "rows_per_tile", "n_slabs", "piece_cap")))
+    assert plan.for_vector_alus(freq, gpu._LUT_BUDGET, gpu._word_image) is plan  # nothing smaller asked for
