@@ -29,10 +29,13 @@ SMALL_MATRIX = 8 << 20  # elements below which the walk, not the machine, bounds
 
 
 def choose_segment(cols, preferred=None, rows=None):
-    """Segment length that divides the row length: 64 by default (index 1 bit per weight).
-    A launch takes at least one segment's worth of dependent steps (0.1 us each), so matrices too
+    """Segment length that divides the row length: the one asked for (``preferred``), or 64 by
+    default (index 1 bit per weight).  A launch takes at least one segment's worth of dependent steps (0.1 us each), so matrices too
     small to fill the GPU several times over get 32 (2 bits per weight of index), the smallest
-    16.  GPU time of a product of 1, 8 and 32 rows and of decode(), us:
+    16 (4 bits).  That is paid in device memory: bits per weight in all, by default and at 64, 2048 x
+    5120 13.5 and 12.5, 2048 x 1024 19.1 and 16.1 (5.5 of them tables, which do not shrink with the
+    matrix).  A caller that asks for a length asks for its index: where it does not divide, matrices
+    under 8 M weights get 32, others 64, before anything shorter.  GPU time of a product of 1, 8 and 32 rows and of decode(), us:
       3500 x 1024   32: 12.0 15.3 16.1 12.3   16: 11.0 11.3 11.5 11.3
       300 x 4096    32: 11.3 15.0 15.4 10.8   16: 10.2 12.9 13.1  8.9
       2000 x 2048   32: 11.7 13.8 13.9 11.9   16: 11.8 13.7 14.1 11.8
@@ -41,11 +44,11 @@ def choose_segment(cols, preferred=None, rows=None):
     Long rows pay for the short segments in sums per row, and keep the longer ones earlier:
       256 x 15360   32: 13.0 16.8 17.4 11.6   16: 14.4 18.6 19.1 10.9
       640 x 16384   64: 21.9 23.4 26.3 22.1   32: 19.5 25.2 27.6 18.2"""
-    order = [preferred] if preferred else []
     weights = rows * cols if rows is not None else 1 << 32
-    if cols <= 4096 and weights < 15 << 18:
+    order = [preferred] if preferred else []
+    if not preferred and cols <= 4096 and weights < 15 << 18:
         order += [16]
-    elif weights < (11 << 20 if cols <= 8192 else SMALL_MATRIX):
+    elif weights < (11 << 20 if not preferred and cols <= 8192 else SMALL_MATRIX):
         order += [32, 64, 16, 128, 256]
     else:
         order += [64, 128, 32, 256, 16]

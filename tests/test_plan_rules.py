@@ -17,6 +17,14 @@ def test_segment_length_by_size(rows, cols, segment):
     assert _fused.choose_segment(cols, 16, rows=rows) == 16  # a caller's choice stands
 
 
+@pytest.mark.parametrize("rows,cols,asked,segment", [
+    (300, 1024, 64, 64), (300, 1056, 64, 32), (300, 1040, 64, 16), (300, 1152, 256, 32), (17408, 1152, 256, 64),
+    (300, 1088, 128, 32), (2000, 5280, 64, 32), (300, 144, 48, 48), (300, 1024, 8, 32), (17408, 1024, 8, 64),
+])
+def test_a_caller_that_asks_for_a_length_does_not_get_the_smallest_matrices_index(rows, cols, asked, segment):
+    assert _fused.choose_segment(cols, asked, rows=rows) == segment
+
+
 @pytest.mark.parametrize("class_rows,spr,whole", [
     ([64] * 16, 160, True),     # sixteen waves, one workgroup a compute unit
     ([16] * 15 + [17], 35, True),  # two a unit, 17 tiles for 512 slots
