@@ -99,6 +99,40 @@ def test_row_gather_clamps_rejects_and_reports(cols, segment):
     assert t.error.item() != 0
 
 
+@pytest.mark.parametrize("cols,segment", [(64 * 65, 64), (16 * 9, 16), (32 * 7, 32)])
+def test_gather_by_a_tiling_of_the_callers(cols, segment):
+    """grf_bctx_fused_gather, for callers of the C interface that name the rows in a slab tiling: any
+    order, a row twice, an empty slot, which leaves its output as it was."""
+    import ctypes
+    import torch
+    from georefine_amd import _fused, _hip_abi
+    from georefine_amd import bitexact_context_codec as codec
+    from georefine_amd.bitexact_context_gpu import HipContextTensor
+    rng = np.random.default_rng(cols)
+    words = (rng.choice([0x3C00, 0x3C20, 0x3D00], (70, cols)) | rng.integers(0, 32, (70, cols))).astype(np.uint16)
+    t = HipContextTensor(codec.encode(words), fused_segment=segment)
+    assert t.fused is not None
+    rows = np.array([69, 3, 3, 0xFFFFFFFF, 0, 41], dtype=np.uint32)
+    classes = np.array([t._plan.row_class[r] if r < 70 else 0 for r in rows], dtype=np.uint8)
+    spr = cols // segment
+    lanes = min(spr, 64)
+    scalars = dict(threads=64, lanes_per_row=lanes, rows_per_tile=1, n_slabs=-(-spr // lanes), n_tiles=len(rows),
+                   piece_cap=t._plan._cap(lanes), scheme=_fused.SCHEME_SLABS, k_parts=0)
+    block, position, _ = t._plan.residual_order()
+    _fused.validate_host(t._plan, dict(scalars=scalars, tile_rows=rows, tile_class=classes), "gather", row_pos=position, block=block)
+    on_device = torch.from_numpy(rows.view(np.int32)).cuda(), torch.from_numpy(classes).cuda()
+    g = _hip_abi.GrfFusedTiling()
+    g.tile_rows, g.tile_class = (a.data_ptr() for a in on_device)
+    for key, value in scalars.items():
+        setattr(g, key, value)
+    out = torch.full((len(rows) + 1, cols), 0x5A5A, device="cuda", dtype=torch.int16)
+    t._launch(t._lib.grf_bctx_fused_gather, ctypes.byref(t.fused), ctypes.byref(g), out.data_ptr(), t.error.data_ptr())
+    got = out.cpu().numpy().view(np.uint16)
+    for j, row in enumerate(rows):
+        assert np.array_equal(got[j], words[row] if row < 70 else np.full(cols, 0x5A5A, dtype=np.uint16)), j
+    assert (got[-1] == 0x5A5A).all() and t.error.item() == 0
+
+
 def test_row_gather_when_another_thread_took_the_last_word(monkeypatch):
     """The words that gathers report to are shared by threads: a list that was not empty a moment ago
     is no row outside the matrix."""
