@@ -39,9 +39,9 @@
 
 namespace grf {
 int set_error(int code, const std::string &what);                                          // decode_general.hip
-// fused_gemv.hip; wave_units: the entry point takes GRF_TILE_WAVES tilings
-enum TilingUse { kSlabTiling, kGemvTiling, kGemmTiling, kStoreTiling };  // what an entry point does with the tiling it is given
-// pointers: also refuse null device pointers (a host-side validation has none to give)
+// what an entry point does with the tiling it is given (kSlabTiling: takes no wave tilings)
+enum TilingUse { kSlabTiling, kGemvTiling, kGemmTiling, kStoreTiling };
+// fused_gemv.hip; pointers: also refuse null device pointers (a host-side validation has none to give)
 int check_fused_frame(const grf_bctx_fused &f, const grf_fused_tiling &g, const char *who, TilingUse use = kSlabTiling,
                       bool pointers = true);
 
@@ -1282,7 +1282,9 @@ __device__ __forceinline__ void fused_gemm_body(uint8_t *lds, const grf_bctx_fus
   if (bad) atomicOr(error, (int)bad);
 }
 
-// Up to four activation tiles: 80 vector registers, six waves per SIMD.
+// Up to four activation tiles: 80 vector registers, six waves per SIMD.  (Four tiles spill what is
+// needed before and after the slab loop only: 6 registers alone, 2 in the group form; the predictive
+// walker 2 and none.)
 template <class Walk, int MT, int SCAN, bool ROWS>
 __global__ __launch_bounds__(grf::kFusedMaxThreads) __attribute__((amdgpu_waves_per_eu(6))) void fused_gemm_kernel(
     grf_bctx_fused f, grf_fused_tiling g, GemmX x, uint32_t m_rows, uint16_t *y, uint32_t ldy,
@@ -1303,8 +1305,10 @@ __global__ __launch_bounds__(grf::kFusedMaxThreads) void fused_gemm_wide_kernel(
 }
 
 // Eight activation tiles where two workgroups can share a compute unit (shares_units): 80 registers,
-// six waves per SIMD, by holding the operands of two tiles at a time; ten waves more are resident in
-// return for waiting on the L2 three times a half group.  128 rows: q+k+v 6144 + 1024 + 1024 x 5120
+// six waves per SIMD, by holding the operands of two tiles at a time and by spilling, outside the slab
+// loop, what only the launch's beginning and end need (17 registers alone, 9 in the group form; the
+// predictive walker 7 and 6).  Ten waves more are resident in return for waiting on the L2 three times
+// a half group.  128 rows: q+k+v 6144 + 1024 + 1024 x 5120
 // 68.1 -> 59.5 us, gate+up 251 -> 234; 2048 x 5120 at 100 rows 34.1 -> 30.2.
 template <class Walk, int MT, int SCAN>
 __global__ __launch_bounds__(grf::kFusedMaxThreads) __attribute__((amdgpu_waves_per_eu(6))) void fused_gemm_shared_kernel(

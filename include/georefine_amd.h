@@ -346,7 +346,8 @@ int grf_bctx_fused_gather(const grf_bctx_fused *frame, const grf_fused_tiling *t
  * number of times; row_class: u8 [rows]; a wave walks `lanes` (4, 8, .. 64) segments of a row, and piece_cap is the
  * capacity of a piece of that many.  An id
  * outside the matrix sets GRF_ERR_INDEX in *index_error and leaves its output as it was; with index_error null
- * ids are clamped into the matrix.  error and index_error may be device memory or pinned host memory. */
+ * ids are clamped into the matrix.  out is 16-byte aligned.  error and index_error may be device memory or pinned
+ * host memory. */
 int grf_bctx_gather_rows(const grf_bctx_fused *frame, uint32_t lanes, uint32_t piece_cap, const uint8_t *row_class,
                          const int64_t *ids, uint32_t count, uint16_t *out, int32_t *error, int32_t *index_error, void *hip_stream);
 
@@ -361,9 +362,10 @@ int grf_bctx_gather_rows(const grf_bctx_fused *frame, uint32_t lanes, uint32_t p
  * a wave walks four lane-segments of 16 rows and feeds the words it decodes to the matrix
  * cores from its registers.  workspace: device memory, 16-byte
  * aligned, at least grf_gemm_workspace_bytes(cols, m_rows) bytes (grf_gemm_workspace_bytes_split
- * for a tiling with k_parts > 1); each launch first writes
- * its activation rows there in operand order (a copy of x: cols * 32 + 256 bytes per 16 rows),
- * so calls that share a workspace must be ordered on one stream. */
+ * for a tiling with k_parts > 1).  A launch of more than 64 rows, or of more than 2^27 weights x
+ * rows, first writes its activation rows there in operand order (a copy of x: cols * 32 + 256
+ * bytes per 16 rows); a smaller one reads x where it is.  Calls that share a workspace must be
+ * ordered on one stream. */
 int grf_bctx_gemm(const grf_bctx_fused *frame, const grf_fused_tiling *tiling, const uint16_t *x, uint32_t ldx,
                   uint32_t m_rows, uint16_t *y, uint32_t ldy, const uint16_t *bias, void *workspace,
                   size_t workspace_bytes, int32_t *error, void *hip_stream);
