@@ -1,0 +1,174 @@
+"""Profiles bench.py's workloads with rocprofv3 and writes the summaries that lie beside this file.
+
+    python3 profiles/summarize.py OUT [NAME ...]
+
+NAME: a key of WORKLOADS (default: all).  For each, one kernel trace and four counter runs (a run holds
+so many counters of a block), then OUT/NAME.txt, a table for readers, and OUT/NAME_traffic.json, which
+bench.py reads while the kernel sources are the ones recorded in it.
+
+What the derived lines say (MI355X: 8 XCDs, 256 compute units, 1024 SIMDs):
+  cycles of a launch     GRBM_GUI_ACTIVE / 8, since every XCD counts its own
+  VALU busy              4 SQ_ACTIVE_INST_VALU / (1024 cycles): the counter is in quad-cycles, summed over SIMDs
+  LDS busy               SQ_LDS_IDX_ACTIVE / (256 cycles): cycles the units' LDS pipes worked on indexed accesses
+                         (SQ_ACTIVE_INST_LDS counts the issue of the instructions only, and says next to
+                         nothing about the pipe), with the share SQ_LDS_BANK_CONFLICT of them
+  per wave step          totals / (weights / 64): a wave step is one symbol for each of a wave's 64 lanes
+"""
+import collections
+import csv
+import glob
+import json
+import os
+import statistics
+import subprocess
+import sys
+import tempfile
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+sys.path.insert(0, ROOT)
+import bench  # noqa: E402
+
+MLP = "Qwen-27B-like MLP (gate, up: 17408x5120; down: 5120x17408), MI355X (gfx950)"
+MATRIX = 5120 * 17408
+# title, bench.py's options, {kernel: weights a launch walks}, what the traffic record is called
+WORKLOADS = {
+    "fused_gemv_m1_qwen27b_mlp": (
+        f"Fused decode-GEMV (wave units), batch 1, {MLP}\n"
+        "one step = gate and up in one grouped launch (they take the same activations) + down in a launch of its own",
+        [], {"fused_wave_group_kernel": 2 * MATRIX, "fused_wave_kernel": MATRIX}, "Qwen-27B-like MLP batch 1"),
+    "fused_gemm_m64_qwen27b_mlp": (
+        f"Fused decode-GEMM (matrix cores), batch 64, {MLP}\n"
+        "one step = gate and up in one grouped launch + down cut in three along K",
+        ["--batch", "64"], {"fused_gemm_group_kernel": 2 * MATRIX, "fused_gemm_kernel": MATRIX}, "Qwen-27B-like MLP batch 64"),
+    "fused_store_decode_qwen27b_mlp": (
+        f"Fused decode to dense BF16 (store sink over wave units), {MLP}\none step = three launches",
+        ["--workload", "decode"], {"fused_wave_store_kernel": MATRIX}, "Qwen-27B-like MLP decode"),
+    "ppcx_gemv_m1_5120x17408": (
+        "Fused decode-GEMV of a predictive (PPCX) weight, 5120x17408, batch 1, MI355X (gfx950)",
+        ["--workload", "ppcx", "--batch", "1"], {"fused_wave_kernel": MATRIX}, "PPCX 5120x17408 batch 1"),
+    "ppcx_gemm_m96_5120x17408": (
+        "Fused decode-GEMM of a predictive (PPCX) weight, 5120x17408, 96 rows, MI355X (gfx950)",
+        ["--workload", "ppcx", "--batch", "96"],
+        {"fused_gemm_wide_kernel": MATRIX, "pack_activations_kernel": 0, "gemm_sum_parts_kernel": 0}, "PPCX 5120x17408 batch 96"),
+}
+COUNTERS = (
+    "SQ_WAVES SQ_INSTS_VALU SQ_INSTS_LDS SQ_INSTS_SALU SQ_ACTIVE_INST_VALU SQ_ACTIVE_INST_LDS SQ_BUSY_CU_CYCLES SQ_WAVE_CYCLES",
+    "SQ_LDS_BANK_CONFLICT SQ_LDS_IDX_ACTIVE SQ_LDS_ADDR_CONFLICT SQ_WAIT_INST_LDS SQ_WAIT_INST_ANY SQ_INSTS_VMEM_RD "
+    "SQ_LDS_UNALIGNED_STALL GRBM_GUI_ACTIVE",
+    "FETCH_SIZE", "WRITE_SIZE")
+COPY_BYTES = 128 << 20  # of bench.py's calibration copy, read once and written once
+RUN_SECONDS = 150
+
+
+def short(kernel):
+    return kernel.split("(")[0].split("<")[0].split("::")[-1].replace("void ", "").strip()
+
+
+def profiled(scratch, tag, options, arguments):
+    """One profiled run of bench.py; the directory with its CSV files."""
+    into = os.path.join(scratch, tag)
+    done = subprocess.run(
+        ["timeout", "-s", "KILL", str(RUN_SECONDS), "rocprofv3", *options, "-d", into, "-o", "r", "-f", "csv", "--", "python3",
+         os.path.join(ROOT, "bench.py"), "--no-cpu-baseline", "--no-extras", "--calibrate-copy", *arguments],
+        cwd=scratch, env=dict(os.environ, TMPDIR=scratch), stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    finished = any(line.startswith('{"metric"') for line in done.stdout.splitlines())
+    print(tag, done.returncode, flush=True)
+    if not finished:
+        sys.exit(done.stdout[-2000:])
+    return into
+
+
+def counters(directory):
+    """{kernel: {counter: [value of every dispatch]}}"""
+    found = collections.defaultdict(lambda: collections.defaultdict(list))
+    for path in glob.glob(directory + "/**/*counter_collection.csv", recursive=True):
+        total, kernel = collections.defaultdict(float), {}
+        for row in csv.DictReader(open(path)):
+            total[row["Dispatch_Id"], row["Counter_Name"]] += float(row["Counter_Value"])
+            kernel[row["Dispatch_Id"]] = row["Kernel_Name"]
+        for (dispatch, counter), value in total.items():
+            found[kernel[dispatch]][counter].append(value)
+    return found
+
+
+def derived(m, weights):
+    """The lines of one kernel's mean counters ``m`` that the totals do not show."""
+    cycles = m["GRBM_GUI_ACTIVE"] / 8
+    lines = [f"  -> {m['SQ_WAVES']:.0f} waves; VALU instructions per wave {m['SQ_INSTS_VALU'] / m['SQ_WAVES']:.0f}, LDS instructions "
+             f"per wave {m['SQ_INSTS_LDS'] / m['SQ_WAVES']:.0f}; cycles of the launch {cycles:.0f} (GRBM_GUI_ACTIVE / 8 XCDs)"]
+    if weights:
+        steps = weights / 64
+        lines.append(f"  -> per wave and symbol step, everything outside the step loop included: {m['SQ_INSTS_VALU'] / steps:.1f} VALU, "
+                     f"{m['SQ_INSTS_LDS'] / steps:.2f} LDS, {m['SQ_INSTS_SALU'] / steps:.1f} SALU, {m['SQ_INSTS_VMEM_RD'] / steps:.3f} "
+                     f"vector-memory read instructions; {m['SQ_LDS_IDX_ACTIVE'] / steps:.1f} LDS cycles")
+    conflicts = m["SQ_LDS_BANK_CONFLICT"] / m["SQ_LDS_IDX_ACTIVE"] if m["SQ_LDS_IDX_ACTIVE"] else 0.0
+    lines.append(f"  -> VALU busy {100 * 4 * m['SQ_ACTIVE_INST_VALU'] / (1024 * cycles):.1f} % of the launch's cycles (SQ_ACTIVE_INST_VALU "
+                 f"counts quad-cycles, 1024 SIMDs); LDS busy {100 * m['SQ_LDS_IDX_ACTIVE'] / (256 * cycles):.1f} % (SQ_LDS_IDX_ACTIVE, 256 "
+                 f"units), of which bank conflicts {100 * conflicts:.1f} %; waves waiting on anything "
+                 f"{100 * m['SQ_WAIT_INST_ANY'] / m['SQ_WAVE_CYCLES']:.1f} % of their cycles")
+    return lines
+
+
+def summarize(name, out, scratch):
+    title, arguments, kernels, workload = WORKLOADS[name]
+    fewer = [*arguments, "--steps", "20", "--warmup", "10"]
+    times = collections.defaultdict(list)
+    for path in glob.glob(profiled(scratch, name + "_trace", ["--kernel-trace", "--stats"], arguments) + "/**/*kernel_trace.csv",
+                          recursive=True):
+        for row in csv.DictReader(open(path)):
+            start, end = int(row["Start_Timestamp"]), int(row["End_Timestamp"])
+            times[row["Kernel_Name"]].append((start, (end - start) / 1e3))
+    text = [title, "rocprofv3 summaries (profiles/summarize.py); every run profiles the same command:",
+            "  T = python3 bench.py " + " ".join(["--no-cpu-baseline", "--no-extras", "--calibrate-copy", *arguments])
+            + "      (the bench line's own warm-up and timed steps)",
+            "  B = T --steps 20 --warmup 10      (counter runs serialise the kernels: fewer steps)",
+            "  (warm-up launches are eager; the timed ones are replays of HIP graphs, launched back to back as in the bench line;",
+            "   steps and launches take several device copies of the matrices in turn, so no matrix is found in the last-level cache;",
+            "   --calibrate-copy adds one plain copy kernel of known size, read by the two traffic counters below)",
+            "  rocprofv3 --kernel-trace --stats -- T", *(f"  rocprofv3 --pmc {c} -- B" for c in COUNTERS), "", "kernel trace:"]
+    whole = sum(t for launches in times.values() for _, t in launches)
+    for kernel, launches in sorted(times.items(), key=lambda item: -sum(t for _, t in item[1]))[:8]:
+        total = sum(t for _, t in launches)
+        text.append(f"  {kernel[:96]:<96} calls {len(launches):4d} total {total:10.1f} us  avg {total / len(launches):8.2f} us  "
+                    f"{100 * total / whole:5.1f}%")
+    for kernel in kernels:
+        us = [t for _, t in sorted(x for k, launches in times.items() if short(k) == kernel for x in launches)]
+        text.append(f"  {kernel}: {len(us)} launches, mean {statistics.mean(us):.2f} us, median {statistics.median(us):.2f} us, mean of "
+                    f"the later half {statistics.mean(us[len(us) // 2:]):.2f} us, fastest {min(us):.2f} us")
+    values, copy = collections.defaultdict(lambda: collections.defaultdict(list)), collections.defaultdict(list)
+    for i, names in enumerate(COUNTERS):
+        for kernel, found in counters(profiled(scratch, f"{name}_counters{i}", ["--pmc", *names.split()], fewer)).items():
+            for counter, of in found.items():
+                if short(kernel) in kernels:
+                    values[short(kernel)][counter] += of
+                elif "CUDAFunctorOnSelf_add<int>" in kernel:  # the calibration copy
+                    copy[counter] += of
+    fetch_scale, write_scale = (COPY_BYTES / (statistics.mean(copy[c]) * 1024) for c in ("FETCH_SIZE", "WRITE_SIZE"))
+    traffic = {}
+    for kernel, weights in kernels.items():
+        m = {counter: statistics.mean(of) for counter, of in values[kernel].items()}
+        fetched, written = m["FETCH_SIZE"] * 1024 * fetch_scale, m["WRITE_SIZE"] * 1024 * write_scale
+        traffic[kernel] = fetched + written
+        text += ["", f"counters, mean per launch of {kernel} (whole GPU):", *(f"  {c:<30} {m[c]:14.1f}" for c in sorted(m)),
+                 f"  -> HBM-side traffic per launch: fetch {fetched / 1e6:.1f} MB + write {written / 1e6:.2f} MB = "
+                 f"{(fetched + written) / 1e6:.1f} MB", *derived(m, weights)]
+    sources = bench.kernel_sources_sha256()
+    text += ["", f"traffic scale from the copy kernel: FETCH_SIZE x {fetch_scale:.4f}, WRITE_SIZE x {write_scale:.4f} KiB",
+             "kernel sources sha256 " + sources]
+    if workload.startswith("PPCX"):  # (a product may be several launches)
+        traffic = {"product": sum(traffic.values()), **traffic}
+    with open(os.path.join(out, name + ".txt"), "w") as f:
+        f.write("\n".join(text) + "\n")
+    with open(os.path.join(out, name + "_traffic.json"), "w") as f:
+        f.write(json.dumps({"workload": workload, "traffic_bytes_per_launch": traffic, "fetch_scale": fetch_scale,
+                            "write_scale": write_scale, "kernel_sources_sha256": sources}) + "\n")
+
+
+if __name__ == "__main__":
+    if len(sys.argv) < 2 or any(n not in WORKLOADS for n in sys.argv[2:]):
+        sys.exit(__doc__)
+    os.makedirs(sys.argv[1], exist_ok=True)
+    with tempfile.TemporaryDirectory() as scratch_dir:
+        for wanted in sys.argv[2:] or WORKLOADS:
+            summarize(wanted, os.path.abspath(sys.argv[1]), scratch_dir)
+            print(wanted, "done", flush=True)
