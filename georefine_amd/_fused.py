@@ -334,14 +334,18 @@ def search_wave_tilings(lengths, piece_cap_fn, lds_fn, cus, table_bytes):
                     longest = max(longest, busiest(units) * unit_steps[k])
                     tiles += counts[k][heights[k]]
                     steps += counts[k][heights[k]] * (units * unit_steps[k] + nwaves * table_steps)
+                chain, issue = (longest + table_steps) * WAVE_LATENCY_RATIO, steps / cus / 4  # (of one round)
+                if best is not None and max(chain, issue) >= best[0]:  # taller tiles only make longer chains
+                    if chain >= best[0]:
+                        break
+                    continue
                 lds = lds_fn(threads, p, heights, cap)
                 if lds > MAX_LDS:
                     break
                 # six waves per SIMD by registers; a little LDS stays with the system
                 per_cu = max(1, min(24 // nwaves, (MAX_LDS - 1024) // lds))
                 rounds = -(-tiles // (cus * per_cu))
-                chain = rounds * (longest + table_steps) * WAVE_LATENCY_RATIO
-                issue = steps / cus / 4
+                chain *= rounds
                 time = (chain ** 3 + issue ** 3) ** (1 / 3)
                 if best is None or time < best[0] * 0.9999:
                     best = (time, threads, p, tuple(heights), tiles, cap, lds, rounds * cus * per_cu)
