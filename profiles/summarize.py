@@ -4,7 +4,7 @@
 
 NAME: a key of WORKLOADS (default: all).  For each, one kernel trace and four counter runs (a run holds
 so many counters of a block), then OUT/NAME.txt, a table for readers, and OUT/NAME_traffic.json, which
-bench.py reads while the kernel sources are the ones recorded in it.
+bench.py reads while the kernel sources are the ones recorded in it.  The whole stack is traced only.
 
 What the derived lines say (MI355X: 8 XCDs, 256 compute units, 1024 SIMDs):
   cycles of a launch     GRBM_GUI_ACTIVE / 8, since every XCD counts its own
@@ -50,6 +50,10 @@ WORKLOADS = {
         "Fused decode-GEMM of a predictive (PPCX) weight, 5120x17408, 96 rows, MI355X (gfx950)",
         ["--workload", "ppcx", "--batch", "96"],
         {"fused_gemm_wide_kernel": MATRIX, "pack_activations_kernel": 0, "gemm_sum_parts_kernel": 0}, "PPCX 5120x17408 batch 96"),
+    "fused_gemm_m64_stack_64_layers": (
+        "Whole stack at the 27B model's shapes: 64 layers (48 with gated-delta-net projections, 16 with attention q/k/v/o) x "
+        "(projections, gate, up, down) + embedding and head (248320x5120), batch 64, MI355X (gfx950)",
+        ["--workload", "stack", "--steps", "3", "--warmup", "1"], {}, ""),
 }
 COUNTERS = (
     "SQ_WAVES SQ_INSTS_VALU SQ_INSTS_LDS SQ_INSTS_SALU SQ_ACTIVE_INST_VALU SQ_ACTIVE_INST_LDS SQ_BUSY_CU_CYCLES SQ_WAVE_CYCLES",
@@ -118,14 +122,14 @@ def summarize(name, out, scratch):
         for row in csv.DictReader(open(path)):
             start, end = int(row["Start_Timestamp"]), int(row["End_Timestamp"])
             times[row["Kernel_Name"]].append((start, (end - start) / 1e3))
-    text = [title, "rocprofv3 summaries (profiles/summarize.py); every run profiles the same command:",
+    text = [title, "rocprofv3 summaries (profiles/summarize.py) of",
             "  T = python3 bench.py " + " ".join(["--no-cpu-baseline", "--no-extras", "--calibrate-copy", *arguments])
             + "      (the bench line's own warm-up and timed steps)",
-            "  B = T --steps 20 --warmup 10      (counter runs serialise the kernels: fewer steps)",
+            *(["  B = T --steps 20 --warmup 10      (counter runs serialise the kernels: fewer steps)"] if kernels else []),
             "  (warm-up launches are eager; the timed ones are replays of HIP graphs, launched back to back as in the bench line;",
             "   steps and launches take several device copies of the matrices in turn, so no matrix is found in the last-level cache;",
-            "   --calibrate-copy adds one plain copy kernel of known size, read by the two traffic counters below)",
-            "  rocprofv3 --kernel-trace --stats -- T", *(f"  rocprofv3 --pmc {c} -- B" for c in COUNTERS), "", "kernel trace:"]
+            "   --calibrate-copy adds one plain copy kernel of known size, read by the traffic counters of the runs that take them)",
+            "  rocprofv3 --kernel-trace --stats -- T", *(f"  rocprofv3 --pmc {c} -- B" for c in COUNTERS if kernels), "", "kernel trace:"]
     whole = sum(t for launches in times.values() for _, t in launches)
     for kernel, launches in sorted(times.items(), key=lambda item: -sum(t for _, t in item[1]))[:8]:
         total = sum(t for _, t in launches)
@@ -135,6 +139,11 @@ def summarize(name, out, scratch):
         us = [t for _, t in sorted(x for k, launches in times.items() if short(k) == kernel for x in launches)]
         text.append(f"  {kernel}: {len(us)} launches, mean {statistics.mean(us):.2f} us, median {statistics.median(us):.2f} us, mean of "
                     f"the later half {statistics.mean(us[len(us) // 2:]):.2f} us, fastest {min(us):.2f} us")
+    sources = bench.kernel_sources_sha256()
+    if not kernels:
+        with open(os.path.join(out, name + ".txt"), "w") as f:
+            f.write("\n".join([*text, "", "kernel sources sha256 " + sources]) + "\n")
+        return
     values, copy = collections.defaultdict(lambda: collections.defaultdict(list)), collections.defaultdict(list)
     for i, names in enumerate(COUNTERS):
         for kernel, found in counters(profiled(scratch, f"{name}_counters{i}", ["--pmc", *names.split()], fewer)).items():
@@ -152,7 +161,6 @@ def summarize(name, out, scratch):
         text += ["", f"counters, mean per launch of {kernel} (whole GPU):", *(f"  {c:<30} {m[c]:14.1f}" for c in sorted(m)),
                  f"  -> HBM-side traffic per launch: fetch {fetched / 1e6:.1f} MB + write {written / 1e6:.2f} MB = "
                  f"{(fetched + written) / 1e6:.1f} MB", *derived(m, weights)]
-    sources = bench.kernel_sources_sha256()
     text += ["", f"traffic scale from the copy kernel: FETCH_SIZE x {fetch_scale:.4f}, WRITE_SIZE x {write_scale:.4f} KiB",
              "kernel sources sha256 " + sources]
     if workload.startswith("PPCX"):  # (a product may be several launches)
