@@ -412,7 +412,12 @@ std::vector<EncodeCell> encode_cells(const uint32_t *freq, uint32_t nctx, uint32
 template <class Fn>
 void in_parts(uint64_t n, uint64_t least, uint32_t parts, Fn fn) {
   parts = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>({parts, n / std::max<uint64_t>(1, least), std::max(1u, std::thread::hardware_concurrency())}));
-  std::vector<std::thread> others;
+  struct Threads : std::vector<std::thread> {  // joined however this ends: the work is on the caller's memory
+    ~Threads() {
+      for (auto &t : *this) t.join();
+    }
+  } others;
+  others.reserve(parts);
   uint32_t k = 0;
   for (; k + 1 < parts; ++k) try {
       others.emplace_back(fn, k, n * k / parts, n * (k + 1) / parts);
@@ -420,7 +425,6 @@ void in_parts(uint64_t n, uint64_t least, uint32_t parts, Fn fn) {
       break;
     }
   fn(k, n * k / parts, n);
-  for (auto &t : others) t.join();
 }
 
 // How far a walk has got, published now and then for a thread that follows it.
