@@ -128,12 +128,13 @@ def gemm_shape(p, r):
     return row_blocks, quads, row_blocks * quads * 64
 
 
-def lds_bytes_gemm(nc, lognb, tabn, p, r, piece_cap):
-    """Tables, then sixteen row pieces of four segments per wave; later every wave's partial sums."""
+def lds_bytes_gemm(nc, lognb, tabn, p, r, piece_cap, wave_bytes=0):
+    """Tables, then sixteen row pieces of four segments per wave (``wave_bytes`` for the sixteen, where
+    given); later every wave's partial sums."""
     a16 = lambda v: (v + 15) // 16 * 16
     waves = gemm_shape(p, r)[2] // 64
     total = a16(nc * (a16((tabn + 1) * 8) + (1 << lognb)))
-    total = a16(total + waves * 16 * piece_cap)
+    total = a16(total + waves * (wave_bytes or 16 * piece_cap))
     return max(total, waves * GEMM_MAX_TILES * 1024)
 
 
@@ -383,14 +384,22 @@ GEMM_K_PARTS = (1, 2, 3, 4, 6, 8)  # cuts along K the planner tries for a single
 
 
 def choose_gemm_tiling(spr, class_rows, piece_cap_fn, lds_fn, cus=256, seg_len=64, table_bytes=0, split=False):
+    """``plan_gemm_tiling`` where every row's piece is given the LDS of the longest."""
+    return plan_gemm_tiling(spr, class_rows, piece_cap_fn, lambda p, r, cap, _: lds_fn(p, r, cap), cus, seg_len, table_bytes,
+                            split)[:8]
+
+
+def plan_gemm_tiling(spr, class_rows, piece_cap_fn, lds_fn, cus=256, seg_len=64, table_bytes=0, split=False, unit_fn=None):
     """Tiling of the GEMM kernel: workgroups of (row blocks of 16) x (quads of 4
     lane-segments) waves.  Same model as choose_tiling, counted in waves: a wave is busy
     for as long as its busiest lane, so idle lanes inside a wave are free, idle waves and
     idle CUs are not.  With ``split`` the launch may also be cut into k parts along K (every
     row tile k times, each copy walking a k-th of the slabs, the parts' sums added by a small
     second kernel): a matrix with few rows then fills the machine with full blocks of sixteen
-    rows.  Returns (threads, lanes per row, rows per tile, slabs, tiles of the launch, piece
-    capacity, LDS bytes, k)."""
+    rows.  ``unit_fn()``: the LDS that the pieces of any sixteen rows take together, a fifth to a
+    third less than sixteen of the longest; a tiling reserves that where it lets more workgroups
+    share a compute unit.  Returns (threads, lanes per row, rows per tile, slabs, tiles of the
+    launch, piece capacity, LDS bytes, k, LDS bytes of a wave's pieces or 0)."""
     best = None
     total_rows = sum(int(c) for c in class_rows)
     tile_counts = _tile_counts(class_rows, 1024)
@@ -410,11 +419,16 @@ def choose_gemm_tiling(spr, class_rows, piece_cap_fn, lds_fn, cus=256, seg_len=6
         if k > n_slabs:
             continue
         cap = piece_cap_fn(p)
-        lds = lds_fn(p, r, cap)
+        by_waves = GEMM_WAVES_PER_SIMD // -(-(threads // 64) // 4)
+        lds, unit = lds_fn(p, r, cap, 0), 0
+        # (a quad's first segment is then a multiple of four, as in unit_fn's count)
+        if MAX_LDS // lds < by_waves and unit_fn is not None and (p % 4 == 0 or n_slabs == 1):
+            tight = lds_fn(p, r, cap, unit_fn())
+            if min(by_waves, MAX_LDS // tight) > MAX_LDS // lds:
+                lds, unit = tight, unit_fn()
         if lds > MAX_LDS:
             continue
-        per_simd = -(-(threads // 64) // 4)
-        per_cu = max(1, min(GEMM_WAVES_PER_SIMD // per_simd, MAX_LDS // lds))
+        per_cu = max(1, min(by_waves, MAX_LDS // lds))
         slots = cus * per_cu
         rounds = -(-(tile_counts[r] * k) // slots)
         # Spread over idle workgroup slots, except a single block of rows where one workgroup has a
@@ -436,7 +450,7 @@ def choose_gemm_tiling(spr, class_rows, piece_cap_fn, lds_fn, cus=256, seg_len=6
         if k > 1:  # the second kernel, and every part's sums written and read once more
             score *= 0.97 - 0.015 * k
         if best is None or score > best[0] + 1e-9:
-            best = (score, threads, p, r_used, n_slabs, tiles_used, cap, lds_fn(p, r_used, cap), k)
+            best = (score, threads, p, r_used, n_slabs, tiles_used, cap, lds_fn(p, r_used, cap, unit), k, unit)
     if best is None:
         raise FusedUnsupported("no GEMM tiling fits in LDS")
     return best[1:]
@@ -703,6 +717,18 @@ class FramePlan:
             self._caps["quad"] = quad_piece_capacity(self.seg_offset, self.rows, self.spr)
         return self._caps["quad"]
 
+    def quad_bytes(self):
+        """LDS bytes that the pieces of four segments of any sixteen rows that follow one another in a
+        class take, one behind the other in 16-byte units (``grf_unit_pieces``)."""
+        if "quads" not in self._caps:
+            order = np.argsort(self.row_class, kind="stable").astype(np.uint32)
+            most = ctypes.c_uint32()
+            if _native.codec().grf_unit_pieces(_native.ptr(self.seg_offset, ctypes.c_uint32), self.rows, self.spr,
+                                               _native.ptr(order, ctypes.c_uint32), 4, 16, ctypes.byref(most)):
+                raise FusedUnsupported("index offsets")
+            self._caps["quads"] = 16 * most.value
+        return self._caps["quads"]
+
     def _cap(self, p):
         if p not in self._caps:
             self._caps[p] = piece_capacity(self.seg_offset, self.rows, self.spr, p)
@@ -770,17 +796,17 @@ class FramePlan:
         """The one tiling every fused GEMM launch uses, whatever its row count: the order in
         which an output element accumulates follows the tiling, so it must not change with M."""
         self._wave_limits()
-        threads, p, r, n_slabs, n_tiles, cap, lds, k = choose_gemm_tiling(
+        threads, p, r, n_slabs, n_tiles, cap, lds, k, unit = plan_gemm_tiling(
             self.spr, self.class_rows, lambda lanes: self.quad_cap(),
-            lambda p_, r_, cap_: lds_bytes_gemm(self.nc, self.lognb, self.tabn, p_, r_, cap_),
-            seg_len=self.seg_len, table_bytes=self.table_bytes(), split=GEMM_SPLIT)
+            lambda p_, r_, cap_, unit_: lds_bytes_gemm(self.nc, self.lognb, self.tabn, p_, r_, cap_, unit_),
+            seg_len=self.seg_len, table_bytes=self.table_bytes(), split=GEMM_SPLIT, unit_fn=self.quad_bytes)
         # the row tiles; the launch has k of each
         tile_rows, tile_class, r, _ = build_gemm_tiles(self.row_class, self.nr, r)
         n_tiles = len(tile_class) * k
-        lds = lds_bytes_gemm(self.nc, self.lognb, self.tabn, p, r, cap)
+        lds = lds_bytes_gemm(self.nc, self.lognb, self.tabn, p, r, cap, unit)
         return dict(tile_rows=tile_rows, tile_class=tile_class,
                     scalars=dict(threads=threads, lanes_per_row=p, rows_per_tile=r, n_slabs=n_slabs,
-                                 n_tiles=n_tiles, piece_cap=cap, scheme=SCHEME_WAVES, k_parts=k), lds=lds)
+                                 n_tiles=n_tiles, piece_cap=cap, scheme=SCHEME_WAVES, k_parts=k, wave_bytes=unit), lds=lds)
 
 
 def plan_group(plans, m=None, gemm=False, waves=False, mixed=False):
@@ -808,10 +834,12 @@ def plan_group(plans, m=None, gemm=False, waves=False, mixed=False):
             pl._wave_limits()
     if gemm:
         scheme = SCHEME_WAVES
-        lds_fn = lambda p_, r_, cap_: max(lds_bytes_gemm(pl.nc, pl.lognb, pl.tabn, p_, r_, cap_) for pl in plans)
+        lds_fn = lambda p_, r_, cap_, unit_: max(lds_bytes_gemm(pl.nc, pl.lognb, pl.tabn, p_, r_, cap_, unit_) for pl in plans)
         quad_cap = max(pl.quad_cap() for pl in plans)
-        threads, p, r, _, _, cap, lds, _ = choose_gemm_tiling(first.spr, class_rows, lambda lanes: quad_cap, lds_fn,
-                                                              seg_len=first.seg_len, table_bytes=table)
+        # (lanes per row follow the first member's length: where another's differs, a slab may begin between two quads)
+        unit_fn = (lambda: max(pl.quad_bytes() for pl in plans)) if all(pl.spr == first.spr for pl in plans) else None
+        threads, p, r, _, _, cap, lds, _, unit = plan_gemm_tiling(first.spr, class_rows, lambda lanes: quad_cap, lds_fn,
+                                                                  seg_len=first.seg_len, table_bytes=table, unit_fn=unit_fn)
     elif waves:
         scheme = SCHEME_WAVES
         seg_lens = list(dict.fromkeys(pl.seg_len for pl in [first, *plans]))
@@ -838,7 +866,7 @@ def plan_group(plans, m=None, gemm=False, waves=False, mixed=False):
             cut.append(build_gemm_tiles(pl.row_class, pl.nr, r, first_tile=at, lead=lead))
             at, lead = at + len(cut[-1][1]), lead + cut[-1][3]
         height = max(c[2] for c in cut)
-        lds = lds_fn(p, height, cap)
+        lds = lds_fn(p, height, cap, unit)
         for pl, (tile_rows, tile_class, r_, _) in zip(plans, cut):
             if r_ != height:  # (a member the cut did not pay for: its slots widened to the common stride)
                 wide = np.full((len(tile_class), height), 0xFFFFFFFF, dtype=np.uint32)
@@ -846,7 +874,7 @@ def plan_group(plans, m=None, gemm=False, waves=False, mixed=False):
                 tile_rows = wide.reshape(-1)
             tilings.append(dict(tile_rows=tile_rows, tile_class=tile_class,
                                 scalars=dict(threads=threads, lanes_per_row=p, rows_per_tile=height, n_slabs=slabs(pl, p),
-                                             n_tiles=len(tile_class), piece_cap=cap, scheme=scheme), lds=lds))
+                                             n_tiles=len(tile_class), piece_cap=cap, scheme=scheme, wave_bytes=unit), lds=lds))
         return tilings
     for pl in plans:
         height = height_of[pl.seg_len] if waves else r

@@ -41,6 +41,16 @@ class GrfFusedTiling(ctypes.Structure):
         (name, ctypes.c_uint32) for name in (
             "threads", "lanes_per_row", "rows_per_tile", "n_slabs", "n_tiles", "piece_cap", "scheme", "k_parts")]
 
+    @property
+    def wave_bytes(self):
+        """LDS bytes reserved for the stream pieces of a matrix-core wave (bits 8 and above of ``scheme``,
+        in 16-byte units; 0: sixteen times ``piece_cap``)."""
+        return (self.scheme >> 8) * 16
+
+    @wave_bytes.setter
+    def wave_bytes(self, value):
+        self.scheme = (self.scheme & 0xFF) | (value // 16) << 8
+
 
 class GrfPpcxFused(ctypes.Structure):
     _fields_ = [(name, ctypes.c_void_p) for name in (

@@ -121,6 +121,8 @@ def codec():
             L.grf_sparse_tables.restype = _int
             L.grf_order_records.argtypes = [U8P, _u32, _u32, _u32, _u32, _u32, U32P, _u32, U8P]
             L.grf_order_records.restype = _int
+            L.grf_unit_pieces.argtypes = [U32P, _u32, _u32, U32P, _u32, _u32, U32P]
+            L.grf_unit_pieces.restype = _int
             L.p_encode.argtypes = [U16P, U16P, _u64, _u32, _u32, ctypes.POINTER(U32P), ctypes.POINTER(U8P),
                                    ctypes.POINTER(_sz)]
             L.p_decode.argtypes = [U8P, _sz, _u64, U16P, _u32, _u32, U32P, U16P]

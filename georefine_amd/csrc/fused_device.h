@@ -29,6 +29,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "georefine_amd.h"
 #include "rans_device.h"
 
@@ -45,6 +47,13 @@ __host__ __device__ inline uint32_t align_up(uint32_t v, uint32_t a) { return (v
 // lookup bytes.  With the block base in a register the table read needs no further
 // address arithmetic and the lookup read adds the uniform table size.
 __host__ __device__ inline uint32_t fused_table_bytes(const grf_bctx_fused &f) { return align_up((f.tabn + 1) * 8, 16); }
+
+// A tiling's scheme proper, and the LDS bytes that it reserves for the sixteen stream pieces of a
+// matrix-core wave (grf_fused_tiling.scheme).
+__host__ __device__ inline uint32_t tile_scheme(const grf_fused_tiling &g) { return g.scheme & 0xFFu; }
+__host__ __device__ inline uint32_t gemm_region_bytes(const grf_fused_tiling &g) {
+  return 16 * (g.scheme >> 8 ? g.scheme >> 8 : g.piece_cap);
+}
 
 // byte offsets of the LDS regions; shared by host (size) and device (carve).
 struct FusedLdsLayout {
@@ -472,33 +481,52 @@ __device__ __forceinline__ uint32_t fused_stage_piece_dma(uint8_t *lds, uint32_t
   return g0 & ~15u;
 }
 
-// The copy of a matrix-core wave's sixteen row pieces (four segments each, `cap` bytes of LDS a
-// piece).  Such a piece is 14 or so 16-byte units, so one row an instruction, as above, leaves three
-// quarters of the lanes idle and costs the wave some two hundred instructions a slab, a tenth of
-// what it issues: here the lanes are dealt to as many rows as fit (64 / (cap / 16)), and each
-// asks the row's own lane (lane r holds row r's byte range) where its unit lies.  Lane l's unit
-// lands at base + 16 l, which is its row's place because a row takes cap / 16 lanes.
-// Batch 64 gate+up 170 -> 156 us, attention q+k+v at 32 rows 45.5 -> 43, down at 6 rows 78 -> 76.
-__device__ __forceinline__ uint32_t fused_stage_rows_dma(uint8_t *lds, uint32_t region, uint32_t cap, const grf_bctx_fused &f,
-                                                         uint32_t g0, uint32_t g1, uint32_t lane) {
+constexpr uint32_t kPieceWindow = 8;  // bytes the refill reads from the aligned cursor on
+
+// The copy of a matrix-core wave's sixteen row pieces (four segments each).  Such a piece is ten or
+// eleven 16-byte units, so one row an instruction, as above, would leave most lanes idle: here the
+// units of all sixteen rows are numbered through, row after row, and an instruction moves 64 of
+// them to where they lie one behind the other.  Which row a unit belongs to: a row's units begin where those of the rows before it end (a
+// running sum over sixteen lanes); the row that begins at unit u of an instruction's 64 marks lane
+// u, and a lane counts the marks up to its own.  Lanes 0..15, and every sixteen after them, hold
+// the rows' byte ranges.  The region holds the most that any sixteen rows take together (166 of these
+// units on average and 175 at most in 17408 x 5120, where sixteen of the longest piece are 240), so
+// three workgroups of six waves share a compute unit that had two of ten.  Four rows an instruction at
+// the longest piece's pitch took as many instructions: gate+up at 64 rows 157.0 -> 155.6 us, at 128 rows
+// 230 -> 224, down at 64 rows 84.4 -> 83.0, 1500 x 2064 at 6 rows 15.8 -> 14.5.
+__device__ __forceinline__ uint32_t fused_stage_rows_dma(uint8_t *lds, uint32_t region, const grf_bctx_fused &f, uint32_t g0,
+                                                         uint32_t g1, uint32_t lane, uint32_t &piece_off) {
   typedef __attribute__((address_space(3))) void lds_void;
+  const uint32_t a0 = g0 & ~15u;
 #if defined(__HIP_DEVICE_COMPILE__)
-  const uint32_t units = cap >> 4;  // lanes per row (uniform)
-  if (units > 32) return fused_stage_piece_dma(lds, region, cap, f, g0, g1, lane, 0, 16);
-  const uint32_t rows = 64 / units;  // per instruction (uniform, scalar division)
-  const uint32_t mine = (lane * (65536 / units + 1)) >> 16, unit = lane - mine * units;  // lane / units, exact below 64
-  for (uint32_t r0 = 0; r0 < 16; r0 += rows) {  // uniform
-    const uint32_t r = r0 + mine;
-    const uint32_t s0 = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(r << 2), (int)g0) & ~15u;
-    const uint32_t s1 = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(r << 2), (int)g1);
-    const uint32_t o = s0 + unit * 16;
-    if (mine < rows && r < 16 && o < s1)
-      __builtin_amdgcn_global_load_lds(f.main_bytes + o, (lds_void *)(lds + (region + r0 * cap)), 16, 0, 0);
+  const uint32_t units = (g1 - a0 + kPieceWindow + 15) >> 4;  // (at least one: an empty slot's is never read)
+  uint32_t past = units;                                      // units of the rows up to and including the lane's
+  auto before = [&](auto ctrl) {  // the same of the lane so many rows before, 0 where there is none
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)past, decltype(ctrl)::value, 0xF, 0xF, true);
+  };
+  past += before(std::integral_constant<int, 0x111>{});  // row_shr:1
+  past += before(std::integral_constant<int, 0x112>{});
+  past += before(std::integral_constant<int, 0x114>{});
+  past += before(std::integral_constant<int, 0x118>{});
+  const uint32_t first = past - units;
+  piece_off = region + first * 16;
+  const uint32_t source = a0 - first * 16;  // unit u of the row comes from here + 16 u
+  const uint32_t total = __builtin_amdgcn_readlane(past, 15);
+  for (uint32_t u0 = 0; u0 < total; u0 += 64) {  // uniform
+    // the lane before the one that the next row begins at; the others push a zero to a lane that counts nothing
+    const uint32_t mark = past - u0 - 1;
+    const uint32_t hit = (uint32_t)__builtin_amdgcn_ds_permute((int)(min(mark, 63u) << 2), mark < 63 ? 1 : 0);
+    const uint64_t marks = __ballot(hit != 0);
+    const uint32_t done = (uint32_t)__builtin_popcountll(__ballot(past <= u0) & 0xFFFFu);  // rows that end before u0
+    const uint32_t row = __builtin_amdgcn_mbcnt_hi((uint32_t)(marks >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)marks, done));
+    const uint32_t o = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(row << 2), (int)source) + (u0 + lane) * 16;
+    if (u0 + lane < total && o < f.main_n_bytes)
+      __builtin_amdgcn_global_load_lds(f.main_bytes + o, (lds_void *)(lds + (region + u0 * 16)), 16, 0, 0);
   }
 #else
-  (void)lds, (void)region, (void)cap, (void)f, (void)g1, (void)lane;
+  (void)lds, (void)region, (void)f, (void)g1, (void)lane, (void)piece_off;
 #endif
-  return g0 & ~15u;
+  return a0;
 }
 
 // BF16 word in bits 0..15 (bits above are unspecified): symbol bits | mantissa low 5 bits
@@ -506,6 +534,21 @@ __device__ __forceinline__ uint32_t fused_stage_rows_dma(uint8_t *lds, uint32_t 
 // its low five bits are kept, one and-or.
 __device__ __forceinline__ uint32_t fused_word_bits(uint32_t hi, uint32_t r6_sign_extended) {
   return (r6_sign_extended & 0x801Fu) | hi;
+}
+
+// Two finished words as a pair, in a register of its own at once: left alone, the compiler puts the
+// merge of symbols and residuals off to the end of the eight steps, and what they are merged from
+// takes three times the registers meanwhile (GEMV of two rows 80 registers and 11 spilled -> 70; store
+// sink 80 and 9 spilled -> 70; matrix-core kernels of one, two and four tiles 66, 75 and 80 with 7
+// spilled -> 54, 63 and 79).  KEEP false: it may; a kernel that has the registers (GEMV of one row) then
+// waits for its residuals eight steps later, 1 % of the smallest launches.
+template <bool KEEP>
+__device__ __forceinline__ uint32_t fused_word_pair(uint32_t first, uint32_t second) {
+  uint32_t pair = __builtin_amdgcn_perm(second, first, 0x05040100u);
+#if defined(__HIP_DEVICE_COMPILE__)
+  if constexpr (KEEP) asm volatile("" : "+v"(pair));
+#endif
+  return pair;
 }
 
 // A lane's walk over one segment: rANS cursor, plus the registers that hold the packed
@@ -602,7 +645,7 @@ struct SegmentWalkT {
   }
   // Half H (0 or 1) of the group: eight symbols into four BF16 pairs (word k in the low
   // half, k+1 in the high half).
-  template <int H, int SCAN = kScanAny>
+  template <int H, int SCAN = kScanAny, bool KEEP = true>
   __device__ __forceinline__ void half(const FusedParams &q, uint32_t (&pair)[4]) {
     uint32_t bits[8];
 #define GRF_STEP2(i)                                                                   \
@@ -611,11 +654,10 @@ struct SegmentWalkT {
     fused_symbol_pair<8 * H + (i), SCAN>(c, cw[(8 * H + (i)) / 4], q, h0, h1);         \
     bits[i] = fused_word_bits(h0, rr.field<8 * H + (i)>());                            \
     bits[(i) + 1] = fused_word_bits(h1, rr.field<8 * H + (i) + 1>());                  \
+    pair[(i) / 2] = fused_word_pair<KEEP>(bits[i], bits[(i) + 1]);                     \
   }
     GRF_STEP2(0) GRF_STEP2(2) GRF_STEP2(4) GRF_STEP2(6)
 #undef GRF_STEP2
-#pragma unroll
-    for (int k = 0; k < 4; ++k) pair[k] = __builtin_amdgcn_perm(bits[2 * k + 1], bits[2 * k], 0x05040100u);
   }
   // Symbols [t, t+16) of the segment into eight BF16 pairs.
   __device__ __forceinline__ void decode16(uint32_t t, uint32_t S, const FusedParams &q, uint32_t (&pair)[8]) {

@@ -13,18 +13,18 @@ int check_fused_frame(const grf_bctx_fused &f, const grf_fused_tiling &g, const 
     return bad("segment length must be a multiple of 16 that divides the row length");
   if (!g.threads || g.threads % 64 || g.threads > (uint32_t)grf::kFusedMaxThreads) return bad("thread count");
   // (row positions too stay below 2^24: they go up to the rows rounded up to 16, plus 16 per row class)
-  if ((use == kGemmTiling || g.scheme == GRF_TILE_WAVES) &&
+  if ((use == kGemmTiling || grf::tile_scheme(g) == GRF_TILE_WAVES) &&
       ((uint64_t)f.rows + 16 + 16ull * f.nr >= (1u << 24) || f.cols >= (1u << 24)))
     return grf::set_error(GRF_UNSUPPORTED, std::string(who) + ": wave tilings take fewer than 2^24 rows and columns");
   if (use == kGemmTiling) {  // waves of 16 rows x 4 segments with their own stream pieces
-    if (g.scheme != GRF_TILE_WAVES) return bad("the GEMM takes a wave tiling (piece_cap for pieces of four segments)");
+    if (grf::tile_scheme(g) != GRF_TILE_WAVES) return bad("the GEMM takes a wave tiling (piece_cap for pieces of four segments)");
     if (!g.lanes_per_row || !g.rows_per_tile) return bad("empty tile");
-  } else if (g.scheme == GRF_TILE_WAVES) {
+  } else if (grf::tile_scheme(g) == GRF_TILE_WAVES) {
     if (use != kGemvTiling && use != kStoreTiling) return bad("this entry point takes slab tilings only");
     const uint32_t lanes = g.lanes_per_row;
     if (lanes < 4 || lanes > 64 || (lanes & (lanes - 1))) return bad("a wave unit has 4, 8, 16, 32 or 64 lanes per row");
     if (!g.rows_per_tile) return bad("empty tile");
-  } else if (g.scheme != GRF_TILE_SLABS) {
+  } else if (grf::tile_scheme(g) != GRF_TILE_SLABS) {
     return bad("tiling scheme");
   } else if (!g.lanes_per_row || !g.rows_per_tile || g.lanes_per_row * g.rows_per_tile > g.threads) {
     return bad("tile does not fit one workgroup");
@@ -34,6 +34,7 @@ int check_fused_frame(const grf_bctx_fused &f, const grf_fused_tiling &g, const 
   if (f.shift > 12 || f.lognb != 16 - f.shift) return bad("bucket shift");
   if (f.tabn == 0 || f.tabn > 255) return bad("sparse table size");
   if (g.piece_cap % 16 || g.piece_cap < 16) return bad("piece capacity");
+  if (g.scheme >> 8 && (use != kGemmTiling || g.scheme >> 8 > 160 * 1024 / 16)) return bad("LDS reserved for a wave's pieces");
   if ((uint64_t)f.rows * f.cols > 0xFFFFFFFFull) return bad("matrix too large");
   if (f.raw_interleaved > 16 || (f.raw_interleaved & (f.raw_interleaved - 1)))
     return bad("raw_interleaved is 0 or a block of 1, 2, 4, 8 or 16 rows");
@@ -107,11 +108,27 @@ int validate_fused_host(const grf_bctx_fused &f, const grf_fused_tiling &g, Tili
       for (uint32_t s = b; s < std::min(spr, b + g.lanes_per_row); s += lanes) {
         const uint32_t last = std::min(std::min(spr, b + g.lanes_per_row), s + lanes);
         const uint64_t span = (uint64_t)off[last] - (off[s] & ~15u) + 8;
-        if (span > g.piece_cap)
+        if (!(g.scheme >> 8) && span > g.piece_cap)
           return bad("the stream piece of row " + std::to_string(row) + " from segment " + std::to_string(s) +
                      " needs " + std::to_string(span) + " bytes, piece_cap is " + std::to_string(g.piece_cap));
       }
   }
+  if (g.scheme >> 8)  // the pieces of a matrix-core wave's sixteen slots together (an empty slot takes a unit)
+    for (uint32_t t = 0; t < row_tiles; ++t)
+      for (uint32_t r0 = 0; r0 < g.rows_per_tile; r0 += 16)
+        for (uint32_t b = 0; b < spr; b += g.lanes_per_row)
+          for (uint32_t s = b; s < std::min(spr, b + g.lanes_per_row); s += lanes) {
+            const uint32_t last = std::min(std::min(spr, b + g.lanes_per_row), s + lanes);
+            uint64_t sum = 0;
+            for (uint32_t r = r0; r < r0 + 16; ++r) {
+              const uint32_t row = r < g.rows_per_tile ? tile_rows[(uint64_t)t * g.rows_per_tile + r] : grf::kNoRow;
+              sum += row == grf::kNoRow ? 16 : (entry(row, last) - (uint64_t)(entry(row, s) & ~15u) + 8 + 15) / 16 * 16;
+            }
+            if (sum > gemm_region_bytes(g))
+              return bad("the stream pieces of slots " + std::to_string(r0) + " on of tile " + std::to_string(t) + " from segment " +
+                         std::to_string(s) + " need " + std::to_string(sum) + " bytes, the tiling reserves " +
+                         std::to_string(gemm_region_bytes(g)));
+          }
   if (row_pos) {  // one-to-one positions inside the residual array
     if (!f.raw_interleaved) return bad("row positions belong to the interleaved residual order");
     uint32_t top = 0;
@@ -124,7 +141,7 @@ int validate_fused_host(const grf_bctx_fused &f, const grf_fused_tiling &g, Tili
   }
   uint32_t lds = 0;
   if (use == kGemmTiling) lds = GemmLdsLayout(f, g).total;
-  else if (g.scheme == GRF_TILE_WAVES) lds = WaveLdsLayout(f, g, use == kStoreTiling ? 0 : kWaveRowsPerPass).total;
+  else if (grf::tile_scheme(g) == GRF_TILE_WAVES) lds = WaveLdsLayout(f, g, use == kStoreTiling ? 0 : kWaveRowsPerPass).total;
   else lds = FusedLdsLayout(f, g, use == kGemvTiling ? 1 : 0).total;
   if (lds > 160 * 1024) return bad("the launch needs " + std::to_string(lds) + " bytes of LDS");
   return GRF_OK;
@@ -135,7 +152,7 @@ extern "C" {
 
 uint32_t grf_bctx_fused_lds_bytes(const grf_bctx_fused *frame, const grf_fused_tiling *tiling, uint32_t m_rows) {
   if (!frame || !tiling) return 0;
-  if (tiling->scheme == GRF_TILE_WAVES)  // passes of at most two activation rows
+  if (grf::tile_scheme(*tiling) == GRF_TILE_WAVES)  // passes of at most two activation rows
     return grf::WaveLdsLayout(*frame, *tiling, m_rows < grf::kWaveRowsPerPass ? m_rows : grf::kWaveRowsPerPass).total;
   return grf::FusedLdsLayout(*frame, *tiling, m_rows).total;
 }
@@ -172,7 +189,7 @@ int grf_bctx_fused_decode(const grf_bctx_fused *frame, const grf_fused_tiling *t
   if (!frame || !tiling || !out || !error)
     return grf::set_error(GRF_BAD_ARGUMENT, "grf_bctx_fused_decode: null argument");
   if (int rc = grf::check_fused_frame(*frame, *tiling, "grf_bctx_fused_decode", grf::kStoreTiling)) return rc;
-  if (tiling->scheme == GRF_TILE_WAVES)
+  if (grf::tile_scheme(*tiling) == GRF_TILE_WAVES)
     return grf::launch_wave_store<grf::SegmentWalk>(*frame, *tiling, out, error, (hipStream_t)hip_stream);
   if (grf::reads_ahead(*frame))
     return grf::launch_walk<grf::SegmentWalkAhead, 1, grf::kStore>(*frame, *tiling, nullptr, 0, nullptr, 0, nullptr,

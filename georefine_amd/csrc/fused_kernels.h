@@ -3,7 +3,7 @@
 // in fused_ppcx.hip).  A walker provides prefetch(frame, segment, first element, first
 // column, segment's number in its row, the row's position in the residual order),
 // start(piece offset, staged-from offset),
-// begin16(t, S) + half<0|1, scan kind>(params, pair[4]) for the two halves of a group of
+// begin16(t, S) + half<0|1, scan kind, keep pairs>(params, pair[4]) for the two halves of a group of
 // 16 symbols (decode16 = all three) and ended_on_checkpoint(frame).
 //
 // GEMV: reduction order of one output element, fixed for every M: the S products of a
@@ -345,17 +345,6 @@ __device__ __forceinline__ void transpose_quad(uint32_t (&u)[4][4], uint32_t lan
 #endif
 }
 
-// Keeps four finished pairs of words in four registers: left alone, the compiler puts the merge of
-// symbols and residuals off to where the words are used, and what they are merged from takes
-// three times the registers meanwhile (and was spilled in the loop).
-__device__ __forceinline__ void pin_words(uint32_t (&v)[4]) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]));
-#else
-  (void)v;
-#endif
-}
-
 // The walk of a unit whose words go to the dense matrix; every lane of the wave takes part (the
 // exchange above reads all of a quad's lanes), those without a segment (`walks` false) store nothing.
 // first: the segment's first word in the output.  S is a multiple of 16.
@@ -381,14 +370,10 @@ __device__ __forceinline__ void store_segment(Walk &w, const grf::FusedParams &q
     uint32_t u[4][4];
     if (walks) {
       w.template half<0, SCAN>(q, u[0]);
-      pin_words(u[0]);
       w.template half<1, SCAN>(q, u[1]);
-      pin_words(u[1]);
       w.begin16(t + 16, S);
       w.template half<0, SCAN>(q, u[2]);
-      pin_words(u[2]);
       w.template half<1, SCAN>(q, u[3]);
-      pin_words(u[3]);
       // (the next group's loads leave before the stores: memory operations complete in order, so a
       // wait for a load that followed them would wait for them too)
       if (t + 32 < S) w.begin16(t + 32, S);
@@ -586,10 +571,10 @@ __device__ __forceinline__ void fused_wave_body(uint8_t *lds, const grf_bctx_fus
         uint32_t pair[4];
         load_x(xb, t + 8);
         w.begin16(t, S);
-        w.template half<0, SCAN>(q, pair);
+        w.template half<0, SCAN, M != 1>(q, pair);
         contract(pair, xa);
         load_x(xa, min(t + 16, S - 8));  // the last group loads a half again rather than branch around the load
-        w.template half<1, SCAN>(q, pair);
+        w.template half<1, SCAN, M != 1>(q, pair);
         contract(pair, xb);
       };
       // two groups per trip: the registers that carry the next group's residuals, classes and
@@ -926,7 +911,7 @@ int launch_gemv(const char *who, const grf_bctx_fused &f, const grf_fused_tiling
     return grf::set_error(GRF_BAD_ARGUMENT,
                           std::string(who) + ": x must be 4-byte aligned with an even leading dimension");
   using Ahead = typename ahead_of<Walk>::type;
-  if (g.scheme == GRF_TILE_WAVES) return launch_wave_rows<Walk>(who, f, g, x, ldx, m_rows, y, ldy, bias, error, s);
+  if (grf::tile_scheme(g) == GRF_TILE_WAVES) return launch_wave_rows<Walk>(who, f, g, x, ldx, m_rows, y, ldy, bias, error, s);
   if (!std::is_same<Ahead, Walk>::value && reads_ahead(f) && m_rows <= kAheadMaxRows) switch (m_rows) {
       case 1: return launch_walk<Ahead, 1, kDot>(f, g, x, ldx, y, ldy, bias, nullptr, error, s);
       case 2: return launch_walk<Ahead, 2, kDot>(f, g, x, ldx, y, ldy, bias, nullptr, error, s);
@@ -975,17 +960,17 @@ struct GemmShape {
   }
 };
 
-// Tables, then for every wave the pieces of its sixteen rows (piece_cap: the capacity of a
-// piece of four segments); the same memory later holds the partial sums of every wave (1 KiB
-// per wave and activation tile).
+// Tables, then for every wave the pieces of its sixteen rows (gemm_region_bytes); the same memory
+// later holds the partial sums of every wave (1 KiB per wave and activation tile).
 struct GemmLdsLayout {
-  uint32_t blocks, block_pitch, stream, total;
+  uint32_t blocks, block_pitch, region, stream, total;
   __host__ __device__ GemmLdsLayout(const grf_bctx_fused &f, const grf_fused_tiling &g) {
     blocks = 0;
     block_pitch = grf::fused_table_bytes(f) + (1u << f.lognb);
     stream = grf::align_up(f.nc * block_pitch, 16);
     const uint32_t waves = GemmShape(g).threads / 64;
-    total = grf::align_up(stream + waves * 16 * g.piece_cap, 16);
+    region = grf::gemm_region_bytes(g);
+    total = grf::align_up(stream + waves * region, 16);
     const uint32_t sums = waves * kSumTiles * 1024;
     if (total < sums) total = sums;
   }
@@ -1126,11 +1111,9 @@ __device__ __forceinline__ void fused_gemm_body(uint8_t *lds, const grf_bctx_fus
 
   // A wave keeps its sixteen rows and its quad of lane-segments for the whole launch and goes
   // through the slabs on its own: in slab b it walks segments b * P + 4 * quad .. + 3 of every
-  // row.  It copies the rows' pieces of those four segments to its own part of the LDS (the
-  // loads write the LDS directly, one row per instruction), so the waves of a workgroup share
-  // the tables and nothing else until their partial sums meet at the end.
-  const uint32_t region = L.stream + wave * 16 * g.piece_cap;
-  const uint32_t piece_off = region + (lane % 16) * g.piece_cap;
+  // row.  It copies the rows' pieces of those four segments to its own part of the LDS, so the
+  // waves of a workgroup share the tables and nothing else until their partial sums meet at the end.
+  const uint32_t region = L.stream + wave * L.region;
   // byte range of the lane's row piece in a slab; lanes without a row, and slabs past the row's
   // end, read the matrix's first entry and get an empty range (no load sits in a branch)
   auto span_of = [&](uint32_t b, uint32_t &g0, uint32_t &g1) {
@@ -1165,7 +1148,8 @@ __device__ __forceinline__ void fused_gemm_body(uint8_t *lds, const grf_bctx_fus
     const bool active = row != grf::kNoRow && p4 < nseg;
     const uint32_t col0 = mul24(first_seg + p4, S);
     // the pieces first: their ranges arrived during the walk before
-    const uint32_t a0 = grf::fused_stage_rows_dma(lds, region, g.piece_cap, f, g0, g1, lane);
+    uint32_t piece_off;
+    const uint32_t a0 = grf::fused_stage_rows_dma(lds, region, f, g0, g1, lane, piece_off);
     Walk w;
     {
       const uint32_t seg = grf::fused_seg_slot<true>(f, active ? row : 0, active ? rpos : 0, active ? first_seg + p4 : 0);
@@ -1282,9 +1266,7 @@ __device__ __forceinline__ void fused_gemm_body(uint8_t *lds, const grf_bctx_fus
   if (bad) atomicOr(error, (int)bad);
 }
 
-// Up to four activation tiles: 80 vector registers, six waves per SIMD.  (Four tiles spill what is
-// needed before and after the slab loop only: 6 registers alone, 2 in the group form; the predictive
-// walker 2 and none.)
+// Up to four activation tiles: at most 80 vector registers, six waves per SIMD, and none spilled.
 template <class Walk, int MT, int SCAN, bool ROWS>
 __global__ __launch_bounds__(grf::kFusedMaxThreads) __attribute__((amdgpu_waves_per_eu(6))) void fused_gemm_kernel(
     grf_bctx_fused f, grf_fused_tiling g, GemmX x, uint32_t m_rows, uint16_t *y, uint32_t ldy,
@@ -1306,8 +1288,7 @@ __global__ __launch_bounds__(grf::kFusedMaxThreads) void fused_gemm_wide_kernel(
 
 // Eight activation tiles where two workgroups can share a compute unit (shares_units): 80 registers,
 // six waves per SIMD, by holding the operands of two tiles at a time and by spilling, outside the slab
-// loop, what only the launch's beginning and end need (17 registers alone, 9 in the group form; the
-// predictive walker 7 and 6).  Ten waves more are resident in return for waiting on the L2 three times
+// loop, three registers that only the launch's beginning and end need (the predictive walker none).  Ten waves more are resident in return for waiting on the L2 three times
 // a half group.  128 rows: q+k+v 6144 + 1024 + 1024 x 5120
 // 68.1 -> 59.5 us, gate+up 251 -> 234; 2048 x 5120 at 100 rows 34.1 -> 30.2.
 template <class Walk, int MT, int SCAN>
@@ -1529,7 +1510,7 @@ inline int build_group(const char *who, const GroupSpec &spec, bool gemm, FusedG
     if (int rc = grf::check_fused_frame(f, g, who, gemm ? kGemmTiling : kGemvTiling)) return rc;
     if (f.cols != spec.frames[0]->cols) return bad("members must have one width");
     if (g.threads != spec.tilings[0]->threads) return bad("member tilings must share one thread count");
-    if (g.scheme != spec.tilings[0]->scheme) return bad("member tilings must share one scheme");
+    if (grf::tile_scheme(g) != grf::tile_scheme(*spec.tilings[0])) return bad("member tilings must share one scheme");
     if (g.k_parts > 1) return bad("grouped launches take tilings that are not cut along K (k_parts <= 1)");
     if (gemm && GemmShape(g).threads != g.threads)
       return bad("tiling threads must be 64 x ceil(rows_per_tile / 16) x ceil(lanes_per_row / 4)");
@@ -1568,7 +1549,7 @@ int launch_gemv_group(const char *who, const GroupSpec &spec, const uint16_t *x,
   if (!x || ldx < a.f[0].cols || (ldx & 1) || ((uintptr_t)x & 3))
     return grf::set_error(GRF_BAD_ARGUMENT,
                           std::string(who) + ": x must be 4-byte aligned with an even leading dimension");
-  if (a.g[0].scheme == GRF_TILE_WAVES) {
+  if (grf::tile_scheme(a.g[0]) == GRF_TILE_WAVES) {
     uint32_t lds = 0;
     for (uint32_t i = 0; i < a.n; ++i) {
       if (int rc = check_wave_operands(who, a.f[i], x, ldx)) return rc;

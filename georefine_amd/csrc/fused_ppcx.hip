@@ -185,7 +185,7 @@ struct PpcxWalk {
     n2 = d[2];
     nb = group_bins(next);
   }
-  template <int H, int SCAN = grf::kScanAny>
+  template <int H, int SCAN = grf::kScanAny, bool KEEP = true>
   __device__ __forceinline__ void half(const grf::FusedParams &q, uint32_t (&pair)[4]) {
     uint32_t bits[8];
 #define GRF_STEP2(i)                                                                                  \
@@ -196,11 +196,10 @@ struct PpcxWalk {
     grf::fused_symbol_pair_in<SCAN>(c, __umul24(bin0, q.block_pitch), __umul24(bin1, q.block_pitch), q, h0, h1); \
     bits[i] = h0 | rr.field<8 * H + (i)>();                                                           \
     bits[(i) + 1] = h1 | rr.field<8 * H + (i) + 1>();                                                 \
+    pair[(i) / 2] = grf::fused_word_pair<KEEP>(bits[i], bits[(i) + 1]);                               \
   }
     GRF_STEP2(0) GRF_STEP2(2) GRF_STEP2(4) GRF_STEP2(6)
 #undef GRF_STEP2
-#pragma unroll
-    for (int k = 0; k < 4; ++k) pair[k] = __builtin_amdgcn_perm(bits[2 * k + 1], bits[2 * k], 0x05040100u);
   }
   __device__ __forceinline__ void decode16(uint32_t t, uint32_t S, const grf::FusedParams &q, uint32_t (&pair)[8]) {
     begin16(t, S);
@@ -283,7 +282,7 @@ int grf_ppcx_fused_decode(const grf_ppcx_fused *frame, const grf_fused_tiling *t
   if (!out || !error) return grf::set_error(GRF_BAD_ARGUMENT, "grf_ppcx_fused_decode: null argument");
   grf_bctx_fused f;
   if (int rc = walker_frame(frame, tiling, bins, "grf_ppcx_fused_decode", f, grf::kStoreTiling)) return rc;
-  if (tiling->scheme == GRF_TILE_WAVES)
+  if (grf::tile_scheme(*tiling) == GRF_TILE_WAVES)
     return grf::launch_wave_store<PpcxWalk>(f, *tiling, out, error, (hipStream_t)hip_stream);
   return grf::launch_walk<PpcxWalk, 1, grf::kStore>(f, *tiling, nullptr, 0, nullptr, 0, nullptr, out, error,
                                              (hipStream_t)hip_stream);

@@ -915,6 +915,33 @@ int grf_order_records(const uint8_t *src, uint32_t rows, uint32_t spr, uint32_t 
   return 0;
 }
 
+int grf_unit_pieces(const uint32_t *offsets, uint32_t rows, uint32_t spr, const uint32_t *row_order, uint32_t lanes,
+                    uint32_t together, uint32_t *most) {
+  if (!offsets || !row_order || !most || !spr || !lanes || !together) return 1;
+  const uint32_t slabs = (spr + lanes - 1) / lanes;
+  try {
+    // per slab, the units of the last `together` rows (the slots before the first are empty) and their sum
+    std::vector<uint32_t> units((size_t)together * slabs, 1), sum(slabs, together);
+    uint32_t top = together;
+    for (uint32_t i = 0, slot = 0; i < rows; ++i, slot = slot + 1 == together ? 0 : slot + 1) {
+      if (row_order[i] >= rows) return 1;
+      const uint32_t *at = offsets + (size_t)row_order[i] * spr;
+      uint32_t *oldest = units.data() + (size_t)slot * slabs;
+      for (uint32_t b = 0; b < slabs; ++b) {
+        const uint32_t first = at[b * lanes], last = at[std::min(spr, (b + 1) * lanes)];
+        const uint32_t n = (last - (first & ~15u) + 8 + 15) / 16;
+        sum[b] += n - oldest[b];
+        oldest[b] = n;
+        top = std::max(top, sum[b]);
+      }
+    }
+    *most = top;
+  } catch (...) {
+    return 3;
+  }
+  return 0;
+}
+
 // 10-bit main symbols + 6-bit residuals -> BF16 words (no reference counterpart:
 // the reference recombines in numpy, GCR/bitexact_context_codec.py:426).
 int grf_bctx_join(const uint16_t *main_sym, const uint16_t *res_sym, uint64_t n, uint16_t *out) {

@@ -82,6 +82,12 @@ int grf_sparse_tables(const uint32_t *freq, uint32_t nctx, uint32_t vocab, uint3
  * (((q / block * per_segment + t) * spr + s) * block + q % block).  dst holds `held` rows. */
 int grf_order_records(const uint8_t *src, uint32_t rows, uint32_t spr, uint32_t per_segment, uint32_t record_bytes,
                       uint32_t block, const uint32_t *position, uint32_t held, uint8_t *dst);
+/* The most 16-byte units of LDS that the stream pieces of `together` consecutive rows take in a slab of
+ * `lanes` segments, rows in the order given (row_order[rows]; past the last row an empty slot's one unit):
+ * a piece from the 16-byte aligned start of its first segment to the end of its last, + 8, in whole
+ * units.  offsets: the index in the frame's order, rows * spr + 1 entries. */
+int grf_unit_pieces(const uint32_t *offsets, uint32_t rows, uint32_t spr, const uint32_t *row_order, uint32_t lanes,
+                    uint32_t together, uint32_t *most);
 /* The stream bcx_encode writes, given the frequencies of bcx_frequencies, in the caller's buffer of at least
  * 2 n + 8 bytes: the stream is buffer[*begin .. buffer_bytes). */
 int grf_bctx_encode(const uint16_t *w, uint32_t rows, uint32_t cols, const uint8_t *rc, const uint8_t *cc, uint32_t nr,
@@ -272,6 +278,10 @@ typedef struct grf_bctx_fused {
  *               lanes_per_row segments for the whole launch and stages its own stream pieces
  *               (see grf_bctx_gemm for threads and piece_cap).
  *               Wave tilings take matrices with fewer than 2^24 rows and 2^24 columns.
+ *               Bits 8 and above of scheme (GEMM): the LDS reserved for the sixteen stream pieces of
+ *               a wave, in 16-byte units.  They lie one behind the other, each in as many units as
+ *               it needs (its span as above, + 8; an empty slot takes one): at least the most that any
+ *               wave's take together.  0: sixteen times piece_cap.
  *   k_parts     0 or 1: every tile walks all slabs.  k > 1 (grf_bctx_gemm / grf_ppcx_gemm only):
  *               the launch is cut along K: tile_rows / tile_class describe n_tiles / k row
  *               tiles, which must hold every row of the matrix once; launch tile t is row tile
@@ -281,6 +291,7 @@ typedef struct grf_bctx_fused {
  * n_slabs = ceil(segs_per_row / lanes_per_row) in both schemes. */
 #define GRF_TILE_SLABS 0
 #define GRF_TILE_WAVES 1
+#define GRF_TILE_WAVE_UNITS(units) ((uint32_t)(units) << 8)
 typedef struct grf_fused_tiling {
   const uint32_t *tile_rows;
   const uint8_t *tile_class;
