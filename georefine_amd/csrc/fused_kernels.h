@@ -1190,33 +1190,59 @@ __device__ __forceinline__ void fused_gemm_body(uint8_t *lds, const grf_bctx_fus
                        : ((feeds ? col0 / 8 : K / 8) * m_pad + ln % 16) * 16;
     // (zeros for the lanes that do not walk, once: a walking lane overwrites its own)
     uint32_t words[4] = {0u, 0u, 0u, 0u};
-    uint4 xa[XT];
-    load_x(xa, xl);
-    auto contract = [&]() {
-      gemm_contract<0>(acc, xa, words);
-      auto next = [&](auto first) {  // (XT < MT only)
-        load_x(xa, xl + decltype(first)::value * 256u);
-        gemm_contract<decltype(first)::value>(acc, xa, words);
+    if constexpr (ROWS && MT == 1) {
+      // A group's two operands at once, so that a line of x is visited four times a segment instead of eight,
+      // and none past the segment's end (in place, half by half and so: 5120 x 17408 at two rows 70.9 -> 69.5
+      // us, 6144 + 1024 + 1024 x 5120 at six 41.8 -> 41.0).  Two groups at once gain no more and cost short
+      // segments 1 %; two tiles of rows gain nothing.
+      uint4 xa[1], xb[1];
+      auto fetch = [&]() {
+        load_x(xa, xl);
+        load_x(xb, xl + 16);
       };
-      if constexpr (XT < MT) {
-        static_assert(MT == 4 * XT && !ROWS);
-        next(std::integral_constant<int, XT>{});
-        next(std::integral_constant<int, 2 * XT>{});
-        next(std::integral_constant<int, 3 * XT>{});
+      fetch();
+      for (uint32_t t = 0;;) {
+        if (active) {
+          w.begin16(t, S);
+          w.template half<0, SCAN>(q, words);
+        }
+        gemm_contract<0>(acc, xa, words);
+        if (active) w.template half<1, SCAN>(q, words);
+        gemm_contract<0>(acc, xb, words);
+        t += 16;
+        if (t >= S) break;
+        xl += 2 * x_step;
+        fetch();
       }
-    };
-    for (uint32_t t = 0; t < S; t += 16) {
-      if (active) {
-        w.begin16(t, S);
-        w.template half<0, SCAN>(q, words);
+    } else {
+      uint4 xa[XT];
+      load_x(xa, xl);
+      auto contract = [&]() {
+        gemm_contract<0>(acc, xa, words);
+        auto next = [&](auto first) {  // (XT < MT only)
+          load_x(xa, xl + decltype(first)::value * 256u);
+          gemm_contract<decltype(first)::value>(acc, xa, words);
+        };
+        if constexpr (XT < MT) {
+          static_assert(MT == 4 * XT && !ROWS);
+          next(std::integral_constant<int, XT>{});
+          next(std::integral_constant<int, 2 * XT>{});
+          next(std::integral_constant<int, 3 * XT>{});
+        }
+      };
+      for (uint32_t t = 0; t < S; t += 16) {
+        if (active) {
+          w.begin16(t, S);
+          w.template half<0, SCAN>(q, words);
+        }
+        contract();
+        xl += x_step;
+        load_x(xa, xl);
+        if (active) w.template half<1, SCAN>(q, words);
+        contract();
+        xl += x_step;
+        load_x(xa, xl);
       }
-      contract();
-      xl += x_step;
-      load_x(xa, xl);
-      if (active) w.template half<1, SCAN>(q, words);
-      contract();
-      xl += x_step;
-      load_x(xa, xl);
     }
     if (active && !w.ended_on_checkpoint(f)) bad |= GRF_ERR_CHECKPOINT;
   }
@@ -1348,18 +1374,21 @@ static __global__ __launch_bounds__(256) void gemm_sum_parts_kernel(const float 
   y[(size_t)m * ldy + n] = round_bf16(sum);
 }
 
-// A small product reads the activations from the caller's own rows, which saves the launch of
-// the packing kernel (2.3 us of the host's time, 1.5 to 2.5 us of the GPU's).  In return a load's
-// lanes touch a cache line each instead of sharing eight or so, measured at 16 ns per million
-// (weights x rows): 17408 and 17408 x 5120 at 16 rows 143 -> 184 us, 6144 + 1024 + 1024 x 5120 at
-// 32 rows 43 -> 61, but 1024 x 5120 at 8 rows 17.8 -> 16.0, 1500 x 2048 at 20 rows 17.2 -> 15.5.
-// They break even near 200 million; the line is drawn at 128.  (Above four tiles of rows such a
+// A product of few rows, or a small one, reads the activations from the caller's own rows, which saves
+// the launch of the packing kernel (2.3 us of the host's time, 1.5 to 3 us of the GPU's).  In return a
+// load's lanes touch a cache line each instead of sharing eight or so.  Rows that a launch does not have cost
+// nothing (gemm_load_rows), so up to six rows it pays at any size: packed and in place, 5120 x 17408 at
+// two rows 72.4 -> 69.5 us, at six 73.2 -> 72.0, 17408 and 17408 x 5120 at four 143.3 -> 140.0, 6144 +
+// 1024 + 1024 x 5120 at six 42.3 -> 41.0; at sixteen rows 72.8 -> 88.8, 143.4 -> 149.0, 42 -> 46.  Above
+// six rows the line is drawn at 128 million weights x rows (1024 x 5120 at 8 rows 17.8 -> 16.0, 1500 x
+// 2048 at 20 rows 17.2 -> 15.5; 5120 x 6144 at 24 rows, 755 million, 42 -> 54).  (Above four tiles of rows such a
 // matrix has two million weights at most and the copy is a small part of the product.)
+inline constexpr uint32_t kOwnRowsAlways = 6;
 inline constexpr uint32_t kOwnRowsMax = 64;
 inline constexpr uint64_t kOwnRowsWork = 128u << 20;
 
 inline bool own_rows(const uint16_t *x, uint32_t ldx, uint32_t m_rows, uint64_t weights) {
-  return x && m_rows <= kOwnRowsMax && weights * m_rows <= kOwnRowsWork &&
+  return x && m_rows <= kOwnRowsMax && (m_rows <= kOwnRowsAlways || weights * m_rows <= kOwnRowsWork) &&
          (uint64_t)ldx * 2 * 16 * gemm_tiles(m_rows) < (1u << 31);  // (offsets are 32 bits wide)
 }
 

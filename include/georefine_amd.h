@@ -373,9 +373,9 @@ int grf_bctx_gather_rows(const grf_bctx_fused *frame, uint32_t lanes, uint32_t p
  * a wave walks four lane-segments of 16 rows and feeds the words it decodes to the matrix
  * cores from its registers.  workspace: device memory, 16-byte
  * aligned, at least grf_gemm_workspace_bytes(cols, m_rows) bytes (grf_gemm_workspace_bytes_split
- * for a tiling with k_parts > 1).  A launch of more than 64 rows, or of more than 2^27 weights x
- * rows, first writes its activation rows there in operand order (a copy of x: cols * 32 + 256
- * bytes per 16 rows); a smaller one reads x where it is.  Calls that share a workspace must be
+ * for a tiling with k_parts > 1).  A launch of more than 64 rows, or of more than six rows and
+ * 2^27 weights x rows, first writes its activation rows there in operand order (a copy of x: cols *
+ * 32 + 256 bytes per 16 rows); a smaller one reads x where it is.  Calls that share a workspace must be
  * ordered on one stream. */
 int grf_bctx_gemm(const grf_bctx_fused *frame, const grf_fused_tiling *tiling, const uint16_t *x, uint32_t ldx,
                   uint32_t m_rows, uint16_t *y, uint32_t ldy, const uint16_t *bias, void *workspace,
