@@ -1361,16 +1361,27 @@ __global__ __launch_bounds__(grf::kFusedMaxThreads) void fused_gemm_wide_group_k
 }
 
 // y[m][n] = bf16(partials[0][m][n] + partials[1][m][n] + ... + bias[n]): the parts of a
-// K-split launch, added in part order
+// K-split launch, added in part order.  The work is the latency of its loads, so a thread has four
+// parts' and the bias under way at a time (one after the other, and so: 700 x 9216 in four parts at six rows
+// 18.4 -> 17.6 us, 2048 x 5120 at 32 rows 21.3 -> 20.7).
 static __global__ __launch_bounds__(256) void gemm_sum_parts_kernel(const float *partials, uint32_t parts, uint32_t m_rows,
                                                                     uint32_t rows, const uint16_t *bias, uint16_t *y,
                                                                     uint32_t ldy) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= m_rows * rows) return;
-  const uint32_t m = i / rows, n = i - m * rows;
-  float sum = partials[i];
-  for (uint32_t p = 1; p < parts; ++p) sum += partials[(size_t)p * m_rows * rows + i];
-  if (bias) sum += __uint_as_float((uint32_t)bias[n] << 16);
+  const uint32_t n = blockIdx.x * blockDim.x + threadIdx.x, m = blockIdx.y;
+  if (n >= rows) return;
+  const float *own = partials + (size_t)m * rows + n;
+  const size_t pitch = (size_t)m_rows * rows;
+  const uint32_t b = bias ? bias[n] : 0;
+  float sum = 0.f;
+  for (uint32_t p = 0; p < parts; p += 4) {
+    float v[4];
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) v[k] = own[min(p + k, parts - 1) * pitch];  // (the last one again rather than a branch)
+    sum = p ? sum + v[0] : v[0];
+#pragma unroll
+    for (uint32_t k = 1; k < 4; ++k) sum = p + k < parts ? sum + v[k] : sum;
+  }
+  if (bias) sum += __uint_as_float(b << 16);
   y[(size_t)m * ldy + n] = round_bf16(sum);
 }
 
@@ -1435,7 +1446,7 @@ int launch_gemm_rows(const grf_bctx_fused &f, const grf_fused_tiling &g, const u
   };
   if (int rc = launch_scan_and_rows<MT>(f.whole_range, source.pitch != 0, launch)) return rc;
   if (g.k_parts > 1)
-    hipLaunchKernelGGL(gemm_sum_parts_kernel, dim3((m_rows * f.rows + 255) / 256), dim3(256), 0, s, partials, g.k_parts,
+    hipLaunchKernelGGL(gemm_sum_parts_kernel, dim3((f.rows + 255) / 256, m_rows), dim3(256), 0, s, partials, g.k_parts,
                        m_rows, f.rows, bias, y, ldy);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return grf::set_error(GRF_LAUNCH_FAILED, std::string("fused GEMM: ") + hipGetErrorString(e));
