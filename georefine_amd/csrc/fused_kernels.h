@@ -1100,9 +1100,6 @@ __device__ __forceinline__ void fused_gemm_body(uint8_t *lds, const grf_bctx_fus
 #else
   const uint32_t wave = tid / 64;
 #endif
-  // (the tables' copy first: it is under way while the reads below follow one another)
-  const bool tables_by_dma = grf::fused_tables_by_dma(f);
-  if (tables_by_dma) grf::fused_load_tables_dma(lds, L.blocks, L.block_pitch, f, cls, wave, nthreads / 64, lane);
   const uint32_t rb = wave % shape.row_blocks, quad = wave / shape.row_blocks;
   const uint32_t r = rb * 16 + lane % 16, p4 = lane / 16;
   uint32_t row = r < R ? g.tile_rows[tile * R + r] : grf::kNoRow;
@@ -1125,8 +1122,13 @@ __device__ __forceinline__ void fused_gemm_body(uint8_t *lds, const grf_bctx_fus
     g1 = grf::fused_index_entry(f.seg_offset, slot + mul24(past, grf::fused_seg_step(f)));
   };
   uint32_t g0, g1;
-  span_of(b_first, g0, g1);  // started before the table copy so that the latencies overlap
-  if (!tables_by_dma) grf::fused_load_tables(lds, L.blocks, L.block_pitch, f, cls, tid, nthreads);
+  // The first byte ranges before the tables' copy: reads return in order, so behind the copy the chain of
+  // reads that ends in them (row, position, range) would wait for it at every link (as it did: 1500 x 2064 at
+  // 100 rows 26.95 -> 26.4 us, 5000 x 1536 at six 15.05 -> 14.55, 17408 and 17408 x 5120 at sixteen 143.3 ->
+  // 142.3.  The one-row kernel, with one link fewer and more waves to start, is faster the other way round).
+  span_of(b_first, g0, g1);
+  if (grf::fused_tables_by_dma(f)) grf::fused_load_tables_dma(lds, L.blocks, L.block_pitch, f, cls, wave, nthreads / 64, lane);
+  else grf::fused_load_tables(lds, L.blocks, L.block_pitch, f, cls, tid, nthreads);
 
   float4v acc[MT];
 #pragma unroll
