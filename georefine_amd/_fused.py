@@ -260,6 +260,8 @@ def choose_tiling(spr, class_rows, piece_cap_fn, lds_fn, cus=256, seg_len=64, ta
 
 SCHEME_SLABS, SCHEME_WAVES = 0, 1
 WAVE_ROWS_PER_PASS = 2  # activation rows one launch of the wave-unit kernel carries
+WAVES_PER_CU = 24       # of the wave-unit kernels, by their registers
+LINES_WAVES_PER_CU = 16  # of the one that stores whole lines
 WAVE_UNIT_OVERHEAD = 8  # decode steps' worth of staging, reduction and bookkeeping per unit
 
 
@@ -267,7 +269,7 @@ WAVE_PIECE_OVERHEAD = 1.7   # decode steps' worth of staging per row piece of a 
 WAVE_LATENCY_RATIO = 4.5    # a lone wave's time for a step / its share of a saturated SIMD's issue time
 
 
-def choose_wave_tiling(spr, class_rows, piece_cap_fn, lds_fn, cus=256, seg_len=64, table_bytes=0):
+def choose_wave_tiling(spr, class_rows, piece_cap_fn, lds_fn, cus=256, seg_len=64, table_bytes=0, waves=WAVES_PER_CU):
     """Tiling of the wave-unit GEMV: a wave walks units of 64 / P rows x P consecutive
     segments (P a power of two) and the waves of a workgroup share out the units of its tile
     without meeting at a barrier; a tile is a whole number of units (a unit's rows are then a
@@ -292,11 +294,11 @@ def choose_wave_tiling(spr, class_rows, piece_cap_fn, lds_fn, cus=256, seg_len=6
         return t_, p_, r_, n_slabs, _tiles(class_rows, r_), cap, lds_fn(t_, p_, r_, n_slabs, cap)
     threads, p, (r,), tiles, cap, lds = search_wave_tilings(
         [(spr, seg_len, class_rows)], piece_cap_fn, lambda t_, p_, heights, cap_: lds_fn(t_, p_, heights[0], -(-spr // p_), cap_),
-        cus, table_bytes)
+        cus, table_bytes, waves)
     return threads, p, r, -(-spr // p), tiles, cap, lds
 
 
-def search_wave_tilings(lengths, piece_cap_fn, lds_fn, cus, table_bytes):
+def search_wave_tilings(lengths, piece_cap_fn, lds_fn, cus, table_bytes, waves=WAVES_PER_CU):
     """The fastest wave tiling by ``choose_wave_tiling``'s model, as (threads, lanes per row, rows per
     tile of every length, tiles, piece capacity, LDS bytes), of a launch over matrices of one width
     indexed at several ``lengths``: (segments per row, segment length, rows per class) each, the one
@@ -318,7 +320,7 @@ def search_wave_tilings(lengths, piece_cap_fn, lds_fn, cus, table_bytes):
         # rows needs larger pieces, and one wave less per workgroup then keeps two of them resident --
         # 17408 x 5120 with pieces of 912 bytes: 68.7 us with 11 waves against 95.0 with 12 and
         # tiles cut down to 8 rows)
-        for threads in (1024, 768, 704, 640, 576, 512):
+        for threads in (1024, 768, 704, 640, 576, 512) if waves > LINES_WAVES_PER_CU else (1024, 512):
             nwaves = threads // 64
             busiest = lambda units: 0.5 * -(-units // nwaves) + 0.5 * units / nwaves  # units of the wave that has most
             heights = [rpw] * len(lengths)
@@ -343,8 +345,8 @@ def search_wave_tilings(lengths, piece_cap_fn, lds_fn, cus, table_bytes):
                 lds = lds_fn(threads, p, heights, cap)
                 if lds > MAX_LDS:
                     break
-                # six waves per SIMD by registers; a little LDS stays with the system
-                per_cu = max(1, min(24 // nwaves, (MAX_LDS - 1024) // lds))
+                # (the waves that the kernel's registers allow; a little LDS stays with the system)
+                per_cu = max(1, min(waves // nwaves, (MAX_LDS - 1024) // lds))
                 rounds = -(-tiles // (cus * per_cu))
                 chain *= rounds
                 time = (chain ** 3 + issue ** 3) ** (1 / 3)
@@ -369,7 +371,7 @@ def wave_time(tiling, seg_len, table_bytes, cus=256):
     nwaves, rpw = g["threads"] // 64, 64 // g["lanes_per_row"]
     unit_steps, table_steps = seg_len + WAVE_UNIT_OVERHEAD + WAVE_PIECE_OVERHEAD * rpw, 3 + table_bytes / 12288
     units = -(-g["rows_per_tile"] // rpw) * g["n_slabs"]
-    rounds = -(-g["n_tiles"] // (cus * max(1, min(24 // nwaves, (MAX_LDS - 1024) // tiling["lds"]))))
+    rounds = -(-g["n_tiles"] // (cus * max(1, min(WAVES_PER_CU // nwaves, (MAX_LDS - 1024) // tiling["lds"]))))
     chain = rounds * ((0.5 * -(-units // nwaves) + 0.5 * units / nwaves) * unit_steps + table_steps) * WAVE_LATENCY_RATIO
     issue = g["n_tiles"] / cus * (units * unit_steps + nwaves * table_steps) / 4
     return (chain ** 3 + issue ** 3) ** (1 / 3)
@@ -504,19 +506,15 @@ def build_tiles(row_class, nr, r):
     """Rows grouped by class (index order inside a class), cut into tiles of r rows."""
     order = np.argsort(row_class, kind="stable").astype(np.uint32)
     counts = np.bincount(row_class, minlength=nr)
-    tiles, classes = [], []
-    at = 0
-    for rho in range(nr):
+    tiles = -(-counts // r)
+    out = np.full(int(tiles.sum()) * r, 0xFFFFFFFF, dtype=np.uint32)
+    at = slot = 0
+    for rho in np.flatnonzero(counts):
         cnt = int(counts[rho])
-        rows_of_class = order[at:at + cnt]
+        out[slot:slot + cnt] = order[at:at + cnt]
         at += cnt
-        for lo in range(0, cnt, r):
-            slot = np.full(r, 0xFFFFFFFF, dtype=np.uint32)
-            chunk = rows_of_class[lo:lo + r]
-            slot[:chunk.size] = chunk
-            tiles.append(slot)
-            classes.append(rho)
-    return np.concatenate(tiles), np.asarray(classes, dtype=np.uint8)
+        slot += int(tiles[rho]) * r
+    return out, np.repeat(np.arange(len(counts), dtype=np.uint8), tiles)
 
 
 def build_balanced_tiles(row_class, nr, unit_rows, slots, max_rows):
@@ -548,23 +546,25 @@ def build_balanced_tiles(row_class, nr, unit_rows, slots, max_rows):
     tallest = max(height(rho) for rho in live) * unit_rows
     if tallest > max_rows:
         return None
-    out_rows, out_class = [], []
-    first = np.concatenate(([0], np.cumsum(counts)[:-1]))
-    for rho in live:
-        rows_of_class = order[first[rho]:first[rho] + counts[rho]]
-        n, u = tiles[rho], units[rho]
-        at = 0
-        for k in range(n):  # units per tile differ by at most one
-            take = (u // n + (1 if k < u % n else 0)) * unit_rows
-            chunk = rows_of_class[at:at + take]
-            at += take
-            if chunk.size == 0:
+    used = [min(tiles[rho], units[rho]) for rho in live]  # (tiles without a row are left out)
+    out = np.full((sum(used), tallest), 0xFFFFFFFF, dtype=np.uint32)
+    at = tile = 0
+    for rho, n in zip(live, used):
+        rows, u = int(counts[rho]), units[rho]
+        # units per tile differ by at most one: u % n tiles of one more, then the rest
+        tall, low = u % n, u // n * unit_rows
+        split = min(tall * (low + unit_rows), rows)
+        for first, height, count, t in ((0, low + unit_rows, split, tile), (split, low, rows - split, tile + tall)):
+            if not count:
                 continue
-            slot = np.full(tallest, 0xFFFFFFFF, dtype=np.uint32)
-            slot[:chunk.size] = chunk
-            out_rows.append(slot)
-            out_class.append(rho)
-    return np.concatenate(out_rows), np.asarray(out_class, dtype=np.uint8), tallest
+            whole = count // height
+            out[t:t + whole, :height] = order[at + first:at + first + whole * height].reshape(whole, height)
+            rest = count - whole * height
+            if rest:
+                out[t + whole, :rest] = order[at + first + whole * height:at + first + count]
+        at += rows
+        tile += n
+    return out.reshape(-1), np.repeat(np.asarray(live, dtype=np.uint8), used), tallest
 
 
 GEMM_BALANCE = os.environ.get("GEOREFINE_GEMM_BALANCE", "1") != "0"  # "0": tiles of one height (experiments)
@@ -753,26 +753,36 @@ class FramePlan:
                     scalars=dict(threads=threads, lanes_per_row=p, rows_per_tile=r, n_slabs=n_slabs,
                                  n_tiles=n_tiles, piece_cap=cap, scheme=SCHEME_SLABS), lds=lds)
 
-    def _wave_tiling(self):
+    def lines_tiling(self):
+        """The wave units of the kernel that stores whole lines (fused_wave_lines_kernel), which
+        holds 64 columns back and has registers for sixteen waves a compute unit: workgroups of
+        sixteen or eight.  None where the walk's segments are no multiple of 64."""
+        if self.seg_len % 64:
+            return None
+        key = "lines", os.environ.get("GEOREFINE_FUSED_WAVE_TILING")
+        if key not in self._tilings:
+            self._tilings[key] = self._wave_tiling(0, LINES_WAVES_PER_CU)
+        return self._tilings[key]
+
+    def _wave_tiling(self, m=WAVE_ROWS_PER_PASS, waves=WAVES_PER_CU):
         self._wave_limits()
         threads, p, r, n_slabs, n_tiles, cap, lds = choose_wave_tiling(
             self.spr, self.class_rows, self._cap,
-            lambda t_, p_, r_, s_, cap_: lds_bytes_waves(self.nc, self.lognb, self.tabn, WAVE_ROWS_PER_PASS, t_, p_,
-                                                         r_, s_, cap_),
-            seg_len=self.seg_len, table_bytes=self.table_bytes())
+            lambda t_, p_, r_, s_, cap_: lds_bytes_waves(self.nc, self.lognb, self.tabn, m, t_, p_, r_, s_, cap_),
+            seg_len=self.seg_len, table_bytes=self.table_bytes(), waves=waves)
         tile_rows, tile_class = build_tiles(self.row_class, self.nr, r)
         assert len(tile_class) == n_tiles
         if not os.environ.get("GEOREFINE_FUSED_WAVE_TILING"):
             # classes of very different sizes: the same workgroup slots, cut so that no tile is
             # taller than it has to be (the kernel walks a tile's real height)
             nwaves, rpw = threads // 64, 64 // p
-            per_cu = max(1, min(24 // nwaves, (MAX_LDS - 1024) // lds))
+            per_cu = max(1, min(waves // nwaves, (MAX_LDS - 1024) // lds))
             slots = -(-n_tiles // (256 * per_cu)) * 256 * per_cu
             even = build_balanced_tiles(self.row_class, self.nr, rpw, slots, r)
             if even is not None and (even[2] < r or (even[2] == r and len(even[1]) > n_tiles)):
                 tile_rows, tile_class, r = even
                 n_tiles = len(tile_class)
-                lds = lds_bytes_waves(self.nc, self.lognb, self.tabn, WAVE_ROWS_PER_PASS, threads, p, r, n_slabs, cap)
+                lds = lds_bytes_waves(self.nc, self.lognb, self.tabn, m, threads, p, r, n_slabs, cap)
         return dict(tile_rows=tile_rows, tile_class=tile_class,
                     scalars=dict(threads=threads, lanes_per_row=p, rows_per_tile=r, n_slabs=n_slabs,
                                  n_tiles=n_tiles, piece_cap=cap, scheme=SCHEME_WAVES), lds=lds)

@@ -451,7 +451,6 @@ class HipContextTensor:
         the row counts in between."""
         if m and GEMV_WAVES and "waves" in self._tilings:
             return self._tilings["waves"]
-        import torch
         if m == 0:
             bucket = 0
         elif GEMV_WAVES:
@@ -459,21 +458,31 @@ class HipContextTensor:
         else:
             bucket = next(v for v in (1, 2, 4, 8) if v >= m)
         if bucket not in self._tilings:
-            host = self._plan.tiling(WAVE_ROWS if bucket == "waves" else bucket, waves=bucket == "waves")
-            rows = torch.from_numpy(host["tile_rows"]).to(self.device)
-            classes = torch.from_numpy(host["tile_class"]).to(self.device)
-            g = _hip_abi.GrfFusedTiling()
-            g.tile_rows, g.tile_class = rows.data_ptr(), classes.data_ptr()
-            for key, value in host["scalars"].items():
-                setattr(g, key, value)
-            self._tilings[bucket] = (g, rows, classes, dict(host["scalars"], lds=host["lds"]))
-            self.resident_bytes += rows.numel() * 4 + classes.numel()
+            self._upload_tiling(bucket, self._plan.tiling(WAVE_ROWS if bucket == "waves" else bucket, waves=bucket == "waves"))
         return self._tilings[bucket]
 
+    def _upload_tiling(self, bucket, host):
+        import torch
+        rows = torch.from_numpy(host["tile_rows"]).to(self.device)
+        classes = torch.from_numpy(host["tile_class"]).to(self.device)
+        g = _hip_abi.GrfFusedTiling()
+        g.tile_rows, g.tile_class = rows.data_ptr(), classes.data_ptr()
+        for key, value in host["scalars"].items():
+            setattr(g, key, value)
+        self._tilings[bucket] = (g, rows, classes, dict(host["scalars"], lds=host["lds"]))
+        self.resident_bytes += rows.numel() * 4 + classes.numel()
+
     def _store_tiling(self):
-        """The tiling decode() uses: the GEMV's wave units (their blocks of rows are the blocks of
-        the resident residual order); the slab tiling of the store sink only with the slab GEMV."""
-        return self._tiling(1 if GEMV_WAVES else 0)
+        """The tiling decode() uses: wave units of the kernel that stores whole lines where the segments
+        allow it, else the GEMV's; the slab tiling of the store sink only with the slab GEMV."""
+        if not GEMV_WAVES:
+            return self._tiling(0)
+        if "lines" not in self._tilings:
+            host = self._plan.lines_tiling()
+            if host is None:
+                return self._tiling(1)
+            self._upload_tiling("lines", host)
+        return self._tilings["lines"]
 
     # ------------------------------------------------------------------ decode
     def _decode_blocks(self, blocks=None, *, check=True):

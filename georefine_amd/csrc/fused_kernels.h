@@ -398,8 +398,68 @@ __device__ __forceinline__ void store_segment(Walk &w, const grf::FusedParams &q
   }
 }
 
-// SINK kDot: products with M activation rows; kStore: the words to `out` (M = 0).
-template <class Walk, int M, int SCAN, int SINK = kDot>
+// Decoded words of a unit that are still to be stored: the last 32 * H columns of every lane's segment,
+// quads already exchanged, so that u[h][k] of lane j is 16-byte unit 4 * h + j of what lane k decoded.
+template <int H>
+struct HeldWords {
+  static constexpr uint32_t kNowhere = 0xFFFFFFFFu;
+  uint32_t u[H][4][4];
+  uint32_t unit = kNowhere;  // the lane's first 16-byte unit in the output
+  __device__ __forceinline__ void flush(uint16_t *out, uint32_t lane) {
+    auto run = [&](auto k) {
+      constexpr int K = decltype(k)::value;
+#if defined(__HIP_DEVICE_COMPILE__)
+      const uint32_t at = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)unit, 0x55 * K, 0xF, 0xF, false);
+#else
+      const uint32_t at = unit;
+#endif
+      if (at == kNowhere) return;
+      words8_t *dst = reinterpret_cast<words8_t *>(out) + ((size_t)at + (lane & 3));
+#pragma unroll
+      for (int h = 0; h < H; ++h)
+        dst[4 * h] = (words8_t){u[h][K][0], u[h][K][1], u[h][K][2], u[h][K][3]};
+    };
+    run(std::integral_constant<int, 0>{});
+    run(std::integral_constant<int, 1>{});
+    run(std::integral_constant<int, 2>{});
+    run(std::integral_constant<int, 3>{});
+    unit = kNowhere;
+  }
+};
+template <>
+struct HeldWords<0> {
+  __device__ __forceinline__ void flush(uint16_t *, uint32_t) {}
+};
+
+// The same walk for a kernel that goes on to another unit (S a multiple of 32 * H): the words of 32 * H columns
+// are held back, the unit's last ones until the next unit's pieces have arrived.  A wave waits for the
+// bytes of a unit with its whole counter of memory operations, so stores just before that wait would
+// be waited for as well.
+template <class Walk, int SCAN, int H>
+__device__ __forceinline__ void hold_segment(Walk &w, const grf::FusedParams &q, uint32_t S, bool walks, uint32_t first,
+                                             uint16_t *out, uint32_t lane, HeldWords<H> &held) {
+  held.flush(out, lane);  // the unit before
+  for (uint32_t t = 0; t < S; t += 32 * H) {
+    if (t) held.flush(out, lane);
+#pragma unroll
+    for (int h = 0; h < H; ++h) {
+      uint32_t(&u)[4][4] = held.u[h];
+      if (walks) {
+        w.begin16(t + 32 * h, S);
+        w.template half<0, SCAN>(q, u[0]);
+        w.template half<1, SCAN>(q, u[1]);
+        w.begin16(t + 32 * h + 16, S);
+        w.template half<0, SCAN>(q, u[2]);
+        w.template half<1, SCAN>(q, u[3]);
+      }
+      transpose_quad(u, lane);
+    }
+    held.unit = walks ? (first + t) / 8 : HeldWords<H>::kNowhere;  // (fits 32 bits: rows are multiples of 16 words)
+  }
+}
+
+// SINK kDot: products with M activation rows; kStore: the words to `out` (M = 0), 32 * HOLD columns at a time.
+template <class Walk, int M, int SCAN, int SINK = kDot, int HOLD = 0>
 __device__ __forceinline__ void fused_wave_body(uint8_t *lds, const grf_bctx_fused &f, const grf_fused_tiling &g,
                                                 const uint16_t *x, uint32_t ldx, uint16_t *y, uint32_t ldy,
                                                 const uint16_t *bias, int32_t *error, uint32_t tile,
@@ -493,6 +553,7 @@ __device__ __forceinline__ void fused_wave_body(uint8_t *lds, const grf_bctx_fus
   __syncthreads();
   const uint32_t later_half = blockIdx.x >= gridDim.x / 2 ? 1u : 0u;
   uint32_t left = wave < units ? (units - 1 - wave) / nwaves : 0;  // units after the current one
+  HeldWords<HOLD> held;
   for (uint32_t u = wave; u < units; u += nwaves, --left) {  // wave-uniform
 #if defined(__HIP_DEVICE_COMPILE__)
     // Waves with more units still to do go first.  Left alone the arbiter prefers the older
@@ -539,7 +600,8 @@ __device__ __forceinline__ void fused_wave_body(uint8_t *lds, const grf_bctx_fus
     }
 #endif
     if constexpr (SINK == kStore) {
-      store_segment<Walk, SCAN>(w, q, S, walks, walks ? mul24(row, K) + col0 : 0, out, lane);
+      if constexpr (HOLD > 0) hold_segment<Walk, SCAN>(w, q, S, walks, walks ? mul24(row, K) + col0 : 0, out, lane, held);
+      else store_segment<Walk, SCAN>(w, q, S, walks, walks ? mul24(row, K) + col0 : 0, out, lane);
       if (walks && !w.ended_on_checkpoint(f)) bad |= GRF_ERR_CHECKPOINT;
       continue;
     }
@@ -606,6 +668,7 @@ __device__ __forceinline__ void fused_wave_body(uint8_t *lds, const grf_bctx_fus
     }
   }
   if constexpr (SINK == kStore) {
+    held.flush(out, lane);
     if (bad) atomicOr(error, (int)bad);
     return;
   }
@@ -651,28 +714,45 @@ __global__ __launch_bounds__(grf::kFusedMaxThreads) __attribute__((amdgpu_waves_
   fused_wave_body<Walk, M, SCAN>(lds, f, g, x, ldx, y, ldy, bias, error, blockIdx.x);
 }
 
-// The store sink over wave units (decode()).  Bound by the walk (VALU issue, as the GEMV) and the
-// traffic behind it together: 17408 x 5120 takes 98.6 us where the walk alone takes 70 and its 307 MB
-// at the rate of a large copy 59; slab tilings with 64-byte runs stored by the lanes that decoded
-// them took 148.  Output held back to whole 128-byte lines (88 registers, 16 waves a compute unit)
-// measured the same (93-98 us), streaming stores 2 % more.
-template <class Walk, int SCAN>
-__global__ __launch_bounds__(grf::kFusedMaxThreads) __attribute__((amdgpu_waves_per_eu(6))) void fused_wave_store_kernel(
+// The store sink over wave units (decode()).  Bound by the walk and the traffic behind it together, and
+// most of all by how the words leave.  HOLD 2 (segments of whole lines): a lane's 128 bytes are held back and
+// its line is written at one visit; written half by half, 20 % of the lines left the second-level cache
+// half written (5120 x 17408: 227 MB written, so 178, which is the matrix).  It takes 88 registers, so sixteen
+// waves a compute unit, and is faster for that too: twenty-four waves hold 6 MB of lines per XCD open,
+// and with eight registers spilled took as long as the halves did.  One workgroup of sixteen waves copies
+// the tables once where two of eight copy them twice (91.3 and 92.6 us).  HOLD 1 (segments of 32, 96, ..
+// columns, whose neighbours complete the line, and workgroups that would leave a unit to twelve waves).
+// Both keep a unit's last words until the next unit's bytes have arrived (hold_segment), 3 us of 94.
+// Before and now: 5120 x 17408 104.6 -> 91.2 us, 17408 x 5120 -> 87.4, 5120 x 6144 43.9 -> 38.9, 4096 x 4096
+// 24.8 -> 23.0, 2560 x 5120 27.1 -> 22.4; HOLD 1 alone 104.6 -> 102.0 and, PPCX 4096 x 4096, 26.2 -> 25.4.  With
+// the stores absorbed by the cache the first takes 76.  Streaming stores cost 6 %.
+template <class Walk, int SCAN, int HOLD>
+__global__ __launch_bounds__(grf::kFusedMaxThreads) __attribute__((amdgpu_waves_per_eu(HOLD == 2 ? 4 : 6))) void fused_wave_store_kernel(
     grf_bctx_fused f, grf_fused_tiling g, uint16_t *out, int32_t *error) {
   extern __shared__ __align__(16) uint8_t lds[];
-  fused_wave_body<Walk, 0, SCAN, kStore>(lds, f, g, nullptr, 0, nullptr, 0, nullptr, error, blockIdx.x, out);
+  fused_wave_body<Walk, 0, SCAN, kStore, HOLD>(lds, f, g, nullptr, 0, nullptr, 0, nullptr, error, blockIdx.x, out);
 }
+
+template <auto Kernel>
+struct KernelOf { static constexpr auto value = Kernel; };
 
 template <class Walk>
 int launch_wave_store(const grf_bctx_fused &f, const grf_fused_tiling &g, uint16_t *out, int32_t *error, hipStream_t s) {
   const WaveLdsLayout L(f, g, 0);
   if (L.total > 160 * 1024) return grf::set_error(GRF_UNSUPPORTED, "fused decode: LDS demand exceeds 160 KiB");
-  auto launch = [&](auto scan) -> int {
-    constexpr auto kernel = &fused_wave_store_kernel<Walk, decltype(scan)::value>;
+  auto start = [&](auto of) -> int {
+    constexpr auto kernel = decltype(of)::value;
     if (L.total > 64 * 1024)
       if (int rc = allow_full_lds<kernel>()) return rc;
     hipLaunchKernelGGL(kernel, dim3(g.n_tiles), dim3(g.threads), L.total, s, f, g, out, error);
     return GRF_OK;
+  };
+  auto launch = [&](auto scan) -> int {
+    constexpr int kScan = decltype(scan)::value;
+    if (f.seg_len % 32) return start(KernelOf<&fused_wave_store_kernel<Walk, kScan, 0>>{});
+    if (f.seg_len % 64 == 0 && (g.threads == 1024 || g.threads <= 512))
+      return start(KernelOf<&fused_wave_store_kernel<Walk, kScan, 2>>{});
+    return start(KernelOf<&fused_wave_store_kernel<Walk, kScan, 1>>{});
   };
   if (int rc = f.whole_range ? launch(std::integral_constant<int, grf::kScanAny>{})
                              : launch(std::integral_constant<int, grf::kScanNoWholeRange>{}))
@@ -1411,9 +1491,6 @@ inline GemmX gemm_source(const uint16_t *x, uint32_t ldx, uint32_t m_rows, uint3
   if (x) launch_pack(x, ldx, m_rows, cols, gemm_tiles(m_rows) * 16, xp, s);  // else the caller packed these rows already
   return GemmX{xp, 0, 0};
 }
-
-template <auto Kernel>
-struct KernelOf { static constexpr auto value = Kernel; };
 
 // launch(scan, rows) for the scan the frames need and the activations' form
 template <int MT, class Launch>
