@@ -188,12 +188,14 @@ struct PpcxWalk {
   template <int H, int SCAN = grf::kScanAny, bool KEEP = true>
   __device__ __forceinline__ void half(const grf::FusedParams &q, uint32_t (&pair)[4]) {
     uint32_t bits[8];
+    // The eight 4-bit bins as bytes, which the multiply that makes a block offset selects by itself: three
+    // instructions a half where each bin's extraction was one (4096 x 4096 at 96 rows 44.1 -> 43.8 us).
+    const uint32_t even = bw[H] & 0x0F0F0F0Fu, odd = (bw[H] >> 4) & 0x0F0F0F0Fu;
 #define GRF_STEP2(i)                                                                                  \
   {                                                                                                   \
-    const uint32_t bin0 = __builtin_amdgcn_ubfe(bw[H], 4 * (i), 4);                                   \
-    const uint32_t bin1 = __builtin_amdgcn_ubfe(bw[H], 4 * (i) + 4, 4);                               \
     uint32_t h0, h1;                                                                                  \
-    grf::fused_symbol_pair_in<SCAN>(c, __umul24(bin0, q.block_pitch), __umul24(bin1, q.block_pitch), q, h0, h1); \
+    grf::fused_symbol_pair_in<SCAN>(c, grf::fused_block_offset<(i) / 2>(even, q.block_pitch),         \
+                                    grf::fused_block_offset<(i) / 2>(odd, q.block_pitch), q, h0, h1); \
     bits[i] = h0 | rr.field<8 * H + (i)>();                                                           \
     bits[(i) + 1] = h1 | rr.field<8 * H + (i) + 1>();                                                 \
     pair[(i) / 2] = grf::fused_word_pair<KEEP>(bits[i], bits[(i) + 1]);                               \
