@@ -668,6 +668,44 @@ class FramePlan:
         gain = wave_time(tall, self.seg_len, self.table_bytes()) / wave_time(fine, self.seg_len, other.table_bytes())
         return other if units > g["threads"] // 64 and gain >= 1.14 else self
 
+    def for_matrix_cores(self, main_freq, budget, image=None):
+        """This plan, or one like it with lookups of at most ``budget`` bytes where the matrix-core
+        launches of the matrix are the faster for them: where three workgroups of eight waves then share
+        a compute unit that had one of ten to sixteen, each with half as many slabs to walk in a row,
+        which ``plan_gemm_tiling``'s model sees as half as much again.  Only tilings that the kernels
+        for more than 64 rows can share a unit with too (``shares_units`` in fused_kernels.h).  Fewer
+        bytes mean more scans, 13 % of the same tiling's time.  Six, 32 and 96 rows, us, predictive
+        frames at 64 / 16 KiB, and the modelled advantage:
+          4096 x 4096    1.86   37.0 39.9 51.7 / 31.6 34.8 43.5
+          8192 x 2048    1.97   31.9 35.3 41.9 / 29.3 32.3 39.5
+          16384 x 1024   1.97   30.9 34.8 41.6 / 30.0 33.4 40.0
+          5120 x 5120    1.09   37.7 41.6 52.8 / 46.2 49.6 62.1
+          7000 x 1600    1.06   20.8 23.9 29.5 / 27.8 31.3 38.4
+          2048 x 8192    1.83   37.7 40.8 52.6 / 34.8 37.5 58.2  (704 threads)
+          5120 x 17408   1.54   90.7 96.0 135 / 92.9 98.1 156  (768 threads)
+        A grouped launch keeps this plan's (three of 4096 x 4096: 67.2 69.2 96 / 72.6 74.8 125)."""
+        other = self.with_lookups(main_freq, budget, image)
+        if other.lognb >= self.lognb:
+            return self
+        try:
+            tall, fine = self.gemm_tiling(), other.gemm_tiling()
+        except FusedUnsupported:
+            return self
+        g = fine["scalars"]
+        shared = g["n_tiles"] > 256 and g["threads"] <= 640 and fine["lds"] <= 79 * 1024
+        return other if shared and other.gemm_share(fine) >= 1.5 * self.gemm_share(tall) else self
+
+    def gemm_share(self, tiling):
+        """What ``plan_gemm_tiling``'s model says of one tiling: the share of the machine's wave slots that do
+        useful steps."""
+        g = tiling["scalars"]
+        waves, k = g["threads"] // 64, max(1, g["k_parts"])
+        per_cu = max(1, min(GEMM_WAVES_PER_SIMD // -(-waves // 4), MAX_LDS // tiling["lds"]))
+        slabs, slots = -(-g["n_slabs"] // k), 256 * per_cu
+        paid = -(-g["n_tiles"] // slots) * slots * waves * 64 * slabs
+        share = self.rows * self.spr / paid * min(1.0, per_cu * waves / 24) * _walk_share(slabs, self.seg_len, self.table_bytes())
+        return share * (0.97 - 0.015 * k) if k > 1 else share
+
     def with_lookups(self, main_freq, budget, image=None):
         """This plan with lookups of at most ``budget`` bytes."""
         other = copy.copy(self)

@@ -51,11 +51,13 @@ def _checkpoints(stream, ctx, freq, vocab, stride):
 # a bucket's minority symbol: 35 % of the steps with 1 KiB per context, 21 % with 2 KiB, 12 % with
 # 4 KiB.  At 64 KiB one workgroup of sixteen waves has a compute unit to itself instead of two of
 # twelve, and still wins for products on the matrix cores (16 / 32 / 64 KiB in all, us: 4096 x 4096
-# at 96 rows 61.2 / 53.9 / 51.8, 3000 x 4096 36.4 / 32.6 / 31.9, 5120 x 17408 164 / 140 / 137, 512 x 1024 at
-# 64 rows 15.8 / 15.2 / 15.1).  One row and decode() take 32 KiB where those are faster
-# (FramePlan.for_vector_alus); the tensor then keeps both lookups, half a MiB more.
+# at 96 rows 43.5 / 53.1 / 51.7, 3000 x 4096 36.4 / 32.6 / 31.9, 5120 x 17408 156 / 142 / 135, 512 x 1024 at
+# 64 rows 15.8 / 15.2 / 15.1), except where three of eight waves at 16 KiB do (FramePlan.for_matrix_cores).
+# One row and decode() take 32 KiB where those are faster (FramePlan.for_vector_alus).  The tensor keeps
+# every lookup it uses, half and a quarter MiB more.
 _LUT_BUDGET, _WALK_LUT_BUDGET = ((int(os.environ["GEOREFINE_FUSED_LUT_BYTES"]),) * 2
                                  if "GEOREFINE_FUSED_LUT_BYTES" in os.environ else (64 * 1024, 32 * 1024))
+_MATRIX_LUT_BUDGET = 16 * 1024
 
 
 def _word_image(main):
@@ -121,6 +123,7 @@ def _read_frame(frame, reference, stride, *, fused=False, fused_segment=None):
             result["fused_plan"] = _fused.FramePlan((r, c), 16, 16, info["labels"], freq, fs, fo, len(info["stream"]),
                                                     seg_len, image=_word_image, lut_budget=_LUT_BUDGET)
             result["walk_plan"] = result["fused_plan"].for_vector_alus(freq, _WALK_LUT_BUDGET, _word_image)
+            result["matrix_plan"] = result["fused_plan"].for_matrix_cores(freq, _MATRIX_LUT_BUDGET, _word_image)
             result["resident_mode"] = 0
         except _fused.FusedUnsupported as exc:
             result["fused_reason"] = str(exc)
@@ -162,8 +165,9 @@ class HipPredictiveTensor:
         self.n = math.prod(self.shape)
         self.stride, self.mode = stride, ix["mode"]
         self.resident_mode = ix.get("resident_mode", self.mode)
-        self._plan = ix.pop("fused_plan", None)         # of the matrix-core launches ...
-        self._walk_plan = ix.pop("walk_plan", None)     # ... and of the others (the same one for most matrices)
+        self._plan = ix.pop("fused_plan", None)         # of grouped matrix-core launches ...
+        self._matrix_plan = ix.pop("matrix_plan", None)  # ... of the others of these ...
+        self._walk_plan = ix.pop("walk_plan", None)     # ... and of one row and the store sink (one plan for most matrices)
         self.fused_reason = ix.pop("fused_reason", None)
         self.device = torch.device(device)
         for key in ("source_sha256", "target_sha256", "reference_sha256", "frame_sha256", "frame_bytes"):
@@ -241,7 +245,7 @@ class HipPredictiveTensor:
             f.rows, f.cols = self.shape
             f.mode, f.stride = self.resident_mode, self.stride
             self._frame = f
-        self.fused = self.fused_gemm = None
+        self.fused = self.fused_gemm = self.fused_matrix = None
         if self._plan is not None:
             try:
                 self._prepare_fused()
@@ -276,10 +280,12 @@ class HipPredictiveTensor:
             spr, position = self.shape[1] // self._raw5_segment, b["row_pos"].cpu().numpy()
             states = _fused.order_index(states, self.shape[0], spr, self._raw5_block, position, self._rows_held)
             offsets = _fused.order_index(offsets, self.shape[0], spr, self._raw5_block, position, self._rows_held)
-        walk = self._walk_plan
+        walk, matrix = self._walk_plan, self._matrix_plan
         arrays = {"fused_seg_state": states, "fused_seg_offset": offsets, "fused_lut": plan.lut, "fused_tab": plan.tab.view(np.int64)}
         if walk is not plan:
             arrays["fused_walk_lut"] = walk.lut
+        if matrix is not plan:
+            arrays["fused_matrix_lut"] = matrix.lut
         for name, array in arrays.items():
             if name not in b:  # (a clone already holds its copies)
                 b[name] = torch.from_numpy(np.ascontiguousarray(array)).to(self.device)
@@ -300,6 +306,7 @@ class HipPredictiveTensor:
             return f
 
         self.fused_gemm = frame(plan, "fused_lut")
+        self.fused_matrix = self.fused_gemm if matrix is plan else frame(matrix, "fused_matrix_lut")
         self.fused = self.fused_gemm if walk is plan else frame(walk, "fused_walk_lut")
         self.fused_plan = dict(walk.scalars(), **self._tiling_for("waves")[3])
 
@@ -319,7 +326,7 @@ class HipPredictiveTensor:
         reach: 0 = store sink, 1/2/4/8 = GEMV row buckets."""
         if key not in self._tilings:
             import torch
-            host = (self._plan.gemm_tiling() if key == "gemm" else self._walk_plan.tiling(_fused.WAVE_ROWS_PER_PASS, waves=True)
+            host = (self._matrix_plan.gemm_tiling() if key == "gemm" else self._walk_plan.tiling(_fused.WAVE_ROWS_PER_PASS, waves=True)
                     if key == "waves" else self._walk_plan.tiling(key))
             rows = torch.from_numpy(host["tile_rows"].view(np.int32)).to(self.device)
             classes = torch.from_numpy(host["tile_class"]).to(self.device)
@@ -423,7 +430,7 @@ class HipPredictiveTensor:
             if not status:
                 extra = ()
                 if use_gemm:
-                    fn, frame, tiling = self._lib.grf_ppcx_gemm, self.fused_gemm, self._tiling_for("gemm")[0]
+                    fn, frame, tiling = self._lib.grf_ppcx_gemm, self.fused_matrix, self._tiling_for("gemm")[0]
                     key = m if m <= PackedActivations.MAX_ROWS else PackedActivations.MAX_ROWS
                     size = self._workspace.get((key, tiling.k_parts))
                     if size is None:

@@ -72,3 +72,18 @@ def test_vector_alu_launches_take_the_smaller_lookups_where_those_are_faster(row
         assert fine["lds"] == _fused.lds_bytes_waves(16, 11, walk.tabn, 2, *(fine["scalars"][k] for k in (
             "threads", "lanes_per_row", "rows_per_tile", "n_slabs", "piece_cap")))
     assert plan.for_vector_alus(freq, gpu._LUT_BUDGET, gpu._word_image) is plan  # nothing smaller asked for
+
+
+@pytest.mark.parametrize("rows,cols,smaller", [(4096, 4096, True), (8192, 2048, True), (5120, 5120, False), (2048, 2048, False),
+                                               (2048, 8192, False)])
+def test_matrix_core_launches_take_smaller_lookups_where_three_workgroups_share_a_unit(rows, cols, smaller):
+    from georefine_amd import bitexact_predictive_gpu as gpu
+    freq, plan = _predictive_plan(rows, cols)
+    matrix = plan.for_matrix_cores(freq, gpu._MATRIX_LUT_BUDGET, gpu._word_image)
+    assert (matrix is not plan) == smaller and plan.lognb == 12
+    if smaller:
+        assert matrix.lognb == 10 and np.array_equal(matrix.lut, _fused.sparse_tables(freq, 16, 16, 6, gpu._word_image)[0])
+        tall, fine = plan.gemm_tiling(), matrix.gemm_tiling()
+        assert tall["scalars"]["n_tiles"] <= 256 < fine["scalars"]["n_tiles"] and 3 * fine["lds"] <= _fused.MAX_LDS
+        assert fine["scalars"]["threads"] <= 640 and 0 < plan.gemm_share(tall) < matrix.gemm_share(fine) <= 1
+    assert plan.for_matrix_cores(freq, gpu._LUT_BUDGET, gpu._word_image) is plan  # nothing smaller asked for
