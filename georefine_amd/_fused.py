@@ -391,7 +391,44 @@ def choose_gemm_tiling(spr, class_rows, piece_cap_fn, lds_fn, cus=256, seg_len=6
                             split)[:8]
 
 
-def plan_gemm_tiling(spr, class_rows, piece_cap_fn, lds_fn, cus=256, seg_len=64, table_bytes=0, split=False, unit_fn=None):
+# gemm_times: rows, then steps' worth of work a slab, of work a table copy per 12 KiB, the latency of a step in
+# issue slots, the exponent that joins chain and issue, and us: of a launch, of a cut along K, of each part, of
+# an issue slot; and the weight of the fullest compute unit against the mean one.
+GEMM_TIMES = ((6, 0.827, 5.44, 3.759, 3.167, 4.93, 2.66, 0.0, 0.036, 0.842), (32, 0.165, 7.23, 3.57, 3.264, 5.64, 2.94, 0.0, 0.041, 0.812),
+              (64, 1.861, 11.06, 3.283, 3.076, 5.54, 3.27, 0.0, 0.043, 0.762), (100, 0.0, 10.05, 2.271, 3.486, 4.85, 3.8, 0.405, 0.07, 0.615))
+
+
+def gemm_times(threads, tallest, blocks, n_slabs, tiles, k, lds, spr, seg_len, table_bytes, cus=256):
+    """Modelled us of matrix-core launches of 6, 32, 64 and 100 rows with each of several tilings (arrays;
+    ``tallest``, ``blocks``: blocks of sixteen rows the tallest tile has, and a tile on average), for frames of the context codec.  A launch is bounded by the chain of slabs a wave walks one after
+    the other and by what the fullest SIMD issues, joined as a power mean.  The waves of a workgroup
+    are dealt to the four SIMDs in turn, so a count that is no multiple of four fills one SIMD before the
+    others (two workgroups of ten: 6 waves where 5 are the mean); waves whose quad a row's last slab
+    does not reach leave, and cost nothing there.  Above 64 rows fewer workgroups share a compute unit
+    (``shares_units`` in fused_kernels.h).  Fitted on 2200 forced tilings of fourteen matrices,
+    300 x 4096 to 17408 x 5120, each timed at the four row counts: 7 to 10 % rms."""
+    waves, quads = threads // 64, -(-spr // 4)
+    each = -(-n_slabs // k)
+    most, fullest = np.maximum(1, np.minimum(GEMM_WAVES_PER_SIMD // -(-waves // 4), MAX_LDS // lds)), -(-tiles // cus)
+    shared = (tiles > 256) & (threads <= 640) & (lds <= 79 * 1024)
+    fewer = np.where(shared, most, np.maximum(1, np.minimum(4 // -(-waves // 4), MAX_LDS // lds)))
+    times = []
+    for rows, unit, table, latency, power, launch, cut, part, slot, weight in GEMM_TIMES:
+        per_cu = most if rows <= 64 else fewer
+        at_once, rest = np.minimum(fullest, per_cu), waves % 4
+        extra = np.where(rest == 0, 0, np.where(at_once == 1, 1, np.where(at_once == 2, 1 + (rest >= 2), -(-at_once * rest // 4) + (rest == 2))))
+        uneven = 4 * (at_once * (waves // 4) + np.minimum(extra, at_once)) / (at_once * waves)
+        copy = table * table_bytes / 12288
+        chain = -(-fullest // per_cu) * (each * (seg_len + unit) + copy) * latency
+        walks = (fullest * weight * tallest + tiles / cus * (1 - weight) * blocks) * quads / k
+        copies = (fullest * weight + tiles / cus * (1 - weight)) * waves
+        issue = (walks * (seg_len + unit) * uneven + copies * copy) / 4
+        times.append(slot * (chain ** power + issue ** power) ** (1 / power) + launch + np.where(k > 1, cut + part * k, 0.0))
+    return np.stack(times)
+
+
+def plan_gemm_tiling(spr, class_rows, piece_cap_fn, lds_fn, cus=256, seg_len=64, table_bytes=0, split=False, unit_fn=None,
+                     fitted=False):
     """Tiling of the GEMM kernel: workgroups of (row blocks of 16) x (quads of 4
     lane-segments) waves.  Same model as choose_tiling, counted in waves: a wave is busy
     for as long as its busiest lane, so idle lanes inside a wave are free, idle waves and
@@ -400,9 +437,15 @@ def plan_gemm_tiling(spr, class_rows, piece_cap_fn, lds_fn, cus=256, seg_len=64,
     second kernel): a matrix with few rows then fills the machine with full blocks of sixteen
     rows.  ``unit_fn()``: the LDS that the pieces of any sixteen rows take together, a fifth to a
     third less than sixteen of the longest; a tiling reserves that where it lets more workgroups
-    share a compute unit.  Returns (threads, lanes per row, rows per tile, slabs, tiles of the
-    launch, piece capacity, LDS bytes, k, LDS bytes of a wave's pieces or 0)."""
-    best = None
+    share a compute unit.  ``fitted``: that choice against the one that
+    ``gemm_times`` finds the fastest, taken where it is 4 % faster at every row count and 5 % over them
+    all, 8 % where its workgroups are dealt less evenly (us at 4, 20, 50, 100 rows, the slot model's choice and the fitted one: 5120 x 6144 38.3 42.6 46.9
+    70.8 / 36.2 39.4 43.3 57.4, 3000 x 3072 19.3 21.4 23.5 33.4 / 18.5 20.7 21.9 25.0, 450 x 6144 16.3 15.8
+    18.7 23.0 / 13.9 14.1 18.2 20.9, 1024 x 5120 16.5 16.0 19.1 23.6 / 15.3 15.1 19.4 21.8; not taken,
+    5000 x 1536 15.7 19.3 21.0 31.3 / 17.1 20.0 21.1 24.5, 1300 x 11008 25.8 28.9 31.8 45.1 / 26.6 28.7 32.1
+    47.8).  Returns (threads, lanes per row,
+    rows per tile, slabs, tiles of the launch, piece capacity, LDS bytes, k, LDS bytes of a wave's pieces or 0)."""
+    best, timed, whole_blocks = None, [], sum(-(-int(c) // 16) for c in class_rows)
     total_rows = sum(int(c) for c in class_rows)
     tile_counts = _tile_counts(class_rows, 1024)
     forced = os.environ.get("GEOREFINE_FUSED_GEMM_TILING")  # "lanes_per_row,rows[,k_parts]": experiments only
@@ -453,8 +496,32 @@ def plan_gemm_tiling(spr, class_rows, piece_cap_fn, lds_fn, cus=256, seg_len=64,
             score *= 0.97 - 0.015 * k
         if best is None or score > best[0] + 1e-9:
             best = (score, threads, p, r_used, n_slabs, tiles_used, cap, lds_fn(p, r_used, cap, unit), k, unit)
+        # (workgroups below eight waves copy the tables too often for the other model to be held to them)
+        if fitted and threads >= 512 and p >= 8:
+            r_used = r if row_blocks == 1 else r_used
+            # (a taller tile's blocks are cut whole where a class allows, build_gemm_tiles)
+            average = whole_blocks / tile_counts[r_used]
+            if row_blocks == 1 or average > row_blocks - 1:  # (else spread so far that a block fewer holds them)
+                timed.append((threads, p, r_used, n_slabs, tile_counts[r_used] * k, cap, lds_fn(p, r_used, cap, unit), k, unit,
+                              1.0 if row_blocks == 1 else average))
     if best is None:
         raise FusedUnsupported("no GEMM tiling fits in LDS")
+    if timed:
+        taller = -(-best[3] // 16) > 1
+        timed.append((*best[1:], whole_blocks * best[8] / best[5] if taller else 1.0))
+        columns = [np.array(v) for v in zip(*timed)]
+        threads, _, r, n_slabs, tiles, _, lds, k, _, blocks = columns
+        times = np.log(gemm_times(threads, -(-r // 16), blocks, n_slabs, tiles, k, lds, spr, seg_len, table_bytes, cus))
+        # (one tile of rows serves 2 to 16 of them, the others 17 to 32, 33 to 64, 65 to 128: three octaves and
+        # one each)
+        gain = times[:, -1:] - times
+        total = np.array([3, 1, 1, 1]) / 6 @ gain
+        even = tiles / (-(-tiles // cus) * cus)  # (the fit is least sure of workgroups dealt less evenly to the units)
+        total[(gain < 0.04).any(axis=0) | (total < np.where(even < even[-1], 0.08, 0.05))] = 0.0
+        # (of those that the model cannot tell apart the one with the fewest parts; and the slot model's choice
+        # unless the gain is past what the fit is mostly wrong by between two tilings of one matrix)
+        if total.max() > 0:
+            return timed[min(np.flatnonzero(total >= total.max() - 0.02), key=lambda i: (k[i], -total[i]))][:9]
     return best[1:]
 
 
@@ -847,9 +914,10 @@ class FramePlan:
         threads, p, r, n_slabs, n_tiles, cap, lds, k, unit = plan_gemm_tiling(
             self.spr, self.class_rows, lambda lanes: self.quad_cap(),
             lambda p_, r_, cap_, unit_: lds_bytes_gemm(self.nc, self.lognb, self.tabn, p_, r_, cap_, unit_),
-            seg_len=self.seg_len, table_bytes=self.table_bytes(), split=GEMM_SPLIT, unit_fn=self.quad_bytes)
+            seg_len=self.seg_len, table_bytes=self.table_bytes(), split=GEMM_SPLIT, unit_fn=self.quad_bytes, fitted=GEMM_SPLIT and self.nc <= 4)
         # the row tiles; the launch has k of each
         tile_rows, tile_class, r, _ = build_gemm_tiles(self.row_class, self.nr, r)
+        threads = gemm_shape(p, r)[2]  # (classes that fit fewer blocks of sixteen rows than were planned)
         n_tiles = len(tile_class) * k
         lds = lds_bytes_gemm(self.nc, self.lognb, self.tabn, p, r, cap, unit)
         return dict(tile_rows=tile_rows, tile_class=tile_class,

@@ -87,3 +87,29 @@ def test_matrix_core_launches_take_smaller_lookups_where_three_workgroups_share_
         assert tall["scalars"]["n_tiles"] <= 256 < fine["scalars"]["n_tiles"] and 3 * fine["lds"] <= _fused.MAX_LDS
         assert fine["scalars"]["threads"] <= 640 and 0 < plan.gemm_share(tall) < matrix.gemm_share(fine) <= 1
     assert plan.for_matrix_cores(freq, gpu._LUT_BUDGET, gpu._word_image) is plan  # nothing smaller asked for
+
+
+@pytest.mark.parametrize("class_rows,spr,seg,fitted", [
+    ([320] * 16, 96, 64, True),     # 5120 x 6144: ten of sixteen rows a tile in 512 tiles, or whole blocks in 480
+    ([64] * 16, 160, 32, True),     # 1024 x 5120
+    ([320] * 16, 272, 64, False),   # 5120 x 17408: the two models agree
+    ([312] * 15 + [320], 48, 32, False),  # 5000 x 1536: faster at many rows, slower at few
+])
+def test_fitted_gemm_tilings_only_where_every_row_count_gains(class_rows, spr, seg, fitted):
+    table = 35456
+    lds = lambda p, r, cap, unit: max(table + _fused.gemm_shape(p, r)[2] // 64 * (unit or 16 * cap),
+                                      _fused.gemm_shape(p, r)[2] // 64 * 4096)
+    args = (spr, np.array(class_rows), lambda lanes: 240 if seg == 64 else 112, lds)
+    plan = lambda f: _fused.plan_gemm_tiling(*args, seg_len=seg, table_bytes=table, split=True, fitted=f,
+                                             unit_fn=lambda: 2832 if seg == 64 else 16 * 112)
+    plain, other = plan(False), plan(True)
+    assert (other != plain) == fitted
+    times = []
+    for threads, p, r, n_slabs, tiles, _, lds_bytes, k, _ in (plain, other):
+        assert threads == _fused.gemm_shape(p, r)[2] and n_slabs == -(-spr // p) and lds_bytes <= _fused.MAX_LDS
+        assert tiles == sum(-(-c // r) for c in class_rows) * k and k <= n_slabs
+        taller = r > 16
+        blocks = sum(-(-c // 16) for c in class_rows) * k / tiles if taller else 1.0
+        times.append(_fused.gemm_times(*(np.array([v]) for v in (threads, -(-r // 16), blocks, n_slabs, tiles, k, lds_bytes)),
+                                       spr, seg, table)[:, 0])
+    assert np.all(times[0] >= 1.04 * times[1]) if fitted else plain == other
