@@ -364,14 +364,14 @@ def search_wave_tilings(lengths, piece_cap_fn, lds_fn, cus, table_bytes, waves=W
     return threads, p, tuple(heights), tiles, cap, lds
 
 
-def wave_time(tiling, seg_len, table_bytes, cus=256):
+def wave_time(tiling, seg_len, table_bytes, cus=256, waves=WAVES_PER_CU):
     """What ``choose_wave_tiling``'s model says of one tiling (as ``FramePlan.tiling`` returns it), in
     decode steps of a SIMD."""
     g = tiling["scalars"]
     nwaves, rpw = g["threads"] // 64, 64 // g["lanes_per_row"]
     unit_steps, table_steps = seg_len + WAVE_UNIT_OVERHEAD + WAVE_PIECE_OVERHEAD * rpw, 3 + table_bytes / 12288
     units = -(-g["rows_per_tile"] // rpw) * g["n_slabs"]
-    rounds = -(-g["n_tiles"] // (cus * max(1, min(WAVES_PER_CU // nwaves, (MAX_LDS - 1024) // tiling["lds"]))))
+    rounds = -(-g["n_tiles"] // (cus * max(1, min(waves // nwaves, (MAX_LDS - 1024) // tiling["lds"]))))
     chain = rounds * ((0.5 * -(-units // nwaves) + 0.5 * units / nwaves) * unit_steps + table_steps) * WAVE_LATENCY_RATIO
     issue = g["n_tiles"] / cus * (units * unit_steps + nwaves * table_steps) / 4
     return (chain ** 3 + issue ** 3) ** (1 / 3)
@@ -859,14 +859,20 @@ class FramePlan:
                                  n_tiles=n_tiles, piece_cap=cap, scheme=SCHEME_SLABS), lds=lds)
 
     def lines_tiling(self):
-        """The wave units of the kernel that stores whole lines (fused_wave_lines_kernel), which
+        """The wave units of the kernel that stores whole lines (HOLD 2 of fused_wave_store_kernel), which
         holds 64 columns back and has registers for sixteen waves a compute unit: workgroups of
-        sixteen or eight.  None where the walk's segments are no multiple of 64."""
+        sixteen or eight.  None where the walk's segments are no multiple of 64, and where the
+        model's time with sixteen waves is 1.25 times the GEMV's with twenty-four (a wave that has a
+        unit and a little walks two; 9000 x 2048, 1.37: 29.8 us where the GEMV's tiling takes 27.3; 5120 x
+        17408, 1.20: 91.2 and 102)."""
         if self.seg_len % 64:
             return None
         key = "lines", os.environ.get("GEOREFINE_FUSED_WAVE_TILING")
         if key not in self._tilings:
-            self._tilings[key] = self._wave_tiling(0, LINES_WAVES_PER_CU)
+            lines, walk = self._wave_tiling(0, LINES_WAVES_PER_CU), self.tiling(WAVE_ROWS_PER_PASS, waves=True)
+            slower = (wave_time(lines, self.seg_len, self.table_bytes(), waves=LINES_WAVES_PER_CU)
+                      > 1.25 * wave_time(walk, self.seg_len, self.table_bytes()))
+            self._tilings[key] = None if slower and not key[1] else lines
         return self._tilings[key]
 
     def _wave_tiling(self, m=WAVE_ROWS_PER_PASS, waves=WAVES_PER_CU):

@@ -438,7 +438,7 @@ struct HeldWords<0> {
 template <class Walk, int SCAN, int H>
 __device__ __forceinline__ void hold_segment(Walk &w, const grf::FusedParams &q, uint32_t S, bool walks, uint32_t first,
                                              uint16_t *out, uint32_t lane, HeldWords<H> &held) {
-  held.flush(out, lane);  // the unit before
+  held.flush(out, lane);  // the unit before (after the next group's loads instead: 4 % slower)
   for (uint32_t t = 0; t < S; t += 32 * H) {
     if (t) held.flush(out, lane);
 #pragma unroll
@@ -720,11 +720,13 @@ __global__ __launch_bounds__(grf::kFusedMaxThreads) __attribute__((amdgpu_waves_
 // half written (5120 x 17408: 227 MB written, so 178, which is the matrix).  It takes 88 registers, so sixteen
 // waves a compute unit, and is faster for that too: twenty-four waves hold 6 MB of lines per XCD open,
 // and with eight registers spilled took as long as the halves did.  One workgroup of sixteen waves copies
-// the tables once where two of eight copy them twice (91.3 and 92.6 us).  HOLD 1 (segments of 32, 96, ..
-// columns, whose neighbours complete the line, and workgroups that would leave a unit to twelve waves).
-// Both keep a unit's last words until the next unit's bytes have arrived (hold_segment), 3 us of 94.
+// the tables once where two of eight copy them twice (91.3 and 92.6 us).  HOLD 1: segments of 32, 96, ..
+// columns, whose neighbours complete the line, and segments of 64 in workgroups that would leave a unit to
+// twelve waves, where some wave has a second unit; with one each nothing is gained by holding (9000 x 2048
+// 27.3 -> 28.2) and HOLD 0 stores as it goes.
+// 1 and 2 keep a unit's last words until the next unit's bytes have arrived (hold_segment), 3 us of 94.
 // Before and now: 5120 x 17408 104.6 -> 91.2 us, 17408 x 5120 -> 87.4, 5120 x 6144 43.9 -> 38.9, 4096 x 4096
-// 24.8 -> 23.0, 2560 x 5120 27.1 -> 22.4; HOLD 1 alone 104.6 -> 102.0 and, PPCX 4096 x 4096, 26.2 -> 25.4.  With
+// 24.8 -> 23.0, 2560 x 5120 27.1 -> 22.4; HOLD 1 alone 104.6 -> 102.0; 700 x 9216 at segments of 32 15.5 -> 14.9.  With
 // the stores absorbed by the cache the first takes 76.  Streaming stores cost 6 %.
 template <class Walk, int SCAN, int HOLD>
 __global__ __launch_bounds__(grf::kFusedMaxThreads) __attribute__((amdgpu_waves_per_eu(HOLD == 2 ? 4 : 6))) void fused_wave_store_kernel(
@@ -749,9 +751,12 @@ int launch_wave_store(const grf_bctx_fused &f, const grf_fused_tiling &g, uint16
   };
   auto launch = [&](auto scan) -> int {
     constexpr int kScan = decltype(scan)::value;
-    if (f.seg_len % 32) return start(KernelOf<&fused_wave_store_kernel<Walk, kScan, 0>>{});
-    if (f.seg_len % 64 == 0 && (g.threads == 1024 || g.threads <= 512))
+    const uint32_t waves = g.threads / 64, rpw = 64 / g.lanes_per_row;
+    const bool one_each = (g.rows_per_tile + rpw - 1) / rpw * g.n_slabs <= waves;  // units
+    // (sixteen waves a unit: in one workgroup, or in all that a unit gets)
+    if (f.seg_len % 64 == 0 && (g.threads == 1024 || g.n_tiles * waves <= 256 * 16))
       return start(KernelOf<&fused_wave_store_kernel<Walk, kScan, 2>>{});
+    if (f.seg_len % 32 || (f.seg_len % 64 == 0 && one_each)) return start(KernelOf<&fused_wave_store_kernel<Walk, kScan, 0>>{});
     return start(KernelOf<&fused_wave_store_kernel<Walk, kScan, 1>>{});
   };
   if (int rc = f.whole_range ? launch(std::integral_constant<int, grf::kScanAny>{})

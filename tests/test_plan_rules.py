@@ -113,3 +113,20 @@ def test_fitted_gemm_tilings_only_where_every_row_count_gains(class_rows, spr, s
         times.append(_fused.gemm_times(*(np.array([v]) for v in (threads, -(-r // 16), blocks, n_slabs, tiles, k, lds_bytes)),
                                        spr, seg, table)[:, 0])
     assert np.all(times[0] >= 1.04 * times[1]) if fitted else plain == other
+
+
+@pytest.mark.parametrize("rows,cols,lines", [(5120, 6144, True), (9000, 2048, False), (1024, 5120, None)])
+def test_whole_lines_where_sixteen_waves_a_unit_are_enough(rows, cols, lines):
+    rng = np.random.default_rng(rows)
+    seg = 64 if lines is not None else 32
+    n = rows * cols // seg
+    offsets = 4 + np.arange(n, dtype=np.int64) * seg * 9 // 16 + rng.integers(0, 4, n)
+    plan = _fused.FramePlan((rows, cols), 16, 4, (np.arange(rows) % 16).astype(np.uint8), np.tile(
+        np.r_[np.full(64, 1024), np.zeros(192)].astype(np.uint32), (64, 1)), np.full(n, 1 << 23, dtype=np.uint32), offsets,
+        int(offsets[-1]) + 64, seg)
+    tiling = plan.lines_tiling()
+    assert (tiling is not None) == bool(lines)
+    if lines:
+        g = tiling["scalars"]
+        assert g["threads"] in (512, 1024) and sorted(tiling["tile_rows"][tiling["tile_rows"] < rows]) == list(range(rows))
+        assert tiling["lds"] * (1024 // g["threads"]) <= _fused.MAX_LDS
