@@ -655,7 +655,8 @@ class HipContextTensor:
         callers that vouch for their ids and must not synchronise (a HIP graph capture); ids
         outside the matrix are then clamped into it."""
         import torch
-        ids = ids.to(device=self.device, dtype=torch.int64)
+        if ids.dtype is not torch.int64 or ids.get_device() != self._index:
+            ids = ids.to(device=self.device, dtype=torch.int64)
         if ids.numel() == 0:
             return torch.empty((*ids.shape, self.shape[1]), device=self.device, dtype=torch.bfloat16)
         if self.fused is not None and self._gather is None:
@@ -682,20 +683,21 @@ class HipContextTensor:
         import torch
         ids = ids.contiguous()
         out = torch.empty((*ids.shape, self.shape[1]), device=self.device, dtype=torch.bfloat16)
-        word = None
+        word = where = None
         if check or validate:
             word = _host_word()
+            where = word.data_ptr()
         if check and self._error_open:  # between checks the word keeps what earlier launches reported
             self.error.zero_()
             self._error_open = False
         elif not check:
             self._error_open = True
         self._launch(self._lib.grf_bctx_gather_rows, ctypes.byref(self.fused), *self._gather, self.buffers["rows"].data_ptr(),
-                     ids.data_ptr(), ids.numel(), out.data_ptr(), word.data_ptr() if check else self.error.data_ptr(),
-                     word.data_ptr() if validate else None)
+                     ids.data_ptr(), ids.numel(), out.data_ptr(), where if check else self.error.data_ptr(),
+                     where if validate else None)
         if word is not None:
-            torch.cuda.current_stream(self.device).synchronize()
-            found = int(word[0])
+            torch.cuda.current_stream(self._index).synchronize()
+            found = ctypes.c_int32.from_address(where).value  # (a tensor's element costs twice the time)
             if found:
                 word[0] = 0
             if len(_host_words) < HOST_WORDS_KEPT:
