@@ -326,7 +326,7 @@ class HipPredictiveTensor:
         reach: 0 = store sink, 1/2/4/8 = GEMV row buckets."""
         if key not in self._tilings:
             import torch
-            host = (self._matrix_plan.gemm_tiling() if key == "gemm" else self._walk_plan.tiling(_fused.WAVE_ROWS_PER_PASS, waves=True)
+            host = (self._matrix_plan.gemm_tiling(self._matrix_plan is self._plan) if key == "gemm" else self._walk_plan.tiling(_fused.WAVE_ROWS_PER_PASS, waves=True)
                     if key == "waves" else self._walk_plan.tiling(key))
             rows = torch.from_numpy(host["tile_rows"].view(np.int32)).to(self.device)
             classes = torch.from_numpy(host["tile_class"]).to(self.device)

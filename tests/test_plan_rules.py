@@ -130,3 +130,15 @@ def test_whole_lines_where_sixteen_waves_a_unit_are_enough(rows, cols, lines):
         g = tiling["scalars"]
         assert g["threads"] in (512, 1024) and sorted(tiling["tile_rows"][tiling["tile_rows"] < rows]) == list(range(rows))
         assert tiling["lds"] * (1024 // g["threads"]) <= _fused.MAX_LDS
+
+
+@pytest.mark.parametrize("rows,cols,other", [(1024, 4096, True), (2048, 2048, False), (5120, 5120, False)])
+def test_predictive_products_take_the_fitted_tiling_where_it_is_sure(rows, cols, other):
+    from georefine_amd import bitexact_predictive_gpu as gpu
+    _, plan = _predictive_plan(rows, cols)
+    plain, fitted = plan.gemm_tiling(), plan.gemm_tiling(True)
+    assert (plain["scalars"] != fitted["scalars"]) == other and fitted["lds"] <= _fused.MAX_LDS
+    g = fitted["scalars"]
+    tiles = fitted["tile_rows"].reshape(-1, g["rows_per_tile"])
+    assert sorted(tiles[tiles < rows].tolist()) == list(range(rows)) and g["n_tiles"] == len(tiles) * g["k_parts"]
+    assert g["threads"] == _fused.gemm_shape(g["lanes_per_row"], g["rows_per_tile"])[2]
