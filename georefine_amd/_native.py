@@ -94,7 +94,7 @@ def codec():
     global _codec
     with _lock:
         if _codec is None:
-            if _stale(CODEC_LIB, codec_sources()):
+            if _stale(CODEC_LIB, [*codec_sources(), CSRC / "piece_units.h"]):
                 build_codec()
             L = ctypes.CDLL(str(CODEC_LIB))
             L.bcx_encode.argtypes = [U16P, _u64, _u32, _u32, U8P, U8P, _u32, _u32, _u32, U32P,

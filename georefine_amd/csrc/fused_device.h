@@ -32,6 +32,7 @@
 #include <type_traits>
 
 #include "georefine_amd.h"
+#include "piece_units.h"
 #include "rans_device.h"
 
 namespace grf {
@@ -487,26 +488,24 @@ __device__ __forceinline__ uint32_t fused_stage_piece_dma(uint8_t *lds, uint32_t
   return g0 & ~15u;
 }
 
-constexpr uint32_t kPieceWindow = 8;  // bytes the refill reads from the aligned cursor on
-
 // The copy of a matrix-core wave's sixteen row pieces (four segments each).  Such a piece is ten or
 // eleven 16-byte units, so one row an instruction, as above, would leave most lanes idle: here the
 // units of all sixteen rows are numbered through, row after row, and an instruction moves 64 of
 // them to where they lie one behind the other.  Which row a unit belongs to: a row's units begin where those of the rows before it end (a
 // running sum over sixteen lanes); the row that begins at unit u of an instruction's 64 marks lane
 // u, and a lane counts the marks up to its own.  Lanes 0..15, and every sixteen after them, hold
-// the rows' byte ranges.  The region holds the most that any sixteen rows take together (166 of these
+// the rows' byte ranges, `held` where the lane's slot has a row.  The region holds the most that any sixteen rows take together (166 of these
 // units on average and 175 at most in 17408 x 5120, where sixteen of the longest piece are 240), so
 // three workgroups of six waves share a compute unit that had two of ten.  Four rows an instruction at
 // the longest piece's pitch took as many instructions: gate+up at 64 rows 157.0 -> 155.6 us, at 128 rows
 // 230 -> 224, down at 64 rows 84.4 -> 83.0, 1500 x 2064 at 6 rows 15.8 -> 14.5.
 __device__ __forceinline__ uint32_t fused_stage_rows_dma(uint8_t *lds, uint32_t region, const grf_bctx_fused &f, uint32_t g0,
-                                                         uint32_t g1, uint32_t lane, uint32_t &piece_off) {
+                                                         uint32_t g1, bool held, uint32_t lane, uint32_t &piece_off) {
   typedef __attribute__((address_space(3))) void lds_void;
   const uint32_t a0 = g0 & ~15u;
 #if defined(__HIP_DEVICE_COMPILE__)
-  const uint32_t units = (g1 - a0 + kPieceWindow + 15) >> 4;  // (at least one: an empty slot's is never read)
-  uint32_t past = units;                                      // units of the rows up to and including the lane's
+  const uint32_t units = piece_units(held, g0, g1);  // (at least one: an empty slot's is never read)
+  uint32_t past = units;                             // units of the rows up to and including the lane's
   auto before = [&](auto ctrl) {  // the same of the lane so many rows before, 0 where there is none
     return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)past, decltype(ctrl)::value, 0xF, 0xF, true);
   };
@@ -530,7 +529,7 @@ __device__ __forceinline__ uint32_t fused_stage_rows_dma(uint8_t *lds, uint32_t 
       __builtin_amdgcn_global_load_lds(f.main_bytes + o, (lds_void *)(lds + (region + u0 * 16)), 16, 0, 0);
   }
 #else
-  (void)lds, (void)region, (void)f, (void)g1, (void)lane, (void)piece_off;
+  (void)lds, (void)region, (void)f, (void)g1, (void)held, (void)lane, (void)piece_off;
 #endif
   return a0;
 }

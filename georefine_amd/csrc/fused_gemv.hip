@@ -122,7 +122,8 @@ int validate_fused_host(const grf_bctx_fused &f, const grf_fused_tiling &g, Tili
             uint64_t sum = 0;
             for (uint32_t r = r0; r < r0 + 16; ++r) {
               const uint32_t row = r < g.rows_per_tile ? tile_rows[(uint64_t)t * g.rows_per_tile + r] : grf::kNoRow;
-              sum += row == grf::kNoRow ? 16 : (entry(row, last) - (uint64_t)(entry(row, s) & ~15u) + 8 + 15) / 16 * 16;
+              const bool held = row != grf::kNoRow;  // (64 bits: an offset may be near the end of 32)
+              sum += 16 * piece_units<uint64_t>(held, held ? entry(row, s) : 0, held ? entry(row, last) : 0);
             }
             if (sum > gemm_region_bytes(g))
               return bad("the stream pieces of slots " + std::to_string(r0) + " on of tile " + std::to_string(t) + " from segment " +

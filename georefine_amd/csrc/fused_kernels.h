@@ -1236,7 +1236,7 @@ __device__ __forceinline__ void fused_gemm_body(uint8_t *lds, const grf_bctx_fus
     const uint32_t col0 = mul24(first_seg + p4, S);
     // the pieces first: their ranges arrived during the walk before
     uint32_t piece_off;
-    const uint32_t a0 = grf::fused_stage_rows_dma(lds, region, f, g0, g1, lane, piece_off);
+    const uint32_t a0 = grf::fused_stage_rows_dma(lds, region, f, g0, g1, row != grf::kNoRow, lane, piece_off);
     Walk w;
     {
       const uint32_t seg = grf::fused_seg_slot<true>(f, active ? row : 0, active ? rpos : 0, active ? first_seg + p4 : 0);

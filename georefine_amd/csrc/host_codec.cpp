@@ -26,6 +26,8 @@
 #include <type_traits>
 #include <vector>
 
+#include "piece_units.h"
+
 namespace {
 
 constexpr uint32_t kScaleBits = 16;
@@ -921,15 +923,16 @@ int grf_unit_pieces(const uint32_t *offsets, uint32_t rows, uint32_t spr, const 
   const uint32_t slabs = (spr + lanes - 1) / lanes;
   try {
     // per slab, the units of the last `together` rows (the slots before the first are empty) and their sum
-    std::vector<uint32_t> units((size_t)together * slabs, 1), sum(slabs, together);
-    uint32_t top = together;
+    const uint32_t empty = grf::piece_units(false, 0u, 0u);
+    std::vector<uint32_t> units((size_t)together * slabs, empty), sum(slabs, together * empty);
+    uint32_t top = together * empty;
     for (uint32_t i = 0, slot = 0; i < rows; ++i, slot = slot + 1 == together ? 0 : slot + 1) {
       if (row_order[i] >= rows) return 1;
       const uint32_t *at = offsets + (size_t)row_order[i] * spr;
       uint32_t *oldest = units.data() + (size_t)slot * slabs;
       for (uint32_t b = 0; b < slabs; ++b) {
         const uint32_t first = at[b * lanes], last = at[std::min(spr, (b + 1) * lanes)];
-        const uint32_t n = (last - (first & ~15u) + 8 + 15) / 16;
+        const uint32_t n = grf::piece_units(true, first, last);
         sum[b] += n - oldest[b];
         oldest[b] = n;
         top = std::max(top, sum[b]);
