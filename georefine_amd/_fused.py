@@ -18,6 +18,15 @@ import numpy as np
 from . import _native
 
 MAX_LDS = 160 * 1024
+LDS_UNIT = 1280  # what a compute unit's LDS is given out in
+
+
+def lds_share(lds):
+    """Workgroups of ``lds`` bytes (a number or an array) that a compute unit's LDS holds: it is given out in
+    units of 1280 bytes, and all 128 of them are there to be had.  Measured with workgroups of one wave
+    that stay: two of 81920 bytes share a unit, three of 53760 and not of 53776, four of 40960, five of 32000 and
+    not of 32016, six of 26880 and not of 26896."""
+    return MAX_LDS // (-(-lds // LDS_UNIT) * LDS_UNIT)
 LUT_BUDGET = int(os.environ.get("GEOREFINE_FUSED_LUT_BYTES", 32 * 1024))
 
 
@@ -236,7 +245,7 @@ def choose_tiling(spr, class_rows, piece_cap_fn, lds_fn, cus=256, seg_len=64, ta
             # A workgroup's waves are dealt round-robin to the CU's four SIMDs; the kernels use
             # up to 72 vector registers, which allows 7 waves per SIMD.
             per_simd = -(-(threads // 64) // 4)
-            per_cu = max(1, min(7 // per_simd, MAX_LDS // lds))
+            per_cu = max(1, min(7 // per_simd, lds_share(lds)))
             waves = per_cu * (threads // 64)
             slots = cus * per_cu
             rounds = -(-tiles // slots)
@@ -345,8 +354,8 @@ def search_wave_tilings(lengths, piece_cap_fn, lds_fn, cus, table_bytes, waves=W
                 lds = lds_fn(threads, p, heights, cap)
                 if lds > MAX_LDS:
                     break
-                # (the waves that the kernel's registers allow; a little LDS stays with the system)
-                per_cu = max(1, min(waves // nwaves, (MAX_LDS - 1024) // lds))
+                # (the waves that the kernel's registers allow)
+                per_cu = max(1, min(waves // nwaves, lds_share(lds)))
                 rounds = -(-tiles // (cus * per_cu))
                 chain *= rounds
                 time = (chain ** 3 + issue ** 3) ** (1 / 3)
@@ -371,7 +380,7 @@ def wave_time(tiling, seg_len, table_bytes, cus=256, waves=WAVES_PER_CU):
     nwaves, rpw = g["threads"] // 64, 64 // g["lanes_per_row"]
     unit_steps, table_steps = seg_len + WAVE_UNIT_OVERHEAD + WAVE_PIECE_OVERHEAD * rpw, 3 + table_bytes / 12288
     units = -(-g["rows_per_tile"] // rpw) * g["n_slabs"]
-    rounds = -(-g["n_tiles"] // (cus * max(1, min(waves // nwaves, (MAX_LDS - 1024) // tiling["lds"]))))
+    rounds = -(-g["n_tiles"] // (cus * max(1, min(waves // nwaves, lds_share(tiling["lds"])))))
     chain = rounds * ((0.5 * -(-units // nwaves) + 0.5 * units / nwaves) * unit_steps + table_steps) * WAVE_LATENCY_RATIO
     issue = g["n_tiles"] / cus * (units * unit_steps + nwaves * table_steps) / 4
     return (chain ** 3 + issue ** 3) ** (1 / 3)
@@ -409,9 +418,9 @@ def gemm_times(threads, tallest, blocks, n_slabs, tiles, k, lds, spr, seg_len, t
     300 x 4096 to 17408 x 5120, each timed at the four row counts: 7 to 10 % rms."""
     waves, quads = threads // 64, -(-spr // 4)
     each = -(-n_slabs // k)
-    most, fullest = np.maximum(1, np.minimum(GEMM_WAVES_PER_SIMD // -(-waves // 4), MAX_LDS // lds)), -(-tiles // cus)
+    most, fullest = np.maximum(1, np.minimum(GEMM_WAVES_PER_SIMD // -(-waves // 4), lds_share(lds))), -(-tiles // cus)
     shared = (tiles > 256) & (threads <= 640) & (lds <= 79 * 1024)
-    fewer = np.where(shared, most, np.maximum(1, np.minimum(4 // -(-waves // 4), MAX_LDS // lds)))
+    fewer = np.where(shared, most, np.maximum(1, np.minimum(4 // -(-waves // 4), lds_share(lds))))
     times = []
     for rows, unit, table, latency, power, launch, cut, part, slot, weight in GEMM_TIMES:
         per_cu = most if rows <= 64 else fewer
@@ -467,13 +476,13 @@ def plan_gemm_tiling(spr, class_rows, piece_cap_fn, lds_fn, cus=256, seg_len=64,
         by_waves = GEMM_WAVES_PER_SIMD // -(-(threads // 64) // 4)
         lds, unit = lds_fn(p, r, cap, 0), 0
         # (a quad's first segment is then a multiple of four, as in unit_fn's count)
-        if MAX_LDS // lds < by_waves and unit_fn is not None and (p % 4 == 0 or n_slabs == 1):
+        if lds_share(lds) < by_waves and unit_fn is not None and (p % 4 == 0 or n_slabs == 1):
             tight = lds_fn(p, r, cap, unit_fn())
-            if min(by_waves, MAX_LDS // tight) > MAX_LDS // lds:
+            if min(by_waves, lds_share(tight)) > lds_share(lds):
                 lds, unit = tight, unit_fn()
         if lds > MAX_LDS:
             continue
-        per_cu = max(1, min(by_waves, MAX_LDS // lds))
+        per_cu = max(1, min(by_waves, lds_share(lds)))
         slots = cus * per_cu
         rounds = -(-(tile_counts[r] * k) // slots)
         # Spread over idle workgroup slots, except a single block of rows where one workgroup has a
@@ -767,7 +776,7 @@ class FramePlan:
         useful steps."""
         g = tiling["scalars"]
         waves, k = g["threads"] // 64, max(1, g["k_parts"])
-        per_cu = max(1, min(GEMM_WAVES_PER_SIMD // -(-waves // 4), MAX_LDS // tiling["lds"]))
+        per_cu = max(1, min(GEMM_WAVES_PER_SIMD // -(-waves // 4), lds_share(tiling["lds"])))
         slabs, slots = -(-g["n_slabs"] // k), 256 * per_cu
         paid = -(-g["n_tiles"] // slots) * slots * waves * 64 * slabs
         share = self.rows * self.spr / paid * min(1.0, per_cu * waves / 24) * _walk_share(slabs, self.seg_len, self.table_bytes())
@@ -887,7 +896,7 @@ class FramePlan:
             # classes of very different sizes: the same workgroup slots, cut so that no tile is
             # taller than it has to be (the kernel walks a tile's real height)
             nwaves, rpw = threads // 64, 64 // p
-            per_cu = max(1, min(waves // nwaves, (MAX_LDS - 1024) // lds))
+            per_cu = max(1, min(waves // nwaves, lds_share(lds)))
             slots = -(-n_tiles // (256 * per_cu)) * 256 * per_cu
             even = build_balanced_tiles(self.row_class, self.nr, rpw, slots, r)
             if even is not None and (even[2] < r or (even[2] == r and len(even[1]) > n_tiles)):
