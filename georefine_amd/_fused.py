@@ -414,8 +414,10 @@ def gemm_times(threads, tallest, blocks, n_slabs, tiles, k, lds, spr, seg_len, t
     are dealt to the four SIMDs in turn, so a count that is no multiple of four fills one SIMD before the
     others (two workgroups of ten: 6 waves where 5 are the mean); waves whose quad a row's last slab
     does not reach leave, and cost nothing there.  Above 64 rows fewer workgroups share a compute unit
-    (``shares_units`` in fused_kernels.h).  Fitted on 2200 forced tilings of fourteen matrices,
-    300 x 4096 to 17408 x 5120, each timed at the four row counts: 7 to 10 % rms."""
+    (``shares_units`` in fused_kernels.h).  Fitted to forced tilings of fourteen matrices with kernels before the
+    present ones.  Against those (profiles/gemm_tilings.csv: 1655 tilings of 44 matrices, made by the program
+    beside it) the times are 5, 7, 6 and 3 % long on average, and 9, 12, 13 and 14 % rms around that; what that is
+    worth between two tilings of one matrix is what ``gain_to_ask`` goes by."""
     waves, quads = threads // 64, -(-spr // 4)
     each = -(-n_slabs // k)
     most, fullest = np.maximum(1, np.minimum(GEMM_WAVES_PER_SIMD // -(-waves // 4), lds_share(lds))), -(-tiles // cus)
@@ -436,6 +438,40 @@ def gemm_times(threads, tallest, blocks, n_slabs, tiles, k, lds, spr, seg_len, t
     return np.stack(times)
 
 
+def gain_to_ask(threads, tiles, k, lds, rows, cus=256):
+    """What ``gemm_times`` has to promise (as a logarithm, over all row counts) before each of several
+    tilings is taken in place of the last one, the slot model's choice, of a matrix of ``rows`` rows: 0.05, and
+    0.08 where the workgroups are dealt less evenly to the compute units or have more waves.  Where the slot
+    model's workgroups share units, the model makes their launch too slow, and it does not know that the
+    sums of the parts of K are written and read once more.  There the lines are what measuring says of
+    tilings below and above them (profiles/gemm_tilings.csv, 281 pairs; mean over 2 to 128 rows by the promise):
+      fewer parts: 0.05, as above: 38 pairs from 0.084 on gain 4 to 44 %
+      cut where the slot model does not cut: 0.147 +5 % (4506 x 2752), 0.132 -1 %, below -2 to -12 %; 0.168 +7 % (6144
+        x 5120).  Never with three workgroups a unit (0.172 -2 %, 8232 x 3072), nor in more than two parts where ten
+        waves or fewer share units above 64 rows too (0.136 -4 %, -20 % at 128 rows, 4837 x 2496)
+      cut finer: 0.05 with up to 8192 sums a row of activations (0.117 +11 %, 1500 x 2064), else 0.165 (0.141 -7 %, 2932 x
+        12160; 0.159 +3 %; 0.184 +5 %, 1483 x 9856)
+      as many parts: 0.15 (0.088 -6 %, 15289 x 768; 0.198 +15 %, 7576 x 512), 0.05 for one workgroup a unit in place of
+        two, 0.19 for one in place of three of eight waves, which fill the unit (0.188 -1 %, 16003 x 512)
+    Of the 227 pairs that pass none loses in the mean; 13 % is gained, and 8 % lost at most at one row count.
+    With 0.05 and 0.08 for all, 35 of 281 lost up to 12 % in the mean and up to 20 % at a row count."""
+    at_once = np.maximum(1, np.minimum(np.minimum(GEMM_WAVES_PER_SIMD // -(-(threads // 64) // 4), lds_share(lds)), -(-tiles // cus)))
+    even = tiles / (-(-tiles // cus) * cus)  # (the fit is least sure of workgroups dealt less evenly to the units)
+    ask = np.where(even < even[-1], 0.08, 0.05)
+    if at_once[-1] == 1:
+        return np.where(threads > threads[-1], 0.08, ask)
+    if k[-1] == 1:
+        refused = (at_once[-1] >= 3) | ((threads[-1] <= 640) & (k > 2))
+        finer = np.where(refused, np.inf, 0.165)
+    else:
+        finer = np.where(rows * k <= 8192, ask, 0.165)
+    if at_once[-1] == 2:
+        alike = np.where(at_once == 1, ask, 0.15)
+    else:
+        alike = np.where((threads[-1] >= 512) & (at_once == 1), 0.19, 0.15)
+    return np.where(k > k[-1], finer, np.where(k < k[-1], ask, alike))
+
+
 def plan_gemm_tiling(spr, class_rows, piece_cap_fn, lds_fn, cus=256, seg_len=64, table_bytes=0, split=False, unit_fn=None,
                      fitted=False):
     """Tiling of the GEMM kernel: workgroups of (row blocks of 16) x (quads of 4
@@ -446,13 +482,11 @@ def plan_gemm_tiling(spr, class_rows, piece_cap_fn, lds_fn, cus=256, seg_len=64,
     second kernel): a matrix with few rows then fills the machine with full blocks of sixteen
     rows.  ``unit_fn()``: the LDS that the pieces of any sixteen rows take together, a fifth to a
     third less than sixteen of the longest; a tiling reserves that where it lets more workgroups
-    share a compute unit.  ``fitted``: that choice against the one that
-    ``gemm_times`` finds the fastest, taken where it is 4 % faster at every row count and 5 % over them
-    all, 8 % where its workgroups are dealt less evenly (us at 4, 20, 50, 100 rows, the slot model's choice and the fitted one: 5120 x 6144 38.3 42.6 46.9
-    70.8 / 36.2 39.4 43.3 57.4, 3000 x 3072 19.3 21.4 23.5 33.4 / 18.5 20.7 21.9 25.0, 450 x 6144 16.3 15.8
-    18.7 23.0 / 13.9 14.1 18.2 20.9, 1024 x 5120 16.5 16.0 19.1 23.6 / 15.3 15.1 19.4 21.8; not taken,
-    5000 x 1536 15.7 19.3 21.0 31.3 / 17.1 20.0 21.1 24.5, 1300 x 11008 25.8 28.9 31.8 45.1 / 26.6 28.7 32.1
-    47.8).  Returns (threads, lanes per row,
+    share a compute unit.  ``fitted``: that choice against the one that ``gemm_times`` finds the fastest, taken
+    where it is modelled 4 % faster at every row count and as much faster over them all as ``gain_to_ask`` says (us
+    at 6, 20, 50, 100 rows, the slot model's choice and the fitted one: 5120 x 6144 36.1 38.5 41.1 61.4 / 32.7 36.2 40.2
+    53.5, 2560 x 5120 23.2 26.0 28.0 33.4 / 19.4 22.3 24.9 32.3, 1024 x 5120 15.0 15.5 18.6 22.1 / 13.5 14.0 17.3 20.6,
+    450 x 6144 15.1 15.7 18.8 22.5 / 12.3 12.7 16.3 19.4).  Returns (threads, lanes per row,
     rows per tile, slabs, tiles of the launch, piece capacity, LDS bytes, k, LDS bytes of a wave's pieces or 0)."""
     best, timed, whole_blocks = None, [], sum(-(-int(c) // 16) for c in class_rows)
     total_rows = sum(int(c) for c in class_rows)
@@ -475,14 +509,15 @@ def plan_gemm_tiling(spr, class_rows, piece_cap_fn, lds_fn, cus=256, seg_len=64,
         cap = piece_cap_fn(p)
         by_waves = GEMM_WAVES_PER_SIMD // -(-(threads // 64) // 4)
         lds, unit = lds_fn(p, r, cap, 0), 0
+        share = lds_share(lds)
         # (a quad's first segment is then a multiple of four, as in unit_fn's count)
-        if lds_share(lds) < by_waves and unit_fn is not None and (p % 4 == 0 or n_slabs == 1):
+        if share < by_waves and unit_fn is not None and (p % 4 == 0 or n_slabs == 1):
             tight = lds_fn(p, r, cap, unit_fn())
-            if min(by_waves, lds_share(tight)) > lds_share(lds):
-                lds, unit = tight, unit_fn()
+            if min(by_waves, lds_share(tight)) > share:
+                lds, unit, share = tight, unit_fn(), lds_share(tight)
         if lds > MAX_LDS:
             continue
-        per_cu = max(1, min(by_waves, lds_share(lds)))
+        per_cu = max(1, min(by_waves, share))
         slots = cus * per_cu
         rounds = -(-(tile_counts[r] * k) // slots)
         # Spread over idle workgroup slots, except a single block of rows where one workgroup has a
@@ -525,8 +560,7 @@ def plan_gemm_tiling(spr, class_rows, piece_cap_fn, lds_fn, cus=256, seg_len=64,
         # one each)
         gain = times[:, -1:] - times
         total = np.array([3, 1, 1, 1]) / 6 @ gain
-        even = tiles / (-(-tiles // cus) * cus)  # (the fit is least sure of workgroups dealt less evenly to the units)
-        total[(gain < 0.04).any(axis=0) | (total < np.where(even < even[-1], 0.08, 0.05))] = 0.0
+        total[(gain < 0.04).any(axis=0) | (total < gain_to_ask(threads, tiles, k, lds, total_rows, cus))] = 0.0
         # (of those that the model cannot tell apart the one with the fewest parts; and the slot model's choice
         # unless the gain is past what the fit is mostly wrong by between two tilings of one matrix)
         if total.max() > 0:
