@@ -729,6 +729,11 @@ def build_gemm_tiles(row_class, nr, r, first_tile=0, lead=0, cus=256):
 GATHER_LANES = 32
 
 
+def lines_limit(rows, cols):
+    """Up to how many times the GEMV's modelled time the whole-line tiling of a decode is taken (``FramePlan.lines_tiling``)."""
+    return 1.25 if 2 * rows * cols >= 48 << 20 else 1.14
+
+
 class FramePlan:
     """Frame-level derived arrays (shared by every tiling) and a tiling factory."""
 
@@ -905,16 +910,19 @@ class FramePlan:
         """The wave units of the kernel that stores whole lines (HOLD 2 of fused_wave_store_kernel), which
         holds 64 columns back and has registers for sixteen waves a compute unit: workgroups of
         sixteen or eight.  None where the walk's segments are no multiple of 64, and where the
-        model's time with sixteen waves is 1.25 times the GEMV's with twenty-four (a wave that has a
-        unit and a little walks two; 9000 x 2048, 1.37: 29.8 us where the GEMV's tiling takes 27.3; 5120 x
-        17408, 1.20: 91.2 and 102)."""
+        model's time with sixteen waves is too far above the GEMV's with twenty-four: 1.25 times it where the
+        result is 48 MiB or more, which the caches do not take up beside what is read, else 1.14 times.  us,
+        four results written in turn, the GEMV's tiling and this one (profiles/whole_lines.csv, 125 matrices): from
+        48 MiB 1.20 5120 x 17408 109.0 93.1, 1.085 5120 x 6144 44.7 41.3, 1.24 8658 x 3904 47.2 42.0 (one result over and
+        over, which stays in the last-level cache, 33.1 35.4 for 5120 x 6144); below 1.13 621 x 13696 20.9 18.3, 1.07
+        4096 x 4096 20.8 21.5, 1.16 1062 x 16384 25.0 25.8, 1.19 3177 x 5760 25.6 27.6, 1.25 11580 x 2048 28.5 33.0."""
         if self.seg_len % 64:
             return None
         key = "lines", os.environ.get("GEOREFINE_FUSED_WAVE_TILING")
         if key not in self._tilings:
             lines, walk = self._wave_tiling(0, LINES_WAVES_PER_CU), self.tiling(WAVE_ROWS_PER_PASS, waves=True)
             slower = (wave_time(lines, self.seg_len, self.table_bytes(), waves=LINES_WAVES_PER_CU)
-                      > 1.25 * wave_time(walk, self.seg_len, self.table_bytes()))
+                      > lines_limit(self.rows, self.cols) * wave_time(walk, self.seg_len, self.table_bytes()))
             self._tilings[key] = None if slower and not key[1] else lines
         return self._tilings[key]
 
