@@ -734,6 +734,20 @@ def lines_limit(rows, cols):
     return 1.25 if 2 * rows * cols >= 48 << 20 else 1.14
 
 
+def fewer_lookups_pay(seg_len, spr, tiling, lds, gain):
+    """Whether a predictive weight's matrix-core products take their small lookups, whose ``tiling`` uses
+    ``gain`` times the share of the wave slots by ``plan_gemm_tiling``'s model: where that is half as much again,
+    three workgroups of eight waves, all that a unit holds, share it, and their waves' quads leave at
+    most a sixteenth of the lanes without a segment of 64 symbols.  Two, six and 96 rows, us, 64 / 16 KiB
+    (profiles/predictive_lookups.csv, 229 matrices): 4096 x 4096 34.3 34.1 44.1 / 30.3 30.2 41.2, 16384 x 1024
+    29.6 29.4 39.7 / 28.1 27.9 37.8, 8489 x 1984 30.8 30.4 39.0 / 29.1 28.7 38.5; not with shorter segments (4926 x 1952
+    22.0 21.6 29.2 / 24.4 23.9 31.4), emptier slabs (8650 x 1856 29.7 29.3 37.6 / 32.9 32.2 41.8), seven waves (9821 x
+    1728 29.9 29.4 38.0 / 32.4 31.9 42.4) or two workgroups (2048 x 8192 34.7 34.3 44.7 / 30.7 30.4 52.7)."""
+    lanes = -(-tiling["lanes_per_row"] // 4) * 4 * tiling["n_slabs"]
+    return (gain >= 1.5 and seg_len >= 64 and tiling["threads"] == 512 and tiling["n_tiles"] > 512 and lds_share(lds) >= 3
+            and 16 * spr >= 15 * lanes)
+
+
 class FramePlan:
     """Frame-level derived arrays (shared by every tiling) and a tiling factory."""
 
@@ -785,20 +799,9 @@ class FramePlan:
 
     def for_matrix_cores(self, main_freq, budget, image=None):
         """This plan, or one like it with lookups of at most ``budget`` bytes where the matrix-core
-        launches of the matrix are the faster for them: where three workgroups of eight waves then share
-        a compute unit that had one of ten to sixteen, each with half as many slabs to walk in a row,
-        which ``plan_gemm_tiling``'s model sees as half as much again.  Only tilings that the kernels
-        for more than 64 rows can share a unit with too (``shares_units`` in fused_kernels.h).  Fewer
-        bytes mean more scans, 13 % of the same tiling's time.  Six, 32 and 96 rows, us, predictive
-        frames at 64 / 16 KiB, and the modelled advantage:
-          4096 x 4096    1.86   37.0 39.9 51.7 / 31.6 34.8 43.5
-          8192 x 2048    1.97   31.9 35.3 41.9 / 29.3 32.3 39.5
-          16384 x 1024   1.97   30.9 34.8 41.6 / 30.0 33.4 40.0
-          5120 x 5120    1.09   37.7 41.6 52.8 / 46.2 49.6 62.1
-          7000 x 1600    1.06   20.8 23.9 29.5 / 27.8 31.3 38.4
-          2048 x 8192    1.83   37.7 40.8 52.6 / 34.8 37.5 58.2  (704 threads)
-          5120 x 17408   1.54   90.7 96.0 135 / 92.9 98.1 156  (768 threads)
-        A grouped launch keeps this plan's (three of 4096 x 4096: 67.2 69.2 96 / 72.6 74.8 125)."""
+        launches of the matrix are the faster for them (``fewer_lookups_pay``).  Fewer bytes mean more scans,
+        13 % of the same tiling's time, and let three workgroups share a unit that had one.  A grouped launch keeps
+        this plan's (three of 4096 x 4096 at six, 32 and 96 rows: 67.2 69.2 96 us / 72.6 74.8 125)."""
         other = self.with_lookups(main_freq, budget, image)
         if other.lognb >= self.lognb:
             return self
@@ -806,9 +809,8 @@ class FramePlan:
             tall, fine = self.gemm_tiling(), other.gemm_tiling()
         except FusedUnsupported:
             return self
-        g = fine["scalars"]
-        shared = g["n_tiles"] > 256 and g["threads"] <= 640 and fine["lds"] <= 79 * 1024
-        return other if shared and other.gemm_share(fine) >= 1.5 * self.gemm_share(tall) else self
+        gain = other.gemm_share(fine) / self.gemm_share(tall)
+        return other if fewer_lookups_pay(self.seg_len, self.spr, fine["scalars"], fine["lds"], gain) else self
 
     def gemm_share(self, tiling):
         """What ``plan_gemm_tiling``'s model says of one tiling: the share of the machine's wave slots that do

@@ -50,9 +50,9 @@ def _checkpoints(stream, ctx, freq, vocab, stride):
 # Sixteen bin contexts share the lookup bytes.  A wave scans on whenever one of its 64 lanes meets
 # a bucket's minority symbol: 35 % of the steps with 1 KiB per context, 21 % with 2 KiB, 12 % with
 # 4 KiB.  At 64 KiB one workgroup of sixteen waves has a compute unit to itself instead of two of
-# twelve, and still wins for products on the matrix cores (16 / 32 / 64 KiB in all, us: 4096 x 4096
-# at 96 rows 43.5 / 53.1 / 51.7, 3000 x 4096 36.4 / 32.6 / 31.9, 5120 x 17408 156 / 142 / 135, 512 x 1024 at
-# 64 rows 15.8 / 15.2 / 15.1), except where three of eight waves at 16 KiB do (FramePlan.for_matrix_cores).
+# twelve, and still wins for products on the matrix cores (16 / 32 / 64 KiB in all, us: 3000 x 4096
+# at 96 rows 36.4 / 32.6 / 31.9, 5120 x 17408 156 / 142 / 135, 512 x 1024 at 64 rows 15.8 / 15.2 / 15.1), except
+# where three of eight waves at 16 KiB do (_fused.fewer_lookups_pay).
 # One row and decode() take 32 KiB where those are faster (FramePlan.for_vector_alus).  The tensor keeps
 # every lookup it uses, half and a quarter MiB more.
 _LUT_BUDGET, _WALK_LUT_BUDGET = ((int(os.environ["GEOREFINE_FUSED_LUT_BYTES"]),) * 2

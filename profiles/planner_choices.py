@@ -7,7 +7,8 @@
 (``FramePlan.for_matrix_cores``), us a call among others at 2 to 128 rows.  ``lines``: decode to dense with the GEMV's
 tiling and with that of the kernel that stores whole lines (``FramePlan.lines_tiling``), by how many results are written
 in turn (one stays in the last-level cache while it fits, four do not).  One line per matrix, with the
-tilings and what the planner's model says of them; ``taken``: what the planner takes.
+tilings and what the planner's model says of them.  predictive_lookups.csv holds such a run and one over
+more matrices where three workgroups share a unit.
 """
 import collections
 import csv
@@ -62,7 +63,10 @@ def described(name, tiling):
 def predictive_matrices(rng):
     whole = lambda low, high: int(round(math.exp(rng.uniform(math.log(low), math.log(high)))))
     yield from [(4096, 4096), (8192, 2048), (16384, 1024), (3152, 4544), (1624, 4800), (1092, 12480), (2048, 8192)]
-    for _ in range(420):
+    for _ in range(60):  # about where three workgroups share a unit
+        cols = 64 * rng.choice((rng.randint(12, 16), rng.randint(24, 32), rng.randint(52, 64)))
+        yield whole((13 << 20) // cols, min(17408, (17 << 20) // cols)), cols
+    for _ in range(240):
         step = 64 if rng.random() < 0.75 else 32
         cols = max(512, whole(512, 17408) // step * step)
         rows = whole(512, min(17408, (16 << 20) // cols))
@@ -75,7 +79,7 @@ def lookups(rng):
     for rows, cols in predictive_matrices(rng):
         w, g = weights(rows, cols)
         reference = words(w.bfloat16().float() + 0.002 * torch.randn(rows, cols, device="cuda", generator=g))
-        frame, sides, taken, ratio = predictive.encode(words(w), reference), [], None, 0.0
+        frame, sides = predictive.encode(words(w), reference), []
         _fused.FramePlan.for_matrix_cores = lambda plan, *a: plan
         try:
             sides.append(HipPredictiveTensor(frame, reference, device="cuda:0"))
@@ -86,30 +90,19 @@ def lookups(rng):
             sides.append(HipPredictiveTensor(frame, reference, device="cuda:0"))
         finally:
             _fused.FramePlan.for_matrix_cores = choice
-        freq = codec_frequencies(frame, reference)
-        taken = plan.for_matrix_cores(freq, 16 << 10, _word_image()) is not plan
         other = sides[1]._matrix_plan
         tall, fitted, fine = plan.gemm_tiling(False), plan.gemm_tiling(True), other.gemm_tiling(False)
         g = fine["scalars"]
         if g["n_tiles"] <= 256 or _fused.lds_share(fine["lds"]) < 2:  # (a workgroup a unit on either side)
             continue
         copies = [[t, t.clone(), t.clone()] for t in sides]
-        line = dict(rows=rows, cols=cols, seg_len=plan.seg_len, taken=int(taken), share_64=round(plan.gemm_share(tall), 4),
+        line = dict(rows=rows, cols=cols, seg_len=plan.seg_len, share_64=round(plan.gemm_share(tall), 4),
                     share_64_fitted=round(plan.gemm_share(fitted), 4), share_16=round(other.gemm_share(fine), 4),
                     **described("slot", tall), **described("fitted", fitted), **described("small", fine))
         for m in ROWS:
             x = torch.randn(m, cols, device="cuda").bfloat16()
             line[f"us64_{m}"], line[f"us16_{m}"] = both_us([lambda j, c=c: c[j].linear(None, x) for c in copies])
         yield line
-
-
-def codec_frequencies(frame, reference):
-    return predictive.parse(frame, reference)["main_freq"].reshape(predictive.MAIN_CONTEXTS, predictive.MAIN_VOCAB)
-
-
-def _word_image():
-    from georefine_amd import bitexact_predictive_gpu
-    return bitexact_predictive_gpu._word_image
 
 
 def whole_lines(rng):
@@ -123,8 +116,6 @@ def whole_lines(rng):
         plan = tensor._plan
         if plan is None or plan.seg_len % 64:
             continue
-        plan._tilings.pop(("lines", None), None)
-        taken = plan.lines_tiling() is not None
         plan._tilings.pop(("lines", None), None)
         _fused.wave_time = lambda *a, **k: 1.0
         try:
@@ -142,8 +133,7 @@ def whole_lines(rng):
         for results in (1, 2, 4):  # how many the program writes in turn: a result's buffer is free once no one holds it
             kept = collections.deque(maxlen=results - 1)
             us[results] = both_us([lambda j, c=c: kept.append(c[j].decode(check=False)) for c in copies])
-        yield dict(rows=rows, cols=cols, seg_len=plan.seg_len, taken=int(taken),
-                   model_walk=round(rule(walk, plan.seg_len, plan.table_bytes()), 1),
+        yield dict(rows=rows, cols=cols, seg_len=plan.seg_len, model_walk=round(rule(walk, plan.seg_len, plan.table_bytes()), 1),
                    model_lines=round(rule(lines, plan.seg_len, plan.table_bytes(), waves=_fused.LINES_WAVES_PER_CU), 1),
                    **described("walk", walk), **described("lines", lines),
                    **{f"us_{name}_{n}": us[n][i] for n in us for i, name in enumerate(("walk", "lines"))})
@@ -158,7 +148,7 @@ def main():
                 writer.writeheader()
             writer.writerow(line)
             file.flush()
-            print(line["rows"], line["cols"], line["taken"], flush=True)
+            print(line["rows"], line["cols"], flush=True)
 
 
 if __name__ == "__main__":

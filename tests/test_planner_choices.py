@@ -29,3 +29,17 @@ def test_whole_lines_are_taken_where_they_were_measured_faster():
 @pytest.mark.parametrize("rows,cols,limit", [(4096, 6144, 1.25), (4095, 6144, 1.14), (17408, 5120, 1.25), (256, 512, 1.14)])
 def test_whole_lines_limit_by_the_size_of_the_result(rows, cols, limit):
     assert _fused.lines_limit(rows, cols) == limit
+
+
+def test_small_predictive_lookups_are_taken_where_they_were_measured_faster():
+    taken, refused = [], []
+    for line in _measured("predictive_lookups.csv"):
+        one = lambda name: int(line[name])
+        tiling = {key: one("small_" + key) for key in ("threads", "lanes_per_row", "n_slabs", "n_tiles")}
+        pays = _fused.fewer_lookups_pay(one("seg_len"), one("cols") // one("seg_len"), tiling, one("small_lds"),
+                                        float(line["share_16"]) / float(line["share_64"]))
+        (taken if pays else refused).append([float(line[f"us64_{m}"]) / float(line[f"us16_{m}"]) - 1 for m in (2, 6, 20, 32, 64, 96, 128)])
+    taken, refused = np.array(taken), np.array(refused)
+    assert len(taken) > 10 and len(refused) > 100
+    assert taken.mean() > 0.04 and taken.mean(axis=1).min() > -0.03 and taken.min() > -0.06
+    assert refused.mean() < -0.05
