@@ -1015,10 +1015,14 @@ def plan_group(plans, m=None, gemm=False, waves=False, mixed=False):
         scheme = SCHEME_WAVES
         lds_fn = lambda p_, r_, cap_, unit_: max(lds_bytes_gemm(pl.nc, pl.lognb, pl.tabn, p_, r_, cap_, unit_) for pl in plans)
         quad_cap = max(pl.quad_cap() for pl in plans)
-        # (lanes per row follow the first member's length: where another's differs, a slab may begin between two quads)
-        unit_fn = (lambda: max(pl.quad_bytes() for pl in plans)) if all(pl.spr == first.spr for pl in plans) else None
-        threads, p, r, _, _, cap, lds, _, unit = plan_gemm_tiling(first.spr, class_rows, lambda lanes: quad_cap, lds_fn,
-                                                                  seg_len=first.seg_len, table_bytes=table, unit_fn=unit_fn)
+        plan = dict(seg_len=first.seg_len, table_bytes=table)
+        if all(pl.spr == first.spr for pl in plans):
+            threads, p, r, _, _, cap, lds, _, unit = plan_gemm_tiling(first.spr, class_rows, lambda lanes: quad_cap, lds_fn, **plan,
+                                                                      unit_fn=lambda: max(pl.quad_bytes() for pl in plans))
+        else:  # (lanes per row follow the first member's length: a slab of another's may begin between two quads)
+            threads, p, r, _, _, cap, lds, _ = choose_gemm_tiling(first.spr, class_rows, lambda lanes: quad_cap,
+                                                                  lambda p_, r_, cap_: lds_fn(p_, r_, cap_, 0), **plan)
+            unit = 0
     elif waves:
         scheme = SCHEME_WAVES
         seg_lens = list(dict.fromkeys(pl.seg_len for pl in [first, *plans]))

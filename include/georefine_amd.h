@@ -291,7 +291,6 @@ typedef struct grf_bctx_fused {
  * n_slabs = ceil(segs_per_row / lanes_per_row) in both schemes. */
 #define GRF_TILE_SLABS 0
 #define GRF_TILE_WAVES 1
-#define GRF_TILE_WAVE_UNITS(units) ((uint32_t)(units) << 8)
 typedef struct grf_fused_tiling {
   const uint32_t *tile_rows;
   const uint8_t *tile_class;
