@@ -496,7 +496,9 @@ __device__ __forceinline__ uint32_t fused_stage_piece_dma(uint8_t *lds, uint32_t
 // u, and a lane counts the marks up to its own.  Lanes 0..15, and every sixteen after them, hold
 // the rows' byte ranges, `held` where the lane's slot has a row.  The region holds the most that any sixteen rows take together (166 of these
 // units on average and 175 at most in 17408 x 5120, where sixteen of the longest piece are 240), so
-// three workgroups of six waves share a compute unit that had two of ten.  Four rows an instruction at
+// three workgroups of six waves share a compute unit that had two of ten; half as many workgroups again copy
+// the tables for it, and the numbering is work of its own (gate+up at 64 rows reads and writes 323 MB, so 308,
+// at 22.1 VALU instructions and 18.4 LDS cycles a step, so 21.4 and 17.7).  Four rows an instruction at
 // the longest piece's pitch took as many instructions: gate+up at 64 rows 157.0 -> 155.6 us, at 128 rows
 // 230 -> 224, down at 64 rows 84.4 -> 83.0, 1500 x 2064 at 6 rows 15.8 -> 14.5.
 __device__ __forceinline__ uint32_t fused_stage_rows_dma(uint8_t *lds, uint32_t region, const grf_bctx_fused &f, uint32_t g0,
