@@ -438,6 +438,22 @@ def gemm_times(threads, tallest, blocks, n_slabs, tiles, k, lds, spr, seg_len, t
     return np.stack(times)
 
 
+def spread_apart(tiles, slots, unit):
+    """Whether a launch whose workgroups share compute units by the tight reservation (``unit`` bytes a wave) is spread
+    over the ``slots`` it had without: where its tiles all have one of those, shorter tiles only mean more
+    copies of the tables (three of 4612 x 768 at one, 32, 100 rows in 480 tiles or spread to 768: 19.5 22.7 31.8 us, 21.0
+    24.4 33.6; 7162 x 1408 in 512 or 720: 16.9 19.5 26.9, 19.8 22.9 30.4)."""
+    return unit > 0 and tiles <= slots
+
+
+def closer_workgroups_pay(p, n_slabs):
+    """Whether the tight reservation, which lets more and smaller workgroups share a compute unit, is worth taking for
+    tiles of ``p`` lanes a row: not where a wave walks one slab of two quads, 512 columns of 64-symbol segments,
+    which is little beside its copy of the tables (two of 14853 x 512 at one, 32, 100 rows in 512 tiles of eight
+    waves or 768 of six: 20.1 25.0 37.1 us, 21.8 26.6 38.1; 7609 and 5555 x 512 16.1 19.5 30.2, 17.1 20.9 31.6)."""
+    return p > 8 or n_slabs > 1
+
+
 def gain_to_ask(threads, tiles, k, lds, rows, cus=256):
     """What ``gemm_times`` has to promise (as a logarithm, over all row counts) before each of several
     tilings is taken in place of the last one, the slot model's choice, of a matrix of ``rows`` rows: 0.05, and
@@ -511,7 +527,8 @@ def plan_gemm_tiling(spr, class_rows, piece_cap_fn, lds_fn, cus=256, seg_len=64,
         lds, unit = lds_fn(p, r, cap, 0), 0
         share = lds_share(lds)
         # (a quad's first segment is then a multiple of four, as in unit_fn's count)
-        if share < by_waves and unit_fn is not None and (p % 4 == 0 or n_slabs == 1):
+        apart = share  # workgroups a unit where every piece has the LDS of the longest
+        if share < by_waves and unit_fn is not None and (p % 4 == 0 or n_slabs == 1) and closer_workgroups_pay(p, n_slabs):
             tight = lds_fn(p, r, cap, unit_fn())
             if min(by_waves, lds_share(tight)) > share:
                 lds, unit, share = tight, unit_fn(), lds_share(tight)
@@ -527,8 +544,10 @@ def plan_gemm_tiling(spr, class_rows, piece_cap_fn, lds_fn, cus=256, seg_len=64,
         # -> 16.2 us, 901 x 8192 20.1 -> 19.2; 257 tiles of one row against 17: 257 x 560 10.7 ->
         # 8.9).  Where they pay: 3000 x 3072, 512 tiles of 12 rows 21.2, 384 of 16 21.7.
         whole = row_blocks == 1 and (per_cu == 1 or 2 * tile_counts[r] * k <= slots)
-        r_used = r if forced or whole else _spread_rows(tile_counts, r, rounds * slots // k,
-                                                        floor=16 * (row_blocks - 1) + 1)
+        room = rounds * slots
+        if spread_apart(tile_counts[r] * k, cus * apart, unit):
+            room = cus * apart
+        r_used = r if forced or whole else _spread_rows(tile_counts, r, room // k, floor=16 * (row_blocks - 1) + 1)
         tiles_used = tile_counts[r_used] * k
         slabs_each = -(-n_slabs // k)
         # work = lane-steps; capacity = every wave slot of every round for the whole walk

@@ -35,3 +35,16 @@ def test_the_models_see_the_round_that_does_not_fit(lds, rounds):
     times = [_fused.gemm_times(np.array([512]), np.array([1]), np.array([1.0]), np.array([3]), many, np.array([1]), np.array([v]), 24, 64, 0)
              for v in (50000, lds)]
     assert bool((times[0] == times[1]).all()) == (rounds == 1)
+
+
+@pytest.mark.parametrize("rows,siblings,spr,tiles,tight", [
+    (4612, 3, 12, 480, True),    # three workgroups a unit may share: 768 slots, and 512 without the tight reservation
+    (7162, 1, 22, 512, True),
+    (14853, 2, 8, 512, False),   # one slab of two quads
+])
+def test_tiles_that_all_run_at_once_are_not_cut_shorter_to_fill_the_closer_slots(rows, siblings, spr, tiles, tight):
+    table = 35200
+    lds = lambda p, r, cap, unit: max(table + _fused.gemm_shape(p, r)[2] // 64 * (unit or 16 * cap), _fused.gemm_shape(p, r)[2] // 64 * 4096)
+    class_rows = np.concatenate([np.bincount(np.arange(rows) % 16)] * siblings)
+    found = _fused.plan_gemm_tiling(spr, class_rows, lambda lanes: 208, lds, seg_len=64, table_bytes=table, unit_fn=lambda: 2816)
+    assert found[4] == tiles and (found[8] == 2816) == tight and _fused.lds_share(found[6]) >= (3 if tight else 2)
