@@ -991,12 +991,20 @@ class FramePlan:
         ``fitted`` (default: for the context codec): may be ``gemm_times``' choice.  The fit is the context
         codec's; predictive frames with lookups of 64 KiB, a workgroup a unit, gain by it as well (1024 x
         4096 at six and 96 rows 18.5 24.6 -> 15.9 22.1 us, 512 x 8192 18.5 26.2 -> 16.8 24.1, 1000 x 16384
-        40.1 56.4 -> 35.0 48.3; eight others keep their tiling)."""
+        40.1 56.4 -> 35.0 48.3; eight others keep their tiling).  Planned once for a matrix and its clones: it
+        takes 1.7 ms, a third more than before there was a fit, and a predictive tensor's first product paid for it."""
+        fitted = GEMM_SPLIT and (self.nc <= 4 if fitted is None else fitted)
+        key = "gemm", fitted, GEMM_SPLIT, GEMM_BALANCE, GEMM_WAVES_PER_SIMD, os.environ.get("GEOREFINE_FUSED_GEMM_TILING")
+        if key not in self._tilings:
+            self._tilings[key] = self._gemm_tiling(fitted)
+        return self._tilings[key]
+
+    def _gemm_tiling(self, fitted):
         self._wave_limits()
         threads, p, r, n_slabs, n_tiles, cap, lds, k, unit = plan_gemm_tiling(
             self.spr, self.class_rows, lambda lanes: self.quad_cap(),
             lambda p_, r_, cap_, unit_: lds_bytes_gemm(self.nc, self.lognb, self.tabn, p_, r_, cap_, unit_),
-            seg_len=self.seg_len, table_bytes=self.table_bytes(), split=GEMM_SPLIT, unit_fn=self.quad_bytes, fitted=GEMM_SPLIT and (self.nc <= 4 if fitted is None else fitted))
+            seg_len=self.seg_len, table_bytes=self.table_bytes(), split=GEMM_SPLIT, unit_fn=self.quad_bytes, fitted=fitted)
         # the row tiles; the launch has k of each
         tile_rows, tile_class, r, _ = build_gemm_tiles(self.row_class, self.nr, r)
         threads = gemm_shape(p, r)[2]  # (classes that fit fewer blocks of sixteen rows than were planned)

@@ -114,7 +114,7 @@ def most_promised(plan):
     asked = _fused.gain_to_ask
     _fused.gain_to_ask = lambda threads, tiles, k, lds, rows, cus=256: np.full(len(k), 0.05)
     try:
-        return plan.gemm_tiling()
+        return plan._gemm_tiling(True)
     finally:
         _fused.gain_to_ask = asked
 

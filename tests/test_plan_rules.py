@@ -142,3 +142,17 @@ def test_predictive_products_take_the_fitted_tiling_where_it_is_sure(rows, cols,
     tiles = fitted["tile_rows"].reshape(-1, g["rows_per_tile"])
     assert sorted(tiles[tiles < rows].tolist()) == list(range(rows)) and g["n_tiles"] == len(tiles) * g["k_parts"]
     assert g["threads"] == _fused.gemm_shape(g["lanes_per_row"], g["rows_per_tile"])[2]
+
+
+def test_a_matrix_core_tiling_is_planned_once_for_a_plan_and_anew_for_other_lookups_and_settings(monkeypatch):
+    from georefine_amd import bitexact_predictive_gpu as gpu
+    freq, plan = _predictive_plan(1024, 4096)
+    plain, fitted = plan.gemm_tiling(), plan.gemm_tiling(True)
+    assert plan.gemm_tiling() is plain and plan.gemm_tiling(False) is plain and plan.gemm_tiling(True) is fitted is not plain
+    other = plan.with_lookups(freq, gpu._MATRIX_LUT_BUDGET, gpu._word_image).gemm_tiling()
+    assert other is not plain and other["lds"] != plain["lds"] and plan.gemm_tiling() is plain
+    monkeypatch.setenv("GEOREFINE_FUSED_GEMM_TILING", "16,16,1")
+    assert plan.gemm_tiling()["scalars"]["lanes_per_row"] == 16
+    monkeypatch.delenv("GEOREFINE_FUSED_GEMM_TILING")
+    monkeypatch.setattr(_fused, "GEMM_SPLIT", False)
+    assert plan.gemm_tiling(True)["scalars"]["k_parts"] == 1 < fitted["scalars"]["k_parts"]
