@@ -208,6 +208,44 @@ def bias_for(bias, index, device):
     return bias.to(device=device, dtype=torch.bfloat16).contiguous()
 
 
+def _plain(t, index):
+    """A BF16 tensor on the GPU that is nothing but its values: no subclass, no gradient asked for."""
+    import torch
+    return (type(t) in (torch.Tensor, torch.nn.Parameter) and t.dtype is torch.bfloat16 and t.get_device() == index
+            and t.layout is torch.strided and not t.is_neg() and not (t.requires_grad and torch.is_grad_enabled()))
+
+
+def _observed():
+    """Whether torch would do more with an operator than run it: a transform, a mode, a tracer, autocast."""
+    import torch
+    return (torch.is_autocast_enabled("cuda") or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
+            or torch._C._functorch.peek_interpreter_stack() is not None or torch._C._get_tracing_state() is not None
+            or torch.autograd.forward_ad._current_level >= 0)
+
+
+def dense_linear(lib, x, weight, bias, index):
+    """``F.linear`` of activations with a decoded matrix on GPU ``index``: the library's product, or the one of
+    ``grf_dense_gemm`` where that is the faster (its plan says so by the sizes) and nothing but the values
+    is asked for.  What torch would refuse, differentiate, trace or convert goes to torch."""
+    import torch
+    rows, cols = weight.shape
+    m = x.numel() // cols if cols else 0
+    size = lib.grf_dense_gemm_plan(rows, cols, m) if m < 1 << 30 else -1  # (first: the calls that it sends on pay nothing else)
+    if (size < 0 or not _plain(x, index) or not x.dim() or x.shape[-1] != cols or not weight.is_contiguous() or weight.data_ptr() & 15
+            or bias is not None and not (_plain(bias, index) and bias.shape == (rows,) and bias.is_contiguous()) or _observed()):
+        return torch.nn.functional.linear(x, weight, bias)
+    x2, ldx = rows_for(x, cols, index, x.device)
+    if not cols <= ldx <= 1 << 21:  # (rows that overlap, or lie too far apart)
+        x2, ldx = x2.clone(memory_format=torch.contiguous_format), cols
+    y = x2.new_empty((*x.shape[:-1], rows))
+    space = x2.new_empty(size // 2) if size else None
+    status = launch_on(index, lib.grf_dense_gemm, weight.data_ptr(), rows, cols, x2.data_ptr(), ldx, m, y.data_ptr(), rows,
+                       bias.data_ptr() if bias is not None else None, space.data_ptr() if size else None, size)
+    if status:
+        raise base.CodecError(f"device launch failed ({status}): " + lib.grf_last_error().decode(errors="replace"))
+    return y
+
+
 class PackedActivations:
     """Activation rows copied once into the operand order of the matrix-core kernels, for
     several coded matrices that take the same input (q/k/v, gate/up): ``gemm`` and
@@ -527,14 +565,14 @@ class HipContextTensor:
             return self.buffers["raw"].view(torch.bfloat16).reshape(self.shape)
         if self.fused is None or general:
             return self._decode_blocks(check=check)[:self.n].reshape(self.shape)
-        out = torch.empty(self.n, device=self.device, dtype=torch.uint16)
+        out = torch.empty(self.shape, device=self.device, dtype=torch.bfloat16)
         if check:  # between checks the word keeps what earlier launches reported
             self.error.zero_()
         self._error_open = True
         self._launch(self._lib.grf_bctx_fused_decode, ctypes.byref(self.fused), ctypes.byref(self._store_tiling()[0]),
                      out.data_ptr(), self.error.data_ptr())
         self._check(check)
-        return out.view(torch.bfloat16).reshape(self.shape)
+        return out
 
     def _gemm_tiling(self):
         if "gemm" not in self._tilings:
@@ -625,7 +663,7 @@ class HipContextTensor:
         The row count picks the kernel family (``route_rows``): by default the fastest one --
         the fused decode-GEMV for one row (and two rows of a short-row matrix), the fused
         decode-GEMM to 128 rows (one launch), above that a fused decode to a dense transient
-        and the library matmul (a second GEMM launch would decode the matrix again).
+        and a matmul (``dense_linear``; a second GEMM launch would decode the matrix again).
         ``batch_invariant=True`` -- or the tensor's ``m_invariant`` policy, which is the default
         when the argument is left out -- sends every row count through the GEMM, so that a
         row's output never depends on the batch it arrives in: ``linear(x[:1])`` is
@@ -640,8 +678,7 @@ class HipContextTensor:
         m = x.numel() // width if width else math.prod(x.shape[:-1])
         route = "dense" if self.fused is None else route_rows(m, self.shape[1], batch_invariant)
         if route == "dense":
-            import torch.nn.functional as F
-            return F.linear(x.to(self.device), self.decode(check=check), bias)
+            return dense_linear(self._lib, x.to(self.device), self.decode(check=check), bias, self._index)
         if route == "gemm":
             return self.gemm(x, bias, check=check)
         return self.gemv(x, bias, check=check)

@@ -512,6 +512,20 @@ int grf_ppcx_gemm_group(uint32_t n, const grf_ppcx_fused *const *frames, const g
                         uint16_t *const *y, const uint32_t *ldy, const uint16_t *const *bias, void *workspace,
                         size_t workspace_bytes, int32_t *error, void *hip_stream);
 
+/* y = x W^T (+ bias) for a dense BF16 matrix W [rows][cols], on the matrix cores: the second half of a product of
+ * more rows than the fused kernels take, after the decode (F.linear, GCR/bitexact_context_serving.py:365-376).
+ * fp32 sums in a fixed order for given sizes, the bias in fp32, one rounding.
+ *   grf_dense_gemm_plan             bytes of workspace the product takes, or -1 where the library's
+ *                                   matmul is the better choice (or the sizes are not taken); needs no GPU
+ *   grf_dense_gemm_workspace_bytes  the same bytes, whichever is better
+ * cols is a multiple of 8, ldx one of at least cols; both at most 2^21; rows * m_rows at most 2^30.  w, x and
+ * workspace are 16-byte, y is 8-byte aligned.  It allocates nothing and can be captured. */
+int64_t grf_dense_gemm_plan(uint32_t rows, uint32_t cols, uint32_t m_rows);
+size_t grf_dense_gemm_workspace_bytes(uint32_t rows, uint32_t cols, uint32_t m_rows);
+int grf_dense_gemm(const uint16_t *w, uint32_t rows, uint32_t cols, const uint16_t *x, uint32_t ldx, uint32_t m_rows,
+                   uint16_t *y, uint32_t ldy, const uint16_t *bias, void *workspace, size_t workspace_bytes,
+                   void *hip_stream);
+
 /* A one-lane kernel that writes slot[0] = the device's constant-rate counter
  * (grf_wall_clock_khz), slot[1] = its shader-clock counter and slot[2] = the identifier of the
  * compute unit it ran on, all read when the kernel runs, i.e. in stream order after the work
