@@ -116,10 +116,10 @@ def _index_views(frame, stride, fused_segment, raw6_residual):
     return out
 
 
-def _device_stream(buffers, name, vocab, nctx):
+def _device_stream(buffers, name, stream, vocab, nctx):
     s = _hip_abi.GrfStream()
-    s.bytes = buffers[name + "_stream"].data_ptr()
-    s.n_bytes = buffers[name + "_stream"].numel()
+    s.bytes = buffers[stream].data_ptr()
+    s.n_bytes = buffers[stream].numel()
     s.vocab, s.nctx = vocab, nctx
     if name + "_cum" in buffers:
         s.cum = buffers[name + "_cum"].data_ptr()
@@ -284,6 +284,28 @@ class PackedActivations:
         return self.buffer
 
 
+class _Buffers(dict):
+    """A tensor's device arrays by name.  ``residual_stream`` of a tensor that keeps its residual groups in pair
+    form (``residual_pairs``, ``GRF_RAW_PAIRS``) is made when it is asked for: packed fields, not kept."""
+
+    def __missing__(self, name):
+        if name != "residual_stream" or "residual_pairs" not in self:
+            raise KeyError(name)
+        return _residual_form(self["residual_pairs"].clone(), False)
+
+
+def _residual_form(groups, to_pairs):
+    """12-byte residual groups on the device turned to pair form, or back to packed fields, where they are."""
+    import torch
+    lib = _native.hip()
+    with torch.cuda.device(groups.device):
+        status = lib.grf_pair_residuals(groups.data_ptr(), groups.numel(), int(to_pairs),
+                                        torch.cuda.current_stream(groups.device).cuda_stream)
+    if status:
+        raise base.CodecError(f"device launch failed ({status}): " + lib.grf_last_error().decode(errors="replace"))
+    return groups
+
+
 class HipContextTensor:
     """A BCTX-coded BF16 matrix resident on one MI355X."""
 
@@ -372,7 +394,7 @@ class HipContextTensor:
         self.device = torch.device(device)
         self._index = device_index(self.device)
         self._error_open = True  # the error word may hold what an unchecked launch reported
-        self.buffers = {}
+        self.buffers = _Buffers()
         self.fused = None
         self.fused_reason = prepared["reason"]
         self._main_bytes = prepared["main_bytes"]
@@ -385,6 +407,9 @@ class HipContextTensor:
                 cum = _tables.cumulative(indexed[name + "_freq"])
                 self.buffers[name + "_cum"] = torch.from_numpy(cum).to(self.device)
                 self.buffers[name + "_bucket"] = torch.from_numpy(_tables.coarse_buckets(cum)).to(self.device)
+        if self._raw6_segment and GEMV_WAVES:  # (the slab kernels' read-ahead is for packed fields)
+            self.buffers["residual_pairs"] = _residual_form(self.buffers.pop("residual_stream"), True)
+            torch.cuda.current_stream(self.device).synchronize()  # (a first product may be on another stream)
         self.error = torch.zeros((), device=self.device, dtype=torch.int32)
         self.resident_bytes = int(sum(t.numel() * t.element_size() for t in self.buffers.values())
                                   + self.error.numel() * self.error.element_size())
@@ -396,15 +421,18 @@ class HipContextTensor:
         the kernels take), and the first tilings."""
         plan = self._plan
         self._frame = None
+        # (an array of packed fields that a caller put in the pairs' place goes first)
+        raw = "residual_pairs" if "residual_pairs" in self.buffers and "residual_stream" not in self.buffers else "residual_stream"
+        form = _hip_abi.RAW_PAIRS if raw == "residual_pairs" else 0
         if self.mode != 1:
             f = _hip_abi.GrfBctxFrame()
-            f.main = _device_stream(self.buffers, "main", 1024, self.nr * self.nc)
-            f.residual = _device_stream(self.buffers, "residual", 64, 1024)
+            f.main = _device_stream(self.buffers, "main", "main_stream", 1024, self.nr * self.nc)
+            f.residual = _device_stream(self.buffers, "residual", raw, 64, 1024)
             f.row_class = self.buffers["rows"].data_ptr()
             f.col_class = self.buffers["columns"].data_ptr()
             f.rows, f.cols = self.shape
             f.nc, f.mode, f.stride = self.nc, self.resident_mode, self.stride
-            f.raw6_segment, f.raw6_block_rows = self._raw6_segment, self._raw6_block
+            f.raw6_segment, f.raw6_block_rows = self._raw6_segment, self._raw6_block | form
             f.raw6_row_pos = self.buffers["row_pos"].data_ptr() if self._raw6_segment else None
             f.main.n_bytes = self._main_bytes
             self._frame = f
@@ -414,7 +442,7 @@ class HipContextTensor:
         if plan is not None:
             d = _hip_abi.GrfBctxFused()
             b = self.buffers
-            d.main_bytes, d.raw6 = b["main_stream"].data_ptr(), b["residual_stream"].data_ptr()
+            d.main_bytes, d.raw6 = b["main_stream"].data_ptr(), b[raw].data_ptr()
             d.seg_state, d.seg_offset = b["fused_seg_state"].data_ptr(), b["fused_seg_offset"].data_ptr()
             d.lut, d.tab, d.col_class = b["fused_lut"].data_ptr(), b["fused_tab"].data_ptr(), b["columns"].data_ptr()
             d.main_n_bytes = self._main_bytes
@@ -422,6 +450,7 @@ class HipContextTensor:
             d.row_pos = b["row_pos"].data_ptr() if self._raw6_segment else None
             for key, value in plan.scalars().items():
                 setattr(d, key, value)
+            d.nc |= form
             self.fused = d
             self.fused_plan = plan.scalars()
             self.fused_reason = ""
@@ -449,16 +478,17 @@ class HipContextTensor:
         import copy
         import torch
         other = copy.copy(self)
-        other.buffers = {k: v.clone() for k, v in self.buffers.items()}
+        other.buffers = _Buffers((k, v.clone()) for k, v in self.buffers.items())
         if residual_block is not None and self._raw6_segment and residual_block != self._raw6_block:
             if residual_block not in (1, 2, 4, 8, 16):
                 raise ValueError("residual blocks have 1, 2, 4, 8 or 16 rows")
             old, groups, spr = self._raw6_block, self._raw6_segment // 16, self.shape[1] // self._raw6_segment
-            raw = other.buffers["residual_stream"]
+            kept = "residual_stream" if "residual_stream" in other.buffers else "residual_pairs"
+            raw = other.buffers[kept]
             held = raw.numel() // (groups * spr * 12)  # a multiple of 16: every class starts on one
             by_row = raw[:held * groups * spr * 12].view(held // old, groups, spr, old, 12).permute(0, 3, 1, 2, 4)
             by_row = by_row.reshape(held // residual_block, residual_block, groups, spr, 12)
-            other.buffers["residual_stream"] = by_row.permute(0, 2, 3, 1, 4).contiguous().view(-1)
+            other.buffers[kept] = by_row.permute(0, 2, 3, 1, 4).contiguous().view(-1)
             for name in ("fused_seg_state", "fused_seg_offset"):  # the index is in the same blocked order
                 kind = other.buffers[name].dtype
                 index = other.buffers[name].view(torch.int32).view(held // old, spr + 1, old).permute(0, 2, 1)

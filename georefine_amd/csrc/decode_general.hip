@@ -7,8 +7,7 @@
 #include <mutex>
 #include <string>
 
-#include "georefine_amd.h"
-#include "rans_device.h"
+#include "fused_device.h"
 
 namespace grf {
 thread_local std::string g_error;
@@ -36,9 +35,51 @@ __device__ __forceinline__ uint64_t raw6_index(const grf_bctx_frame &f, uint32_t
   return group * 16 + col % 16;
 }
 
+// The residual of an element whose group is kept in pair form: its half of the pair's bits.
+__device__ __forceinline__ uint32_t paired_residual(const uint8_t *bytes, uint64_t index) {
+  const uint32_t *from = reinterpret_cast<const uint32_t *>(bytes + index / 16 * 12);
+  const uint32_t d[3] = {from[0], from[1], from[2]}, k = (uint32_t)(index % 16);
+  uint32_t pair = 0;
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+    if (k / 2 == (uint32_t)i) pair = grf::residual_pair(d, i);
+  const uint32_t word = k % 2 ? pair >> 16 : pair;
+  return (word & 31u) | (word >> 15 & 1u) << 5;
+}
+
+// Groups of sixteen packed 6-bit fields to pair form, or back, each where it is: one thread a group.
+__global__ __launch_bounds__(kThreads) void pair_residuals_kernel(uint32_t *groups, uint64_t count, bool to_pairs) {
+  const uint64_t g = (uint64_t)blockIdx.x * kThreads + threadIdx.x;
+  if (g >= count) return;
+  uint32_t *own = groups + g * 3;
+  const uint32_t in[3] = {own[0], own[1], own[2]};
+  uint32_t pair[8], out[3];
+  if (to_pairs) {
+    grf::Raw6x16 packed;
+    packed.set(in[0], in[1], in[2]);
+    auto words = [&](auto i) { pair[decltype(i)::value] = packed.words<decltype(i)::value>(0, 0) & grf::kPairBits; };
+    words(std::integral_constant<int, 0>{}), words(std::integral_constant<int, 1>{}), words(std::integral_constant<int, 2>{});
+    words(std::integral_constant<int, 3>{}), words(std::integral_constant<int, 4>{}), words(std::integral_constant<int, 5>{});
+    words(std::integral_constant<int, 6>{}), words(std::integral_constant<int, 7>{});
+    grf::residual_group(pair, out);
+  } else {
+    uint32_t w[3] = {0, 0, 0};  // big-endian dwords
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+      const uint32_t word = grf::residual_pair(in, k / 2) >> (k % 2 * 16), field = (word & 31u) | (word >> 15 & 1u) << 5;
+      const int bit = 6 * k, at = bit / 32, past = bit % 32 + 6;
+      w[at] |= past <= 32 ? field << (32 - past) : field >> (past - 32);
+      if (past > 32) w[at + 1] |= field << (64 - past);
+    }
+#pragma unroll
+    for (int k = 0; k < 3; ++k) out[k] = __builtin_bswap32(w[k]);
+  }
+  own[0] = out[0], own[1] = out[1], own[2] = out[2];
+}
+
 template <bool MODE128>
 __global__ __launch_bounds__(kThreads) void bctx_decode_kernel(grf_bctx_frame f, const int64_t *block_ids,
-                                                                uint32_t count, uint16_t *out, int32_t *error) {
+                                                                uint32_t count, bool pairs, uint16_t *out, int32_t *error) {
   const uint32_t lane = blockIdx.x * kThreads + threadIdx.x;
   if (lane >= count) return;
   const uint64_t n = (uint64_t)f.rows * f.cols;
@@ -67,6 +108,8 @@ __global__ __launch_bounds__(kThreads) void bctx_decode_kernel(grf_bctx_frame f,
     if (MODE128)
       r = grf::rans_step_global(rstate, rip, f.residual.bytes, f.residual.n_bytes,
                                 f.residual.cum + (size_t)m * 65, f.residual.bucket + (size_t)m * 256, bad);
+    else if (pairs)
+      r = paired_residual(f.residual.bytes, raw6_index(f, row, col));
     else
       r = grf::packed_field<6>(f.residual.bytes, f.residual.n_bytes, raw6_index(f, row, col));
     dst[t] = (uint16_t)grf::bctx_word(m, r);
@@ -224,7 +267,9 @@ int grf_timestamp(uint64_t *slot, void *hip_stream) {
 int grf_bctx_decode(const grf_bctx_frame *frame, const int64_t *block_ids, uint32_t count, uint16_t *out,
                     int32_t *error, void *hip_stream) {
   if (!frame || !out || !error) return fail(GRF_BAD_ARGUMENT, "grf_bctx_decode: null argument");
-  const grf_bctx_frame &f = *frame;
+  grf_bctx_frame f = *frame;
+  const bool pairs = f.raw6_segment && f.raw6_block_rows & GRF_RAW_PAIRS;
+  if (pairs) f.raw6_block_rows &= ~GRF_RAW_PAIRS;
   if (!f.rows || !f.cols || !f.stride || f.stride > 65536 || !f.nc || f.nc > 16 || !f.row_class || !f.col_class)
     return fail(GRF_BAD_ARGUMENT, "grf_bctx_decode: bad geometry");
   if (f.mode != 0 && f.mode != 128) return fail(GRF_UNSUPPORTED, "grf_bctx_decode: mode must be 0 or 128");
@@ -238,16 +283,29 @@ int grf_bctx_decode(const grf_bctx_frame *frame, const int64_t *block_ids, uint3
       (f.raw6_segment % 16 || f.cols % f.raw6_segment || f.raw6_block_rows > 16 ||
        (f.raw6_block_rows & (f.raw6_block_rows - 1))))
     return fail(GRF_BAD_ARGUMENT, "grf_bctx_decode: residual order (segment length, block rows)");
+  if (pairs && (f.mode != 0 || (uintptr_t)f.residual.bytes & 3))
+    return fail(GRF_BAD_ARGUMENT, "grf_bctx_decode: residuals in pair form are mode 0's, from a multiple of 4 bytes on");
   const uint64_t segments = (n + f.stride - 1) / f.stride;
   if (!count) return GRF_OK;
   if (!block_ids && count > segments) return fail(GRF_BAD_ARGUMENT, "grf_bctx_decode: count exceeds segments");
   const dim3 grid((count + kThreads - 1) / kThreads), block(kThreads);
   hipStream_t s = (hipStream_t)hip_stream;
   if (f.mode == 128)
-    hipLaunchKernelGGL(bctx_decode_kernel<true>, grid, block, 0, s, f, block_ids, count, out, error);
+    hipLaunchKernelGGL(bctx_decode_kernel<true>, grid, block, 0, s, f, block_ids, count, pairs, out, error);
   else
-    hipLaunchKernelGGL(bctx_decode_kernel<false>, grid, block, 0, s, f, block_ids, count, out, error);
+    hipLaunchKernelGGL(bctx_decode_kernel<false>, grid, block, 0, s, f, block_ids, count, pairs, out, error);
   return launch_status("grf_bctx_decode");
+}
+
+int grf_pair_residuals(void *groups, uint64_t bytes, int to_pairs, void *hip_stream) {
+  if (!groups || (uintptr_t)groups & 3 || bytes % 12)
+    return fail(GRF_BAD_ARGUMENT, "grf_pair_residuals: whole groups of 12 bytes from a multiple of 4 on");
+  const uint64_t count = bytes / 12;
+  if (!count) return GRF_OK;
+  if (count > 0xFFFFFFFFull) return fail(GRF_BAD_ARGUMENT, "grf_pair_residuals: too many groups");
+  hipLaunchKernelGGL(pair_residuals_kernel, dim3((unsigned)((count + kThreads - 1) / kThreads)), dim3(kThreads), 0,
+                     (hipStream_t)hip_stream, static_cast<uint32_t *>(groups), count, to_pairs != 0);
+  return launch_status("grf_pair_residuals");
 }
 
 int grf_ppcx_decode(const grf_ppcx_frame *frame, const uint16_t *reference, uint16_t *out, int32_t *error,

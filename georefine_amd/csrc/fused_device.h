@@ -33,6 +33,7 @@
 
 #include "georefine_amd.h"
 #include "piece_units.h"
+#include "residual_pairs.h"
 #include "rans_device.h"
 
 namespace grf {
@@ -237,6 +238,8 @@ __device__ __forceinline__ void fused_scan_whole(uint32_t state, StepFetch &s, u
   s.e0 = e;
 }
 
+// (One asm for the product and the count; no early clobber: every input is read by the first of the two, and the
+// product can then go straight to the upper half of the pair that is shifted, one move a symbol less.)
 // state' = freq * (state >> 16) + rel, then the refill: n = 0, 1 or 2 bytes are shifted in
 // while the state is below 2^23.  Without branches or condition registers: the state is
 // below 2^31 and at least 2^7, so 8 n = (clz(state') - 1) & 24, and one 64-bit shift of
@@ -246,7 +249,7 @@ __device__ __forceinline__ void fused_advance(Cursor &c, StepFetch &s, uint32_t 
 #if defined(__HIP_DEVICE_COMPILE__)
   asm("v_mad_u32_u16 %0, %2, %3, %4 op_sel:[1,1,0,0]\n\t"
       "v_ffbh_u32 %1, %0"
-      : "=&v"(x), "=v"(lead)
+      : "=v"(x), "=v"(lead)
       : "v"(s.e0.x), "v"(c.state), "v"(rel));
 #else
   x = (s.e0.x >> 16) * (c.state >> 16) + rel;
@@ -299,6 +302,13 @@ __device__ __forceinline__ void fused_symbol_pair(Cursor &c, uint32_t ccw, const
                        q, hi0, hi1);
 }
 
+// BF16 word in bits 0..15 (bits above are unspecified): symbol bits | mantissa low 5 bits
+// | sign << 15, from the sign-extended residual field: its copy of the sign at bit 15 and
+// its low five bits are kept, one and-or.
+__device__ __forceinline__ uint32_t fused_word_bits(uint32_t hi, uint32_t r6_sign_extended) {
+  return (r6_sign_extended & 0x801Fu) | hi;
+}
+
 // Sixteen packed 6-bit residuals (12 bytes, MSB first) -> field k, k compile-time, sign
 // extended: bits 0..4 are the mantissa's low bits, every bit from 5 up copies the sign.
 struct Raw6x16 {
@@ -319,6 +329,25 @@ struct Raw6x16 {
       const uint32_t b = word == 0 ? w1 : w2;
       return (uint32_t)__builtin_amdgcn_sbfe((int32_t)__builtin_amdgcn_alignbit(a, b, 64 - 6 - off), 0, 6);
     }
+  }
+  // the words 2 I and 2 I + 1 of the group, from the symbols' bits
+  template <int I>
+  __device__ __forceinline__ uint32_t words(uint32_t hi0, uint32_t hi1) const {
+    return __builtin_amdgcn_perm(fused_word_bits(hi1, field<2 * I + 1>()), fused_word_bits(hi0, field<2 * I>()), 0x05040100u);
+  }
+};
+
+// The same sixteen residuals in pair form (GRF_RAW_PAIRS, residual_pairs.h): a pair's twelve bits lie as they do
+// in the pair of BF16 words, turned by a constant, so that one rotation and one and-or serve two words.  Against the fields
+// one by one 1.6 instructions a symbol with the merge, so 2.8 (the whole step 15.5, so 16.6): 17408 and 17408 x 5120 at one
+// row 113.8 -> 110.1 us, at 64 rows 155.1 -> 150.6, 5120 x 17408 at six rows 70.1 -> 68.5, 6144 + 1024 + 1024 x 5120
+// at 32 rows 39.3 -> 38.2 (with the move that fused_advance no longer makes, about a third of it).
+struct Raw6Pairs {
+  uint32_t d[3];
+  __device__ __forceinline__ void set(uint32_t a, uint32_t b, uint32_t c) { d[0] = a, d[1] = b, d[2] = c; }
+  template <int I>
+  __device__ __forceinline__ uint32_t words(uint32_t hi0, uint32_t hi1) const {
+    return (residual_pair(d, I) & kPairBits) | __builtin_amdgcn_perm(hi1, hi0, 0x05040100u);
   }
 };
 
@@ -536,13 +565,6 @@ __device__ __forceinline__ uint32_t fused_stage_rows_dma(uint8_t *lds, uint32_t 
   return a0;
 }
 
-// BF16 word in bits 0..15 (bits above are unspecified): symbol bits | mantissa low 5 bits
-// | sign << 15, from the sign-extended residual field: its copy of the sign at bit 15 and
-// its low five bits are kept, one and-or.
-__device__ __forceinline__ uint32_t fused_word_bits(uint32_t hi, uint32_t r6_sign_extended) {
-  return (r6_sign_extended & 0x801Fu) | hi;
-}
-
 // Two finished words as a pair, in a register of its own at once: left alone, the compiler puts the
 // merge of symbols and residuals off to the end of the eight steps, and what they are merged from
 // takes three times the registers meanwhile (GEMV of two rows 80 registers and 11 spilled -> 70; store
@@ -550,8 +572,7 @@ __device__ __forceinline__ uint32_t fused_word_bits(uint32_t hi, uint32_t r6_sig
 // spilled -> 54, 63 and 79).  KEEP false: it may; a kernel that has the registers (GEMV of one row) then
 // waits for its residuals eight steps later, 1 % of the smallest launches.
 template <bool KEEP>
-__device__ __forceinline__ uint32_t fused_word_pair(uint32_t first, uint32_t second) {
-  uint32_t pair = __builtin_amdgcn_perm(second, first, 0x05040100u);
+__device__ __forceinline__ uint32_t fused_word_pair(uint32_t pair) {
 #if defined(__HIP_DEVICE_COMPILE__)
   if constexpr (KEEP) asm volatile("" : "+v"(pair));
 #endif
@@ -562,8 +583,8 @@ __device__ __forceinline__ uint32_t fused_word_pair(uint32_t first, uint32_t sec
 // residuals and the column classes of the next 16 symbols.  AHEAD (segments of 64 symbols
 // only): the residuals of the whole segment, 48 bytes, are read when the segment starts; a
 // line of the residual section is then fetched once instead of on four visits a group
-// apart, between which the L2 may have dropped it.
-template <bool AHEAD>
+// apart, between which the L2 may have dropped it.  PAIRS: the residual groups are in pair form.
+template <bool AHEAD, bool PAIRS = false>
 struct SegmentWalkT {
   static constexpr bool kAhead = AHEAD;
   Cursor c;
@@ -575,7 +596,7 @@ struct SegmentWalkT {
   uint32_t n0, n1, n2;             // !AHEAD: the next group's residual words
   uint32_t rw[AHEAD ? 12 : 1];     // AHEAD: the segment's residual words
   uint4 nc4;
-  Raw6x16 rr;      // the group being decoded
+  std::conditional_t<PAIRS, Raw6Pairs, Raw6x16> rr;  // the group being decoded
   uint32_t cw[4];
 
   // Global reads for the segment whose checkpoint is entry `slot_` of the index arrays
@@ -654,14 +675,11 @@ struct SegmentWalkT {
   // half, k+1 in the high half).
   template <int H, int SCAN = kScanAny, bool KEEP = true>
   __device__ __forceinline__ void half(const FusedParams &q, uint32_t (&pair)[4]) {
-    uint32_t bits[8];
-#define GRF_STEP2(i)                                                                   \
-  {                                                                                    \
-    uint32_t h0, h1;                                                                   \
-    fused_symbol_pair<8 * H + (i), SCAN>(c, cw[(8 * H + (i)) / 4], q, h0, h1);         \
-    bits[i] = fused_word_bits(h0, rr.field<8 * H + (i)>());                            \
-    bits[(i) + 1] = fused_word_bits(h1, rr.field<8 * H + (i) + 1>());                  \
-    pair[(i) / 2] = fused_word_pair<KEEP>(bits[i], bits[(i) + 1]);                     \
+#define GRF_STEP2(i)                                                                         \
+  {                                                                                          \
+    uint32_t h0, h1;                                                                         \
+    fused_symbol_pair<8 * H + (i), SCAN>(c, cw[(8 * H + (i)) / 4], q, h0, h1);               \
+    pair[(i) / 2] = fused_word_pair<KEEP>(rr.template words<4 * H + (i) / 2>(h0, h1));       \
   }
     GRF_STEP2(0) GRF_STEP2(2) GRF_STEP2(4) GRF_STEP2(6)
 #undef GRF_STEP2
@@ -681,5 +699,6 @@ struct SegmentWalkT {
 };
 using SegmentWalk = SegmentWalkT<false>;
 using SegmentWalkAhead = SegmentWalkT<true>;
+using SegmentWalkPairs = SegmentWalkT<false, true>;
 
 }  // namespace grf

@@ -31,13 +31,32 @@ int scratch_address(void **out) {
   return GRF_OK;
 }
 
+// The members of a grouped launch in the walk's own structure, all of one residual form.
+struct ContextMembers {
+  grf_bctx_fused frames[grf::kMaxGroup];
+  const grf_bctx_fused *pointers[grf::kMaxGroup];
+  bool pairs = false;
+  int fill(const char *who, uint32_t n, const grf_bctx_fused *const *members) {
+    if (n < 1 || n > grf::kMaxGroup || !members) return GRF_OK;  // (refused by the launcher, as any launch's)
+    for (uint32_t i = 0; i < n; ++i) {
+      pointers[i] = nullptr;
+      if (!members[i]) continue;
+      const grf::ContextFrame f(*members[i]);
+      if (i && members[0] && f.pairs != pairs)
+        return grf::set_error(GRF_BAD_ARGUMENT, std::string(who) + ": members must keep their residuals in one form");
+      frames[i] = f, pointers[i] = &frames[i], pairs = f.pairs;
+    }
+    return GRF_OK;
+  }
+};
+
 }  // namespace
 
 extern "C" {
 
 uint32_t grf_bctx_gemm_lds_bytes(const grf_bctx_fused *frame, const grf_fused_tiling *tiling) {
   if (!frame || !tiling) return 0;
-  return grf::gemm_lds_bytes(*frame, *tiling);
+  return grf::gemm_lds_bytes(grf::ContextFrame(*frame), *tiling);
 }
 
 size_t grf_gemm_workspace_bytes(uint32_t cols, uint32_t m_rows) { return grf::gemm_workspace_bytes(cols, m_rows); }
@@ -56,9 +75,12 @@ int grf_bctx_gemm(const grf_bctx_fused *frame, const grf_fused_tiling *tiling, c
                   size_t workspace_bytes, int32_t *error, void *hip_stream) {
   if (!frame || !tiling || !y || !error)  // x may be null: rows packed by grf_pack_activations
     return grf::set_error(GRF_BAD_ARGUMENT, "grf_bctx_gemm: null argument");
-  if (int rc = grf::check_fused_frame(*frame, *tiling, "grf_bctx_gemm", grf::kGemmTiling)) return rc;
-  return grf::launch_gemm<grf::SegmentWalk>("grf_bctx_gemm", *frame, *tiling, x, ldx, m_rows, y, ldy, bias, workspace,
-                                            workspace_bytes, error, (hipStream_t)hip_stream);
+  const grf::ContextFrame f(*frame);
+  if (int rc = grf::check_fused_frame(f, *tiling, "grf_bctx_gemm", grf::kGemmTiling)) return rc;
+  return grf::with_walk(f.pairs, [&](auto walk) {
+    return grf::launch_gemm<typename decltype(walk)::type>("grf_bctx_gemm", f, *tiling, x, ldx, m_rows, y, ldy, bias, workspace,
+                                                           workspace_bytes, error, (hipStream_t)hip_stream);
+  });
 }
 
 size_t grf_gemm_noalloc_limit_bytes(void) { return kScratchBytes; }
@@ -73,22 +95,29 @@ int grf_bctx_gemm_noalloc(const grf_bctx_fused *frame, const grf_fused_tiling *t
                           "grf_bctx_gemm_noalloc: the packed activations (and partial sums) of one launch exceed the "
                           "8 MiB scratch (grf_gemm_workspace_bytes_split(cols, rows, k_parts, m_rows) > "
                           "grf_gemm_noalloc_limit_bytes()); use grf_bctx_gemm with a workspace");
-  if (int rc = grf::check_fused_frame(*frame, *tiling, "grf_bctx_gemm_noalloc", grf::kGemmTiling)) return rc;
+  const grf::ContextFrame f(*frame);
+  if (int rc = grf::check_fused_frame(f, *tiling, "grf_bctx_gemm_noalloc", grf::kGemmTiling)) return rc;
   void *ptr = nullptr;
   if (int rc = scratch_address(&ptr)) return rc;
   // every launch writes all it reads of the scratch (its rows, zero rows up to the tile, the
   // chunk of zeros after the last column), so nothing of an earlier call shows through
-  return grf::launch_gemm<grf::SegmentWalk>("grf_bctx_gemm_noalloc", *frame, *tiling, x, ldx, m_rows, y, ldy, bias, ptr,
-                                            kScratchBytes, error, (hipStream_t)hip_stream);
+  return grf::with_walk(f.pairs, [&](auto walk) {
+    return grf::launch_gemm<typename decltype(walk)::type>("grf_bctx_gemm_noalloc", f, *tiling, x, ldx, m_rows, y, ldy, bias, ptr,
+                                                           kScratchBytes, error, (hipStream_t)hip_stream);
+  });
 }
 
 int grf_bctx_gemv_group(uint32_t n, const grf_bctx_fused *const *frames, const grf_fused_tiling *const *tilings,
                         const uint16_t *x, uint32_t ldx, uint32_t m_rows, uint16_t *const *y, const uint32_t *ldy,
                         const uint16_t *const *bias, int32_t *error, void *hip_stream) {
   if (!error) return grf::set_error(GRF_BAD_ARGUMENT, "grf_bctx_gemv_group: null argument");
-  const grf::GroupSpec spec{n, frames, tilings, y, ldy, bias};
-  return grf::launch_gemv_group<grf::SegmentWalk>("grf_bctx_gemv_group", spec, x, ldx, m_rows, error,
-                                                  (hipStream_t)hip_stream);
+  ContextMembers members;
+  if (int rc = members.fill("grf_bctx_gemv_group", n, frames)) return rc;
+  const grf::GroupSpec spec{n, frames ? members.pointers : nullptr, tilings, y, ldy, bias};
+  return grf::with_walk(members.pairs, [&](auto walk) {
+    return grf::launch_gemv_group<typename decltype(walk)::type>("grf_bctx_gemv_group", spec, x, ldx, m_rows, error,
+                                                                 (hipStream_t)hip_stream);
+  });
 }
 
 int grf_bctx_gemm_group(uint32_t n, const grf_bctx_fused *const *frames, const grf_fused_tiling *const *tilings,
@@ -96,9 +125,14 @@ int grf_bctx_gemm_group(uint32_t n, const grf_bctx_fused *const *frames, const g
                         const uint16_t *const *bias, void *workspace, size_t workspace_bytes, int32_t *error,
                         void *hip_stream) {
   if (!error) return grf::set_error(GRF_BAD_ARGUMENT, "grf_bctx_gemm_group: null argument");
-  const grf::GroupSpec spec{n, frames, tilings, y, ldy, bias};
-  return grf::launch_gemm_group<grf::SegmentWalk>("grf_bctx_gemm_group", spec, x, ldx, m_rows, workspace,
-                                                  workspace_bytes, error, (hipStream_t)hip_stream);
+  ContextMembers members;
+  if (int rc = members.fill("grf_bctx_gemm_group", n, frames)) return rc;
+  const grf::GroupSpec spec{n, frames ? members.pointers : nullptr, tilings, y, ldy, bias};
+  return grf::with_walk(members.pairs, [&](auto walk) {
+    return grf::launch_gemm_group<typename decltype(walk)::type>("grf_bctx_gemm_group", spec, x, ldx, m_rows, workspace,
+                                                                 workspace_bytes, error,
+                                                                 (hipStream_t)hip_stream);
+  });
 }
 
 }  // extern "C"

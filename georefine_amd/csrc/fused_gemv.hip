@@ -153,9 +153,10 @@ extern "C" {
 
 uint32_t grf_bctx_fused_lds_bytes(const grf_bctx_fused *frame, const grf_fused_tiling *tiling, uint32_t m_rows) {
   if (!frame || !tiling) return 0;
+  const grf::ContextFrame f(*frame);
   if (grf::tile_scheme(*tiling) == GRF_TILE_WAVES)  // passes of at most two activation rows
-    return grf::WaveLdsLayout(*frame, *tiling, m_rows < grf::kWaveRowsPerPass ? m_rows : grf::kWaveRowsPerPass).total;
-  return grf::FusedLdsLayout(*frame, *tiling, m_rows).total;
+    return grf::WaveLdsLayout(f, *tiling, m_rows < grf::kWaveRowsPerPass ? m_rows : grf::kWaveRowsPerPass).total;
+  return grf::FusedLdsLayout(f, *tiling, m_rows).total;
 }
 
 int grf_bctx_fused_validate_host(const grf_bctx_fused *frame, const grf_fused_tiling *tiling, int use,
@@ -168,7 +169,7 @@ int grf_bctx_fused_validate_host(const grf_bctx_fused *frame, const grf_fused_ti
                                 : use == 1 ? grf::kGemvTiling
                                 : use == 2 ? grf::kGemmTiling
                                            : grf::kSlabTiling;
-    return grf::validate_fused_host(*frame, *tiling, kind, use != 3, seg_offset, tile_rows, tile_class, row_class,
+    return grf::validate_fused_host(grf::ContextFrame(*frame), *tiling, kind, use != 3, seg_offset, tile_rows, tile_class, row_class,
                                     row_pos);
   } catch (...) {
     return grf::set_error(GRF_BAD_ARGUMENT, "grf_bctx_fused_validate_host: out of memory");
@@ -180,32 +181,41 @@ int grf_bctx_gemv(const grf_bctx_fused *frame, const grf_fused_tiling *tiling, c
                   void *hip_stream) {
   if (!frame || !tiling || !x || !y || !error)
     return grf::set_error(GRF_BAD_ARGUMENT, "grf_bctx_gemv: null argument");
-  if (int rc = grf::check_fused_frame(*frame, *tiling, "grf_bctx_gemv", grf::kGemvTiling)) return rc;
-  return grf::launch_gemv<grf::SegmentWalk>("grf_bctx_gemv", *frame, *tiling, x, ldx, m_rows, y, ldy, bias, error,
-                                            (hipStream_t)hip_stream);
+  const grf::ContextFrame f(*frame);
+  if (int rc = grf::check_fused_frame(f, *tiling, "grf_bctx_gemv", grf::kGemvTiling)) return rc;
+  return grf::with_walk(f.pairs, [&](auto walk) {
+    return grf::launch_gemv<typename decltype(walk)::type>("grf_bctx_gemv", f, *tiling, x, ldx, m_rows, y, ldy, bias, error,
+                                                           (hipStream_t)hip_stream);
+  });
 }
 
 int grf_bctx_fused_decode(const grf_bctx_fused *frame, const grf_fused_tiling *tiling, uint16_t *out,
                           int32_t *error, void *hip_stream) {
   if (!frame || !tiling || !out || !error)
     return grf::set_error(GRF_BAD_ARGUMENT, "grf_bctx_fused_decode: null argument");
-  if (int rc = grf::check_fused_frame(*frame, *tiling, "grf_bctx_fused_decode", grf::kStoreTiling)) return rc;
-  if (grf::tile_scheme(*tiling) == GRF_TILE_WAVES)
-    return grf::launch_wave_store<grf::SegmentWalk>(*frame, *tiling, out, error, (hipStream_t)hip_stream);
-  if (grf::reads_ahead(*frame))
-    return grf::launch_walk<grf::SegmentWalkAhead, 1, grf::kStore>(*frame, *tiling, nullptr, 0, nullptr, 0, nullptr,
-                                                                   out, error, (hipStream_t)hip_stream);
-  return grf::launch_walk<grf::SegmentWalk, 1, grf::kStore>(*frame, *tiling, nullptr, 0, nullptr, 0, nullptr, out, error,
-                                                            (hipStream_t)hip_stream);
+  const grf::ContextFrame f(*frame);
+  if (int rc = grf::check_fused_frame(f, *tiling, "grf_bctx_fused_decode", grf::kStoreTiling)) return rc;
+  return grf::with_walk(f.pairs, [&](auto walk) {
+    using Walk = typename decltype(walk)::type;
+    using Ahead = typename grf::ahead_of<Walk>::type;
+    hipStream_t s = (hipStream_t)hip_stream;
+    if (grf::tile_scheme(*tiling) == GRF_TILE_WAVES) return grf::launch_wave_store<Walk>(f, *tiling, out, error, s);
+    if (grf::reads_ahead(f))
+      return grf::launch_walk<Ahead, 1, grf::kStore>(f, *tiling, nullptr, 0, nullptr, 0, nullptr, out, error, s);
+    return grf::launch_walk<Walk, 1, grf::kStore>(f, *tiling, nullptr, 0, nullptr, 0, nullptr, out, error, s);
+  });
 }
 
 int grf_bctx_fused_gather(const grf_bctx_fused *frame, const grf_fused_tiling *tiling, uint16_t *out,
                           int32_t *error, void *hip_stream) {
   if (!frame || !tiling || !out || !error)
     return grf::set_error(GRF_BAD_ARGUMENT, "grf_bctx_fused_gather: null argument");
-  if (int rc = grf::check_fused_frame(*frame, *tiling, "grf_bctx_fused_gather")) return rc;
-  return grf::launch_walk<grf::SegmentWalk, 1, grf::kGather>(*frame, *tiling, nullptr, 0, nullptr, 0, nullptr, out,
-                                                             error, (hipStream_t)hip_stream);
+  const grf::ContextFrame f(*frame);
+  if (int rc = grf::check_fused_frame(f, *tiling, "grf_bctx_fused_gather")) return rc;
+  return grf::with_walk(f.pairs, [&](auto walk) {
+    return grf::launch_walk<typename decltype(walk)::type, 1, grf::kGather>(f, *tiling, nullptr, 0, nullptr, 0, nullptr, out,
+                                                                            error, (hipStream_t)hip_stream);
+  });
 }
 
 int grf_bctx_gather_rows(const grf_bctx_fused *frame, uint32_t lanes, uint32_t piece_cap, const uint8_t *row_class,
@@ -220,9 +230,12 @@ int grf_bctx_gather_rows(const grf_bctx_fused *frame, uint32_t lanes, uint32_t p
   one.rows_per_tile = one.n_tiles = 1;
   one.n_slabs = (frame->segs_per_row + 63) / 64;
   one.piece_cap = piece_cap;
-  if (int rc = grf::check_fused_frame(*frame, one, "grf_bctx_gather_rows")) return rc;
-  return grf::launch_gather<grf::SegmentWalk>("grf_bctx_gather_rows", *frame, lanes, piece_cap, row_class, ids, count, out,
-                                              error, index_error, (hipStream_t)hip_stream);
+  const grf::ContextFrame f(*frame);
+  if (int rc = grf::check_fused_frame(f, one, "grf_bctx_gather_rows")) return rc;
+  return grf::with_walk(f.pairs, [&](auto walk) {
+    return grf::launch_gather<typename decltype(walk)::type>("grf_bctx_gather_rows", f, lanes, piece_cap, row_class, ids, count,
+                                                             out, error, index_error, (hipStream_t)hip_stream);
+  });
 }
 
 }  // extern "C"

@@ -45,6 +45,20 @@ enum TilingUse { kSlabTiling, kGemvTiling, kGemmTiling, kStoreTiling };
 int check_fused_frame(const grf_bctx_fused &f, const grf_fused_tiling &g, const char *who, TilingUse use = kSlabTiling,
                       bool pointers = true);
 
+// A context frame as an entry point is given it: the walk's own structure, and the form of its residuals
+// (GRF_RAW_PAIRS, which is in the class count for it had no other bits in use).
+struct ContextFrame : grf_bctx_fused {
+  bool pairs;
+  explicit ContextFrame(const grf_bctx_fused &f) : grf_bctx_fused(f), pairs(f.nc & GRF_RAW_PAIRS) { nc &= ~GRF_RAW_PAIRS; }
+};
+template <class Walk>
+struct WalkOf { using type = Walk; };
+// fn(WalkOf<the walker of the frame's residual form>)
+template <class Fn>
+int with_walk(bool pairs, const Fn &fn) {
+  return pairs ? fn(WalkOf<grf::SegmentWalkPairs>{}) : fn(WalkOf<grf::SegmentWalk>{});
+}
+
 // A kernel may ask for more than 64 KiB of dynamic LDS only after its limit has been raised;
 // done once per kernel and device (not per launch: it is a driver call, and a launch that
 // is being captured into a graph should consist of the launch alone).

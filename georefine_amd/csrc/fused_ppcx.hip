@@ -198,7 +198,7 @@ struct PpcxWalk {
                                     grf::fused_block_offset<(i) / 2>(odd, q.block_pitch), q, h0, h1); \
     bits[i] = h0 | rr.field<8 * H + (i)>();                                                           \
     bits[(i) + 1] = h1 | rr.field<8 * H + (i) + 1>();                                                 \
-    pair[(i) / 2] = grf::fused_word_pair<KEEP>(bits[i], bits[(i) + 1]);                               \
+    pair[(i) / 2] = grf::fused_word_pair<KEEP>(__builtin_amdgcn_perm(bits[(i) + 1], bits[i], 0x05040100u)); \
   }
     GRF_STEP2(0) GRF_STEP2(2) GRF_STEP2(4) GRF_STEP2(6)
 #undef GRF_STEP2

@@ -143,13 +143,25 @@ typedef struct grf_stream {
   const uint32_t *offsets;
 } grf_stream;
 
+/* Pair form of packed 6-bit residuals: a group of sixteen keeps its 12 bytes, but three little-endian dwords in
+ * which the bits of two neighbouring residuals lie as in the pair of BF16 words they complete (sign at 15 and 31,
+ * the five low bits at 0 and 16), turned left: with P(i) these twelve bits of residuals 2 i and 2 i + 1 and rol
+ * a rotation of 32 bits, inner = 0x001E001E, outer = 0x80018001:
+ *   dword 0 = P(0) | rol(P(1), 6) | rol(P(6) & inner, 10)
+ *   dword 1 = P(2) | rol(P(3), 6) | rol(P(7) & inner, 10)
+ *   dword 2 = P(4) | rol(P(5), 6) | rol(P(6) & outer, 12) | rol(P(7) & outer, 14)
+ * The fused kernels complete two words with it for the work of one.  It is set in grf_bctx_fused.nc and in
+ * grf_bctx_frame.raw6_block_rows; the members of a grouped launch all have it or none has. */
+#define GRF_RAW_PAIRS 0x100u
+
 /* A BCTX frame as the decode kernels see it (the buffers CudaContextTensor keeps,
  * GCR/bitexact_context_gpu.py:96-125). mode 0: residual.bytes is the packed 6-bit
  * stream and the other residual fields are unused; mode 128: residual is a full stream.
  * raw6_segment (mode 0): 0 when the 6-bit fields are in the frame's own order (element e at
  * bit 6 e); S > 0 when the 12-byte groups of 16 fields are kept in the order the fused
  * kernels read them for segments of S symbols: raw6_block_rows and raw6_row_pos are then
- * grf_bctx_fused.raw_interleaved and grf_bctx_fused.row_pos of the same tensor. */
+ * grf_bctx_fused.raw_interleaved and grf_bctx_fused.row_pos of the same tensor, and
+ * raw6_block_rows | GRF_RAW_PAIRS says that the groups are in pair form. */
 typedef struct grf_bctx_frame {
   grf_stream main;
   grf_stream residual;
@@ -170,6 +182,10 @@ typedef struct grf_bctx_frame {
  * block_ids is NULL.  out holds count*stride words: out[j*stride + t]. */
 int grf_bctx_decode(const grf_bctx_frame *frame, const int64_t *block_ids, uint32_t count, uint16_t *out,
                     int32_t *error, void *hip_stream);
+
+/* Groups of sixteen packed 6-bit residuals (12 bytes each, from a multiple of 4 on) to pair form (to_pairs) or
+ * back, in place. */
+int grf_pair_residuals(void *groups, uint64_t bytes, int to_pairs, void *hip_stream);
 
 /* A PPCX frame (the buffers CudaPredictiveTensor keeps, GCR/bitexact_predictive_gpu.py:116-132).
  * mode 0: residual.bytes is the packed 5-bit stream; mode 1: residual is a full stream. */
@@ -235,6 +251,7 @@ int grf_mix_predict(const uint16_t *up, const uint16_t *gate, const uint16_t *co
  * ceil(max position / B) * B (the array holds that many rows; positions no row has are never
  * read).  The host side orders the rows by row class, as the tilings do, and starts every
  * class on a multiple of 16, so that the rows of a unit are the rows of a block.
+ * nc: the column classes, and GRF_RAW_PAIRS if raw6 is in pair form.
  * whole_range: nonzero if some context is a single symbol of frequency 65536 (entry field 0,
  * the state does not change there); 0 promises there is none, and the scan for lanes whose
  * lookup byte names a neighbour of their symbol then leaves that case out.
