@@ -33,10 +33,13 @@ def _product(x, w, bias):
     return y, size
 
 
-# rows x cols at m rows: each tile (256 x 256, 128 x 128, 128 x 64), cut along K and whole, with rows and columns that do and
-# do not end on a tile, on a step of 64 columns, on four rows; fewer columns than a step, than two; one row and column
+# rows x cols at m rows: each tile (256 x 256, 256 x 192, 256 x 128, 128 x 128, 128 x 64), cut along K and whole, with rows
+# and columns that do and do not end on a tile, on a step of 64 columns, on four rows; fewer columns than a step, than two;
+# one row and column
 SHAPES = [(1, 1, 8), (129, 65, 24), (130, 63, 64), (128, 64, 128), (257, 127, 72), (129, 300, 136), (200, 255, 528), (256, 256, 2048),
-          (257, 770, 16), (300, 4099, 1040), (1000, 2050, 600), (513, 2305, 10304), (1000, 1028, 16448), (160, 5120, 17408)]
+          (257, 770, 16), (300, 4099, 1040), (1000, 2050, 600), (513, 2305, 10304), (1000, 1028, 16448), (160, 5120, 17408),
+          (129, 257, 520), (257, 2049, 1032), (257, 2049, 4104), (129, 4100, 4104), (257, 12290, 1032), (1000, 3001, 4104),
+          (1000, 8193, 520), (129, 12290, 4104), (1000, 12290, 1032)]
 
 
 @pytest.mark.parametrize("m,rows,cols", SHAPES)
