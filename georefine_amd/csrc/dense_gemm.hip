@@ -291,6 +291,9 @@ constexpr DenseTile kTiles[] = {{256, 256, 1, 7.7, 0.0, 1.163, 7.43, 0.0, 0.114}
                                 {128, 64, 2, 5.5, 0.369, 0.685, 1.20, 1.9, 0.160}};
 constexpr uint32_t kTileCount = sizeof(kTiles) / sizeof(kTiles[0]);
 constexpr uint32_t kUnits = 256;  // compute units
+// A product that is cut takes two calls, and the host 3.5 us more: beside a short decode it is never sooner than this
+// (with the decode, 306 x 768 at 156 rows 20.7 us in four parts, 18.3 whole; 490 x 512 at 160, whole, 17.3).
+constexpr double kCutAtLeast = 12.5;
 
 DensePlan plan_dense(uint32_t rows, uint32_t cols, uint32_t m_rows) {
   auto up = [](uint32_t v, uint32_t by) { return v / by + (v % by != 0); };
@@ -309,7 +312,7 @@ DensePlan plan_dense(uint32_t rows, uint32_t cols, uint32_t m_rows) {
       const uint32_t on_unit = (uint32_t)((tiles * parts + kUnits - 1) / kUnits);
       const double step = g.full * (on_unit / g.resident) + (on_unit % g.resident ? g.part : 0.0);
       double us = g.start + per * step + g.round * up(on_unit, g.resident);
-      if (parts > 1) us += g.second + g.sums * 8e-6 * parts * m_rows * rows;
+      if (parts > 1) us = std::max(us + g.second + g.sums * 8e-6 * parts * m_rows * rows, kCutAtLeast);
       if (us < best.us) best = DensePlan{t, tiles_m, tiles_n, parts, per, us};
     }
   }

@@ -38,7 +38,7 @@ def _product(x, w, bias):
 # one row and column
 SHAPES = [(1, 1, 8), (129, 65, 24), (130, 63, 64), (128, 64, 128), (257, 127, 72), (129, 300, 136), (200, 255, 528), (256, 256, 2048),
           (257, 770, 16), (300, 4099, 1040), (1000, 2050, 600), (513, 2305, 10304), (1000, 1028, 16448), (160, 5120, 17408),
-          (129, 257, 520), (257, 2049, 1032), (257, 2049, 4104), (129, 4100, 4104), (257, 12290, 1032), (1000, 3001, 4104),
+          (129, 257, 1032), (257, 2049, 1032), (257, 2049, 4104), (129, 4100, 4104), (257, 12290, 1032), (1000, 3001, 4104),
           (1000, 8193, 520), (129, 12290, 4104), (1000, 12290, 1032)]
 
 
