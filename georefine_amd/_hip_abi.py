@@ -61,10 +61,12 @@ class GrfPpcxFused(ctypes.Structure):
 
 
 ERR_INDEX = 16  # GRF_ERR_INDEX
+GATHER_DONE = 0x40000000  # GRF_GATHER_DONE
+GATHER_COUNTER_BYTES = 4224  # GRF_GATHER_COUNTER_BYTES
 RAW_PAIRS = 0x100  # GRF_RAW_PAIRS
 
 DEVICE_SYMBOLS = ("grf_bctx_decode", "grf_ppcx_decode", "grf_mix_predict", "grf_bctx_gemv",
-                  "grf_bctx_fused_decode", "grf_bctx_fused_gather", "grf_bctx_gather_rows", "grf_bctx_fused_validate_host", "grf_bctx_fused_lds_bytes", "grf_bctx_gemm", "grf_bctx_gemm_lds_bytes",
+                  "grf_bctx_fused_decode", "grf_bctx_fused_gather", "grf_bctx_gather_rows", "grf_bctx_gather_rows_done", "grf_wait_word", "grf_bctx_fused_validate_host", "grf_bctx_fused_lds_bytes", "grf_bctx_gemm", "grf_bctx_gemm_lds_bytes",
                   "grf_gemm_workspace_bytes", "grf_gemm_workspace_bytes_split", "grf_bctx_gemm_noalloc", "grf_gemm_noalloc_limit_bytes", "grf_pack_activations", "grf_bctx_gemv_group", "grf_bctx_gemm_group",
                   "grf_ppcx_bins", "grf_ppcx_bins_ordered", "grf_ppcx_fused_decode", "grf_ppcx_gemv", "grf_ppcx_gemm", "grf_ppcx_gemv_group", "grf_ppcx_gemm_group", "grf_dense_gemm_plan", "grf_dense_gemm_workspace_bytes", "grf_dense_gemm", "grf_pair_residuals", "grf_last_error",
                   "grf_abi_version", "grf_timestamp", "grf_wall_clock_khz")
@@ -106,6 +108,10 @@ def declare(L):
     L.grf_bctx_fused_gather.restype = i
     L.grf_bctx_gather_rows.argtypes = [ctypes.POINTER(GrfBctxFused), u32, u32, vp, vp, u32, vp, vp, vp, vp]
     L.grf_bctx_gather_rows.restype = i
+    L.grf_bctx_gather_rows_done.argtypes = [ctypes.POINTER(GrfBctxFused), u32, u32, vp, vp, u32, vp, vp, vp, vp, vp, vp]
+    L.grf_bctx_gather_rows_done.restype = i
+    L.grf_wait_word.argtypes = [vp, i, u32]
+    L.grf_wait_word.restype = i
     L.grf_bctx_fused_validate_host.argtypes = [ctypes.POINTER(GrfBctxFused), tiling, i, vp, vp, vp, vp, vp]
     L.grf_bctx_fused_validate_host.restype = i
     L.grf_bctx_fused_lds_bytes.argtypes = [ctypes.POINTER(GrfBctxFused), tiling, u32]

@@ -149,6 +149,22 @@ def _host_word():
         return torch.zeros(1, dtype=torch.int32, pin_memory=True)
 
 
+# Counters of gathers under way, by device; a call takes some and gives them back, as it does a word.
+_done_counters = {}
+
+
+def _counters_for(index):
+    try:
+        return _done_counters.setdefault(index, []).pop()
+    except IndexError:
+        import torch
+        return torch.zeros(_hip_abi.GATHER_COUNTER_BYTES // 4, dtype=torch.int32, device=f"cuda:{index}")
+
+
+# How long a gather is polled for before the thread sleeps until the stream is done.
+GATHER_SPIN_US = 100
+
+
 def route_rows(m, cols, invariant=False):
     """The kernel family that takes ``m`` activation rows of a matrix with ``cols`` columns:
     ``"gemv"`` (vector ALUs), ``"gemm"`` (matrix cores) or ``"dense"`` (fused decode + library
@@ -745,36 +761,39 @@ class HipContextTensor:
         return self._decode_blocks(blocks, check=check).reshape(*ids.shape, self.shape[1])
 
     def _gather_fused(self, ids, check, validate):
-        """One launch, which also looks up classes and tests the ids, and one wait for it: what it
-        finds wrong it writes to a word of pinned host memory, which nothing has to copy back."""
+        """One launch, which also looks up classes and tests the ids; what it finds wrong it writes to a word of
+        pinned host memory, which nothing has to copy back, and that it is over to the same word, which
+        is polled: a wait for the stream takes 2 us longer (777 rows of 8192 x 5120 31.0 -> 28.6, one row 26.9 -> 25.8)."""
         import torch
         ids = ids.contiguous()
         out = torch.empty((*ids.shape, self.shape[1]), device=self.device, dtype=torch.bfloat16)
-        word = where = None
-        if check or validate:
-            word = _host_word()
-            where = word.data_ptr()
         if check and self._error_open:  # between checks the word keeps what earlier launches reported
             self.error.zero_()
             self._error_open = False
         elif not check:
             self._error_open = True
-        self._launch(self._lib.grf_bctx_gather_rows, ctypes.byref(self.fused), *self._gather, self.buffers["rows"].data_ptr(),
-                     ids.data_ptr(), ids.numel(), out.data_ptr(), where if check else self.error.data_ptr(),
-                     where if validate else None)
-        if word is not None:
+        about = (ctypes.byref(self.fused), *self._gather, self.buffers["rows"].data_ptr(), ids.data_ptr(), ids.numel(), out.data_ptr())
+        if not (check or validate):
+            self._launch(self._lib.grf_bctx_gather_rows, *about, self.error.data_ptr(), None)
+            return out
+        word, counters = _host_word(), _counters_for(self._index)
+        where = word.data_ptr()
+        self._launch(self._lib.grf_bctx_gather_rows_done, *about, where if check else self.error.data_ptr(),
+                     where if validate else None, counters.data_ptr(), where)
+        if not self._lib.grf_wait_word(where, _hip_abi.GATHER_DONE, GATHER_SPIN_US):
             torch.cuda.current_stream(self._index).synchronize()
-            found = ctypes.c_int32.from_address(where).value  # (a tensor's element costs twice the time)
-            if found:
-                word[0] = 0
-            if len(_host_words) < HOST_WORDS_KEPT:
-                _host_words.append(word)
-            if found & _hip_abi.ERR_INDEX:
-                raise IndexError("embedding row outside tensor")
-            if found:
-                self.error.fill_(found)
-                self._error_open = True
-                raise base.CodecError("HIP decoder checkpoint mismatch")
+        value = ctypes.c_int32.from_address(where)  # (a tensor's element costs twice the time)
+        found, value.value = value.value & ~_hip_abi.GATHER_DONE, 0
+        if len(_host_words) < HOST_WORDS_KEPT:
+            _host_words.append(word)
+        if len(_done_counters[self._index]) < HOST_WORDS_KEPT:
+            _done_counters[self._index].append(counters)
+        if found & _hip_abi.ERR_INDEX:
+            raise IndexError("embedding row outside tensor")
+        if found:
+            self.error.fill_(found)
+            self._error_open = True
+            raise base.CodecError("HIP decoder checkpoint mismatch")
         return out
 
 

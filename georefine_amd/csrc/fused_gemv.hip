@@ -2,6 +2,8 @@
 // and of the store sink that backs decode() for fused frames.  Kernels: fused_kernels.h.
 #include "fused_kernels.h"
 
+#include <chrono>
+
 namespace grf {
 int check_fused_frame(const grf_bctx_fused &f, const grf_fused_tiling &g, const char *who, TilingUse use, bool pointers) {
   auto bad = [&](const char *why) { return grf::set_error(GRF_BAD_ARGUMENT, std::string(who) + ": " + why); };
@@ -149,6 +151,30 @@ int validate_fused_host(const grf_bctx_fused &f, const grf_fused_tiling &g, Tili
 }
 }  // namespace grf
 
+namespace {
+
+int gather(const char *who, const grf_bctx_fused *frame, uint32_t lanes, uint32_t piece_cap, const uint8_t *row_class,
+           const int64_t *ids, uint32_t count, uint16_t *out, int32_t *error, int32_t *index_error, const grf::GatherDone &done,
+           void *hip_stream) {
+  if (!frame || !row_class || !ids || !out || !error) return grf::set_error(GRF_BAD_ARGUMENT, std::string(who) + ": null argument");
+  grf_fused_tiling one{};  // (the frame's own checks, with a tiling that cannot fail them)
+  one.tile_rows = reinterpret_cast<const uint32_t *>(ids);
+  one.tile_class = row_class;
+  one.threads = 64;
+  one.lanes_per_row = 64;
+  one.rows_per_tile = one.n_tiles = 1;
+  one.n_slabs = (frame->segs_per_row + 63) / 64;
+  one.piece_cap = piece_cap;
+  const grf::ContextFrame f(*frame);
+  if (int rc = grf::check_fused_frame(f, one, who)) return rc;
+  return grf::with_walk(f.pairs, [&](auto walk) {
+    return grf::launch_gather<typename decltype(walk)::type>(who, f, lanes, piece_cap, row_class, ids, count, out, error,
+                                                             index_error, done, (hipStream_t)hip_stream);
+  });
+}
+
+}  // namespace
+
 extern "C" {
 
 uint32_t grf_bctx_fused_lds_bytes(const grf_bctx_fused *frame, const grf_fused_tiling *tiling, uint32_t m_rows) {
@@ -220,22 +246,28 @@ int grf_bctx_fused_gather(const grf_bctx_fused *frame, const grf_fused_tiling *t
 
 int grf_bctx_gather_rows(const grf_bctx_fused *frame, uint32_t lanes, uint32_t piece_cap, const uint8_t *row_class,
                          const int64_t *ids, uint32_t count, uint16_t *out, int32_t *error, int32_t *index_error, void *hip_stream) {
-  if (!frame || !row_class || !ids || !out || !error)
-    return grf::set_error(GRF_BAD_ARGUMENT, "grf_bctx_gather_rows: null argument");
-  grf_fused_tiling one{};  // (the frame's own checks, with a tiling that cannot fail them)
-  one.tile_rows = reinterpret_cast<const uint32_t *>(ids);
-  one.tile_class = row_class;
-  one.threads = 64;
-  one.lanes_per_row = 64;
-  one.rows_per_tile = one.n_tiles = 1;
-  one.n_slabs = (frame->segs_per_row + 63) / 64;
-  one.piece_cap = piece_cap;
-  const grf::ContextFrame f(*frame);
-  if (int rc = grf::check_fused_frame(f, one, "grf_bctx_gather_rows")) return rc;
-  return grf::with_walk(f.pairs, [&](auto walk) {
-    return grf::launch_gather<typename decltype(walk)::type>("grf_bctx_gather_rows", f, lanes, piece_cap, row_class, ids, count,
-                                                             out, error, index_error, (hipStream_t)hip_stream);
-  });
+  return gather("grf_bctx_gather_rows", frame, lanes, piece_cap, row_class, ids, count, out, error, index_error, {}, hip_stream);
+}
+
+int grf_bctx_gather_rows_done(const grf_bctx_fused *frame, uint32_t lanes, uint32_t piece_cap, const uint8_t *row_class,
+                              const int64_t *ids, uint32_t count, uint16_t *out, int32_t *error, int32_t *index_error,
+                              void *counters, int32_t *done, void *hip_stream) {
+  if (!counters || !done || !count || (uintptr_t)counters & 127)
+    return grf::set_error(GRF_BAD_ARGUMENT, "grf_bctx_gather_rows_done: counters (128-byte aligned), a word and ids are needed");
+  return gather("grf_bctx_gather_rows_done", frame, lanes, piece_cap, row_class, ids, count, out, error, index_error,
+                {static_cast<uint32_t *>(counters), done}, hip_stream);
+}
+
+int grf_wait_word(const int32_t *word, int32_t bits, uint32_t microseconds) {
+  if (!word) return 0;
+  const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(microseconds);
+  for (;;) {
+    for (int i = 0; i < 64; ++i) {
+      if (__atomic_load_n(word, __ATOMIC_ACQUIRE) & bits) return 1;
+      __builtin_ia32_pause();
+    }
+    if (std::chrono::steady_clock::now() >= until) return 0;
+  }
 }
 
 }  // extern "C"

@@ -378,6 +378,18 @@ int grf_bctx_fused_gather(const grf_bctx_fused *frame, const grf_fused_tiling *t
 int grf_bctx_gather_rows(const grf_bctx_fused *frame, uint32_t lanes, uint32_t piece_cap, const uint8_t *row_class,
                          const int64_t *ids, uint32_t count, uint16_t *out, int32_t *error, int32_t *index_error, void *hip_stream);
 
+/* The same launch, which also sets GRF_GATHER_DONE in *done, a word of pinned (coherent) host memory, when the output and
+ * both error words are complete: a host that polls it learns so without a wait for the stream.  `done` may be the word
+ * that the errors go to.  counters: GRF_GATHER_COUNTER_BYTES of device memory, 128-byte aligned, zero, of this
+ * launch alone until it is over, and zero again then.  count is at least 1. */
+#define GRF_GATHER_DONE 0x40000000
+#define GRF_GATHER_COUNTER_BYTES 4224
+int grf_bctx_gather_rows_done(const grf_bctx_fused *frame, uint32_t lanes, uint32_t piece_cap, const uint8_t *row_class,
+                              const int64_t *ids, uint32_t count, uint16_t *out, int32_t *error, int32_t *index_error,
+                              void *counters, int32_t *done, void *hip_stream);
+/* Host: whether any of `bits` appears in *word within that time; spins. */
+int grf_wait_word(const int32_t *word, int32_t bits, uint32_t microseconds);
+
 /* Fused decode-GEMM on the matrix cores for any number of activation rows; same operand
  * meaning as grf_bctx_gemv.  Batch-invariant in the sense of GS/bi_csrc/bi_gemm.cuh:1-17:
  * with one tiling, row m of y is a function of row m of x and of W only.  x must be
