@@ -359,34 +359,44 @@ __device__ __forceinline__ void transpose_quad(uint32_t (&u)[4][4], uint32_t lan
 #endif
 }
 
-// The walk of a unit whose words go to the dense matrix; every lane of the wave takes part (the
-// exchange above reads all of a quad's lanes), those without a segment (`walks` false) store nothing.
-// first: the segment's first word in the output.  S is a multiple of 16.
-// THROUGH: `out` is one 16-byte aligned row of row_bytes, and the stores go past the caches, so that they are where every
-// reader looks once the wave's memory counter says so.
-template <class Walk, int SCAN, bool THROUGH = false>
-__device__ __forceinline__ void store_segment(Walk &w, const grf::FusedParams &q, uint32_t S, bool walks, uint32_t first,
-                                              uint16_t *out, uint32_t lane, uint32_t row_bytes = 0) {
-  constexpr uint32_t kNowhere = 0xFFFFFFFFu;
-  auto put = [&](size_t word, words8_t v) {
+// How far a store goes before the wave is done with it: to its XCD's second-level cache, which writes back when it needs
+// the room and at the end of the launch; through it to what the device shares, the last-level cache first of all; or
+// to where the host and other streams look as well.
+enum Far : int { kKept = 0, kDevice = 16, kSystem = 17 };  // (bits sc0 and sc1 of a store)
+
+// Where words go: any address, or, to go further, `bytes` from a 16-byte aligned one on, up to 4 GiB.
+template <int FAR>
+struct Words {
+  uint16_t *data;
+  uint32_t bytes = 0;
+  __device__ __forceinline__ void put(size_t word, words8_t v) const {
 #if defined(__HIP_DEVICE_COMPILE__)
-    if constexpr (THROUGH) {
+    if constexpr (FAR != kKept) {
       typedef uint32_t uint4v __attribute__((ext_vector_type(4)));
-      const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(out, 0, (int)row_bytes, 0x00020000);
-      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(uint4v, v), rsrc, (uint32_t)word * 2u, 0, 17);  // sc0 sc1
+      const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(data, 0, (int)bytes, 0x00020000);
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(uint4v, v), rsrc, (uint32_t)word * 2u, 0, FAR);
       return;
     }
 #endif
-    *reinterpret_cast<words8_t *>(out + word) = v;
-  };
+    *reinterpret_cast<words8_t *>(data + word) = v;
+  }
+};
+
+// The walk of a unit whose words go to the dense matrix; every lane of the wave takes part (the
+// exchange above reads all of a quad's lanes), those without a segment (`walks` false) store nothing.
+// first: the segment's first word in the output.  S is a multiple of 16.
+template <class Walk, int SCAN, int FAR = kKept>
+__device__ __forceinline__ void store_segment(Walk &w, const grf::FusedParams &q, uint32_t S, bool walks, uint32_t first,
+                                              const Words<FAR> &out, uint32_t lane) {
+  constexpr uint32_t kNowhere = 0xFFFFFFFFu;
   if (S % 32) {  // segments of 16 words: a lane's 32 bytes, next to its neighbours'
     for (uint32_t t = 0; walks && t < S; t += 16) {
       uint32_t pair[8];
       w.begin16(t, S);
       w.template half<0, SCAN>(q, reinterpret_cast<uint32_t(&)[4]>(pair[0]));
       w.template half<1, SCAN>(q, reinterpret_cast<uint32_t(&)[4]>(pair[4]));
-      put((size_t)first + t, (words8_t){pair[0], pair[1], pair[2], pair[3]});
-      put((size_t)first + t + 8, (words8_t){pair[4], pair[5], pair[6], pair[7]});
+      out.put((size_t)first + t, (words8_t){pair[0], pair[1], pair[2], pair[3]});
+      out.put((size_t)first + t + 8, (words8_t){pair[4], pair[5], pair[6], pair[7]});
     }
     return;
   }
@@ -414,7 +424,7 @@ __device__ __forceinline__ void store_segment(Walk &w, const grf::FusedParams &q
 #else
       const uint32_t at = unit;
 #endif
-      if (at != kNowhere) put(((size_t)at + t / 8 + (lane & 3)) * 8, (words8_t){v[0], v[1], v[2], v[3]});
+      if (at != kNowhere) out.put(((size_t)at + t / 8 + (lane & 3)) * 8, (words8_t){v[0], v[1], v[2], v[3]});
     };
     flush(std::integral_constant<int, 0>{}, u[0]);
     flush(std::integral_constant<int, 1>{}, u[1]);
@@ -425,12 +435,12 @@ __device__ __forceinline__ void store_segment(Walk &w, const grf::FusedParams &q
 
 // Decoded words of a unit that are still to be stored: the last 32 * H columns of every lane's segment,
 // quads already exchanged, so that u[h][k] of lane j is 16-byte unit 4 * h + j of what lane k decoded.
-template <int H>
+template <int H, int FAR = kKept>
 struct HeldWords {
   static constexpr uint32_t kNowhere = 0xFFFFFFFFu;
   uint32_t u[H][4][4];
   uint32_t unit = kNowhere;  // the lane's first 16-byte unit in the output
-  __device__ __forceinline__ void flush(uint16_t *out, uint32_t lane) {
+  __device__ __forceinline__ void flush(const Words<FAR> &out, uint32_t lane) {
     auto run = [&](auto k) {
       constexpr int K = decltype(k)::value;
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -439,10 +449,9 @@ struct HeldWords {
       const uint32_t at = unit;
 #endif
       if (at == kNowhere) return;
-      words8_t *dst = reinterpret_cast<words8_t *>(out) + ((size_t)at + (lane & 3));
 #pragma unroll
       for (int h = 0; h < H; ++h)
-        dst[4 * h] = (words8_t){u[h][K][0], u[h][K][1], u[h][K][2], u[h][K][3]};
+        out.put(((size_t)at + (lane & 3) + 4 * h) * 8, (words8_t){u[h][K][0], u[h][K][1], u[h][K][2], u[h][K][3]});
     };
     run(std::integral_constant<int, 0>{});
     run(std::integral_constant<int, 1>{});
@@ -451,18 +460,18 @@ struct HeldWords {
     unit = kNowhere;
   }
 };
-template <>
-struct HeldWords<0> {
-  __device__ __forceinline__ void flush(uint16_t *, uint32_t) {}
+template <int FAR>
+struct HeldWords<0, FAR> {
+  __device__ __forceinline__ void flush(const Words<FAR> &, uint32_t) {}
 };
 
 // The same walk for a kernel that goes on to another unit (S a multiple of 32 * H): the words of 32 * H columns
 // are held back, the unit's last ones until the next unit's pieces have arrived.  A wave waits for the
 // bytes of a unit with its whole counter of memory operations, so stores just before that wait would
 // be waited for as well.
-template <class Walk, int SCAN, int H>
+template <class Walk, int SCAN, int H, int FAR>
 __device__ __forceinline__ void hold_segment(Walk &w, const grf::FusedParams &q, uint32_t S, bool walks, uint32_t first,
-                                             uint16_t *out, uint32_t lane, HeldWords<H> &held) {
+                                             const Words<FAR> &out, uint32_t lane, HeldWords<H, FAR> &held) {
   held.flush(out, lane);  // the unit before (after the next group's loads instead: 4 % slower)
   for (uint32_t t = 0; t < S; t += 32 * H) {
     if (t) held.flush(out, lane);
@@ -479,12 +488,12 @@ __device__ __forceinline__ void hold_segment(Walk &w, const grf::FusedParams &q,
       }
       transpose_quad(u, lane);
     }
-    held.unit = walks ? (first + t) / 8 : HeldWords<H>::kNowhere;  // (fits 32 bits: rows are multiples of 16 words)
+    held.unit = walks ? (first + t) / 8 : HeldWords<H, FAR>::kNowhere;  // (fits 32 bits: rows are multiples of 16 words)
   }
 }
 
 // SINK kDot: products with M activation rows; kStore: the words to `out` (M = 0), 32 * HOLD columns at a time.
-template <class Walk, int M, int SCAN, int SINK = kDot, int HOLD = 0>
+template <class Walk, int M, int SCAN, int SINK = kDot, int HOLD = 0, int FAR = kKept>
 __device__ __forceinline__ void fused_wave_body(uint8_t *lds, const grf_bctx_fused &f, const grf_fused_tiling &g,
                                                 const uint16_t *x, uint32_t ldx, uint16_t *y, uint32_t ldy,
                                                 const uint16_t *bias, int32_t *error, uint32_t tile,
@@ -578,7 +587,8 @@ __device__ __forceinline__ void fused_wave_body(uint8_t *lds, const grf_bctx_fus
   __syncthreads();
   const uint32_t later_half = blockIdx.x >= gridDim.x / 2 ? 1u : 0u;
   uint32_t left = wave < units ? (units - 1 - wave) / nwaves : 0;  // units after the current one
-  HeldWords<HOLD> held;
+  HeldWords<HOLD, FAR> held;
+  const Words<FAR> words_out{out, f.rows * f.cols * 2};
   for (uint32_t u = wave; u < units; u += nwaves, --left) {  // wave-uniform
 #if defined(__HIP_DEVICE_COMPILE__)
     // Waves with more units still to do go first.  Left alone the arbiter prefers the older
@@ -625,8 +635,8 @@ __device__ __forceinline__ void fused_wave_body(uint8_t *lds, const grf_bctx_fus
     }
 #endif
     if constexpr (SINK == kStore) {
-      if constexpr (HOLD > 0) hold_segment<Walk, SCAN>(w, q, S, walks, walks ? mul24(row, K) + col0 : 0, out, lane, held);
-      else store_segment<Walk, SCAN>(w, q, S, walks, walks ? mul24(row, K) + col0 : 0, out, lane);
+      if constexpr (HOLD > 0) hold_segment<Walk, SCAN>(w, q, S, walks, walks ? mul24(row, K) + col0 : 0, words_out, lane, held);
+      else store_segment<Walk, SCAN>(w, q, S, walks, walks ? mul24(row, K) + col0 : 0, words_out, lane);
       if (walks && !w.ended_on_checkpoint(f)) bad |= GRF_ERR_CHECKPOINT;
       continue;
     }
@@ -693,7 +703,7 @@ __device__ __forceinline__ void fused_wave_body(uint8_t *lds, const grf_bctx_fus
     }
   }
   if constexpr (SINK == kStore) {
-    held.flush(out, lane);
+    held.flush(words_out, lane);
     if (bad) atomicOr(error, (int)bad);
     return;
   }
@@ -753,11 +763,11 @@ __global__ __launch_bounds__(grf::kFusedMaxThreads) __attribute__((amdgpu_waves_
 // Before and now: 5120 x 17408 104.6 -> 91.2 us, 17408 x 5120 -> 87.4, 5120 x 6144 43.9 -> 38.9, 4096 x 4096
 // 24.8 -> 23.0, 2560 x 5120 27.1 -> 22.4; HOLD 1 alone 104.6 -> 102.0; 700 x 9216 at segments of 32 15.5 -> 14.9.  With
 // the stores absorbed by the cache the first takes 76.  Streaming stores cost 6 %.
-template <class Walk, int SCAN, int HOLD>
+template <class Walk, int SCAN, int HOLD, int FAR>
 __global__ __launch_bounds__(grf::kFusedMaxThreads) __attribute__((amdgpu_waves_per_eu(HOLD == 2 ? 4 : 6))) void fused_wave_store_kernel(
     grf_bctx_fused f, grf_fused_tiling g, uint16_t *out, int32_t *error) {
   extern __shared__ __align__(16) uint8_t lds[];
-  fused_wave_body<Walk, 0, SCAN, kStore, HOLD>(lds, f, g, nullptr, 0, nullptr, 0, nullptr, error, blockIdx.x, out);
+  fused_wave_body<Walk, 0, SCAN, kStore, HOLD, FAR>(lds, f, g, nullptr, 0, nullptr, 0, nullptr, error, blockIdx.x, out);
 }
 
 template <auto Kernel>
@@ -774,19 +784,27 @@ int launch_wave_store(const grf_bctx_fused &f, const grf_fused_tiling &g, uint16
     hipLaunchKernelGGL(kernel, dim3(g.n_tiles), dim3(g.threads), L.total, s, f, g, out, error);
     return GRF_OK;
   };
-  auto launch = [&](auto scan) -> int {
-    constexpr int kScan = decltype(scan)::value;
+  auto launch = [&](auto scan, auto far) -> int {
+    constexpr int kScan = decltype(scan)::value, kFar = decltype(far)::value;
     const uint32_t waves = g.threads / 64, rpw = 64 / g.lanes_per_row;
     const bool one_each = (g.rows_per_tile + rpw - 1) / rpw * g.n_slabs <= waves;  // units
     // (sixteen waves a unit: in one workgroup, or in all that a unit gets)
     if (f.seg_len % 64 == 0 && (g.threads == 1024 || g.n_tiles * waves <= 256 * 16))
-      return start(KernelOf<&fused_wave_store_kernel<Walk, kScan, 2>>{});
-    if (f.seg_len % 32 || (f.seg_len % 64 == 0 && one_each)) return start(KernelOf<&fused_wave_store_kernel<Walk, kScan, 0>>{});
-    return start(KernelOf<&fused_wave_store_kernel<Walk, kScan, 1>>{});
+      return start(KernelOf<&fused_wave_store_kernel<Walk, kScan, 2, kFar>>{});
+    if (f.seg_len % 32 || (f.seg_len % 64 == 0 && one_each)) return start(KernelOf<&fused_wave_store_kernel<Walk, kScan, 0, kFar>>{});
+    return start(KernelOf<&fused_wave_store_kernel<Walk, kScan, 1, kFar>>{});
   };
-  if (int rc = f.whole_range ? launch(std::integral_constant<int, grf::kScanAny>{})
-                             : launch(std::integral_constant<int, grf::kScanNoWholeRange>{}))
-    return rc;
+  auto launch_far = [&](auto far) {
+    return f.whole_range ? launch(std::integral_constant<int, grf::kScanAny>{}, far)
+                         : launch(std::integral_constant<int, grf::kScanNoWholeRange>{}, far);
+  };
+  // Results that the last-level cache takes up beside what is read go straight to it: nothing is then left to write
+  // back when the launch ends.  us, four results written in turn, and one with a product of 256 rows after it:
+  //   1024 x 1024 8.5 26.5 -> 8.2 26.6, 2048 x 2048 11.8 26.1 -> 10.9 26.2, 4096 x 2048 14.3 27.3 -> 12.7 25.9,
+  //   4096 x 4096 22.4 39.5 -> 20.4 38.5; 5120 x 6144, which it does not take up, 42.6 86.3 -> 44.3 90.7, and past that
+  //   cache too 33.9 94.6: faster where nobody reads the result soon, which this call cannot know.
+  const bool far = (uint64_t)f.rows * f.cols * 2 < (48u << 20) && !((uintptr_t)out & 15);
+  if (int rc = far ? launch_far(std::integral_constant<int, kDevice>{}) : launch_far(std::integral_constant<int, kKept>{})) return rc;
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return grf::set_error(GRF_LAUNCH_FAILED, std::string("fused decode: ") + hipGetErrorString(e));
   return GRF_OK;
@@ -873,7 +891,7 @@ __global__ __launch_bounds__(grf::kFusedMaxThreads) void fused_gather_kernel(grf
   const grf::FusedParams q{f.shift, L.block_pitch, grf::fused_table_bytes(f), f.whole_range};
   if (grf::fused_tables_by_dma(f)) grf::fused_load_tables_dma(lds, 0, L.block_pitch, f, cls, wave, nwaves, lane);
   const uint32_t S = f.seg_len, units = (f.segs_per_row + lanes - 1) / lanes, region = L.stream + wave * piece_cap;
-  uint16_t *dst = out + (size_t)blockIdx.x * f.cols;
+  const Words<kSystem> dst{out + (size_t)blockIdx.x * f.cols, f.cols * 2};
   uint32_t bad = 0;
   for (uint32_t u = wave; u - wave < units; u += nwaves) {  // uniform, and as many trips for every wave (the barrier)
     const bool any = u < units;
@@ -895,7 +913,7 @@ __global__ __launch_bounds__(grf::kFusedMaxThreads) void fused_gather_kernel(grf
       __syncthreads();
     }
     __builtin_amdgcn_wave_barrier();
-    store_segment<Walk, SCAN, true>(w, q, S, walks, col0, dst, lane, f.cols * 2);
+    store_segment<Walk, SCAN>(w, q, S, walks, col0, dst, lane);
     if (walks && !w.ended_on_checkpoint(f)) bad |= GRF_ERR_CHECKPOINT;
   }
   if (bad) atomicOr_system(error, (int)bad);
