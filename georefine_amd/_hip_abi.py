@@ -60,6 +60,11 @@ class GrfPpcxFused(ctypes.Structure):
             "whole_range", "raw_interleaved")]
 
 
+class GrfPlanes(ctypes.Structure):
+    _fields_ = [(name, ctypes.c_void_p) for name in ("planes", "bases", "listed_at", "listed")] + [
+        (name, ctypes.c_uint32) for name in ("rows", "cols", "splits", "parts")]
+
+
 ERR_INDEX = 16  # GRF_ERR_INDEX
 GATHER_DONE = 0x40000000  # GRF_GATHER_DONE
 GATHER_COUNTER_BYTES = 4224  # GRF_GATHER_COUNTER_BYTES
@@ -68,7 +73,8 @@ RAW_PAIRS = 0x100  # GRF_RAW_PAIRS
 DEVICE_SYMBOLS = ("grf_bctx_decode", "grf_ppcx_decode", "grf_mix_predict", "grf_bctx_gemv",
                   "grf_bctx_fused_decode", "grf_bctx_fused_gather", "grf_bctx_gather_rows", "grf_bctx_gather_rows_done", "grf_wait_word", "grf_take_word", "grf_bctx_fused_validate_host", "grf_bctx_fused_lds_bytes", "grf_bctx_gemm", "grf_bctx_gemm_lds_bytes",
                   "grf_gemm_workspace_bytes", "grf_gemm_workspace_bytes_split", "grf_bctx_gemm_noalloc", "grf_gemm_noalloc_limit_bytes", "grf_pack_activations", "grf_bctx_gemv_group", "grf_bctx_gemm_group",
-                  "grf_ppcx_bins", "grf_ppcx_bins_ordered", "grf_ppcx_fused_decode", "grf_ppcx_gemv", "grf_ppcx_gemm", "grf_ppcx_gemv_group", "grf_ppcx_gemm_group", "grf_dense_gemm_plan", "grf_dense_gemm_workspace_bytes", "grf_dense_gemm", "grf_pair_residuals", "grf_last_error",
+                  "grf_ppcx_bins", "grf_ppcx_bins_ordered", "grf_ppcx_fused_decode", "grf_ppcx_gemv", "grf_ppcx_gemm", "grf_ppcx_gemv_group", "grf_ppcx_gemm_group", "grf_dense_gemm_plan", "grf_dense_gemm_workspace_bytes", "grf_dense_gemm", "grf_pair_residuals", "grf_planes_bytes", "grf_planes_visits", "grf_planes_count", "grf_planes_fill",
+                  "grf_planes_workspace_bytes", "grf_planes_linear", "grf_planes_group", "grf_planes_decode", "grf_planes_gather", "grf_last_error",
                   "grf_abi_version", "grf_timestamp", "grf_wall_clock_khz")
 
 
@@ -141,6 +147,25 @@ def declare(L):
     L.grf_dense_gemm_workspace_bytes.restype = ctypes.c_size_t
     L.grf_dense_gemm.argtypes = [vp, u32, u32, vp, u32, u32, vp, u32, vp, vp, ctypes.c_size_t, vp]
     L.grf_dense_gemm.restype = i
+    size = ctypes.c_size_t
+    L.grf_planes_bytes.argtypes = [u32, u32]
+    L.grf_planes_bytes.restype = ctypes.c_uint64
+    L.grf_planes_visits.argtypes = [u32, u32]
+    L.grf_planes_visits.restype = u32
+    L.grf_planes_count.argtypes = [vp, u32, u32, vp, vp, vp]
+    L.grf_planes_count.restype = i
+    L.grf_planes_fill.argtypes = [vp, u32, u32, vp, vp, vp, vp, vp]
+    L.grf_planes_fill.restype = i
+    L.grf_planes_workspace_bytes.argtypes = [u32, vp, u32]
+    L.grf_planes_workspace_bytes.restype = size
+    L.grf_planes_linear.argtypes = [vp, vp, u32, u32, u32, vp, vp, vp, size, vp]
+    L.grf_planes_linear.restype = i
+    L.grf_planes_group.argtypes = [u32, vp, vp, u32, u32, u32, vp, vp, vp, vp, size, vp]
+    L.grf_planes_group.restype = i
+    L.grf_planes_decode.argtypes = [vp, vp, vp]
+    L.grf_planes_decode.restype = i
+    L.grf_planes_gather.argtypes = [vp, vp, u32, vp, vp, vp, vp, vp]
+    L.grf_planes_gather.restype = i
     L.grf_timestamp.argtypes = [vp, vp]
     L.grf_timestamp.restype = i
     L.grf_wall_clock_khz.argtypes = []

@@ -1,0 +1,124 @@
+"""Matrices resident as planes: which ones, how a product's sums are split, and the device arrays.
+
+The planes (``csrc/word_planes.h``, ``csrc/planes.hip``) hold a matrix's words at fixed places in 11.5 bits a weight and a
+list of the few whose exponent is outside the eleven that hold most of their row.  A context frame with
+the index its walk needs takes as much (5120 x 17408 of normal weights with a scale a row: 11.6 bits either way;
+small matrices, whose index is finer and whose tables do not shrink, 13 to 30), and its walk is bound by the vector ALUs where the planes are
+read at the memory's pace.  us, walk / planes: one row of 17408 x 5120 twice 110 / 51, six of 5120 x 17408 69 / 37, 64 of the
+first 151 / 104, a decode of 5120 x 6144 39 / 25, 777 of 8192 rows looked up 16 / 7.
+"""
+from __future__ import annotations
+
+import ctypes
+
+import numpy as np
+
+from . import _hip_abi, _native
+
+VISIT, UNIT, VISIT_BYTES, UNIT_BYTES = 256, 64, 5888, 1536  # csrc/word_planes.h
+EXPONENTS = 11
+MAX_COLS = 1 << 17
+IN_PLACE_ROWS = 16  # activation rows that a launch reads where they are and needs no workspace for
+# Weights from which a matrix is laid out.  The kernels are the shorter below it too (one row of 512 x 640 4.4 us, walked 8.4;
+# 32 rows 8.6 and 8.2), but a call is as long as its host path there (502 x 640 at three rows 10.1 and 10.5), and a
+# tensor whose arrays are asked for changes the bits of its products, which the small ones that are looked at do not.
+FROM_WEIGHTS = 1 << 19
+# How much more memory than the frame's arrays the planes may take (frames of few exponents code far below 11.5 bits
+# and stay frames).
+MEMORY = 1.04
+
+
+def visits(cols):
+    """Visits of 256 columns, the last one of up to three units of 64."""
+    return cols // VISIT + (cols % VISIT > 0)
+
+
+def plane_bytes(rows, cols):
+    units = (cols % VISIT + UNIT - 1) // UNIT
+    return -(-rows // 16) * (cols // VISIT * VISIT_BYTES + units * UNIT_BYTES)
+
+
+def listed_share(row_class, col_class, main_freq, nr, nc):
+    """The share of words that the planes would list, by the frame's own frequencies: outside the best eleven
+    exponents of each row class (a row's own are no worse on average)."""
+    exponents = np.asarray(main_freq, dtype=np.float64).reshape(nr, nc, 256, 4).sum(axis=3) / 65536
+    by_row = np.einsum("rce,c->re", exponents, np.bincount(col_class, minlength=nc) / len(col_class))
+    running = np.concatenate((np.zeros((nr, 1)), np.cumsum(by_row, axis=1)), axis=1)
+    inside = (running[:, EXPONENTS:] - running[:, :-EXPONENTS]).max(axis=1)
+    return float((1 - inside) @ np.bincount(row_class, minlength=nr) / len(row_class))
+
+
+def possible(info):
+    """Whether the matrix of a parsed context frame (``bitexact_context_codec.read_words``) can be held as planes."""
+    rows, cols = info["shape"]
+    if info["mode"] not in (0, 128) or cols > MAX_COLS or cols % 16 or rows * cols > 0xFFFFFFFF:
+        return False
+    return 0 < int((info["main_freq"] > 0).sum(axis=1).max()) <= 255  # (what the fused kernels refuse stays refused)
+
+
+def worth(info, segment):
+    """Whether it is, where the walk would index it at ``segment``: from ``FROM_WEIGHTS`` on, where the planes take no more memory
+    than the frame's arrays and 4 %."""
+    rows, cols = info["shape"]
+    n, nr, nc = rows * cols, info["nr"], info["nc"]
+    if n < FROM_WEIGHTS:
+        return False
+    live = int((info["main_freq"] > 0).sum(axis=1).max())
+    tables = nr * nc * 9 * 1024 + nr * (nc * 8 * (live + 1) + 32768)
+    frame = len(info["main_stream"]) + n * 3 // 4 + 8 * rows * (cols // segment + 1) + tables
+    listed = listed_share(info["rows"], info["columns"], info["main_freq"], nr, nc) * n
+    return plane_bytes(rows, cols) + 4 * (listed + rows + rows // 16 * visits(cols)) <= MEMORY * frame
+
+
+def sum_splits(rows, cols):
+    """(splits, parts) of a product's sums (``grf_planes``), by the matrix's sizes alone: as few splits, in parts of
+    two, as give the GPU 3800 waves of up to sixteen rows, so that every member of a group of one width that is
+    not much smaller has the same number.  us for one and 64 rows by splits: 17408 x 5120 twice 2: 53 115, 4: 51 104;
+    5120 x 17408 6: 41 66, 8: 37 65, 12: 34 52; 6144, 1024 and 1024 x 5120 4, 10 and 10: 19 35, 10 each 15.5 37."""
+    v, blocks = visits(cols), -(-rows // 16)
+    fits = [s for s in range(2, 17, 2) if -(-v // s) * (s - 1) < v and -(-v // s) <= 63]
+    if not fits:
+        return 1, 1
+    s = next((s for s in fits if blocks * s >= 3800), fits[-1])
+    return s, s // 2
+
+
+class Planes:
+    """The device arrays of one matrix and the structure the kernels take."""
+
+    ARRAYS = ("planes", "bases", "listed_at", "listed")
+
+    def __init__(self, rows, cols, arrays):
+        self.rows, self.cols, self.arrays = rows, cols, arrays
+        self.splits, self.parts = sum_splits(rows, cols)
+        self.struct = _hip_abi.GrfPlanes(*(arrays[name].data_ptr() for name in self.ARRAYS), rows, cols, self.splits, self.parts)
+        self.address = ctypes.addressof(self.struct)
+        self.nbytes = sum(a.numel() * a.element_size() for a in arrays.values())
+        self._workspace = {}
+
+    @classmethod
+    def of_words(cls, words, launch):
+        """Of a dense matrix of BF16 words on the device.  ``launch(function, *arguments)`` adds the stream."""
+        import torch
+        lib = _native.hip()
+        rows, cols = words.shape
+        make = lambda n, kind: torch.empty(n, device=words.device, dtype=kind)
+        count = lib.grf_planes_visits(rows, cols)
+        bases, counts = make(-(-rows // 16) * 16, torch.int32), make(count, torch.int32)
+        launch(lib.grf_planes_count, words.data_ptr(), rows, cols, bases.data_ptr(), counts.data_ptr())
+        listed_at = torch.zeros(count + 1, device=words.device, dtype=torch.int32)
+        torch.cumsum(counts, 0, out=listed_at[1:])
+        listed = torch.zeros(int(listed_at[-1]) + 1, device=words.device, dtype=torch.int32)  # (the last is nobody's)
+        planes = make(lib.grf_planes_bytes(rows, cols), torch.uint8)
+        launch(lib.grf_planes_fill, words.data_ptr(), rows, cols, bases.data_ptr(), listed_at.data_ptr(), planes.data_ptr(), listed.data_ptr())
+        return cls(rows, cols, {"planes": planes, "bases": bases, "listed_at": listed_at, "listed": listed})
+
+    def clone(self):
+        return Planes(self.rows, self.cols, {k: v.clone() for k, v in self.arrays.items()})
+
+    def workspace(self, m):
+        """Bytes a product of ``m`` rows needs."""
+        m = min(m, 128)
+        if m not in self._workspace:
+            self._workspace[m] = int(_native.hip().grf_planes_workspace_bytes(1, ctypes.byref(ctypes.pointer(self.struct)), m))
+        return self._workspace[m]

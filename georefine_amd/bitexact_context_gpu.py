@@ -4,13 +4,16 @@
 ``index_frame`` / ``CudaContextTensor`` (GCR/bitexact_context_gpu.py:66-106 and
 :109-168): the loader calls ``factory(frame, stride=..., device=...)`` and uses
 ``shape``, ``source_sha256``, ``frame_sha256``, ``frame_bytes``, ``resident_bytes``,
-``decode(check=)`` and ``gather_rows(ids, check=)``.  The frame's main stream stays
-resident byte for byte.  So does the residual section, with one exception: a frame that
-the fused kernels take and whose residuals are a conditional rANS stream (mode 128) has
-them decoded once on the host at load and kept as packed 6-bit fields, the form mode 0
+``decode(check=)`` and ``gather_rows(ids, check=)``.
+
+A frame is validated and decoded on the host when it is loaded, and its matrix is then held in one of two forms.  Most
+are laid out as planes (``_planes``: signs and mantissas as they are, exponents two to seven bits), which
+take the memory of the frame with its index and go at the memory's pace.  Small matrices and those whose frames are much
+smaller than planes stay as frames, and so does a tensor whose arrays are asked for: the main stream byte for
+byte, with a checkpoint index, and the residual section, with one exception: conditional residuals (mode 128) of a frame
+that the fused kernels take are kept as packed 6-bit fields, the form mode 0
 frames carry (``resident_mode`` 0, ``mode`` 128; ``resident_bytes`` then exceeds the
-frame's size by the difference).  The checkpoint index is built once on the host and the
-decode runs in hand-written HIP kernels through the C ABI.
+frame's size by the difference).  Every kernel is hand-written HIP behind the C ABI.
 """
 from __future__ import annotations
 
@@ -22,7 +25,7 @@ import threading
 
 import numpy as np
 
-from . import _fused, _hip_abi, _native, _tables
+from . import _fused, _hip_abi, _native, _planes, _tables
 from . import bitexact_context_codec as base
 
 # The GEMV's tiling scheme: wave units unless the environment asks for the slab kernels.
@@ -77,6 +80,11 @@ def index_frame(frame: bytes, stride: int = 1024, *, fused_segment=None, raw6_re
 def _index_views(frame, stride, fused_segment, raw6_residual):
     """``index_frame`` with the two streams as read-only views (of the frame; a re-packed residual
     section: of its own bytes), for a caller that makes arrays of its own from them."""
+    return _views_of(*_read_frame(frame, stride, fused_segment, raw6_residual))
+
+
+def _read_frame(frame, stride, fused_segment, raw6_residual):
+    """The validated walk of a frame; what it gives is for ``_views_of``, whose arguments come after it."""
     if not isinstance(stride, int) or not 1 <= stride <= 65536:
         raise base.CodecError("invalid checkpoint stride")
     if len(frame) < base.HEADER.size + 32:
@@ -86,15 +94,20 @@ def _index_views(frame, stride, fused_segment, raw6_residual):
     fine = fused_segment if fused_segment and (mode == 0 or repack) else None
     one_walk = fine is not None and stride % fine == 0  # every stride // fine-th entry of the fine index is the coarse one
     info = base.read_words(frame, fine if one_walk else stride, "checkpoint validation failed ({})".format)
+    if mode != 1 and info["words_digest"] != info["digest"]:
+        raise base.CodecError("indexed source checksum mismatch")
+    return info, len(frame), stride, fine, repack
+
+
+def _views_of(info, frame_bytes, stride, fine, repack):
     r, c = info["shape"]
+    mode, one_walk = info["mode"], fine is not None and stride % fine == 0
     out = {"shape": (r, c), "mode": mode, "nr": info["nr"], "nc": info["nc"], "stride": stride,
-           "source_sha256": info["digest"].hex(), "frame_sha256": info["frame_sha256"], "frame_bytes": len(frame)}
+           "source_sha256": info["digest"].hex(), "frame_sha256": info["frame_sha256"], "frame_bytes": frame_bytes}
     if mode == 1:
         out["raw"] = info["raw"].reshape(-1).astype(np.uint16)
         out["resident_mode"] = 1
         return out
-    if info["words_digest"] != info["digest"]:
-        raise base.CodecError("indexed source checksum mismatch")
     rows, columns, sf = info["rows"], info["columns"], info["main_freq"]
     out["resident_mode"] = 0 if repack else mode
     states, offsets = info["main_states"], info["main_offsets"]
@@ -343,6 +356,7 @@ class _Buffers(dict):
 
 
 _packed_lock = threading.Lock()
+_form_lock = threading.RLock()  # (what puts a tensor into its other form reads attributes of it)
 
 
 def _residual_form(groups, to_pairs):
@@ -355,6 +369,70 @@ def _residual_form(groups, to_pairs):
     if status:
         raise base.CodecError(f"device launch failed ({status}): " + lib.grf_last_error().decode(errors="replace"))
     return groups
+
+
+def _stream_arrays(read, fused, residual_block):
+    """The arrays of a frame that is walked where it lies, from what ``_read_frame`` gave."""
+    indexed = _views_of(*read)
+    plan, reason = None, "disabled" if not fused else "frame mode or geometry"
+    if "fused_states" in indexed:
+        try:
+            plan = _fused.FramePlan(indexed["shape"], indexed["nr"], indexed["nc"], indexed["rows"],
+                                    indexed["main_freq"], indexed.pop("fused_states"), indexed.pop("fused_offsets"),
+                                    len(indexed["main_stream"]), indexed["fused_segment"])
+        except _fused.FusedUnsupported as exc:
+            reason = str(exc)
+            indexed.pop("fused_states", None)
+            indexed.pop("fused_offsets", None)
+    main_bytes = len(indexed["main_stream"]) if "main_stream" in indexed else 0
+    raw6_segment = raw6_block = 0
+    if plan is not None:  # the fused kernels read 16-byte vectors: pad the stream's allocation
+        indexed["main_stream"] = np.concatenate((indexed["main_stream"], np.zeros(16, dtype=np.uint8)))
+        # The packed residuals in the order the tile walker reads them (a permutation of the
+        # 12-byte groups of 16 fields, no field is touched): rows by class as the tilings take
+        # them, in blocks of as many rows as a wave unit of the GEMV has; inside a block by
+        # position in the segment, then by segment, then by row.  The lanes of a unit walk
+        # neighbouring segments of the block's rows in step, so they read one run of bytes per
+        # visit and a 128-byte line is used in a single visit; in the frame's order a line came
+        # back from memory about twice per launch.
+        rows_, cols_ = indexed["shape"]
+        seg = indexed["fused_segment"]
+        raw = indexed["residual_stream"]
+        if raw.size == rows_ * cols_ * 3 // 4:
+            block, position, held = plan.residual_order(residual_block)
+            indexed["residual_stream"] = _fused.order_residuals(raw, rows_, cols_, seg, block, position, held)
+            indexed["row_pos"] = position
+            raw6_segment, raw6_block = seg, block
+        states, offsets = plan.seg_state, plan.seg_offset
+        if raw6_segment:  # the segment index in the same blocked order (``_fused.order_index``)
+            spr_ = cols_ // seg
+            states = _fused.order_index(states, rows_, spr_, block, position, held)
+            offsets = _fused.order_index(offsets, rows_, spr_, block, position, held)
+        indexed.update(fused_seg_state=states, fused_seg_offset=offsets, fused_lut=plan.lut, fused_tab=plan.tab)
+    for name in ("main_stream", "residual_stream"):  # what is still a view: callers may keep the result for long
+        if name in indexed and not indexed[name].flags.writeable:
+            indexed[name] = indexed[name].copy()
+    return {"indexed": indexed, "plan": plan, "reason": reason, "main_bytes": main_bytes, "raw6_segment": raw6_segment,
+            "raw6_block": raw6_block}
+
+
+class _Prepared(dict):
+    """What ``HipContextTensor.host_prepare`` gives for a matrix that is held as planes: its words, and what the frame says of
+    itself.  The arrays of the walk (``_stream_arrays``) are made when they are asked for."""
+
+    def __init__(self, read, asked, **fields):
+        super().__init__(asked, **fields)
+        self._read = read
+
+    def __missing__(self, name):
+        if name not in ("indexed", "plan", "reason", "main_bytes", "raw6_segment", "raw6_block"):
+            raise KeyError(name)
+        self.update(_stream_arrays(self._read, True, self["block"]))
+        return self[name]
+
+    def __reduce__(self):  # (the streams are views of the frame)
+        info = {k: bytes(v) if isinstance(v, memoryview) else v for k, v in self._read[0].items()}
+        return _Prepared, ((info, *self._read[1:]), dict(self))
 
 
 class HipContextTensor:
@@ -375,47 +453,21 @@ class HipContextTensor:
                 segment = _fused.choose_segment(header[6], fused_segment, rows=header[5])
             except _fused.FusedUnsupported:
                 segment = None
-        indexed = _index_views(frame, stride, segment, segment is not None)
-        plan, reason = None, "disabled" if not fused else "frame mode or geometry"
-        if "fused_states" in indexed:
-            try:
-                plan = _fused.FramePlan(indexed["shape"], indexed["nr"], indexed["nc"], indexed["rows"],
-                                        indexed["main_freq"], indexed.pop("fused_states"), indexed.pop("fused_offsets"),
-                                        len(indexed["main_stream"]), indexed["fused_segment"])
-            except _fused.FusedUnsupported as exc:
-                reason = str(exc)
-                indexed.pop("fused_states", None)
-                indexed.pop("fused_offsets", None)
-        main_bytes = len(indexed["main_stream"]) if "main_stream" in indexed else 0
-        raw6_segment = raw6_block = 0
-        if plan is not None:  # the fused kernels read 16-byte vectors: pad the stream's allocation
-            indexed["main_stream"] = np.concatenate((indexed["main_stream"], np.zeros(16, dtype=np.uint8)))
-            # The packed residuals in the order the tile walker reads them (a permutation of the
-            # 12-byte groups of 16 fields, no field is touched): rows by class as the tilings take
-            # them, in blocks of as many rows as a wave unit of the GEMV has; inside a block by
-            # position in the segment, then by segment, then by row.  The lanes of a unit walk
-            # neighbouring segments of the block's rows in step, so they read one run of bytes per
-            # visit and a 128-byte line is used in a single visit; in the frame's order a line came
-            # back from memory about twice per launch.
-            rows_, cols_ = indexed["shape"]
-            seg = indexed["fused_segment"]
-            raw = indexed["residual_stream"]
-            if raw.size == rows_ * cols_ * 3 // 4:
-                block, position, held = plan.residual_order(residual_block)
-                indexed["residual_stream"] = _fused.order_residuals(raw, rows_, cols_, seg, block, position, held)
-                indexed["row_pos"] = position
-                raw6_segment, raw6_block = seg, block
-            states, offsets = plan.seg_state, plan.seg_offset
-            if raw6_segment:  # the segment index in the same blocked order (``_fused.order_index``)
-                spr_ = cols_ // seg
-                states = _fused.order_index(states, rows_, spr_, block, position, held)
-                offsets = _fused.order_index(offsets, rows_, spr_, block, position, held)
-            indexed.update(fused_seg_state=states, fused_seg_offset=offsets, fused_lut=plan.lut, fused_tab=plan.tab)
-        for name in ("main_stream", "residual_stream"):  # what is still a view: callers may keep the result for long
-            if name in indexed and not indexed[name].flags.writeable:
-                indexed[name] = indexed[name].copy()
-        return {"indexed": indexed, "plan": plan, "reason": reason, "stride": stride, "fused": fused,
-                "asked_segment": fused_segment, "main_bytes": main_bytes, "raw6_segment": raw6_segment, "raw6_block": raw6_block}
+        read = _read_frame(frame, stride, segment, segment is not None)
+        info = read[0]
+        could = segment is not None and GEMV_WAVES and _planes.possible(info)
+        sections = None
+        if could:  # the frame's labels and tables, as it has them
+            meta, tables = base.HEADER.unpack_from(frame)[7:9]
+            at = base.HEADER.size
+            sections = bytes(frame[at:at + meta]), bytes(frame[at + meta:at + meta + tables])
+        asked = {"stride": stride, "fused": fused, "asked_segment": fused_segment, "sections": sections, "block": residual_block}
+        if not could or not _planes.worth(info, segment):
+            return {**asked, **_stream_arrays(read, fused, residual_block)}
+        if residual_block not in (None, 1, 2, 4, 8, 16):
+            raise _fused.FusedUnsupported("residual blocks have 1, 2, 4, 8 or 16 rows")
+        return _Prepared(read, asked, words=info["words"], shape=info["shape"], mode=info["mode"], nr=info["nr"], nc=info["nc"],
+                         source_sha256=info["digest"].hex(), frame_sha256=info["frame_sha256"], frame_bytes=len(frame))
 
     def __init__(self, frame: bytes, *, stride: int = 1024, device="cuda:0", fused=True, fused_segment=None,
                  m_invariant=False, prepared=None, residual_block=None):
@@ -431,37 +483,110 @@ class HipContextTensor:
                                          residual_block=residual_block)
         elif prepared["stride"] != stride or prepared["fused"] != fused:
             raise ValueError("the frame was prepared with another stride or fused setting")
-        indexed, plan = prepared["indexed"], prepared["plan"]
-        self.asked_segment = prepared["asked_segment"]  # None: the length was left to ``choose_segment``
-        self.shape = indexed["shape"]
-        self.n = math.prod(self.shape)
         self.stride = stride
-        self.mode, self.nr, self.nc = indexed["mode"], indexed["nr"], indexed["nc"]
-        # form of the residual section on the device: 0 = packed 6-bit, 128 = rANS stream
-        self.resident_mode = indexed["resident_mode"]
-        self.source_sha256 = indexed["source_sha256"]
-        self.frame_sha256 = indexed["frame_sha256"]
-        self.frame_bytes = indexed["frame_bytes"]
+        self.asked_segment = prepared["asked_segment"]  # None: the length was left to ``choose_segment``
         self.device = torch.device(device)
         self._index = device_index(self.device)
         self._error_open = True  # the error word may hold what an unchecked launch reported
-        self.buffers = _Buffers()
+        self.error = torch.zeros((), device=self.device, dtype=torch.int32)
+        about = prepared if isinstance(prepared, _Prepared) else prepared["indexed"]
+        self.shape = about["shape"]
+        self.n = math.prod(self.shape)
+        self.mode, self.nr, self.nc = about["mode"], about["nr"], about["nc"]
+        self.source_sha256 = about["source_sha256"]
+        self.frame_sha256 = about["frame_sha256"]
+        self.frame_bytes = about["frame_bytes"]
+        self._sections, self._block = prepared["sections"], prepared["block"]
+        if isinstance(prepared, _Prepared):
+            self.resident_mode = 0  # (as the walk would hold it, should it be asked for)
+            self.fused_reason = ""
+            words = torch.from_numpy(prepared["words"].view(np.int16)).to(self.device).view(self.shape)
+            self._hold_planes(words)
+        else:
+            # form of the residual section on the device: 0 = packed 6-bit, 128 = rANS stream
+            self.resident_mode = about["resident_mode"]
+            self._hold_streams(prepared)
+
+    # A tensor is held in one of two forms.  As planes (``_planes``) it answers products, decode and lookups.  The
+    # other is the frame's own arrays, which the walk of its states takes: frames that the planes do not take
+    # are held so from the start, and a tensor whose arrays, plan or descriptors are asked for, for the C interface
+    # or to be looked at, is put into that form then, and stays in it.
+    _planes = None
+    _STREAM_FORM = frozenset(("buffers", "fused", "fused_plan", "_plan", "_frame", "_tilings", "_workspace", "_gather", "_main_bytes",
+                              "_raw6_segment", "_raw6_block", "_gather_waves"))
+
+    def __getattr__(self, name):  # (only of what the object does not have)
+        if name in HipContextTensor._STREAM_FORM and self.__dict__.get("_planes") is not None:
+            with _form_lock:
+                if self._planes is not None:
+                    self._leave_planes()
+            return getattr(self, name)
+        raise AttributeError(f"{type(self).__name__!r} object has no attribute {name!r}")
+
+    @property
+    def fusable(self):
+        """Whether products take a kernel of their own (``fused``, asked without changing the form a tensor is held in)."""
+        return self._planes is not None or self.fused is not None
+
+    def _hold_planes(self, words):
+        import torch
+        planes = _planes.Planes.of_words(words, self._launch)
+        torch.cuda.current_stream(self.device).synchronize()  # (a first product may be on another stream)
+        self.resident_bytes = planes.nbytes + self.error.numel() * self.error.element_size()
+        self._planes = planes
+
+    def take_planes(self):
+        """Puts a tensor that is walked into planes, for a launch with others that are held so; one whose arrays were
+        asked for stays as it is, and so does one that could not be held so."""
+        import torch
+        with _form_lock:
+            if self._planes is None and self._sections is not None and self.fused is not None:
+                self._hold_planes(self.decode(check=False).view(torch.int16))
+                for name in HipContextTensor._STREAM_FORM:
+                    self.__dict__.pop(name, None)
+        return self._planes is not None
+
+    def _leave_planes(self):
+        """The frame's arrays in the planes' place: the words, coded once more with the frame's own labels and frequencies,
+        which gives the same main stream, and packed residuals, the form that the walk takes."""
+        import zlib
+        import torch
+        words = self.decode(check=False).view(torch.int16).cpu().numpy().view(np.uint16)
+        meta, tables = self._sections
+        labels = base._inflate_exact(meta, sum(self.shape))
+        rows, columns = (np.frombuffer(part, dtype=np.uint8) for part in (labels[:self.shape[0]], labels[self.shape[0]:]))
+        frequencies = zlib.decompress(tables)[:self.nr * self.nc * base.MAIN_VOCAB * 4]
+        lib = base._lib()
+        main = base._encode_stream(lib, words, rows, columns, self.nr, self.nc, 0, frequencies)
+        frame = base._sealed(base._sections(0, self.nr, self.nc, *self.shape, meta, zlib.compress(frequencies, 1), main, base._pack6(lib, words),
+                                            b"", bytes.fromhex(self.source_sha256)))
+        segment = _fused.choose_segment(self.shape[1], self.asked_segment, rows=self.shape[0])
+        self._hold_streams(_stream_arrays(_read_frame(frame, self.stride, segment, True), True, self._block))
+        self._plan_gather()
+        self._planes = self._sections = None
+
+    def _hold_streams(self, prepared):
+        """The device arrays of a frame that is walked where it lies."""
+        import torch
+        indexed, plan = prepared["indexed"], prepared["plan"]
+        self._gather = None  # (lanes, piece capacity) of the row gather once planned; False: not possible
         self.fused = None
         self.fused_reason = prepared["reason"]
         self._main_bytes = prepared["main_bytes"]
         self._raw6_segment, self._raw6_block = prepared["raw6_segment"], prepared["raw6_block"]
+        buffers = _Buffers()
         for name, array in indexed.items():
             if isinstance(array, np.ndarray):
-                self.buffers[name] = torch.from_numpy(np.ascontiguousarray(array)).to(self.device)
+                buffers[name] = torch.from_numpy(np.ascontiguousarray(array)).to(self.device)
         for name in ("main", "residual"):
             if name + "_freq" in indexed:
                 cum = _tables.cumulative(indexed[name + "_freq"])
-                self.buffers[name + "_cum"] = torch.from_numpy(cum).to(self.device)
-                self.buffers[name + "_bucket"] = torch.from_numpy(_tables.coarse_buckets(cum)).to(self.device)
+                buffers[name + "_cum"] = torch.from_numpy(cum).to(self.device)
+                buffers[name + "_bucket"] = torch.from_numpy(_tables.coarse_buckets(cum)).to(self.device)
         if self._raw6_segment and GEMV_WAVES:  # (the slab kernels' read-ahead is for packed fields)
-            self.buffers["residual_pairs"] = _residual_form(self.buffers.pop("residual_stream"), True)
+            buffers["residual_pairs"] = _residual_form(buffers.pop("residual_stream"), True)
             torch.cuda.current_stream(self.device).synchronize()  # (a first product may be on another stream)
-        self.error = torch.zeros((), device=self.device, dtype=torch.int32)
+        self.buffers = buffers
         self.resident_bytes = int(sum(t.numel() * t.element_size() for t in self.buffers.values())
                                   + self.error.numel() * self.error.element_size())
         self._plan = plan
@@ -529,6 +654,14 @@ class HipContextTensor:
         import copy
         import torch
         other = copy.copy(self)
+        if self._planes is not None:
+            if residual_block is not None:
+                if residual_block not in (1, 2, 4, 8, 16):
+                    raise ValueError("residual blocks have 1, 2, 4, 8 or 16 rows")
+                other._block = residual_block
+            other._planes = self._planes.clone()
+            other.error = torch.zeros_like(self.error)
+            return other
         other.buffers = _Buffers((k, v.clone()) for k, v in self.buffers.items())
         if residual_block is not None and self._raw6_segment and residual_block != self._raw6_block:
             if residual_block not in (1, 2, 4, 8, 16):
@@ -642,6 +775,10 @@ class HipContextTensor:
         """Dense BF16 matrix.  Fused frames use the store sink of the fused walker;
         ``general=True`` forces the one-lane-per-segment kernel."""
         import torch
+        if self._planes is not None and not general:
+            out = torch.empty(self.shape, device=self.device, dtype=torch.bfloat16)
+            self._launch(self._lib.grf_planes_decode, self._planes.address, out.data_ptr())
+            return out
         if self.mode == 1:
             return self.buffers["raw"].view(torch.bfloat16).reshape(self.shape)
         if self.fused is None or general:
@@ -719,9 +856,42 @@ class HipContextTensor:
                 self._check(check)
         return y
 
+    def _planes_call(self, x, bias):
+        """A product of a tensor that is held as planes, of any number of rows; a row's bits depend on neither
+        the batch nor the call.  (Nothing is walked, so there is no checkpoint to miss.)"""
+        import torch
+        rows, cols = self.shape
+        p, packed = self._planes, isinstance(x, PackedActivations)
+        if packed:
+            if x.cols != cols or x.buffer.device != self.device:
+                raise ValueError("packed activations of another width or device")
+            lead, m, ldx, x2 = x.lead, x.rows, cols, x.buffer
+            y = self.error.new_empty((*lead, rows), dtype=torch.bfloat16)
+        else:
+            if x.dtype is not torch.bfloat16 or x.shape[-1] != cols:
+                raise ValueError("activation must be bfloat16 with the weight's input width")
+            x2, ldx = rows_for(x, cols, self._index, self.device)
+            if not cols <= ldx <= 1 << 24:  # (rows that overlap, or lie too far apart)
+                x2, ldx = x2.reshape(-1, cols).clone(memory_format=torch.contiguous_format), cols
+            m = x2.numel() // cols
+            y = x2.new_empty((*x.shape[:-1], rows))
+        if m:
+            bias = bias_for(bias, self._index, self.device)
+            size = p.workspace(m) if m > _planes.IN_PLACE_ROWS else 0
+            space = self.error.new_empty(size // 4) if size else None
+            status = launch_on(self._index, self._lib.grf_planes_linear, p.address, x2.data_ptr(), ldx, m, packed, y.data_ptr(),
+                               bias.data_ptr() if bias is not None else None, space.data_ptr() if size else None, size)
+            if status:
+                self._raise_launch(status)
+        return y
+
     def gemv(self, x, bias=None, *, check=False):
         """Fused decode-GEMV (vector ALUs) for 1..8 activation rows; the result of a row does
         not depend on how many rows the call carries."""
+        if self._planes is not None:
+            if not 1 <= (x.numel() // x.shape[-1] if x.shape[-1] else 0) <= 8:
+                raise ValueError("gemv takes 1..8 activation rows")
+            return self._planes_call(x, bias)
         if self.fused is None:
             raise base.CodecError("frame is not eligible for the fused kernels: " + self.fused_reason)
         m = x.numel() // x.shape[-1] if x.shape[-1] else 0
@@ -732,6 +902,8 @@ class HipContextTensor:
     def gemm(self, x, bias=None, *, check=False):
         """Fused decode-GEMM (matrix cores) for any number of activation rows, batch-invariant:
         a row's output bits are the same whatever else is in the batch."""
+        if self._planes is not None:
+            return self._planes_call(x, bias)
         if self.fused is None:
             raise base.CodecError("frame is not eligible for the fused kernels: " + self.fused_reason)
         if isinstance(x, PackedActivations):
@@ -757,11 +929,14 @@ class HipContextTensor:
             batch_invariant = self.m_invariant
         width = x.shape[-1]
         m = x.numel() // width if width else math.prod(x.shape[:-1])
-        route = "dense" if self.fused is None else route_rows(m, self.shape[1], batch_invariant)
+        held = self._planes is not None
+        if held and (m <= DENSE_ABOVE or batch_invariant):
+            return self._planes_call(x, bias)
+        route = "dense" if held or self.fused is None else route_rows(m, self.shape[1], batch_invariant)
         if route == "dense":
             import torch
             x, weight = x.to(self.device), self.decode(check=check)
-            if self.fused is None:  # any number of rows, and another decode (or none) than the product's plan counts on
+            if not held and self.fused is None:  # any number of rows, and another decode (or none) than the product's plan counts on
                 return torch.nn.functional.linear(x, weight, bias)
             return dense_linear(self._lib, x, weight, bias, self._index)
         if route == "gemm":
@@ -781,13 +956,9 @@ class HipContextTensor:
             ids = ids.to(device=self.device, dtype=torch.int64)
         if ids.numel() == 0:
             return torch.empty((*ids.shape, self.shape[1]), device=self.device, dtype=torch.bfloat16)
-        if self.fused is not None and self._gather is None:
-            try:
-                shape = self._plan.gather_shape()
-                self._gather_waves = min(16, -(-self.fused.segs_per_row // shape[0]))
-                self._gather = shape  # (last: another thread goes by it)
-            except _fused.FusedUnsupported:
-                self._gather = False
+        if self._planes is not None:
+            return self._gather_planes(ids, validate)
+        self._plan_gather()
         if self.fused is not None and self._gather:
             return self._gather_fused(ids, check, validate)
         if validate:
@@ -800,6 +971,15 @@ class HipContextTensor:
         per_row = self.shape[1] // self.stride
         blocks = (ids.reshape(-1, 1) * per_row + torch.arange(per_row, device=self.device)).reshape(-1)
         return self._decode_blocks(blocks, check=check).reshape(*ids.shape, self.shape[1])
+
+    def _plan_gather(self):
+        if self.fused is not None and self._gather is None:
+            try:
+                shape = self._plan.gather_shape()
+                self._gather_waves = min(16, -(-self.fused.segs_per_row // shape[0]))
+                self._gather = shape  # (last: another thread goes by it)
+            except _fused.FusedUnsupported:
+                self._gather = False
 
     def _gather_fused(self, ids, check, validate):
         """One launch, which also looks up classes and tests the ids; what it finds wrong it writes to a word of
@@ -820,17 +1000,31 @@ class HipContextTensor:
         if not (check or validate):
             self._launch(self._lib.grf_bctx_gather_rows, *about, self.error.data_ptr(), None)
             return out
-        polled = gather_polled(ids.numel(), self._gather_waves)
-        word, counters = _host_word(), _counters_for(self._index) if polled else None
-        where = word.data_ptr()
-        report = where if check else self.error.data_ptr(), where if validate else None
-        try:
-            if polled:
+
+        def launch(where, counters):
+            report = where if check else self.error.data_ptr(), where if validate else None
+            if counters is not None:
                 self._launch(self._lib.grf_bctx_gather_rows_done, *about, *report, counters.data_ptr(), where)
-                found = self._lib.grf_take_word(where, _hip_abi.GATHER_DONE, GATHER_SPIN_US)
             else:
                 self._launch(self._lib.grf_bctx_gather_rows, *about, *report)
-                found = 0
+
+        found = self._told(launch, gather_polled(ids.numel(), self._gather_waves))
+        if found & _hip_abi.ERR_INDEX:
+            raise IndexError("embedding row outside tensor")
+        if found:
+            self.error.fill_(found)
+            self._error_open = True
+            raise base.CodecError("HIP decoder checkpoint mismatch")
+        return out
+
+    def _told(self, launch, polled):
+        """What a lookup reports, once it is over: ``launch(address of the word, counters or None)`` starts it."""
+        import torch
+        word, counters = _host_word(), _counters_for(self._index) if polled else None
+        where = word.data_ptr()
+        try:
+            launch(where, counters)
+            found = self._lib.grf_take_word(where, _hip_abi.GATHER_DONE, GATHER_SPIN_US) if polled else 0
             if not found:
                 torch.cuda.current_stream(self._index).synchronize()
                 value = ctypes.c_int32.from_address(where)  # (a tensor's element costs twice the time)
@@ -838,17 +1032,25 @@ class HipContextTensor:
         except BaseException:
             _left_behind.append((word, counters))
             raise
-        found &= ~_hip_abi.GATHER_DONE
         if len(_host_words) < HOST_WORDS_KEPT:
             _host_words.append(word)
         if polled and len(_done_counters[self._index]) < HOST_WORDS_KEPT:
             _done_counters[self._index].append(counters)
-        if found & _hip_abi.ERR_INDEX:
+        return found & ~_hip_abi.GATHER_DONE
+
+    def _gather_planes(self, ids, validate):
+        """Of a tensor that is held as planes: one launch, of whose findings only refused ids are left to wait for."""
+        import torch
+        ids = ids.contiguous()
+        out = torch.empty((*ids.shape, self.shape[1]), device=self.device, dtype=torch.bfloat16)
+        about = self._planes.address, ids.data_ptr(), ids.numel(), out.data_ptr()
+        launch = lambda where, counters: self._launch(self._lib.grf_planes_gather, *about, where,
+                                                      counters.data_ptr() if counters is not None else None,
+                                                      where if counters is not None else None)
+        if not validate:
+            launch(None, None)
+        elif self._told(launch, gather_polled(ids.numel(), -(-_planes.visits(self.shape[1]) // 16))):
             raise IndexError("embedding row outside tensor")
-        if found:
-            self.error.fill_(found)
-            self._error_open = True
-            raise base.CodecError("HIP decoder checkpoint mismatch")
         return out
 
 
@@ -867,7 +1069,7 @@ class HipLinearGroup:
             raise ValueError("a group has 1..4 members")
         first = self.tensors[0]
         for t in self.tensors:
-            if t.fused is None:
+            if not t.fusable:
                 raise base.CodecError("frame is not eligible for the fused kernels: " + t.fused_reason)
             if t.shape[1] != first.shape[1] or t.device != first.device:
                 raise ValueError("group members need one width and one device")
@@ -879,6 +1081,14 @@ class HipLinearGroup:
         self.m_invariant = any(t.m_invariant for t in self.tensors) if m_invariant is None else bool(m_invariant)
         self.error = torch.zeros((), device=self.device, dtype=torch.int32)
         self._tilings, self._pointer_arrays, self._workspace = {}, {}, {}
+        self._walked = None  # (members whose frames are walked, their group) where some are held as planes
+        if any(t._planes is not None for t in self.tensors):  # (two kinds of members are two launches)
+            for t in self.tensors:
+                t.take_planes()
+        else:
+            self._plan_tilings()
+
+    def _plan_tilings(self):
         for key in (1, 2, "gemm"):
             self._tiling(key)  # raises FusedUnsupported when the members cannot share a tiling
 
@@ -941,6 +1151,9 @@ class HipLinearGroup:
         if route == "dense":
             return [t.linear(x, b, check=check, batch_invariant=False)
                     for t, b in zip(self.tensors, biases if biases is not None else [None] * n)]
+        planes = [t._planes for t in self.tensors]
+        if any(p is not None for p in planes):
+            return self._linear_planes(planes, x, m, lead, biases, check, batch_invariant)
         if packed is not None:
             if packed.cols != cols or packed.buffer.device != self.device:
                 raise ValueError("packed activations of another width or device")
@@ -977,6 +1190,54 @@ class HipLinearGroup:
                                       + self._lib.grf_last_error().decode(errors="replace"))
             if check and self.error.item() != 0:
                 raise base.CodecError("HIP decoder checkpoint mismatch")
+        return outs
+
+
+    def _linear_planes(self, planes, x, m, lead, biases, check, batch_invariant):
+        """Up to 128 rows of a group some of whose members are held as planes: one launch for those, and one for the rest."""
+        import torch
+        n, outs = len(planes), [None] * len(planes)
+        held = [i for i in range(n) if planes[i] is not None]
+        if len(held) < n:
+            rest = [i for i in range(n) if planes[i] is None]
+            if self._walked is None or self._walked[0] != rest:
+                self._walked = rest, HipLinearGroup([self.tensors[i] for i in rest], m_invariant=self.m_invariant)
+            walked = self._walked[1].linear(x, [biases[i] for i in rest] if biases is not None else None, check=check,
+                                            batch_invariant=batch_invariant)
+            for i, y in zip(rest, walked):
+                outs[i] = y
+        cols, packed = self.tensors[0].shape[1], isinstance(x, PackedActivations)
+        if packed:
+            if x.cols != cols or x.buffer.device != self.device:
+                raise ValueError("packed activations of another width or device")
+            x2, ldx = x.buffer, cols
+        else:
+            if x.dtype is not torch.bfloat16 or x.shape[-1] != cols:
+                raise ValueError("activation must be bfloat16 with the weights' input width")
+            x2, ldx = rows_for(x, cols, self._index, self.device)
+            if not cols <= ldx <= 1 << 24:  # (rows that overlap, or lie too far apart)
+                x2, ldx = x2.reshape(-1, cols).clone(memory_format=torch.contiguous_format), cols
+        for i in held:
+            outs[i] = self.error.new_empty((*lead, self.tensors[i].shape[0]), dtype=torch.bfloat16)
+        if m:
+            count = len(held)
+            biases = [bias_for(biases[i], self._index, self.device) for i in held] if biases is not None else None
+            kept = self._pointer_arrays.get("planes")
+            if kept is None or kept[0] != [planes[i].address for i in held]:
+                kept = self._pointer_arrays["planes"] = (
+                    [planes[i].address for i in held], (ctypes.c_void_p * count)(*[planes[i].address for i in held]),
+                    (ctypes.c_uint32 * count)(*[planes[i].rows for i in held]), ctypes.c_void_p * count)
+            _, members, ldy, pointers = kept
+            size = 0
+            if m > _planes.IN_PLACE_ROWS:
+                size = sum(planes[i].workspace(m) for i in held)
+            space = self.error.new_empty(size // 4) if size else None
+            status = launch_on(self._index, self._lib.grf_planes_group, count, members, x2.data_ptr(), ldx, m, packed,
+                               pointers(*[outs[i].data_ptr() for i in held]), ldy,
+                               pointers(*[b.data_ptr() if b is not None else None for b in biases]) if biases is not None else None,
+                               space.data_ptr() if size else None, size)
+            if status:
+                raise base.CodecError(f"device launch failed ({status}): " + self._lib.grf_last_error().decode(errors="replace"))
         return outs
 
 

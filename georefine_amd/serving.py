@@ -656,7 +656,7 @@ def load_bctx_model(package, *, model_factory, device="cuda:0", dtype=torch.bflo
         native = getattr(context, "row_major", None) or getattr(context, "native", context)
         if not hasattr(native, "resident_mode"):
             return {}
-        fused = getattr(native, "fused", None) is not None
+        fused = native.fusable if hasattr(native, "fusable") else getattr(native, "fused", None) is not None
         reason = getattr(native, "fused_reason", "")
         return dict(frame_mode=native.mode, resident_mode=native.resident_mode,
                     residual_repacked=native.resident_mode != native.mode, fused=fused,

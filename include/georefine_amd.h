@@ -558,6 +558,56 @@ int grf_dense_gemm(const uint16_t *w, uint32_t rows, uint32_t cols, const uint16
                    uint16_t *y, uint32_t ldy, const uint16_t *bias, void *workspace, size_t workspace_bytes,
                    void *hip_stream);
 
+/* A matrix resident as planes: what a context frame decodes to, laid out once at load at fixed places (11.5 bits a weight:
+ * signs and mantissas as they are, exponents two to seven bits, and a list of the words outside the eleven exponents that
+ * hold most of their row; csrc/word_planes.h has the places).  It takes the memory of the frame with its index, and
+ * products, decode and lookups go at the memory's pace where the walk of a frame's states goes at the vector ALUs'.
+ * The reference's servers lay their context weights out anew at start-up as well (GS/predictive_tbe.py:1-15).
+ *   planes     grf_planes_bytes(rows, cols) bytes, 16-byte aligned
+ *   bases      u32 [rows in whole sixteens]: a row's lowest exponent << 7, in both halves
+ *   listed_at  u32 [grf_planes_visits(rows, cols) + 1]: where a visit's listed words begin
+ *   listed     u32 [listed_at's last + 1]: place in the visit << 16 | word
+ *   splits     1 to 16 waves that share the visits of sixteen rows in a product, at most 63 each
+ *   parts      divides splits; the sums of a part's splits are added in their order, then the parts: the order of a product's
+ *              sums, in which nothing else has a part.
+ * cols is a multiple of 8 and at most GRF_PLANES_MAX_COLS.
+ *
+ * grf_planes_count  bases of a dense BF16 matrix (16-byte aligned), and counts u32 [grf_planes_visits]: the words
+ *                   a visit will list, whose running sum listed_at is
+ * grf_planes_fill   planes and list, given those
+ * grf_planes_linear, _group  y = x W^T (+ bias) for any number of rows and up to four matrices of one width:
+ *                   fp32 sums in an order that the matrix's sizes and splits fix, so that a row has the same bits in every
+ *                   batch and group.  workspace: grf_planes_workspace_bytes, 16-byte aligned.  x: 16-byte aligned, ldx a multiple of 8; or, with `packed`, up to 128 rows as
+ *                   grf_pack_activations leaves them
+ * grf_planes_decode the words, dense
+ * grf_planes_gather rows by index as grf_bctx_gather_rows takes and reports them; with `done` as
+ *                   grf_bctx_gather_rows_done.
+ * They allocate nothing and can be captured. */
+#define GRF_PLANES_MAX_COLS (1u << 17)
+typedef struct grf_planes {
+  const uint8_t *planes;
+  const uint32_t *bases;
+  const uint32_t *listed_at;
+  const uint32_t *listed;
+  uint32_t rows, cols;
+  uint32_t splits, parts;
+} grf_planes;
+
+uint64_t grf_planes_bytes(uint32_t rows, uint32_t cols);
+uint32_t grf_planes_visits(uint32_t rows, uint32_t cols);
+int grf_planes_count(const uint16_t *words, uint32_t rows, uint32_t cols, uint32_t *bases, uint32_t *counts, void *hip_stream);
+int grf_planes_fill(const uint16_t *words, uint32_t rows, uint32_t cols, const uint32_t *bases, const uint32_t *listed_at, void *planes,
+                    uint32_t *listed, void *hip_stream);
+size_t grf_planes_workspace_bytes(uint32_t n, const grf_planes *const *planes, uint32_t m_rows);
+int grf_planes_linear(const grf_planes *planes, const uint16_t *x, uint32_t ldx, uint32_t m_rows, uint32_t packed, uint16_t *y,
+                      const uint16_t *bias, void *workspace, size_t workspace_bytes, void *hip_stream);
+int grf_planes_group(uint32_t n, const grf_planes *const *planes, const uint16_t *x, uint32_t ldx, uint32_t m_rows, uint32_t packed,
+                     uint16_t *const *y, const uint32_t *ldy, const uint16_t *const *bias, void *workspace, size_t workspace_bytes,
+                     void *hip_stream);
+int grf_planes_decode(const grf_planes *planes, uint16_t *out, void *hip_stream);
+int grf_planes_gather(const grf_planes *planes, const int64_t *ids, uint32_t count, uint16_t *out, int32_t *index_error, void *counters,
+                      int32_t *done, void *hip_stream);
+
 /* A one-lane kernel that writes slot[0] = the device's constant-rate counter
  * (grf_wall_clock_khz), slot[1] = its shader-clock counter and slot[2] = the identifier of the
  * compute unit it ran on, all read when the kernel runs, i.e. in stream order after the work

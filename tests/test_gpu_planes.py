@@ -1,0 +1,181 @@
+"""Matrices held as planes: every sink against the words they were laid out from."""
+import numpy as np
+import pytest
+
+from conftest import bf16_words, weight_like
+
+pytestmark = pytest.mark.gpu
+
+
+def _launch(fn, *args):
+    import torch
+    assert fn(*args, torch.cuda.current_stream().cuda_stream) == 0
+
+
+def _planes(words):
+    import torch
+    from georefine_amd._planes import Planes
+    return Planes.of_words(torch.from_numpy(words.view(np.int16)).cuda(), _launch)
+
+
+def _words(kind, rows, cols, seed):
+    rng = np.random.default_rng(seed)
+    if kind == "any":  # every bit pattern: most words are listed
+        return rng.integers(0, 1 << 16, (rows, cols)).astype(np.uint16)
+    words = weight_like(rng, rows, cols)
+    words[rng.random((rows, cols)) < 0.01] = 0
+    words.flat[rng.integers(0, words.size, 6)] = (0x7F80, 0xFF80, 0x7FC1, 0x0001, 0x8000, 0x7F7F)
+    return words
+
+
+SHAPES = [(1, 16), (16, 64), (15, 256), (17, 240), (33, 272), (16, 448), (100, 4096), (31, 4112), (257, 1040), (40, 17408)]
+
+
+@pytest.mark.parametrize("kind", ["weights", "any"])
+@pytest.mark.parametrize("rows,cols", SHAPES)
+def test_words_and_rows_come_back_and_nothing_around_them_is_written(rows, cols, kind):
+    import torch
+    from georefine_amd import _native
+    lib, words = _native.hip(), _words(kind, rows, cols, rows + cols)
+    p = _planes(words)
+    around = torch.full((rows * cols + 256,), 0x5A5A, device="cuda", dtype=torch.int16)
+    _launch(lib.grf_planes_decode, p.address, around.data_ptr() + 256)
+    got = around.cpu().numpy().view(np.uint16)
+    assert np.array_equal(got[128:-128].reshape(rows, cols), words)
+    assert np.all(got[:128] == 0x5A5A) and np.all(got[-128:] == 0x5A5A)
+    ids = torch.from_numpy(np.random.default_rng(1).integers(0, rows, 19)).cuda()
+    out = torch.full((21, cols), 0x5A5A, device="cuda", dtype=torch.int16)
+    _launch(lib.grf_planes_gather, p.address, ids.data_ptr(), 19, out[1:].data_ptr(), None, None, None)
+    got = out.cpu().numpy().view(np.uint16)
+    assert np.array_equal(got[1:-1], words[ids.cpu().numpy()]) and np.all(got[0] == 0x5A5A) and np.all(got[-1] == 0x5A5A)
+
+
+@pytest.mark.parametrize("splits,parts", [(1, 1), (2, 1), (2, 2), (4, 2), (8, 4)])
+@pytest.mark.parametrize("rows,cols", SHAPES)
+def test_products_against_float64_with_one_set_of_bits_a_row(rows, cols, splits, parts):
+    import torch
+    from georefine_amd import _hip_abi, _native
+    from georefine_amd._planes import visits
+    from georefine_amd.bitexact_context_gpu import PackedActivations
+    if not (splits - 1) * -(-visits(cols) // splits) < visits(cols) <= 63 * splits:
+        pytest.skip("splits of 1 to 63 visits")
+    lib, rng = _native.hip(), np.random.default_rng(rows)
+    words = weight_like(rng, rows, cols)
+    words[rng.random((rows, cols)) < 0.02] = 0  # (listed)
+    p = _planes(words)
+    p.struct.splits, p.struct.parts = splits, parts
+    around = torch.full((130, cols + 8), float("nan"), device="cuda", dtype=torch.bfloat16)
+    x = around[1:129, :cols]  # rows apart, with what must not be read around them
+    x.copy_(torch.from_numpy(rng.standard_normal((128, cols), dtype=np.float32)))
+    bias = torch.from_numpy(rng.standard_normal(rows, dtype=np.float32)).cuda().bfloat16()
+    space = torch.empty(parts * 128 * rows + 64, device="cuda", dtype=torch.float32)
+
+    def product(rows_of_x, m, packed=0, b=None):
+        y = torch.full((m + 2, rows), 7.0, device="cuda", dtype=torch.bfloat16)
+        _launch(lib.grf_planes_linear, p.address, rows_of_x.data_ptr(), cols + 8, m, packed, y[1:].data_ptr(),
+                b.data_ptr() if b is not None else None, space.data_ptr(), space.numel() * 4)
+        assert bool((y[0] == 7).all() and (y[-1] == 7).all())
+        return y[1:-1]
+
+    full, shifted = product(x, 128), product(x, 128, b=bias)
+    w, xd = torch.from_numpy((words.astype(np.uint32) << 16).view(np.float32)).double(), x.cpu().double()
+    for got, exact in ((full, xd @ w.T), (shifted, xd @ w.T + bias.cpu().double())):
+        # one rounding to BF16 (2^-9 of the value) and cols additions of fp32, each 2^-24 of the sum of magnitudes
+        bound = exact.abs() * 2.0 ** -8 + (xd.abs() @ w.abs().T + 8) * cols * 2.0 ** -24
+        assert bool(((got.cpu().double() - exact).abs() <= bound).all())
+    for m in (1, 15, 16, 17, 32, 33, 64, 65, 127):
+        assert torch.equal(product(x, m), full[:m]), m
+        xp = PackedActivations(x[:m])
+        assert torch.equal(product(xp.buffer, m, packed=1), full[:m]), m
+
+
+def test_infinities_and_nan_go_where_the_dense_product_puts_them():
+    import torch
+    from georefine_amd import _native
+    rng = np.random.default_rng(8)
+    words = weight_like(rng, 40, 544) & 0x7FFF  # positive: an infinite activation gives no NaN
+    words[3, 500], words[5, 7], words[6, 100], words[7, :] = 0x7F80, 0x7FC0, 0, 0x3F80
+    p = _planes(words)
+    dense = torch.from_numpy(words.view(np.int16)).view(torch.bfloat16).cuda()
+    space = torch.empty(1 << 16, device="cuda", dtype=torch.float32)
+    for m in (1, 20, 64, 70):
+        x = torch.from_numpy(rng.random((m, 544), dtype=np.float32) + 0.5).cuda().bfloat16()
+        x[0, 100] = float("inf")
+        x[m - 1, 543] = float("nan") if m > 1 else x[0, 543]
+        y = torch.empty(m, 40, device="cuda", dtype=torch.bfloat16)
+        _launch(_native.hip().grf_planes_linear, p.address, x.data_ptr(), 544, m, 0, y.data_ptr(), None, space.data_ptr(), space.numel() * 4)
+        want = x.double() @ dense.double().T
+        for state in (torch.isnan, torch.isposinf, torch.isneginf):
+            assert torch.equal(state(y), state(want)), (m, state)
+
+
+def test_a_tensor_answers_as_planes_and_leaves_them_when_its_arrays_are_asked_for():
+    import torch
+    from georefine_amd import bitexact_context_codec as codec
+    from georefine_amd.bitexact_context_gpu import HipContextTensor, HipLinearGroup
+    rng = np.random.default_rng(12)
+    words = weight_like(rng, 700, 1040)
+    for residual in ("auto", "raw6"):
+        frame = codec.encode(words, residual=residual)
+        t = HipContextTensor(frame)
+        assert t.fusable and t._planes is not None and t.fused_reason == ""
+        other, small = t.clone(residual_block=16), HipContextTensor(codec.encode(weight_like(rng, 48, 1040)))
+        assert small._planes is None
+        ids = torch.tensor([3, 40])
+        rows_of_small = small.gather_rows(ids)
+        group = HipLinearGroup([t, small, other])
+        assert small._planes is not None and torch.equal(small.gather_rows(ids).view(torch.int16), rows_of_small.view(torch.int16))
+        x = torch.from_numpy(bf16_words(rng.normal(0, 1, (140, 1040)))).view(torch.bfloat16).cuda()
+        for m in (1, 2, 20, 128, 140):
+            want = t.linear(x[:m], batch_invariant=True)
+            assert torch.equal(t.linear(x[:m], batch_invariant=True, check=True), want)
+            got = group.linear(x[:m], batch_invariant=True)
+            assert torch.equal(got[0], want) and torch.equal(got[2], want)
+            assert torch.equal(got[1], small.linear(x[:m], batch_invariant=True))
+        ids = torch.tensor([[0, 699], [5, 5]])
+        assert np.array_equal(t.gather_rows(ids).view(torch.int16).cpu().numpy().view(np.uint16), words[ids.numpy()])
+        for bad in (-1, 700):
+            with pytest.raises(IndexError):
+                t.gather_rows(torch.tensor([3, bad]))
+            last = t.gather_rows(torch.tensor([3, bad]), check=False, validate=False)[1]
+            assert np.array_equal(last.view(torch.int16).cpu().numpy().view(np.uint16), words[0 if bad < 0 else 699])
+        as_planes = t.resident_bytes
+        assert other.resident_bytes == as_planes and t._planes is not None
+        streams = HipContextTensor.host_prepare(frame)["indexed"]
+        assert t.fused is not None and t._planes is None  # the frame's arrays, the same as it had held from the start
+        for name in ("main_stream", "rows", "columns", "main_freq", "fused_seg_state", "fused_seg_offset", "residual_stream"):
+            assert np.array_equal(t.buffers[name].cpu().numpy()[:streams[name].size], streams[name]), name
+        assert t.mode == frame[5] and t.frame_bytes == len(frame) and other._planes is not None
+        assert np.array_equal(t.decode().view(torch.int16).cpu().numpy().view(np.uint16), words)
+        assert not t.take_planes()
+        mixed, walked = group.linear(x[:20]), HipLinearGroup([t]).linear(x[:20])  # (two launches from here on)
+        assert torch.equal(mixed[0], walked[0]) and torch.equal(mixed[1], small.linear(x[:20])) and torch.equal(mixed[2], other.linear(x[:20]))
+        assert np.array_equal(other.decode(general=True).view(torch.int16).cpu().numpy().view(np.uint16), words) and other._raw6_block == 16
+
+
+def test_captured_launches_replay_on_new_rows():
+    import torch
+    from georefine_amd import bitexact_context_codec as codec
+    from georefine_amd.bitexact_context_gpu import HipContextTensor, HipLinearGroup
+    rng = np.random.default_rng(13)
+    t = HipContextTensor(codec.encode(weight_like(rng, 640, 1024)))
+    group = HipLinearGroup([t, t.clone()])
+    draw = lambda m: torch.from_numpy(bf16_words(rng.normal(0, 1, (m, 1024)))).view(torch.bfloat16).cuda()
+    x1, x40, ids = draw(1), draw(40), torch.from_numpy(rng.integers(0, 640, 33)).cuda()
+    step = lambda: [t.linear(x1), *group.linear(x40), t.decode(check=False), t.gather_rows(ids, check=False, validate=False)]
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        step()
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = step()
+    for _ in range(3):
+        x1.copy_(draw(1)), x40.copy_(draw(40)), ids.copy_(torch.from_numpy(rng.integers(0, 640, 33)))
+        eager = [v.clone() for v in step()]
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a.view(torch.int16), b.view(torch.int16)) for a, b in zip(captured, eager))

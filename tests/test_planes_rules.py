@@ -1,0 +1,64 @@
+"""Which matrices are held as planes, how their sums are split, and that the sizes agree with the library's (no GPU)."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from georefine_amd import _fused, _hip_abi, _native, _planes
+from georefine_amd import bitexact_context_codec as codec
+from georefine_amd.bitexact_context_gpu import HipContextTensor
+
+from conftest import weight_like
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 16), (16, 64), (17, 80), (255, 240), (1000, 256), (4097, 272), (5120, 17408), (64, 131072)])
+def test_sizes_are_the_librarys_and_no_split_is_empty(rows, cols):
+    lib = _native.hip()
+    assert _planes.plane_bytes(rows, cols) == lib.grf_planes_bytes(rows, cols)
+    assert -(-rows // 16) * _planes.visits(cols) == lib.grf_planes_visits(rows, cols)
+    splits, parts = _planes.sum_splits(rows, cols)
+    each = -(-_planes.visits(cols) // splits)
+    assert 1 <= splits <= 16 and splits % parts == 0 and splits // parts <= 2
+    assert (splits - 1) * each < _planes.visits(cols) and each <= 63
+
+
+@pytest.mark.parametrize("change", [dict(splits=0), dict(splits=17), dict(splits=4), dict(parts=0), dict(cols=1028), dict(cols=1 << 18), dict(rows=0),
+                                    dict(planes=8), dict(listed=None)])
+def test_what_the_kernels_would_not_take_is_refused_before_a_launch(change):
+    lib = _native.hip()
+    good = dict(planes=4096, bases=4096, listed_at=4096, listed=4096, rows=64, cols=1024, splits=2, parts=1)
+    if change.get("splits") == 4:
+        good.update(cols=1280)  # five visits, two a split: nothing is left for the fourth
+    p = _hip_abi.GrfPlanes(**{**good, **change})
+    assert lib.grf_planes_decode(ctypes.addressof(p), 4096, None) != 0 and b"grf_planes_decode" in lib.grf_last_error()
+    assert lib.grf_planes_linear(ctypes.addressof(p), 4096, 2048, 1, 0, 4096, None, None, 0, None) != 0
+
+
+def test_small_sparse_and_odd_frames_stay_frames():
+    rng = np.random.default_rng(3)
+    large = codec.encode(weight_like(rng, 512, 1024))
+    few = codec.encode((rng.choice([0x3C00, 0x3C20], (4096, 1024)) | rng.integers(0, 32, (4096, 1024))).astype(np.uint16))
+    assert "words" in HipContextTensor.host_prepare(large)
+    for frame, how in ((codec.encode(weight_like(rng, 511, 1024)), {}), (large, {"fused": False}), (few, {"fused_segment": 64})):
+        assert "words" not in HipContextTensor.host_prepare(frame, **how)
+
+
+def test_the_walks_arrays_are_made_when_asked_for_and_travel():
+    import pickle
+    words = weight_like(np.random.default_rng(4), 512, 1040)
+    prepared = HipContextTensor.host_prepare(codec.encode(words))
+    assert np.array_equal(prepared["words"].reshape(words.shape), words)
+    there = pickle.loads(pickle.dumps(prepared))
+    for p in (prepared, there):
+        assert isinstance(p["plan"], _fused.FramePlan) and p["raw6_segment"] == 16
+        assert p["indexed"]["main_stream"].flags.writeable
+        with pytest.raises(KeyError):
+            p["no such entry"]
+
+
+def test_listed_share_counts_what_is_outside_eleven_exponents():
+    freq = np.zeros((2, 1024), dtype=np.uint32)  # two row classes, one column class
+    freq[0, 4 * 100:4 * 111] = 1489  # eleven exponents
+    freq[0, 4 * 100] += 65536 - 44 * 1489
+    freq[1, 4 * 50] = freq[1, 4 * 80] = 32768
+    assert _planes.listed_share(np.array([0, 0, 0, 1]), np.zeros(7, dtype=np.uint8), freq, 2, 1) == pytest.approx(0.125)
