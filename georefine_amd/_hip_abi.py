@@ -62,7 +62,7 @@ class GrfPpcxFused(ctypes.Structure):
 
 class GrfPlanes(ctypes.Structure):
     _fields_ = [(name, ctypes.c_void_p) for name in ("planes", "bases", "listed_at", "listed")] + [
-        (name, ctypes.c_uint32) for name in ("rows", "cols", "splits", "parts")]
+        (name, ctypes.c_uint32) for name in ("rows", "cols", "splits")]
 
 
 ERR_INDEX = 16  # GRF_ERR_INDEX

@@ -4,8 +4,8 @@ The planes (``csrc/word_planes.h``, ``csrc/planes.hip``) hold a matrix's words a
 list of the few whose exponent is outside the eleven that hold most of their row.  A context frame with
 the index its walk needs takes as much (5120 x 17408 of normal weights with a scale a row: 11.6 bits either way;
 small matrices, whose index is finer and whose tables do not shrink, 13 to 30), and its walk is bound by the vector ALUs where the planes are
-read at the memory's pace.  us, walk / planes: one row of 17408 x 5120 twice 110 / 51, six of 5120 x 17408 69 / 37, 64 of the
-first 151 / 104, a decode of 5120 x 6144 39 / 25, 777 of 8192 rows looked up 16 / 7.
+read at the memory's pace.  us, walk / planes: one row of 17408 x 5120 twice 110 / 51, six of 5120 x 17408 69 / 36, 64 of the
+first 151 / 73, a decode of 5120 x 6144 39 / 25, 777 of 8192 rows looked up 16 / 7.
 """
 from __future__ import annotations
 
@@ -18,7 +18,7 @@ from . import _hip_abi, _native
 VISIT, UNIT, VISIT_BYTES, UNIT_BYTES = 256, 64, 5888, 1536  # csrc/word_planes.h
 EXPONENTS = 11
 MAX_COLS = 1 << 17
-IN_PLACE_ROWS = 16  # activation rows that a launch reads where they are and needs no workspace for
+OWN_ROWS = 8  # activation rows up to which no launch needs a workspace
 # Weights from which a matrix is laid out.  The kernels are the shorter below it too (one row of 512 x 640 4.4 us, walked 8.4;
 # 32 rows 8.6 and 8.2), but a call is as long as its host path there (502 x 640 at three rows 10.1 and 10.5), and a
 # tensor whose arrays are asked for changes the bits of its products, which the small ones that are looked at do not.
@@ -71,16 +71,21 @@ def worth(info, segment):
 
 
 def sum_splits(rows, cols):
-    """(splits, parts) of a product's sums (``grf_planes``), by the matrix's sizes alone: as few splits, in parts of
-    two, as give the GPU 3800 waves of up to sixteen rows, so that every member of a group of one width that is
-    not much smaller has the same number.  us for one and 64 rows by splits: 17408 x 5120 twice 2: 53 115, 4: 51 104;
-    5120 x 17408 6: 41 66, 8: 37 65, 12: 34 52; 6144, 1024 and 1024 x 5120 4, 10 and 10: 19 35, 10 each 15.5 37."""
+    """Splits of a product's sums (``grf_planes``), by the matrix's sizes alone.  A batch's workgroups, eight row blocks of one split
+    each, are dealt to 256 compute units: the busiest one's visits count (a lone workgroup there hides less: a quarter more),
+    and every split's sums go through memory, the more the more rows there are.  Large matrices, which come in pairs, have
+    two.  us for 1, 32 and 64 rows by splits: 17408 x 5120 twice 1: 50 73 86, 2: 52 62 75, 4: 49 67 85; 5120 x 17408 6: 34 44 49, 8: 32 41 48,
+    12: 34 39 46; 6144, 1024 and 1024 x 5120 4: 16 23 30, 5: 16 23 31, 7: 16 26 32; 1024 x 5120 5: 10 13 22, 10: 8 12 18."""
     v, blocks = visits(cols), -(-rows // 16)
-    fits = [s for s in range(2, 17, 2) if -(-v // s) * (s - 1) < v and -(-v // s) <= 63]
-    if not fits:
-        return 1, 1
-    s = next((s for s in fits if blocks * s >= 3800), fits[-1])
-    return s, s // 2
+    fits = [s for s in range(1, 17) if -(-v // s) * (s - 1) < v and -(-v // s) <= 63]
+    if blocks >= 768:
+        return next((s for s in fits if s >= (2 if blocks < 4096 else 1)), fits[-1])
+
+    def cost(s):
+        groups = -(-blocks // 8) * s
+        return -(-groups // 256) * -(-v // s) * (1.25 if groups <= 256 else 1) + s * (0.2 + blocks / 2560)
+
+    return min(fits, key=cost)
 
 
 class Planes:
@@ -90,8 +95,8 @@ class Planes:
 
     def __init__(self, rows, cols, arrays):
         self.rows, self.cols, self.arrays = rows, cols, arrays
-        self.splits, self.parts = sum_splits(rows, cols)
-        self.struct = _hip_abi.GrfPlanes(*(arrays[name].data_ptr() for name in self.ARRAYS), rows, cols, self.splits, self.parts)
+        self.splits = sum_splits(rows, cols)
+        self.struct = _hip_abi.GrfPlanes(*(arrays[name].data_ptr() for name in self.ARRAYS), rows, cols, self.splits)
         self.address = ctypes.addressof(self.struct)
         self.nbytes = sum(a.numel() * a.element_size() for a in arrays.values())
         self._workspace = {}

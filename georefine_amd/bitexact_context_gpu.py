@@ -877,7 +877,7 @@ class HipContextTensor:
             y = x2.new_empty((*x.shape[:-1], rows))
         if m:
             bias = bias_for(bias, self._index, self.device)
-            size = p.workspace(m) if m > _planes.IN_PLACE_ROWS else 0
+            size = p.workspace(m) if m > _planes.OWN_ROWS else 0
             space = self.error.new_empty(size // 4) if size else None
             status = launch_on(self._index, self._lib.grf_planes_linear, p.address, x2.data_ptr(), ldx, m, packed, y.data_ptr(),
                                bias.data_ptr() if bias is not None else None, space.data_ptr() if size else None, size)
@@ -1229,7 +1229,7 @@ class HipLinearGroup:
                     (ctypes.c_uint32 * count)(*[planes[i].rows for i in held]), ctypes.c_void_p * count)
             _, members, ldy, pointers = kept
             size = 0
-            if m > _planes.IN_PLACE_ROWS:
+            if m > _planes.OWN_ROWS:
                 size = sum(planes[i].workspace(m) for i in held)
             space = self.error.new_empty(size // 4) if size else None
             status = launch_on(self._index, self._lib.grf_planes_group, count, members, x2.data_ptr(), ldx, m, packed,

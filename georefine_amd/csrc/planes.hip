@@ -25,15 +25,18 @@ typedef uint16_t pair16 __attribute__((ext_vector_type(2)));
 
 constexpr uint32_t kMaxMembers = 4;
 constexpr uint32_t kMaxTileRows = 128;  // activation rows of a launch
-constexpr uint32_t kInPlaceRows = 16;   // up to which x is read where it is
-constexpr uint32_t kMaxSharing = 2;    // splits of a part
+// Rows of x up to which every wave brings its own: it needs no other wave and no second launch, but reads x once a row block where
+// four waves share it once in eight.  us, own and shared: one row 17408 x 5120 twice 52 and 57, 16 rows 65 and 58; 16 rows of 6144,
+// 1024 and 1024 x 5120 18 and 24, 32 rows 23 and 27; 32 rows of 5120 x 17408 64 and 39.
+constexpr uint32_t kOwnAlways = 8;                    // up to which it always does
+constexpr uint32_t kOwnRows = 32, kOwnVisits = 16384;  // and, in launches of fewer visits than that
 constexpr uint32_t kPatch = 4096;       // LDS bytes in which a wave's half visit is completed
 
 struct PlanesMember {
   grf_planes p;
   uint16_t *y;
   const uint16_t *bias;
-  float *partials;                   // [parts][activation rows][rows]
+  float *partials;                   // [splits][activation rows][rows]
   uint32_t ldy, first, blocks_each;  // first workgroup; row blocks a workgroup
 };
 
@@ -64,12 +67,15 @@ __device__ __forceinline__ void wave_order() {
 __device__ __forceinline__ void join_words(uint32_t s0, uint32_t s1, uint32_t first, uint32_t second, uint32_t base, uint32_t (&o)[4]) {
 #if defined(__HIP_DEVICE_COMPILE__)
   const pair16 b = __builtin_bit_cast(pair16, base);
+  uint32_t place = 0x00800080u;  // (as a constant it would be a shift and an addition in place of one multiply-add)
+  asm("" : "+s"(place));
+  const pair16 k = __builtin_bit_cast(pair16, place);
   auto two = [&](uint32_t codes, uint32_t s, uint32_t &low, uint32_t &high) {
     const pair16 p = __builtin_bit_cast(pair16, codes);
     const pair16 q = (p * (uint16_t)187) >> (uint16_t)11;  // p / 11 for p < 121
     const pair16 r = p - q * (uint16_t)11;
-    const uint32_t lo = __builtin_bit_cast(uint32_t, (pair16)(r * (uint16_t)128 + b));
-    const uint32_t hi = __builtin_bit_cast(uint32_t, (pair16)(q * (uint16_t)128 + b));
+    const uint32_t lo = __builtin_bit_cast(uint32_t, (pair16)(r * k + b));
+    const uint32_t hi = __builtin_bit_cast(uint32_t, (pair16)(q * k + b));
     low = (s & grf::kSignMantissa) | lo;
     high = (__builtin_amdgcn_alignbit(s, s, 8) & grf::kSignMantissa) | hi;
   };
@@ -80,20 +86,54 @@ __device__ __forceinline__ void join_words(uint32_t s0, uint32_t s1, uint32_t fi
 #endif
 }
 
+// A row block's whole visits [0, full), beyond which a load gives zeros and reads nothing: the visit after the last one is
+// asked for like the rest, and the loads under way are never waited for at a branch.
+struct VisitBytes {
+#if defined(__HIP_DEVICE_COMPILE__)
+  __amdgpu_buffer_rsrc_t bytes;
+  __device__ __forceinline__ VisitBytes(const uint8_t *block, uint32_t full)
+      : bytes(__builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(block), 0, (int)(full * grf::kVisitBytes), 0x00020000)) {}
+  __device__ __forceinline__ uint4v four(uint32_t at) const { return __builtin_bit_cast(uint4v, __builtin_amdgcn_raw_buffer_load_b128(bytes, at, 0, 0)); }
+  __device__ __forceinline__ uint3v three(uint32_t at) const { return __builtin_bit_cast(uint3v, __builtin_amdgcn_raw_buffer_load_b96(bytes, at, 0, 0)); }
+#else
+  __device__ VisitBytes(const uint8_t *, uint32_t) {}
+  __device__ uint4v four(uint32_t) const { return {}; }
+  __device__ uint3v three(uint32_t) const { return {}; }
+#endif
+};
+
 // What a lane holds of a visit.
-struct Visit {
-  uint4v s[4];  // steps 2 j and 2 j + 1
+struct Exponents {
   uint4v e0;
   uint3v e1;
+  __device__ __forceinline__ void load(const VisitBytes &from, uint32_t v, uint32_t slot) {
+    e0 = from.four(v * grf::kVisitBytes + 4096 + slot * 16);
+    e1 = from.three(v * grf::kVisitBytes + 5120 + slot * 12);
+  }
+};
+
+struct Visit {
+  uint4v s[4];  // steps 2 j and 2 j + 1
+  Exponents e;
   __device__ __forceinline__ void load(const uint8_t *at, uint32_t slot) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) s[j] = *reinterpret_cast<const uint4v *>(at + j * 1024 + slot * 16);
-    e0 = *reinterpret_cast<const uint4v *>(at + 4096 + slot * 16);
-    e1 = *reinterpret_cast<const uint3v *>(at + 5120 + slot * 12);
+    e.e0 = *reinterpret_cast<const uint4v *>(at + 4096 + slot * 16);
+    e.e1 = *reinterpret_cast<const uint3v *>(at + 5120 + slot * 12);
+  }
+  __device__ __forceinline__ void load_signs(const VisitBytes &from, uint32_t v, uint32_t j, uint32_t slot) {
+    s[j] = from.four(v * grf::kVisitBytes + j * 1024 + slot * 16);
+  }
+  __device__ __forceinline__ void load(const VisitBytes &from, uint32_t v, uint32_t slot) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) load_signs(from, v, j, slot);
+    e.load(from, v, slot);
   }
   template <int T>
   __device__ __forceinline__ void step(uint32_t base, uint32_t (&o)[4]) const {
     constexpr uint32_t kCodes = grf::kCodeFields;
+    const uint4v &e0 = e.e0;
+    const uint3v &e1 = e.e1;
     uint32_t d;
     if constexpr (T < 4) {
       d = e0[T];
@@ -151,135 +191,224 @@ struct Listed {
 
 struct PlanesX {
   const uint8_t *data;
-  uint32_t row_bytes, chunk_bytes, m_rows, cols;  // bytes from a row to the next, from eight columns to the next
+  uint32_t row_bytes, chunk_bytes, m_rows, cols, packed;  // bytes from a row to the next, from eight columns to the next
 };
 
-// MT: tiles of sixteen activation rows.  A workgroup's waves share out the visits of `blocks_each` row blocks, `splits`
-// waves a block, and add their sums in wave order: what a row of x gives depends on nothing but the matrix's
-// sizes, so all row counts, single and grouped launches agree bit for bit.
-template <int MT>
-__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(6))) void planes_product_kernel(PlanesGroup g, PlanesX x) {
-  extern __shared__ __align__(16) uint8_t lds[];
+// Where a quarter of a visit, 64 columns, of x lies in LDS.  Copy i is eight rows, a line each: lane l brings sixteen bytes of row l / 8,
+// and which of the eight is turned by the row, so that the operand reads meet no bank twice.  (Sixteen rows a copy, in operand
+// order, are an access of its own a lane: TCP 92 accesses a KiB where lines take 16.)  Packed activations are in operand order as they are.
+struct XPlaces {
+  uint32_t first, second;  // the lane's operands of the two steps
+  uint32_t packed, rows, lane;
+  __device__ __forceinline__ XPlaces(const PlanesX &x, uint32_t l) : packed(x.packed), rows(x.m_rows), lane(l) {
+    const uint32_t r = l % 16, q = l / 16;
+    first = packed ? l * 16 : r * 128 + (q ^ r % 8) * 16;
+    second = packed ? first + 1024 : first ^ 64;
+  }
+  __device__ __forceinline__ void source(uint32_t i, uint32_t &row, uint32_t &chunk) const {
+    row = min(packed ? i / 2 * 16 + lane % 16 : i * 8 + lane / 8, rows - 1);
+    chunk = packed ? i % 2 * 4 + lane / 16 : (lane % 8) ^ (lane / 8);
+  }
+};
+
+// Sixteen bytes a lane from base + from straight to LDS, lane l's at `to` + 16 l (the compiler would let every LDS read wait
+// for all copies that it knows of), when the wave's reads there are done.
+__device__ __forceinline__ void copy_to_lds(const uint8_t *base, uint32_t from, uint32_t to) {
 #if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(from), "s"(base), "s"(to) : "memory");
+#else
+  (void)base, (void)from, (void)to;
+#endif
+}
+
+// All but the wave's last LEFT loads are answered; its LDS operations are done as well, and the workgroup's waves here.
+template <int LEFT>
+__device__ __forceinline__ void wait_for_loads() {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LEFT) : "memory");
+#endif
+}
+
+template <int LEFT>
+__device__ __forceinline__ void meet_after_loads() {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(LEFT) : "memory");
+#endif
+}
+
+constexpr uint32_t kUnits = 256;  // the chip's compute units
+
+// LDS of a wave that has its own x.
+template <int HR>
+struct Product {
+  static constexpr uint32_t kRing = HR == 4 ? 3 : 4;            // quarters of a visit of x
+  static constexpr uint32_t kFirst = kRing * HR * 1024 + 2048;  // before it a quarter's words, there the sums of the first split of two
+  static constexpr uint32_t kWaveBytes = kFirst + (HR + 1) / 2 * 1024;
+};
+
+// Few rows of x, HR eights of them.  A workgroup's waves share out the visits of
+// `blocks_each` row blocks, a split or two a wave, and the splits' sums are added in their order: what a row of x gives depends on nothing
+// but the matrix's sizes, so all row counts, single and grouped launches agree bit for bit.  A wave brings its own x into LDS,
+// a quarter of a visit at a time and two or three ahead (a ring), and meets no other wave until its sums are there.  One row is
+// bound by memory (17408 x 5120 twice 5.0 TB/s), more by the lines of x that every wave reads; us with x read where it is, in operand
+// order, and now: one row of 5120 x 17408 37 and 34, 16 of 6144, 1024 and 1024 x 5120 21 and 18, of 17408 x 5120 twice 73 and 65.
+template <int HR>
+__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) void planes_product_kernel(PlanesGroup g, PlanesX x) {
+  extern __shared__ __align__(16) uint8_t lds[];  // (all of the kernel's: copies go by absolute address)
+#if defined(__HIP_DEVICE_COMPILE__)
+  constexpr int MT = (HR + 1) / 2;
+  constexpr uint32_t kQuarterX = HR * 1024, kWave = Product<HR>::kWaveBytes, kRing = Product<HR>::kRing, kAhead = kRing - 1;
   const uint32_t lane = threadIdx.x % 64, wave = scalar(threadIdx.x / 64);
   uint32_t i = 0;
   while (i + 1 < g.n && blockIdx.x >= g.m[i + 1].first) ++i;
   const PlanesMember &m = g.m[i];
-  const uint32_t splits = m.p.splits, sub = wave / splits, split = wave % splits;
+  const uint32_t splits = m.p.splits, waves = blockDim.x / 64;
+  const uint32_t at_once = splits > waves ? (splits + 1) / 2 : splits, sub = wave / at_once;  // (a wave has one split or two)
   const uint32_t blocks = (m.p.rows + 15) / 16, block = (blockIdx.x - m.first) * m.blocks_each + sub;
   const grf::PlanesShape shape(x.cols);
+  const uint32_t each = (shape.visits() + splits - 1) / splits;
   const bool works = sub < m.blocks_each && block < blocks;
   float4v acc[MT] = {};
-  if (works) {
-    const uint32_t each = (shape.visits() + splits - 1) / splits;
+  float4v *const before = reinterpret_cast<float4v *>(lds + wave * kWave + Product<HR>::kFirst) + lane;
+  for (uint32_t split = wave % at_once; works && split < splits; split += at_once) {
+#pragma unroll
+    for (int j = 0; j < MT; ++j) before[j * 64] = acc[j], acc[j] = (float4v){};
     const uint32_t v0 = min(split * each, shape.visits()), v1 = min(v0 + each, shape.visits()), full = min(v1, shape.full);
-    const uint32_t q = lane / 16, r = lane % 16, slot = r * 4 + q;
-    uint8_t *patch = lds + wave * kPatch;
+    const uint32_t q = lane / 16, r = lane % 16, slot = r * 4 + q, at_wave = wave * kWave;
+    uint8_t *const own = lds + at_wave, *const patch = own + kRing * kQuarterX;
     const uint8_t *at = m.p.planes + (size_t)block * shape.block_bytes();
     const uint32_t base = m.p.bases[block * 16 + r];
     const uint32_t ends = m.p.listed_at[block * shape.visits() + min(v0 + lane, shape.visits())];  // (of up to 63 visits)
-    auto end_of = [&](uint32_t v) { return (uint32_t)__builtin_amdgcn_readlane(ends, v - v0); };
-    const uint8_t *xr[MT];
+    auto end_of = [&](uint32_t v) { return (uint32_t)__builtin_amdgcn_readlane(ends, min(v, v1) - v0); };
+    auto first_listed = [&](uint32_t v) {  // (the list ends with an entry that nobody owns)
+      const uint32_t from = end_of(v), count = end_of(v + 1) - from;
+      return m.p.listed[from + min(lane, count ? count - 1 : 0)];
+    };
+    const XPlaces places(x, lane);
+    uint32_t xr[HR];  // (up to 31 rows of 2^25 bytes)
 #pragma unroll
-    for (int j = 0; j < MT; ++j) xr[j] = x.data + (size_t)min(r + 16 * j, x.m_rows - 1) * x.row_bytes + q * x.chunk_bytes;
-
-    auto multiply = [&](const uint32_t (&o)[4], const uint8_t *const (&from)[MT], uint32_t offset) {
-      const bf16x8_t w = __builtin_bit_cast(bf16x8_t, (uint4v){o[0], o[1], o[2], o[3]});
+    for (int k = 0; k < HR; ++k) {
+      uint32_t row, chunk;
+      places.source(k, row, chunk);
+      xr[k] = row * x.row_bytes + chunk * x.chunk_bytes;
+    }
+    auto copy_x = [&](uint32_t quarter) {  // 64 columns
+      const uint8_t *from = x.data + (size_t)(quarter * 8) * x.chunk_bytes;
 #pragma unroll
-      for (int j = 0; j < MT; ++j)
-        acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4v *>(from[j] + offset)), w,
-                                                         acc[j], 0, 0, 0);
+      for (int k = 0; k < HR; ++k) copy_to_lds(from, xr[k], at_wave + quarter % kRing * kQuarterX + k * 1024);
+    };
+    auto complete = [&](uint32_t(&o)[2][4], auto &&put) {
+      uint4v *words = reinterpret_cast<uint4v *>(patch);
+#pragma unroll
+      for (int t = 0; t < 2; ++t) words[t * 64 + lane] = (uint4v){o[t][0], o[t][1], o[t][2], o[t][3]};
+      wave_order();
+      put();
+      wave_order();
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const uint4v w = words[t * 64 + lane];
+        o[t][0] = w[0], o[t][1] = w[1], o[t][2] = w[2], o[t][3] = w[3];
+      }
+      wave_order();
+    };
+    auto multiply = [&](const uint32_t(&o)[2][4], uint32_t quarter) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int j = 0; j < MT; ++j)
+          acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4v *>(own + quarter * kQuarterX + j * 2048 + (t ? places.second : places.first))),
+              __builtin_bit_cast(bf16x8_t, (uint4v){o[t][0], o[t][1], o[t][2], o[t][3]}), acc[j], 0, 0, 0);
     };
 
     if (v0 < full) {
+      // A visit's words are asked for a visit ahead, each as soon as the register is free that they come into.
+      const VisitBytes bytes(at, full);
+      const uint32_t end = full * 4;  // quarters
+      Visit now;
+#pragma unroll
+      for (uint32_t k = 0; k < kAhead; ++k) copy_x(v0 * 4 + k);
+      now.load(bytes, v0, slot);
+      uint32_t entry = first_listed(v0);
       for (uint32_t v = v0; v < full; ++v) {
-        Visit now;
-        Listed listed;
-        now.load(at + (size_t)v * grf::kVisitBytes, slot);
-        listed.load(m.p.listed, end_of(v), end_of(v + 1), lane);
-        const uint32_t x0 = v * 32 * x.chunk_bytes, xs = 4 * x.chunk_bytes;
-        auto half = [&](auto which) {
-          constexpr int H = decltype(which)::value;
-          uint32_t o[4][4];
-          now.step<4 * H>(base, o[0]);
-          now.step<4 * H + 1>(base, o[1]);
-          now.step<4 * H + 2>(base, o[2]);
-          now.step<4 * H + 3>(base, o[3]);
-          if (listed.count) {
-            uint4v *words = reinterpret_cast<uint4v *>(patch);
-#pragma unroll
-            for (int t = 0; t < 4; ++t) words[t * 64 + lane] = (uint4v){o[t][0], o[t][1], o[t][2], o[t][3]};
-            wave_order();
-            listed.patch<H * 2048, 2048>(patch, lane);
-            wave_order();
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-              const uint4v w = words[t * 64 + lane];
-              o[t][0] = w[0], o[t][1] = w[1], o[t][2] = w[2], o[t][3] = w[3];
-            }
-            wave_order();
-          }
-#pragma unroll
-          for (int t = 0; t < 4; ++t) multiply(o[t], xr, x0 + (4 * H + t) * xs);
+        Exponents next;
+        uint32_t next_entry;
+        const uint32_t from = end_of(v), count = end_of(v + 1) - from;
+        auto quarter = [&](auto which) {
+          constexpr int Q = decltype(which)::value;
+          const uint32_t h = 4 * v + Q;
+          if (h + kAhead < end) copy_x(h + kAhead);
+          if constexpr (Q == 0) next.load(bytes, v + 1, slot), next_entry = first_listed(v + 1);
+          uint32_t o[2][4];
+          now.step<2 * Q>(base, o[0]);
+          now.step<2 * Q + 1>(base, o[1]);
+          now.load_signs(bytes, v + 1, Q, slot);
+          if (count) complete(o, [&] { Listed{m.p.listed, from, count, entry}.patch<Q * 1024, 1024>(patch, lane); });
+          // This quarter's x was asked for kAhead quarters ago: since then as many more (at the end, none) and the words
+          // of these quarters and this one, four or one load each.
+          constexpr int kAfter = kAhead == 3 ? 7 : Q == 3 ? 3 : 6;
+          if (h + kAhead < end) wait_for_loads<kAfter + kAhead * HR>();
+          else wait_for_loads<kAfter>();
+          multiply(o, h % kRing);
         };
-        half(std::integral_constant<int, 0>{});
-        half(std::integral_constant<int, 1>{});
+        quarter(std::integral_constant<int, 0>{});
+        quarter(std::integral_constant<int, 1>{});
+        quarter(std::integral_constant<int, 2>{});
+        quarter(std::integral_constant<int, 3>{});
+        now.e = next, entry = next_entry;
       }
     }
-    if (v0 < v1 && v1 > shape.full) {  // the shorter visit, a unit at a time
-      Listed listed;
-      listed.load(m.p.listed, end_of(shape.full), end_of(shape.full + 1), lane);
+    if (v0 < v1 && v1 > shape.full) {  // the shorter visit, a unit at a time; zeros in x's columns past the last one
+      const uint32_t from = end_of(shape.full), count = end_of(shape.full + 1) - from;
       for (uint32_t u = 0; u < shape.units; ++u) {
+#pragma unroll
+        for (int k = 0; k < HR; ++k) {
+          uint32_t row, chunk;
+          places.source(k, row, chunk);
+          chunk += shape.full * 32 + u * 8;
+          uint4v one = {0, 0, 0, 0};
+          if (chunk * 8 < x.cols) one = *reinterpret_cast<const uint4v *>(x.data + (size_t)row * x.row_bytes + (size_t)chunk * x.chunk_bytes);
+          reinterpret_cast<uint4v *>(own)[k * 64 + lane] = one;
+        }
         ShortVisit now;
         now.load(at + shape.full * grf::kVisitBytes + u * grf::kUnitBytes, slot);
         uint32_t o[2][4];
         now.step<0>(base, o[0]);
         now.step<1>(base, o[1]);
-        uint4v *words = reinterpret_cast<uint4v *>(patch);  // (the unit's steps are 2 u and 2 u + 1 of the visit)
-#pragma unroll
-        for (int t = 0; t < 2; ++t) words[t * 64 + lane] = (uint4v){o[t][0], o[t][1], o[t][2], o[t][3]};
-        wave_order();
-        for (uint32_t k = 0; k < listed.count; k += 64) {
-          const uint32_t mine = k ? listed.list[listed.first + min(k + lane, listed.count - 1)] : listed.entry;
-          if (k + lane < listed.count && (mine >> 16) / 1024 == u) *reinterpret_cast<uint16_t *>(patch + (mine >> 16) % 1024 * 2) = (uint16_t)mine;
-        }
-        wave_order();
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          const uint4v w = words[t * 64 + lane];
-          // columns past the last one: the planes hold numbers there, x is not read and counts as zeros
-          const uint32_t chunk = (shape.full * 8 + u * 2 + t) * 4 + q;
-          const bool inside = chunk * 8 < x.cols;
-#pragma unroll
-          for (int j = 0; j < MT; ++j) {
-            uint4v a = *reinterpret_cast<const uint4v *>(xr[j] + (inside ? (chunk - q) * x.chunk_bytes : 0));
-            if (!inside) a = (uint4v){0, 0, 0, 0};
-            acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, w), acc[j], 0, 0, 0);
+        complete(o, [&] {
+          for (uint32_t k = lane; k < count; k += 64) {
+            const uint32_t mine = m.p.listed[from + k];
+            if ((mine >> 16) / 1024 == u) *reinterpret_cast<uint16_t *>(patch + (mine >> 16) % 1024 * 2) = (uint16_t)mine;
           }
-        }
+        });
+        multiply(o, 0);
         wave_order();
       }
     }
   }
-  __syncthreads();  // the words of all waves are read
-  float4v *sums = reinterpret_cast<float4v *>(lds);
+  const uint32_t split0 = wave % at_once;
+  const bool two = works && split0 + at_once < splits;
+  float4v first[MT];
 #pragma unroll
-  for (int j = 0; j < MT; ++j) sums[(wave * MT + j) * 64 + lane] = acc[j];
+  for (int j = 0; j < MT; ++j) first[j] = two ? before[j * 64] : acc[j];
+  __syncthreads();  // x, words and sums of all waves are read
+  float4v *sums = reinterpret_cast<float4v *>(lds);
+  if (works) {
+#pragma unroll
+    for (int j = 0; j < MT; ++j) {
+      sums[((sub * splits + split0) * MT + j) * 64 + lane] = first[j];
+      if (two) sums[((sub * splits + split0 + at_once) * MT + j) * 64 + lane] = acc[j];
+    }
+  }
   __syncthreads();
   // Four activation rows of one weight row at a time: the waves' sums in their order, the bias, one rounding.
   for (uint32_t t = threadIdx.x; t < m.blocks_each * MT * 64; t += blockDim.x) {
     const uint32_t l = t % 64, j = t / 64 % MT, s = t / (64 * MT);
     const uint32_t row = ((blockIdx.x - m.first) * m.blocks_each + s) * 16 + l % 16, m0 = j * 16 + l / 16 * 4;
     if (row >= m.p.rows || m0 >= x.m_rows) continue;
-    // a part's splits one after the other, then the parts
-    const uint32_t per_part = splits / m.p.parts;
-    float4v sum = {};
-    for (uint32_t part = 0; part < m.p.parts; ++part) {
-      const float4v *from = sums + ((s * splits + part * per_part) * MT + j) * 64 + l;
-      float4v one = *from;
-      for (uint32_t w = 1; w < per_part; ++w) one += from[w * MT * 64];
-      sum = part ? sum + one : one;
-    }
+    const float4v *from = sums + (s * splits * MT + j) * 64 + l;
+    float4v sum = *from;
+    for (uint32_t w = 1; w < splits; ++w) sum += from[w * MT * 64];
     const float b = m.bias ? __uint_as_float((uint32_t)m.bias[row] << 16) : 0.0f;
 #pragma unroll
     for (int k = 0; k < 4; ++k)
@@ -290,176 +419,239 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(6))) void 
 #endif
 }
 
-// More than sixteen rows of x: a wave has a row block and one split of its visits.  The four waves of a workgroup that
-// share a split share its x as well, which comes into LDS a quarter of a visit at a time in operand order, the next
-// while this one is multiplied.  (In place every row block reads all of x: 64 rows of 17408 x 5120 109 us, the
-// lines of a step in few cache sets.)  A workgroup has the splits of one part.
-constexpr uint32_t kBatchBlocks = 4;
-template <int MT>
-__global__ __launch_bounds__(kBatchBlocks * kMaxSharing * 64) __attribute__((amdgpu_waves_per_eu(MT == 8 ? 4 : 5))) void planes_batch_kernel(
+// More rows of x: a wave has two row blocks and one split of their visits, W waves share the split's x, and an operand that
+// is read meets both blocks.  What bounds it, besides memory, is how evenly the workgroups fall on the compute units (product()
+// chooses W; 64 rows of 17408 x 5120 twice 84 us with four waves, 75 with three) and how far ahead the words are asked for: a
+// wave's loads are answered in order, so whatever it waits for ends the waits for all before.  x therefore goes past the
+// registers, straight into LDS, a quarter of a visit at a time and three ahead (a ring of four), words come a visit ahead,
+// each as soon as the register is free that they come into, and between a copy of x and its use lie exactly the loads
+// that kAfter counts, which stay under way.  us for 32 of 6144, 1024 and 1024 x 5120 26 (through registers, one block
+// a wave) and 23; 64 of 17408 x 5120 twice 107 and 75, 128 164 and 114; 128 of 5120 x 17408 103 and 59.
+constexpr uint32_t kBatchEach = 2;                   // row blocks a wave
+constexpr uint32_t kBatchPatch = kBatchEach * 2048;  // LDS bytes in which a wave's quarters of a visit are completed
+
+template <int MT, int W>
+__global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(MT == 8 ? 2 : MT == 4 ? 3 : 4))) void planes_batch_kernel(
     PlanesGroup g, PlanesX x) {
-  extern __shared__ __align__(16) uint8_t lds[];
+  extern __shared__ __align__(16) uint8_t lds[];  // (all of the kernel's: copies go by absolute address)
 #if defined(__HIP_DEVICE_COMPILE__)
-  constexpr int kCopies = MT / 2;                   // operands that a wave brings for a quarter
-  constexpr uint32_t kQuarterX = 2 * MT * 1024;     // bytes of x for a quarter
-  const uint32_t lane = threadIdx.x % 64, wave = scalar(threadIdx.x / 64), own = wave % kBatchBlocks, share = wave / kBatchBlocks;
+  constexpr int kCopies = (2 * MT + W - 1) / W;  // of 1 KiB that a wave makes a quarter (some twice where W does not divide them)
+  constexpr uint32_t kQuarterX = 2 * MT * 1024;
+  const uint32_t lane = threadIdx.x % 64, own = scalar(threadIdx.x / 64);
   uint32_t i = 0;
   while (i + 1 < g.n && blockIdx.x >= g.m[i + 1].first) ++i;
   const PlanesMember &m = g.m[i];
   const grf::PlanesShape shape(x.cols);
-  const uint32_t blocks = (m.p.rows + 15) / 16, groups = (blocks + kBatchBlocks - 1) / kBatchBlocks;
-  const uint32_t part = (blockIdx.x - m.first) / groups, wanted = (blockIdx.x - m.first) % groups * kBatchBlocks + own;
-  const uint32_t sharing = m.p.splits / m.p.parts;  // (members of a group may have fewer than the launch)
-  const uint32_t block = min(wanted, blocks - 1);   // (a wave without a block copies and waits like the rest)
-  const uint32_t each = (shape.visits() + m.p.splits - 1) / m.p.splits, split = part * sharing + min(share, sharing - 1);
+  const uint32_t blocks = (m.p.rows + 15) / 16, groups = (blocks + (W * kBatchEach) - 1) / (W * kBatchEach);
+  const uint32_t split = (blockIdx.x - m.first) / groups, wanted = (blockIdx.x - m.first) % groups * (W * kBatchEach) + own * kBatchEach;
+  const uint32_t each = (shape.visits() + m.p.splits - 1) / m.p.splits;
   const uint32_t v0 = split * each, v1 = min(v0 + each, shape.visits()), full = min(v1, shape.full);
   const uint32_t q = lane / 16, r = lane % 16, slot = r * 4 + q;
-  uint8_t *const xlds = lds + share * 2 * kQuarterX, *const patch = lds + blockDim.x / (kBatchBlocks * 64) * 2 * kQuarterX + wave * (kPatch / 2);
-  const uint8_t *at = m.p.planes + (size_t)block * shape.block_bytes();
-  const uint32_t base = m.p.bases[block * 16 + r];
-  const uint32_t *listed_at = m.p.listed_at + block * shape.visits();
+  uint8_t *const patch = lds + 4 * kQuarterX + own * kBatchPatch;
 
-  uint4v held[kCopies];
-  const uint8_t *xr[kCopies];
+  const XPlaces places(x, lane);
+  uint32_t xr[kCopies];  // (up to 127 rows of 2^25 bytes)
 #pragma unroll
-  for (int j = 0; j < kCopies; ++j) xr[j] = x.data + (size_t)min(r + 16 * ((own + kBatchBlocks * j) % MT), x.m_rows - 1) * x.row_bytes;
-  auto fetch_x = [&](uint32_t quarter) {
+  for (int k = 0; k < kCopies; ++k) {
+    uint32_t row, chunk;
+    places.source((own + W * k) % (2 * MT), row, chunk);
+    xr[k] = row * x.row_bytes + chunk * x.chunk_bytes;
+  }
+  auto copy_x = [&](uint32_t quarter) {  // 64 columns
+    const uint8_t *from = x.data + (size_t)(quarter * 8) * x.chunk_bytes;
 #pragma unroll
-    for (int j = 0; j < kCopies; ++j) {
-      const uint32_t chunk = (quarter * 2 + (own + kBatchBlocks * j) / MT) * 4 + q;
-      held[j] = *reinterpret_cast<const uint4v *>(xr[j] + (size_t)(chunk * 8 < x.cols ? chunk : 0) * x.chunk_bytes);
-      if (chunk * 8 >= x.cols) held[j] = (uint4v){0, 0, 0, 0};  // columns past the last one
-    }
+    for (int k = 0; k < kCopies; ++k) copy_to_lds(from, xr[k], quarter % 4 * kQuarterX + (own + W * k) % (2 * MT) * 1024);
   };
-  auto keep_x = [&](uint32_t quarter) {
-    uint4v *to = reinterpret_cast<uint4v *>(xlds + quarter % 2 * kQuarterX);
-#pragma unroll
-    for (int j = 0; j < kCopies; ++j) to[(own + kBatchBlocks * j) * 64 + lane] = held[j];
-  };
-  // The workgroup's LDS is written; loads under way stay so.
-  auto meet = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
 
-  float4v acc[MT] = {};
-  Visit now;
-  Listed listed;
-  auto fetch = [&](uint32_t v) {
-    const uint32_t there = min(v, shape.visits() - 1);
-    if (v < full) now.load(at + (size_t)there * grf::kVisitBytes, slot);
-    listed.load(m.p.listed, listed_at[there], listed_at[there + 1], lane);
+  // (a wave without a block reads the last one's list, no planes, and waits like the rest)
+  const uint8_t *at[kBatchEach];
+  uint32_t base[kBatchEach], ends[kBatchEach];
+#pragma unroll
+  for (uint32_t b = 0; b < kBatchEach; ++b) {
+    const uint32_t block = min(wanted + b, blocks - 1);
+    at[b] = m.p.planes + (size_t)block * shape.block_bytes();
+    base[b] = m.p.bases[block * 16 + r];
+    ends[b] = m.p.listed_at[block * shape.visits() + min(v0 + lane, shape.visits())];  // (of up to 63 visits)
+  }
+  auto end_of = [&](uint32_t b, uint32_t v) { return (uint32_t)__builtin_amdgcn_readlane(ends[b], min(v, v1) - v0); };
+  auto first_listed = [&](uint32_t b, uint32_t v) {  // (the list ends with an entry that nobody owns)
+    const uint32_t from = end_of(b, v), count = end_of(b, v + 1) - from;
+    return m.p.listed[from + min(lane, count ? count - 1 : 0)];
   };
-  fetch_x(4 * v0);
-  fetch(v0);
-  keep_x(4 * v0);
-  meet();
-  for (uint32_t v = v0; v < v0 + each; ++v) {  // (as many for all: they meet)
-    auto quarter = [&](auto which) {
-      constexpr int Q = decltype(which)::value;
-      const uint32_t h = 4 * v + Q;
-      fetch_x(h + 1);
-      if (v < v1) {
-        uint32_t o[2][4] = {};
-        if (v < shape.full) {
-          now.step<2 * Q>(base, o[0]);
-          now.step<2 * Q + 1>(base, o[1]);
-        } else if (Q < shape.units) {
-          ShortVisit one;
-          one.load(at + (size_t)v * grf::kVisitBytes + Q * grf::kUnitBytes, slot);
-          one.step<0>(base, o[0]);
-          one.step<1>(base, o[1]);
-        }
-        if (listed.count) {
-          uint4v *words = reinterpret_cast<uint4v *>(patch);
+  // The words of two steps with those of the list that belong there, which `put` writes.
+  auto complete = [&](uint32_t(&o)[kBatchEach][2][4], auto &&put) {
+    uint4v *words = reinterpret_cast<uint4v *>(patch);
 #pragma unroll
-          for (int t = 0; t < 2; ++t) words[t * 64 + lane] = (uint4v){o[t][0], o[t][1], o[t][2], o[t][3]};
-          wave_order();
-          listed.patch<Q * 1024, 1024>(patch, lane);
-          wave_order();
+    for (uint32_t b = 0; b < kBatchEach; ++b)
 #pragma unroll
-          for (int t = 0; t < 2; ++t) {
-            const uint4v w = words[t * 64 + lane];
-            o[t][0] = w[0], o[t][1] = w[1], o[t][2] = w[2], o[t][3] = w[3];
-          }
-          wave_order();
-        }
-        if constexpr (Q == 3) fetch(v + 1);  // (into the registers that this visit no longer needs)
-        const uint4v *from = reinterpret_cast<const uint4v *>(xlds + h % 2 * kQuarterX);
+      for (int t = 0; t < 2; ++t) words[(b * 2 + t) * 64 + lane] = (uint4v){o[b][t][0], o[b][t][1], o[b][t][2], o[b][t][3]};
+    wave_order();
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          const bf16x8_t w = __builtin_bit_cast(bf16x8_t, (uint4v){o[t][0], o[t][1], o[t][2], o[t][3]});
+    for (uint32_t b = 0; b < kBatchEach; ++b) put(b, patch + b * 2048);
+    wave_order();
 #pragma unroll
-          for (int j = 0; j < MT; ++j)
-            acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, from[(t * MT + j) * 64 + lane]), w, acc[j], 0, 0, 0);
-        }
+    for (uint32_t b = 0; b < kBatchEach; ++b)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const uint4v w = words[(b * 2 + t) * 64 + lane];
+        o[b][t][0] = w[0], o[b][t][1] = w[1], o[b][t][2] = w[2], o[b][t][3] = w[3];
       }
-      keep_x(h + 1);
-      meet();
-    };
-    quarter(std::integral_constant<int, 0>{});
-    quarter(std::integral_constant<int, 1>{});
-    quarter(std::integral_constant<int, 2>{});
-    quarter(std::integral_constant<int, 3>{});
-  }
-  // The splits' sums in their order, in the first one's wave.
-  float4v *sums = reinterpret_cast<float4v *>(lds);
-  for (uint32_t k = 1; k < sharing; ++k) {
-    if (share == k)
+    wave_order();
+  };
+
+  float4v acc[kBatchEach][MT] = {};
+  auto multiply = [&](const uint32_t(&o)[kBatchEach][2][4], uint32_t quarter) {
 #pragma unroll
-      for (int j = 0; j < MT; ++j) sums[(own * MT + j) * 64 + lane] = acc[j];
-    __syncthreads();
-    if (!share)
+    for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int j = 0; j < MT; ++j) acc[j] += sums[(own * MT + j) * 64 + lane];
-    __syncthreads();
-  }
-  const uint32_t row = block * 16 + r;
-  if (share || wanted >= blocks || row >= m.p.rows) return;
-  const float b = m.bias ? __uint_as_float((uint32_t)m.bias[row] << 16) : 0.0f;
+      for (int j = 0; j < MT; ++j) {
+        const bf16x8_t a = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4v *>(lds + quarter * kQuarterX + j * 2048 + (t ? places.second : places.first)));
 #pragma unroll
-  for (int j = 0; j < MT; ++j)
+        for (uint32_t b = 0; b < kBatchEach; ++b)
+          acc[b][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              a, __builtin_bit_cast(bf16x8_t, (uint4v){o[b][t][0], o[b][t][1], o[b][t][2], o[b][t][3]}), acc[b][j], 0, 0, 0);
+      }
+  };
+
+  if (v0 < full) {
+    const VisitBytes bytes[kBatchEach] = {{at[0], wanted < blocks ? full : 0}, {at[1], wanted + 1 < blocks ? full : 0}};
+    const uint32_t end = full * 4;  // quarters
+    Visit now[kBatchEach];
+    uint32_t entry[kBatchEach];
+    copy_x(v0 * 4), copy_x(v0 * 4 + 1), copy_x(v0 * 4 + 2);
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const uint32_t xrow = j * 16 + q * 4 + k;
-      if (xrow >= x.m_rows) continue;
-      if (m.p.parts > 1)
-        m.partials[((size_t)part * x.m_rows + xrow) * m.p.rows + row] = acc[j][k];
-      else
-        m.y[(size_t)xrow * m.ldy + row] = round_bf16(m.bias ? acc[j][k] + b : acc[j][k]);
+    for (uint32_t b = 0; b < kBatchEach; ++b) now[b].load(bytes[b], v0, slot), entry[b] = first_listed(b, v0);
+    meet_after_loads<2 * kCopies + kBatchEach * 7>();
+    for (uint32_t v = v0; v < full; ++v) {
+      Exponents next[kBatchEach];
+      uint32_t from[kBatchEach], count[kBatchEach], next_entry[kBatchEach];
+#pragma unroll
+      for (uint32_t b = 0; b < kBatchEach; ++b) from[b] = end_of(b, v), count[b] = end_of(b, v + 1) - from[b];
+      auto quarter = [&](auto which) {
+        constexpr int Q = decltype(which)::value;
+        const uint32_t h = 4 * v + Q;
+        if (h + 3 < end) copy_x(h + 3);
+        if constexpr (Q == 0) {
+#pragma unroll
+          for (uint32_t b = 0; b < kBatchEach; ++b) next[b].load(bytes[b], v + 1, slot), next_entry[b] = first_listed(b, v + 1);
+        }
+        uint32_t o[kBatchEach][2][4];
+#pragma unroll
+        for (uint32_t b = 0; b < kBatchEach; ++b) {
+          now[b].template step<2 * Q>(base[b], o[b][0]);
+          now[b].template step<2 * Q + 1>(base[b], o[b][1]);
+          now[b].load_signs(bytes[b], v + 1, Q, slot);
+        }
+        if (count[0] | count[1])
+          complete(o, [&](uint32_t b, uint8_t *there) { Listed{m.p.listed, from[b], count[b], entry[b]}.patch<Q * 1024, 1024>(there, lane); });
+        multiply(o, Q);
+        // The next quarter's x was asked for two quarters ago: since then two (here and below, at the end, none) more of x,
+        // this quarter's words and the two quarters' before, four or one load a block each.
+        constexpr int kAfter = kBatchEach * (Q == 3 ? 3 : 6);
+        if (h + 3 < end) meet_after_loads<kAfter + 2 * kCopies>();
+        else meet_after_loads<kAfter>();
+      };
+      quarter(std::integral_constant<int, 0>{});
+      quarter(std::integral_constant<int, 1>{});
+      quarter(std::integral_constant<int, 2>{});
+      quarter(std::integral_constant<int, 3>{});
+#pragma unroll
+      for (uint32_t b = 0; b < kBatchEach; ++b) now[b].e = next[b], entry[b] = next_entry[b];
     }
+  }
+  if (v1 > shape.full) {  // the shorter visit: x in the ring's place, zeros in columns past the last one, then a unit at a time
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (the loop's copies were waited for, but for the last barrier's)
+    for (uint32_t k = own; k < 2 * shape.units * MT; k += W) {
+      uint32_t row, chunk;
+      places.source(k % (2 * MT), row, chunk);
+      chunk += shape.full * 32 + k / (2 * MT) * 8;
+      uint4v one = {0, 0, 0, 0};
+      if (chunk * 8 < x.cols) one = *reinterpret_cast<const uint4v *>(x.data + (size_t)row * x.row_bytes + (size_t)chunk * x.chunk_bytes);
+      reinterpret_cast<uint4v *>(lds)[k * 64 + lane] = one;
+    }
+    __syncthreads();
+    uint32_t from[kBatchEach], count[kBatchEach];
+#pragma unroll
+    for (uint32_t b = 0; b < kBatchEach; ++b) from[b] = end_of(b, shape.full), count[b] = end_of(b, shape.full + 1) - from[b];
+    for (uint32_t u = 0; u < shape.units; ++u) {
+      uint32_t o[kBatchEach][2][4];
+#pragma unroll
+      for (uint32_t b = 0; b < kBatchEach; ++b) {
+        ShortVisit one;
+        one.load(at[b] + shape.full * grf::kVisitBytes + u * grf::kUnitBytes, slot);
+        one.step<0>(base[b], o[b][0]);
+        one.step<1>(base[b], o[b][1]);
+      }
+      complete(o, [&](uint32_t b, uint8_t *there) {
+        for (uint32_t k = lane; k < count[b]; k += 64) {
+          const uint32_t mine = m.p.listed[from[b] + k];
+          if ((mine >> 16) / 1024 == u) *reinterpret_cast<uint16_t *>(there + (mine >> 16) % 1024 * 2) = (uint16_t)mine;
+        }
+      });
+      multiply(o, u);
+    }
+  }
+#pragma unroll
+  for (uint32_t b = 0; b < kBatchEach; ++b) {
+    const uint32_t row = (wanted + b) * 16 + r;
+    if (row >= m.p.rows) continue;
+    const float added = m.bias ? __uint_as_float((uint32_t)m.bias[row] << 16) : 0.0f;
+#pragma unroll
+    for (int j = 0; j < MT; ++j)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const uint32_t xrow = j * 16 + q * 4 + k;
+        if (xrow >= x.m_rows) continue;
+        if (m.p.splits > 1)
+          m.partials[((size_t)split * x.m_rows + xrow) * m.p.rows + row] = acc[b][j][k];
+        else
+          m.y[(size_t)xrow * m.ldy + row] = round_bf16(m.bias ? acc[b][j][k] + added : acc[b][j][k]);
+      }
+  }
 #else
   (void)g, (void)x, (void)lds;
 #endif
 }
 
-// The parts of a batch's members in order, the bias, one rounding.
+// The splits' sums of a batch's members in order, the bias, one rounding.  A thread has N rows of W.
+template <int N>
 __global__ __launch_bounds__(256) void planes_sum_kernel(PlanesGroup g, uint32_t m_rows) {
+  typedef float floats __attribute__((ext_vector_type(N)));
+  typedef uint16_t halves __attribute__((ext_vector_type(N)));
   uint32_t i = 0;
   while (i + 1 < g.n && blockIdx.x >= g.m[i + 1].first) ++i;
   const PlanesMember &m = g.m[i];
-  const uint32_t columns = (m.p.rows + 255) / 256, at = blockIdx.x - m.first;
-  const uint32_t row = at % columns * 256 + threadIdx.x, xrow = at / columns;
+  const uint32_t columns = (m.p.rows + 256 * N - 1) / (256 * N), at = blockIdx.x - m.first;
+  const uint32_t row = (at % columns * 256 + threadIdx.x) * N, xrow = at / columns;
   if (row >= m.p.rows) return;
   const float *from = m.partials + (size_t)xrow * m.p.rows + row;
   const size_t pitch = (size_t)m_rows * m.p.rows;
-  float sum = *from;
-  for (uint32_t k = 1; k < m.p.parts; ++k) sum += from[k * pitch];
-  if (m.bias) sum += __uint_as_float((uint32_t)m.bias[row] << 16);
-  m.y[(size_t)xrow * m.ldy + row] = round_bf16(sum);
+  floats sum = *reinterpret_cast<const floats *>(from);
+  for (uint32_t k = 1; k < m.p.splits; ++k) sum += *reinterpret_cast<const floats *>(from + k * pitch);
+  halves out;
+#pragma unroll
+  for (int k = 0; k < N; ++k) out[k] = round_bf16(m.bias ? sum[k] + __uint_as_float((uint32_t)m.bias[row + k] << 16) : sum[k]);
+  *reinterpret_cast<halves *>(m.y + (size_t)xrow * m.ldy + row) = out;
 }
 
-template <int MT>
-int launch_batch(const PlanesGroup &g, const PlanesX &x, uint32_t sharing, uint32_t grid, hipStream_t s) {
-  constexpr auto kernel = &planes_batch_kernel<MT>;
-  const uint32_t bytes = sharing * (2 * 2 * MT * 1024 + kBatchBlocks * kPatch / 2);
-  if (bytes > 64 * 1024)
+template <int MT, int W>
+int launch_batch_w(const PlanesGroup &g, const PlanesX &x, uint32_t grid, hipStream_t s) {
+  constexpr auto kernel = &planes_batch_kernel<MT, W>;
+  constexpr uint32_t kBytes = 8 * MT * 1024 + W * kBatchPatch;
+  if (kBytes > 64 * 1024)
     if (int rc = grf::allow_full_lds<kernel>()) return rc;
-  hipLaunchKernelGGL(kernel, dim3(grid), dim3(sharing * kBatchBlocks * 64), bytes, s, g, x);
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(W * 64), kBytes, s, g, x);
   return GRF_OK;
 }
-
 template <int MT>
+int launch_batch(const PlanesGroup &g, const PlanesX &x, uint32_t waves, uint32_t grid, hipStream_t s) {
+  return waves == 3 ? launch_batch_w<MT, 3>(g, x, grid, s) : launch_batch_w<MT, 4>(g, x, grid, s);
+}
+
+template <int HR>
 int launch_product(const PlanesGroup &g, const PlanesX &x, uint32_t waves, uint32_t grid, hipStream_t s) {
-  constexpr auto kernel = &planes_product_kernel<MT>;
-  const uint32_t bytes = waves * std::max<uint32_t>(kPatch, MT * 1024);
+  constexpr auto kernel = &planes_product_kernel<HR>;
+  const uint32_t bytes = waves * Product<HR>::kWaveBytes;
   if (bytes > 64 * 1024)
     if (int rc = grf::allow_full_lds<kernel>()) return rc;
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(waves * 64), bytes, s, g, x);
@@ -473,14 +665,14 @@ int check_planes(const char *who, const grf_planes *p) {
   if (!p->rows || !p->cols || p->cols % 8 || ((uintptr_t)p->planes & 15) || p->rows > 1u << 28 || p->cols > GRF_PLANES_MAX_COLS)
     return grf::set_error(GRF_BAD_ARGUMENT, std::string(who) + ": sizes or alignment of the planes");
   const uint32_t each = p->splits ? (shape.visits() + p->splits - 1) / p->splits : 0;
-  if (!each || p->splits > 16 || each > 63 || each * (p->splits - 1) >= shape.visits() || !p->parts || p->splits % p->parts || p->splits / p->parts > kMaxSharing)
-    return grf::set_error(GRF_BAD_ARGUMENT, std::string(who) + ": 1 to 16 splits of 1 to 63 visits each, in parts of one or two");
+  if (!each || p->splits > 16 || each > 63 || each * (p->splits - 1) >= shape.visits())
+    return grf::set_error(GRF_BAD_ARGUMENT, std::string(who) + ": 1 to 16 splits of 1 to 63 visits each");
   return GRF_OK;
 }
 
 // fp32 sums of a launch of `m` rows whose members are cut in parts, in bytes.
 size_t partial_bytes(const grf_planes &p, uint32_t m) {
-  return m > kInPlaceRows && p.parts > 1 ? ((size_t)p.parts * m * p.rows * 4 + 255) / 256 * 256 : 0;
+  return m > kOwnAlways && p.splits > 1 ? ((size_t)p.splits * m * p.rows * 4 + 255) / 256 * 256 : 0;
 }
 
 int product(const char *who, uint32_t n, const grf_planes *const *planes, const uint16_t *x, uint32_t ldx, uint32_t m_rows, bool packed,
@@ -488,51 +680,70 @@ int product(const char *who, uint32_t n, const grf_planes *const *planes, const 
   if (!n || n > kMaxMembers || !planes || !x || !y || !ldy) return grf::set_error(GRF_BAD_ARGUMENT, std::string(who) + ": null argument or member count");
   PlanesGroup g{};
   g.n = n;
-  uint32_t waves = 1, sharing = 1;
+  uint32_t waves = 1, longest = 0;
+  uint64_t visits = 0;
   size_t space = 0;
   const uint32_t cols = planes[0] ? planes[0]->cols : 0, most = std::min(m_rows, kMaxTileRows);
   for (uint32_t i = 0; i < n; ++i) {
     if (int rc = check_planes(who, planes[i])) return rc;
     if (!y[i] || ldy[i] < planes[i]->rows || planes[i]->cols != cols)
       return grf::set_error(GRF_BAD_ARGUMENT, std::string(who) + ": output rows or member widths");
-    waves = std::max(waves, planes[i]->splits), sharing = std::max(sharing, planes[i]->splits / planes[i]->parts);
+    if (planes[i]->rows > longest) {
+      longest = planes[i]->rows, waves = planes[i]->splits;
+      if (waves > 8 && longest > 16 * kUnits) waves = (waves + 1) / 2;  // (some units get two workgroups: one row of 5120 x 17408 37 us, 34)
+    }
+    visits += (uint64_t)((planes[i]->rows + 15) / 16) * grf::PlanesShape(cols).visits();
     g.m[i] = {*planes[i], y[i], bias ? bias[i] : nullptr, reinterpret_cast<float *>(static_cast<uint8_t *>(workspace) + space), ldy[i], 0, 0};
     space += partial_bytes(*planes[i], most);
   }
+  for (uint32_t i = 0; i < n; ++i) waves = std::max(waves, (planes[i]->splits + 1) / 2);  // the largest member's, and no wave more than two
   if (((uintptr_t)x & 15) || (!packed && (ldx < cols || ldx % 8 || ldx > 1u << 24)) || (packed && m_rows > kMaxTileRows))
     return grf::set_error(GRF_BAD_ARGUMENT, std::string(who) + ": activation rows are 16-byte aligned");
   if (space && (!workspace || workspace_bytes < space || ((uintptr_t)workspace & 15)))
     return grf::set_error(GRF_BAD_ARGUMENT, std::string(who) + ": workspace too small (grf_planes_workspace_bytes)");
   for (uint32_t done = 0; done < m_rows; done += kMaxTileRows) {
     const uint32_t m = std::min(kMaxTileRows, m_rows - done), m_pad = 16 * grf::gemm_tiles(m);
-    const bool batch = m > kInPlaceRows;
-    const PlanesX rows{reinterpret_cast<const uint8_t *>(x) + (size_t)done * ldx * 2, packed ? 16 : ldx * 2, packed ? m_pad * 16 : 16, m, cols};
-    uint32_t grid = 0;
-    bool parts = false;
+    const bool batch = m > kOwnRows || (m > kOwnAlways && visits >= kOwnVisits) || (m > 16 && waves * Product<4>::kWaveBytes > 160 * 1024);
+    const PlanesX rows{reinterpret_cast<const uint8_t *>(x) + (size_t)done * ldx * 2, packed ? 16 : ldx * 2, packed ? m_pad * 16 : 16, m, cols, packed};
+    uint32_t grid = 0, batch_waves = 4, busiest = ~0u;
+    for (uint32_t w : {4u, 3u}) {  // the visits of a compute unit that has most of them
+      uint32_t count = 0;
+      for (uint32_t i = 0; i < n; ++i) count += ((g.m[i].p.rows + 15) / 16 + w * kBatchEach - 1) / (w * kBatchEach) * g.m[i].p.splits;
+      const uint32_t most = (count + kUnits - 1) / kUnits * w;
+      if (most < busiest) busiest = most, batch_waves = w;
+    }
+    bool split = false;
     for (uint32_t i = 0; i < n; ++i) {
       PlanesMember &one = g.m[i];
       const uint32_t blocks = (one.p.rows + 15) / 16;
-      one.blocks_each = batch ? kBatchBlocks : waves / one.p.splits;
+      one.blocks_each = batch ? batch_waves * kBatchEach : std::max(1u, waves / one.p.splits);
       one.y = y[i] + (size_t)done * ldy[i];
       one.first = grid;
-      grid += (blocks + one.blocks_each - 1) / one.blocks_each * (batch ? one.p.parts : 1);
-      parts |= batch && one.p.parts > 1;
+      grid += (blocks + one.blocks_each - 1) / one.blocks_each * (batch ? one.p.splits : 1);
+      split |= batch && one.p.splits > 1;
     }
-    if (int rc = !batch   ? launch_product<1>(g, rows, waves, grid, s)
-                 : m <= 32 ? launch_batch<2>(g, rows, sharing, grid, s)
-                 : m <= 64 ? launch_batch<4>(g, rows, sharing, grid, s)
-                           : launch_batch<8>(g, rows, sharing, grid, s))
+    if (int rc = !batch ? (m <= 8 && !packed ? launch_product<1>(g, rows, waves, grid, s)
+                           : m <= 16         ? launch_product<2>(g, rows, waves, grid, s)
+                                             : launch_product<4>(g, rows, waves, grid, s))
+                 : m <= 16 ? launch_batch<1>(g, rows, batch_waves, grid, s)
+                 : m <= 32 ? launch_batch<2>(g, rows, batch_waves, grid, s)
+                 : m <= 64 ? launch_batch<4>(g, rows, batch_waves, grid, s)
+                           : launch_batch<8>(g, rows, batch_waves, grid, s))
       return rc;
-    if (parts) {
+    if (split) {
       PlanesGroup sums{};
+      uint32_t each = 4;
+      for (uint32_t i = 0; i < n; ++i)
+        if ((g.m[i].p.rows | g.m[i].ldy) % 4 || (uintptr_t)g.m[i].y & 7) each = 1;
       grid = 0;
       for (uint32_t i = 0; i < n; ++i)
-        if (g.m[i].p.parts > 1) {
+        if (g.m[i].p.splits > 1) {
           sums.m[sums.n] = g.m[i];
           sums.m[sums.n++].first = grid;
-          grid += (g.m[i].p.rows + 255) / 256 * m;
+          grid += (g.m[i].p.rows + 256 * each - 1) / (256 * each) * m;
         }
-      hipLaunchKernelGGL(planes_sum_kernel, dim3(grid), dim3(256), 0, s, sums, m);
+      if (each == 4) hipLaunchKernelGGL(planes_sum_kernel<4>, dim3(grid), dim3(256), 0, s, sums, m);
+      else hipLaunchKernelGGL(planes_sum_kernel<1>, dim3(grid), dim3(256), 0, s, sums, m);
     }
   }
   hipError_t e = hipGetLastError();

@@ -567,9 +567,8 @@ int grf_dense_gemm(const uint16_t *w, uint32_t rows, uint32_t cols, const uint16
  *   bases      u32 [rows in whole sixteens]: a row's lowest exponent << 7, in both halves
  *   listed_at  u32 [grf_planes_visits(rows, cols) + 1]: where a visit's listed words begin
  *   listed     u32 [listed_at's last + 1]: place in the visit << 16 | word
- *   splits     1 to 16 waves that share the visits of sixteen rows in a product, at most 63 each
- *   parts      divides splits; the sums of a part's splits are added in their order, then the parts: the order of a product's
- *              sums, in which nothing else has a part.
+ *   splits     1 to 16 that share the visits of sixteen rows in a product, at most 63 each; their sums are added in order,
+ *              and nothing else has a part in that order
  * cols is a multiple of 8 and at most GRF_PLANES_MAX_COLS.
  *
  * grf_planes_count  bases of a dense BF16 matrix (16-byte aligned), and counts u32 [grf_planes_visits]: the words
@@ -590,7 +589,7 @@ typedef struct grf_planes {
   const uint32_t *listed_at;
   const uint32_t *listed;
   uint32_t rows, cols;
-  uint32_t splits, parts;
+  uint32_t splits;
 } grf_planes;
 
 uint64_t grf_planes_bytes(uint32_t rows, uint32_t cols);

@@ -50,9 +50,9 @@ def test_words_and_rows_come_back_and_nothing_around_them_is_written(rows, cols,
     assert np.array_equal(got[1:-1], words[ids.cpu().numpy()]) and np.all(got[0] == 0x5A5A) and np.all(got[-1] == 0x5A5A)
 
 
-@pytest.mark.parametrize("splits,parts", [(1, 1), (2, 1), (2, 2), (4, 2), (8, 4)])
+@pytest.mark.parametrize("splits", [1, 2, 3, 5, 8])
 @pytest.mark.parametrize("rows,cols", SHAPES)
-def test_products_against_float64_with_one_set_of_bits_a_row(rows, cols, splits, parts):
+def test_products_against_float64_with_one_set_of_bits_a_row(rows, cols, splits):
     import torch
     from georefine_amd import _hip_abi, _native
     from georefine_amd._planes import visits
@@ -63,12 +63,12 @@ def test_products_against_float64_with_one_set_of_bits_a_row(rows, cols, splits,
     words = weight_like(rng, rows, cols)
     words[rng.random((rows, cols)) < 0.02] = 0  # (listed)
     p = _planes(words)
-    p.struct.splits, p.struct.parts = splits, parts
+    p.struct.splits = splits
     around = torch.full((130, cols + 8), float("nan"), device="cuda", dtype=torch.bfloat16)
     x = around[1:129, :cols]  # rows apart, with what must not be read around them
     x.copy_(torch.from_numpy(rng.standard_normal((128, cols), dtype=np.float32)))
     bias = torch.from_numpy(rng.standard_normal(rows, dtype=np.float32)).cuda().bfloat16()
-    space = torch.empty(parts * 128 * rows + 64, device="cuda", dtype=torch.float32)
+    space = torch.empty(splits * 128 * rows + 64, device="cuda", dtype=torch.float32)
 
     def product(rows_of_x, m, packed=0, b=None):
         y = torch.full((m + 2, rows), 7.0, device="cuda", dtype=torch.bfloat16)
@@ -87,6 +87,53 @@ def test_products_against_float64_with_one_set_of_bits_a_row(rows, cols, splits,
         assert torch.equal(product(x, m), full[:m]), m
         xp = PackedActivations(x[:m])
         assert torch.equal(product(xp.buffer, m, packed=1), full[:m]), m
+
+
+@pytest.mark.parametrize("rows,cols", [(29968, 2320), (65555, 1040)])
+def test_rows_of_x_that_large_matrices_share_have_the_bits_of_single_ones(rows, cols):
+    import torch
+    from georefine_amd import _native
+    from georefine_amd.bitexact_context_gpu import PackedActivations
+    lib, g = _native.hip(), torch.Generator(device="cuda").manual_seed(rows)
+    words = (torch.randn(rows, cols, device="cuda", generator=g) * 0.02).bfloat16()
+    x = torch.randn(32, cols, device="cuda", generator=g).bfloat16()
+    p = _planes(words.view(torch.int16).cpu().numpy().view(np.uint16))
+
+    def product(rows_of_x, m, packed=0):
+        space = torch.empty(p.workspace(m) // 4 + 4, device="cuda", dtype=torch.float32)
+        y = torch.empty(m, rows, device="cuda", dtype=torch.bfloat16)
+        _launch(lib.grf_planes_linear, p.address, rows_of_x.data_ptr(), cols, m, packed, y.data_ptr(), None, space.data_ptr(), p.workspace(m))
+        return y
+
+    want = torch.cat([product(x[i:i + 1], 1) for i in range(32)])
+    exact = x.double() @ words.double().T
+    bound = exact.abs() * 2.0 ** -8 + x.double().abs() @ words.double().abs().T * cols * 2.0 ** -24
+    assert bool(((want.double() - exact).abs() <= bound).all())
+    for m in (8, 9, 16, 17, 32):
+        assert torch.equal(product(x, m), want[:m]), m
+        assert torch.equal(product(PackedActivations(x[:m]).buffer, m, packed=1), want[:m]), m
+
+
+def test_members_of_more_splits_than_the_largest_one_have_two_a_wave():
+    import ctypes
+    import torch
+    from georefine_amd import _native
+    lib, rng, cols = _native.hip(), np.random.default_rng(9), 2320  # ten visits
+    members = [_planes(weight_like(rng, rows, cols)) for rows in (900, 70, 33)]
+    for p, splits in zip(members, (3, 5, 10)):  # (the last one's ten need waves of two where three would do)
+        p.struct.splits = splits
+    x = torch.from_numpy(rng.standard_normal((40, cols), dtype=np.float32)).cuda().bfloat16()
+    for m in (1, 8, 12, 31, 40):
+        space = torch.empty(1 << 20, device="cuda", dtype=torch.float32)
+        alone, together = ([torch.empty(m, p.rows, device="cuda", dtype=torch.bfloat16) for p in members] for _ in range(2))
+        for p, y in zip(members, alone):
+            _launch(lib.grf_planes_linear, p.address, x.data_ptr(), cols, m, 0, y.data_ptr(), None, space.data_ptr(), space.numel() * 4)
+        for order in ((0, 1, 2), (2, 1, 0), (1, 2)):
+            n, of = len(order), lambda kind, values: (kind * len(values))(*values)
+            _launch(lib.grf_planes_group, n, of(ctypes.c_void_p, [members[i].address for i in order]), x.data_ptr(), cols, m, 0,
+                    of(ctypes.c_void_p, [together[i].data_ptr() for i in order]), of(ctypes.c_uint32, [members[i].rows for i in order]), None,
+                    space.data_ptr(), space.numel() * 4)
+            assert all(torch.equal(together[i], alone[i]) for i in order), (m, order)
 
 
 def test_infinities_and_nan_go_where_the_dense_product_puts_them():

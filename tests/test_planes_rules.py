@@ -16,17 +16,17 @@ def test_sizes_are_the_librarys_and_no_split_is_empty(rows, cols):
     lib = _native.hip()
     assert _planes.plane_bytes(rows, cols) == lib.grf_planes_bytes(rows, cols)
     assert -(-rows // 16) * _planes.visits(cols) == lib.grf_planes_visits(rows, cols)
-    splits, parts = _planes.sum_splits(rows, cols)
+    splits = _planes.sum_splits(rows, cols)
     each = -(-_planes.visits(cols) // splits)
-    assert 1 <= splits <= 16 and splits % parts == 0 and splits // parts <= 2
+    assert 1 <= splits <= 16
     assert (splits - 1) * each < _planes.visits(cols) and each <= 63
 
 
-@pytest.mark.parametrize("change", [dict(splits=0), dict(splits=17), dict(splits=4), dict(parts=0), dict(cols=1028), dict(cols=1 << 18), dict(rows=0),
+@pytest.mark.parametrize("change", [dict(splits=0), dict(splits=17), dict(splits=4), dict(cols=1028), dict(cols=1 << 18), dict(rows=0),
                                     dict(planes=8), dict(listed=None)])
 def test_what_the_kernels_would_not_take_is_refused_before_a_launch(change):
     lib = _native.hip()
-    good = dict(planes=4096, bases=4096, listed_at=4096, listed=4096, rows=64, cols=1024, splits=2, parts=1)
+    good = dict(planes=4096, bases=4096, listed_at=4096, listed=4096, rows=64, cols=1024, splits=2)
     if change.get("splits") == 4:
         good.update(cols=1280)  # five visits, two a split: nothing is left for the fourth
     p = _hip_abi.GrfPlanes(**{**good, **change})
