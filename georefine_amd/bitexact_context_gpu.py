@@ -435,6 +435,76 @@ class _Prepared(dict):
         return _Prepared, ((info, *self._read[1:]), dict(self))
 
 
+def planes_product(tensor, p, x, bias):
+    """A product of a tensor that is held as the planes ``p``, of any number of rows; a row's bits depend on neither
+    the batch nor the call.  (Nothing is walked, so there is no checkpoint to miss.)"""
+    import torch
+    rows, cols = tensor.shape
+    packed = isinstance(x, PackedActivations)
+    if packed:
+        if x.cols != cols or x.buffer.device != tensor.device:
+            raise ValueError("packed activations of another width or device")
+        lead, m, ldx, x2 = x.lead, x.rows, cols, x.buffer
+        y = tensor.error.new_empty((*lead, rows), dtype=torch.bfloat16)
+    else:
+        if x.dtype is not torch.bfloat16 or x.shape[-1] != cols:
+            raise ValueError("activation must be bfloat16 with the weight's input width")
+        x2, ldx = rows_for(x, cols, tensor._index, tensor.device)
+        if not cols <= ldx <= 1 << 24:  # (rows that overlap, or lie too far apart)
+            x2, ldx = x2.reshape(-1, cols).clone(memory_format=torch.contiguous_format), cols
+        m = x2.numel() // cols
+        y = x2.new_empty((*x.shape[:-1], rows))
+    if m:
+        bias = bias_for(bias, tensor._index, tensor.device)
+        size = p.workspace(m) if m > _planes.OWN_ROWS else 0
+        space = tensor.error.new_empty(size // 4) if size else None
+        status = launch_on(tensor._index, tensor._lib.grf_planes_linear, p.address, x2.data_ptr(), ldx, m, packed, y.data_ptr(),
+                           bias.data_ptr() if bias is not None else None, space.data_ptr() if size else None, size)
+        if status:
+            tensor._raise_launch(status)
+    return y
+
+
+def planes_group(owner, planes, x, biases):
+    """The products of members that are held as ``planes`` (None: another launch's), in one launch: [y or None].  ``owner``
+    is the group."""
+    import torch
+    n, outs = len(planes), [None] * len(planes)
+    held = [i for i in range(n) if planes[i] is not None]
+    cols, packed = planes[held[0]].cols, isinstance(x, PackedActivations)
+    if packed:
+        if x.cols != cols or x.buffer.device != owner.device:
+            raise ValueError("packed activations of another width or device")
+        x2, ldx, m, lead = x.buffer, cols, x.rows, x.lead
+    else:
+        if x.dtype is not torch.bfloat16 or x.shape[-1] != cols:
+            raise ValueError("activation must be bfloat16 with the weights' input width")
+        m, lead = math.prod(x.shape[:-1]), tuple(x.shape[:-1])
+        x2, ldx = rows_for(x, cols, owner._index, owner.device)
+        if not cols <= ldx <= 1 << 24:  # (rows that overlap, or lie too far apart)
+            x2, ldx = x2.reshape(-1, cols).clone(memory_format=torch.contiguous_format), cols
+    for i in held:
+        outs[i] = owner.error.new_empty((*lead, planes[i].rows), dtype=torch.bfloat16)
+    if m:
+        count = len(held)
+        biases = [bias_for(biases[i], owner._index, owner.device) for i in held] if biases is not None else None
+        addresses = [planes[i].address for i in held]
+        kept = owner._pointer_arrays.get("planes")
+        if kept is None or kept[0] != addresses:
+            kept = owner._pointer_arrays["planes"] = (
+                addresses, (ctypes.c_void_p * count)(*addresses), (ctypes.c_uint32 * count)(*[planes[i].rows for i in held]), ctypes.c_void_p * count)
+        _, members, ldy, pointers = kept
+        size = sum(planes[i].workspace(m) for i in held) if m > _planes.OWN_ROWS else 0
+        space = owner.error.new_empty(size // 4) if size else None
+        status = launch_on(owner._index, owner._lib.grf_planes_group, count, members, x2.data_ptr(), ldx, m, packed,
+                           pointers(*[outs[i].data_ptr() for i in held]), ldy,
+                           pointers(*[b.data_ptr() if b is not None else None for b in biases]) if biases is not None else None,
+                           space.data_ptr() if size else None, size)
+        if status:
+            raise base.CodecError(f"device launch failed ({status}): " + owner._lib.grf_last_error().decode(errors="replace"))
+    return outs
+
+
 class HipContextTensor:
     """A BCTX-coded BF16 matrix resident on one MI355X."""
 
@@ -512,6 +582,7 @@ class HipContextTensor:
     # are held so from the start, and a tensor whose arrays, plan or descriptors are asked for, for the C interface
     # or to be looked at, is put into that form then, and stays in it.
     _planes = None
+    _used = None  # the form that the tensor was held in before
     _STREAM_FORM = frozenset(("buffers", "fused", "fused_plan", "_plan", "_frame", "_tilings", "_workspace", "_gather", "_main_bytes",
                               "_raw6_segment", "_raw6_block", "_gather_waves"))
 
@@ -542,13 +613,14 @@ class HipContextTensor:
         with _form_lock:
             if self._planes is None and self._sections is not None and self.fused is not None:
                 self._hold_planes(self.decode(check=False).view(torch.int16))
-                for name in HipContextTensor._STREAM_FORM:
-                    self.__dict__.pop(name, None)
+                # (kept: calls of other threads and streams and captured launches may be reading them, and small tensors do this)
+                self._used = [self.__dict__.pop(name, None) for name in HipContextTensor._STREAM_FORM]
         return self._planes is not None
 
     def _leave_planes(self):
         """The frame's arrays in the planes' place: the words, coded once more with the frame's own labels and frequencies,
-        which gives the same main stream, and packed residuals, the form that the walk takes."""
+        which gives the same main stream, and packed residuals, the form that the walk takes.  The planes stay allocated:
+        calls of other threads and streams and captured launches may be reading them."""
         import zlib
         import torch
         words = self.decode(check=False).view(torch.int16).cpu().numpy().view(np.uint16)
@@ -563,7 +635,8 @@ class HipContextTensor:
         segment = _fused.choose_segment(self.shape[1], self.asked_segment, rows=self.shape[0])
         self._hold_streams(_stream_arrays(_read_frame(frame, self.stride, segment, True), True, self._block))
         self._plan_gather()
-        self._planes = self._sections = None
+        self._used, self._planes, self._sections = self._planes, None, None
+        self.resident_bytes += self._used.nbytes
 
     def _hold_streams(self, prepared):
         """The device arrays of a frame that is walked where it lies."""
@@ -654,12 +727,13 @@ class HipContextTensor:
         import copy
         import torch
         other = copy.copy(self)
-        if self._planes is not None:
+        other._used = None
+        if other._planes is not None:
             if residual_block is not None:
                 if residual_block not in (1, 2, 4, 8, 16):
                     raise ValueError("residual blocks have 1, 2, 4, 8 or 16 rows")
                 other._block = residual_block
-            other._planes = self._planes.clone()
+            other._planes = other._planes.clone()
             other.error = torch.zeros_like(self.error)
             return other
         other.buffers = _Buffers((k, v.clone()) for k, v in self.buffers.items())
@@ -775,9 +849,10 @@ class HipContextTensor:
         """Dense BF16 matrix.  Fused frames use the store sink of the fused walker;
         ``general=True`` forces the one-lane-per-segment kernel."""
         import torch
-        if self._planes is not None and not general:
+        p = self._planes  # (another thread may ask for the arrays)
+        if p is not None and not general:
             out = torch.empty(self.shape, device=self.device, dtype=torch.bfloat16)
-            self._launch(self._lib.grf_planes_decode, self._planes.address, out.data_ptr())
+            self._launch(self._lib.grf_planes_decode, p.address, out.data_ptr())
             return out
         if self.mode == 1:
             return self.buffers["raw"].view(torch.bfloat16).reshape(self.shape)
@@ -856,42 +931,14 @@ class HipContextTensor:
                 self._check(check)
         return y
 
-    def _planes_call(self, x, bias):
-        """A product of a tensor that is held as planes, of any number of rows; a row's bits depend on neither
-        the batch nor the call.  (Nothing is walked, so there is no checkpoint to miss.)"""
-        import torch
-        rows, cols = self.shape
-        p, packed = self._planes, isinstance(x, PackedActivations)
-        if packed:
-            if x.cols != cols or x.buffer.device != self.device:
-                raise ValueError("packed activations of another width or device")
-            lead, m, ldx, x2 = x.lead, x.rows, cols, x.buffer
-            y = self.error.new_empty((*lead, rows), dtype=torch.bfloat16)
-        else:
-            if x.dtype is not torch.bfloat16 or x.shape[-1] != cols:
-                raise ValueError("activation must be bfloat16 with the weight's input width")
-            x2, ldx = rows_for(x, cols, self._index, self.device)
-            if not cols <= ldx <= 1 << 24:  # (rows that overlap, or lie too far apart)
-                x2, ldx = x2.reshape(-1, cols).clone(memory_format=torch.contiguous_format), cols
-            m = x2.numel() // cols
-            y = x2.new_empty((*x.shape[:-1], rows))
-        if m:
-            bias = bias_for(bias, self._index, self.device)
-            size = p.workspace(m) if m > _planes.OWN_ROWS else 0
-            space = self.error.new_empty(size // 4) if size else None
-            status = launch_on(self._index, self._lib.grf_planes_linear, p.address, x2.data_ptr(), ldx, m, packed, y.data_ptr(),
-                               bias.data_ptr() if bias is not None else None, space.data_ptr() if size else None, size)
-            if status:
-                self._raise_launch(status)
-        return y
-
     def gemv(self, x, bias=None, *, check=False):
         """Fused decode-GEMV (vector ALUs) for 1..8 activation rows; the result of a row does
         not depend on how many rows the call carries."""
-        if self._planes is not None:
+        p = self._planes
+        if p is not None:
             if not 1 <= (x.numel() // x.shape[-1] if x.shape[-1] else 0) <= 8:
                 raise ValueError("gemv takes 1..8 activation rows")
-            return self._planes_call(x, bias)
+            return planes_product(self, p, x, bias)
         if self.fused is None:
             raise base.CodecError("frame is not eligible for the fused kernels: " + self.fused_reason)
         m = x.numel() // x.shape[-1] if x.shape[-1] else 0
@@ -902,8 +949,9 @@ class HipContextTensor:
     def gemm(self, x, bias=None, *, check=False):
         """Fused decode-GEMM (matrix cores) for any number of activation rows, batch-invariant:
         a row's output bits are the same whatever else is in the batch."""
-        if self._planes is not None:
-            return self._planes_call(x, bias)
+        p = self._planes
+        if p is not None:
+            return planes_product(self, p, x, bias)
         if self.fused is None:
             raise base.CodecError("frame is not eligible for the fused kernels: " + self.fused_reason)
         if isinstance(x, PackedActivations):
@@ -929,9 +977,10 @@ class HipContextTensor:
             batch_invariant = self.m_invariant
         width = x.shape[-1]
         m = x.numel() // width if width else math.prod(x.shape[:-1])
-        held = self._planes is not None
+        p = self._planes
+        held = p is not None
         if held and (m <= DENSE_ABOVE or batch_invariant):
-            return self._planes_call(x, bias)
+            return planes_product(self, p, x, bias)
         route = "dense" if held or self.fused is None else route_rows(m, self.shape[1], batch_invariant)
         if route == "dense":
             import torch
@@ -956,8 +1005,9 @@ class HipContextTensor:
             ids = ids.to(device=self.device, dtype=torch.int64)
         if ids.numel() == 0:
             return torch.empty((*ids.shape, self.shape[1]), device=self.device, dtype=torch.bfloat16)
-        if self._planes is not None:
-            return self._gather_planes(ids, validate)
+        p = self._planes
+        if p is not None:
+            return self._gather_planes(p, ids, validate)
         self._plan_gather()
         if self.fused is not None and self._gather:
             return self._gather_fused(ids, check, validate)
@@ -1038,12 +1088,12 @@ class HipContextTensor:
             _done_counters[self._index].append(counters)
         return found & ~_hip_abi.GATHER_DONE
 
-    def _gather_planes(self, ids, validate):
+    def _gather_planes(self, p, ids, validate):
         """Of a tensor that is held as planes: one launch, of whose findings only refused ids are left to wait for."""
         import torch
         ids = ids.contiguous()
         out = torch.empty((*ids.shape, self.shape[1]), device=self.device, dtype=torch.bfloat16)
-        about = self._planes.address, ids.data_ptr(), ids.numel(), out.data_ptr()
+        about = p.address, ids.data_ptr(), ids.numel(), out.data_ptr()
         launch = lambda where, counters: self._launch(self._lib.grf_planes_gather, *about, where,
                                                       counters.data_ptr() if counters is not None else None,
                                                       where if counters is not None else None)
@@ -1153,7 +1203,7 @@ class HipLinearGroup:
                     for t, b in zip(self.tensors, biases if biases is not None else [None] * n)]
         planes = [t._planes for t in self.tensors]
         if any(p is not None for p in planes):
-            return self._linear_planes(planes, x, m, lead, biases, check, batch_invariant)
+            return self._linear_planes(planes, x, biases, check, batch_invariant)
         if packed is not None:
             if packed.cols != cols or packed.buffer.device != self.device:
                 raise ValueError("packed activations of another width or device")
@@ -1193,51 +1243,17 @@ class HipLinearGroup:
         return outs
 
 
-    def _linear_planes(self, planes, x, m, lead, biases, check, batch_invariant):
+    def _linear_planes(self, planes, x, biases, check, batch_invariant):
         """Up to 128 rows of a group some of whose members are held as planes: one launch for those, and one for the rest."""
-        import torch
-        n, outs = len(planes), [None] * len(planes)
-        held = [i for i in range(n) if planes[i] is not None]
-        if len(held) < n:
-            rest = [i for i in range(n) if planes[i] is None]
-            if self._walked is None or self._walked[0] != rest:
-                self._walked = rest, HipLinearGroup([self.tensors[i] for i in rest], m_invariant=self.m_invariant)
-            walked = self._walked[1].linear(x, [biases[i] for i in rest] if biases is not None else None, check=check,
-                                            batch_invariant=batch_invariant)
-            for i, y in zip(rest, walked):
+        outs = planes_group(self, planes, x, biases)
+        rest = [i for i, p in enumerate(planes) if p is None]
+        if rest:
+            walked = self._walked
+            if walked is None or walked[0] != rest:
+                walked = self._walked = rest, HipLinearGroup([self.tensors[i] for i in rest], m_invariant=self.m_invariant)
+            for i, y in zip(rest, walked[1].linear(x, [biases[i] for i in rest] if biases is not None else None, check=check,
+                                                   batch_invariant=batch_invariant)):
                 outs[i] = y
-        cols, packed = self.tensors[0].shape[1], isinstance(x, PackedActivations)
-        if packed:
-            if x.cols != cols or x.buffer.device != self.device:
-                raise ValueError("packed activations of another width or device")
-            x2, ldx = x.buffer, cols
-        else:
-            if x.dtype is not torch.bfloat16 or x.shape[-1] != cols:
-                raise ValueError("activation must be bfloat16 with the weights' input width")
-            x2, ldx = rows_for(x, cols, self._index, self.device)
-            if not cols <= ldx <= 1 << 24:  # (rows that overlap, or lie too far apart)
-                x2, ldx = x2.reshape(-1, cols).clone(memory_format=torch.contiguous_format), cols
-        for i in held:
-            outs[i] = self.error.new_empty((*lead, self.tensors[i].shape[0]), dtype=torch.bfloat16)
-        if m:
-            count = len(held)
-            biases = [bias_for(biases[i], self._index, self.device) for i in held] if biases is not None else None
-            kept = self._pointer_arrays.get("planes")
-            if kept is None or kept[0] != [planes[i].address for i in held]:
-                kept = self._pointer_arrays["planes"] = (
-                    [planes[i].address for i in held], (ctypes.c_void_p * count)(*[planes[i].address for i in held]),
-                    (ctypes.c_uint32 * count)(*[planes[i].rows for i in held]), ctypes.c_void_p * count)
-            _, members, ldy, pointers = kept
-            size = 0
-            if m > _planes.OWN_ROWS:
-                size = sum(planes[i].workspace(m) for i in held)
-            space = self.error.new_empty(size // 4) if size else None
-            status = launch_on(self._index, self._lib.grf_planes_group, count, members, x2.data_ptr(), ldx, m, packed,
-                               pointers(*[outs[i].data_ptr() for i in held]), ldy,
-                               pointers(*[b.data_ptr() if b is not None else None for b in biases]) if biases is not None else None,
-                               space.data_ptr() if size else None, size)
-            if status:
-                raise base.CodecError(f"device launch failed ({status}): " + self._lib.grf_last_error().decode(errors="replace"))
         return outs
 
 

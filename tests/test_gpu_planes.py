@@ -226,3 +226,9 @@ def test_captured_launches_replay_on_new_rows():
         graph.replay()
         torch.cuda.synchronize()
         assert all(torch.equal(a.view(torch.int16), b.view(torch.int16)) for a, b in zip(captured, eager))
+    assert t.buffers["main_stream"].is_cuda and t._planes is None  # what was captured still reads the planes
+    torch.cuda.empty_cache()
+    x1.copy_(draw(1)), x40.copy_(draw(40))
+    graph.replay()
+    want = t.take_planes() or group.tensors[1].linear(x1)  # (the clone's planes, the same words)
+    assert torch.equal(captured[0], want) and torch.equal(captured[1], captured[2])
