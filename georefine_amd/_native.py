@@ -135,6 +135,7 @@ def codec():
             L.grf_order_records.restype = _int
             L.grf_unit_pieces.argtypes = [U32P, _u32, _u32, U32P, _u32, _u32, U32P]
             L.grf_unit_pieces.restype = _int
+            L.ppcx_encode_given.argtypes = [U16P, U16P, _u64, _u32, _u32, U32P, ctypes.POINTER(U8P), ctypes.POINTER(_sz)]
             L.p_encode.argtypes = [U16P, U16P, _u64, _u32, _u32, ctypes.POINTER(U32P), ctypes.POINTER(U8P),
                                    ctypes.POINTER(_sz)]
             L.p_decode.argtypes = [U8P, _sz, _u64, U16P, _u32, _u32, U32P, U16P]
@@ -143,7 +144,7 @@ def codec():
             L.ppcx_checkpoint.argtypes = [U8P, _sz, _u64, U16P, _u32, _u32, U32P, _u32, U32P, U32P, U16P]
             L.ppcx_checkpoint_binary.argtypes = L.ppcx_checkpoint.argtypes
             for name in ("bcx_encode", "bcx_frequencies", "bcx_decode", "bcx_decode_compact", "bcx_pack6",
-                         "bcx_unpack6", "bcx_checkpoint", "p_encode", "p_decode", "ppcx_checkpoint",
+                         "bcx_unpack6", "bcx_checkpoint", "p_encode", "ppcx_encode_given", "p_decode", "ppcx_checkpoint",
                          "ppcx_checkpoint_binary"):
                 getattr(L, name).restype = _int
             _codec = L

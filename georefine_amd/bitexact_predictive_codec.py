@@ -202,6 +202,21 @@ def _rans_encode(vals, ctx, nctx, vocab):
     return zlib.compress(table, 6), data
 
 
+def _encode_given(vals, ctx, freq):
+    """The main stream of symbols that were decoded with these frequencies, as ``encode`` would give it."""
+    lib = _lib()
+    vals, ctx, freq = (np.ascontiguousarray(a, dtype=t) for a, t in ((vals, "<u2"), (ctx, "<u2"), (freq, "<u4")))
+    stream, size = _native.U8P(), ctypes.c_size_t()
+    status = lib.ppcx_encode_given(_native.ptr(vals, ctypes.c_uint16), _native.ptr(ctx, ctypes.c_uint16), vals.size, MAIN_CONTEXTS, MAIN_VOCAB,
+                                   _native.ptr(freq, ctypes.c_uint32), ctypes.byref(stream), ctypes.byref(size))
+    if status:
+        raise CodecError(f"rANS encode failed ({status})")
+    try:
+        return ctypes.string_at(stream, size.value)
+    finally:
+        lib.p_free(stream)
+
+
 def _rans_decode(stream, ctx, nctx, vocab, freq, what):
     if len(stream) < 4:
         raise CodecError(f"{what} stream truncated")

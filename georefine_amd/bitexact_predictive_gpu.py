@@ -6,7 +6,9 @@
 ``shape``, ``frame_sha256``, ``source_sha256``, ``resident_bytes`` and
 ``decode(reference_bf16_device, check=)``.  The reference words are an input of every
 decode: the kernel derives each symbol's context from the reference word at the same
-position (sign alignment per row, ordinal key, threshold bin).
+position (sign alignment per row, ordinal key, threshold bin).  A tensor that keeps its contexts
+needs no reference in a call; its words are then held as planes (``_planes``: 96 rows of 4096 x 4096
+23.5 us where the walk takes 40.8, in 24 MB where that takes 34), small ones as the frame's arrays.
 """
 from __future__ import annotations
 
@@ -17,7 +19,7 @@ import os
 
 import numpy as np
 
-from . import _fused, _hip_abi, _native, _tables
+from . import _fused, _hip_abi, _native, _planes, _tables
 from . import bitexact_predictive_codec as codec
 
 
@@ -98,8 +100,15 @@ def _read_frame(frame, reference, stride, *, fused=False, fused_segment=None):
             raise codec.CodecError("target checksum mismatch")
         result["raw"] = target
         return result
-    freq = info["main_freq"].reshape(codec.MAIN_CONTEXTS, codec.MAIN_VOCAB)
     ctx = codec.contexts(info["reference"], info["labels"], info["flips"], info["thresholds"])
+    return _indexed(result, info, ctx, stride, fused, fused_segment)
+
+
+def _indexed(result, info, ctx, stride, fused, fused_segment):
+    """``_read_frame`` from the sections of a frame and the contexts on."""
+    r, c = result["shape"]
+    n, target_hash = r * c, bytes.fromhex(result["target_sha256"])
+    freq = info["main_freq"].reshape(codec.MAIN_CONTEXTS, codec.MAIN_VOCAB)
     seg_len = None
     if fused:
         try:
@@ -145,6 +154,48 @@ def _read_frame(frame, reference, stride, *, fused=False, fused_segment=None):
     return result
 
 
+def _read_words(frame, reference, stride, fused_segment):
+    """The words of a frame that can be held as planes, validated, with what is needed to make its arrays later (``_indexed``); None
+    of one that cannot: what the fused kernels refuse, raw words and small matrices (``_planes``)."""
+    if not isinstance(frame, (bytes, bytearray, memoryview)) or len(frame) < codec.HEADER.size:
+        return None  # (``_read_frame`` says what is wrong)
+    mode, (r, c) = frame[5], codec.HEADER.unpack_from(frame)[4:6]
+    n = r * c
+    if mode == 2 or n < _planes.FROM_WEIGHTS or c > _planes.MAX_COLS:
+        return None
+    try:
+        seg_len = _fused_segment((r, c), fused_segment)
+    except _fused.FusedUnsupported:
+        return None
+    info = codec.parse(frame, reference)
+    freq = info["main_freq"].reshape(codec.MAIN_CONTEXTS, codec.MAIN_VOCAB)
+    live, sums = (freq > 0).sum(axis=1), freq.sum(axis=1, dtype=np.uint64)
+    if not 0 < live.max() <= 255 or not np.isin(sums, (0, 65536)).all():
+        return None
+    ctx = codec.contexts(info["reference"], info["labels"], info["flips"], info["thresholds"])
+    _, _, main = _checkpoints(info["stream"], ctx, freq, codec.MAIN_VOCAB, stride)
+    if mode == 0:
+        residual = codec._unpackbits(info["data"], 5, n, "raw5")
+    else:
+        rf = info["residual_freq"].reshape(codec.RES_CONTEXTS, codec.RES_VOCAB)
+        _, _, residual = _checkpoints(info["residual_stream"], main, rf, codec.RES_VOCAB, stride)
+    words = codec.join_symbols(main, residual)
+    if hashlib.sha256(words.tobytes()).digest() != info["target_sha256"]:
+        raise codec.CodecError("target checksum mismatch")
+    about = dict(shape=(r, c), mode=mode, frame_bytes=len(frame), frame_sha256=hashlib.sha256(bytes(frame)).hexdigest(),
+                 source_sha256=info["target_sha256"].hex(), target_sha256=info["target_sha256"].hex(),
+                 reference_sha256=info["reference_sha256"].hex())
+    # what the arrays of the walk would take: streams, bins, the index and the tables
+    walked = len(info["stream"]) + n * 9 // 8 + 8 * r * (c // seg_len + 1) + 16 * (16 * 8 * (int(live.max()) + 1) + _LUT_BUDGET)
+    return dict(about=about, words=words.view(np.int16).reshape(r, c), bins=_pairs(ctx), meta=info["meta"], table=info["table"], walked=walked)
+
+
+def _pairs(ctx):
+    """The bins of contexts (their low four bits), two a byte, as the device's plane has them."""
+    low = ctx.astype(np.uint8) & 15
+    return low[0::2] | low[1::2] << 4
+
+
 class HipPredictiveTensor:
     """A PPCX-coded BF16 matrix resident on one MI355X; decoding needs the reference matrix."""
 
@@ -155,52 +206,24 @@ class HipPredictiveTensor:
                  fused_segment=None, resident_contexts=True, m_invariant=False):
         if not isinstance(stride, int) or not 1 <= stride <= 65536:
             raise codec.CodecError("invalid checkpoint stride")
-        ix = _read_frame(frame, reference_uint16_numpy, stride, fused=fused, fused_segment=fused_segment)
+        read = _read_words(frame, reference_uint16_numpy, stride, fused_segment) if fused and resident_contexts else None
+        ix = _read_frame(frame, reference_uint16_numpy, stride, fused=fused, fused_segment=fused_segment) if read is None else None
         import torch
         if not torch.cuda.is_available():
             raise RuntimeError("a ROCm GPU is required")
+        from .bitexact_context_gpu import device_index
         self._lib = _native.hip()
         self.m_invariant = bool(m_invariant)  # linear()'s default for batch_invariant
-        self.shape = ix["shape"]
-        self.n = math.prod(self.shape)
-        self.stride, self.mode = stride, ix["mode"]
-        self.resident_mode = ix.get("resident_mode", self.mode)
-        self._plan = ix.pop("fused_plan", None)         # of grouped matrix-core launches ...
-        self._matrix_plan = ix.pop("matrix_plan", None)  # ... of the others of these ...
-        self._walk_plan = ix.pop("walk_plan", None)     # ... and of one row and the store sink (one plan for most matrices)
-        self.fused_reason = ix.pop("fused_reason", None)
+        self.stride = stride
         self.device = torch.device(device)
-        for key in ("source_sha256", "target_sha256", "reference_sha256", "frame_sha256", "frame_bytes"):
-            setattr(self, key, ix[key])
-        self.buffers = {}
-        # The packed residuals -- and the plane of reference bins made below -- in the order the
-        # tile walker reads them: records of 32 symbols (20 and 16 bytes), rows by label as the
-        # tilings take them, in blocks of as many rows as a wave unit of the GEMV has; inside a
-        # block by position in the segment, then by segment, then by row (the order the context
-        # codec's tensors give their 12-byte groups, for the same reason: the lanes of a unit then
-        # read one run of bytes per visit and a 128-byte line is not visited four times).
-        self._raw5_segment = self._raw5_block = self._rows_held = 0
-        if self._plan is not None and "raw5" in ix and self.resident_mode == 0:
-            block, position, held = self._walk_plan.residual_order()
-            rows_, cols_ = self.shape
-            ix["raw5"] = _fused.order_records(ix["raw5"], rows_, cols_, self._plan.seg_len, block, position, held, 32, 20)
-            ix["row_pos"] = position
-            self._raw5_segment, self._raw5_block, self._rows_held = self._plan.seg_len, block, held
-        for name, array in ix.items():
-            if isinstance(array, np.ndarray) and name != "residual_symbols":
-                if name in ("raw5", "main_stream"):  # the kernels read whole dwords / 16-byte chunks at the end
-                    array = np.concatenate((array, np.zeros(16, dtype=np.uint8)))
-                self.buffers[name] = torch.from_numpy(np.ascontiguousarray(array)).to(self.device)
-        for name in ("main", "residual"):
-            if name + "_freq" in ix:
-                cum = _tables.cumulative(ix[name + "_freq"])
-                self.buffers[name + "_cum"] = torch.from_numpy(cum).to(self.device)
-                self.buffers[name + "_bucket"] = torch.from_numpy(_tables.coarse_buckets(cum)).to(self.device)
-        self.error = torch.zeros((), device=self.device, dtype=torch.int32)
-        from .bitexact_context_gpu import device_index
         self._index = device_index(self.device)
-        self._tilings, self._workspace = {}, {}
-        self._bind()
+        self._asked_segment = fused_segment
+        self.error = torch.zeros((), device=self.device, dtype=torch.int32)
+        if read is not None and self._hold_planes(read):
+            return
+        if ix is None:
+            ix = _read_frame(frame, reference_uint16_numpy, stride, fused=fused, fused_segment=fused_segment)
+        self._hold_streams(ix)
         # What the tile walker needs of the reference is the 4-bit bin of every word (the
         # decoded word itself comes from the frame's symbols alone), and the reference is given
         # here, once.  Keeping that plane, half a byte per weight, takes the reference out of
@@ -219,6 +242,115 @@ class HipPredictiveTensor:
             self.buffers["context_bins"] = bins
             self.has_contexts = True
             del ref
+
+    # As the context codec's tensors are (``HipContextTensor``), one that keeps its contexts is held in one of two forms: the
+    # words laid out as planes, which need no contexts and take the memory of the frame with them, or the frame's own
+    # arrays, which a tensor is put into when they, a plan or a descriptor are asked for.
+    _planes = None
+    _used = None  # the planes that the tensor was held as before
+    _STREAM_FORM = frozenset(("buffers", "fused", "fused_gemm", "fused_matrix", "fused_plan", "_plan", "_matrix_plan", "_walk_plan", "_frame",
+                              "_tilings", "_workspace", "_raw5_segment", "_raw5_block", "_rows_held"))
+
+    def __getattr__(self, name):  # (only of what the object does not have)
+        if name in HipPredictiveTensor._STREAM_FORM and self.__dict__.get("_planes") is not None:
+            from .bitexact_context_gpu import _form_lock
+            with _form_lock:
+                if self._planes is not None:
+                    self._leave_planes()
+            return getattr(self, name)
+        raise AttributeError(f"{type(self).__name__!r} object has no attribute {name!r}")
+
+    @property
+    def fusable(self):
+        """Whether products take a kernel of their own (``fused``, asked without changing the form a tensor is held in)."""
+        return self._planes is not None or self.fused is not None
+
+    def _launch(self, fn, *args):
+        from .bitexact_context_gpu import launch_on
+        self._status(launch_on(self._index, fn, *args), False)
+
+    def _hold_planes(self, read):
+        """Holds the words as planes unless they list so many that the walk's arrays are smaller."""
+        import torch
+        planes = _planes.Planes.of_words(torch.from_numpy(read["words"]).to(self.device), self._launch)
+        if planes.nbytes > _planes.MEMORY * read["walked"]:
+            return False
+        torch.cuda.current_stream(self.device).synchronize()  # (a first product may be on another stream)
+        for name, value in read["about"].items():
+            setattr(self, name, value)
+        self.n = math.prod(self.shape)
+        self.resident_mode, self.fused_reason, self.has_contexts = 0, None, True
+        self._kept = {name: read[name] for name in ("bins", "meta", "table")}
+        self._planes = planes
+        return True
+
+    def _leave_planes(self):
+        """The frame's arrays in the planes' place: the words, coded once more with the frame's own frequencies in the
+        contexts that were kept of the reference, which gives the same main stream, and packed residuals.  The planes
+        stay allocated: calls of other threads and streams and captured launches may be reading them."""
+        import torch
+        r, c = self.shape
+        words = self.decode(None, check=False).view(torch.int16).cpu().numpy().view(np.uint16)
+        main, residual = codec.split_symbols(words.reshape(-1))
+        meta = codec._inflate(self._kept["meta"], 2 * r + 30)
+        labels, flips = (np.frombuffer(meta[i * r:(i + 1) * r], dtype=np.uint8).copy() for i in range(2))
+        freq = np.frombuffer(codec._inflate(self._kept["table"], codec.MAIN_CONTEXTS * codec.MAIN_VOCAB * 4), dtype="<u4").copy()
+        bins = self._kept["bins"]
+        ctx = np.repeat(labels.astype(np.uint16) * 16, c)
+        ctx[0::2] += bins & 15
+        ctx[1::2] += bins >> 4
+        info = dict(mode=0, labels=labels, flips=flips, thresholds=np.frombuffer(meta[2 * r:], dtype="<u2").copy(), main_freq=freq,
+                    stream=codec._encode_given(main, ctx, freq), data=codec._packbits(residual, 5))
+        about = dict(shape=self.shape, mode=self.mode, target_sha256=self.target_sha256)
+        self._hold_streams(_indexed(about, info, ctx, self.stride, True, self._asked_segment))
+        if self._raw5_segment:
+            rows, cols = self.shape
+            bins = _fused.order_records(bins, rows, cols, self._raw5_segment, self._raw5_block, self.buffers["row_pos"].cpu().numpy(),
+                                        self._rows_held, 32, 16)
+        self.buffers["context_bins"] = torch.from_numpy(np.ascontiguousarray(bins).view(np.int32)).to(self.device)
+        self._used, self._planes, self._kept = self._planes, None, None
+
+    def _hold_streams(self, ix):
+        """The device arrays of a frame that is walked where it lies, from what ``_read_frame`` gave."""
+        import torch
+        self.shape = ix["shape"]
+        self.n = math.prod(self.shape)
+        self.mode = ix["mode"]
+        self.resident_mode = ix.get("resident_mode", self.mode)
+        self._plan = ix.pop("fused_plan", None)         # of grouped matrix-core launches ...
+        self._matrix_plan = ix.pop("matrix_plan", None)  # ... of the others of these ...
+        self._walk_plan = ix.pop("walk_plan", None)     # ... and of one row and the store sink (one plan for most matrices)
+        self.fused_reason = ix.pop("fused_reason", None)
+        for key in ("source_sha256", "target_sha256", "reference_sha256", "frame_sha256", "frame_bytes"):
+            if key in ix:
+                setattr(self, key, ix[key])
+        buffers = {}
+        # The packed residuals -- and the plane of reference bins made below -- in the order the
+        # tile walker reads them: records of 32 symbols (20 and 16 bytes), rows by label as the
+        # tilings take them, in blocks of as many rows as a wave unit of the GEMV has; inside a
+        # block by position in the segment, then by segment, then by row (the order the context
+        # codec's tensors give their 12-byte groups, for the same reason: the lanes of a unit then
+        # read one run of bytes per visit and a 128-byte line is not visited four times).
+        self._raw5_segment = self._raw5_block = self._rows_held = 0
+        if self._plan is not None and "raw5" in ix and self.resident_mode == 0:
+            block, position, held = self._walk_plan.residual_order()
+            rows_, cols_ = self.shape
+            ix["raw5"] = _fused.order_records(ix["raw5"], rows_, cols_, self._plan.seg_len, block, position, held, 32, 20)
+            ix["row_pos"] = position
+            self._raw5_segment, self._raw5_block, self._rows_held = self._plan.seg_len, block, held
+        for name, array in ix.items():
+            if isinstance(array, np.ndarray) and name != "residual_symbols":
+                if name in ("raw5", "main_stream"):  # the kernels read whole dwords / 16-byte chunks at the end
+                    array = np.concatenate((array, np.zeros(16, dtype=np.uint8)))
+                buffers[name] = torch.from_numpy(np.ascontiguousarray(array)).to(self.device)
+        for name in ("main", "residual"):
+            if name + "_freq" in ix:
+                cum = _tables.cumulative(ix[name + "_freq"])
+                buffers[name + "_cum"] = torch.from_numpy(cum).to(self.device)
+                buffers[name + "_bucket"] = torch.from_numpy(_tables.coarse_buckets(cum)).to(self.device)
+        self._tilings, self._workspace = {}, {}
+        self.buffers = buffers
+        self._bind()
 
     def _bind(self):
         """Descriptors over this object's device buffers (their addresses go into the structures
@@ -258,6 +390,11 @@ class HipPredictiveTensor:
         import copy
         import torch
         other = copy.copy(self)
+        other._used = None
+        if other._planes is not None:
+            other._planes = other._planes.clone()
+            other.error = torch.zeros_like(self.error)
+            return other
         other.buffers = {k: v.clone() for k, v in self.buffers.items()}
         other.error = torch.zeros_like(self.error)
         other._tilings, other._workspace = {}, {}
@@ -267,7 +404,10 @@ class HipPredictiveTensor:
     @property
     def resident_bytes(self):
         """Every device allocation this tensor holds: buffers, tilings made so far, the error word."""
-        total = sum(t.numel() * t.element_size() for t in self.buffers.values()) + 4
+        p = self._planes
+        if p is not None:
+            return p.nbytes + 4
+        total = sum(t.numel() * t.element_size() for t in self.buffers.values()) + 4 + (self._used.nbytes if self._used is not None else 0)
         total += sum(rows.numel() * 4 + classes.numel() for _, rows, classes, _ in self._tilings.values())
         return int(total)
 
@@ -383,7 +523,7 @@ class HipPredictiveTensor:
         if batch_invariant is None:  # the tensor's policy
             batch_invariant = self.m_invariant
         m = x.numel() // x.shape[-1] if x.shape[-1] else 0
-        if self.fused is None or x.dtype != torch.bfloat16:
+        if not self.fusable or x.dtype != torch.bfloat16:
             return torch.nn.functional.linear(x, self.decode(reference_bf16_device, check=check), bias)
         if m > self.DENSE_ABOVE and not batch_invariant:
             return dense_linear(self._lib, x, self.decode(reference_bf16_device, check=check), bias, self._index)
@@ -402,9 +542,14 @@ class HipPredictiveTensor:
 
     def _product(self, reference_bf16_device, x, bias, check, use_gemm):
         import torch
+        from .bitexact_context_gpu import PackedActivations, bias_for, launch_on, planes_product, rows_for
+        p = self._planes  # (another thread may ask for the arrays)
+        if p is not None:
+            if not use_gemm and isinstance(x, PackedActivations):
+                raise ValueError("packed activations go to the GEMM of a weight of their width on their device")
+            return planes_product(self, p, x, bias)
         if self.fused is None:
             raise codec.CodecError("frame is not eligible for the fused kernels: " + str(self.fused_reason))
-        from .bitexact_context_gpu import PackedActivations, bias_for, launch_on, rows_for
         packed = x if isinstance(x, PackedActivations) else None
         rows, cols = self.shape
         if packed is not None:
@@ -449,6 +594,9 @@ class HipPredictiveTensor:
             self._status(status, check)
         return y
 
+    def _raise_launch(self, status):
+        self._status(status, False)
+
     def _status(self, status, check):
         if status:
             raise codec.CodecError(f"device decode launch failed ({status}): "
@@ -460,6 +608,11 @@ class HipPredictiveTensor:
         """BF16 [rows, cols].  Frames the tile walker supports take two launches (bins of the
         reference, then the walk); ``general`` forces the one-lane-per-checkpoint kernel."""
         import torch
+        p = self._planes
+        if p is not None and not general:
+            out = torch.empty(self.shape, device=self.device, dtype=torch.bfloat16)
+            self._launch(self._lib.grf_planes_decode, p.address, out.data_ptr())
+            return out
         if self.mode == 2:
             return self.buffers["raw"].view(torch.bfloat16).reshape(self.shape)
         if self.fused is not None and not general:
@@ -502,7 +655,7 @@ class HipPredictiveGroup:
             raise ValueError("a group has 1..4 members")
         first = self.tensors[0]
         for t in self.tensors:
-            if t.fused is None:
+            if not t.fusable:
                 raise codec.CodecError("frame is not eligible for the fused kernels: " + str(t.fused_reason))
             if not t.has_contexts:
                 raise ValueError("group members keep their context planes resident (resident_contexts=True)")
@@ -512,7 +665,8 @@ class HipPredictiveGroup:
         self.m_invariant = any(t.m_invariant for t in self.tensors) if m_invariant is None else bool(m_invariant)
         self.error = torch.zeros((), device=self.device, dtype=torch.int32)
         self._tilings, self._pointer_arrays = {}, {}
-        for key in ("waves", "gemm"):
+        self._index, self._walked = first._index, None  # (members whose frames are walked, their group) where some are held as planes
+        for key in () if any(t._planes is not None for t in self.tensors) else ("waves", "gemm"):
             self._tiling(key)  # raises FusedUnsupported when the members cannot share a tiling
 
     def _tiling(self, key):
@@ -551,7 +705,7 @@ class HipPredictiveGroup:
         One activation row goes to the vector-ALU kernel, up to 128 to the matrix cores (every
         row count under ``batch_invariant``), more than that to the members' own ``linear``."""
         import torch
-        from .bitexact_context_gpu import PackedActivations, bias_for, launch_on, rows_for
+        from .bitexact_context_gpu import PackedActivations, bias_for, launch_on, planes_group, rows_for
         n = len(self.tensors)
         biases = list(biases) if biases is not None else [None] * n
         if len(biases) != n:
@@ -566,6 +720,17 @@ class HipPredictiveGroup:
         if packed is None and m > first.DENSE_ABOVE and not batch_invariant:
             return [t.linear(None, x, b, check=check, batch_invariant=False) for t, b in zip(self.tensors, biases)]
         use_gemm = packed is not None or batch_invariant or m > first.GEMV_UP_TO
+        planes = [t._planes for t in self.tensors]
+        if any(p is not None for p in planes):
+            outs = planes_group(self, planes, x, biases)
+            rest = [i for i, p in enumerate(planes) if p is None]
+            if rest:  # two kinds of members are two launches
+                walked = self._walked
+                if walked is None or walked[0] != rest:
+                    walked = self._walked = rest, HipPredictiveGroup([self.tensors[i] for i in rest], m_invariant=self.m_invariant)
+                for i, y in zip(rest, walked[1].linear(x, [biases[i] for i in rest], check=check, batch_invariant=batch_invariant)):
+                    outs[i] = y
+            return outs
         if packed is not None:
             if packed.cols != cols or packed.buffer.device != self.device:
                 raise ValueError("packed activations of another width or device")

@@ -1000,6 +1000,30 @@ int p_encode(const uint16_t *v, const uint16_t *cx, uint64_t n, uint32_t nc, uin
       5, 5);
 }
 
+// The stream that p_encode would give with the frequencies it is given, one thread, for symbols that were decoded with them.
+int ppcx_encode_given(const uint16_t *v, const uint16_t *cx, uint64_t n, uint32_t nc, uint32_t vocab, const uint32_t *freq,
+                      uint8_t **streamp, size_t *sn) {
+  return guarded(
+      [&]() -> int {
+        if (!v || !cx || !n || n > 100000000u || !nc || !vocab || vocab > kTotal || !freq || !streamp || !sn) return 1;
+        for (uint64_t i = 0; i < n; ++i)
+          if (cx[i] >= nc || v[i] >= vocab || !freq[(size_t)cx[i] * vocab + v[i]]) return 2;
+        const std::unique_ptr<uint8_t[]> bytes(new uint8_t[2 * n + 8]);
+        uint8_t *end = bytes.get() + 2 * n + 8;
+        const std::vector<EncodeCell> table = encode_cells(freq, nc, vocab);
+        const uint8_t *at = encode_stream(
+            n, [&](uint64_t i) -> const EncodeCell & { return table[(size_t)cx[i] * vocab + v[i]]; }, bytes.get(), end);
+        if (!at) return 3;
+        const size_t size = (size_t)(end - at);
+        auto *sp = (uint8_t *)std::malloc(size);
+        if (!sp) return 4;
+        std::memcpy(sp, at, size);
+        *streamp = sp, *sn = size;
+        return 0;
+      },
+      5, 5);
+}
+
 // Status categories follow GCR/bitexact_predictive_ans.cpp:11 (1 arguments,
 // 2 initial state, 3 table row overflow, 4 row does not sum to the total,
 // 5 context out of range, 8 stream exhausted, 9 terminal state/length).

@@ -32,6 +32,11 @@ def hip_tensor_factory(frame, *, stride=1024, device="cuda:0", fused_segment=Non
                             residual_block=residual_block)
 
 
+def fusable(native):
+    """Whether a native tensor's products take a kernel of their own."""
+    return native.fusable if hasattr(native, "fusable") else getattr(native, "fused", None) is not None
+
+
 def hip_predictive_factory(frame, reference_uint16_numpy, stride=1024, device="cuda:0", *, fused_segment=None):
     """The ``predictive_factory`` of ``load_predictive_model`` (GCR/bitexact_predictive_serving.py:918-924).
     ``fused_segment``: the tile walker's segment length, given by the loader to siblings that
@@ -242,7 +247,7 @@ class PredictiveContextTensor:
     def _needs_reference(self):
         """False when the native tensor keeps the contexts of its reference and takes the tile
         walker: nothing of the references is then read after load."""
-        return not (getattr(self.native, "has_contexts", False) and getattr(self.native, "fused", None) is not None)
+        return not (getattr(self.native, "has_contexts", False) and fusable(self.native))
 
     def reframe(self, tensor_factory, *, stride, device, encoder=None):
         """A frame stored transposed holds W^T row by row: the walk produces words along the
@@ -656,7 +661,7 @@ def load_bctx_model(package, *, model_factory, device="cuda:0", dtype=torch.bflo
         native = getattr(context, "row_major", None) or getattr(context, "native", context)
         if not hasattr(native, "resident_mode"):
             return {}
-        fused = native.fusable if hasattr(native, "fusable") else getattr(native, "fused", None) is not None
+        fused = fusable(native)
         reason = getattr(native, "fused_reason", "")
         return dict(frame_mode=native.mode, resident_mode=native.resident_mode,
                     residual_repacked=native.resident_mode != native.mode, fused=fused,

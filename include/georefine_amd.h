@@ -99,6 +99,9 @@ int grf_bctx_sums(const uint16_t *w, uint32_t rows, uint32_t cols, uint64_t *row
 /* GCR/bitexact_predictive_ans.cpp:10-12  generic context coder of the predictive frames */
 int p_encode(const uint16_t *v, const uint16_t *cx, uint64_t n, uint32_t nc, uint32_t vocab, uint32_t **freq,
              uint8_t **stream, size_t *stream_n);
+/* p_encode's stream with given frequencies, those that the symbols were decoded with */
+int ppcx_encode_given(const uint16_t *v, const uint16_t *cx, uint64_t n, uint32_t nc, uint32_t vocab, const uint32_t *freq,
+                      uint8_t **stream, size_t *stream_n);
 int p_decode(const uint8_t *st, size_t bytes, uint64_t n, const uint16_t *cx, uint32_t nc, uint32_t vocab,
              const uint32_t *freq, uint16_t *out);
 void p_free(void *p);

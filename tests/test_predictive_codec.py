@@ -295,3 +295,14 @@ def test_mix_validation_and_fit():
     coeff = fit_mixed_coefficients(target, up, gate)
     assert coeff[1, 0] == 0 and coeff[1, 1] == 0
     assert np.array_equal(predict(up, gate, coeff)[1], np.full(8, coeff[1, 2], dtype=np.uint16))
+
+
+def test_a_stream_is_coded_again_from_its_symbols_and_frequencies():
+    rng = np.random.default_rng(77)
+    ref = rng.integers(0x3A00, 0x3C00, (400, 960)).astype(np.uint16)
+    info = codec.parse(codec.encode(ref ^ rng.integers(0, 4, ref.shape).astype(np.uint16), ref), ref)
+    ctx = codec.contexts(info["reference"], info["labels"], info["flips"], info["thresholds"])
+    main = codec._rans_decode(info["stream"], ctx, codec.MAIN_CONTEXTS, codec.MAIN_VOCAB, info["main_freq"], "main")
+    assert codec._encode_given(main, ctx, info["main_freq"]) == info["stream"]
+    with pytest.raises(codec.CodecError):  # a symbol that the frequencies do not hold
+        codec._encode_given(main, ctx, np.zeros_like(info["main_freq"]))
