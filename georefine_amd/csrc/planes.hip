@@ -237,6 +237,7 @@ __device__ __forceinline__ void meet_after_loads() {
 }
 
 constexpr uint32_t kUnits = 256;  // the chip's compute units
+constexpr uint32_t kLdsBytes = 160 * 1024;  // of one of them
 
 // LDS of a wave that has its own x.
 template <int HR>
@@ -703,7 +704,9 @@ int product(const char *who, uint32_t n, const grf_planes *const *planes, const 
     return grf::set_error(GRF_BAD_ARGUMENT, std::string(who) + ": workspace too small (grf_planes_workspace_bytes)");
   for (uint32_t done = 0; done < m_rows; done += kMaxTileRows) {
     const uint32_t m = std::min(kMaxTileRows, m_rows - done), m_pad = 16 * grf::gemm_tiles(m);
-    const bool batch = m > kOwnRows || (m > kOwnAlways && visits >= kOwnVisits) || (m > 16 && waves * Product<4>::kWaveBytes > 160 * 1024);
+    const bool batch = m > kOwnRows || (m > kOwnAlways && visits >= kOwnVisits) || (m > 16 && waves * Product<4>::kWaveBytes > kLdsBytes);
+    // (fifteen or sixteen waves with two eights of rows do not fit in a unit's LDS; eight have the splits two each)
+    const uint32_t own_waves = waves * Product<2>::kWaveBytes > kLdsBytes && (m > 8 || packed) ? 8 : waves;
     const PlanesX rows{reinterpret_cast<const uint8_t *>(x) + (size_t)done * ldx * 2, packed ? 16 : ldx * 2, packed ? m_pad * 16 : 16, m, cols, packed};
     uint32_t grid = 0, batch_waves = 4, busiest = ~0u;
     for (uint32_t w : {4u, 3u}) {  // the visits of a compute unit that has most of them
@@ -716,15 +719,15 @@ int product(const char *who, uint32_t n, const grf_planes *const *planes, const 
     for (uint32_t i = 0; i < n; ++i) {
       PlanesMember &one = g.m[i];
       const uint32_t blocks = (one.p.rows + 15) / 16;
-      one.blocks_each = batch ? batch_waves * kBatchEach : std::max(1u, waves / one.p.splits);
+      one.blocks_each = batch ? batch_waves * kBatchEach : std::max(1u, own_waves / one.p.splits);
       one.y = y[i] + (size_t)done * ldy[i];
       one.first = grid;
       grid += (blocks + one.blocks_each - 1) / one.blocks_each * (batch ? one.p.splits : 1);
       split |= batch && one.p.splits > 1;
     }
-    if (int rc = !batch ? (m <= 8 && !packed ? launch_product<1>(g, rows, waves, grid, s)
-                           : m <= 16         ? launch_product<2>(g, rows, waves, grid, s)
-                                             : launch_product<4>(g, rows, waves, grid, s))
+    if (int rc = !batch ? (m <= 8 && !packed ? launch_product<1>(g, rows, own_waves, grid, s)
+                           : m <= 16         ? launch_product<2>(g, rows, own_waves, grid, s)
+                                             : launch_product<4>(g, rows, own_waves, grid, s))
                  : m <= 16 ? launch_batch<1>(g, rows, batch_waves, grid, s)
                  : m <= 32 ? launch_batch<2>(g, rows, batch_waves, grid, s)
                  : m <= 64 ? launch_batch<4>(g, rows, batch_waves, grid, s)

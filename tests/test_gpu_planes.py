@@ -136,6 +136,28 @@ def test_members_of_more_splits_than_the_largest_one_have_two_a_wave():
             assert all(torch.equal(together[i], alone[i]) for i in order), (m, order)
 
 
+@pytest.mark.parametrize("splits", [11, 14, 15, 16])
+def test_rows_past_eight_of_many_splits_fit_in_a_units_memory(splits):
+    import torch
+    from georefine_amd import _native
+    from georefine_amd.bitexact_context_gpu import PackedActivations
+    lib, rng, rows, cols = _native.hip(), np.random.default_rng(splits), 50, splits * 256 - 80
+    p = _planes(weight_like(rng, rows, cols))
+    p.struct.splits = splits
+    x = torch.from_numpy(rng.standard_normal((33, cols), dtype=np.float32)).cuda().bfloat16()
+    space = torch.empty(splits * 64 * rows, device="cuda", dtype=torch.float32)
+
+    def product(rows_of_x, m, packed=0):
+        y = torch.empty(m, rows, device="cuda", dtype=torch.bfloat16)
+        _launch(lib.grf_planes_linear, p.address, rows_of_x.data_ptr(), cols, m, packed, y.data_ptr(), None, space.data_ptr(), space.numel() * 4)
+        return y
+
+    want = product(x, 33)
+    for m in (1, 8, 9, 16, 17, 32):
+        assert torch.equal(product(x, m), want[:m]), m
+        assert torch.equal(product(PackedActivations(x[:m]).buffer, m, packed=1), want[:m]), m
+
+
 def test_infinities_and_nan_go_where_the_dense_product_puts_them():
     import torch
     from georefine_amd import _native
