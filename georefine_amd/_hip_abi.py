@@ -74,7 +74,7 @@ DEVICE_SYMBOLS = ("grf_bctx_decode", "grf_ppcx_decode", "grf_mix_predict", "grf_
                   "grf_bctx_fused_decode", "grf_bctx_fused_gather", "grf_bctx_gather_rows", "grf_bctx_gather_rows_done", "grf_wait_word", "grf_take_word", "grf_bctx_fused_validate_host", "grf_bctx_fused_lds_bytes", "grf_bctx_gemm", "grf_bctx_gemm_lds_bytes",
                   "grf_gemm_workspace_bytes", "grf_gemm_workspace_bytes_split", "grf_bctx_gemm_noalloc", "grf_gemm_noalloc_limit_bytes", "grf_pack_activations", "grf_bctx_gemv_group", "grf_bctx_gemm_group",
                   "grf_ppcx_bins", "grf_ppcx_bins_ordered", "grf_ppcx_fused_decode", "grf_ppcx_gemv", "grf_ppcx_gemm", "grf_ppcx_gemv_group", "grf_ppcx_gemm_group", "grf_dense_gemm_plan", "grf_dense_gemm_workspace_bytes", "grf_dense_gemm", "grf_pair_residuals", "grf_planes_bytes", "grf_planes_visits", "grf_planes_count", "grf_planes_fill",
-                  "grf_planes_workspace_bytes", "grf_planes_linear", "grf_planes_group", "grf_planes_decode", "grf_planes_gather", "grf_last_error",
+                  "grf_planes_workspace_bytes", "grf_planes_linear", "grf_planes_group", "grf_planes_prompt_plan", "grf_planes_prompt_workspace_bytes", "grf_planes_prompt", "grf_planes_decode", "grf_planes_gather", "grf_last_error",
                   "grf_abi_version", "grf_timestamp", "grf_wall_clock_khz")
 
 
@@ -162,6 +162,12 @@ def declare(L):
     L.grf_planes_linear.restype = i
     L.grf_planes_group.argtypes = [u32, vp, vp, u32, u32, u32, vp, vp, vp, vp, size, vp]
     L.grf_planes_group.restype = i
+    L.grf_planes_prompt_plan.argtypes = [u32, u32, u32]
+    L.grf_planes_prompt_plan.restype = ctypes.c_int64
+    L.grf_planes_prompt_workspace_bytes.argtypes = [u32, u32, u32]
+    L.grf_planes_prompt_workspace_bytes.restype = size
+    L.grf_planes_prompt.argtypes = [vp, vp, u32, u32, u32, vp, u32, vp, vp, size, vp]
+    L.grf_planes_prompt.restype = i
     L.grf_planes_decode.argtypes = [vp, vp, vp]
     L.grf_planes_decode.restype = i
     L.grf_planes_gather.argtypes = [vp, vp, u32, vp, vp, vp, vp, vp]

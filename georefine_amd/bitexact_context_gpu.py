@@ -263,6 +263,39 @@ def _observed():
             or torch.autograd.forward_ad._current_level >= 0)
 
 
+def _only_values(x, bias, rows, cols, index):
+    """Whether a product of many rows is asked for nothing but its values, in a form that torch would take."""
+    return (_plain(x, index) and x.dim() and x.shape[-1] == cols
+            and (bias is None or _plain(bias, index) and bias.shape == (rows,) and bias.is_contiguous()) and not _observed())
+
+
+def _prompt_rows(x, cols, index):
+    import torch
+    x2, ldx = rows_for(x, cols, index, x.device)
+    if not cols <= ldx <= 1 << 21:  # (rows that overlap, or lie too far apart)
+        return x2.clone(memory_format=torch.contiguous_format), cols
+    return x2, ldx
+
+
+def planes_prompt(tensor, p, x, bias):
+    """The product of many rows with the planes ``p`` as they are, or None where the decoded matrix is the faster
+    way (``grf_planes_prompt_plan``) or more than the values is asked for, as in ``dense_linear``."""
+    rows, cols = tensor.shape
+    lib, index, m = tensor._lib, tensor._index, x.numel() // cols
+    plan = lib.grf_planes_prompt_plan(rows, cols, m) if m < 1 << 30 else -1
+    if plan < 0 or not _only_values(x, bias, rows, cols, index):
+        return None
+    x2, ldx = _prompt_rows(x, cols, index)
+    y = x2.new_empty((*x.shape[:-1], rows))
+    size = lib.grf_planes_prompt_workspace_bytes(rows, m, plan)
+    space = x2.new_empty(size // 2) if size else None
+    status = launch_on(index, lib.grf_planes_prompt, p.address, x2.data_ptr(), ldx, m, plan, y.data_ptr(), rows,
+                       bias.data_ptr() if bias is not None else None, space.data_ptr() if size else None, size)
+    if status:
+        tensor._raise_launch(status)
+    return y
+
+
 def dense_linear(lib, x, weight, bias, index):
     """``F.linear`` of activations with a decoded matrix on GPU ``index``: the library's product, or the one of
     ``grf_dense_gemm`` where that is the faster (its plan says so by the sizes) and nothing but the values
@@ -271,12 +304,9 @@ def dense_linear(lib, x, weight, bias, index):
     rows, cols = weight.shape
     m = x.numel() // cols if cols else 0
     size = lib.grf_dense_gemm_plan(rows, cols, m) if m < 1 << 30 else -1  # (first: the calls that it sends on pay nothing else)
-    if (size < 0 or not _plain(x, index) or not x.dim() or x.shape[-1] != cols or not weight.is_contiguous() or weight.data_ptr() & 15
-            or bias is not None and not (_plain(bias, index) and bias.shape == (rows,) and bias.is_contiguous()) or _observed()):
+    if size < 0 or not _only_values(x, bias, rows, cols, index) or not weight.is_contiguous() or weight.data_ptr() & 15:
         return torch.nn.functional.linear(x, weight, bias)
-    x2, ldx = rows_for(x, cols, index, x.device)
-    if not cols <= ldx <= 1 << 21:  # (rows that overlap, or lie too far apart)
-        x2, ldx = x2.clone(memory_format=torch.contiguous_format), cols
+    x2, ldx = _prompt_rows(x, cols, index)
     y = x2.new_empty((*x.shape[:-1], rows))
     space = x2.new_empty(size // 2) if size else None
     status = launch_on(index, lib.grf_dense_gemm, weight.data_ptr(), rows, cols, x2.data_ptr(), ldx, m, y.data_ptr(), rows,
@@ -964,7 +994,8 @@ class HipContextTensor:
         The row count picks the kernel family (``route_rows``): by default the fastest one --
         the fused decode-GEMV for one row (and two rows of a short-row matrix), the fused
         decode-GEMM to 128 rows (one launch), above that a fused decode to a dense transient
-        and a matmul (``dense_linear``; a second GEMM launch would decode the matrix again).
+        and a matmul (``dense_linear``; a second GEMM launch would decode the matrix again), or of planes
+        the product of many rows where that is the faster (``planes_prompt``).
         ``batch_invariant=True`` -- or the tensor's ``m_invariant`` policy, which is the default
         when the argument is left out -- sends every row count through the GEMM, so that a
         row's output never depends on the batch it arrives in: ``linear(x[:1])`` is
@@ -984,7 +1015,11 @@ class HipContextTensor:
         route = "dense" if held or self.fused is None else route_rows(m, self.shape[1], batch_invariant)
         if route == "dense":
             import torch
-            x, weight = x.to(self.device), self.decode(check=check)
+            x = x.to(self.device)
+            y = planes_prompt(self, p, x, bias) if held else None
+            if y is not None:
+                return y
+            weight = self.decode(check=check)
             if not held and self.fused is None:  # any number of rows, and another decode (or none) than the product's plan counts on
                 return torch.nn.functional.linear(x, weight, bias)
             return dense_linear(self._lib, x, weight, bias, self._index)

@@ -513,11 +513,12 @@ class HipPredictiveTensor:
     def linear(self, reference_bf16_device, x, bias=None, *, check=False, batch_invariant=None):
         """y = x W^T + bias with W decoded on the fly against the reference: the fused GEMV for
         one activation row, the fused GEMM (matrix cores, one launch) for up to 128; above that
-        the fused decode to a dense transient plus a matmul (``dense_linear``) is faster, unless
+        the fused decode to a dense transient plus a matmul (``dense_linear``), or of planes the product of
+        many rows (``planes_prompt``), is faster, unless
         ``batch_invariant`` asks for the fused GEMM throughout, whose rows do not depend on
         the batch.  Frames the tile walker cannot take are decoded and multiplied densely."""
         import torch
-        from .bitexact_context_gpu import PackedActivations, dense_linear
+        from .bitexact_context_gpu import PackedActivations, dense_linear, planes_prompt
         if isinstance(x, PackedActivations):  # packed for the matrix-core kernel, which is what it gets
             return self._product(reference_bf16_device, x, bias, check, True)
         if batch_invariant is None:  # the tensor's policy
@@ -526,6 +527,10 @@ class HipPredictiveTensor:
         if not self.fusable or x.dtype != torch.bfloat16:
             return torch.nn.functional.linear(x, self.decode(reference_bf16_device, check=check), bias)
         if m > self.DENSE_ABOVE and not batch_invariant:
+            p = self._planes
+            y = planes_prompt(self, p, x, bias) if p is not None else None
+            if y is not None:
+                return y
             return dense_linear(self._lib, x, self.decode(reference_bf16_device, check=check), bias, self._index)
         return self._product(reference_bf16_device, x, bias, check, batch_invariant or m > self.GEMV_UP_TO)
 

@@ -581,6 +581,10 @@ int grf_dense_gemm(const uint16_t *w, uint32_t rows, uint32_t cols, const uint16
  *                   fp32 sums in an order that the matrix's sizes and splits fix, so that a row has the same bits in every
  *                   batch and group.  workspace: grf_planes_workspace_bytes, 16-byte aligned.  x: 16-byte aligned, ldx a multiple of 8; or, with `packed`, up to 128 rows as
  *                   grf_pack_activations leaves them
+ * grf_planes_prompt the product of many rows of x (any number from one on) without the dense matrix.  plan: rows of x a workgroup takes (128 or 256), and
+ *                   the parts of K (whole visits, up to 63 each) from bit 16 on, as grf_planes_prompt_plan gives it, or -1
+ *                   where grf_planes_decode and grf_dense_gemm (or a library's product) are as fast.  A row's
+ *                   bits depend on the plan.  y is 8-byte aligned, ldx up to 2^21
  * grf_planes_decode the words, dense
  * grf_planes_gather rows by index as grf_bctx_gather_rows takes and reports them; with `done` as
  *                   grf_bctx_gather_rows_done.
@@ -606,6 +610,10 @@ int grf_planes_linear(const grf_planes *planes, const uint16_t *x, uint32_t ldx,
 int grf_planes_group(uint32_t n, const grf_planes *const *planes, const uint16_t *x, uint32_t ldx, uint32_t m_rows, uint32_t packed,
                      uint16_t *const *y, const uint32_t *ldy, const uint16_t *const *bias, void *workspace, size_t workspace_bytes,
                      void *hip_stream);
+int64_t grf_planes_prompt_plan(uint32_t rows, uint32_t cols, uint32_t m_rows);
+size_t grf_planes_prompt_workspace_bytes(uint32_t rows, uint32_t m_rows, uint32_t plan);
+int grf_planes_prompt(const grf_planes *planes, const uint16_t *x, uint32_t ldx, uint32_t m_rows, uint32_t plan, uint16_t *y,
+                      uint32_t ldy, const uint16_t *bias, void *workspace, size_t workspace_bytes, void *hip_stream);
 int grf_planes_decode(const grf_planes *planes, uint16_t *out, void *hip_stream);
 int grf_planes_gather(const grf_planes *planes, const int64_t *ids, uint32_t count, uint16_t *out, int32_t *index_error, void *counters,
                       int32_t *done, void *hip_stream);

@@ -62,3 +62,31 @@ def test_listed_share_counts_what_is_outside_eleven_exponents():
     freq[0, 4 * 100] += 65536 - 44 * 1489
     freq[1, 4 * 50] = freq[1, 4 * 80] = 32768
     assert _planes.listed_share(np.array([0, 0, 0, 1]), np.zeros(7, dtype=np.uint8), freq, 2, 1) == pytest.approx(0.125)
+
+
+def test_plans_of_many_rows_are_what_the_launch_takes():
+    lib = _native.hip()
+    taken = 0
+    for rows, cols, m in [(1, 16, 129), (17, 240, 2048), (300, 1040, 129), (5120, 17408, 200), (5120, 17408, 1000), (17408, 5120, 300), (64, 131072, 150),
+                          (1024, 8192, 160), (65536, 512, 4000), (1 << 20, 512, 1024), (1 << 20, 512, 1025), (512, 1028, 200), (512, 1024, 128)]:
+        plan = lib.grf_planes_prompt_plan(rows, cols, m)
+        if cols % 8 or m <= 128 or rows * m > 1 << 30:
+            assert plan == -1
+        if plan < 0:
+            continue
+        taken += 1
+        tile, parts = plan & 0xFFFF, plan >> 16
+        each = -(-_planes.visits(cols) // parts)
+        assert tile in (128, 256) and each <= 63 and (parts - 1) * each < _planes.visits(cols)
+        assert lib.grf_planes_prompt_workspace_bytes(rows, m, plan) == (parts * m * ((rows + 3) & ~3) * 4 if parts > 1 else 0)
+    assert taken >= 3
+
+
+@pytest.mark.parametrize("change", [dict(plan=0), dict(plan=1 << 16 | 64), dict(plan=5 << 16 | 128), dict(plan=2 << 16 | 128), dict(ldx=1016),
+                                    dict(ldx=1 << 22), dict(ldy=63), dict(y=4098), dict(x=4100), dict(m=0)])
+def test_products_of_many_rows_that_a_launch_would_not_take_are_refused(change):
+    lib = _native.hip()
+    p = _hip_abi.GrfPlanes(planes=4096, bases=4096, listed_at=4096, listed=4096, rows=64, cols=1024, splits=2)
+    a = {**dict(x=4096, ldx=1024, m=200, plan=1 << 16 | 128, y=4096, ldy=64), **change}
+    assert lib.grf_planes_prompt(ctypes.addressof(p), a["x"], a["ldx"], a["m"], a["plan"], a["y"], a["ldy"], None, None, 0, None) != 0
+    assert b"grf_planes_prompt" in lib.grf_last_error()
