@@ -18,7 +18,7 @@ from . import _hip_abi, _native
 VISIT, UNIT, VISIT_BYTES, UNIT_BYTES = 256, 64, 5888, 1536  # csrc/word_planes.h
 EXPONENTS = 11
 MAX_COLS = 1 << 17
-OWN_ROWS = 8  # activation rows up to which no launch needs a workspace
+OWN_ROWS = 8  # activation rows up to which a launch needs no workspace (a matrix alone is given one where it pays)
 # Weights from which a matrix is laid out.  The kernels are the shorter below it too (one row of 512 x 640 4.4 us, walked 8.4;
 # 32 rows 8.6 and 8.2), but a call is as long as its host path there (502 x 640 at three rows 10.1 and 10.5), and a
 # tensor whose arrays are asked for changes the bits of its products, which the small ones that are looked at do not.

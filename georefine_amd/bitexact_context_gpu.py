@@ -486,7 +486,7 @@ def planes_product(tensor, p, x, bias):
         y = x2.new_empty((*x.shape[:-1], rows))
     if m:
         bias = bias_for(bias, tensor._index, tensor.device)
-        size = p.workspace(m) if m > _planes.OWN_ROWS else 0
+        size = p.workspace(m)
         space = tensor.error.new_empty(size // 4) if size else None
         status = launch_on(tensor._index, tensor._lib.grf_planes_linear, p.address, x2.data_ptr(), ldx, m, packed, y.data_ptr(),
                            bias.data_ptr() if bias is not None else None, space.data_ptr() if size else None, size)

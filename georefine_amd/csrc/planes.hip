@@ -42,6 +42,7 @@ struct PlanesMember {
   const uint16_t *bias;
   float *partials;                   // [splits][activation rows][rows]
   uint32_t ldy, first, blocks_each;  // first workgroup; row blocks a workgroup
+  uint32_t parts;                    // workgroups that share a row block's splits, few rows of x
 };
 
 struct PlanesGroup {
@@ -146,13 +147,16 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) void 
   const PlanesMember &m = g.m[i];
   const uint32_t splits = m.p.splits, waves = blockDim.x / 64;
   const uint32_t at_once = splits > waves ? (splits + 1) / 2 : splits, sub = wave / at_once;  // (a wave has one split or two)
-  const uint32_t blocks = (m.p.rows + 15) / 16, block = (blockIdx.x - m.first) * m.blocks_each + sub;
+  const uint32_t blocks = (m.p.rows + 15) / 16, in_parts = m.parts > 1;
+  const uint32_t block = in_parts ? (blockIdx.x - m.first) % blocks : (blockIdx.x - m.first) * m.blocks_each + sub;
   const grf::PlanesShape shape(x.cols);
   const uint32_t each = (shape.visits() + splits - 1) / splits;
-  const bool works = sub < m.blocks_each && block < blocks;
+  const bool works = in_parts || (sub < m.blocks_each && block < blocks);
+  const uint32_t split0 = in_parts ? (blockIdx.x - m.first) / blocks * waves + wave : wave % at_once;
+  const uint32_t next_split = in_parts ? splits : at_once;
   float4v acc[MT] = {};
   float4v *const before = reinterpret_cast<float4v *>(lds + wave * kWave + Product<HR>::kFirst) + lane;
-  for (uint32_t split = wave % at_once; works && split < splits; split += at_once) {
+  for (uint32_t split = split0; works && split < splits; split += next_split) {
 #pragma unroll
     for (int j = 0; j < MT; ++j) before[j * 64] = acc[j], acc[j] = (float4v){};
     const uint32_t v0 = min(split * each, shape.visits()), v1 = min(v0 + each, shape.visits()), full = min(v1, shape.full);
@@ -268,7 +272,18 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) void 
       }
     }
   }
-  const uint32_t split0 = wave % at_once;
+  if (in_parts) {  // (uniform) the sums are added by a launch of their own
+    const uint32_t row = block * 16 + lane % 16;
+    if (split0 >= splits || row >= m.p.rows) return;
+#pragma unroll
+    for (int j = 0; j < MT; ++j)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const uint32_t xrow = j * 16 + lane / 16 * 4 + k;
+        if (xrow < x.m_rows) m.partials[((size_t)split0 * x.m_rows + xrow) * m.p.rows + row] = acc[j][k];
+      }
+    return;
+  }
   const bool two = works && split0 + at_once < splits;
   float4v first[MT];
 #pragma unroll
@@ -552,9 +567,27 @@ int check_planes(const char *who, const grf_planes *p) {
   return GRF_OK;
 }
 
-// fp32 sums of a launch of `m` rows whose members are cut in parts, in bytes.
-size_t partial_bytes(const grf_planes &p, uint32_t m) {
-  return m > kOwnAlways && p.splits > 1 ? ((size_t)p.splits * m * p.rows * 4 + 255) / 256 * 256 : 0;
+// fp32 sums of all splits for `m` rows, and those that a launch of `m` rows of n members has to have room for, in bytes.
+size_t sums_bytes(const grf_planes &p, uint32_t m) { return ((size_t)p.splits * m * p.rows * 4 + 255) / 256 * 256; }
+size_t partial_bytes(const grf_planes &p, uint32_t m) { return m > kOwnAlways && p.splits > 1 ? sums_bytes(p, m) : 0; }
+
+// Workgroups that share the splits of a row block where few rows of x meet a matrix alone.  Whole row blocks fall unevenly on the units:
+// of 320 blocks some have two and most one, and the last of 5120 x 17408 ends after 136 visits where 85 are a unit's share (256
+// blocks of these 23 us, 320 36).  Four workgroups of three splits a block leave the busiest 90 and cost a launch that adds the sums: us,
+// one row and six of 5120 x 17408 35.6 and 37.3, in parts 33.2 and 33.9; of 4200 x 17408 32.2 35.2, 31.9 32.4.  It is
+// left where less than 40 visits are saved (6144 x 17408, 28: 35.3 and 36.9; 5120 x 6144, 16: 15.8 and 16.1; 9000 x 9728, 18: 34.1 and 33.3).
+constexpr uint64_t kSaved = 40;
+
+uint32_t own_parts(const grf_planes &p) {
+  const uint64_t blocks = (p.rows + 15) / 16, visits = grf::PlanesShape(p.cols).visits(), each = (visits + p.splits - 1) / p.splits;
+  uint32_t best = 1;
+  uint64_t least = (blocks + kUnits - 1) / kUnits * each * p.splits;
+  least = least > kSaved ? least - kSaved + 1 : 0;  // to be below
+  for (uint32_t waves = p.splits - 1; waves >= 3; --waves) {
+    const uint64_t parts = (p.splits + waves - 1) / waves, busiest = (blocks * parts + kUnits - 1) / kUnits * waves * each;
+    if (busiest < least) least = busiest, best = (uint32_t)parts;
+  }
+  return best;
 }
 
 int product(const char *who, uint32_t n, const grf_planes *const *planes, const uint16_t *x, uint32_t ldx, uint32_t m_rows, bool packed,
@@ -587,7 +620,9 @@ int product(const char *who, uint32_t n, const grf_planes *const *planes, const 
     const uint32_t m = std::min(kMaxTileRows, m_rows - done), m_pad = 16 * grf::gemm_tiles(m);
     const bool batch = m > kOwnRows || (m > kOwnAlways && visits >= kOwnVisits) || (m > 16 && waves * Product<4>::kWaveBytes > kLdsBytes);
     // (fifteen or sixteen waves with two eights of rows do not fit in a unit's LDS; eight have the splits two each)
-    const uint32_t own_waves = waves * Product<2>::kWaveBytes > kLdsBytes && (m > 8 || packed) ? 8 : waves;
+    const uint32_t parts = batch || n > 1 || workspace_bytes < sums_bytes(*planes[0], m) ? 1 : own_parts(*planes[0]);
+    const uint32_t own_waves = parts > 1 ? (planes[0]->splits + parts - 1) / parts
+                               : waves * Product<2>::kWaveBytes > kLdsBytes && (m > 8 || packed) ? 8 : waves;
     const PlanesX rows{reinterpret_cast<const uint8_t *>(x) + (size_t)done * ldx * 2, packed ? 16 : ldx * 2, packed ? m_pad * 16 : 16, m, cols, packed};
     uint32_t grid = 0, batch_waves = 4, busiest = ~0u;
     for (uint32_t w : {4u, 3u}) {  // the visits of a compute unit that has most of them
@@ -603,8 +638,9 @@ int product(const char *who, uint32_t n, const grf_planes *const *planes, const 
       one.blocks_each = batch ? batch_waves * kBatchEach : std::max(1u, own_waves / one.p.splits);
       one.y = y[i] + (size_t)done * ldy[i];
       one.first = grid;
-      grid += (blocks + one.blocks_each - 1) / one.blocks_each * (batch ? one.p.splits : 1);
-      split |= batch && one.p.splits > 1;
+      one.parts = parts;
+      grid += parts > 1 ? blocks * parts : (blocks + one.blocks_each - 1) / one.blocks_each * (batch ? one.p.splits : 1);
+      split |= parts > 1 || (batch && one.p.splits > 1);
     }
     if (int rc = !batch ? (m <= 8 && !packed ? launch_product<1>(g, rows, own_waves, grid, s)
                            : m <= 16         ? launch_product<2>(g, rows, own_waves, grid, s)
@@ -902,7 +938,10 @@ int grf_planes_fill(const uint16_t *words, uint32_t rows, uint32_t cols, const u
 size_t grf_planes_workspace_bytes(uint32_t n, const grf_planes *const *planes, uint32_t m_rows) {
   size_t bytes = 0;
   for (uint32_t i = 0; planes && i < n; ++i)
-    if (planes[i]) bytes += partial_bytes(*planes[i], std::min(m_rows, kMaxTileRows));
+    if (planes[i]) {
+      const uint32_t m = std::min(m_rows, kMaxTileRows);
+      bytes += n == 1 && own_parts(*planes[i]) > 1 ? sums_bytes(*planes[i], m) : partial_bytes(*planes[i], m);
+    }
   return bytes;
 }
 

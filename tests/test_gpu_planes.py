@@ -114,6 +114,32 @@ def test_rows_of_x_that_large_matrices_share_have_the_bits_of_single_ones(rows, 
         assert torch.equal(product(PackedActivations(x[:m]).buffer, m, packed=1), want[:m]), m
 
 
+@pytest.mark.parametrize("rows,cols,splits", [(4097, 17408, 12), (4200, 16400, 13)])
+def test_row_blocks_that_workgroups_share_give_the_bits_of_whole_ones(rows, cols, splits):
+    import torch
+    from georefine_amd import _native
+    lib, g = _native.hip(), torch.Generator(device="cuda").manual_seed(rows)
+    words = (torch.randn(rows, cols, device="cuda", generator=g) * 0.02).bfloat16()
+    words.view(-1)[torch.randint(0, rows * cols, (100000,), device="cuda", generator=g)] = 0  # (listed)
+    x = torch.randn(8, cols, device="cuda", generator=g).bfloat16()
+    bias = torch.randn(rows, device="cuda", generator=g).bfloat16()
+    from georefine_amd._planes import Planes
+    p = Planes.of_words(words.view(torch.int16), _launch)
+    p.struct.splits = splits
+    size = p.workspace(8)
+    assert size >= splits * 8 * rows * 4
+    space = torch.full((size // 4 + 64,), 5.0, device="cuda", dtype=torch.float32)
+    exact = x.double() @ words.double().T + bias.double()
+    bound = exact.abs() * 2.0 ** -8 + (x.double().abs() @ words.double().abs().T + 8) * cols * 2.0 ** -24
+    for m in (1, 2, 7, 8):
+        whole, shared = (torch.full((m + 2, rows), 7.0, device="cuda", dtype=torch.bfloat16) for _ in range(2))
+        for y, s, n in ((whole, None, 0), (shared, space.data_ptr(), size)):  # without a workspace blocks are whole
+            _launch(lib.grf_planes_linear, p.address, x.data_ptr(), cols, m, 0, y[1:].data_ptr(), bias.data_ptr(), s, n)
+        assert torch.equal(whole, shared) and bool((shared[0] == 7).all() and (shared[-1] == 7).all())
+        assert bool(((shared[1:-1].double() - exact[:m]).abs() <= bound[:m]).all())
+    assert bool((space[size // 4:] == 5).all())
+
+
 def test_members_of_more_splits_than_the_largest_one_have_two_a_wave():
     import ctypes
     import torch
