@@ -87,12 +87,15 @@ GEMV_UP_TO = 2  # rows linear() gives to the vector-ALU kernel; read from HipCon
 
 
 def algorithmic_bytes(t, m, gemm=None):
-    """Bytes one fused GEMV / GEMM launch has to touch once: both streams, the fused index,
-    the per-class lookup tables, labels, activations and outputs.  ``gemm``: the launch runs
+    """Bytes one fused GEMV / GEMM launch has to touch once: the planes of a matrix held as such, or both streams, the
+    fused index, the per-class lookup tables and labels; activations and outputs.  ``gemm``: the launch runs
     the matrix-core kernel (default: from the row count, as linear() routes)."""
+    rows, cols = t.shape
+    if t._planes is not None:  # what the matrix is resident as: its planes and the listed words
+        held = t._planes.nbytes
+        return dict(total=held + m * (rows + cols) * 2, payload=held, index=0, tables=0)
     b = t.buffers
     n = lambda k: b[k].numel() * b[k].element_size()
-    rows, cols = t.shape
     # (the resident residual array starts every row class on a multiple of 16 rows: the rows it
     # holds beyond the matrix's are never read and are not counted)
     payload = t._main_bytes + min(n("residual_pairs" if "residual_pairs" in b else "residual_stream"), rows * cols * 3 // 4)
@@ -295,7 +298,7 @@ def run_attention(args, as_dict=False):
         # q, k and v share a launch, so they are indexed at one segment length
         base[name] = HipContextTensor(codec.encode(synth_weights(10 + i, rows, cols)), stride=1024, device="cuda:0",
                                       fused_segment=64)
-        if base[name].fused is None:
+        if base[name]._planes is None and base[name].fused is None:
             sys.exit(f"bench.py: {name} is not eligible for the fused kernels: {base[name].fused_reason}")
     resident = sum(t.resident_bytes for t in base.values())
     copies = max(1, -(-2 * LAST_LEVEL_CACHE_BYTES // resident))
@@ -325,7 +328,8 @@ def run_attention(args, as_dict=False):
         alg = alg_of(m, invariant or m > GEMV_UP_TO)
         dom = max(alg, key=lambda k: alg[k])
         gemm = invariant or m > GEMV_UP_TO
-        kernel = (f"grf::fused_gemm_group_kernel / fused_gemm_wide_group_kernel<{WALK}, MT, 1>" if gemm
+        planes = all(t._planes is not None for t in base.values())
+        kernel = (kernel_name(False, m, True, True) if planes else f"grf::fused_gemm_group_kernel / fused_gemm_wide_group_kernel<{WALK}, MT, 1>" if gemm
                   else kernel_name(False, m, True))
         total = sum(alg.values())
         return {"ms_per_pass": round(ms_step, 4), "GBps": round(total / (ms_step * 1e-3) / 1e9, 2), "launch": launch,
@@ -567,7 +571,7 @@ def run_stack(args, as_dict=False, prep=None):
     base, frame_len = {}, {}
     for key, (frame_bytes, prepared) in done.items():
         t = HipContextTensor(b"", stride=1024, device="cuda:0", prepared=prepared)
-        if t.fused is None:
+        if t._planes is None and t.fused is None:
             sys.exit(f"bench.py: {key} is not eligible for the fused kernels: {t.fused_reason}")
         base[key], frame_len[key] = t, frame_bytes
     done.clear()
@@ -587,7 +591,8 @@ def run_stack(args, as_dict=False, prep=None):
         vocab = {"embedding": head.clone(), "head": head}
     everything = [t for _, layer in layers for t in layer.values()] + (list(vocab.values()) if vocab else [])
     for t in everything:
-        t._gemm_tiling() if gemm else t._tiling(m)
+        if t._planes is None:
+            t._gemm_tiling() if gemm else t._tiling(m)
     torch.cuda.synchronize()
     frame_bytes = 0
     # frame bytes of the whole stack: every layer's frames (copies are the same frames again)
@@ -644,7 +649,7 @@ def run_stack(args, as_dict=False, prep=None):
     value = step_bytes / (ms_per_step * 1e-3) / 1e9
     share = {label: per_ms[label] * count[label] for label in per_ms}  # ms of a pass spent in each kind of launch
     dom = max((l_ for l_ in alg if l_ != "embedding"), key=lambda l_: alg[l_])  # the kind that moves most bytes
-    kernel = kernel_name(False, max(m, GEMV_UP_TO + 1) if gemm else m, "+" in dom)
+    kernel = kernel_name(False, max(m, GEMV_UP_TO + 1) if gemm else m, "+" in dom, all(t._planes is not None for t in everything))
     shapes_text = "; ".join(f"{k}: " + ", ".join(f"{n_} {c}->{r}" for n_, (r, c) in spec[k].items())
                             for k in ("attn", "gdn") if spec[k])
     result = {
@@ -773,12 +778,14 @@ def main():
         tensors[name] = HipContextTensor(frame, stride=1024, device="cuda:0", fused_segment=args.segment or None,
                                          residual_block=residual_block)
         t2 = time.perf_counter()
-        if tensors[name].fused is None:
+        held = tensors[name]._planes is not None
+        if not held and tensors[name].fused is None:
             sys.exit(f"bench.py: {name} is not eligible for the fused kernel: {tensors[name].fused_reason}")
         log(f"{name}: {rows}x{cols} mode {tensors[name].mode} frame {len(frame)} B "
             f"({8 * len(frame) / w.size:.3f} bit/weight) encode {t1 - t0:.1f}s index+upload {t2 - t1:.1f}s "
-            f"resident mode {tensors[name].resident_mode} plan {tensors[name].fused_plan} "
-            f"tiling {(tensors[name]._tiling(args.batch) if args.batch <= GEMV_UP_TO else tensors[name]._gemm_tiling())[3]}")
+            + (f"held as planes, {tensors[name]._planes.splits} splits" if held else
+               f"resident mode {tensors[name].resident_mode} plan {tensors[name].fused_plan} "
+               f"tiling {(tensors[name]._tiling(args.batch) if args.batch <= GEMV_UP_TO else tensors[name]._gemm_tiling())[3]}"))
         frames[name] = frame
         words_of[name] = w
     log(f"setup {time.perf_counter() - t_setup:.1f}s")
@@ -820,7 +827,7 @@ def main():
         per_layer = [units_of(*layer) for layer in layers]
         units = per_layer[0]
         if pair is not None and not decode_only:
-            log(f"batch {m} gate+up: one launch, tiling {pair._tiling('waves' if m <= GEMV_UP_TO else 'gemm')[0][3]}")
+            log(f"batch {m} gate+up: one launch")
         ms_per_step, per_kernel_ms, launch, timing, clocks = time_launches(
             torch, per_layer, args.steps, args.warmup, args.graph,
             lambda: sorted({n_ for ts, pr in layers for n_ in names if ts[n_].error.item()}
@@ -840,7 +847,8 @@ def main():
         value = step_bytes / (ms_per_step * 1e-3) / 1e9
         eff_bf16 = dense_bytes / (ms_per_step * 1e-3) / 1e9
         dom = max(per_kernel_ms, key=lambda n_: per_kernel_ms[n_])
-        kernel = kernel_name(decode_only, m, "+" in dom)
+        planes = all(t._planes is not None for t in tensors.values())
+        kernel = kernel_name(decode_only, m, "+" in dom, planes)
         traffic, traffic_source = recorded_traffic(decode_only, m, kernel)
         achieved = alg[dom]["total"] / (per_kernel_ms[dom] * 1e-3) / 1e9
         fields = {
@@ -848,11 +856,11 @@ def main():
             "config": {"workload": ("fused decode to dense BF16 (decode())" if decode_only else
                                     "fused decode-" + ("GEMV" if m <= GEMV_UP_TO else "GEMM") + ", batch %d" % m)
                                    + ", Qwen-27B-like MLP: gate/up 5120->17408, down 17408->5120, BCTX (16,4) frames"
-                                   + (", residuals resident in packed 6-bit form"
+                                   + (", resident as planes" if planes else ", residuals resident in packed 6-bit form"
                                       if any(tensors[n_].resident_mode != tensors[n_].mode for n_ in names) else ""),
                        "batch": m, "matrices": names, "launches": [u[0] for u in units],
-                       "segment": tensors[names[0]].fused_plan["seg_len"], "launch": launch, "per_kernel_timing": timing,
-                       "layer_copies": n_layers, "residual_block_rows": tensors[names[0]]._raw6_block},
+                       "segment": None if planes else tensors[names[0]].fused_plan["seg_len"], "launch": launch, "per_kernel_timing": timing,
+                       "layer_copies": n_layers, "residual_block_rows": None if planes else tensors[names[0]]._raw6_block},
             "effective_bf16_GBps": round(eff_bf16, 2),
             "tok_s_equiv": round(eff_bf16 * 1e9 / MODEL_BF16_BYTES * m, 3) if m else None,
             **clocks,
@@ -937,8 +945,11 @@ def main():
 WALK = "grf::SegmentWalkT<false, true>"  # (the walker of residuals in pair form, which is how tensors keep them)
 
 
-def kernel_name(decode_only, m, grouped):
+def kernel_name(decode_only, m, grouped, planes=False):
     """The kernel a launch of the workload runs (as rocprofv3 names it)."""
+    if planes:
+        return ("planes_decode_kernel" if decode_only else "planes_product_kernel" if m <= 8 else
+                "planes_product_kernel or planes_batch_kernel" if m <= 32 else "planes_batch_kernel" if m <= 128 else "planes_prompt_kernel")
     # (template argument 1 after the walker and the rows: the scan for frames without whole-range contexts, which these are)
     if decode_only:  # (two groups of columns held back, stores to the second-level cache: matrices of this size)
         return f"grf::fused_wave_store_kernel<{WALK}, 1, 2, 0>"
