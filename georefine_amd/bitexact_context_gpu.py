@@ -636,17 +636,6 @@ class HipContextTensor:
         self.resident_bytes = planes.nbytes + self.error.numel() * self.error.element_size()
         self._planes = planes
 
-    def take_planes(self):
-        """Puts a tensor that is walked into planes, for a launch with others that are held so; one whose arrays were
-        asked for stays as it is, and so does one that could not be held so."""
-        import torch
-        with _form_lock:
-            if self._planes is None and self._sections is not None and self.fused is not None:
-                self._hold_planes(self.decode(check=False).view(torch.int16))
-                # (kept: calls of other threads and streams and captured launches may be reading them, and small tensors do this)
-                self._used = [self.__dict__.pop(name, None) for name in HipContextTensor._STREAM_FORM]
-        return self._planes is not None
-
     def _leave_planes(self):
         """The frame's arrays in the planes' place: the words, coded once more with the frame's own labels and frequencies,
         which gives the same main stream, and packed residuals, the form that the walk takes.  The planes stay allocated:
@@ -1166,12 +1155,15 @@ class HipLinearGroup:
         self.m_invariant = any(t.m_invariant for t in self.tensors) if m_invariant is None else bool(m_invariant)
         self.error = torch.zeros((), device=self.device, dtype=torch.int32)
         self._tilings, self._pointer_arrays, self._workspace = {}, {}, {}
-        self._walked = None  # (members whose frames are walked, their group) where some are held as planes
-        if any(t._planes is not None for t in self.tensors):  # (two kinds of members are two launches)
-            for t in self.tensors:
-                t.take_planes()
-        else:
+        # Members whose frames are walked, beside others that are held as planes, have a launch of their own: laid out for the planes' launch
+        # they would lose the bits of their own products, which the vector-ALU route gives every member.
+        self._walked = None  # (their places, their group)
+        rest = [i for i, t in enumerate(self.tensors) if t._planes is None]
+        if len(rest) == len(self.tensors):
             self._plan_tilings()
+        elif rest:
+            self._walked = rest, HipLinearGroup([self.tensors[i] for i in rest], m_invariant=self.m_invariant)
+            self._walked[1].error = self.error  # (what a caller polls)
 
     def _plan_tilings(self):
         for key in (1, 2, "gemm"):
@@ -1286,6 +1278,7 @@ class HipLinearGroup:
             walked = self._walked
             if walked is None or walked[0] != rest:
                 walked = self._walked = rest, HipLinearGroup([self.tensors[i] for i in rest], m_invariant=self.m_invariant)
+                walked[1].error = self.error
             for i, y in zip(rest, walked[1].linear(x, [biases[i] for i in rest] if biases is not None else None, check=check,
                                                    batch_invariant=batch_invariant)):
                 outs[i] = y

@@ -216,17 +216,17 @@ def test_a_tensor_answers_as_planes_and_leaves_them_when_its_arrays_are_asked_fo
         assert t.fusable and t._planes is not None and t.fused_reason == ""
         other, small = t.clone(residual_block=16), HipContextTensor(codec.encode(weight_like(rng, 48, 1040)))
         assert small._planes is None
-        ids = torch.tensor([3, 40])
-        rows_of_small = small.gather_rows(ids)
-        group = HipLinearGroup([t, small, other])
-        assert small._planes is not None and torch.equal(small.gather_rows(ids).view(torch.int16), rows_of_small.view(torch.int16))
+        held = small.resident_bytes
+        group, alone = HipLinearGroup([t, small, other]), HipLinearGroup([small])
+        assert small._planes is None and small.resident_bytes == held
         x = torch.from_numpy(bf16_words(rng.normal(0, 1, (140, 1040)))).view(torch.bfloat16).cuda()
         for m in (1, 2, 20, 128, 140):
             want = t.linear(x[:m], batch_invariant=True)
             assert torch.equal(t.linear(x[:m], batch_invariant=True, check=True), want)
             got = group.linear(x[:m], batch_invariant=True)
             assert torch.equal(got[0], want) and torch.equal(got[2], want)
-            assert torch.equal(got[1], small.linear(x[:m], batch_invariant=True))
+            assert torch.equal(got[1], alone.linear(x[:m], batch_invariant=True)[0])
+        assert torch.equal(group.linear(x[:1])[1], small.linear(x[:1]))  # (the vector-ALU route gives every member its own bits)
         ids = torch.tensor([[0, 699], [5, 5]])
         assert np.array_equal(t.gather_rows(ids).view(torch.int16).cpu().numpy().view(np.uint16), words[ids.numpy()])
         for bad in (-1, 700):
@@ -242,9 +242,8 @@ def test_a_tensor_answers_as_planes_and_leaves_them_when_its_arrays_are_asked_fo
             assert np.array_equal(t.buffers[name].cpu().numpy()[:streams[name].size], streams[name]), name
         assert t.mode == frame[5] and t.frame_bytes == len(frame) and other._planes is not None
         assert np.array_equal(t.decode().view(torch.int16).cpu().numpy().view(np.uint16), words)
-        assert not t.take_planes()
         mixed, walked = group.linear(x[:20]), HipLinearGroup([t]).linear(x[:20])  # (two launches from here on)
-        assert torch.equal(mixed[0], walked[0]) and torch.equal(mixed[1], small.linear(x[:20])) and torch.equal(mixed[2], other.linear(x[:20]))
+        assert torch.equal(mixed[0], walked[0]) and torch.equal(mixed[1], alone.linear(x[:20])[0]) and torch.equal(mixed[2], other.linear(x[:20]))
         assert np.array_equal(other.decode(general=True).view(torch.int16).cpu().numpy().view(np.uint16), words) and other._raw6_block == 16
 
 
@@ -278,5 +277,5 @@ def test_captured_launches_replay_on_new_rows():
     torch.cuda.empty_cache()
     x1.copy_(draw(1)), x40.copy_(draw(40))
     graph.replay()
-    want = t.take_planes() or group.tensors[1].linear(x1)  # (the clone's planes, the same words)
+    want = group.tensors[1].linear(x1)  # (the clone's planes, the same words)
     assert torch.equal(captured[0], want) and torch.equal(captured[1], captured[2])
