@@ -19,9 +19,9 @@ VISIT, UNIT, VISIT_BYTES, UNIT_BYTES = 256, 64, 5888, 1536  # csrc/word_planes.h
 EXPONENTS = 11
 MAX_COLS = 1 << 17
 OWN_ROWS = 8  # activation rows up to which a launch needs no workspace (a matrix alone is given one where it pays)
-# Weights from which a matrix is laid out.  The kernels are the shorter below it too (one row of 512 x 640 4.4 us, walked 8.4;
-# 32 rows 8.6 and 8.2), but a call is as long as its host path there (502 x 640 at three rows 10.1 and 10.5), and a
-# tensor whose arrays are asked for changes the bits of its products, which the small ones that are looked at do not.
+# Weights from which a matrix is laid out: where a call of its own stops gaining.  Below, it is as long as its host path either way (502 x
+# 640 at three rows 10.1 us, walked 10.5); the kernels are shorter there too for few rows (one row of 512 x 640 4.4 us, walked
+# 8.4; 32 rows 8.6 and 8.2), which only captured launches of small matrices would gain.
 FROM_WEIGHTS = 1 << 19
 # How much more memory than the frame's arrays the planes may take (frames of few exponents code far below 11.5 bits
 # and stay frames).

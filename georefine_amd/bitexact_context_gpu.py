@@ -9,8 +9,8 @@
 A frame is validated and decoded on the host when it is loaded, and its matrix is then held in one of two forms.  Most
 are laid out as planes (``_planes``: signs and mantissas as they are, exponents two to seven bits), which
 take the memory of the frame with its index and go at the memory's pace.  Small matrices and those whose frames are much
-smaller than planes stay as frames, and so does a tensor whose arrays are asked for: the main stream byte for
-byte, with a checkpoint index, and the residual section, with one exception: conditional residuals (mode 128) of a frame
+smaller than planes stay as frames; of one that is held as planes the frame's arrays are made beside them should they be asked for.  They are the
+main stream byte for byte, with a checkpoint index, and the residual section, with one exception: conditional residuals (mode 128) of a frame
 that the fused kernels take are kept as packed 6-bit fields, the form mode 0
 frames carry (``resident_mode`` 0, ``mode`` 128; ``resident_bytes`` then exceeds the
 frame's size by the difference).  Every kernel is hand-written HIP behind the C ABI.
@@ -386,7 +386,7 @@ class _Buffers(dict):
 
 
 _packed_lock = threading.Lock()
-_form_lock = threading.RLock()  # (what puts a tensor into its other form reads attributes of it)
+_walk_lock = threading.RLock()  # (what makes a tensor's walk attributes reads attributes of it)
 
 
 def _residual_form(groups, to_pairs):
@@ -607,26 +607,27 @@ class HipContextTensor:
             self.resident_mode = about["resident_mode"]
             self._hold_streams(prepared)
 
-    # A tensor is held in one of two forms.  As planes (``_planes``) it answers products, decode and lookups.  The
-    # other is the frame's own arrays, which the walk of its states takes: frames that the planes do not take
-    # are held so from the start, and a tensor whose arrays, plan or descriptors are asked for, for the C interface
-    # or to be looked at, is put into that form then, and stays in it.
+    # A tensor that is held as planes (``_planes``) runs its products, decode and lookups on them for good.  The frame's own
+    # arrays, which the walk of its states takes, their plan and descriptors are made when they are asked for, for the C interface, the
+    # one-lane decode or to be looked at, and are held beside the planes from then on: what a call runs, and with it a
+    # product's bits, never depends on what was looked at.  Frames that the planes do not take have nothing but those arrays.
     _planes = None
-    _used = None  # the form that the tensor was held in before
-    _STREAM_FORM = frozenset(("buffers", "fused", "fused_plan", "_plan", "_frame", "_tilings", "_workspace", "_gather", "_main_bytes",
-                              "_raw6_segment", "_raw6_block", "_gather_waves"))
+    _WALK = frozenset(("buffers", "fused", "fused_plan", "_plan", "_frame", "_tilings", "_workspace", "_gather", "_main_bytes",
+                       "_raw6_segment", "_raw6_block", "_gather_waves"))
 
     def __getattr__(self, name):  # (only of what the object does not have)
-        if name in HipContextTensor._STREAM_FORM and self.__dict__.get("_planes") is not None:
-            with _form_lock:
-                if self._planes is not None:
-                    self._leave_planes()
-            return getattr(self, name)
+        held = self.__dict__
+        if name in HipContextTensor._WALK and held.get("_planes") is not None:
+            with _walk_lock:
+                if "buffers" not in held:
+                    held.update(self._walk_attributes())  # (all at once: other threads look without the lock)
+            if name in held:
+                return held[name]
         raise AttributeError(f"{type(self).__name__!r} object has no attribute {name!r}")
 
     @property
     def fusable(self):
-        """Whether products take a kernel of their own (``fused``, asked without changing the form a tensor is held in)."""
+        """Whether products take a kernel of their own (asked without having the walk's arrays made, as ``fused`` has)."""
         return self._planes is not None or self.fused is not None
 
     def _hold_planes(self, words):
@@ -636,10 +637,10 @@ class HipContextTensor:
         self.resident_bytes = planes.nbytes + self.error.numel() * self.error.element_size()
         self._planes = planes
 
-    def _leave_planes(self):
-        """The frame's arrays in the planes' place: the words, coded once more with the frame's own labels and frequencies,
-        which gives the same main stream, and packed residuals, the form that the walk takes.  The planes stay allocated:
-        calls of other threads and streams and captured launches may be reading them."""
+    def _walk_attributes(self):
+        """The walk's attributes of a tensor that is held as planes: of the words, coded once more with the frame's own labels
+        and frequencies, which gives the same main stream, and packed residuals, the form that the walk takes."""
+        import copy
         import zlib
         import torch
         words = self.decode(check=False).view(torch.int16).cpu().numpy().view(np.uint16)
@@ -652,10 +653,13 @@ class HipContextTensor:
         frame = base._sealed(base._sections(0, self.nr, self.nc, *self.shape, meta, zlib.compress(frequencies, 1), main, base._pack6(lib, words),
                                             b"", bytes.fromhex(self.source_sha256)))
         segment = _fused.choose_segment(self.shape[1], self.asked_segment, rows=self.shape[0])
-        self._hold_streams(_stream_arrays(_read_frame(frame, self.stride, segment, True), True, self._block))
-        self._plan_gather()
-        self._used, self._planes, self._sections = self._planes, None, None
-        self.resident_bytes += self._used.nbytes
+        other = copy.copy(self)  # (so that this object has none of them until all are made)
+        other._planes = None
+        other._hold_streams(_stream_arrays(_read_frame(frame, self.stride, segment, True), True, self._block))
+        other._plan_gather()
+        made = {name: value for name, value in vars(other).items() if name in HipContextTensor._WALK}
+        beside = self._planes.nbytes  # (the error word is counted with the arrays)
+        return {**made, "fused_reason": other.fused_reason, "resident_bytes": other.resident_bytes + beside}
 
     def _hold_streams(self, prepared):
         """The device arrays of a frame that is walked where it lies."""
@@ -746,14 +750,17 @@ class HipContextTensor:
         import copy
         import torch
         other = copy.copy(self)
-        other._used = None
-        if other._planes is not None:
+        if other._planes is not None:  # (the copy makes its walk's arrays itself, should they be asked for)
             if residual_block is not None:
                 if residual_block not in (1, 2, 4, 8, 16):
                     raise ValueError("residual blocks have 1, 2, 4, 8 or 16 rows")
                 other._block = residual_block
+            for name in HipContextTensor._WALK:
+                vars(other).pop(name, None)
+            other.fused_reason = ""
             other._planes = other._planes.clone()
             other.error = torch.zeros_like(self.error)
+            other.resident_bytes = other._planes.nbytes + other.error.numel() * other.error.element_size()
             return other
         other.buffers = _Buffers((k, v.clone()) for k, v in self.buffers.items())
         if residual_block is not None and self._raw6_segment and residual_block != self._raw6_block:
@@ -1273,14 +1280,10 @@ class HipLinearGroup:
     def _linear_planes(self, planes, x, biases, check, batch_invariant):
         """Up to 128 rows of a group some of whose members are held as planes: one launch for those, and one for the rest."""
         outs = planes_group(self, planes, x, biases)
-        rest = [i for i, p in enumerate(planes) if p is None]
-        if rest:
-            walked = self._walked
-            if walked is None or walked[0] != rest:
-                walked = self._walked = rest, HipLinearGroup([self.tensors[i] for i in rest], m_invariant=self.m_invariant)
-                walked[1].error = self.error
-            for i, y in zip(rest, walked[1].linear(x, [biases[i] for i in rest] if biases is not None else None, check=check,
-                                                   batch_invariant=batch_invariant)):
+        if self._walked is not None:
+            rest, walked = self._walked
+            for i, y in zip(rest, walked.linear(x, [biases[i] for i in rest] if biases is not None else None, check=check,
+                                                batch_invariant=batch_invariant)):
                 outs[i] = y
         return outs
 

@@ -243,26 +243,27 @@ class HipPredictiveTensor:
             self.has_contexts = True
             del ref
 
-    # As the context codec's tensors are (``HipContextTensor``), one that keeps its contexts is held in one of two forms: the
-    # words laid out as planes, which need no contexts and take the memory of the frame with them, or the frame's own
-    # arrays, which a tensor is put into when they, a plan or a descriptor are asked for.
+    # As a ``HipContextTensor`` does, one that is held as planes (the words laid out, which needs no contexts and takes less than the
+    # frame with them) runs its calls on them for good; the frame's own arrays, plans and descriptors are made when they
+    # are asked for and held beside the planes from then on.
     _planes = None
-    _used = None  # the planes that the tensor was held as before
-    _STREAM_FORM = frozenset(("buffers", "fused", "fused_gemm", "fused_matrix", "fused_plan", "_plan", "_matrix_plan", "_walk_plan", "_frame",
-                              "_tilings", "_workspace", "_raw5_segment", "_raw5_block", "_rows_held"))
+    _WALK = frozenset(("buffers", "fused", "fused_gemm", "fused_matrix", "fused_plan", "_plan", "_matrix_plan", "_walk_plan", "_frame",
+                       "_tilings", "_workspace", "_raw5_segment", "_raw5_block", "_rows_held"))
 
     def __getattr__(self, name):  # (only of what the object does not have)
-        if name in HipPredictiveTensor._STREAM_FORM and self.__dict__.get("_planes") is not None:
-            from .bitexact_context_gpu import _form_lock
-            with _form_lock:
-                if self._planes is not None:
-                    self._leave_planes()
-            return getattr(self, name)
+        held = self.__dict__
+        if name in HipPredictiveTensor._WALK and held.get("_planes") is not None:
+            from .bitexact_context_gpu import _walk_lock
+            with _walk_lock:
+                if "buffers" not in held:
+                    held.update(self._walk_attributes())  # (all at once: other threads look without the lock)
+            if name in held:
+                return held[name]
         raise AttributeError(f"{type(self).__name__!r} object has no attribute {name!r}")
 
     @property
     def fusable(self):
-        """Whether products take a kernel of their own (``fused``, asked without changing the form a tensor is held in)."""
+        """Whether products take a kernel of their own (asked without having the walk's arrays made, as ``fused`` has)."""
         return self._planes is not None or self.fused is not None
 
     def _launch(self, fn, *args):
@@ -284,10 +285,10 @@ class HipPredictiveTensor:
         self._planes = planes
         return True
 
-    def _leave_planes(self):
-        """The frame's arrays in the planes' place: the words, coded once more with the frame's own frequencies in the
-        contexts that were kept of the reference, which gives the same main stream, and packed residuals.  The planes
-        stay allocated: calls of other threads and streams and captured launches may be reading them."""
+    def _walk_attributes(self):
+        """The walk's attributes of a tensor that is held as planes: of the words, coded once more with the frame's own frequencies
+        in the contexts that were kept of the reference, which gives the same main stream, and packed residuals."""
+        import copy
         import torch
         r, c = self.shape
         words = self.decode(None, check=False).view(torch.int16).cpu().numpy().view(np.uint16)
@@ -302,13 +303,15 @@ class HipPredictiveTensor:
         info = dict(mode=0, labels=labels, flips=flips, thresholds=np.frombuffer(meta[2 * r:], dtype="<u2").copy(), main_freq=freq,
                     stream=codec._encode_given(main, ctx, freq), data=codec._packbits(residual, 5))
         about = dict(shape=self.shape, mode=self.mode, target_sha256=self.target_sha256)
-        self._hold_streams(_indexed(about, info, ctx, self.stride, True, self._asked_segment))
-        if self._raw5_segment:
-            rows, cols = self.shape
-            bins = _fused.order_records(bins, rows, cols, self._raw5_segment, self._raw5_block, self.buffers["row_pos"].cpu().numpy(),
-                                        self._rows_held, 32, 16)
-        self.buffers["context_bins"] = torch.from_numpy(np.ascontiguousarray(bins).view(np.int32)).to(self.device)
-        self._used, self._planes, self._kept = self._planes, None, None
+        other = copy.copy(self)  # (so that this object has none of them until all are made)
+        other._planes = None
+        other._hold_streams(_indexed(about, info, ctx, self.stride, True, self._asked_segment))
+        if other._raw5_segment:
+            bins = _fused.order_records(bins, r, c, other._raw5_segment, other._raw5_block, other.buffers["row_pos"].cpu().numpy(),
+                                        other._rows_held, 32, 16)
+        other.buffers["context_bins"] = torch.from_numpy(np.ascontiguousarray(bins).view(np.int32)).to(self.device)
+        made = {name: value for name, value in vars(other).items() if name in HipPredictiveTensor._WALK}
+        return {**made, "fused_reason": other.fused_reason}
 
     def _hold_streams(self, ix):
         """The device arrays of a frame that is walked where it lies, from what ``_read_frame`` gave."""
@@ -390,8 +393,10 @@ class HipPredictiveTensor:
         import copy
         import torch
         other = copy.copy(self)
-        other._used = None
-        if other._planes is not None:
+        if other._planes is not None:  # (the copy makes its walk's arrays itself, should they be asked for)
+            for name in HipPredictiveTensor._WALK:
+                vars(other).pop(name, None)
+            other.fused_reason = None
             other._planes = other._planes.clone()
             other.error = torch.zeros_like(self.error)
             return other
@@ -405,9 +410,10 @@ class HipPredictiveTensor:
     def resident_bytes(self):
         """Every device allocation this tensor holds: buffers, tilings made so far, the error word."""
         p = self._planes
-        if p is not None:
-            return p.nbytes + 4
-        total = sum(t.numel() * t.element_size() for t in self.buffers.values()) + 4 + (self._used.nbytes if self._used is not None else 0)
+        total = 4 + (p.nbytes if p is not None else 0)
+        if p is not None and "buffers" not in vars(self):
+            return total
+        total += sum(t.numel() * t.element_size() for t in self.buffers.values())
         total += sum(rows.numel() * 4 + classes.numel() for _, rows, classes, _ in self._tilings.values())
         return int(total)
 
@@ -670,9 +676,16 @@ class HipPredictiveGroup:
         self.m_invariant = any(t.m_invariant for t in self.tensors) if m_invariant is None else bool(m_invariant)
         self.error = torch.zeros((), device=self.device, dtype=torch.int32)
         self._tilings, self._pointer_arrays = {}, {}
-        self._index, self._walked = first._index, None  # (members whose frames are walked, their group) where some are held as planes
-        for key in () if any(t._planes is not None for t in self.tensors) else ("waves", "gemm"):
-            self._tiling(key)  # raises FusedUnsupported when the members cannot share a tiling
+        self._index = first._index
+        # members whose frames are walked, beside others that are held as planes, have a launch of their own
+        self._walked = None  # (their places, their group)
+        rest = [i for i, t in enumerate(self.tensors) if t._planes is None]
+        if len(rest) == len(self.tensors):
+            for key in ("waves", "gemm"):
+                self._tiling(key)  # raises FusedUnsupported when the members cannot share a tiling
+        elif rest:
+            self._walked = rest, HipPredictiveGroup([self.tensors[i] for i in rest], m_invariant=self.m_invariant)
+            self._walked[1].error = self.error  # (what a caller polls)
 
     def _tiling(self, key):
         import torch
@@ -728,12 +741,9 @@ class HipPredictiveGroup:
         planes = [t._planes for t in self.tensors]
         if any(p is not None for p in planes):
             outs = planes_group(self, planes, x, biases)
-            rest = [i for i, p in enumerate(planes) if p is None]
-            if rest:  # two kinds of members are two launches
-                walked = self._walked
-                if walked is None or walked[0] != rest:
-                    walked = self._walked = rest, HipPredictiveGroup([self.tensors[i] for i in rest], m_invariant=self.m_invariant)
-                for i, y in zip(rest, walked[1].linear(x, [biases[i] for i in rest], check=check, batch_invariant=batch_invariant)):
+            if self._walked is not None:
+                rest, walked = self._walked
+                for i, y in zip(rest, walked.linear(x, [biases[i] for i in rest], check=check, batch_invariant=batch_invariant)):
                     outs[i] = y
             return outs
         if packed is not None:

@@ -163,9 +163,10 @@ def tilings(probe, out, seed):
 def linear(out, seed):
     import numpy as np
     import torch
-    from georefine_amd import _native, bitexact_context_codec as codec
+    from georefine_amd import _native, _planes, bitexact_context_codec as codec
     from georefine_amd.bitexact_context_gpu import HipContextTensor, dense_linear
     lib = _native.hip()
+    _planes.FROM_WEIGHTS = 1 << 40  # what is timed follows the walk's decode: matrices of every size stay frames
 
     class Asked:
         """The library, with its plan's answer given."""

@@ -20,8 +20,10 @@ sys.path.insert(0, str(Path(__file__).resolve().parents[1]))
 import numpy as np
 import torch
 
-from georefine_amd import _fused, bitexact_context_codec as codec
+from georefine_amd import _fused, _planes, bitexact_context_codec as codec
 from georefine_amd.bitexact_context_gpu import HipContextTensor
+
+_planes.FROM_WEIGHTS = 1 << 40  # what is timed is the walk: matrices of every size stay frames
 
 NAMED = [(300, 4096), (450, 6144), (600, 5120), (1024, 5120), (1500, 2064), (700, 9216), (2048, 5120), (2560, 5120), (3000, 3072),
          (4096, 4096), (5120, 6144), (6144, 5120), (5120, 17408), (17408, 5120)]

@@ -21,9 +21,11 @@ sys.path.insert(0, str(Path(__file__).resolve().parents[1]))
 import numpy as np
 import torch
 
-from georefine_amd import _fused, bitexact_context_codec as codec, bitexact_predictive_codec as predictive
+from georefine_amd import _fused, _planes, bitexact_context_codec as codec, bitexact_predictive_codec as predictive
 from georefine_amd.bitexact_context_gpu import HipContextTensor
 from georefine_amd.bitexact_predictive_gpu import HipPredictiveTensor
+
+_planes.FROM_WEIGHTS = 1 << 40  # what is timed is the walk: matrices of every size stay frames
 
 ROWS = (2, 6, 20, 32, 64, 96, 128)
 

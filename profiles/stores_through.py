@@ -78,8 +78,9 @@ def libraries(folder):
 def coded(rows, cols):
     import numpy as np
     import torch
-    from georefine_amd import bitexact_context_codec as codec
+    from georefine_amd import _planes, bitexact_context_codec as codec
     from georefine_amd.bitexact_context_gpu import HipContextTensor
+    _planes.FROM_WEIGHTS = 1 << 40  # what is timed is the walk: matrices of every size stay frames
     g = torch.Generator(device="cuda").manual_seed(rows * cols)
     w = torch.randn(rows, cols, device="cuda", generator=g) * 0.02 * torch.exp(0.5 * torch.randn(rows, 1, device="cuda", generator=g))
     w = torch.where(torch.rand(rows, cols, device="cuda", generator=g) < 1e-3, 10.0 * w, w)
@@ -89,8 +90,9 @@ def coded(rows, cols):
 def coded_predictive(rows, cols):
     import numpy as np
     import torch
-    from georefine_amd import bitexact_predictive_codec as predictive
+    from georefine_amd import _planes, bitexact_predictive_codec as predictive
     from georefine_amd.bitexact_predictive_gpu import HipPredictiveTensor
+    _planes.FROM_WEIGHTS = 1 << 40  # (as in coded)
     g = torch.Generator(device="cuda").manual_seed(rows * cols)
     w = torch.randn(rows, cols, device="cuda", generator=g) * 0.02 * torch.exp(0.5 * torch.randn(rows, 1, device="cuda", generator=g))
     near = w + 0.002 * torch.randn(rows, cols, device="cuda", generator=g)

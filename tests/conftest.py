@@ -36,6 +36,13 @@ def weight_like(rng, rows, cols, sigma=0.02, row_scale=True, outliers=True):
     return bf16_words(w)
 
 
+@pytest.fixture
+def walked(monkeypatch):
+    """Matrices of every size stay frames, as small ones do: for the tests of the kernels that walk them."""
+    from georefine_amd import _planes
+    monkeypatch.setattr(_planes, "FROM_WEIGHTS", 1 << 40)
+
+
 @pytest.fixture(scope="session")
 def oracle():
     from oracle import codec_oracle

@@ -6,7 +6,7 @@ import pytest
 
 from conftest import SPECIAL_WORDS, weight_like
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("walked")]
 
 
 def _cases():

@@ -4,7 +4,7 @@ import pytest
 
 from conftest import bf16_words, weight_like, words_to_float
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("walked")]
 
 
 def _tensor(words, nr=16, nc=4, **kw):

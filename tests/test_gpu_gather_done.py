@@ -9,6 +9,14 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
+@pytest.fixture(params=["walked", "planes"])
+def form(request):
+    """The tensors of a test as frames, then as planes."""
+    if request.param == "walked":
+        request.getfixturevalue("walked")
+    return request.param
+
+
 def _tensor(rows=300, cols=64 * 30, seed=3, **options):
     from georefine_amd import bitexact_context_codec as codec
     from georefine_amd.bitexact_context_gpu import HipContextTensor
@@ -43,10 +51,10 @@ def test_counters_return_to_zero(count):
 
 @pytest.mark.parametrize("segment", [16, 32, 64])
 @pytest.mark.parametrize("count", [1, 777, 3999, 4000])
-def test_lookups_that_are_polled_for_and_that_are_not(segment, count):
+def test_lookups_that_are_polled_for_and_that_are_not(segment, count, form):
     import torch
     t, words = _tensor(fused_segment=segment)
-    assert t.fused.seg_len == segment
+    assert (t._planes is not None) == (form == "planes") and t.fused.seg_len == segment
     ids = torch.from_numpy(np.random.default_rng(count).integers(0, 300, count))
     want, on_device = words[ids.numpy()], ids.cuda()
     for options in ({}, {"check": False}, {"check": False, "validate": False}):
@@ -86,7 +94,7 @@ def test_a_refused_row_keeps_its_output(count):
 
 
 @pytest.mark.parametrize("spin", [0, 100])
-def test_threads_on_streams_of_their_own(spin, monkeypatch):
+def test_threads_on_streams_of_their_own(spin, form, monkeypatch):
     import torch
     from georefine_amd import bitexact_context_gpu as gpu
     monkeypatch.setattr(gpu, "GATHER_SPIN_US", spin)  # 0: every call waits for its stream

@@ -6,7 +6,7 @@ import pytest
 
 from conftest import bf16_words, weight_like
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("walked")]
 
 
 def _members(shapes, seed, segment=32):

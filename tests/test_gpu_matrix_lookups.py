@@ -4,7 +4,7 @@ import pytest
 
 from conftest import bf16_words, weight_like, words_to_float
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("walked")]
 
 
 @pytest.mark.parametrize("shape", [(200, 1280), (67, 320), (530, 2048)])

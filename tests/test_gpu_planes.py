@@ -204,7 +204,7 @@ def test_infinities_and_nan_go_where_the_dense_product_puts_them():
             assert torch.equal(state(y), state(want)), (m, state)
 
 
-def test_a_tensor_answers_as_planes_and_leaves_them_when_its_arrays_are_asked_for():
+def test_a_tensor_answers_as_planes_whatever_is_looked_at():
     import torch
     from georefine_amd import bitexact_context_codec as codec
     from georefine_amd.bitexact_context_gpu import HipContextTensor, HipLinearGroup
@@ -234,16 +234,18 @@ def test_a_tensor_answers_as_planes_and_leaves_them_when_its_arrays_are_asked_fo
                 t.gather_rows(torch.tensor([3, bad]))
             last = t.gather_rows(torch.tensor([3, bad]), check=False, validate=False)[1]
             assert np.array_equal(last.view(torch.int16).cpu().numpy().view(np.uint16), words[0 if bad < 0 else 699])
-        as_planes = t.resident_bytes
-        assert other.resident_bytes == as_planes and t._planes is not None
+        as_planes, before, grouped = t.resident_bytes, t.linear(x[:20]), group.linear(x[:20])
+        assert other.resident_bytes == as_planes
         streams = HipContextTensor.host_prepare(frame)["indexed"]
-        assert t.fused is not None and t._planes is None  # the frame's arrays, the same as it had held from the start
+        assert t.fused is not None  # the frame's arrays, the same as of one that is walked
         for name in ("main_stream", "rows", "columns", "main_freq", "fused_seg_state", "fused_seg_offset", "residual_stream"):
             assert np.array_equal(t.buffers[name].cpu().numpy()[:streams[name].size], streams[name]), name
-        assert t.mode == frame[5] and t.frame_bytes == len(frame) and other._planes is not None
-        assert np.array_equal(t.decode().view(torch.int16).cpu().numpy().view(np.uint16), words)
-        mixed, walked = group.linear(x[:20]), HipLinearGroup([t]).linear(x[:20])  # (two launches from here on)
-        assert torch.equal(mixed[0], walked[0]) and torch.equal(mixed[1], alone.linear(x[:20])[0]) and torch.equal(mixed[2], other.linear(x[:20]))
+        assert t.mode == frame[5] and t.frame_bytes == len(frame) and t.resident_bytes > as_planes == other.resident_bytes
+        for general in (False, True):
+            assert np.array_equal(t.decode(general=general).view(torch.int16).cpu().numpy().view(np.uint16), words)
+        # and what calls run is what they ran before
+        assert torch.equal(t.linear(x[:20]), before) and all(torch.equal(a, b) for a, b in zip(group.linear(x[:20]), grouped))
+        assert torch.equal(grouped[0], before) and torch.equal(grouped[1], alone.linear(x[:20])[0]) and torch.equal(grouped[2], other.linear(x[:20]))
         assert np.array_equal(other.decode(general=True).view(torch.int16).cpu().numpy().view(np.uint16), words) and other._raw6_block == 16
 
 
@@ -273,9 +275,43 @@ def test_captured_launches_replay_on_new_rows():
         graph.replay()
         torch.cuda.synchronize()
         assert all(torch.equal(a.view(torch.int16), b.view(torch.int16)) for a, b in zip(captured, eager))
-    assert t.buffers["main_stream"].is_cuda and t._planes is None  # what was captured still reads the planes
+    assert t.buffers["main_stream"].is_cuda and t.decode(general=True).is_cuda
     torch.cuda.empty_cache()
     x1.copy_(draw(1)), x40.copy_(draw(40))
     graph.replay()
-    want = group.tensors[1].linear(x1)  # (the clone's planes, the same words)
+    want = t.linear(x1)
     assert torch.equal(captured[0], want) and torch.equal(captured[1], captured[2])
+
+
+def test_captured_launches_of_a_small_member_outlive_groups_and_looks():
+    import gc
+    import torch
+    from georefine_amd import bitexact_context_codec as codec
+    from georefine_amd.bitexact_context_gpu import HipContextTensor, HipLinearGroup
+    rng = np.random.default_rng(14)
+    small, large = (HipContextTensor(codec.encode(weight_like(rng, rows, 1040))) for rows in (48, 700))
+    pair = HipLinearGroup([small, HipContextTensor(codec.encode(weight_like(rng, 40, 1040)))])
+    draw = lambda m: torch.from_numpy(bf16_words(rng.normal(0, 1, (m, 1040)))).view(torch.bfloat16).cuda()
+    x1, x9 = draw(1), draw(9)
+    step = lambda: [small.linear(x1), *pair.linear(x9), small.decode(check=False)]
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        step()
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = step()
+    group = HipLinearGroup([large, small])
+    group.linear(x9)
+    assert small.fused is not None and small.buffers["main_stream"].is_cuda
+    gc.collect()
+    torch.cuda.empty_cache()
+    for _ in range(3):
+        x1.copy_(draw(1)), x9.copy_(draw(9))
+        eager = [v.clone() for v in step()]
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a.view(torch.int16), b.view(torch.int16)) for a, b in zip(captured, eager))

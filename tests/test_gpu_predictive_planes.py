@@ -1,4 +1,6 @@
-"""Predictive matrices held as planes: the same answers as the walk's, and the way back to its arrays."""
+"""Predictive matrices held as planes: the same answers as the walk's, and the walk's arrays beside them."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -14,7 +16,7 @@ def _pair(rng, rows, cols):
 
 
 @pytest.mark.parametrize("rows,cols", [(517, 1056), (1024, 2080)])
-def test_products_decode_and_the_way_back(rows, cols, monkeypatch):
+def test_products_decode_and_the_walks_arrays(rows, cols, monkeypatch):
     import torch
     from georefine_amd import _planes
     from georefine_amd import bitexact_predictive_codec as codec
@@ -49,12 +51,17 @@ def test_products_decode_and_the_way_back(rows, cols, monkeypatch):
     assert torch.equal(t.linear(None, PackedActivations(x[:9])), whole[:9]) and torch.equal(t.gemv(None, x[:8]), whole[:8])
     with pytest.raises(ValueError):
         t.gemv(None, x[:9])
-    # the frame's arrays, the same as had been held from the start
+    # the frame's arrays, the same as of one that is walked, and what calls run is what they ran before
     for name, array in w.buffers.items():
         mine = t.buffers[name]
         assert mine.dtype == array.dtype and (name == "context_bins" or torch.equal(mine, array)), name
-    assert t._planes is None and set(t.buffers) == set(w.buffers) and other._planes is not None
+    assert set(t.buffers) == set(w.buffers) and t.resident_bytes > other.resident_bytes
+    # (the plane of bins where it is read)
+    own = torch.empty(t.shape, device="cuda", dtype=torch.int16)
+    t._launch(t._lib.grf_ppcx_fused_decode, ctypes.byref(t.fused), ctypes.byref(t._tiling_for("waves")[0]), t.buffers["context_bins"].data_ptr(),
+              own.data_ptr(), t.error.data_ptr())
+    assert np.array_equal(own.cpu().numpy().view(np.uint16), target) and t.error.item() == 0
     assert torch.equal(t.decode(None).view(torch.int16), other.decode(None).view(torch.int16))
-    assert torch.equal(t.linear(None, x[:20]), w.linear(None, x[:20]))  # (which takes the plane of bins where it is read)
+    assert torch.equal(t.gemm(None, x), whole) and torch.equal(group.linear(x[:20], batch_invariant=True)[0], whole[:20])
     ref = torch.from_numpy(near.view(np.int16)).view(torch.bfloat16).cuda()
     assert np.array_equal(other.decode(ref, general=True).view(torch.int16).cpu().numpy().view(np.uint16), target)

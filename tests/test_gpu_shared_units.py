@@ -4,7 +4,7 @@ import pytest
 
 from georefine_amd import bitexact_context_codec as codec
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("walked")]
 
 
 @pytest.mark.parametrize("rows,cols,members", [(2048, 5120, 1), (2047, 5104, 1), (4096, 2560, 2), (1024, 5120, 1)])

@@ -4,7 +4,7 @@ import pytest
 
 from georefine_amd import bitexact_context_codec as codec
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("walked")]
 
 
 @pytest.mark.parametrize("rows,cols", [(256, 512), (257, 560), (1000, 1040), (3839, 1024), (900, 4096)])

@@ -3,7 +3,7 @@ what a host sum over the parts in the workspace gives, for part counts around th
 import numpy as np
 import pytest
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("walked")]
 
 
 @pytest.mark.parametrize("parts", [2, 3, 4, 5, 8, 9])
