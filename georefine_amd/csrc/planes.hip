@@ -938,7 +938,7 @@ int grf_planes_fill(const uint16_t *words, uint32_t rows, uint32_t cols, const u
 size_t grf_planes_workspace_bytes(uint32_t n, const grf_planes *const *planes, uint32_t m_rows) {
   size_t bytes = 0;
   for (uint32_t i = 0; planes && i < n; ++i)
-    if (planes[i]) {
+    if (check_planes("grf_planes_workspace_bytes", planes[i]) == GRF_OK) {  // (what a launch refuses needs none)
       const uint32_t m = std::min(m_rows, kMaxTileRows);
       bytes += n == 1 && own_parts(*planes[i]) > 1 ? sums_bytes(*planes[i], m) : partial_bytes(*planes[i], m);
     }

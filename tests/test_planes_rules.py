@@ -34,6 +34,16 @@ def test_what_the_kernels_would_not_take_is_refused_before_a_launch(change):
     assert lib.grf_planes_linear(ctypes.addressof(p), 4096, 2048, 1, 0, 4096, None, None, 0, None) != 0
 
 
+@pytest.mark.parametrize("change", [{}, dict(splits=0), dict(splits=17), dict(rows=0), dict(cols=0), dict(planes=8), dict(listed=None)])
+def test_a_workspace_is_asked_for_what_a_launch_takes_and_nothing_else(change):
+    lib = _native.hip()
+    p = _hip_abi.GrfPlanes(**{**dict(planes=4096, bases=4096, listed_at=4096, listed=4096, rows=5120, cols=17408, splits=12), **change})
+    one = (ctypes.c_void_p * 2)(ctypes.addressof(p), None)
+    for n, m, want in ((1, 1, 12 * 5120 * 4), (1, 6, 12 * 6 * 5120 * 4), (1, 128, 12 * 128 * 5120 * 4), (2, 8, 0), (2, 9, 12 * 9 * 5120 * 4)):
+        assert lib.grf_planes_workspace_bytes(n, one, m) == (0 if change else want), (n, m)
+    assert lib.grf_planes_workspace_bytes(2, None, 6) == 0
+
+
 def test_small_sparse_and_odd_frames_stay_frames():
     rng = np.random.default_rng(3)
     large = codec.encode(weight_like(rng, 512, 1024))
