@@ -619,8 +619,10 @@ int product(const char *who, uint32_t n, const grf_planes *const *planes, const 
   for (uint32_t done = 0; done < m_rows; done += kMaxTileRows) {
     const uint32_t m = std::min(kMaxTileRows, m_rows - done), m_pad = 16 * grf::gemm_tiles(m);
     const bool batch = m > kOwnRows || (m > kOwnAlways && visits >= kOwnVisits) || (m > 16 && waves * Product<4>::kWaveBytes > kLdsBytes);
+    // (rows that need no workspace use one that is there and aligned)
+    const bool room = workspace && !((uintptr_t)workspace & 15) && workspace_bytes >= sums_bytes(*planes[0], m);
+    const uint32_t parts = batch || n > 1 || !room ? 1 : own_parts(*planes[0]);
     // (fifteen or sixteen waves with two eights of rows do not fit in a unit's LDS; eight have the splits two each)
-    const uint32_t parts = batch || n > 1 || workspace_bytes < sums_bytes(*planes[0], m) ? 1 : own_parts(*planes[0]);
     const uint32_t own_waves = parts > 1 ? (planes[0]->splits + parts - 1) / parts
                                : waves * Product<2>::kWaveBytes > kLdsBytes && (m > 8 || packed) ? 8 : waves;
     const PlanesX rows{reinterpret_cast<const uint8_t *>(x) + (size_t)done * ldx * 2, packed ? 16 : ldx * 2, packed ? m_pad * 16 : 16, m, cols, packed};

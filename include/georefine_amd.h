@@ -579,8 +579,8 @@ int grf_dense_gemm(const uint16_t *w, uint32_t rows, uint32_t cols, const uint16
  * grf_planes_fill   planes and list, given those
  * grf_planes_linear, _group  y = x W^T (+ bias) for any number of rows and up to four matrices of one width:
  *                   fp32 sums in an order that the matrix's sizes and splits fix, so that a row has the same bits in every
- *                   batch and group.  workspace: grf_planes_workspace_bytes, 16-byte aligned; up to eight rows run with less or none, and
- *                   then give every row block one workgroup.  x: 16-byte aligned, ldx a multiple of 8; or, with `packed`, up to 128 rows as
+ *                   batch and group.  workspace: grf_planes_workspace_bytes (0 for planes that a launch refuses), 16-byte aligned; up to eight
+ *                   rows run with less, with none or with one that is not aligned, and then give every row block one workgroup.  x: 16-byte aligned, ldx a multiple of 8; or, with `packed`, up to 128 rows as
  *                   grf_pack_activations leaves them
  * grf_planes_prompt the product of many rows of x (any number from one on) without the dense matrix.  plan: rows of x a workgroup takes (128 or 256), and
  *                   the parts of K (whole visits, up to 63 each) from bit 16 on, as grf_planes_prompt_plan gives it, or -1

@@ -132,12 +132,16 @@ def test_row_blocks_that_workgroups_share_give_the_bits_of_whole_ones(rows, cols
     exact = x.double() @ words.double().T + bias.double()
     bound = exact.abs() * 2.0 ** -8 + (x.double().abs() @ words.double().abs().T + 8) * cols * 2.0 ** -24
     for m in (1, 2, 7, 8):
-        whole, shared = (torch.full((m + 2, rows), 7.0, device="cuda", dtype=torch.bfloat16) for _ in range(2))
-        for y, s, n in ((whole, None, 0), (shared, space.data_ptr(), size)):  # without a workspace blocks are whole
+        whole, absent, askew, shared = (torch.full((m + 2, rows), 7.0, device="cuda", dtype=torch.bfloat16) for _ in range(4))
+        # without a workspace blocks are whole, and one that is null or not aligned is none
+        for y, s, n in ((whole, None, 0), (absent, None, size), (askew, space.data_ptr() + 4, size), (shared, space.data_ptr(), size)):
+            if y is shared:
+                assert bool((space == 5).all())
             _launch(lib.grf_planes_linear, p.address, x.data_ptr(), cols, m, 0, y[1:].data_ptr(), bias.data_ptr(), s, n)
         assert torch.equal(whole, shared) and bool((shared[0] == 7).all() and (shared[-1] == 7).all())
+        assert torch.equal(whole, absent) and torch.equal(whole, askew) and bool((space[size // 4:] == 5).all())
+        space.fill_(5)
         assert bool(((shared[1:-1].double() - exact[:m]).abs() <= bound[:m]).all())
-    assert bool((space[size // 4:] == 5).all())
 
 
 def test_members_of_more_splits_than_the_largest_one_have_two_a_wave():
