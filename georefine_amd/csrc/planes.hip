@@ -97,7 +97,7 @@ struct XPlaces {
 // for all copies that it knows of), when the wave's reads there are done.
 __device__ __forceinline__ void copy_to_lds(const uint8_t *base, uint32_t from, uint32_t to) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(from), "s"(base), "s"(to) : "memory");
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(from), "s"(base), "s"(to) : "m0", "memory");
 #else
   (void)base, (void)from, (void)to;
 #endif

@@ -1,5 +1,7 @@
 """Which matrices are held as planes, how their sums are split, and that the sizes agree with the library's (no GPU)."""
 import ctypes
+import re
+from pathlib import Path
 
 import numpy as np
 import pytest
@@ -100,3 +102,13 @@ def test_products_of_many_rows_that_a_launch_would_not_take_are_refused(change):
     a = {**dict(x=4096, ldx=1024, m=200, plan=1 << 16 | 128, y=4096, ldy=64), **change}
     assert lib.grf_planes_prompt(ctypes.addressof(p), a["x"], a["ldx"], a["m"], a["plan"], a["y"], a["ldy"], None, None, 0, None) != 0
     assert b"grf_planes_prompt" in lib.grf_last_error()
+
+
+def test_assembly_that_writes_m0_says_so():
+    found = 0
+    for source in sorted((Path(_native.__file__).parent / "csrc").iterdir()):
+        for statement in re.findall(r"\basm\b[^;]*;", source.read_text()):
+            if re.search(r"\bm0\s*,", statement.split('"::')[0].replace('"m0",', "")):  # (an instruction's first operand)
+                found += 1
+                assert '"m0"' in statement, (source.name, statement)
+    assert found >= 2
