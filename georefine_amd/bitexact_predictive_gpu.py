@@ -80,11 +80,12 @@ def _fused_segment(shape, segment=None):
     return seg_len
 
 
-def _read_frame(frame, reference, stride, *, fused=False, fused_segment=None):
+def _read_frame(frame, reference, stride, *, fused=False, fused_segment=None, planes=False):
     """Parse, validate and index a frame against its reference words.  With ``fused`` the
     result also carries ``fused_plan`` (or ``fused_reason``) with ``walk_plan``, the same with the lookups
     of the vector-ALU launches, and keeps the residuals in the packed 5-bit form whatever the
-    frame's mode (``resident_mode`` 0)."""
+    frame's mode (``resident_mode`` 0).  With ``planes`` as well, a frame that is better held so gives its words and no index
+    (``_words_of``)."""
     if not isinstance(frame, (bytes, bytearray, memoryview)):
         raise codec.CodecError("frame must be bytes")
     info = codec.parse(frame, reference)
@@ -101,6 +102,8 @@ def _read_frame(frame, reference, stride, *, fused=False, fused_segment=None):
         result["raw"] = target
         return result
     ctx = codec.contexts(info["reference"], info["labels"], info["flips"], info["thresholds"])
+    if fused and planes and _worth_planes(info, ctx, fused_segment):
+        return dict(result, **_words_of(info, ctx, stride))
     return _indexed(result, info, ctx, stride, fused, fused_segment)
 
 
@@ -154,40 +157,49 @@ def _indexed(result, info, ctx, stride, fused, fused_segment):
     return result
 
 
-def _read_words(frame, reference, stride, fused_segment):
-    """The words of a frame that can be held as planes, validated, with what is needed to make its arrays later (``_indexed``); None
-    of one that cannot: what the fused kernels refuse, raw words and small matrices (``_planes``)."""
-    if not isinstance(frame, (bytes, bytearray, memoryview)) or len(frame) < codec.HEADER.size:
-        return None  # (``_read_frame`` says what is wrong)
-    mode, (r, c) = frame[5], codec.HEADER.unpack_from(frame)[4:6]
+def _worth_planes(info, ctx, fused_segment):
+    """Whether the words of a parsed frame are held as planes: not where the fused kernels refuse the frame, nor small matrices
+    (``_planes``), nor where the planes would take more than the walk's arrays and 4 %.  What they would list is
+    taken from the frame's own frequencies, as each label's words meet them (a row's own eleven exponents are no worse
+    on average), so that a frame is decoded once either way."""
+    r, c = info["shape"]
     n = r * c
-    if mode == 2 or n < _planes.FROM_WEIGHTS or c > _planes.MAX_COLS:
-        return None
+    if n < _planes.FROM_WEIGHTS or c > _planes.MAX_COLS:
+        return False
     try:
         seg_len = _fused_segment((r, c), fused_segment)
     except _fused.FusedUnsupported:
-        return None
-    info = codec.parse(frame, reference)
+        return False
     freq = info["main_freq"].reshape(codec.MAIN_CONTEXTS, codec.MAIN_VOCAB)
     live, sums = (freq > 0).sum(axis=1), freq.sum(axis=1, dtype=np.uint64)
     if not 0 < live.max() <= 255 or not np.isin(sums, (0, 65536)).all():
-        return None
-    ctx = codec.contexts(info["reference"], info["labels"], info["flips"], info["thresholds"])
+        return False
+    # (a seventh of the words: in all rows, and no multiple of a power of two apart)
+    met = np.bincount(ctx.reshape(-1)[::7], minlength=codec.MAIN_CONTEXTS)
+    exponents = freq.reshape(16, 16, 2, 256, 4).sum(axis=(2, 4), dtype=np.float64) * met.reshape(16, 16, 1) / 65536
+    by_label = exponents.sum(axis=1)
+    running = np.concatenate((np.zeros((16, 1)), np.cumsum(by_label, axis=1)), axis=1)
+    inside = (running[:, _planes.EXPONENTS:] - running[:, :-_planes.EXPONENTS]).max(axis=1).sum()
+    listed = max(0.0, 1 - inside / met.sum()) * n
+    # what the arrays of the walk would take: streams, bins, the index and the tables
+    walked = len(info["stream"]) + n * 9 // 8 + 8 * r * (c // seg_len + 1) + 16 * (16 * 8 * (int(live.max()) + 1) + _LUT_BUDGET)
+    return _planes.plane_bytes(r, c) + 4 * (listed + r + r // 16 * _planes.visits(c)) <= _planes.MEMORY * walked
+
+
+def _words_of(info, ctx, stride):
+    """The words of a frame, validated, with what is needed to make its arrays later (``_indexed``)."""
+    r, c = info["shape"]
+    freq = info["main_freq"].reshape(codec.MAIN_CONTEXTS, codec.MAIN_VOCAB)
     _, _, main = _checkpoints(info["stream"], ctx, freq, codec.MAIN_VOCAB, stride)
-    if mode == 0:
-        residual = codec._unpackbits(info["data"], 5, n, "raw5")
+    if info["mode"] == 0:
+        residual = codec._unpackbits(info["data"], 5, r * c, "raw5")
     else:
         rf = info["residual_freq"].reshape(codec.RES_CONTEXTS, codec.RES_VOCAB)
         _, _, residual = _checkpoints(info["residual_stream"], main, rf, codec.RES_VOCAB, stride)
     words = codec.join_symbols(main, residual)
     if hashlib.sha256(words.tobytes()).digest() != info["target_sha256"]:
         raise codec.CodecError("target checksum mismatch")
-    about = dict(shape=(r, c), mode=mode, frame_bytes=len(frame), frame_sha256=hashlib.sha256(bytes(frame)).hexdigest(),
-                 source_sha256=info["target_sha256"].hex(), target_sha256=info["target_sha256"].hex(),
-                 reference_sha256=info["reference_sha256"].hex())
-    # what the arrays of the walk would take: streams, bins, the index and the tables
-    walked = len(info["stream"]) + n * 9 // 8 + 8 * r * (c // seg_len + 1) + 16 * (16 * 8 * (int(live.max()) + 1) + _LUT_BUDGET)
-    return dict(about=about, words=words.view(np.int16).reshape(r, c), bins=_pairs(ctx), meta=info["meta"], table=info["table"], walked=walked)
+    return dict(words=words.view(np.int16).reshape(r, c), bins=_pairs(ctx), meta=info["meta"], table=info["table"])
 
 
 def _pairs(ctx):
@@ -206,8 +218,7 @@ class HipPredictiveTensor:
                  fused_segment=None, resident_contexts=True, m_invariant=False):
         if not isinstance(stride, int) or not 1 <= stride <= 65536:
             raise codec.CodecError("invalid checkpoint stride")
-        read = _read_words(frame, reference_uint16_numpy, stride, fused_segment) if fused and resident_contexts else None
-        ix = _read_frame(frame, reference_uint16_numpy, stride, fused=fused, fused_segment=fused_segment) if read is None else None
+        ix = _read_frame(frame, reference_uint16_numpy, stride, fused=fused, fused_segment=fused_segment, planes=resident_contexts)
         import torch
         if not torch.cuda.is_available():
             raise RuntimeError("a ROCm GPU is required")
@@ -219,10 +230,9 @@ class HipPredictiveTensor:
         self._index = device_index(self.device)
         self._asked_segment = fused_segment
         self.error = torch.zeros((), device=self.device, dtype=torch.int32)
-        if read is not None and self._hold_planes(read):
+        if "words" in ix:
+            self._hold_planes(ix)
             return
-        if ix is None:
-            ix = _read_frame(frame, reference_uint16_numpy, stride, fused=fused, fused_segment=fused_segment)
         self._hold_streams(ix)
         # What the tile walker needs of the reference is the 4-bit bin of every word (the
         # decoded word itself comes from the frame's symbols alone), and the reference is given
@@ -271,19 +281,15 @@ class HipPredictiveTensor:
         self._status(launch_on(self._index, fn, *args), False)
 
     def _hold_planes(self, read):
-        """Holds the words as planes unless they list so many that the walk's arrays are smaller."""
         import torch
         planes = _planes.Planes.of_words(torch.from_numpy(read["words"]).to(self.device), self._launch)
-        if planes.nbytes > _planes.MEMORY * read["walked"]:
-            return False
         torch.cuda.current_stream(self.device).synchronize()  # (a first product may be on another stream)
-        for name, value in read["about"].items():
-            setattr(self, name, value)
-        self.n = math.prod(self.shape)
+        self.n = math.prod(read["shape"])
+        for name in ("shape", "mode", "frame_bytes", "frame_sha256", "source_sha256", "target_sha256", "reference_sha256"):
+            setattr(self, name, read[name])
         self.resident_mode, self.fused_reason, self.has_contexts = 0, None, True
         self._kept = {name: read[name] for name in ("bins", "meta", "table")}
         self._planes = planes
-        return True
 
     def _walk_attributes(self):
         """The walk's attributes of a tensor that is held as planes: of the words, coded once more with the frame's own frequencies

@@ -1,5 +1,6 @@
 """A tensor that is held as planes stays so whatever is looked at, and a group leaves its members as they are
 (no GPU: device calls are stand-ins, and the arrays are the host's)."""
+import contextlib
 import gc
 import threading
 import types
@@ -22,7 +23,10 @@ class _HostPlanes(_planes.Planes):
 
     def __init__(self, words):
         self.rows, self.cols = words.shape
-        self.words, self.nbytes, self.address = words, words.numel() * 3 // 2, 0
+        exponents = (words.int() >> 7 & 255).long()
+        held = torch.zeros(self.rows, 256, dtype=torch.int64).scatter_add_(1, exponents, torch.ones_like(exponents))
+        listed = words.numel() - int(held.unfold(1, _planes.EXPONENTS, 1).sum(2).amax(1).sum())
+        self.words, self.nbytes, self.address = words, _planes.plane_bytes(*words.shape) + 4 * listed, 0
 
     @classmethod
     def of_words(cls, words, launch):
@@ -109,3 +113,21 @@ def test_another_thread_never_sees_half_of_the_walks_attributes(monkeypatch):
     go.set()
     first.join(), second.join()
     assert seen[0] is not None and seen[0] is t.fused
+
+
+def test_a_predictive_frame_is_decoded_once_whatever_it_is_held_as(monkeypatch):
+    """One whose words the planes would mostly list stays a frame, and is not read a second time for it."""
+    rng, walks = np.random.default_rng(5), []
+    spread = (rng.integers(0, 2, (512, 1024)) << 15 | rng.integers(60, 180, (512, 1024)) << 7 | rng.integers(0, 128, (512, 1024))).astype(np.uint16)
+    near = spread ^ rng.integers(0, 4, spread.shape).astype(np.uint16)
+    counted = pgpu._checkpoints
+    monkeypatch.setattr(pgpu, "_checkpoints", lambda *a: walks.append(len(a[0])) or counted(*a))
+    monkeypatch.setattr(pgpu.HipPredictiveTensor, "_bins", lambda self, ref: (torch.zeros(1, dtype=torch.int32), 0))
+    monkeypatch.setattr(torch.cuda, "device", lambda device: contextlib.nullcontext())
+    monkeypatch.setattr(torch.cuda, "synchronize", lambda device: None)
+    for target, as_planes in ((spread, False), (weight_like(rng, 512, 1024), True)):
+        frame = predictive.encode(target, near)
+        streams = 1 if frame[5] == 0 else 2
+        walks.clear()
+        t = pgpu.HipPredictiveTensor(frame, near, device="cpu")
+        assert (t._planes is not None) == as_planes and len(walks) <= streams, (as_planes, walks)
