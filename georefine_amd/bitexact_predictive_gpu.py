@@ -423,6 +423,12 @@ class HipPredictiveTensor:
         total += sum(rows.numel() * 4 + classes.numel() for _, rows, classes, _ in self._tilings.values())
         return int(total)
 
+    @property
+    def host_bytes(self):
+        """What a tensor that is held as planes keeps in host memory for its walk's arrays, should they be asked for: half a byte a weight, the
+        contexts that its words were coded in (the device had them where the frame was walked), and the frame's tables."""
+        return sum(len(value) for value in self._kept.values()) if self._planes is not None else 0
+
     def _prepare_fused(self):
         """Upload the walker's derived arrays: segment index, per-label tables, store tiling."""
         import torch

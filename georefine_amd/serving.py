@@ -657,7 +657,7 @@ def load_bctx_model(package, *, model_factory, device="cuda:0", dtype=torch.bflo
     def residency(context):
         """What the device holds of a coded tensor, where the backend says so: the frame's mode,
         the mode of the resident form (a frame whose conditional residual stream was re-packed
-        into 6-bit fields at load is resident in mode 0), and whether the fused kernels take it."""
+        into 6-bit fields at load is resident in mode 0), and whether the fused kernels take it; and what the host keeps of it."""
         native = getattr(context, "row_major", None) or getattr(context, "native", context)
         if not hasattr(native, "resident_mode"):
             return {}
@@ -665,7 +665,8 @@ def load_bctx_model(package, *, model_factory, device="cuda:0", dtype=torch.bflo
         reason = getattr(native, "fused_reason", "")
         return dict(frame_mode=native.mode, resident_mode=native.resident_mode,
                     residual_repacked=native.resident_mode != native.mode, fused=fused,
-                    **({} if fused else {"fused_reason": reason}))
+                    **({} if fused else {"fused_reason": reason}),
+                    **({"host_bytes": native.host_bytes} if getattr(native, "host_bytes", 0) else {}))
 
     consumed, replacements = {}, {}
     for module_name, module, weight_name in coded:

@@ -131,3 +131,5 @@ def test_a_predictive_frame_is_decoded_once_whatever_it_is_held_as(monkeypatch):
         walks.clear()
         t = pgpu.HipPredictiveTensor(frame, near, device="cpu")
         assert (t._planes is not None) == as_planes and len(walks) <= streams, (as_planes, walks)
+        # bytes of the host's that a tensor keeps, for as long as it lives
+        assert t.host_bytes == (near.size // 2 + len(t._kept["meta"]) + len(t._kept["table"]) if as_planes else 0)
