@@ -380,13 +380,24 @@ def run_attention(args, as_dict=False):
 PPCX_BATCHES = (1, 96)
 
 
+def predictive_product(t, m):
+    """Bytes that one product of ``m`` rows has to touch once, and the kernels it runs: everything that the tensor keeps on the device
+    for products (its planes; or, where it is walked, the coded target, its index and tables and the 4-bit contexts of the reference),
+    activations, outputs."""
+    rows, cols = t.shape
+    io = m * (rows + cols) * 2
+    if t._planes is not None:
+        return t._planes.nbytes + io, kernel_name(False, m, False, True)
+    return t.resident_bytes + io, ("grf::fused_wave_kernel<PpcxWalk, 1, SCAN>" if m == 1 else
+                                   "pack_activations_kernel + grf::fused_gemm_kernel / fused_gemm_wide_kernel<PpcxWalk, MT, SCAN> (+ gemm_sum_parts_kernel)")
+
+
 def run_predictive(args, as_dict=False):
     """A 5120 x 17408 target coded (PPCX) against a reference that is the target plus N(0, 0.002)
-    noise, as a loaded model serves it: the tensor keeps the 4-bit context plane of its
-    reference from load on, so no reference is resident or decoded.  One step = the product of
-    the coded target with the activation rows, on three resident copies in turn: one row (the
-    fused GEMV) and 96 rows = 16 users x (5 draft tokens + 1), the verify shape (activations
-    packed, then the fused GEMM); --batch picks a single row count."""
+    noise, as a loaded model serves it: the tensor keeps its words as planes from load on, so
+    no reference is resident or decoded.  One step = the product of
+    the coded target with the activation rows, on three resident copies in turn: one row
+    and 96 rows = 16 users x (5 draft tokens + 1), the verify shape; --batch picks a single row count."""
     import torch
     from georefine_amd import bitexact_predictive_codec as ppcx
     from georefine_amd.bitexact_predictive_gpu import HipPredictiveTensor
@@ -402,11 +413,13 @@ def run_predictive(args, as_dict=False):
     t0 = time.perf_counter()
     frame = ppcx.encode(target, ref)
     t = HipPredictiveTensor(frame, ref, stride=1024, device="cuda:0")
-    if t.fused is None:
+    if not t.fusable:
         sys.exit(f"bench.py: the frame is not eligible for the fused kernels: {t.fused_reason}")
+    planes = t._planes is not None
     log(f"PPCX frame {len(frame)} B ({8 * len(frame) / target.size:.3f} bit/weight) mode {t.mode}; setup {time.perf_counter() - t0:.1f}s; "
-        f"rows per label {np.bincount(t.buffers['labels'].cpu().numpy(), minlength=16).tolist()}; GEMV tiling "
-        f"{t._tiling_for('waves')[3]}; GEMM tiling {t._tiling_for('gemm')[3]}")
+        + (f"held as planes, {t._planes.splits} splits" if planes else
+           f"rows per label {np.bincount(t.buffers['labels'].cpu().numpy(), minlength=16).tolist()}; GEMV tiling "
+           f"{t._tiling_for('waves')[3]}; GEMM tiling {t._tiling_for('gemm')[3]}"))
     copies = [t, t.clone(), t.clone()]  # three targets in rotation: more bytes than the caches hold
     steps, warmup = (args.steps, args.warmup) if not as_dict else (max(10, args.steps // 2), max(4, args.warmup // 4))
     x_all = torch.from_numpy(bf16_words(np.random.default_rng(7).normal(0, 1, size=(max(batches), cols)))).view(torch.bfloat16).cuda()
@@ -425,11 +438,7 @@ def run_predictive(args, as_dict=False):
         per_layer = [[("product", ["target"], lambda c=c: c.linear(None, x))] for c in copies]
         ms_step, per_ms, launch, timing, clocks = time_launches(
             torch, per_layer, steps, warmup, args.graph, lambda: ["target"] if any(c.error.item() for c in copies) else [])
-        # bytes one product has to touch once: everything the tensor keeps on the device (the coded
-        # target, its index and tables, the 4-bit context plane of the reference), activations, outputs
-        alg = coded + m * cols * 2 + m * rows * 2
-        kernel = ("grf::fused_wave_kernel<PpcxWalk, 1, SCAN>" if m == 1 else
-                  "pack_activations_kernel + grf::fused_gemm_kernel / fused_gemm_wide_kernel<PpcxWalk, MT, SCAN> (+ gemm_sum_parts_kernel)")
+        alg, kernel = predictive_product(t, m)
         traffic, source = recorded_traffic(False, m, kernel, prefix="ppcx")
         out[str(m)] = {"ms_per_product": round(ms_step, 4), "launch": launch, "per_kernel_timing": timing, **clocks,
                        "GBps": round(alg / (ms_step * 1e-3) / 1e9, 2), "rows_per_s": round(m / (ms_step * 1e-3), 1),
@@ -440,12 +449,13 @@ def run_predictive(args, as_dict=False):
         calibration_copy(torch)
     n = target.size
     result = {
-        "config": {"workload": "PPCX target 5120x17408 coded against a reference (target + N(0, 0.002)), products as "
-                               "served: contexts of the reference resident as a 4-bit plane, no dense reference; three "
-                               "resident copies in turn", "batches": list(batches), "steps": steps, "warmup": warmup},
+        "config": {"workload": "PPCX target 5120x17408 coded against a reference (target + N(0, 0.002)), products as served: "
+                               + ("resident as planes, no reference" if planes else
+                                  "contexts of the reference resident as a 4-bit plane, no dense reference")
+                               + "; three resident copies in turn", "batches": list(batches), "steps": steps, "warmup": warmup},
         "frame_bytes": len(frame), "frame_bits_per_weight": round(8 * len(frame) / n, 3),
         "resident_bytes": coded, "resident_bits_per_weight": round(8 * coded / n, 3),
-        "context_plane_bytes": n // 2, "frame_mode": t.mode, "resident_mode": t.resident_mode,
+        "context_plane_bytes": 0 if planes else n // 2, "host_bytes": t.host_bytes, "frame_mode": t.mode, "resident_mode": t.resident_mode,
         "batch": out,
     }
     copies.clear()

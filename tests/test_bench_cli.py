@@ -3,6 +3,7 @@ need no device."""
 import json
 import subprocess
 import sys
+import types
 from pathlib import Path
 
 import pytest
@@ -41,3 +42,20 @@ def test_kernels_it_names_are_the_ones_that_were_profiled(profile, decode_only, 
     assert name.split(", MT")[0].rstrip(">") in (ROOT / "profiles" / f"{profile}.txt").read_text()
     record = json.loads((ROOT / "profiles" / f"{profile}_traffic.json").read_text())
     assert name.split("<")[0].split("::")[-1] in record["traffic_bytes_per_launch"]
+
+
+class _Held:
+    """A predictive tensor that is held as planes, of which nothing of the walk may be asked."""
+    shape, fusable, host_bytes = (5120, 17408), True, 7
+    _planes = types.SimpleNamespace(nbytes=128000000, splits=12)
+    resident_bytes = 128000004
+
+    def __getattr__(self, name):
+        raise AssertionError(f"{name} was asked for")
+
+
+def test_predictive_products_are_counted_in_the_form_they_are_held_in():
+    sys.path.insert(0, str(ROOT))
+    import bench
+    for m, kernel in ((1, "planes_product_kernel"), (96, "planes_batch_kernel")):
+        assert bench.predictive_product(_Held(), m) == (128000000 + m * 2 * (5120 + 17408), kernel)
