@@ -43,6 +43,14 @@ def walked(monkeypatch):
     monkeypatch.setattr(_planes, "FROM_WEIGHTS", 1 << 40)
 
 
+@pytest.fixture(params=["planes", "walked"])
+def form(request):
+    """The large matrices of a test as planes, the form that they are served in, and then as frames that are walked."""
+    if request.param == "walked":
+        request.getfixturevalue("walked")
+    return request.param
+
+
 @pytest.fixture(scope="session")
 def oracle():
     from oracle import codec_oracle

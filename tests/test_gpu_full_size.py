@@ -2,7 +2,7 @@
 need a CPU decode of the same size: the digest of the decoded words against the digest the
 frame carries, rows of a product that must not depend on the batch, and agreement with a
 dense matmul of the decoded weights on the same device (tolerance 1e-2 relative, the bar for
-the fused products; decode itself is bit-exact)."""
+the fused products; decode itself is bit-exact), in both forms that a matrix is held in."""
 import hashlib
 
 import numpy as np
@@ -44,7 +44,7 @@ def _check_products(t, x, batches, fn):
         assert torch.equal(ym.view(torch.uint16), full[:m].view(torch.uint16)), f"rows differ between M={m} and M={len(x)}"
 
 
-def test_square_4096_gaussian_matrix(oracle):
+def test_square_4096_gaussian_matrix(oracle, form):
     """One 4096 x 4096 matrix, N(0, 0.02), activation N(0, 1): the CPU-runnable configuration,
     so here the CPU oracle and a float64 product are compared directly."""
     import torch
@@ -53,7 +53,7 @@ def test_square_4096_gaussian_matrix(oracle):
     xw = bf16_words(rng.normal(0.0, 1.0, size=(1, 4096)).astype(np.float32))
     frame, t = _tensor(words)
     assert np.array_equal(oracle.bctx_decode(frame), words)
-    assert t.fused is not None, t.fused_reason
+    assert t.fusable and (t._planes is not None) == (form == "planes"), t.fused_reason
     for general in (False, True):
         got = t.decode(check=True, general=general)
         assert np.array_equal(got.view(torch.uint16).cpu().numpy(), words)
@@ -66,14 +66,14 @@ def test_square_4096_gaussian_matrix(oracle):
 
 
 @pytest.mark.parametrize("index,shape", [(0, (17408, 5120)), (2, (5120, 17408))], ids=["gate", "down"])
-def test_mlp_matrices_decode_digest_and_gemv(index, shape):
+def test_mlp_matrices_decode_digest_and_gemv(index, shape, form):
     import torch
     words = weight_like(np.random.default_rng(1000 + index), *shape)
     frame, t = _tensor(words)
-    assert t.fused is not None, t.fused_reason
+    assert t.fusable and (t._planes is not None) == (form == "planes"), t.fused_reason
     want = hashlib.sha256(words.tobytes()).hexdigest()
     assert t.source_sha256 == want
-    assert _digest(t.decode(check=True)) == want              # fused store sink
+    assert _digest(t.decode(check=True)) == want              # planes, or the fused store sink
     assert _digest(t.decode(check=True, general=True)) == want  # one lane per checkpoint
     x = torch.from_numpy(bf16_words(np.random.default_rng(7).normal(0, 1, size=(8, shape[1])))).view(torch.bfloat16).cuda()
     _check_products(t, x, (1, 2, 3, 5, 8), lambda v: t.gemv(v, check=True))
@@ -88,17 +88,17 @@ def test_mlp_matrices_decode_digest_and_gemv(index, shape):
 
 
 @pytest.mark.parametrize("name,shape", [("q", (6144, 5120)), ("k", (1024, 5120)), ("o", (5120, 6144))])
-def test_attention_matrices_gemm_rows_do_not_depend_on_batch(name, shape):
+def test_attention_matrices_gemm_rows_do_not_depend_on_batch(name, shape, form):
     import torch
     words = weight_like(np.random.default_rng(2000 + len(name) + shape[0]), *shape)
     frame, t = _tensor(words)
-    assert t.fused is not None, t.fused_reason
+    assert t.fusable and (t._planes is not None) == (form == "planes"), t.fused_reason
     assert _digest(t.decode(check=True)) == hashlib.sha256(words.tobytes()).hexdigest()
     x = torch.from_numpy(bf16_words(np.random.default_rng(3).normal(0, 1, size=(128, shape[1])))).view(torch.bfloat16).cuda()
     _check_products(t, x, (1, 8, 32, 64, 128), lambda v: t.linear(v, check=True, batch_invariant=True))
 
 
-def test_whole_stack_resident_one_pass_at_batch_64():
+def test_whole_stack_resident_one_pass_at_batch_64(form):
     """64 layers x (q, k, v, o, gate, up, down) resident at once, one pass through every coded
     linear at batch 64.  One layer is encoded; the other 63 are device copies with buffers of
     their own, so the pass covers about 30 GB of coded weights in 256 launches (q/k/v share
@@ -120,7 +120,7 @@ def test_whole_stack_resident_one_pass_at_batch_64():
         frames = dict(pool.map(coded, enumerate(shapes.items())))
     # one segment length throughout, so that q/k/v and gate/up can share a launch
     first = {name: HipContextTensor(frames[name], stride=1024, device="cuda:0", fused_segment=64) for name in shapes}
-    assert all(t.fused is not None for t in first.values())
+    assert all(t.fusable and (t._planes is not None) == (form == "planes") for t in first.values())
     layers = [first] + [{name: t.clone() for name, t in first.items()} for _ in range(63)]
     dense_bytes = 64 * sum(2 * r * c for r, c in shapes.values())
     resident = sum(t.resident_bytes for layer in layers for t in layer.values())
@@ -158,7 +158,7 @@ def test_whole_stack_resident_one_pass_at_batch_64():
     assert _digest(keep.decode(check=True)) == want
 
 
-def test_vocabulary_sized_matrix_decode_products_and_row_lookup():
+def test_vocabulary_sized_matrix_decode_products_and_row_lookup(form):
     """248320 x 5120 (the head and embedding of the 27B model, 1.27 G weights, close to the
     frame format's 2^32 - 1 elements): element and byte offsets beyond 2^31, 19.9 M segments."""
     import torch
@@ -172,7 +172,7 @@ def test_vocabulary_sized_matrix_decode_products_and_row_lookup():
         words = np.concatenate(list(pool.map(chunk, range(rows // step))))
     assert words.shape == (rows, cols)
     frame, t = _tensor(words)
-    assert t.fused is not None, t.fused_reason
+    assert t.fusable and (t._planes is not None) == (form == "planes"), t.fused_reason
     want = hashlib.sha256(words.tobytes()).hexdigest()
     assert t.source_sha256 == want and len(frame) > 1 << 30
     assert _digest(t.decode(check=True)) == want
@@ -184,7 +184,7 @@ def test_vocabulary_sized_matrix_decode_products_and_row_lookup():
     assert np.array_equal(got, words[ids.numpy()])
 
 
-def test_predictive_frame_full_size_decode_and_batch_96():
+def test_predictive_frame_full_size_decode_and_batch_96(form):
     """A 5120 x 17408 target coded against a near-identical reference; the product takes
     16 users x (5 speculative + 1) = 96 rows."""
     import torch
@@ -196,6 +196,7 @@ def test_predictive_frame_full_size_decode_and_batch_96():
     frame = ppcx.encode(target, ref)
     native = serving.hip_predictive_factory(frame, ref, stride=1024, device="cuda:0")
     want = hashlib.sha256(target.tobytes()).hexdigest()
+    assert (native._planes is not None) == (form == "planes")
     assert native.source_sha256 == want and native.shape == target.shape
     ref_dev = torch.from_numpy(ref).view(torch.bfloat16).cuda()
     assert _digest(native.decode(ref_dev, check=True)) == want

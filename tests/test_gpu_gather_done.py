@@ -9,14 +9,6 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-@pytest.fixture(params=["walked", "planes"])
-def form(request):
-    """The tensors of a test as frames, then as planes."""
-    if request.param == "walked":
-        request.getfixturevalue("walked")
-    return request.param
-
-
 def _tensor(rows=300, cols=64 * 30, seed=3, **options):
     from georefine_amd import bitexact_context_codec as codec
     from georefine_amd.bitexact_context_gpu import HipContextTensor

@@ -63,7 +63,7 @@ def test_head_loads_from_frames_and_every_matrix_multiplies_fused(tmp_path):
     rng = np.random.default_rng(9)
     for name, path in MTP_LINEAR_PATHS.items():
         module = mtp.get_submodule(path)
-        assert isinstance(module, BCTXLinear) and module.tensor.fused is not None, (name, module.tensor.fused_reason)
+        assert isinstance(module, BCTXLinear) and module.tensor.fusable, (name, module.tensor.fused_reason)
         k = MTP_SHAPES[name][1]
         x = torch.from_numpy(bf16_words(rng.normal(0, 1, size=(5, k)))).view(torch.bfloat16).cuda()
         w = module.tensor.decode(check=True).float()
@@ -71,7 +71,7 @@ def test_head_loads_from_frames_and_every_matrix_multiplies_fused(tmp_path):
             assert np.array_equal(module.tensor.decode().view(torch.uint16).cpu().numpy(), source[name])
         ref = torch.nn.functional.linear(x.float(), w)
         scale = torch.nn.functional.linear(x.float().abs(), w.abs())
-        for rows in (1, 5):  # one row: the GEMV; five: the matrix-core kernel
+        for rows in (1, 5):
             y = module(x[:rows])
             assert y.shape == (rows, MTP_SHAPES[name][0]) and y.dtype == torch.bfloat16
             assert bool((y.float() - ref[:rows]).abs().le(1e-2 * ref[:rows].abs().clamp_min(1e-3 * scale[:rows])).all()), name
