@@ -574,15 +574,19 @@ size_t partial_bytes(const grf_planes &p, uint32_t m) { return m > kOwnAlways &&
 // Workgroups that share the splits of a row block where few rows of x meet a matrix alone.  Whole row blocks fall unevenly on the units:
 // of 320 blocks some have two and most one, and the last of 5120 x 17408 ends after 136 visits where 85 are a unit's share (256
 // blocks of these 23 us, 320 36).  Four workgroups of three splits a block leave the busiest 90 and cost a launch that adds the sums: us,
-// one row and six of 5120 x 17408 35.6 and 37.3, in parts 33.2 and 33.9; of 4200 x 17408 32.2 35.2, 31.9 32.4.  It is
-// left where less than 40 visits are saved (6144 x 17408, 28: 35.3 and 36.9; 5120 x 6144, 16: 15.8 and 16.1; 9000 x 9728, 18: 34.1 and 33.3).
-constexpr uint64_t kSaved = 40;
-
-uint32_t own_parts(const grf_planes &p) {
+// one row and six of 5120 x 17408 35.8 37.0, in parts 33.9 33.7; of 4200 x 17408 32.9 35.2, 32.6 32.5.  Of fewer blocks than units each has
+// one, and wide matrices end sooner in parts because a block's visits are shared out: 512 x 32768 24.6 27.9, 21.2 22.0.
+// It pays from a number of visits saved on: 40 where blocks are more than units (5120 x 14336, 45: 30.2 31.7, 29.0 29.6; 6144 x 17408, 28: 35.3 whole,
+// 36.9 in parts).  Else 50 (48: 1600 x 24576 21.4 24.2, 23.0 22.5; 50: 1024 x 17408 16.8 18.5, 17.1 17.6; 55: 512 x 17408 16.5 18.0, 16.0 16.7;
+// 40: 512 x 12800 11.7 12.0, 13.0 13.6; 1600 x 17408 17.4 19.2, 19.3 19.5), and for more than eight rows, whose visits are
+// longer, 44 (16 rows: 40: 512 x 12800 13.0, 14.3; 44: 400 x 14336 14.4, 14.3; 50: 1024 x 17408 23.0, 18.6), or 40 of more
+// than 32 blocks (720 x 12800 17.2, 15.5; 1600 x 17408 23.5, 20.3).
+uint32_t own_parts(const grf_planes &p, uint32_t m) {
   const uint64_t blocks = (p.rows + 15) / 16, visits = grf::PlanesShape(p.cols).visits(), each = (visits + p.splits - 1) / p.splits;
+  const uint64_t saved = blocks > kUnits || (m > 8 && blocks > 32) ? 40 : m > 8 ? 44 : 50;
   uint32_t best = 1;
   uint64_t least = (blocks + kUnits - 1) / kUnits * each * p.splits;
-  least = least > kSaved ? least - kSaved + 1 : 0;  // to be below
+  least = least > saved ? least - saved + 1 : 0;  // to be below
   for (uint32_t waves = p.splits - 1; waves >= 3; --waves) {
     const uint64_t parts = (p.splits + waves - 1) / waves, busiest = (blocks * parts + kUnits - 1) / kUnits * waves * each;
     if (busiest < least) least = busiest, best = (uint32_t)parts;
@@ -621,7 +625,7 @@ int product(const char *who, uint32_t n, const grf_planes *const *planes, const 
     const bool batch = m > kOwnRows || (m > kOwnAlways && visits >= kOwnVisits) || (m > 16 && waves * Product<4>::kWaveBytes > kLdsBytes);
     // (rows that need no workspace use one that is there and aligned)
     const bool room = workspace && !((uintptr_t)workspace & 15) && workspace_bytes >= sums_bytes(*planes[0], m);
-    const uint32_t parts = batch || n > 1 || !room ? 1 : own_parts(*planes[0]);
+    const uint32_t parts = batch || n > 1 || !room ? 1 : own_parts(*planes[0], m);
     // (fifteen or sixteen waves with two eights of rows do not fit in a unit's LDS; eight have the splits two each)
     const uint32_t own_waves = parts > 1 ? (planes[0]->splits + parts - 1) / parts
                                : waves * Product<2>::kWaveBytes > kLdsBytes && (m > 8 || packed) ? 8 : waves;
@@ -942,7 +946,7 @@ size_t grf_planes_workspace_bytes(uint32_t n, const grf_planes *const *planes, u
   for (uint32_t i = 0; planes && i < n; ++i)
     if (check_planes("grf_planes_workspace_bytes", planes[i]) == GRF_OK) {  // (what a launch refuses needs none)
       const uint32_t m = std::min(m_rows, kMaxTileRows);
-      bytes += n == 1 && own_parts(*planes[i]) > 1 ? sums_bytes(*planes[i], m) : partial_bytes(*planes[i], m);
+      bytes += n == 1 && own_parts(*planes[i], m) > 1 ? sums_bytes(*planes[i], m) : partial_bytes(*planes[i], m);
     }
   return bytes;
 }

@@ -46,6 +46,16 @@ def test_a_workspace_is_asked_for_what_a_launch_takes_and_nothing_else(change):
     assert lib.grf_planes_workspace_bytes(2, None, 6) == 0
 
 
+@pytest.mark.parametrize("rows,cols,shared", [(256, 12800, 0), (512, 12800, 0), (512, 14336, 0), (1300, 17408, 0), (1600, 17408, 0), (2400, 32768, 0),
+                                              (6144, 17408, 0), (1024, 5120, 0), (512, 17408, 1), (1024, 24576, 1), (256, 32768, 1), (2048, 32768, 1),
+                                              (4200, 17408, 1), (5120, 14336, 1), (5120, 17408, 1)])
+def test_row_blocks_are_shared_where_that_was_measured_to_pay(rows, cols, shared):
+    """One row of x: a workspace is asked for only where workgroups share row blocks (of the sizes beside own_parts)."""
+    p = _hip_abi.GrfPlanes(planes=4096, bases=4096, listed_at=4096, listed=4096, rows=rows, cols=cols, splits=_planes.sum_splits(rows, cols))
+    size = _native.hip().grf_planes_workspace_bytes(1, (ctypes.c_void_p * 1)(ctypes.addressof(p)), 1)
+    assert (size > 0) == bool(shared)
+
+
 def test_small_sparse_and_odd_frames_stay_frames():
     rng = np.random.default_rng(3)
     large = codec.encode(weight_like(rng, 512, 1024))
