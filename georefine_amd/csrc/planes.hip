@@ -30,10 +30,14 @@ using grf::wave_order;
 constexpr uint32_t kMaxMembers = 4;
 constexpr uint32_t kMaxTileRows = 128;  // activation rows of a launch
 // Rows of x up to which every wave brings its own: it needs no other wave and no second launch, but reads x once a row block where
-// four waves share it once in eight.  us, own and shared: one row 17408 x 5120 twice 52 and 57, 16 rows 65 and 58; 16 rows of 6144,
-// 1024 and 1024 x 5120 18 and 24, 32 rows 23 and 27; 32 rows of 5120 x 17408 64 and 39.
+// four waves share it once in eight.  us of launches in a row, own and shared, 16 and 32 rows: 1024 x 5120 8.4 13.4, 10.2 14.8; 4096 x 4096
+// 9.8 15.6, 11.8 17.3; 8192 x 4096 14.4 19.5, 17.8 20.9; 5120 x 5120 16.4 18.7, 21.8 20.4; 10240 x 5120 22.9 26.1, 30.1 28.4; one row of
+// 17408 x 5120 twice 52 57, 16 rows 65 58.  The line by visits is coarse: 16 rows of 4608 x 14336 37.0 30.9, 32 rows of 6144 x 6144 24.9 23.5.
 constexpr uint32_t kOwnAlways = 8;                    // up to which it always does
 constexpr uint32_t kOwnRows = 32, kOwnVisits = 16384;  // and, in launches of fewer visits than that
+// More than sixteen rows take 16 KiB of LDS a wave, so that six waves are alone on a unit; where more such workgroups come than there are
+// units, and a wave has more than one visit, x is shared (32 rows, own and shared: 4112 x 3072 16.2 16.1, 4112 x 5120 21.9 19.2, 5120 x
+// 6144 26.8 20.9, 5120 x 12288 46.7 29.8, 9000 x 6144 39.4 27.6, 11000 x 4096 29.7 26.4; of one visit 5120 x 1536 12.1 13.6).
 constexpr uint32_t kPatch = 4096;       // LDS bytes in which a wave's half visit is completed
 
 struct PlanesMember {
@@ -616,13 +620,21 @@ int product(const char *who, uint32_t n, const grf_planes *const *planes, const 
     space += partial_bytes(*planes[i], most);
   }
   for (uint32_t i = 0; i < n; ++i) waves = std::max(waves, (planes[i]->splits + 1) / 2);  // the largest member's, and no wave more than two
+  uint32_t own_groups = 0, each = 0;  // workgroups of waves with their own x, and the most visits of a split
+  for (uint32_t i = 0; i < n; ++i) {
+    const uint32_t blocks = (planes[i]->rows + 15) / 16, blocks_each = std::max(1u, waves / planes[i]->splits);
+    own_groups += (blocks + blocks_each - 1) / blocks_each;
+    each = std::max(each, (grf::PlanesShape(cols).visits() + planes[i]->splits - 1) / planes[i]->splits);
+  }
   if (((uintptr_t)x & 15) || (!packed && (ldx < cols || ldx % 8 || ldx > 1u << 24)) || (packed && m_rows > kMaxTileRows))
     return grf::set_error(GRF_BAD_ARGUMENT, std::string(who) + ": activation rows are 16-byte aligned");
   if (space && (!workspace || workspace_bytes < space || ((uintptr_t)workspace & 15)))
     return grf::set_error(GRF_BAD_ARGUMENT, std::string(who) + ": workspace too small (grf_planes_workspace_bytes)");
   for (uint32_t done = 0; done < m_rows; done += kMaxTileRows) {
     const uint32_t m = std::min(kMaxTileRows, m_rows - done), m_pad = 16 * grf::gemm_tiles(m);
-    const bool batch = m > kOwnRows || (m > kOwnAlways && visits >= kOwnVisits) || (m > 16 && waves * Product<4>::kWaveBytes > kLdsBytes);
+    const bool alone = m > 16 && waves * Product<4>::kWaveBytes > kLdsBytes / 2;  // (a workgroup on its unit)
+    const bool batch = m > kOwnRows || (m > kOwnAlways && visits >= kOwnVisits) || (alone && own_groups > kUnits && each > 1) ||
+                       (m > 16 && waves * Product<4>::kWaveBytes > kLdsBytes);
     // (rows that need no workspace use one that is there and aligned)
     const bool room = workspace && !((uintptr_t)workspace & 15) && workspace_bytes >= sums_bytes(*planes[0], m);
     const uint32_t parts = batch || n > 1 || !room ? 1 : own_parts(*planes[0], m);

@@ -89,7 +89,8 @@ def test_products_against_float64_with_one_set_of_bits_a_row(rows, cols, splits)
         assert torch.equal(product(xp.buffer, m, packed=1), full[:m]), m
 
 
-@pytest.mark.parametrize("rows,cols", [(29968, 2320), (65555, 1040)])
+# (the last: blocks that are more than units, of waves that fill one: more than sixteen rows share x)
+@pytest.mark.parametrize("rows,cols", [(29968, 2320), (65555, 1040), (4112, 3328)])
 def test_rows_of_x_that_large_matrices_share_have_the_bits_of_single_ones(rows, cols):
     import torch
     from georefine_amd import _native
