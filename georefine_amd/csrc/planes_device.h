@@ -59,15 +59,11 @@ struct VisitBytes {
   __device__ __forceinline__ VisitBytes(const uint8_t *block, uint32_t full)
       : bytes(__builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(block), 0, (int)(full * kVisitBytes), 0x00020000)) {}
   __device__ __forceinline__ uint4v four(uint32_t at) const { return __builtin_bit_cast(uint4v, __builtin_amdgcn_raw_buffer_load_b128(bytes, at, 0, 0)); }
-  __device__ __forceinline__ uint2v two(uint32_t at) const { return __builtin_bit_cast(uint2v, __builtin_amdgcn_raw_buffer_load_b64(bytes, at, 0, 0)); }
-  __device__ __forceinline__ uint32_t one(uint32_t at) const { return __builtin_amdgcn_raw_buffer_load_b32(bytes, at, 0, 0); }
   __device__ __forceinline__ uint3v three(uint32_t at) const { return __builtin_bit_cast(uint3v, __builtin_amdgcn_raw_buffer_load_b96(bytes, at, 0, 0)); }
 #else
   __device__ VisitBytes(const uint8_t *, uint32_t) {}
   __device__ uint4v four(uint32_t) const { return {}; }
   __device__ uint3v three(uint32_t) const { return {}; }
-  __device__ uint2v two(uint32_t) const { return {}; }
-  __device__ uint32_t one(uint32_t) const { return {}; }
 #endif
 };
 
