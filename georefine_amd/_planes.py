@@ -19,9 +19,10 @@ VISIT, UNIT, VISIT_BYTES, UNIT_BYTES = 256, 64, 5888, 1536  # csrc/word_planes.h
 EXPONENTS = 11
 MAX_COLS = 1 << 17
 OWN_ROWS = 8  # activation rows up to which a launch needs no workspace (a matrix alone is given one where it pays)
-# Weights from which a matrix is laid out: where a call of its own stops gaining.  Below, it is as long as its host path either way (502 x
-# 640 at three rows 10.1 us, walked 10.5); the kernels are shorter there too for few rows (one row of 512 x 640 4.4 us, walked
-# 8.4; 32 rows 8.6 and 8.2), which only captured launches of small matrices would gain.
+# Weights from which a matrix is laid out.  Smaller ones have shorter kernels as planes too for up to 32 rows and for more than 128 (us of
+# launches in a row, walked and as planes: 256 x 512 one row 6.6 3.8, 32 rows 6.9 4.5, 200 13.5 11.4; 511 x 1024 8.1 4.1, 9.3 4.9, 15.7 14.0; a call
+# by itself 9.0 8.0), but longer ones between (64 and 128 rows of 256 x 512 8.0 10.2, 11.1 13.9; of 300 x 1744 10.8 13.5, 14.5 19.1; of
+# 511 x 1024 12.4 10.9, 13.7 14.9).
 FROM_WEIGHTS = 1 << 19
 # How much more memory than the frame's arrays the planes may take (frames of few exponents code far below 11.5 bits
 # and stay frames).

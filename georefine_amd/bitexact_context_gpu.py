@@ -1163,7 +1163,8 @@ class HipLinearGroup:
         self.error = torch.zeros((), device=self.device, dtype=torch.int32)
         self._tilings, self._pointer_arrays, self._workspace = {}, {}, {}
         # Members whose frames are walked, beside others that are held as planes, have a launch of their own: laid out for the planes' launch
-        # they would lose the bits of their own products, which the vector-ALU route gives every member.
+        # they would lose the bits of their own products, which the vector-ALU route gives every member.  (Small matrices are walked: one row of
+        # 2048 and 256 x 1024 takes 15.8 us in two launches, where one of planes would take 4.4.)
         self._walked = None  # (their places, their group)
         rest = [i for i, t in enumerate(self.tensors) if t._planes is None]
         if len(rest) == len(self.tensors):
