@@ -88,12 +88,14 @@ GEMV_UP_TO = 2  # rows linear() gives to the vector-ALU kernel; read from HipCon
 
 def algorithmic_bytes(t, m, gemm=None):
     """Bytes one fused GEMV / GEMM launch has to touch once: the planes of a matrix held as such, or both streams, the
-    fused index, the per-class lookup tables and labels; activations and outputs.  ``gemm``: the launch runs
+    fused index, the per-class lookup tables and labels; activations and outputs.  ``frame``: with the frame's own bytes in the place
+    of what the matrix is resident as.  ``gemm``: the launch runs
     the matrix-core kernel (default: from the row count, as linear() routes)."""
     rows, cols = t.shape
+    io = m * (rows + cols) * 2
     if t._planes is not None:  # what the matrix is resident as: its planes and the listed words
         held = t._planes.nbytes
-        return dict(total=held + m * (rows + cols) * 2, payload=held, index=0, tables=0)
+        return dict(total=held + io, payload=held, index=0, tables=0, frame=t.frame_bytes + io)
     b = t.buffers
     n = lambda k: b[k].numel() * b[k].element_size()
     # (the resident residual array starts every row class on a multiple of 16 rows: the rows it
@@ -106,8 +108,12 @@ def algorithmic_bytes(t, m, gemm=None):
              + tile_class.numel() * tile_class.element_size() + (n("row_pos") if "row_pos" in b else 0))
     tables = n("fused_lut") + n("fused_tab")
     labels = cols
-    io = m * cols * 2 + m * rows * 2
-    return dict(total=payload + index + tables + labels + io, payload=payload, index=index, tables=tables)
+    return dict(total=payload + index + tables + labels + io, payload=payload, index=index, tables=tables, frame=t.frame_bytes + io)
+
+
+def dtype_text(planes):
+    """What the words are made of, and what they are multiplied in."""
+    return ("bf16 weights as planes (11.5 bits)" if planes else "u32 rANS state / bf16 weights") + " / fp32 accumulate"
 
 
 def host_description():
@@ -300,6 +306,7 @@ def run_attention(args, as_dict=False):
                                       fused_segment=64)
         if base[name]._planes is None and base[name].fused is None:
             sys.exit(f"bench.py: {name} is not eligible for the fused kernels: {base[name].fused_reason}")
+    planes = all(t._planes is not None for t in base.values())
     resident = sum(t.resident_bytes for t in base.values())
     copies = max(1, -(-2 * LAST_LEVEL_CACHE_BYTES // resident))
     sets = [base] + [{k: v.clone() for k, v in base.items()} for _ in range(copies - 1)]
@@ -319,20 +326,21 @@ def run_attention(args, as_dict=False):
                 for s_, g in zip(sets, groups)]
 
     def alg_of(m, gemm):
-        parts = {n_: algorithmic_bytes(base[n_], m, gemm=gemm)["total"] for n_ in ATTENTION}
-        return {"q+k+v": parts["q"] + parts["k"] + parts["v"] - 2 * m * 5120 * 2, "o": parts["o"]}
+        parts = {n_: algorithmic_bytes(base[n_], m, gemm=gemm) for n_ in ATTENTION}
+        return [{"q+k+v": parts["q"][of] + parts["k"][of] + parts["v"][of] - 2 * m * 5120 * 2, "o": parts["o"][of]}
+                for of in ("total", "frame")]
 
     def one(m, invariant):
         ms_step, per_ms, launch, timing, clocks = time_launches(torch, per_layer(m, invariant), steps, warmup,
                                                                 args.graph, errors)
-        alg = alg_of(m, invariant or m > GEMV_UP_TO)
+        alg, frames = alg_of(m, invariant or m > GEMV_UP_TO)
         dom = max(alg, key=lambda k: alg[k])
         gemm = invariant or m > GEMV_UP_TO
-        planes = all(t._planes is not None for t in base.values())
         kernel = (kernel_name(False, m, True, True) if planes else f"grf::fused_gemm_group_kernel / fused_gemm_wide_group_kernel<{WALK}, MT, 1>" if gemm
                   else kernel_name(False, m, True))
         total = sum(alg.values())
-        return {"ms_per_pass": round(ms_step, 4), "GBps": round(total / (ms_step * 1e-3) / 1e9, 2), "launch": launch,
+        return {"ms_per_pass": round(ms_step, 4), "GBps": round(total / (ms_step * 1e-3) / 1e9, 2),
+                "coded_frames_GBps": round(sum(frames.values()) / (ms_step * 1e-3) / 1e9, 2), "launch": launch,
                 "rows_per_s": round(m / (ms_step * 1e-3), 1), **clocks,
                 "per_kernel": {k: launch_fields(alg[k], per_ms[k]) for k in per_ms},
                 "roofline": roofline_fields(alg[dom], per_ms[dom], f"{kernel} on {dom}")}, timing
@@ -374,7 +382,7 @@ def run_attention(args, as_dict=False):
     print(json.dumps({"metric": "compressed-weight decode-GEMV GB/s", "value": batches["1"]["GBps"], "unit": "GB/s",
                       "n_gpus": 1, "steps": steps, "warmup": warmup, "ms_per_step": batches["1"]["ms_per_pass"],
                       "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
-                      "dtype": "u32 rANS state / bf16 weights / fp32 accumulate", "data": "synthetic", **result}), flush=True)
+                      "dtype": dtype_text(planes), "data": "synthetic", **result}), flush=True)
 
 
 PPCX_BATCHES = (1, 96)
@@ -441,7 +449,9 @@ def run_predictive(args, as_dict=False):
         alg, kernel = predictive_product(t, m)
         traffic, source = recorded_traffic(False, m, kernel, prefix="ppcx")
         out[str(m)] = {"ms_per_product": round(ms_step, 4), "launch": launch, "per_kernel_timing": timing, **clocks,
-                       "GBps": round(alg / (ms_step * 1e-3) / 1e9, 2), "rows_per_s": round(m / (ms_step * 1e-3), 1),
+                       "GBps": round(alg / (ms_step * 1e-3) / 1e9, 2),
+                       "coded_frames_GBps": round((len(frame) + m * (rows + cols) * 2) / (ms_step * 1e-3) / 1e9, 2),
+                       "rows_per_s": round(m / (ms_step * 1e-3), 1),
                        "algorithmic_bytes_per_product": alg,
                        "roofline": roofline_fields(alg, per_ms["product"], kernel + " (all launches of a product)", traffic, source)}
         log(f"ppcx batch {m}: {ms_step:.4f} ms per product")
@@ -466,7 +476,7 @@ def run_predictive(args, as_dict=False):
     first = out[str(batches[-1])]
     print(json.dumps({"metric": "compressed-weight decode-GEMV GB/s", "value": first["GBps"], "unit": "GB/s", "n_gpus": 1,
                       "steps": steps, "warmup": warmup, "ms_per_step": first["ms_per_product"], "higher_is_better": True,
-                      "scaling": "weak", "vs_baseline": None, "dtype": "u32 rANS state / bf16 weights / fp32 accumulate",
+                      "scaling": "weak", "vs_baseline": None, "dtype": dtype_text(planes),
                       "data": "synthetic", **result, "roofline": first["roofline"]}), flush=True)
 
 
@@ -647,31 +657,36 @@ def run_stack(args, as_dict=False, prep=None):
         torch, [launches], args.steps, args.warmup, args.graph,
         lambda: sorted({label for label, members, _ in launches for t in members if t.error.item()}))
     alg, count = {}, {}
+    planes, frame_step = all(t._planes is not None for t in everything), 0
     for label, members, _ in launches:
         if label == "embedding":  # the rows gathered: their share of both streams, written dense
             t = vocab["embedding"]
             total = int(m * (algorithmic_bytes(t, 0, gemm=False)["payload"] / t.shape[0] + 2 * t.shape[1]))
+            frame_step += int(m * (t.frame_bytes / t.shape[0] + 2 * t.shape[1]))
         else:
-            total = sum(algorithmic_bytes(t, m, gemm=gemm)["total"] for t in members) - (len(members) - 1) * m * members[0].shape[1] * 2
+            parts, again = [algorithmic_bytes(t, m, gemm=gemm) for t in members], (len(members) - 1) * m * members[0].shape[1] * 2
+            total = sum(p_["total"] for p_ in parts) - again
+            frame_step += sum(p_["frame"] for p_ in parts) - again
         alg[label] = alg.get(label, 0) + total
         count[label] = count.get(label, 0) + 1
     step_bytes = sum(alg.values())
     value = step_bytes / (ms_per_step * 1e-3) / 1e9
     share = {label: per_ms[label] * count[label] for label in per_ms}  # ms of a pass spent in each kind of launch
     dom = max((l_ for l_ in alg if l_ != "embedding"), key=lambda l_: alg[l_])  # the kind that moves most bytes
-    kernel = kernel_name(False, max(m, GEMV_UP_TO + 1) if gemm else m, "+" in dom, all(t._planes is not None for t in everything))
+    kernel = kernel_name(False, max(m, GEMV_UP_TO + 1) if gemm else m, "+" in dom, planes)
     shapes_text = "; ".join(f"{k}: " + ", ".join(f"{n_} {c}->{r}" for n_, (r, c) in spec[k].items())
                             for k in ("attn", "gdn") if spec[k])
     result = {
         "metric": "compressed-weight decode-GEMV GB/s", "value": round(value, 2), "unit": "GB/s", "n_gpus": 1,
         "steps": args.steps, "warmup": args.warmup, "ms_per_step": round(ms_per_step, 4), "higher_is_better": True,
-        "scaling": "weak", "vs_baseline": None, "dtype": "u32 rANS state / bf16 weights / fp32 accumulate",
+        "scaling": "weak", "vs_baseline": None, "dtype": dtype_text(planes),
         "data": "synthetic",
         "config": {"workload": f"whole stack resident: {args.layers} layers ({prep.counts['attn']} attention, "
                                f"{prep.counts['gdn']} linear-attention; {shapes_text})"
                                + (f", embedding and head {spec['vocab'][0]}x{spec['vocab'][1]}" if vocab else "")
                                + f"; one pass through every coded linear at batch {m} (the embedding: a gather of "
-                                 f"{m} rows); {dense / 1e9:.1f} GB of dense BF16 held as {frame_bytes / 1e9:.1f} GB of frames",
+                                 f"{m} rows); {dense / 1e9:.1f} GB of dense BF16 in {frame_bytes / 1e9:.1f} GB of frames, "
+                                 f"{resident / 1e9:.1f} GB on the device" + (" as planes" if planes else ""),
                    "shapes": args.stack_shapes, "batch": m, "layers": args.layers,
                    "distinct_layers": dict(prep.distinct), "linears": len(everything), "launches_per_pass": len(launches),
                    "launch": launch, "launches": "siblings that take the same rows share a launch" if grouped else "one per linear",
@@ -680,6 +695,7 @@ def run_stack(args, as_dict=False, prep=None):
                                        "copy of the head's frame" if vocab else None},
         "dense_bf16_bytes": dense, "frame_bytes": frame_bytes, "resident_device_bytes": resident,
         "algorithmic_bytes_per_step": step_bytes,
+        "coded_frames_GBps": round(frame_step / (ms_per_step * 1e-3) / 1e9, 2),
         "effective_bf16_GBps": round(dense / (ms_per_step * 1e-3) / 1e9, 2),
         "tok_s_equiv": round(m / (ms_per_step * 1e-3), 1),
         "pct_hbm_roofline": round(100 * value / HBM_PEAK_GBPS, 2), **clocks,
@@ -716,6 +732,8 @@ def main():
                     help="time K eager steps; by default the K timed steps are replays of one captured HIP graph "
                          "of a step (per-kernel durations always come from K eager steps before it)")
     ap.add_argument("--only", default="", help="comma list of gate,up,down (profiling aid)")
+    ap.add_argument("--walked", action="store_true",
+                    help="matrices of every size stay frames whose states are walked, as small ones do (profiling aid)")
     ap.add_argument("--calibrate-copy", action="store_true",
                     help="also run a plain 128 MiB read + 128 MiB write elementwise kernel three times, so that a "
                          "counter profile of this command holds a kernel of known traffic to scale by")
@@ -743,6 +761,9 @@ def main():
         sys.exit("bench.py: this decode path runs on one GPU; --gpus must be 1 (no multi-GPU figure exists)")
     if args.workload == "mlp":
         args.batch = args.batch or 1  # the stack defaults to 64
+    if args.walked:
+        from georefine_amd import _planes
+        _planes.FROM_WEIGHTS = 1 << 40
     decode_only = args.workload == "decode"
     if decode_only:
         args.batch, args.no_groups = 0, True  # no activations: rows = 0 selects the store sink's tiling
@@ -848,10 +869,11 @@ def main():
         for label, members, _ in units:
             parts = [algorithmic_bytes(tensors[n_], m) for n_ in members]
             alg[label] = {k: sum(p_[k] for p_ in parts) for k in parts[0]}
-            if len(members) > 1:  # the members read one x
-                alg[label]["total"] -= (len(members) - 1) * m * SHAPES[members[0]][1] * 2
-            if decode_only:  # the dense matrix is written once
-                alg[label]["total"] += sum(2 * SHAPES[n_][0] * SHAPES[n_][1] for n_ in members)
+            for of in ("total", "frame"):
+                if len(members) > 1:  # the members read one x
+                    alg[label][of] -= (len(members) - 1) * m * SHAPES[members[0]][1] * 2
+                if decode_only:  # the dense matrix is written once
+                    alg[label][of] += sum(2 * SHAPES[n_][0] * SHAPES[n_][1] for n_ in members)
         step_bytes = sum(a_["total"] for a_ in alg.values())
         dense_bytes = sum(2 * SHAPES[n_][0] * SHAPES[n_][1] for n_ in names)
         value = step_bytes / (ms_per_step * 1e-3) / 1e9
@@ -871,6 +893,8 @@ def main():
                        "batch": m, "matrices": names, "launches": [u[0] for u in units],
                        "segment": None if planes else tensors[names[0]].fused_plan["seg_len"], "launch": launch, "per_kernel_timing": timing,
                        "layer_copies": n_layers, "residual_block_rows": None if planes else tensors[names[0]]._raw6_block},
+            # (of the frames' own bytes, in the place of what the matrices are resident as)
+            "coded_frames_GBps": round(sum(a_["frame"] for a_ in alg.values()) / (ms_per_step * 1e-3) / 1e9, 2),
             "effective_bf16_GBps": round(eff_bf16, 2),
             "tok_s_equiv": round(eff_bf16 * 1e9 / MODEL_BF16_BYTES * m, 3) if m else None,
             **clocks,
@@ -898,7 +922,7 @@ def main():
                   else "compressed-weight decode-GEMV GB/s",
         "value": fields.pop("value"), "unit": "GB/s", "n_gpus": 1, "steps": args.steps, "warmup": args.warmup,
         "ms_per_step": fields.pop("ms_per_step"), "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
-        "dtype": "u32 rANS state / bf16 weights / fp32 accumulate", "data": "synthetic",
+        "dtype": dtype_text(all(t._planes is not None for t in tensors.values())), "data": "synthetic",
     }
     result.update(fields)
     copy_rate = measured_copy_gbps(torch)
@@ -984,7 +1008,10 @@ def recorded_traffic(decode_only, m, kernel, prefix=None):
     record (bench.py cannot read hardware counters itself), and where the figure comes from.
     The record names the kernels it measured and the digest of the device sources it was taken
     with; for another kernel or other sources the figure is withheld (None) and the reason given."""
-    name = ((f"ppcx_gemv_m1_5120x17408_traffic.json" if m == 1 else f"ppcx_gemm_m{m}_5120x17408_traffic.json")
+    name = (f"planes_ppcx_m{m}_5120x17408_traffic.json" if kernel.startswith("planes") and prefix == "ppcx" else
+            "planes_decode_qwen27b_mlp_traffic.json" if kernel.startswith("planes") and decode_only else
+            f"planes_m{m}_gate_up_traffic.json" if kernel.startswith("planes") else
+            (f"ppcx_gemv_m1_5120x17408_traffic.json" if m == 1 else f"ppcx_gemm_m{m}_5120x17408_traffic.json")
             if prefix == "ppcx" else
             "fused_store_decode_qwen27b_mlp_traffic.json" if decode_only else
             "fused_gemv_m1_qwen27b_mlp_traffic.json" if m == 1 else
