@@ -1,8 +1,8 @@
 """Prompts and embedding lookups for a profiler (summarize.py):
 
-    python3 profiles/prompts.py {prompt,lookup} [--steps N] [--warmup N] [--calibrate-copy]
+    python3 profiles/prompts.py {prompt,lookup} [--steps N] [--warmup N] [--calibrate-copy] [--walked]
 
-``prompt``: 1000 activation rows of a coded 5120 x 17408 matrix: decode to dense, then the product.  ``lookup``: 777 rows of a
+``prompt``: 1000 activation rows of a coded 5120 x 17408 matrix (``--walked``: decode to dense, then the product).  ``lookup``: 777 rows of a
 coded 8192 x 5120 table.  Three device copies of the matrix in turn, eager calls.  Prints one line of JSON.
 """
 import argparse
@@ -15,7 +15,7 @@ import numpy as np
 import torch
 
 import bench
-from georefine_amd import bitexact_context_codec as codec
+from georefine_amd import _planes, bitexact_context_codec as codec
 from georefine_amd.bitexact_context_gpu import HipContextTensor
 
 SIZES = {"prompt": (5120, 17408, 1000), "lookup": (8192, 5120, 777)}
@@ -27,7 +27,10 @@ def main():
     ap.add_argument("--steps", type=int, default=200)
     ap.add_argument("--warmup", type=int, default=20)
     ap.add_argument("--calibrate-copy", action="store_true")
+    ap.add_argument("--walked", action="store_true", help="the matrix stays a frame")
     args = ap.parse_args()
+    if args.walked:
+        _planes.FROM_WEIGHTS = 1 << 40
     rows, cols, m = SIZES[args.what]
     g = torch.Generator(device="cuda").manual_seed(1)
     w = torch.randn(rows, cols, device="cuda", generator=g) * 0.02 * torch.exp(0.5 * torch.randn(rows, 1, device="cuda", generator=g))

@@ -13,7 +13,7 @@ What the derived lines say (MI355X: 8 XCDs, 256 compute units, 1024 SIMDs):
                          (SQ_ACTIVE_INST_LDS counts the issue of the instructions only, and says next to
                          nothing about the pipe), with the share SQ_LDS_BANK_CONFLICT of them
   matrix cores busy      SQ_VALU_MFMA_BUSY_CYCLES / (1024 cycles)
-  per wave step          totals / (weights / 64): a wave step is one symbol for each of a wave's 64 lanes
+  per wave step          totals / (weights / 64), of the walk: a wave step is one symbol for each of a wave's 64 lanes
 """
 import collections
 import csv
@@ -31,38 +31,64 @@ import bench  # noqa: E402
 
 MLP = "Qwen-27B-like MLP (gate, up: 17408x5120; down: 5120x17408), MI355X (gfx950)"
 MATRIX = 5120 * 17408
-# title, the program's options (the program first where it is not bench.py), {kernel: weights a launch walks}, what the traffic
+# title, the program's options (the program first where it is not bench.py), {kernel: weights a launch walks, or 0}, what the traffic
 # record is called
 WORKLOADS = {
+    "planes_m1_gate_up": (
+        "Product of planes, one row, gate and up (17408x5120 each) in one grouped launch, MI355X (gfx950)",
+        ["--only", "gate,up"], {"planes_product_kernel": 0}, "gate and up in one launch, batch 1"),
+    "planes_m64_gate_up": (
+        "Product of planes, 64 rows, gate and up (17408x5120 each) in one grouped launch, MI355X (gfx950)",
+        ["--batch", "64", "--only", "gate,up"], {"planes_batch_kernel": 0, "planes_sum_kernel": 0}, "gate and up in one launch, batch 64"),
+    "planes_decode_qwen27b_mlp": (
+        f"Planes to dense BF16 (decode()), {MLP}\none step = three launches",
+        ["--workload", "decode"], {"planes_decode_kernel": 0}, "Qwen-27B-like MLP decode"),
+    "planes_ppcx_m1_5120x17408": (
+        "Product of a predictive (PPCX) weight held as planes, 5120x17408, batch 1, MI355X (gfx950)",
+        ["--workload", "ppcx", "--batch", "1"], {"planes_product_kernel": 0, "planes_sum_kernel": 0}, "PPCX 5120x17408 batch 1"),
+    "planes_ppcx_m96_5120x17408": (
+        "Product of a predictive (PPCX) weight held as planes, 5120x17408, 96 rows, MI355X (gfx950)",
+        ["--workload", "ppcx", "--batch", "96"], {"planes_batch_kernel": 0, "planes_sum_kernel": 0}, "PPCX 5120x17408 batch 96"),
+    "planes_prompt_m1000_5120x17408": (
+        "A prompt of 1000 rows through 5120x17408 held as planes, MI355X (gfx950)",
+        ["profiles/prompts.py", "prompt"], {"planes_prompt_kernel": 0, "dense_sum_kernel": 0}, "prompt of 1000 rows, 5120x17408"),
+    "planes_lookup_777_of_8192x5120": (
+        "An embedding lookup, 777 rows of 8192x5120 held as planes, MI355X (gfx950)",
+        ["profiles/prompts.py", "lookup"], {"planes_gather_kernel": 0}, "lookup of 777 rows, 8192x5120"),
+    "planes_m64_stack_64_layers": (
+        "Whole stack at the 27B model's shapes: 64 layers (48 with gated-delta-net projections, 16 with attention q/k/v/o) x "
+        "(projections, gate, up, down) + embedding and head (248320x5120), batch 64, held as planes, MI355X (gfx950)",
+        ["--workload", "stack", "--steps", "3", "--warmup", "1"], {}, ""),
+    # the walk, which small matrices and frames of few exponents take, at the same sizes
     "fused_gemv_m1_qwen27b_mlp": (
         f"Fused decode-GEMV (wave units), batch 1, {MLP}\n"
         "one step = gate and up in one grouped launch (they take the same activations) + down in a launch of its own",
-        [], {"fused_wave_group_kernel": 2 * MATRIX, "fused_wave_kernel": MATRIX}, "Qwen-27B-like MLP batch 1"),
+        ["--walked"], {"fused_wave_group_kernel": 2 * MATRIX, "fused_wave_kernel": MATRIX}, "Qwen-27B-like MLP batch 1"),
     "fused_gemm_m64_qwen27b_mlp": (
         f"Fused decode-GEMM (matrix cores), batch 64, {MLP}\n"
         "one step = gate and up in one grouped launch + down cut in three along K",
-        ["--batch", "64"], {"fused_gemm_group_kernel": 2 * MATRIX, "fused_gemm_kernel": MATRIX}, "Qwen-27B-like MLP batch 64"),
+        ["--walked", "--batch", "64"], {"fused_gemm_group_kernel": 2 * MATRIX, "fused_gemm_kernel": MATRIX}, "Qwen-27B-like MLP batch 64"),
     "fused_store_decode_qwen27b_mlp": (
         f"Fused decode to dense BF16 (store sink over wave units), {MLP}\none step = three launches",
-        ["--workload", "decode"], {"fused_wave_store_kernel": MATRIX}, "Qwen-27B-like MLP decode"),
+        ["--walked", "--workload", "decode"], {"fused_wave_store_kernel": MATRIX}, "Qwen-27B-like MLP decode"),
     "ppcx_gemv_m1_5120x17408": (
         "Fused decode-GEMV of a predictive (PPCX) weight, 5120x17408, batch 1, MI355X (gfx950)",
-        ["--workload", "ppcx", "--batch", "1"], {"fused_wave_kernel": MATRIX}, "PPCX 5120x17408 batch 1"),
+        ["--walked", "--workload", "ppcx", "--batch", "1"], {"fused_wave_kernel": MATRIX}, "PPCX 5120x17408 batch 1"),
     "ppcx_gemm_m96_5120x17408": (
         "Fused decode-GEMM of a predictive (PPCX) weight, 5120x17408, 96 rows, MI355X (gfx950)",
-        ["--workload", "ppcx", "--batch", "96"],
+        ["--walked", "--workload", "ppcx", "--batch", "96"],
         {"fused_gemm_wide_kernel": MATRIX, "pack_activations_kernel": 0, "gemm_sum_parts_kernel": 0}, "PPCX 5120x17408 batch 96"),
     "prompt_m1000_5120x17408": (
         "A prompt of 1000 rows through 5120x17408: fused decode to dense BF16, then the product over it, MI355X (gfx950)",
-        ["profiles/prompts.py", "prompt"], {"dense_gemm_kernel": 0, "dense_sum_kernel": 0, "fused_wave_store_kernel": MATRIX},
+        ["profiles/prompts.py", "prompt", "--walked"], {"dense_gemm_kernel": 0, "dense_sum_kernel": 0, "fused_wave_store_kernel": MATRIX},
         "prompt of 1000 rows, 5120x17408"),
     "lookup_777_of_8192x5120": (
         "An embedding lookup, 777 rows of 8192x5120, MI355X (gfx950)",
-        ["profiles/prompts.py", "lookup"], {"fused_gather_kernel": 777 * 5120}, "lookup of 777 rows, 8192x5120"),
+        ["profiles/prompts.py", "lookup", "--walked"], {"fused_gather_kernel": 777 * 5120}, "lookup of 777 rows, 8192x5120"),
     "fused_gemm_m64_stack_64_layers": (
         "Whole stack at the 27B model's shapes: 64 layers (48 with gated-delta-net projections, 16 with attention q/k/v/o) x "
         "(projections, gate, up, down) + embedding and head (248320x5120), batch 64, MI355X (gfx950)",
-        ["--workload", "stack", "--steps", "3", "--warmup", "1"], {}, ""),
+        ["--walked", "--workload", "stack", "--steps", "3", "--warmup", "1"], {}, ""),
 }
 COUNTERS = (
     "SQ_WAVES SQ_INSTS_VALU SQ_INSTS_LDS SQ_INSTS_SALU SQ_ACTIVE_INST_VALU SQ_ACTIVE_INST_LDS SQ_BUSY_CU_CYCLES SQ_WAVE_CYCLES",

@@ -29,16 +29,20 @@ def test_recorded_traffic_is_withheld_for_other_kernel_sources(monkeypatch):
     figure, source = bench.recorded_traffic(False, 1, name)
     assert figure is None and "other kernel sources" in source
     assert bench.recorded_traffic(False, 7, name)[0] is None  # no counter record for that batch
+    assert "planes_ppcx_m96_5120x17408" in bench.recorded_traffic(False, 96, "planes_batch_kernel", prefix="ppcx")[1]
+    assert "no counter record" in bench.recorded_traffic(False, 32, "planes_product_kernel or planes_batch_kernel")[1]
 
 
 @pytest.mark.parametrize("profile,decode_only,m,grouped", [
     ("fused_gemv_m1_qwen27b_mlp", False, 1, True), ("fused_gemv_m1_qwen27b_mlp", False, 1, False),
     ("fused_gemm_m64_qwen27b_mlp", False, 64, True), ("fused_gemm_m64_qwen27b_mlp", False, 64, False),
-    ("fused_store_decode_qwen27b_mlp", True, 1, False)])
+    ("fused_store_decode_qwen27b_mlp", True, 1, False), ("planes_m1_gate_up", False, 1, True), ("planes_m64_gate_up", False, 64, True),
+    ("planes_decode_qwen27b_mlp", True, 0, False), ("planes_ppcx_m1_5120x17408", False, 1, False),
+    ("planes_ppcx_m96_5120x17408", False, 96, False)])
 def test_kernels_it_names_are_the_ones_that_were_profiled(profile, decode_only, m, grouped):
     sys.path.insert(0, str(ROOT))
     import bench
-    name = bench.kernel_name(decode_only, m, grouped)
+    name = bench.kernel_name(decode_only, m, grouped, planes=profile.startswith("planes"))
     assert name.split(", MT")[0].rstrip(">") in (ROOT / "profiles" / f"{profile}.txt").read_text()
     record = json.loads((ROOT / "profiles" / f"{profile}_traffic.json").read_text())
     assert name.split("<")[0].split("::")[-1] in record["traffic_bytes_per_launch"]
